@@ -1,4 +1,4 @@
-"""ctypes binding of libmdx.so (C ABI declared in include/mdx.h)."""
+"""Loads libmdx.so (ctypes binding of the C ABI declared in include/mdx.h) and the native host module on top of it."""
 from __future__ import annotations
 
 import ctypes
@@ -57,6 +57,21 @@ SIGNATURES = {
 }
 
 _lib = None
+_host = None
+
+
+def host():
+    """The extension module behind mdx.ops and mdx.layers (csrc/host_ops.cpp); raises if it has not been built."""
+    global _host
+    if _host is None:
+        lib()
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise MdxError(f"mdx/_host.so cannot be loaded ({e}): build it with `python mineru-diffusion_amd/build.py`; "
+                           "there is no fallback") from e
+        _host = module
+    return _host
 
 
 def lib() -> ctypes.CDLL:

@@ -5,19 +5,7 @@ import torch
 from torch import nn
 
 from .context import get_context
-from .ops import flash_attn_with_kvcache, sparse_attn_varlen, store_kvcache_maybe4d, unmask_step
-
-
-_side_streams: dict = {}
-
-
-def _side_stream(device: torch.device) -> torch.cuda.Stream:
-    """One extra stream per device (default priority) for work that may run beside the caller's stream."""
-    index = device.index if device.index is not None else torch.cuda.current_device()
-    stream = _side_streams.get(index)
-    if stream is None:
-        stream = _side_streams[index] = torch.cuda.Stream(device=index)
-    return stream
+from .ops import _host
 
 
 class Attention(nn.Module):
@@ -35,29 +23,12 @@ class Attention(nn.Module):
 
     def forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor):
         context = get_context()
-        k_cache, v_cache = self.k_cache, self.v_cache
-        have_cache = bool(k_cache.numel() and v_cache.numel())
         if context.is_prefill:
-            # The prefill attention reads k / v, not the cache: the store is independent of it and runs beside it on a
-            # second stream (its small workgroups fill the gaps between the attention kernel's, which own whole CUs:
-            # config 3, 0.820 -> 0.808 ms for the pair).  The caller's stream waits for both before it goes on.
-            main = torch.cuda.current_stream(q.device)
-            side = _side_stream(q.device) if have_cache else None
-            if side is not None:
-                side.wait_stream(main)
-                with torch.cuda.stream(side):
-                    store_kvcache_maybe4d(k, v, k_cache, v_cache, context.slot_mapping)
-            o = sparse_attn_varlen(q, k, v, cu_seqlens_q=context.cu_seqlens_q, cu_seqlens_k=context.cu_seqlens_k,
-                                   staircase_size=context.block_size,
-                                   max_seqlen=context.max_seqlen_k or None, softmax_scale=self.scale)
-            if side is not None:
-                main.wait_stream(side)
-            return o.flatten(1)
-        if have_cache:
-            store_kvcache_maybe4d(k, v, k_cache, v_cache, context.slot_mapping)
-        o = flash_attn_with_kvcache(q, k_cache, v_cache, cache_seqlens=context.context_lens,
-                                    block_table=context.block_tables, softmax_scale=self.scale, causal=False)
-        return o.flatten(2)
+            # the prefill attention reads k / v, not the cache: for long prompts the store runs beside it on a second stream
+            return _host().attention_prefill(q, k, v, self.k_cache, self.v_cache, context.slot_mapping, context.cu_seqlens_q,
+                                             context.cu_seqlens_k, context.block_size, context.max_seqlen_k or 0, self.scale)
+        return _host().attention_decode(q, k, v, self.k_cache, self.v_cache, context.slot_mapping, context.context_lens,
+                                        context.block_tables, self.scale)
 
 
 class Sampler(nn.Module):
@@ -91,13 +62,12 @@ class Sampler(nn.Module):
         strategy = seqs[0].sampling_params.denoising_strategy
         if strategy != 'low_confidence_dynamic':
             raise NotImplementedError(f"Denoising strategy {strategy} not implemented")
-        threshold = seqs[0].sampling_params.dynamic_threshold
-        x = torch.stack([seq.current_denoising_block for seq in seqs], dim=0).to(logits.device)
-        _, _, transfer, count = unmask_step(logits, x, seqs[0].mask_token_id, threshold, self.k,
-                                            temperatures=temperatures, **self._noise_args(logits))
-        x_cpu, transfer_cpu = x.cpu(), transfer.cpu()
-        for i, seq in enumerate(seqs):
-            seq.current_denoising_block = x_cpu[i]
-            seq.current_step_map[transfer_cpu[i]] = seq.current_denoise_step
+        noise = self._noise_args(logits)
+        blocks, committed = _host().sampler_step(
+            logits, temperatures, [seq.current_denoising_block for seq in seqs], [seq.current_step_map for seq in seqs],
+            [seq.current_denoise_step for seq in seqs], seqs[0].mask_token_id, seqs[0].sampling_params.dynamic_threshold, self.k,
+            noise.get("noise"), noise.get("seed"), noise.get("offset", 0), None, None)
+        for seq, block in zip(seqs, blocks):
+            seq.current_denoising_block = block
             seq.current_denoise_step += 1
-        return int(count.sum().item())
+        return committed
