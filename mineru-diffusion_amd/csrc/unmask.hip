@@ -337,9 +337,18 @@ __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
             if (v > best || (v == best && index < best_idx)) { best = v; best_x = x; best_idx = index; }
         };
         auto noise_at = [&](int64_t e) { return NOISE == 1 ? np[e] : rn.at((int)e); };
+        // The chunks after this one are on their way while it is worked on: few wavefronts share a SIMD here (96 rows:
+        // three), and where the noise of a chunk is skipped there is little else to hide a trip to HBM behind.
+        u32x4 next[kUnroll];
+#pragma unroll
+        for (int k = 0; k < kUnroll; ++k)
+            if (cbeg + tid + k * kThreads < cend) next[k] = __builtin_nontemporal_load(cp + cbeg + tid + k * kThreads);
         for (int64_t ch = cbeg + tid; ch < cend; ch += kThreads) {
             float x[EPC];
-            Elem<T>::unpack(__builtin_nontemporal_load(cp + ch), x);
+            Elem<T>::unpack(next[0], x);
+#pragma unroll
+            for (int k = 0; k + 1 < kUnroll; ++k) next[k] = next[k + 1];
+            if (ch + kUnroll * kThreads < cend) next[kUnroll - 1] = __builtin_nontemporal_load(cp + ch + kUnroll * kThreads);
             const float cmx = take_values(x, ch);
             const int c0 = (int)(lead + ch * EPC);
             // No draw of the generator exceeds kGumbelMax, and rounding is monotonic: an element of this chunk can
@@ -444,29 +453,67 @@ __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
     }
 }
 
-// Merges the row splits: one lane per row.
+// A row's splits merged by the 16 lanes of a group: each takes every 16th, then four exchanges.  (One lane per row walking
+// the splits was a chain of dependent trips to memory: 6.2 us for nine splits, a third of what 96 sampled rows take.)
+constexpr int kMergeLanes = 16;
+template <bool NOISE>
+__device__ __forceinline__ Partial merge_splits(const Partial* __restrict__ partials, int nsplit, int lane16, float c) {
+    Partial r;
+    r.m = kNegBig; r.s = 0.f; r.idx = kNoIndex; r.pick = kNegBig; r.pick_x = 0.f; r.pick_idx = kNoIndex;
+    for (int s = lane16; s < nsplit; s += kMergeLanes) combine(r, partials[s], c, NOISE);
+#pragma unroll
+    for (int off = kMergeLanes / 2; off >= 1; off >>= 1) combine(r, shfl_xor(r, off, NOISE), c, NOISE);
+    return r;
+}
+
 template <bool NOISE>
 __global__ __launch_bounds__(kThreads) void confidence_finalize_kernel(
     const Partial* __restrict__ partials, int nsplit,
     const float* __restrict__ temperatures, int rows_per_temp,
     int64_t rows, int64_t* __restrict__ x0, float* __restrict__ x0_p)
 {
-    const int64_t row = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-    if (row >= rows) return;
-    const float T_ = temperatures ? temperatures[row / rows_per_temp] : 1.0f;
-    const float c = kLog2e / T_;
-    Partial r = partials[row * nsplit];
-    for (int s = 1; s < nsplit; ++s) combine(r, partials[row * nsplit + s], c, NOISE);
+    const int64_t row = (int64_t)blockIdx.x * (kThreads / kMergeLanes) + threadIdx.x / kMergeLanes;
+    const int lane16 = threadIdx.x % kMergeLanes;
+    if (row >= rows) return;                                 // (whole groups)
+    const float c = kLog2e / (temperatures ? temperatures[row / rows_per_temp] : 1.0f);
+    const Partial r = merge_splits<NOISE>(partials + row * nsplit, nsplit, lane16, c);
+    if (lane16 != 0) return;
     int64_t tok; float conf;
     finish_row<NOISE>(r, c, tok, conf);
     x0[row] = tok;
     x0_p[row] = conf;
 }
 
-// One workgroup per sequence; lane p owns block position p.  With FROM_PARTIALS the row splits
-// of the vocabulary pass are merged here (and x0 / x0_p written), saving a launch.
+// Where a selection kernel finds the confidences: written by the vocabulary pass, or as row splits that it merges first
+// (and then writes x0 / x0_p itself), which saves a launch.
+enum Source { kFromRows = 0, kFromSplits = 1, kFromNoisySplits = 2 };
 constexpr int kMaxBlockLen = 1024;
-template <bool FROM_PARTIALS>
+constexpr int kMaxSelectThreads = 1024;
+
+// The block's confidences and picks into LDS, merged from the splits where need be; all threads of the workgroup.
+template <int SOURCE>
+__device__ __forceinline__ void gather_block(float* conf_s, int* pick_s, int64_t* x0, float* x0_p, const Partial* partials, int nsplit,
+                                             const float* temperatures, int b, int block_len)
+{
+    const int lane16 = threadIdx.x % kMergeLanes;
+    const float c = kLog2e / (temperatures ? temperatures[b] : 1.0f);
+    for (int p = threadIdx.x / kMergeLanes; p < block_len; p += blockDim.x / kMergeLanes) {
+        const int64_t at = (int64_t)b * block_len + p;
+        const Partial r = merge_splits<SOURCE == kFromNoisySplits>(partials + at * nsplit, nsplit, lane16, c);
+        if (lane16 == 0) {
+            int64_t tok; float conf;
+            finish_row<SOURCE == kFromNoisySplits>(r, c, tok, conf);
+            x0[at] = tok;
+            x0_p[at] = conf;
+            pick_s[p] = (int)tok;
+            conf_s[p] = conf;
+        }
+    }
+    __syncthreads();
+}
+
+// One workgroup per sequence; lane p owns block position p.
+template <int SOURCE>
 __global__ __launch_bounds__(kMaxBlockLen) void select_transfer_kernel(
     int64_t* __restrict__ x0, float* __restrict__ x0_p, int64_t* __restrict__ tokens,
     const Partial* __restrict__ partials, int nsplit, const float* __restrict__ temperatures,
@@ -474,28 +521,23 @@ __global__ __launch_bounds__(kMaxBlockLen) void select_transfer_kernel(
     uint8_t* __restrict__ transfer, int32_t* __restrict__ count, int block_len)
 {
     __shared__ float conf_s[kMaxBlockLen];
+    __shared__ int pick_s[SOURCE == kFromRows ? 1 : kMaxBlockLen];
     __shared__ int n_hi, n_masked, n_commit;
     const int b = blockIdx.x;
     const int p = threadIdx.x;
     const bool on = p < block_len;
     const int64_t at = (int64_t)b * block_len + p;
     if (p == 0) { n_hi = 0; n_masked = 0; n_commit = 0; }
-    __syncthreads();
     int64_t pick = 0;
     float pick_p = 0.f;
-    if (on) {
-        if (FROM_PARTIALS) {
-            const float c = kLog2e / (temperatures ? temperatures[b] : 1.0f);
-            Partial r = partials[at * nsplit];
-            for (int s = 1; s < nsplit; ++s) combine(r, partials[at * nsplit + s], c, false);
-            finish_row<false>(r, c, pick, pick_p);
-            x0[at] = pick;
-            x0_p[at] = pick_p;
-        } else {
-            pick = x0[at];
-            pick_p = x0_p[at];
-        }
+    if (SOURCE != kFromRows) {
+        gather_block<SOURCE>(conf_s, pick_s, x0, x0_p, partials, nsplit, temperatures, b, block_len);
+        if (on) { pick = pick_s[p]; pick_p = conf_s[p]; }
+    } else if (on) {
+        pick = x0[at];
+        pick_p = x0_p[at];
     }
+    __syncthreads();
     const bool masked = on && tokens[at] == mask_token_id;
     const float conf = masked ? pick_p : -INFINITY;
     const bool hi = conf > threshold;
@@ -531,34 +573,31 @@ __global__ __launch_bounds__(kMaxBlockLen) void select_transfer_kernel(
 // The same rule for blocks of up to 64 positions (the engine's blocks hold 32) with ONE wavefront per
 // sequence: lane p owns position p, counts are ballots, and the rank among the masked positions comes
 // from reading every lane's confidence in turn -- no LDS, no atomics, no barrier, so the launch costs
-// little more than its one round trip to memory.
-template <bool FROM_PARTIALS>
-__global__ __launch_bounds__(mdx::kWave) void select_transfer_wave_kernel(
+// little more than its one round trip to memory.  Where the row splits have to be merged first, the sequence gets
+// 16 lanes per position for that, and its first wavefront goes on alone.
+template <int SOURCE>
+__global__ __launch_bounds__(kMaxSelectThreads) void select_transfer_wave_kernel(
     int64_t* __restrict__ x0, float* __restrict__ x0_p, int64_t* __restrict__ tokens,
     const Partial* __restrict__ partials, int nsplit, const float* __restrict__ temperatures,
     int64_t mask_token_id, float threshold, int k,
     uint8_t* __restrict__ transfer, int32_t* __restrict__ count, int block_len)
 {
+    __shared__ float conf_s[SOURCE == kFromRows ? 1 : mdx::kWave];
+    __shared__ int pick_s[SOURCE == kFromRows ? 1 : mdx::kWave];
     const int b = blockIdx.x;
     const int p = threadIdx.x;
     const bool on = p < block_len;
     const int64_t at = (int64_t)b * block_len + p;
     int64_t pick = 0;
     float pick_p = 0.f;
-    int64_t tok = 0;
-    if (on) {
-        tok = tokens[at];
-        if (FROM_PARTIALS) {
-            const float c = kLog2e / (temperatures ? temperatures[b] : 1.0f);
-            Partial r = partials[at * nsplit];
-            for (int s = 1; s < nsplit; ++s) combine(r, partials[at * nsplit + s], c, false);
-            finish_row<false>(r, c, pick, pick_p);
-            x0[at] = pick;
-            x0_p[at] = pick_p;
-        } else {
-            pick = x0[at];
-            pick_p = x0_p[at];
-        }
+    const int64_t tok = on ? tokens[at] : 0;
+    if (SOURCE != kFromRows) {
+        gather_block<SOURCE>(conf_s, pick_s, x0, x0_p, partials, nsplit, temperatures, b, block_len);
+        if (p >= mdx::kWave) return;
+        if (on) { pick = pick_s[p]; pick_p = conf_s[p]; }
+    } else if (on) {
+        pick = x0[at];
+        pick_p = x0_p[at];
     }
     const bool masked = on && tok == mask_token_id;
     const float conf = masked ? pick_p : -INFINITY;
@@ -583,27 +622,27 @@ __global__ __launch_bounds__(mdx::kWave) void select_transfer_wave_kernel(
     if (p == 0) count[b] = n_commit;
 }
 
-int launch_select(int64_t* x0, float* x0_p, int64_t* tokens, const Partial* partials, int nsplit, const float* temperatures,
+int launch_select(int64_t* x0, float* x0_p, int64_t* tokens, const Partial* partials, int nsplit, bool noisy, const float* temperatures,
                   int64_t mask_token_id, float threshold, int k, uint8_t* transfer, int32_t* count, int bs, int block_len,
                   hipStream_t stream)
 {
-    const bool from_partials = partials != nullptr && nsplit > 1;
+    const int source = partials == nullptr || nsplit <= 1 ? kFromRows : noisy ? kFromNoisySplits : kFromSplits;
+    const int whole_waves = (block_len + mdx::kWave - 1) / mdx::kWave * mdx::kWave;
+    // lanes to merge splits with: 16 per position, as many positions at a time as a workgroup holds
+    const int merging = block_len * kMergeLanes < kMaxSelectThreads ? (block_len * kMergeLanes + mdx::kWave - 1) / mdx::kWave * mdx::kWave : kMaxSelectThreads;
+    const unsigned threads = source == kFromRows ? whole_waves : (merging > whole_waves ? merging : whole_waves);
+#define MDX_SELECT(KERNEL, SOURCE) KERNEL<SOURCE><<<(unsigned)bs, threads, 0, stream>>>( \
+        x0, x0_p, tokens, partials, nsplit, temperatures, mask_token_id, threshold, k, transfer, count, block_len)
     if (block_len <= mdx::kWave) {
-        if (from_partials)
-            select_transfer_wave_kernel<true><<<(unsigned)bs, mdx::kWave, 0, stream>>>(
-                x0, x0_p, tokens, partials, nsplit, temperatures, mask_token_id, threshold, k, transfer, count, block_len);
-        else
-            select_transfer_wave_kernel<false><<<(unsigned)bs, mdx::kWave, 0, stream>>>(
-                x0, x0_p, tokens, nullptr, 1, nullptr, mask_token_id, threshold, k, transfer, count, block_len);
+        if (source == kFromRows)        MDX_SELECT(select_transfer_wave_kernel, kFromRows);
+        else if (source == kFromSplits) MDX_SELECT(select_transfer_wave_kernel, kFromSplits);
+        else                            MDX_SELECT(select_transfer_wave_kernel, kFromNoisySplits);
     } else {
-        const int threads = ((block_len + mdx::kWave - 1) / mdx::kWave) * mdx::kWave;
-        if (from_partials)
-            select_transfer_kernel<true><<<(unsigned)bs, threads, 0, stream>>>(
-                x0, x0_p, tokens, partials, nsplit, temperatures, mask_token_id, threshold, k, transfer, count, block_len);
-        else
-            select_transfer_kernel<false><<<(unsigned)bs, threads, 0, stream>>>(
-                x0, x0_p, tokens, nullptr, 1, nullptr, mask_token_id, threshold, k, transfer, count, block_len);
+        if (source == kFromRows)        MDX_SELECT(select_transfer_kernel, kFromRows);
+        else if (source == kFromSplits) MDX_SELECT(select_transfer_kernel, kFromSplits);
+        else                            MDX_SELECT(select_transfer_kernel, kFromNoisySplits);
     }
+#undef MDX_SELECT
     return mdx::check_launch("select_transfer");
 }
 
@@ -637,7 +676,7 @@ int launch_confidence(const void* logits, int64_t row_stride, const float* tempe
             (const T*)logits, row_stride, temperatures, rows_per_temp, N, vocab, nsplit, partials, x0, x0_p);
     int rc = mdx::check_launch("confidence_argmax");
     if (rc != MDX_OK || nsplit == 1 || !finalize) return rc;
-    const unsigned fgrid = (unsigned)((rows + kThreads - 1) / kThreads);
+    const unsigned fgrid = (unsigned)((rows + kThreads / kMergeLanes - 1) / (kThreads / kMergeLanes));
     if (noisy)
         confidence_finalize_kernel<true><<<fgrid, kThreads, 0, stream>>>(partials, nsplit, temperatures, rows_per_temp, rows, x0, x0_p);
     else
@@ -760,7 +799,7 @@ extern "C" int mdx_select_transfer(const int64_t* x0, const float* x0_p, int64_t
     MDX_REQUIRE(x0 && x0_p && tokens && transfer && count, MDX_EINVAL, "select_transfer: null pointer");
     MDX_REQUIRE(block_len <= kMaxBlockLen, MDX_EUNSUPPORTED, "select_transfer: block_len %d > %d", block_len, kMaxBlockLen);
     MDX_REQUIRE(k >= 0, MDX_EINVAL, "select_transfer: k %d < 0", k);
-    return launch_select(const_cast<int64_t*>(x0), const_cast<float*>(x0_p), tokens, nullptr, 1, nullptr, mask_token_id, threshold, k,
+    return launch_select(const_cast<int64_t*>(x0), const_cast<float*>(x0_p), tokens, nullptr, 1, false, nullptr, mask_token_id, threshold, k,
                          transfer, count, bs, block_len, stream);
 }
 
@@ -778,13 +817,13 @@ int unmask_step_impl(const void* logits, int64_t row_stride, int32_t dtype,
     MDX_REQUIRE(block_len <= kMaxBlockLen, MDX_EUNSUPPORTED, "unmask_step: block_len %d > %d", block_len, kMaxBlockLen);
     if (bs == 0 || block_len == 0) return MDX_OK;
     MDX_REQUIRE(tokens && transfer && count, MDX_EINVAL, "unmask_step: null pointer");
-    // Without noise the selection kernel merges the row splits itself (one launch fewer).
+    // The selection kernel merges the row splits itself (one launch fewer).
     const bool noisy = N.noise != nullptr || N.philox;
     int nsplit = 1;
     int rc = confidence_pass(logits, row_stride, dtype, temperatures, block_len, N,
-                             x0, x0_p, (int64_t)bs * block_len, vocab, workspace, workspace_bytes, noisy, &nsplit, stream);
+                             x0, x0_p, (int64_t)bs * block_len, vocab, workspace, workspace_bytes, false, &nsplit, stream);
     if (rc != MDX_OK) return rc;
-    return launch_select(x0, x0_p, tokens, (nsplit > 1 && !noisy) ? static_cast<const Partial*>(workspace) : nullptr, nsplit, temperatures,
+    return launch_select(x0, x0_p, tokens, nsplit > 1 ? static_cast<const Partial*>(workspace) : nullptr, nsplit, noisy, temperatures,
                          mask_token_id, threshold, k, transfer, count, bs, block_len, stream);
 }
 
