@@ -328,7 +328,10 @@ Tensor paged(const Tensor& q_, const Tensor& k_cache, const Tensor& v_cache, con
     const Tensor bt = int32_list(bt_, "block_table"), lens = int32_list(lens_, "cache_seqlens");
     NEED(bt.dim() == 2 && bt.size(0) == bs && lens.numel() == bs);
     Tensor o = flat ? make(q, q.scalar_type(), bs, sq, hq * d) : make(q, q.scalar_type(), bs, sq, hq, d);
-    const int64_t bytes = mdx_paged_block_attn_workspace_bytes((int32_t)bs, (int32_t)sq, (int32_t)hq, (int32_t)hkv, (int32_t)d, (int32_t)bt.size(1), (int32_t)page);
+    const bool f32_arithmetic = q.scalar_type() == at::kFloat || d > 128 || d % 16 != 0;
+    const int64_t bytes = f32_arithmetic
+        ? mdx_paged_block_attn_f32_workspace_bytes((int32_t)bs, (int32_t)sq, (int32_t)hq, (int32_t)d, (int32_t)bt.size(1), (int32_t)page)
+        : mdx_paged_block_attn_workspace_bytes((int32_t)bs, (int32_t)sq, (int32_t)hq, (int32_t)hkv, (int32_t)d, (int32_t)bt.size(1), (int32_t)page);
     const Tensor ws = bytes > 0 ? make(q, at::kByte, bytes) : Tensor();
     Tensor counters;
     if (counters_arg == Py_None) {         // more than 64 sequences never take the single-launch path

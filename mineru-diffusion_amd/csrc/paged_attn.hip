@@ -619,7 +619,7 @@ int launch_paged_f32(const void* q, void* o, const void* k_cache, const void* v_
                      const int32_t* block_table, int64_t bt_stride, const int32_t* context_lens,
                      int32_t bs, int32_t sq, int32_t num_q_heads, int32_t num_kv_heads,
                      int32_t head_dim, int32_t max_pages, int32_t page_size, int64_t num_pages,
-                     float scale, int32_t dtype, hipStream_t stream);                         // paged_attn_f32.hip
+                     float scale, int32_t dtype, void* workspace, int64_t workspace_bytes, hipStream_t stream);   // paged_attn_f32.hip
 
 // The launch behind every paged entry point of the library.
 int launch_paged(const void* q, void* o, const void* k_cache, const void* v_cache,
@@ -637,7 +637,7 @@ int launch_paged(const void* q, void* o, const void* k_cache, const void* v_cach
     MDX_REQUIRE(bs >= 0 && sq >= 0 && max_pages >= 0 && num_pages >= 0, MDX_EINVAL, "paged_block_attn: negative size");
     MDX_REQUIRE(dtype == MDX_BF16 || dtype == MDX_F16 || dtype == MDX_F32, MDX_EUNSUPPORTED, "paged_block_attn: dtype %d (bf16, fp16 or fp32)", dtype);
     // 16-bit elements and heads of 16, 32, ..., 128 columns run on the 16-bit matrix instructions; fp32 tensors and
-    // the other head widths up to 256 on the fp32 one (paged_attn_f32.hip: no split, no workspace)
+    // the other head widths up to 256 on the fp32 one (paged_attn_f32.hip: cut into as many pieces as the workspace has room for)
     const bool f32_arithmetic = dtype == MDX_F32 || head_dim > kHeadDim || head_dim % 16 != 0;
     MDX_REQUIRE(head_dim >= 4 && head_dim <= 256 && head_dim % 4 == 0, MDX_EUNSUPPORTED,
                 "paged_block_attn: head_dim %d (multiples of 4 up to 256)", head_dim);
@@ -654,7 +654,7 @@ int launch_paged(const void* q, void* o, const void* k_cache, const void* v_cach
     if (f32_arithmetic)
         return launch_paged_f32(q, o, k_cache, v_cache, q_stride_b, q_stride_s, q_stride_h, o_stride_b, o_stride_s, o_stride_h,
                                 cache_stride_page, cache_stride_tok, cache_stride_head, block_table, bt_stride, context_lens,
-                                bs, sq, num_q_heads, num_kv_heads, head_dim, max_pages, page_size, num_pages, scale, dtype, stream);
+                                bs, sq, num_q_heads, num_kv_heads, head_dim, max_pages, page_size, num_pages, scale, dtype, workspace, workspace_bytes, stream);
     MDX_REQUIRE(mdx::aligned16(q) && mdx::aligned16(o) && mdx::aligned16(k_cache) && mdx::aligned16(v_cache) &&
                 q_stride_b % 8 == 0 && q_stride_s % 8 == 0 && q_stride_h % 8 == 0 &&
                 o_stride_b % 8 == 0 && o_stride_s % 8 == 0 && o_stride_h % 8 == 0 &&

@@ -5,10 +5,16 @@
 // itself runs bf16 with d = 128, so this is the path for callers outside the model's own configuration.
 // Arithmetic and layout: attn_f32_tile.h.
 //
-// A workgroup serves one (sequence, query head, tile of 32 queries).  Its NW wavefronts (4 for heads of up to 128
-// columns, 2 for wider ones: what fits in LDS) take consecutive tiles of 32 keys, NW tiles staged at a time, each
-// wavefront with its own running softmax state; at the end the states are merged through LDS and every wavefront
-// writes its share of the head's columns.  No split over workgroups and no workspace.
+// What bounds it is the fp32 matrix instruction: 128 of them, 64 cycles each, per wavefront, head and tile of 32 keys.  So
+// the contexts are cut into pieces of keys until the chip's wavefront slots are filled (one sequence of 1056 keys is 16 x 33
+// such steps for 1024 SIMDs), the pieces' states go to fp32 partials in the workspace, and a second, small launch folds
+// them.  (One workgroup per sequence and query head walking the whole context, the form this replaced, left 240 of 256 CUs
+// idle on that shape: 84 us.)
+//
+// A workgroup serves one (sequence, piece, group of HPW query heads that share a KV head, tile of 32 queries): HPW x KW
+// wavefronts, each on one head and every KW-th tile of 32 keys, KW tiles staged at a time.  Two query heads per workgroup
+// halve what is staged per product, and with 68 KB of LDS two workgroups share a CU, so that one stages while the other
+// multiplies.
 // The semantics are those of the 16-bit kernel: non-causal, the first min(context_lens[b], max_pages x
 // page_size) keys through block_table[b]; keys on a page id outside [0, num_pages) are left out; a sequence
 // without any key yields zeros.
@@ -25,29 +31,57 @@ struct PagedWideParams {
     int64_t c_sp, c_st, c_sh;                       // cache strides: page, token, head
     const int32_t* block_table; int64_t bt_stride;
     const int32_t* context_lens;
-    int sq, heads_per_kv, page_size, max_pages, head_dim;
+    int bs, sq, nqt, num_q_heads, heads_per_kv, page_size, max_pages, head_dim;
     int64_t num_pages;
     float c;                                        // scale * log2(e)
+    int nsplit, pieces;                             // partial slots per sequence; pieces the whole launch should be cut into per (head group, query tile)
+    float* part_o; float* part_ml;                  // [bs, Hq, nqt, nsplit, 32, D] and [bs, Hq, nqt, nsplit, 2, 32]
 };
 
-template <typename T, int D, int NW>
-__global__ __launch_bounds__(64 * NW, 1) void paged_attn_f32_kernel(const PagedWideParams P)
+constexpr int kLeastKeys = 64;                      // keys of a piece: a multiple of this
+constexpr int kMaxSplits = 64;
+
+__device__ __forceinline__ int keys_of(const PagedWideParams& P, int b) {
+    const int64_t room = (int64_t)P.max_pages * P.page_size;
+    const int raw = P.context_lens[b];
+    return max(0, (int)(raw < room ? raw : room));
+}
+
+// Keys per piece of sequence b (all wavefronts of both kernels find the same).  Pieces of one size for all sequences, so that a
+// long sequence gets more of them and all workgroups run equally long: total keys / pieces, but never more pieces of a
+// sequence than it has slots.  Beyond 64 sequences, whose lengths no wavefront holds, a sequence is cut evenly.
+__device__ __forceinline__ int keys_per_piece(const PagedWideParams& P, int ctx, int lane) {
+    int want = (ctx + P.nsplit - 1) / P.nsplit;
+    if (P.bs <= 64) {
+        int total = lane < P.bs ? keys_of(P, lane) : 0;
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) total += __shfl_xor(total, off);
+        want = max(want, (total + P.pieces - 1) / P.pieces);
+    }
+    return max(1, (want + kLeastKeys - 1) / kLeastKeys) * kLeastKeys;
+}
+
+template <typename T, int D, int HPW, int KW>
+__global__ __launch_bounds__(64 * HPW * KW, D <= 128 ? 2 : 1) void paged_attn_f32_kernel(const PagedWideParams P)
 {
-    constexpr int kThreads = 64 * NW;
+    constexpr int kThreads = 64 * HPW * KW;
     constexpr int kTileFloats = Lds<D>::kFloats;
-    extern __shared__ __attribute__((aligned(16))) float lds[];          // NW tiles (K and V of 32 keys each)
+    extern __shared__ __attribute__((aligned(16))) float lds[];          // KW tiles (K and V of 32 keys each), or the states to merge
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int H = lane >> 5, r = lane & 31;
-    const int head = blockIdx.x, qt = blockIdx.y, b = blockIdx.z;
-    const int kvh = head / P.heads_per_kv;
+    const int kw = wave % KW, hw = wave / KW;
+    const int head = (blockIdx.x / P.nqt) * HPW + hw, qt = blockIdx.x % P.nqt, split = blockIdx.y, b = blockIdx.z;
+    const int kvh = (blockIdx.x / P.nqt) * HPW / P.heads_per_kv;
     const int width = P.head_dim;
 
-    const int64_t room = (int64_t)P.max_pages * P.page_size;
-    const int ctx_raw = P.context_lens[b];
-    const int ctx = (int)(ctx_raw < room ? ctx_raw : room);
+    const int ctx = keys_of(P, b);
+    const int span = P.nsplit > 1 ? keys_per_piece(P, ctx, lane) : max(1, ctx);
+    const int n_pieces = max(1, (ctx + span - 1) / span);
+    if (split >= n_pieces) return;
+    const int key_begin = split * span, key_end = min(ctx, key_begin + span);
     const int32_t* bt = P.block_table + (int64_t)b * P.bt_stride;
-    const int n_tiles = ctx > 0 ? (ctx + kTileKeys - 1) / kTileKeys : 0;
+    const int n_tiles = (key_end - key_begin + kTileKeys - 1) / kTileKeys;
 
     const int qrow = qt * 32 + r;                   // this lane's query of the sequence's block
     const bool row_ok = qrow < P.sq;
@@ -58,14 +92,14 @@ __global__ __launch_bounds__(64 * NW, 1) void paged_attn_f32_kernel(const PagedW
     load_q<T, D>(q, row_ok ? static_cast<const T*>(P.q) + (int64_t)b * P.q_sb + (int64_t)qrow * P.q_ss + (int64_t)head * P.q_sh : nullptr, H, width);
     State<D> st;
     st.init();
-    for (int t0 = 0; t0 < n_tiles; t0 += NW) {
-        __syncthreads();                                       // the previous tiles have been read by everybody
-        // ---- tiles t0 .. t0 + NW - 1 into LDS, all threads on each (a tile never straddles a page: page_size % 32 == 0) ----
+    for (int t0 = 0; t0 < n_tiles; t0 += KW) {
+        if (t0) __syncthreads();                               // the previous tiles have been read by everybody
+        // ---- tiles t0 .. t0 + KW - 1 into LDS, all threads on each (a tile never straddles a page: page_size % 32 == 0) ----
         unsigned tile_ok = 0;                                  // bit i: tile t0 + i exists and lies on a valid page (uniform)
 #pragma unroll
-        for (int i = 0; i < NW; ++i) {
-            const int key0 = (t0 + i) * kTileKeys;
-            if (key0 >= ctx) break;
+        for (int i = 0; i < KW; ++i) {
+            const int key0 = key_begin + (t0 + i) * kTileKeys;
+            if (key0 >= key_end) break;
             const int64_t page = bt[key0 / P.page_size];
             if (page < 0 || page >= P.num_pages) continue;
             tile_ok |= 1u << i;
@@ -74,24 +108,27 @@ __global__ __launch_bounds__(64 * NW, 1) void paged_attn_f32_kernel(const PagedW
             for (int p = 0; p < kTileKeys * (D / 4) / kThreads; ++p) {
                 const int u = tid + kThreads * p;
                 const int row = u / (D / 4), c4 = u % (D / 4);
-                const bool real = key0 + row < ctx && 4 * c4 < width;
+                const bool real = key0 + row < key_end && 4 * c4 < width;
                 const int64_t off = base + (int64_t)row * P.c_st + 4 * c4;
                 stage4<T, D>(lds + i * kTileFloats, row, c4, real ? kc + off : nullptr, real ? vc + off : nullptr);
             }
         }
         __syncthreads();
-        if ((tile_ok >> wave) & 1u) {
-            const int key0 = (t0 + wave) * kTileKeys;
-            tile_step<D>(lds + wave * kTileFloats, q, st, P.c, width, lane, [&](int key) { return key0 + key < ctx; });
+        if ((tile_ok >> kw) & 1u) {
+            const int key0 = key_begin + (t0 + kw) * kTileKeys;
+            tile_step<D>(lds + kw * kTileFloats, q, st, P.c, width, lane, [&](int key) { return key0 + key < key_end; });
         }
     }
 
-    // ---- merge the NW states through LDS: every wavefront folds, and stores, the column tiles dt = wave, wave + NW, ... ----
+    // ---- merge the KW states of a head through LDS: each of its wavefronts folds, and stores, every KW-th column tile ----
     constexpr int kStateFloats = (D / 32) * 16 * 64 + 2 * 64;                  // O as [dt][register][lane], then m, l
-    static_assert(NW * kStateFloats <= NW * kTileFloats, "merge buffer exceeds the tile region");
+    static_assert(HPW * KW * kStateFloats <= KW * kTileFloats, "merge buffer exceeds the tile region");
     st.l += __shfl_xor(st.l, 32);                                              // a state is now (m, l, O) per query
-    __syncthreads();                                                           // the last tiles have been read by everybody
-    {
+    float w[KW];
+    float M = st.m, l_all = st.l;
+    const float* states = lds + hw * KW * kStateFloats;
+    if (KW > 1) {
+        __syncthreads();                                                       // the last tiles have been read by everybody
         float* dst = lds + wave * kStateFloats;
 #pragma unroll
         for (int dt = 0; dt < D / 32; ++dt)
@@ -99,57 +136,145 @@ __global__ __launch_bounds__(64 * NW, 1) void paged_attn_f32_kernel(const PagedW
             for (int i = 0; i < 16; ++i) dst[(dt * 16 + i) * 64 + lane] = st.o[dt][i];
         dst[(D / 32) * 16 * 64 + lane] = st.m;
         dst[(D / 32) * 16 * 64 + 64 + lane] = st.l;
-    }
-    __syncthreads();
-    float w[NW];
-    float M = kMinusBig, l_all = 0.f;
+        __syncthreads();
+        M = kMinusBig;
+        l_all = 0.f;
 #pragma unroll
-    for (int s = 0; s < NW; ++s) { w[s] = lds[s * kStateFloats + (D / 32) * 16 * 64 + lane]; M = fmaxf(M, w[s]); }
+        for (int s = 0; s < KW; ++s) { w[s] = states[s * kStateFloats + (D / 32) * 16 * 64 + lane]; M = fmaxf(M, w[s]); }
 #pragma unroll
-    for (int s = 0; s < NW; ++s) {
-        w[s] = __builtin_amdgcn_exp2f(w[s] - M);
-        l_all += lds[s * kStateFloats + (D / 32) * 16 * 64 + 64 + lane] * w[s];
+        for (int s = 0; s < KW; ++s) {
+            w[s] = __builtin_amdgcn_exp2f(w[s] - M);
+            l_all += states[s * kStateFloats + (D / 32) * 16 * 64 + 64 + lane] * w[s];
+        }
     }
     if (!row_ok) return;
     const float inv = l_all > 0.f ? 1.0f / l_all : 0.f;                        // no key at all: zeros
     T* orow = static_cast<T*>(P.o) + (int64_t)b * P.o_sb + (int64_t)qrow * P.o_ss + (int64_t)head * P.o_sh;
+    const int64_t slot = (((int64_t)b * P.num_q_heads + head) * P.nqt + qt) * P.nsplit + split;
+    float* prow = P.part_o + (slot * 32 + r) * D;
 #pragma unroll
     for (int dt = 0; dt < D / 32; ++dt) {
-        if (dt % NW != wave || dt * 32 >= width) continue;                     // (uniform per wavefront)
+        if (dt % KW != kw || dt * 32 >= width) continue;                       // (uniform per wavefront)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int s = 0; s < NW; ++s)
+            for (int e = 0; e < 4; ++e) {
+                if (KW == 1) acc[e] = st.o[dt][4 * g + e];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) acc[e] += lds[s * kStateFloats + (dt * 16 + 4 * g + e) * 64 + lane] * w[s];
+                for (int s = 0; KW > 1 && s < KW; ++s) acc[e] += states[s * kStateFloats + (dt * 16 + 4 * g + e) * 64 + lane] * w[s];
+            }
             const int d = dt * 32 + 8 * g + 4 * H;
-            if (d < width) store4(orow + d, f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv});
+            if (d >= width) continue;
+            if (n_pieces == 1) store4(orow + d, f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv});
+            else *reinterpret_cast<f32x4*>(prow + d) = acc;
         }
+    }
+    if (n_pieces > 1 && kw == 0 && H == 0) {
+        P.part_ml[(slot * 2 + 0) * 32 + r] = M;
+        P.part_ml[(slot * 2 + 1) * 32 + r] = l_all;
     }
 }
 
+// Folds the pieces of a sequence: grid (head x query tile x 4, sequence), a thread takes four columns of one of the eight
+// queries of a quarter tile, eight pieces' loads in flight at a time.
 template <typename T, int D>
-int launch(const PagedWideParams& P, int bs, int num_q_heads, hipStream_t stream)
+__global__ __launch_bounds__(2 * D) void paged_combine_f32_kernel(const PagedWideParams P)
 {
-    constexpr int NW = D <= 128 ? 4 : 2;            // tiles of 32 keys that fit in LDS side by side
-    constexpr int kLdsBytes = NW * Lds<D>::kBytes;
+    const int quarter = blockIdx.x & 3, hq = blockIdx.x >> 2, b = blockIdx.y;
+    const int qt = hq % P.nqt, head = hq / P.nqt;
+    const int s = quarter * 8 + threadIdx.x / (D / 4), d = threadIdx.x % (D / 4) * 4;
+    const int ctx = keys_of(P, b);
+    const int span = keys_per_piece(P, ctx, threadIdx.x & 63);
+    const int n = (ctx + span - 1) / span;
+    const int qrow = qt * 32 + s;
+    if (n <= 1 || qrow >= P.sq || d >= P.head_dim) return;      // one piece: written by the attention kernel
+    const int64_t slot0 = (((int64_t)b * P.num_q_heads + head) * P.nqt + qt) * P.nsplit;
+    float M = kMinusBig, L = 0.f;
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i0 = 0; i0 < n; i0 += 8) {
+        float m[8], l[8];
+        f32x4 po[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int64_t slot = slot0 + min(i0 + i, n - 1);
+            m[i] = i0 + i < n ? P.part_ml[(slot * 2 + 0) * 32 + s] : kMinusBig;
+            l[i] = P.part_ml[(slot * 2 + 1) * 32 + s];
+            po[i] = *reinterpret_cast<const f32x4*>(P.part_o + (slot * 32 + s) * D + d);
+        }
+        float Mn = M;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) Mn = fmaxf(Mn, m[i]);
+        const float keep = __builtin_amdgcn_exp2f(M - Mn);
+        L *= keep;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] *= keep;
+        M = Mn;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float w = i0 + i < n ? __builtin_amdgcn_exp2f(m[i] - M) : 0.f;
+            L += w * l[i];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] += w * po[i][e];
+        }
+    }
+    const float inv = L > 0.f ? 1.0f / L : 0.f;                 // every key on an invalid page: zeros
+    store4(static_cast<T*>(P.o) + (int64_t)b * P.o_sb + (int64_t)qrow * P.o_ss + (int64_t)head * P.o_sh + d,
+           f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv});
+}
+
+int64_t slot_bytes(int head_dim) { return 32 * ((head_dim > 128 ? 256 : 128) + 2) * (int64_t)sizeof(float); }
+
+// Partial slots per sequence: pieces of at least kLeastKeys keys, and no more than fill the chip about four times over (2048
+// slots of one head: 34 MB of partials at most, and pieces enough for the ragged end of a launch to be short).
+int splits_wanted(int64_t bs, int nqt, int num_q_heads, int64_t max_keys) {
+    int64_t n = 2048 / (bs * num_q_heads * nqt);
+    if (n > (max_keys + kLeastKeys - 1) / kLeastKeys) n = (max_keys + kLeastKeys - 1) / kLeastKeys;
+    if (n > kMaxSplits) n = kMaxSplits;
+    return n < 1 ? 1 : (int)n;
+}
+
+template <typename T, int D, int HPW, int KW>
+int launch_groups(const PagedWideParams& P, hipStream_t stream)
+{
+    constexpr int kLdsBytes = KW * Lds<D>::kBytes;
     // the kernel's LDS limit is raised once per device
     static std::atomic<bool> raised[64];
     int device = 0;
     hipError_t e = hipGetDevice(&device);
     MDX_REQUIRE(e == hipSuccess && device >= 0 && device < 64, MDX_ELAUNCH, "paged_block_attn: no current device (%s)", hipGetErrorString(e));
     if (!raised[device].load(std::memory_order_acquire)) {
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(paged_attn_f32_kernel<T, D, NW>), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+        e = hipFuncSetAttribute(reinterpret_cast<const void*>(paged_attn_f32_kernel<T, D, HPW, KW>), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
         MDX_REQUIRE(e == hipSuccess, MDX_ELAUNCH, "paged_block_attn: cannot reserve %d bytes of LDS (%s)", kLdsBytes, hipGetErrorString(e));
         raised[device].store(true, std::memory_order_release);
     }
-    const dim3 grid((unsigned)num_q_heads, (unsigned)((P.sq + 31) / 32), (unsigned)bs);
-    paged_attn_f32_kernel<T, D, NW><<<grid, 64 * NW, kLdsBytes, stream>>>(P);
-    return mdx::check_launch("paged_block_attn (fp32 arithmetic)");
+    const dim3 grid((unsigned)(P.num_q_heads / HPW * P.nqt), (unsigned)P.nsplit, (unsigned)P.bs);
+    paged_attn_f32_kernel<T, D, HPW, KW><<<grid, 64 * HPW * KW, kLdsBytes, stream>>>(P);
+    const int rc = mdx::check_launch("paged_block_attn (fp32 arithmetic)");
+    if (rc != MDX_OK || P.nsplit == 1) return rc;
+    paged_combine_f32_kernel<T, D><<<dim3((unsigned)(P.num_q_heads * P.nqt * 4), (unsigned)P.bs), 2 * D, 0, stream>>>(P);
+    return mdx::check_launch("paged_combine (fp32 arithmetic)");
+}
+
+// KW: tiles of 32 keys staged side by side, two workgroups' worth of LDS per CU.
+template <typename T>
+int launch(const PagedWideParams& P, hipStream_t stream)
+{
+    const bool pairs = P.heads_per_kv % 2 == 0;
+    if (P.head_dim <= 128) return pairs ? launch_groups<T, 128, 2, 2>(P, stream) : launch_groups<T, 128, 1, 2>(P, stream);
+    return pairs ? launch_groups<T, 256, 2, 1>(P, stream) : launch_groups<T, 256, 1, 1>(P, stream);
 }
 
 }  // namespace
+
+extern "C" int64_t mdx_paged_block_attn_f32_workspace_bytes(int32_t bs, int32_t sq, int32_t num_q_heads, int32_t head_dim,
+                                                            int32_t max_pages, int32_t page_size)
+{
+    if (bs <= 0 || sq <= 0 || num_q_heads <= 0 || head_dim <= 0 || max_pages <= 0 || page_size <= 0) return 0;
+    const int nqt = (sq + 31) / 32;
+    const int n = splits_wanted(bs, nqt, num_q_heads, (int64_t)max_pages * page_size);
+    return n <= 1 ? 0 : (int64_t)bs * num_q_heads * nqt * n * slot_bytes(head_dim);
+}
 
 namespace mdx {
 
@@ -162,7 +287,7 @@ int launch_paged_f32(const void* q, void* o, const void* k_cache, const void* v_
                      const int32_t* block_table, int64_t bt_stride, const int32_t* context_lens,
                      int32_t bs, int32_t sq, int32_t num_q_heads, int32_t num_kv_heads,
                      int32_t head_dim, int32_t max_pages, int32_t page_size, int64_t num_pages,
-                     float scale, int32_t dtype, hipStream_t stream)
+                     float scale, int32_t dtype, void* workspace, int64_t workspace_bytes, hipStream_t stream)
 {
     MDX_REQUIRE(head_dim >= 4 && head_dim <= 256 && head_dim % 4 == 0, MDX_EUNSUPPORTED,
                 "paged_block_attn: head_dim %d (fp32 arithmetic: multiples of 4 up to 256)", head_dim);
@@ -179,14 +304,23 @@ int launch_paged_f32(const void* q, void* o, const void* k_cache, const void* v_
     P.o_sb = o_stride_b; P.o_ss = o_stride_s; P.o_sh = o_stride_h;
     P.c_sp = cache_stride_page; P.c_st = cache_stride_tok; P.c_sh = cache_stride_head;
     P.block_table = block_table; P.bt_stride = bt_stride; P.context_lens = context_lens;
-    P.sq = sq; P.heads_per_kv = num_q_heads / num_kv_heads; P.page_size = page_size; P.max_pages = max_pages; P.head_dim = head_dim;
+    P.bs = bs; P.sq = sq; P.nqt = (sq + 31) / 32;
+    P.num_q_heads = num_q_heads; P.heads_per_kv = num_q_heads / num_kv_heads;
+    P.page_size = page_size; P.max_pages = max_pages; P.head_dim = head_dim;
     P.num_pages = num_pages;
     P.c = scale * kLog2e;
-    const bool wide = head_dim > 128;
+    // as many partial slots as the launch wants and the caller's workspace holds; none: whole contexts
+    const int64_t n_rows = (int64_t)bs * num_q_heads * P.nqt, room = workspace && mdx::aligned16(workspace) ? workspace_bytes / (n_rows * slot_bytes(head_dim)) : 0;
+    P.nsplit = splits_wanted(bs, P.nqt, num_q_heads, (int64_t)max_pages * page_size);
+    if (P.nsplit > room) P.nsplit = room > 1 ? (int)room : 1;
+    const int groups = num_q_heads / (P.heads_per_kv % 2 == 0 ? 2 : 1) * P.nqt;
+    P.pieces = 1024 / groups > 0 ? 1024 / groups : 1;          // two pieces for each of the two workgroups that a CU holds
+    P.part_o = static_cast<float*>(workspace);
+    P.part_ml = P.nsplit > 1 ? P.part_o + n_rows * P.nsplit * 32 * (head_dim > 128 ? 256 : 128) : nullptr;
     switch (dtype) {
-    case MDX_F32:  return wide ? launch<float, 256>(P, bs, num_q_heads, stream) : launch<float, 128>(P, bs, num_q_heads, stream);
-    case MDX_F16:  return wide ? launch<_Float16, 256>(P, bs, num_q_heads, stream) : launch<_Float16, 128>(P, bs, num_q_heads, stream);
-    case MDX_BF16: return wide ? launch<__bf16, 256>(P, bs, num_q_heads, stream) : launch<__bf16, 128>(P, bs, num_q_heads, stream);
+    case MDX_F32:  return launch<float>(P, stream);
+    case MDX_F16:  return launch<_Float16>(P, stream);
+    case MDX_BF16: return launch<__bf16>(P, stream);
     }
     return mdx::fail(MDX_EUNSUPPORTED, "paged_block_attn: dtype %d", dtype);
 }

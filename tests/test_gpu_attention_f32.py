@@ -256,3 +256,26 @@ def test_fp32_sequence_bounds_are_clipped_to_the_tensors(dev):
     torch.cuda.synchronize()
     ref = oracle.staircase_attn_varlen(q[:120], k[:120], v[:120], torch.tensor([0, 120], dtype=torch.int32), 32)
     assert (o[:60].cpu() - ref[:60]).abs().max().item() < TOL_F32
+
+
+@pytest.mark.parametrize("ctxs", [[63, 64, 65, 127, 129], [3000] + [40] * 9, [70] * 70])
+@pytest.mark.parametrize("room", [0.0, 0.4, 1.0])
+def test_paged_fp32_contexts_cut_into_pieces(dev, ctxs, room):
+    """Lengths around the edge of a piece of 64 keys, one sequence far longer than the rest, and more sequences than a
+    wavefront has lanes; with no workspace, one that holds some of the pieces, and all of it."""
+    import mdx
+    g = torch.Generator().manual_seed(len(ctxs))
+    hq, hkv, d, page = 4, 2, 128, 64
+    q, kc, vc, bt, lens = (t.to(dev) for t in _paged_inputs(g, ctxs, 32, hq, hkv, d, torch.float32, page=page, pool=160))
+    L, scale, o = mdx.lib(), 1 / math.sqrt(d), torch.empty_like(q)
+    full = L.mdx_paged_block_attn_f32_workspace_bytes(len(ctxs), 32, hq, d, bt.shape[1], page)
+    assert full > 0
+    n_bytes = int(full * room) // 16 * 16
+    ws = torch.empty(n_bytes + 64, dtype=torch.uint8, device=dev).fill_(255)          # NaN everywhere; the last 64 bytes are not offered
+    rc = L.mdx_paged_block_attn(q.data_ptr(), o.data_ptr(), kc.data_ptr(), vc.data_ptr(), *q.stride()[:3], *o.stride()[:3], *kc.stride()[:3],
+                                bt.data_ptr(), bt.stride(0), lens.data_ptr(), len(ctxs), 32, hq, hkv, d, bt.shape[1], page, kc.shape[0],
+                                scale, 2, ws.data_ptr() if n_bytes else None, n_bytes, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    ref = oracle.paged_block_attn(q.cpu(), kc.cpu(), vc.cpu(), bt.cpu(), lens.cpu(), scale)
+    assert (o.cpu() - ref).abs().max().item() < TOL_F32
+    assert (ws[n_bytes:] == 255).all()
