@@ -342,6 +342,22 @@ int mdx_filter_logits(const void* logits, int64_t row_stride, int32_t dtype,
                       int64_t rows, int64_t vocab, mdx_stream_t stream);
 
 /*
+ * mdx_filter_logits followed by mdx_unmask_step or mdx_unmask_step_gumbel on its result, without the filtered copy -- the
+ * HF variant's sampling call (mineru_diffusion/modeling_mineru_diffusion.py:602-615 behind :585-600) and selection
+ * (:518-532) as one call.  Arguments as there; noise (NULL = none) and a seed (seeded != 0) exclude each other.  The
+ * workspace (16-byte aligned, contents need no initialisation) holds candidate lists or row cut-offs.
+ */
+int64_t mdx_unmask_step_filtered_workspace_bytes(int64_t rows, int64_t vocab, int32_t top_k);
+int mdx_unmask_step_filtered(const void* logits, int64_t row_stride, int32_t dtype,
+                             const float* temperatures, int32_t top_k, float top_p,
+                             const float* noise, int64_t noise_row_stride,
+                             int32_t seeded, uint64_t seed, uint64_t offset, const int64_t* offset_dev,
+                             int64_t* tokens, int64_t mask_token_id, float threshold, int32_t k,
+                             int64_t* x0, float* x0_p, uint8_t* transfer, int32_t* count,
+                             int32_t bs, int32_t block_len, int64_t vocab,
+                             void* workspace, int64_t workspace_bytes, mdx_stream_t stream);
+
+/*
  * Fused producer of the attention inputs for one decoder layer: per-head RMSNorm of q and k,
  * rotary embedding, and the KV-cache store, in one pass over the fused QKV projection output --
  * replaces the chain q_norm / k_norm / rotary_emb / store_kvcache of

@@ -591,12 +591,23 @@ PyObject* select_transfer(PyObject*, PyObject* const* a, Py_ssize_t n) {
     });
 }
 
+struct Filter { int64_t top_k; double top_p; bool on() const { return top_k > 0 || top_p < 1.0; } };
+
 void step(const Tensor& logits, int64_t bs, int64_t S, int64_t* tokens, int64_t mask_id, float threshold, int32_t k, const Tensor& temps,
-          const Noise& z, int64_t* x0, float* x0_p, uint8_t* transfer, int32_t* count) {
+          const Filter& f, const Noise& z, int64_t* x0, float* x0_p, uint8_t* transfer, int32_t* count) {
     const Logits l = logits_of(logits);
     NEED(l.rows == bs * S);
     const Tensor t = temperatures_of(temps);
     if (t.defined()) NEED(t.numel() == bs);
+    if (f.on()) {
+        const int64_t bytes = mdx_unmask_step_filtered_workspace_bytes(l.rows, l.vocab, (int32_t)f.top_k);
+        const Tensor ws = make(logits, at::kByte, bytes);
+        check(mdx_unmask_step_filtered(ptr(l.t), l.stride, dtype_of(logits), static_cast<const float*>(ptr_or_null(t)), (int32_t)f.top_k, (float)f.top_p,
+                                       z.data(), z.data() ? l.vocab : 0, z.seeded ? 1 : 0, z.seed, z.offset,
+                                       static_cast<const int64_t*>(ptr_or_null(z.offset_dev)), tokens, mask_id, threshold, k, x0, x0_p, transfer, count,
+                                       (int32_t)bs, (int32_t)S, l.vocab, ptr(ws), bytes, stream_of(logits)), "unmask_step");
+        return;
+    }
     const int64_t bytes = mdx_confidence_argmax_workspace_bytes(l.rows, l.vocab);
     const Tensor ws = bytes > 0 ? make(logits, at::kByte, bytes) : Tensor();
     const float* tp = static_cast<const float*>(ptr_or_null(t));
@@ -613,20 +624,16 @@ void step(const Tensor& logits, int64_t bs, int64_t S, int64_t* tokens, int64_t 
 PyObject* unmask_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
     ARGS(13);
     return guarded([&]() -> PyObject* {
-        Tensor logits = tensor(a[0]);
-        const Tensor &tokens = tensor(a[1]), &temps = optional_tensor(a[5]);
+        const Tensor &logits = tensor(a[0]), &tokens = tensor(a[1]), &temps = optional_tensor(a[5]);
         need_gpu({&logits, &tokens, &temps, &optional_tensor(a[8])});
-        const int64_t top_k = integer(a[6]);
-        const double top_p = real(a[7]);
-        if (optional_tensor(a[8]).defined() && a[9] != Py_None) raise_assert("either a noise tensor or a seed");
-        if (top_k > 0 || top_p < 1.0) logits = filter(logits, top_k, top_p, temps, Tensor());
+        const Filter f{integer(a[6]), real(a[7])};
         NEED(tokens.scalar_type() == at::kLong && tokens.is_contiguous() && tokens.dim() == 2);
         const int64_t bs = tokens.size(0), S = tokens.size(1), vocab = logits.size(-1);
         NEED(logits.numel() == bs * S * vocab);
         Noise z = noise_of(a + 8, bs * S, vocab);
         Tensor x0 = make(tokens, at::kLong, bs, S), x0_p = make(tokens, at::kFloat, bs, S);
         Tensor transfer = make(tokens, at::kBool, bs, S), count = make(tokens, at::kInt, bs);
-        step(logits, bs, S, static_cast<int64_t*>(ptr(tokens)), integer(a[2]), (float)real(a[3]), (int32_t)integer(a[4]), temps, z,
+        step(logits, bs, S, static_cast<int64_t*>(ptr(tokens)), integer(a[2]), (float)real(a[3]), (int32_t)integer(a[4]), temps, f, z,
              static_cast<int64_t*>(ptr(x0)), static_cast<float*>(ptr(x0_p)), static_cast<uint8_t*>(ptr(transfer)), static_cast<int32_t*>(ptr(count)));
         return wrap_tuple(std::move(x0), std::move(x0_p), std::move(transfer), std::move(count));
     });
@@ -660,7 +667,7 @@ PyObject* sampler_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
         }
         const Noise z = noise_of(a + 8, bs * S, vocab);
         Tensor x0 = make(logits, at::kLong, bs, S), x0_p = make(logits, at::kFloat, bs, S);
-        step(logits, bs, S, reinterpret_cast<int64_t*>(host), integer(a[5]), (float)real(a[6]), (int32_t)integer(a[7]), temps, z,
+        step(logits, bs, S, reinterpret_cast<int64_t*>(host), integer(a[5]), (float)real(a[6]), (int32_t)integer(a[7]), temps, Filter{0, 1.0}, z,
              static_cast<int64_t*>(ptr(x0)), static_cast<float*>(ptr(x0_p)), reinterpret_cast<uint8_t*>(host + flags_at),
              reinterpret_cast<int32_t*>(host + counts_at));
         hipError_t rc;

@@ -13,9 +13,13 @@
 // Semantics follow engines/nano_dvlm/nanovllm/layers/sampler.py:11-61 and
 // mineru_diffusion/modeling_mineru_diffusion.py:518-532.
 #include "mdx_common.h"
+#include "gumbel_noise.h"
+#include "filtered_pick.h"
 #include <hip/hip_fp16.h>
 
 namespace {
+
+using namespace mdx_noise;
 
 constexpr int kThreads = 256;
 constexpr int kUnroll = 2;               // 16-byte loads in flight per lane
@@ -140,72 +144,15 @@ __device__ __forceinline__ void visit(Partial& p, float x, int index, float c, f
     }
 }
 
-// --- Gumbel noise drawn in the kernel ------------------------------------------------------------
-// Sampler.prepare draws gumbel = -log(Exponential(1)) per logit (sampler.py:15-16).  Here the draw is
-// a pure function of (seed, offset, row, column): Philox-4x32-10 (Salmon et al., "Parallel random
-// numbers: as easy as 1, 2, 3", 2011) with key = seed and counter = (column / 4, row, offset), whose
-// four 32-bit outputs serve columns 4*(column/4) .. +3.  So the noise does not depend on the launch
-// geometry, a caller reproduces a step from three integers, and nothing is read from memory.
-struct NoiseSpec {
-    const float* noise; int64_t noise_row_stride;      // explicit noise tensor, or
-    bool philox; uint32_t key0, key1;                   // noise from the generator: seed,
-    uint64_t offset; const int64_t* offset_dev;         // offset (+ *offset_dev when given: a counter a graph replay can advance),
-    const int64_t* row_ids;                             // and the row coordinate of each logits row (NULL: the row's own index)
-};
-
-struct U4 { uint32_t x, y, z, w; };
-
-__device__ __forceinline__ U4 philox4x32_10(U4 c, uint32_t k0, uint32_t k1) {
-#pragma unroll
-    for (int r = 0; r < 10; ++r) {
-        // one 32 x 32 -> 64 multiply per product (v_mad_u64_u32) instead of a high and a low one: 32-bit integer
-        // multiplies are what this generator costs, and the full-width form is 6.5 % faster over a logits pass
-        const uint64_t p0 = (uint64_t)0xD2511F53u * (uint64_t)c.x, p1 = (uint64_t)0xCD9E8D57u * (uint64_t)c.z;
-        const uint32_t hi0 = (uint32_t)(p0 >> 32), lo0 = (uint32_t)p0, hi1 = (uint32_t)(p1 >> 32), lo1 = (uint32_t)p1;
-        c = U4{hi1 ^ c.y ^ k0, lo1, hi0 ^ c.w ^ k1, lo0};
-        k0 += 0x9E3779B9u;
-        k1 += 0xBB67AE85u;
-    }
-    return c;
-}
-
-// 32 random bits -> u = (top 23 bits + 1/2) / 2^23 in (0, 1) -> -ln(-ln u), the negated logarithm of a unit
-// exponential.  With t = log2 u: -ln(-ln u) = -ln 2 * log2(-t) - ln(ln 2).  The largest noise values, the ones
-// that decide an argmax, come from u next to 1, where t is tiny: the hardware logarithm keeps its relative
-// accuracy there (over all 2^23 values of u the result is within 2e-6 of the fp64 one).
-constexpr float kGumbelMax = 17.0f;      // above every value of gumbel_of (16.64 at u = 1 - 2^-24)
-__device__ __forceinline__ float gumbel_of(uint32_t bits) {
-    const float u = __builtin_fmaf((float)(bits >> 9), 1.1920928955078125e-07f, 5.9604644775390625e-08f);   // (k + 1/2) * 2^-23
-    const float t = __builtin_amdgcn_logf(u);
-    return __builtin_fmaf(-0.69314718055994531f, __builtin_amdgcn_logf(-t), 0.36651292058166435f);
-}
-
-struct RowNoise {                       // the generator's coordinates of one logits row
-    uint32_t key0, key1, row, off_lo, off_hi;
-    __device__ __forceinline__ U4 group(uint32_t column_group) const {
-        return philox4x32_10(U4{column_group, row, off_lo, off_hi}, key0, key1);
-    }
-    __device__ __forceinline__ float at(int column) const {
-        const U4 r = group((uint32_t)column >> 2);
-        const uint32_t b[4] = {r.x, r.y, r.z, r.w};
-        return gumbel_of(b[column & 3]);
-    }
-};
-
-__device__ __forceinline__ RowNoise row_noise(const NoiseSpec& N, int64_t row) {
-    const uint64_t off = N.offset + (N.offset_dev ? (uint64_t)*N.offset_dev : 0ull);
-    const int64_t rid = N.row_ids ? N.row_ids[row] : row;
-    return RowNoise{N.key0, N.key1, (uint32_t)rid, (uint32_t)off, (uint32_t)(off >> 32)};
-}
-
 // grid = (rows, nsplit).  Each workgroup reduces chunks [split*cps, (split+1)*cps)
 // of one row; split 0 also takes the unaligned head and tail elements.
 // NOISE: 0 = plain argmax, 1 = noise read from a tensor, 2 = noise drawn in the kernel.
-template <typename T, int NOISE>
+// FLOOR: elements below floors[row] count as -inf (what a top-k / top-p filter would have left of the row).
+template <typename T, int NOISE, bool FLOOR>
 __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
     const T* __restrict__ logits, int64_t row_stride,
     const float* __restrict__ temperatures, int rows_per_temp,
-    const NoiseSpec N,
+    const NoiseSpec N, const float* __restrict__ floors,
     int64_t vocab, int nsplit,
     Partial* __restrict__ partials,          // [rows, nsplit] when nsplit > 1
     int64_t* __restrict__ x0, float* __restrict__ x0_p)
@@ -218,6 +165,16 @@ __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
     const float* np = NOISE == 1 ? N.noise + row * N.noise_row_stride : nullptr;
     const float T_ = temperatures ? temperatures[row / rows_per_temp] : 1.0f;
     const float c = kLog2e / T_;
+    const float floor = FLOOR ? floors[row] : 0.f;
+    auto unpack = [&](const u32x4& u, float (&x)[Elem<T>::EPC]) {
+        Elem<T>::unpack(u, x);
+#pragma unroll
+        for (int i = 0; FLOOR && i < Elem<T>::EPC; ++i) x[i] = x[i] >= floor ? x[i] : -INFINITY;
+    };
+    auto one = [&](int64_t e) {
+        const float x = Elem<T>::one(rp + e);
+        return !FLOOR || x >= floor ? x : -INFINITY;
+    };
 
     // Row geometry: `lead` scalar elements up to the first 16-byte boundary,
     // `nchunk` aligned chunks, then a scalar tail.
@@ -281,7 +238,7 @@ __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
     if (NOISE == 0) {
         auto take = [&](const u32x4 u, int64_t chunk) {
             float x[EPC];
-            Elem<T>::unpack(u, x);
+            unpack(u, x);
             take_values(x, chunk);
         };
         int64_t ch = cbeg + tid;
@@ -314,8 +271,8 @@ __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
         for (; ch < cend; ch += kThreads) take(__builtin_nontemporal_load(cp + ch), ch);
         lane_softmax_done();
         if (split == 0) {            // unaligned head and tail, a handful of elements
-            for (int64_t e = tid; e < lead; e += kThreads) visit<false>(p, Elem<T>::one(rp + e), (int)e, c, T_, 0.f);
-            for (int64_t e = tail0 + tid; e < vocab; e += kThreads) visit<false>(p, Elem<T>::one(rp + e), (int)e, c, T_, 0.f);
+            for (int64_t e = tid; e < lead; e += kThreads) visit<false>(p, one(e), (int)e, c, T_, 0.f);
+            for (int64_t e = tail0 + tid; e < vocab; e += kThreads) visit<false>(p, one(e), (int)e, c, T_, 0.f);
         }
     } else {
         // With noise.  The softmax runs over 16-byte chunks as without noise; the noisy argmax is element by
@@ -345,7 +302,7 @@ __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
             if (cbeg + tid + k * kThreads < cend) next[k] = __builtin_nontemporal_load(cp + cbeg + tid + k * kThreads);
         for (int64_t ch = cbeg + tid; ch < cend; ch += kThreads) {
             float x[EPC];
-            Elem<T>::unpack(next[0], x);
+            unpack(next[0], x);
 #pragma unroll
             for (int k = 0; k + 1 < kUnroll; ++k) next[k] = next[k + 1];
             if (ch + kUnroll * kThreads < cend) next[kUnroll - 1] = __builtin_nontemporal_load(cp + ch + kUnroll * kThreads);
@@ -424,8 +381,8 @@ __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
         lane_softmax_done();
         p.pick = best; p.pick_x = best_x; p.pick_idx = best_idx;
         if (split == 0) {
-            for (int64_t e = tid; e < lead; e += kThreads) visit<true>(p, Elem<T>::one(rp + e), (int)e, c, T_, noise_at(e));
-            for (int64_t e = tail0 + tid; e < vocab; e += kThreads) visit<true>(p, Elem<T>::one(rp + e), (int)e, c, T_, noise_at(e));
+            for (int64_t e = tid; e < lead; e += kThreads) visit<true>(p, one(e), (int)e, c, T_, noise_at(e));
+            for (int64_t e = tail0 + tid; e < vocab; e += kThreads) visit<true>(p, one(e), (int)e, c, T_, noise_at(e));
         }
     }
 
@@ -658,22 +615,19 @@ int pick_nsplit(int64_t rows, int64_t vocab) {
     return (int)n;
 }
 
-template <typename T>
+template <typename T, bool FLOOR>
 int launch_confidence(const void* logits, int64_t row_stride, const float* temperatures, int rows_per_temp,
-                      const NoiseSpec& N, int64_t* x0, float* x0_p,
+                      const NoiseSpec& N, const float* floors, int64_t* x0, float* x0_p,
                       int64_t rows, int64_t vocab, int nsplit, Partial* partials, bool finalize, hipStream_t stream)
 {
     const dim3 grid((unsigned)rows, (unsigned)nsplit);
     const bool noisy = N.noise != nullptr || N.philox;
-    if (N.philox)
-        confidence_argmax_kernel<T, 2><<<grid, kThreads, 0, stream>>>(
-            (const T*)logits, row_stride, temperatures, rows_per_temp, N, vocab, nsplit, partials, x0, x0_p);
-    else if (N.noise)
-        confidence_argmax_kernel<T, 1><<<grid, kThreads, 0, stream>>>(
-            (const T*)logits, row_stride, temperatures, rows_per_temp, N, vocab, nsplit, partials, x0, x0_p);
-    else
-        confidence_argmax_kernel<T, 0><<<grid, kThreads, 0, stream>>>(
-            (const T*)logits, row_stride, temperatures, rows_per_temp, N, vocab, nsplit, partials, x0, x0_p);
+#define MDX_CONFIDENCE(NOISE) confidence_argmax_kernel<T, NOISE, FLOOR><<<grid, kThreads, 0, stream>>>( \
+        (const T*)logits, row_stride, temperatures, rows_per_temp, N, floors, vocab, nsplit, partials, x0, x0_p)
+    if (N.philox)     MDX_CONFIDENCE(2);
+    else if (N.noise) MDX_CONFIDENCE(1);
+    else              MDX_CONFIDENCE(0);
+#undef MDX_CONFIDENCE
     int rc = mdx::check_launch("confidence_argmax");
     if (rc != MDX_OK || nsplit == 1 || !finalize) return rc;
     const unsigned fgrid = (unsigned)((rows + kThreads / kMergeLanes - 1) / (kThreads / kMergeLanes));
@@ -699,15 +653,6 @@ __global__ __launch_bounds__(kThreads) void gumbel_noise_kernel(float* __restric
         if (group * 4 + i < vocab) dst[i] = gumbel_of(b[i]);
 }
 
-NoiseSpec no_noise() { return NoiseSpec{nullptr, 0, false, 0, 0, 0, nullptr, nullptr}; }
-NoiseSpec tensor_noise(const float* noise, int64_t stride) { NoiseSpec n = no_noise(); n.noise = noise; n.noise_row_stride = stride; return n; }
-NoiseSpec generator_noise(uint64_t seed, uint64_t offset, const int64_t* offset_dev, const int64_t* row_ids) {
-    NoiseSpec n = no_noise();
-    n.philox = true; n.key0 = (uint32_t)seed; n.key1 = (uint32_t)(seed >> 32);
-    n.offset = offset; n.offset_dev = offset_dev; n.row_ids = row_ids;
-    return n;
-}
-
 }  // namespace
 
 extern "C" int64_t mdx_confidence_argmax_workspace_bytes(int64_t rows, int64_t vocab) {
@@ -720,7 +665,7 @@ namespace {
 
 int confidence_pass(const void* logits, int64_t row_stride, int32_t dtype,
                     const float* temperatures, int32_t rows_per_temp,
-                    const NoiseSpec& N,
+                    const NoiseSpec& N, const float* floors,
                     int64_t* x0, float* x0_p, int64_t rows, int64_t vocab,
                     void* workspace, int64_t workspace_bytes, bool finalize, int* nsplit_out, hipStream_t stream)
 {
@@ -742,12 +687,14 @@ int confidence_pass(const void* logits, int64_t row_stride, int32_t dtype,
     MDX_REQUIRE(need == 0 || (workspace && workspace_bytes >= need), MDX_EWORKSPACE,
                 "confidence_argmax: workspace of %lld bytes needed, %lld given", (long long)need, (long long)workspace_bytes);
     Partial* partials = static_cast<Partial*>(workspace);
+#define MDX_PASS(T, FLOOR) launch_confidence<T, FLOOR>(logits, row_stride, temperatures, rows_per_temp, N, floors, x0, x0_p, rows, vocab, nsplit, partials, finalize, stream)
     switch (dtype) {
-        case MDX_BF16: return launch_confidence<__bf16>(logits, row_stride, temperatures, rows_per_temp, N, x0, x0_p, rows, vocab, nsplit, partials, finalize, stream);
-        case MDX_F16:  return launch_confidence<__half>(logits, row_stride, temperatures, rows_per_temp, N, x0, x0_p, rows, vocab, nsplit, partials, finalize, stream);
-        case MDX_F32:  return launch_confidence<float>(logits, row_stride, temperatures, rows_per_temp, N, x0, x0_p, rows, vocab, nsplit, partials, finalize, stream);
+        case MDX_BF16: return floors ? MDX_PASS(__bf16, true) : MDX_PASS(__bf16, false);
+        case MDX_F16:  return floors ? MDX_PASS(__half, true) : MDX_PASS(__half, false);
+        case MDX_F32:  return MDX_PASS(float, false);                  // (filters take 16-bit logits only)
         default: return mdx::fail(MDX_EUNSUPPORTED, "confidence_argmax: dtype %d", dtype);
     }
+#undef MDX_PASS
 }
 
 }  // namespace
@@ -758,7 +705,7 @@ extern "C" int mdx_confidence_argmax(const void* logits, int64_t row_stride, int
                                      int64_t* x0, float* x0_p, int64_t rows, int64_t vocab,
                                      void* workspace, int64_t workspace_bytes, mdx_stream_t stream)
 {
-    return confidence_pass(logits, row_stride, dtype, temperatures, rows_per_temp, tensor_noise(noise, noise_row_stride), x0, x0_p,
+    return confidence_pass(logits, row_stride, dtype, temperatures, rows_per_temp, tensor_noise(noise, noise_row_stride), nullptr, x0, x0_p,
                            rows, vocab, workspace, workspace_bytes, true, nullptr, static_cast<hipStream_t>(stream));
 }
 
@@ -768,7 +715,7 @@ extern "C" int mdx_confidence_argmax_gumbel(const void* logits, int64_t row_stri
                                             int64_t* x0, float* x0_p, int64_t rows, int64_t vocab,
                                             void* workspace, int64_t workspace_bytes, mdx_stream_t stream)
 {
-    return confidence_pass(logits, row_stride, dtype, temperatures, rows_per_temp, generator_noise(seed, offset, offset_dev, row_ids),
+    return confidence_pass(logits, row_stride, dtype, temperatures, rows_per_temp, generator_noise(seed, offset, offset_dev, row_ids), nullptr,
                            x0, x0_p, rows, vocab, workspace, workspace_bytes, true, nullptr, static_cast<hipStream_t>(stream));
 }
 
@@ -820,14 +767,66 @@ int unmask_step_impl(const void* logits, int64_t row_stride, int32_t dtype,
     // The selection kernel merges the row splits itself (one launch fewer).
     const bool noisy = N.noise != nullptr || N.philox;
     int nsplit = 1;
-    int rc = confidence_pass(logits, row_stride, dtype, temperatures, block_len, N,
+    int rc = confidence_pass(logits, row_stride, dtype, temperatures, block_len, N, nullptr,
                              x0, x0_p, (int64_t)bs * block_len, vocab, workspace, workspace_bytes, false, &nsplit, stream);
     if (rc != MDX_OK) return rc;
     return launch_select(x0, x0_p, tokens, nsplit > 1 ? static_cast<const Partial*>(workspace) : nullptr, nsplit, noisy, temperatures,
                          mask_token_id, threshold, k, transfer, count, bs, block_len, stream);
 }
 
+// What a filtered step keeps in the caller's workspace: the row floors and the vocabulary pass's splits, or the candidates.
+int64_t filtered_workspace(int64_t rows, int64_t vocab, int top_k) {
+    const int64_t lists = mdx::filtered_pick_workspace_bytes(rows, vocab, top_k);
+    return lists > 0 ? lists : (rows * 4 + 15) / 16 * 16 + mdx_confidence_argmax_workspace_bytes(rows, vocab);
+}
+
 }  // namespace
+
+extern "C" int64_t mdx_unmask_step_filtered_workspace_bytes(int64_t rows, int64_t vocab, int32_t top_k)
+{
+    return rows <= 0 || vocab <= 0 ? 0 : filtered_workspace(rows, vocab, top_k);
+}
+
+extern "C" int mdx_unmask_step_filtered(const void* logits, int64_t row_stride, int32_t dtype,
+                                        const float* temperatures, int32_t top_k, float top_p,
+                                        const float* noise, int64_t noise_row_stride,
+                                        int32_t seeded, uint64_t seed, uint64_t offset, const int64_t* offset_dev,
+                                        int64_t* tokens, int64_t mask_token_id, float threshold, int32_t k,
+                                        int64_t* x0, float* x0_p, uint8_t* transfer, int32_t* count,
+                                        int32_t bs, int32_t block_len, int64_t vocab,
+                                        void* workspace, int64_t workspace_bytes, mdx_stream_t stream_)
+{
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    MDX_REQUIRE(bs >= 0 && block_len >= 0, MDX_EINVAL, "unmask_step: negative size");
+    MDX_REQUIRE(k >= 0, MDX_EINVAL, "unmask_step: k %d < 0", k);
+    MDX_REQUIRE(block_len <= kMaxBlockLen, MDX_EUNSUPPORTED, "unmask_step: block_len %d > %d", block_len, kMaxBlockLen);
+    const int64_t rows = (int64_t)bs * block_len;
+    int rc = mdx::check_filter(logits, row_stride, dtype, top_k, top_p, rows, vocab);
+    if (rc != MDX_OK || rows == 0) return rc;
+    MDX_REQUIRE(tokens && transfer && count && x0 && x0_p, MDX_EINVAL, "unmask_step: null pointer");
+    MDX_REQUIRE(!(noise && seeded), MDX_EINVAL, "unmask_step: either a noise tensor or a seed");
+    MDX_REQUIRE(!noise || noise_row_stride >= vocab, MDX_EINVAL, "unmask_step: noise_row_stride < vocab");
+    const int64_t need = filtered_workspace(rows, vocab, top_k);
+    MDX_REQUIRE(workspace && workspace_bytes >= need && mdx::aligned16(workspace), MDX_EWORKSPACE,
+                "unmask_step: workspace of %lld bytes needed (16-byte aligned), %lld given", (long long)need, (long long)workspace_bytes);
+    const NoiseSpec N = seeded ? generator_noise(seed, offset, offset_dev, nullptr) : tensor_noise(noise, noise_row_stride);
+    if (mdx::filtered_pick_workspace_bytes(rows, vocab, top_k) > 0) {
+        rc = mdx::filtered_pick(logits, row_stride, dtype, temperatures, block_len, top_k, top_p, N, x0, x0_p, rows, vocab, workspace, stream);
+        if (rc != MDX_OK) return rc;
+        return launch_select(x0, x0_p, tokens, nullptr, 1, false, nullptr, mask_token_id, threshold, k, transfer, count, bs, block_len, stream);
+    }
+    float* floors = static_cast<float*>(workspace);
+    rc = mdx::filter_floors(logits, row_stride, dtype, temperatures, block_len, top_k, top_p, floors, rows, vocab, stream);
+    if (rc != MDX_OK) return rc;
+    const int64_t at = (rows * 4 + 15) / 16 * 16;
+    void* splits = static_cast<char*>(workspace) + at;
+    int nsplit = 1;
+    rc = confidence_pass(logits, row_stride, dtype, temperatures, block_len, N, floors, x0, x0_p, rows, vocab, splits, workspace_bytes - at,
+                         false, &nsplit, stream);
+    if (rc != MDX_OK) return rc;
+    return launch_select(x0, x0_p, tokens, nsplit > 1 ? static_cast<const Partial*>(splits) : nullptr, nsplit, N.noise || N.philox, temperatures,
+                         mask_token_id, threshold, k, transfer, count, bs, block_len, stream);
+}
 
 extern "C" int mdx_unmask_step(const void* logits, int64_t row_stride, int32_t dtype,
                                const float* temperatures, const float* noise, int64_t noise_row_stride,

@@ -164,3 +164,35 @@ def test_unmask_step_with_filters(dev):
     assert np.array_equal(x0.cpu().numpy(), ex0)
     np.testing.assert_allclose(p.cpu().numpy(), ep, rtol=2e-5)
     assert np.array_equal(tr.cpu().numpy(), etr) and np.array_equal(d_tokens.cpu().numpy(), etok)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("V", [5, 33, 1000, 40961, 151936])
+@pytest.mark.parametrize("k,p", [(1, 1.0), (50, 0.9), (256, 0.7), (300, 0.95), (512, 1.0), (513, 0.9), (0, 0.8), (20, 0.0)])
+@pytest.mark.parametrize("noise", ["none", "seed", "tensor"])
+def test_filtered_step_is_the_filter_and_the_step(dev, dtype, V, k, p, noise):
+    """unmask_step(top_k, top_p), which never writes the filtered copy, against unmask_step on filter_logits' result: rows of
+    random logits, of few distinct values (more ties at the cut-off than a candidate list holds), constant, mostly -inf and all
+    -inf, starting on and off a 16-byte boundary."""
+    import mdx
+    g = torch.Generator(device=dev).manual_seed(V + k)
+    bs, S = 2, 6
+    for pad in (0, 3):
+        buf = (torch.randn(bs * S, V + pad, generator=g, device=dev) * 3).to(dtype)
+        buf[1] = (buf[1].float() / 4).round().to(dtype)
+        buf[2] = 1.5
+        buf[3, : V - min(V, 30)] = float("-inf")
+        buf[4] = float("-inf")
+        buf[5, ::2] = 0.0
+        buf[5, 1::2] = -0.0
+        logits = buf[:, :V].view(bs, S, V) if pad == 0 else buf[:, :V].unflatten(0, (bs, S))
+        temps = torch.tensor([0.7, 1.0], device=dev)
+        opts = dict(none={}, seed=dict(seed=77, offset=3),
+                    tensor=dict(noise=-torch.log(-torch.log(torch.rand(bs, S, V, generator=g, device=dev).clamp_(1e-9, 1 - 1e-6)))))[noise]
+        masks = torch.full((bs, S), 9, dtype=torch.int64, device=dev)
+        a, b = masks.clone(), masks.clone()
+        got = mdx.unmask_step(logits, a, 9, 0.9, 2, temperatures=temps, top_k=k, top_p=p, **opts)
+        want = mdx.unmask_step(mdx.filter_logits(logits, k, p, temps), b, 9, 0.9, 2, temperatures=temps, **opts)
+        assert torch.equal(got[0], want[0])
+        np.testing.assert_allclose(got[1].cpu().numpy(), want[1].cpu().numpy(), rtol=5e-6)
+        assert torch.equal(got[2], want[2]) and torch.equal(got[3], want[3]) and torch.equal(a, b)
