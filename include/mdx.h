@@ -411,6 +411,37 @@ int mdx_silu_and_mul(const void* x, int64_t x_row_stride, void* out, int64_t out
                      int64_t rows, int32_t intermediate, int32_t dtype, mdx_stream_t stream);
 
 /*
+ * Linear layers of a decode pass, x . w^T for few rows (nanovllm/layers/linear.py as called at nanovllm/models/sdar.py:73-112);
+ * x [rows, k], w [n, k], MDX_BF16, row strides in elements (multiples of 8), 16-byte aligned.
+ *
+ * mdx_decode_linear_partials leaves the product as fp32 partial sums over slices of K, partials [splits, rows, n] (dense),
+ * for one of the two kernels below that add them up and round the sum to bf16 as the layer's output; splits =
+ * mdx_decode_linear_splits(rows, n, k), 0 where the shape is not covered (rows up to 128, n a multiple of 64, k of 256).
+ * mdx_decode_linear_silu: w [2 n, k], gate rows then up rows; y [rows, n] = mdx_silu_and_mul of the product, with its
+ * rounding points (rows up to 64, n a multiple of 24, k of 512: mdx_decode_linear_silu_supported).
+ * mdx_add_rms_norm_partials and mdx_qk_norm_rope_store_partials are mdx_add_rms_norm and mdx_qk_norm_rope_store with
+ * x / qkv given as such partial sums ([splits, rows, hidden], [splits, n_tokens, (Hq + 2 Hkv) * d]).
+ */
+int32_t mdx_decode_linear_splits(int64_t rows, int64_t n, int64_t k);
+int mdx_decode_linear_partials(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride,
+                               float* partials, int64_t rows, int64_t n, int64_t k, mdx_stream_t stream);
+int32_t mdx_decode_linear_silu_supported(int64_t rows, int64_t n, int64_t k);
+int mdx_decode_linear_silu(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride,
+                           void* y, int64_t y_row_stride, int64_t rows, int64_t n, int64_t k, mdx_stream_t stream);
+int mdx_add_rms_norm_partials(const float* partials, int32_t splits,
+                              const void* residual_in, int64_t residual_in_row_stride,
+                              void* residual_out, int64_t residual_out_row_stride,
+                              const void* weight, float eps, void* out, int64_t out_row_stride,
+                              int64_t rows, int32_t hidden, int32_t dtype, mdx_stream_t stream);
+int mdx_qk_norm_rope_store_partials(const float* partials, int32_t splits,
+                                    const void* q_weight, const void* k_weight, float eps,
+                                    const float* cos_table, const float* sin_table, int64_t max_positions,
+                                    const int64_t* positions, void* q_out, int64_t q_out_row_stride,
+                                    void* k_cache, void* v_cache, const int32_t* slot_mapping, int64_t num_slots,
+                                    int64_t n_tokens, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                                    int32_t dtype, mdx_stream_t stream);
+
+/*
  * Denoising-block state kept on the device between decode passes (one entry per sequence of the
  * batch, "lane"): tokens [bs, block_len] int64 (the current block, mask_token_id where still masked),
  * lens [bs] (committed tokens), phase [bs] (MDX_PHASE_*), step [bs], step_map [bs, block_len].

@@ -21,6 +21,7 @@
 #include <mutex>
 #include <string>
 #include <utility>
+#include <vector>
 #include "../../include/mdx.h"
 
 namespace {
@@ -253,6 +254,93 @@ PyObject* silu_and_mul(PyObject*, PyObject* const* a, Py_ssize_t n) {
         Tensor out = at::empty(shape, at::TensorOptions().dtype(x.scalar_type()).device(x.device()));
         check(mdx_silu_and_mul(ptr(r.t), r.stride, ptr(out), inter, r.n, (int32_t)inter, dtype_of(x), stream_of(x)), "silu_and_mul");
         return wrap(std::move(out));
+    });
+}
+
+// ---- linear layers of a decode pass -----------------------------------------------------------------
+// x [.., k], w [n, k] -> fp32 partial sums [splits, .., n], or None where the shape is not covered
+PyObject* linear_partials(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    ARGS(2);
+    return guarded([&]() -> PyObject* {
+        const Tensor &x = tensor(a[0]), &w = tensor(a[1]);
+        need_gpu({&x, &w});
+        NEED(x.dim() >= 2 && w.dim() == 2 && x.size(-1) == w.size(1));
+        const int64_t k = w.size(1), cols = w.size(0), rows = k ? x.numel() / k : 0;
+        const int32_t splits = mdx_decode_linear_splits(rows, cols, k);
+        if (splits == 0 || x.scalar_type() != at::kBFloat16 || w.scalar_type() != at::kBFloat16 || x.stride(-1) != 1 || w.stride(1) != 1) Py_RETURN_NONE;
+        const Rows r = rows_of(x, k);
+        std::vector<int64_t> shape{splits};
+        shape.insert(shape.end(), x.sizes().begin(), x.sizes().end() - 1);
+        shape.push_back(cols);
+        Tensor p = at::empty(shape, at::TensorOptions().dtype(at::kFloat).device(x.device()));
+        check(mdx_decode_linear_partials(ptr(r.t), r.stride, ptr(w), w.stride(0), static_cast<float*>(ptr(p)), rows, cols, k, stream_of(x)), "linear_partials");
+        return wrap(std::move(p));
+    });
+}
+
+// x [.., k], w [2 n, k] -> silu_and_mul(x . w^T) [.., n], or None where the shape is not covered
+PyObject* linear_silu(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    ARGS(2);
+    return guarded([&]() -> PyObject* {
+        const Tensor &x = tensor(a[0]), &w = tensor(a[1]);
+        need_gpu({&x, &w});
+        NEED(x.dim() >= 2 && w.dim() == 2 && x.size(-1) == w.size(1) && w.size(0) % 2 == 0);
+        const int64_t k = w.size(1), cols = w.size(0) / 2, rows = k ? x.numel() / k : 0;
+        if (!mdx_decode_linear_silu_supported(rows, cols, k) || x.scalar_type() != at::kBFloat16 || w.scalar_type() != at::kBFloat16 || x.stride(-1) != 1 || w.stride(1) != 1)
+            Py_RETURN_NONE;
+        const Rows r = rows_of(x, k);
+        std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());
+        shape.back() = cols;
+        Tensor y = at::empty(shape, at::TensorOptions().dtype(at::kBFloat16).device(x.device()));
+        check(mdx_decode_linear_silu(ptr(r.t), r.stride, ptr(w), w.stride(0), ptr(y), cols, rows, cols, k, stream_of(x)), "linear_silu");
+        return wrap(std::move(y));
+    });
+}
+
+void need_partials(const Tensor& p) { NEED(p.dim() >= 3 && p.scalar_type() == at::kFloat && p.is_contiguous()); }
+
+// partials [splits, .., hidden], weight, eps, residual [.., hidden] -> normed, new residual
+PyObject* rms_norm_partials(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    ARGS(4);
+    return guarded([&]() -> PyObject* {
+        const Tensor &p = tensor(a[0]), &w = tensor(a[1]), &residual = tensor(a[3]);
+        need_gpu({&p, &w, &residual});
+        need_partials(p);
+        const int64_t hidden = p.size(-1);
+        NEED(residual.sizes() == p.sizes().slice(1) && residual.stride(-1) == 1 && w.dim() == 1 && w.size(0) == hidden && w.is_contiguous() &&
+             w.scalar_type() == residual.scalar_type());
+        const Rows res = rows_of(residual, hidden);
+        const auto options = at::TensorOptions().dtype(w.scalar_type()).device(p.device());
+        Tensor out = at::empty(residual.sizes(), options), r_out = at::empty(residual.sizes(), options);
+        check(mdx_add_rms_norm_partials(static_cast<const float*>(ptr(p)), (int32_t)p.size(0), ptr(res.t), res.stride, ptr(r_out), hidden, ptr(w),
+                                        (float)real(a[2]), ptr(out), hidden, res.n, (int32_t)hidden, dtype_of(w), stream_of(p)), "rms_norm");
+        return wrap_tuple(std::move(out), std::move(r_out));
+    });
+}
+
+// partials [splits, .., (Hq + 2 Hkv) d], q_weight, k_weight, eps, cos, sin, positions, Hq, Hkv, d, k_cache, v_cache, slot_mapping -> q [.., Hq, d]
+PyObject* qk_norm_rope_store_partials(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    ARGS(13);
+    return guarded([&]() -> PyObject* {
+        const Tensor &p = tensor(a[0]), &qw = tensor(a[1]), &kw = tensor(a[2]), &cos = tensor(a[4]), &sin = tensor(a[5]), &positions = tensor(a[6]);
+        const Tensor &k_cache = tensor(a[10]), &v_cache = tensor(a[11]), &slot_mapping = tensor(a[12]);
+        const int64_t hq = integer(a[7]), hkv = integer(a[8]), d = integer(a[9]);
+        need_gpu({&p, &qw, &kw, &cos, &sin, &positions, &k_cache, &v_cache, &slot_mapping});
+        need_partials(p);
+        const int64_t width = (hq + 2 * hkv) * d, rows = p.numel() / p.size(0) / width;
+        NEED(p.size(-1) == width && positions.numel() == rows && positions.scalar_type() == at::kLong && cos.scalar_type() == at::kFloat && sin.scalar_type() == at::kFloat);
+        NEED(k_cache.is_contiguous() && v_cache.is_contiguous() && k_cache.scalar_type() == qw.scalar_type() && slot_mapping.numel() == rows);
+        const Tensor pos = positions.is_contiguous() ? positions : positions.contiguous(), slots = int32_list(slot_mapping, "slot_mapping");
+        std::vector<int64_t> shape(p.sizes().begin() + 1, p.sizes().end() - 1);
+        shape.push_back(hq);
+        shape.push_back(d);
+        Tensor q = at::empty(shape, at::TensorOptions().dtype(qw.scalar_type()).device(p.device()));
+        check(mdx_qk_norm_rope_store_partials(static_cast<const float*>(ptr(p)), (int32_t)p.size(0), ptr(qw), ptr(kw), (float)real(a[3]),
+                                              static_cast<const float*>(ptr(cos)), static_cast<const float*>(ptr(sin)), cos.size(0),
+                                              static_cast<const int64_t*>(ptr(pos)), ptr(q), hq * d, ptr(k_cache), ptr(v_cache),
+                                              static_cast<const int32_t*>(ptr(slots)), k_cache.numel() / (hkv * d), rows, (int32_t)hq, (int32_t)hkv,
+                                              (int32_t)d, dtype_of(qw), stream_of(p)), "qk_norm_rope_store");
+        return wrap(std::move(q));
     });
 }
 
@@ -704,7 +792,8 @@ PyObject* sampler_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 #define ENTRY(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
-    ENTRY(store_kvcache), ENTRY(qk_norm_rope_store), ENTRY(rms_norm), ENTRY(silu_and_mul), ENTRY(sparse_attn_varlen),
+    ENTRY(store_kvcache), ENTRY(qk_norm_rope_store), ENTRY(rms_norm), ENTRY(silu_and_mul), ENTRY(linear_partials), ENTRY(linear_silu),
+    ENTRY(rms_norm_partials), ENTRY(qk_norm_rope_store_partials), ENTRY(sparse_attn_varlen),
     ENTRY(flash_attn_with_kvcache), ENTRY(attention_prefill), ENTRY(attention_decode), ENTRY(confidence_argmax), ENTRY(lm_head_confidence),
     ENTRY(filter_logits), ENTRY(select_transfer), ENTRY(unmask_step), ENTRY(sampler_step),
     {nullptr, nullptr, 0, nullptr},

@@ -18,6 +18,7 @@
 // and the product with the other half is rounded again (the reference's activation is the
 // third-party liger-kernel 0.6.4 SwiGLU forward, which computes silu(a).cast(b.dtype) * b).
 #include "mdx_common.h"
+#include "split_sum.h"
 
 namespace {
 
@@ -27,7 +28,8 @@ constexpr int kNormThreads = 256;
 constexpr int kNormMaxVecs = 4;                  // 16-byte vectors per thread: rows up to 8192 elements
 
 struct NormParams {
-    const __bf16* x; int64_t x_stride;                     // [rows][hidden]
+    const __bf16* x; int64_t x_stride;                     // [rows][hidden], or
+    const float* partials; int splits;                     // [splits][rows][hidden]: x as the partial sums of a K-split product
     const __bf16* residual_in; int64_t res_in_stride;      // null: plain rms_forward
     __bf16* residual_out; int64_t res_out_stride;          // null when residual_in is null
     const __bf16* weight; float eps;
@@ -51,7 +53,8 @@ __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(const NormPa
     for (int i = 0; i < VECS; ++i) {
         const int v = tid + i * kNormThreads;
         if (v < n_vec) {
-            const bf16x8 a = *reinterpret_cast<const bf16x8*>(P.x + row * P.x_stride + 8 * v);
+            const bf16x8 a = P.partials ? mdx_split::sum8(P.partials + row * P.hidden + 8 * v, P.splits, P.rows * P.hidden)
+                                        : *reinterpret_cast<const bf16x8*>(P.x + row * P.x_stride + 8 * v);
 #pragma unroll
             for (int e = 0; e < 8; ++e) s[i][e] = (float)a[e];
             if (P.residual_in) {
@@ -113,7 +116,9 @@ __global__ __launch_bounds__(256) void silu_and_mul_kernel(const __bf16* x, int6
 
 }  // namespace
 
-extern "C" int mdx_add_rms_norm(const void* x, int64_t x_row_stride,
+namespace {
+
+int add_rms_norm(const void* x, int64_t x_row_stride, const float* partials, int splits,
                                 const void* residual_in, int64_t residual_in_row_stride,
                                 void* residual_out, int64_t residual_out_row_stride,
                                 const void* weight, float eps,
@@ -128,19 +133,19 @@ extern "C" int mdx_add_rms_norm(const void* x, int64_t x_row_stride,
                 "%s: hidden %d (multiples of 8 up to %d)", what, hidden, 8 * kNormThreads * kNormMaxVecs);
     MDX_REQUIRE(eps >= 0.f, MDX_EINVAL, "%s: negative eps", what);
     if (rows == 0) return MDX_OK;
-    MDX_REQUIRE(x && weight && out, MDX_EINVAL, "%s: null pointer", what);
+    MDX_REQUIRE((x || partials) && weight && out, MDX_EINVAL, "%s: null pointer", what);
     MDX_REQUIRE((residual_in == nullptr) == (residual_out == nullptr), MDX_EINVAL,
                 "%s: residual_in and residual_out go together", what);
     MDX_REQUIRE(rows <= 0x7fffffffLL, MDX_EUNSUPPORTED, "%s: %lld rows", what, (long long)rows);
-    MDX_REQUIRE(mdx::aligned16(x) && mdx::aligned16(out) && mdx::aligned16(weight) && mdx::aligned16(residual_in) && mdx::aligned16(residual_out) &&
+    MDX_REQUIRE(mdx::aligned16(x) && mdx::aligned16(partials) && mdx::aligned16(out) && mdx::aligned16(weight) && mdx::aligned16(residual_in) && mdx::aligned16(residual_out) &&
                 x_row_stride % 8 == 0 && out_row_stride % 8 == 0 &&
                 (!residual_in || (residual_in_row_stride % 8 == 0 && residual_out_row_stride % 8 == 0)),
                 MDX_EUNSUPPORTED, "%s: rows must be 16-byte aligned", what);
-    MDX_REQUIRE(x_row_stride >= hidden && out_row_stride >= hidden &&
+    MDX_REQUIRE((partials ? splits > 0 : x_row_stride >= hidden) && out_row_stride >= hidden &&
                 (!residual_in || (residual_in_row_stride >= hidden && residual_out_row_stride >= hidden)),
                 MDX_EINVAL, "%s: row stride smaller than the row", what);
     NormParams P;
-    P.x = (const __bf16*)x; P.x_stride = x_row_stride;
+    P.x = (const __bf16*)x; P.x_stride = x_row_stride; P.partials = partials; P.splits = splits;
     P.residual_in = (const __bf16*)residual_in; P.res_in_stride = residual_in_row_stride;
     P.residual_out = (__bf16*)residual_out; P.res_out_stride = residual_out_row_stride;
     P.weight = (const __bf16*)weight; P.eps = eps;
@@ -152,6 +157,29 @@ extern "C" int mdx_add_rms_norm(const void* x, int64_t x_row_stride,
     else if (vecs == 2) add_rms_norm_kernel<2><<<grid, kNormThreads, 0, stream>>>(P);
     else add_rms_norm_kernel<4><<<grid, kNormThreads, 0, stream>>>(P);
     return mdx::check_launch(what);
+}
+
+}  // namespace
+
+extern "C" int mdx_add_rms_norm(const void* x, int64_t x_row_stride,
+                                const void* residual_in, int64_t residual_in_row_stride,
+                                void* residual_out, int64_t residual_out_row_stride,
+                                const void* weight, float eps,
+                                void* out, int64_t out_row_stride,
+                                int64_t rows, int32_t hidden, int32_t dtype, mdx_stream_t stream)
+{
+    return add_rms_norm(x, x_row_stride, nullptr, 0, residual_in, residual_in_row_stride, residual_out, residual_out_row_stride, weight, eps,
+                        out, out_row_stride, rows, hidden, dtype, stream);
+}
+
+extern "C" int mdx_add_rms_norm_partials(const float* partials, int32_t splits,
+                                         const void* residual_in, int64_t residual_in_row_stride,
+                                         void* residual_out, int64_t residual_out_row_stride,
+                                         const void* weight, float eps, void* out, int64_t out_row_stride,
+                                         int64_t rows, int32_t hidden, int32_t dtype, mdx_stream_t stream)
+{
+    return add_rms_norm(nullptr, 0, partials, splits, residual_in, residual_in_row_stride, residual_out, residual_out_row_stride, weight, eps,
+                        out, out_row_stride, rows, hidden, dtype, stream);
 }
 
 extern "C" int mdx_silu_and_mul(const void* x, int64_t x_row_stride, void* out, int64_t out_row_stride,

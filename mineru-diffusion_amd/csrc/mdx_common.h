@@ -1,6 +1,7 @@
 // Shared host-side helpers of libmdx: error reporting and argument checks.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <atomic>
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
@@ -37,6 +38,21 @@ constexpr int kWave = 64;          // gfx950 wavefront
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
 namespace mdx {
+
+// Compute units of the current device, read once per device; 256 where no device can be asked (a shape query in a process
+// without a GPU).
+inline int compute_units() {
+    constexpr int kMaxDevices = 64;
+    static std::atomic<int> cached[kMaxDevices];
+    int device = -1;
+    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= kMaxDevices) return 256;
+    int n = cached[device].load(std::memory_order_relaxed);
+    if (n == 0) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || n <= 0) n = 256;
+        cached[device].store(n, std::memory_order_relaxed);
+    }
+    return n;
+}
 
 }  // namespace mdx
 

@@ -36,7 +36,6 @@
 //    (m, l, O) that a second, small kernel combines.
 #include "mdx_common.h"
 #include "attn_tile.h"
-#include <atomic>
 
 namespace {
 
@@ -556,18 +555,7 @@ __global__ __launch_bounds__(256) void paged_combine_kernel(const PagedParams P)
 // The counts behind those rules (1.95 workgroups per CU, pairs per CU) are taken from the current device's
 // number of compute units, read once per device; 256 on the MI355X that the rules were measured on, and
 // where no device can be asked (a shape query in a process without a GPU).
-int cu_count() {
-    constexpr int kMaxDevices = 64;
-    static std::atomic<int> cached[kMaxDevices];
-    int device = -1;
-    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= kMaxDevices) return 256;
-    int n = cached[device].load(std::memory_order_relaxed);
-    if (n == 0) {
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || n <= 0) n = 256;
-        cached[device].store(n, std::memory_order_relaxed);
-    }
-    return n;
-}
+int cu_count() { return mdx::compute_units(); }
 
 // head_groups counts the workgroups that one (sequence, split) pair launches: head groups x query tiles.
 int pick_chunk(int bs, int head_groups, int max_pages, int page_size, bool* device_span) {

@@ -15,6 +15,7 @@
 // multiplied by the weight in the storage type (layernorm.py:24-25); the rotation is done in
 // fp32 and rounded once (rotary_embedding.py:11-14).
 #include "mdx_common.h"
+#include "split_sum.h"
 
 namespace {
 
@@ -24,7 +25,8 @@ constexpr int kLanesPerHead = 8;
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 
 struct FusedParams {
-    const __bf16* qkv; int64_t qkv_stride;
+    const __bf16* qkv; int64_t qkv_stride;        // or, with PARTIALS,
+    const float* partials; int splits;            // [splits][tokens][rows * d]: the projection as K-split partial sums
     const __bf16* q_w; const __bf16* k_w; float eps;
     const float* cos_t; const float* sin_t; int64_t max_pos; const int64_t* positions;
     __bf16* q_out; int64_t q_out_stride;
@@ -34,6 +36,7 @@ struct FusedParams {
     int64_t n_tokens; int hq, hkv;
 };
 
+template <bool PARTIALS>
 __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(const FusedParams P)
 {
     const int64_t tok = blockIdx.x;
@@ -53,9 +56,17 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(const FusedPara
         sn[e] = pos_ok ? P.sin_t[pos * (kHeadDim / 2) + 8 * j + e] : 0.0f;
     }
     for (int row = threadIdx.x / kLanesPerHead; row < n_rows; row += 256 / kLanesPerHead) {
-        const __bf16* src = P.qkv + tok * P.qkv_stride + (int64_t)row * kHeadDim;
-        bf16x8 a = *reinterpret_cast<const bf16x8*>(src + 8 * j);
-        bf16x8 b = *reinterpret_cast<const bf16x8*>(src + 64 + 8 * j);
+        bf16x8 a, b;
+        if (PARTIALS) {
+            const int64_t width = (int64_t)n_rows * kHeadDim;
+            const float* src = P.partials + tok * width + (int64_t)row * kHeadDim;
+            a = mdx_split::sum8(src + 8 * j, P.splits, P.n_tokens * width);
+            b = mdx_split::sum8(src + 64 + 8 * j, P.splits, P.n_tokens * width);
+        } else {
+            const __bf16* src = P.qkv + tok * P.qkv_stride + (int64_t)row * kHeadDim;
+            a = *reinterpret_cast<const bf16x8*>(src + 8 * j);
+            b = *reinterpret_cast<const bf16x8*>(src + 64 + 8 * j);
+        }
         const bool is_q = row < P.hq, is_k = !is_q && row < P.hq + P.hkv;
         if (is_q || is_k) {
             float ss = 0.f;
@@ -98,7 +109,9 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(const FusedPara
 
 }  // namespace
 
-extern "C" int mdx_qk_norm_rope_store(const void* qkv, int64_t qkv_row_stride,
+namespace {
+
+int qk_norm_rope_store(const void* qkv, int64_t qkv_row_stride, const float* partials, int splits,
                                       const void* q_weight, const void* k_weight, float eps,
                                       const float* cos_table, const float* sin_table, int64_t max_positions,
                                       const int64_t* positions,
@@ -113,19 +126,19 @@ extern "C" int mdx_qk_norm_rope_store(const void* qkv, int64_t qkv_row_stride,
     MDX_REQUIRE(dtype == MDX_BF16, MDX_EUNSUPPORTED, "qk_norm_rope_store: dtype %d (only bf16)", dtype);
     MDX_REQUIRE(head_dim == kHeadDim, MDX_EUNSUPPORTED, "qk_norm_rope_store: head_dim %d (only 128)", head_dim);
     if (n_tokens == 0) return MDX_OK;
-    MDX_REQUIRE(qkv && q_weight && k_weight && cos_table && sin_table && positions && q_out, MDX_EINVAL,
+    MDX_REQUIRE((qkv || partials) && q_weight && k_weight && cos_table && sin_table && positions && q_out, MDX_EINVAL,
                 "qk_norm_rope_store: null pointer");
     MDX_REQUIRE((k_cache == nullptr) == (v_cache == nullptr), MDX_EINVAL, "qk_norm_rope_store: give both caches or neither");
     MDX_REQUIRE(!k_cache || slot_mapping, MDX_EINVAL, "qk_norm_rope_store: caches without slot_mapping");
     MDX_REQUIRE(n_tokens < ((int64_t)1 << 31), MDX_EUNSUPPORTED, "qk_norm_rope_store: too many tokens");
-    MDX_REQUIRE(mdx::aligned16(qkv) && mdx::aligned16(q_out) && mdx::aligned16(q_weight) && mdx::aligned16(k_weight) &&
+    MDX_REQUIRE(mdx::aligned16(qkv) && mdx::aligned16(partials) && mdx::aligned16(q_out) && mdx::aligned16(q_weight) && mdx::aligned16(k_weight) &&
                 (!k_out || mdx::aligned16(k_out)) && (!k_cache || (mdx::aligned16(k_cache) && mdx::aligned16(v_cache))) &&
                 qkv_row_stride % 8 == 0 && q_out_row_stride % 8 == 0 && k_out_row_stride % 8 == 0,
                 MDX_EUNSUPPORTED, "qk_norm_rope_store: tensors must be 16-byte aligned with row strides that are multiples of 8");
-    MDX_REQUIRE(qkv_row_stride >= (int64_t)(num_q_heads + 2 * num_kv_heads) * kHeadDim, MDX_EINVAL,
+    MDX_REQUIRE(partials ? splits > 0 : qkv_row_stride >= (int64_t)(num_q_heads + 2 * num_kv_heads) * kHeadDim, MDX_EINVAL,
                 "qk_norm_rope_store: qkv row stride shorter than a QKV row");
     FusedParams P;
-    P.qkv = (const __bf16*)qkv; P.qkv_stride = qkv_row_stride;
+    P.qkv = (const __bf16*)qkv; P.qkv_stride = qkv_row_stride; P.partials = partials; P.splits = splits;
     P.q_w = (const __bf16*)q_weight; P.k_w = (const __bf16*)k_weight; P.eps = eps;
     P.cos_t = cos_table; P.sin_t = sin_table; P.max_pos = max_positions; P.positions = positions;
     P.q_out = (__bf16*)q_out; P.q_out_stride = q_out_row_stride;
@@ -133,6 +146,37 @@ extern "C" int mdx_qk_norm_rope_store(const void* qkv, int64_t qkv_row_stride,
     P.k_cache = (__bf16*)k_cache; P.v_cache = (__bf16*)v_cache;
     P.slot_mapping = slot_mapping; P.num_slots = num_slots;
     P.n_tokens = n_tokens; P.hq = num_q_heads; P.hkv = num_kv_heads;
-    qk_norm_rope_store_kernel<<<(unsigned)n_tokens, 256, 0, stream>>>(P);
+    if (partials) qk_norm_rope_store_kernel<true><<<(unsigned)n_tokens, 256, 0, stream>>>(P);
+    else          qk_norm_rope_store_kernel<false><<<(unsigned)n_tokens, 256, 0, stream>>>(P);
     return mdx::check_launch("qk_norm_rope_store");
+}
+
+}  // namespace
+
+extern "C" int mdx_qk_norm_rope_store(const void* qkv, int64_t qkv_row_stride,
+                                      const void* q_weight, const void* k_weight, float eps,
+                                      const float* cos_table, const float* sin_table, int64_t max_positions,
+                                      const int64_t* positions,
+                                      void* q_out, int64_t q_out_row_stride,
+                                      void* k_out, int64_t k_out_row_stride,
+                                      void* k_cache, void* v_cache, const int32_t* slot_mapping, int64_t num_slots,
+                                      int64_t n_tokens, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                                      int32_t dtype, mdx_stream_t stream_)
+{
+    return qk_norm_rope_store(qkv, qkv_row_stride, nullptr, 0, q_weight, k_weight, eps, cos_table, sin_table, max_positions, positions,
+                              q_out, q_out_row_stride, k_out, k_out_row_stride, k_cache, v_cache, slot_mapping, num_slots,
+                              n_tokens, num_q_heads, num_kv_heads, head_dim, dtype, stream_);
+}
+
+extern "C" int mdx_qk_norm_rope_store_partials(const float* partials, int32_t splits,
+                                               const void* q_weight, const void* k_weight, float eps,
+                                               const float* cos_table, const float* sin_table, int64_t max_positions,
+                                               const int64_t* positions, void* q_out, int64_t q_out_row_stride,
+                                               void* k_cache, void* v_cache, const int32_t* slot_mapping, int64_t num_slots,
+                                               int64_t n_tokens, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                                               int32_t dtype, mdx_stream_t stream)
+{
+    return qk_norm_rope_store(nullptr, 0, partials, splits, q_weight, k_weight, eps, cos_table, sin_table, max_positions, positions,
+                              q_out, q_out_row_stride, nullptr, 0, k_cache, v_cache, slot_mapping, num_slots,
+                              n_tokens, num_q_heads, num_kv_heads, head_dim, dtype, stream);
 }

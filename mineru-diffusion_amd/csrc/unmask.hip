@@ -410,16 +410,17 @@ __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
     }
 }
 
-// A row's splits merged by the 16 lanes of a group: each takes every 16th, then four exchanges.  (One lane per row walking
-// the splits was a chain of dependent trips to memory: 6.2 us for nine splits, a third of what 96 sampled rows take.)
-constexpr int kMergeLanes = 16;
+// A row's splits merged by a group of lanes: each takes every lanes-th, then the exchanges.  (One lane per row walking
+// the splits was a chain of dependent trips to memory: 6.2 us for nine splits, a third of what 96 sampled rows take.  Two or
+// three splits are walked all the same: a selection launch of 16 lanes per position takes 0.4 us longer than one of one.)
+constexpr int kMergeLanes = 16;                // at most
+int merge_lanes(int nsplit) { return nsplit <= 3 ? 1 : nsplit <= 8 ? 4 : kMergeLanes; }
 template <bool NOISE>
-__device__ __forceinline__ Partial merge_splits(const Partial* __restrict__ partials, int nsplit, int lane16, float c) {
+__device__ __forceinline__ Partial merge_splits(const Partial* __restrict__ partials, int nsplit, int lane, int lanes, float c) {
     Partial r;
     r.m = kNegBig; r.s = 0.f; r.idx = kNoIndex; r.pick = kNegBig; r.pick_x = 0.f; r.pick_idx = kNoIndex;
-    for (int s = lane16; s < nsplit; s += kMergeLanes) combine(r, partials[s], c, NOISE);
-#pragma unroll
-    for (int off = kMergeLanes / 2; off >= 1; off >>= 1) combine(r, shfl_xor(r, off, NOISE), c, NOISE);
+    for (int s = lane; s < nsplit; s += lanes) combine(r, partials[s], c, NOISE);
+    for (int off = lanes / 2; off >= 1; off >>= 1) combine(r, shfl_xor(r, off, NOISE), c, NOISE);
     return r;
 }
 
@@ -433,7 +434,7 @@ __global__ __launch_bounds__(kThreads) void confidence_finalize_kernel(
     const int lane16 = threadIdx.x % kMergeLanes;
     if (row >= rows) return;                                 // (whole groups)
     const float c = kLog2e / (temperatures ? temperatures[row / rows_per_temp] : 1.0f);
-    const Partial r = merge_splits<NOISE>(partials + row * nsplit, nsplit, lane16, c);
+    const Partial r = merge_splits<NOISE>(partials + row * nsplit, nsplit, lane16, kMergeLanes, c);
     if (lane16 != 0) return;
     int64_t tok; float conf;
     finish_row<NOISE>(r, c, tok, conf);
@@ -450,14 +451,14 @@ constexpr int kMaxSelectThreads = 1024;
 // The block's confidences and picks into LDS, merged from the splits where need be; all threads of the workgroup.
 template <int SOURCE>
 __device__ __forceinline__ void gather_block(float* conf_s, int* pick_s, int64_t* x0, float* x0_p, const Partial* partials, int nsplit,
-                                             const float* temperatures, int b, int block_len)
+                                             const float* temperatures, int b, int block_len, int lanes)
 {
-    const int lane16 = threadIdx.x % kMergeLanes;
+    const int lane = threadIdx.x & (lanes - 1);
     const float c = kLog2e / (temperatures ? temperatures[b] : 1.0f);
-    for (int p = threadIdx.x / kMergeLanes; p < block_len; p += blockDim.x / kMergeLanes) {
+    for (int p = threadIdx.x / lanes; p < block_len; p += blockDim.x / lanes) {
         const int64_t at = (int64_t)b * block_len + p;
-        const Partial r = merge_splits<SOURCE == kFromNoisySplits>(partials + at * nsplit, nsplit, lane16, c);
-        if (lane16 == 0) {
+        const Partial r = merge_splits<SOURCE == kFromNoisySplits>(partials + at * nsplit, nsplit, lane, lanes, c);
+        if (lane == 0) {
             int64_t tok; float conf;
             finish_row<SOURCE == kFromNoisySplits>(r, c, tok, conf);
             x0[at] = tok;
@@ -475,7 +476,7 @@ __global__ __launch_bounds__(kMaxBlockLen) void select_transfer_kernel(
     int64_t* __restrict__ x0, float* __restrict__ x0_p, int64_t* __restrict__ tokens,
     const Partial* __restrict__ partials, int nsplit, const float* __restrict__ temperatures,
     int64_t mask_token_id, float threshold, int k,
-    uint8_t* __restrict__ transfer, int32_t* __restrict__ count, int block_len)
+    uint8_t* __restrict__ transfer, int32_t* __restrict__ count, int block_len, int lanes)
 {
     __shared__ float conf_s[kMaxBlockLen];
     __shared__ int pick_s[SOURCE == kFromRows ? 1 : kMaxBlockLen];
@@ -488,7 +489,7 @@ __global__ __launch_bounds__(kMaxBlockLen) void select_transfer_kernel(
     int64_t pick = 0;
     float pick_p = 0.f;
     if (SOURCE != kFromRows) {
-        gather_block<SOURCE>(conf_s, pick_s, x0, x0_p, partials, nsplit, temperatures, b, block_len);
+        gather_block<SOURCE>(conf_s, pick_s, x0, x0_p, partials, nsplit, temperatures, b, block_len, lanes);
         if (on) { pick = pick_s[p]; pick_p = conf_s[p]; }
     } else if (on) {
         pick = x0[at];
@@ -531,13 +532,13 @@ __global__ __launch_bounds__(kMaxBlockLen) void select_transfer_kernel(
 // sequence: lane p owns position p, counts are ballots, and the rank among the masked positions comes
 // from reading every lane's confidence in turn -- no LDS, no atomics, no barrier, so the launch costs
 // little more than its one round trip to memory.  Where the row splits have to be merged first, the sequence gets
-// 16 lanes per position for that, and its first wavefront goes on alone.
+// more lanes per position for that, and its first wavefront goes on alone.
 template <int SOURCE>
 __global__ __launch_bounds__(kMaxSelectThreads) void select_transfer_wave_kernel(
     int64_t* __restrict__ x0, float* __restrict__ x0_p, int64_t* __restrict__ tokens,
     const Partial* __restrict__ partials, int nsplit, const float* __restrict__ temperatures,
     int64_t mask_token_id, float threshold, int k,
-    uint8_t* __restrict__ transfer, int32_t* __restrict__ count, int block_len)
+    uint8_t* __restrict__ transfer, int32_t* __restrict__ count, int block_len, int lanes)
 {
     __shared__ float conf_s[SOURCE == kFromRows ? 1 : mdx::kWave];
     __shared__ int pick_s[SOURCE == kFromRows ? 1 : mdx::kWave];
@@ -549,7 +550,7 @@ __global__ __launch_bounds__(kMaxSelectThreads) void select_transfer_wave_kernel
     float pick_p = 0.f;
     const int64_t tok = on ? tokens[at] : 0;
     if (SOURCE != kFromRows) {
-        gather_block<SOURCE>(conf_s, pick_s, x0, x0_p, partials, nsplit, temperatures, b, block_len);
+        gather_block<SOURCE>(conf_s, pick_s, x0, x0_p, partials, nsplit, temperatures, b, block_len, lanes);
         if (p >= mdx::kWave) return;
         if (on) { pick = pick_s[p]; pick_p = conf_s[p]; }
     } else if (on) {
@@ -585,11 +586,12 @@ int launch_select(int64_t* x0, float* x0_p, int64_t* tokens, const Partial* part
 {
     const int source = partials == nullptr || nsplit <= 1 ? kFromRows : noisy ? kFromNoisySplits : kFromSplits;
     const int whole_waves = (block_len + mdx::kWave - 1) / mdx::kWave * mdx::kWave;
-    // lanes to merge splits with: 16 per position, as many positions at a time as a workgroup holds
-    const int merging = block_len * kMergeLanes < kMaxSelectThreads ? (block_len * kMergeLanes + mdx::kWave - 1) / mdx::kWave * mdx::kWave : kMaxSelectThreads;
+    // lanes to merge splits with, for as many positions at a time as a workgroup holds
+    const int lanes = merge_lanes(nsplit), wanted = (block_len * lanes + mdx::kWave - 1) / mdx::kWave * mdx::kWave;
+    const int merging = wanted < kMaxSelectThreads ? wanted : kMaxSelectThreads;
     const unsigned threads = source == kFromRows ? whole_waves : (merging > whole_waves ? merging : whole_waves);
 #define MDX_SELECT(KERNEL, SOURCE) KERNEL<SOURCE><<<(unsigned)bs, threads, 0, stream>>>( \
-        x0, x0_p, tokens, partials, nsplit, temperatures, mask_token_id, threshold, k, transfer, count, block_len)
+        x0, x0_p, tokens, partials, nsplit, temperatures, mask_token_id, threshold, k, transfer, count, block_len, lanes)
     if (block_len <= mdx::kWave) {
         if (source == kFromRows)        MDX_SELECT(select_transfer_wave_kernel, kFromRows);
         else if (source == kFromSplits) MDX_SELECT(select_transfer_wave_kernel, kFromSplits);

@@ -45,6 +45,13 @@ SIGNATURES = {
                                          _I64, _I32, _I32, _I32, _I32, _P]),
     "mdx_add_rms_norm": (c_int32, [_P, _I64, _P, _I64, _P, _I64, _P, _F, _P, _I64, _I64, _I32, _I32, _P]),
     "mdx_silu_and_mul": (c_int32, [_P, _I64, _P, _I64, _I64, _I32, _I32, _P]),
+    "mdx_decode_linear_splits": (c_int32, [_I64] * 3),
+    "mdx_decode_linear_partials": (c_int32, [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _P]),
+    "mdx_decode_linear_silu_supported": (c_int32, [_I64] * 3),
+    "mdx_decode_linear_silu": (c_int32, [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _P]),
+    "mdx_add_rms_norm_partials": (c_int32, [_P, _I32, _P, _I64, _P, _I64, _P, _F, _P, _I64, _I64, _I32, _I32, _P]),
+    "mdx_qk_norm_rope_store_partials": (c_int32, [_P, _I32, _P, _P, _F, _P, _P, _I64, _P, _P, _I64, _P, _P, _P, _I64,
+                                                  _I64, _I32, _I32, _I32, _I32, _P]),
     "mdx_block_prepare": (c_int32, [_P, _P, _P, _I64, _I32, _I32, _I32, _P, _P, _P, _I32, _P]),
     "mdx_masked_rows": (c_int32, [_P, _P, _I64, _I32, _I32, _P, _I32, _P, _P]),
     "mdx_block_advance": (c_int32, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I32, _P, _P, _I64, _P, _I64, _I32, _I32, _P]),

@@ -11,8 +11,8 @@ kernels can be driven exactly as the engine drives them:
   decoder layer structure         nanovllm/models/sdar.py:68-181, layers/layernorm.py:16-40,
                                   layers/rotary_embedding.py:6-48, layers/embed_head.py:61-67
 
-The decoder is a random-init scaffold whose GEMMs are stock PyTorch (library) GEMMs; attention,
-the KV store, the norms, the activation and the unmask step go through libmdx.  Decode passes can
+The decoder is a random-init scaffold; attention, the KV store, the norms, the activation, the unmask step and the
+linear layers of small decode batches go through libmdx, the other GEMMs are stock PyTorch (library) GEMMs.  Decode passes can
 replay a captured HIP graph (model_runner.py:198-259).  There is no vision tower, tokenizer,
 weight loader or tensor parallelism here.
 """
@@ -32,8 +32,8 @@ from torch import nn
 from . import _lib
 from .context import get_context, reset_context, set_context
 from .layers import Attention
-from .ops import (confidence_argmax, lm_head_confidence, flash_attn_with_kvcache, qk_norm_rope_store, rms_norm, select_transfer, silu_and_mul,
-                  sparse_attn_varlen, unmask_step)
+from .ops import (confidence_argmax, lm_head_confidence, flash_attn_with_kvcache, linear_partials, linear_silu, qk_norm_rope_store,
+                  qk_norm_rope_store_partials, rms_norm, rms_norm_partials, select_transfer, silu_and_mul, sparse_attn_varlen, unmask_step)
 
 PAGE = 256                      # tokens per KV page (Sequence.kvcache_block_size, sequence.py:17)
 
@@ -196,9 +196,11 @@ class DecoderLayer(nn.Module):
         self.attn = Attention(c.num_heads, c.head_dim, c.head_dim ** -0.5, c.num_kv_heads)
 
     def _norm(self, x, residual, w):
-        """layernorm.py:43-51: (normed, new residual)."""
+        """layernorm.py:43-51: (normed, new residual).  x may be the partial sums of a linear layer (one dimension more)."""
         c = self.c
         if c.fused_layer_ops:
+            if residual is not None and x.dim() > residual.dim():
+                return rms_norm_partials(x, w, c.rms_norm_eps, residual)
             if residual is None:
                 return rms_norm(x, w, c.rms_norm_eps), x
             return rms_norm(x, w, c.rms_norm_eps, residual)
@@ -208,10 +210,10 @@ class DecoderLayer(nn.Module):
     def forward(self, positions, x, residual, cos, sin, cos_table=None, sin_table=None):
         c = self.c
         h, residual = self._norm(x, residual, self.input_layernorm)       # sdar.py:147-150
-        qkv = F.linear(h, self.qkv_proj)
         if c.fused_qk_rope_store:
-            o = self._attend_fused(qkv, positions, cos_table, sin_table)
+            o = self._attend_fused(h, positions, cos_table, sin_table)
         else:
+            qkv = F.linear(h, self.qkv_proj)
             q_size, kv_size = c.num_heads * c.head_dim, c.num_kv_heads * c.head_dim
             q, k, v = qkv.split([q_size, kv_size, kv_size], dim=-1)
             shape = (*positions.shape, -1, c.head_dim)
@@ -220,21 +222,34 @@ class DecoderLayer(nn.Module):
             k = _rms(k, self.k_norm, c.rms_norm_eps)
             q, k = _rope(q, cos, sin), _rope(k, cos, sin)
             o = self.attn(q, k, v)
-        x = F.linear(o, self.o_proj)
-        h, residual = self._norm(x, residual, self.post_attention_layernorm)
-        gate_up = F.linear(h, self.gate_up_proj)
+        h, residual = self._norm(self._linear(o, self.o_proj), residual, self.post_attention_layernorm)
         if c.fused_layer_ops:
-            act = silu_and_mul(gate_up)
+            act = linear_silu(h, self.gate_up_proj)
+            if act is None:
+                act = silu_and_mul(F.linear(h, self.gate_up_proj))
         else:
-            gate, up = gate_up.chunk(2, dim=-1)
+            gate, up = F.linear(h, self.gate_up_proj).chunk(2, dim=-1)
             act = F.silu(gate) * up
-        return F.linear(act, self.down_proj), residual
+        return self._linear(act, self.down_proj), residual
 
-    def _attend_fused(self, qkv, positions, cos_table, sin_table):
-        """sdar.py:79-83 + sdar_attention.py:34-57 with the q/k norm, RoPE and cache store done by
+    def _linear(self, x, w):
+        """A linear layer whose output the next norm takes in: the partial sums of libmdx's product for the few rows of a
+        small decode batch, else the library's product."""
+        partials = linear_partials(x, w) if self.c.fused_layer_ops else None
+        return F.linear(x, w) if partials is None else partials
+
+    def _attend_fused(self, h, positions, cos_table, sin_table):
+        """sdar.py:73-83 + sdar_attention.py:34-57 with the q/k norm, RoPE and cache store done by
         one libmdx launch; the attention calls are the same two as in `Attention.forward`."""
         c, attn, ctx = self.c, self.attn, get_context()
         have_cache = attn.k_cache.numel() > 0
+        qkv = linear_partials(h, self.qkv_proj) if have_cache and not ctx.is_prefill else None
+        if qkv is not None:
+            q = qk_norm_rope_store_partials(qkv, self.q_norm, self.k_norm, c.rms_norm_eps, cos_table, sin_table, positions, c.num_heads,
+                                            c.num_kv_heads, c.head_dim, attn.k_cache, attn.v_cache, ctx.slot_mapping)
+            return flash_attn_with_kvcache(q, attn.k_cache, attn.v_cache, cache_seqlens=ctx.context_lens, block_table=ctx.block_tables,
+                                           softmax_scale=attn.scale, causal=False).flatten(2)
+        qkv = F.linear(h, self.qkv_proj)
         q, k, v = qk_norm_rope_store(qkv, self.q_norm, self.k_norm, c.rms_norm_eps, cos_table, sin_table, positions,
                                      c.num_heads, c.num_kv_heads, c.head_dim,
                                      attn.k_cache if have_cache else None, attn.v_cache if have_cache else None,
@@ -287,7 +302,8 @@ class Decoder(nn.Module):
         for layer in self.layers:
             x, residual = layer(positions, x, residual, cos, sin, self.cos, self.sin)
         if self.c.fused_layer_ops:
-            return rms_norm(x, self.norm, self.c.rms_norm_eps, residual)[0]
+            norm = rms_norm_partials if x.dim() > residual.dim() else rms_norm
+            return norm(x, self.norm, self.c.rms_norm_eps, residual)[0]
         return _rms(x + residual, self.norm, self.c.rms_norm_eps)
 
     @torch.inference_mode()

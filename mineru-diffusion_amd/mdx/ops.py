@@ -60,6 +60,31 @@ def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
     return _host().silu_and_mul(x)
 
 
+# --------------------------------------------------------------------------- linear layers of a decode pass
+# x . weight^T for up to 128 rows as fp32 partial sums over slices of K ([splits, ..., n]), which the two functions after it add up
+# on their way; None where the shape is not covered (more rows, other widths), and the caller takes the library's product.
+def linear_partials(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor | None:
+    """The product of a linear layer (nanovllm/layers/linear.py) for rms_norm_partials or qk_norm_rope_store_partials."""
+    return _host().linear_partials(x, weight)
+
+
+def linear_silu(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor | None:
+    """silu_and_mul(x . weight^T) for up to 64 rows in one launch (nanovllm/models/sdar.py:105-111); None as above."""
+    return _host().linear_silu(x, weight)
+
+
+def rms_norm_partials(partials: torch.Tensor, weight: torch.Tensor, eps: float, residual: torch.Tensor):
+    """rms_norm(x, weight, eps, residual) with x given by linear_partials."""
+    return _host().rms_norm_partials(partials, weight, eps, residual)
+
+
+def qk_norm_rope_store_partials(partials, q_weight, k_weight, eps, cos, sin, positions, num_q_heads, num_kv_heads, head_dim,
+                                k_cache, v_cache, slot_mapping) -> torch.Tensor:
+    """The decode form of qk_norm_rope_store with qkv given by linear_partials: returns q; k and v go to the caches."""
+    return _host().qk_norm_rope_store_partials(partials, q_weight, k_weight, eps, cos, sin, positions, num_q_heads, num_kv_heads, head_dim,
+                                               k_cache, v_cache, slot_mapping)
+
+
 # --------------------------------------------------------------------------- staircase prefill
 def sparse_attn_varlen(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_seqlens_q: torch.Tensor,
                        cu_seqlens_k: torch.Tensor, staircase_size: int = 4, *, max_seqlen: int | None = None,
