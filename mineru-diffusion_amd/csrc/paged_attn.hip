@@ -14,7 +14,7 @@
 // rows), so the design goal is to keep the whole chip streaming pages:
 //  * split-KV: a workgroup owns one split of consecutive keys of one sequence
 //    for one group of query heads; the split size is chosen so that there are
-//    1.5 to 1.8 workgroups per CU (pick_chunk), and with a (sequence, KV head)
+//    one to two workgroups per CU at most (pick_chunk and the rule in the kernel), and with a (sequence, KV head)
 //    pair per CU sequences stay whole unless the kernel finds one far longer
 //    than the mean.  Workgroups are numbered densely over the
 //    (sequence, split) pairs that exist (lane b of each wavefront holds the
@@ -97,17 +97,16 @@ struct PagedParams {
     int num_q_heads;
     int head_dim;                                   // <= 128, a multiple of 16: columns beyond it are zeros in LDS and never stored
     float c;                                        // scale * log2(e)
-    float* part_o; float* part_ml;                  // [bs, Hq, nqt, nsplit, 32, 128] and [bs, Hq, nqt, nsplit, 2, 32]
+    float* part_o; float* part_ml;                  // [bs, Hq, nqt, nsplit, 32, 128] and [bs, Hq, nqt, nsplit, 32, (m, l)]
     // non-null: the attention kernel picks the split size (>= chunk) from the lengths and leaves it
     // here for the combine kernel.  A float on purpose: an int store in the attention kernel could
     // alias the int page table and lengths for the compiler, which would then stop fetching those
     // through the scalar cache and wait on the vector-memory counter for them, draining the K/V
     // prefetch queue (measured: 78 -> 120 us).  Split sizes are far below 2^24, so the value is exact.
     float* span_out;
-    // > 0: every sequence is cut (fewer (sequence, head group) pairs than the chip holds workgroups) and the host's
-    // split assumes page tables that are 65 % full.  The attention kernel, which sees the lengths, starts from the
-    // split that fills the chip when the tables are emptier, grows it by a tile at a time until the launch fits this
-    // many resident workgroups -- one round, nobody starts late -- and leaves the split it settled on in span_out.  (Full tables: 16 sequences of 4128 keys 69 -> 60 us, 16 of
+    // > 0: fewer (sequence, head group) pairs than the chip holds workgroups.  The attention kernel, which sees the
+    // lengths, picks the size of a piece, grows it by a tile at a time until the launch fits this
+    // many resident workgroups -- one round, nobody starts late -- and leaves the size it settled on in span_out.  (Full tables: 16 sequences of 4128 keys 69 -> 60 us, 16 of
     // 1000 to 3000 keys in a table 12 pages wide 51 -> 42 us; no shape of the sweep slower.  Cutting each sequence
     // into equal pieces instead of full splits and a short remainder was measured too and loses: the remainders
     // start last and fill the tail.)
@@ -117,83 +116,76 @@ struct PagedParams {
     float* arrive;
 };
 
-// Merges the nv split partials of query s of (sequence b, head hq); the caller's 8 threads c = 0..7
-// of a query take 16 consecutive d values each.  nv comes from `count()`, which is asked only after the
-// loads of the first four slots are on their way: where those slots lie does not depend on it (slots
-// beyond nv hold leftovers and are masked out), so a caller whose split count is still in flight from
-// memory overlaps that latency with the partials'.
-template <typename E, bool AGENT, typename Count>
-__device__ __forceinline__ void combine_query(const PagedParams& P, int b, int hq, int qt, int s, int c, Count count)
+// Running fold of split partials over COLS columns of one query.
+template <int COLS> struct Fold {
+    float M, L, acc[COLS];
+    __device__ __forceinline__ void init() {
+        M = kMinusBig; L = 0.f;
+#pragma unroll
+        for (int e = 0; e < COLS; ++e) acc[e] = 0.f;
+    }
+    // Four slots, of which the first `on` exist (the others hold leftovers).
+    __device__ __forceinline__ void take4(const float (&m_in)[4], const float (&l)[4], const f32x4 (&po)[4][COLS / 4], int on) {
+        float m[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) m[i] = i < on ? m_in[i] : kMinusBig;
+        const float Mn = fmaxf(fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3])), M);
+        const float keep = __builtin_amdgcn_exp2f(M - Mn);
+        L *= keep;
+#pragma unroll
+        for (int e = 0; e < COLS; ++e) acc[e] *= keep;
+        M = Mn;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float w = i < on ? __builtin_amdgcn_exp2f(m[i] - M) : 0.f;
+            L = i < on ? __builtin_fmaf(w, l[i], L) : L;                   // (explicit: both users of this fold give the same bits)
+#pragma unroll
+            for (int k = 0; k < COLS / 4; ++k)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[4 * k + e] = i < on ? __builtin_fmaf(w, po[i][k][e], acc[4 * k + e]) : acc[4 * k + e];
+        }
+    }
+    __device__ __forceinline__ float inverse() const { return L > 0.f ? 1.0f / L : 0.f; }   // no valid key at all (every page id invalid): zeros, like a context of 0
+};
+
+// Single-launch merge: folds the nv split partials of query s of (sequence b, head hq), which other workgroups of this launch
+// have just written; the caller's 8 threads c = 0..7 of a query take 16 consecutive d values each.
+template <typename E>
+__device__ __forceinline__ void combine_query(const PagedParams& P, int b, int hq, int qt, int s, int c, int nv)
 {
     if (c * 16 >= P.head_dim) return;
     const int64_t slot0 = (((int64_t)b * P.num_q_heads + hq) * P.nqt + qt) * P.nsplit;
-    int nv = P.nsplit;                         // until count() is in: every slot that exists
-    float M = kMinusBig, Lsum = 0.f;
-    float acc[16];
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+    Fold<16> F;
+    F.init();
     for (int i0 = 0; i0 < nv; i0 += 4) {
         float m[4], l[4];
         f32x4 po[4][4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int64_t slot = slot0 + min(i0 + i, P.nsplit - 1);
-            const float* ml = P.part_ml + (slot * 2 + 0) * kQTile + s;
+            const float* ml = P.part_ml + (slot * kQTile + s) * 2;
             const float* src = P.part_o + (slot * kQTile + s) * kHeadDim + c * 16;
-            if (AGENT) {
-                m[i] = __hip_atomic_load(ml, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                l[i] = __hip_atomic_load(ml + kQTile, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            m[i] = __hip_atomic_load(ml, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            l[i] = __hip_atomic_load(ml + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
-                for (int k = 0; k < 4; ++k) po[i][k] = load_agent(src + 4 * k);
-            } else {
-                m[i] = ml[0];
-                l[i] = ml[kQTile];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) po[i][k] = *reinterpret_cast<const f32x4*>(src + 4 * k);
-            }
+            for (int k = 0; k < 4; ++k) po[i][k] = load_agent(src + 4 * k);
         }
-        if (AGENT) {
-            // the asm loads are invisible to the compiler's own counting: wait here, and tie every loaded
-            // value to the wait so that no use of it can be scheduled above it
+        // the asm loads are invisible to the compiler's own counting: wait here, and tie every loaded
+        // value to the wait so that no use of it can be scheduled above it
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-                for (int k = 0; k < 4; ++k) asm volatile("s_waitcnt vmcnt(0)" : "+v"(po[i][k]) :: "memory");
-        }
-        if (i0 == 0) {
-            nv = count();
-            if (nv <= 1) return;               // written directly by the attention kernel
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) m[i] = i0 + i < nv ? m[i] : kMinusBig;
-        const float Mn = fmaxf(fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3])), M);
-        const float keep = __builtin_amdgcn_exp2f(M - Mn);
-        Lsum *= keep;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc[e] *= keep;
-        M = Mn;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const bool on = i0 + i < nv;
-            const float w = on ? __builtin_amdgcn_exp2f(m[i] - M) : 0.f;
-            Lsum += on ? w * l[i] : 0.f;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                acc[4 * k + 0] += on ? w * po[i][k].x : 0.f;
-                acc[4 * k + 1] += on ? w * po[i][k].y : 0.f;
-                acc[4 * k + 2] += on ? w * po[i][k].z : 0.f;
-                acc[4 * k + 3] += on ? w * po[i][k].w : 0.f;
-            }
-        }
+            for (int k = 0; k < 4; ++k) asm volatile("s_waitcnt vmcnt(0)" : "+v"(po[i][k]) :: "memory");
+        F.take4(m, l, po, nv - i0);
     }
-    const float inv = Lsum > 0.f ? 1.0f / Lsum : 0.f;   // no valid key at all (every page id invalid): zeros, like a context of 0
+    const float inv = F.inverse();
     typedef typename Elem16<E>::vec8 vec8;
     __bf16* dst = P.o + (int64_t)b * P.o_sb + (int64_t)(qt * kQTile + s) * P.o_ss + (int64_t)hq * P.o_sh + c * 16;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         vec8 out;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) out[e] = (E)(acc[8 * h + e] * inv);
+        for (int e = 0; e < 8; ++e) out[e] = (E)(F.acc[8 * h + e] * inv);
         *reinterpret_cast<vec8*>(dst + 8 * h) = out;
     }
 }
@@ -234,27 +226,21 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
         auto splits_of_lane = [&]() { return lane < P.bs ? max(1, (ctx_l + span - 1) / span) : 0; };   // (padding rows get one)
         int n;
         if (P.fit_slots > 0) {
-            // Tables emptier than assumed: start from the split that would fill the chip, total / (resident workgroups
-            // per head group - a remainder of half a split per sequence) -- at least 512 keys (256 where even pieces
-            // that short leave half of the chip's workgroup slots empty: a launch that small is a chain of
-            // latencies, and the chain is as long as its longest workgroup), no more pieces per sequence than the
-            // launch has room for, and not so many that the combine pass, which walks a sequence's pieces four at a
-            // time, costs more than shorter pieces save (0.6 us per piece against 0.022 us per key of the longest
-            // workgroup: pieces of sqrt(27.6 x longest) keys balance the two; a sequence of tens of thousands of
-            // keys grows its split by the same rule).  A sequence that the host's split leaves whole is only cut
-            // if that takes 256 keys or more off the longest workgroup (what the combine pass and the partials cost).
-            // (Quotients by reciprocal: an estimate is all that is needed, and every workgroup makes the same one;
-            // the "+ 1" keeps the longest sequence within nsplit pieces whatever the rounding.)
+            // One size of piece for all sequences.  A launch of few keys is a chain of latencies as long as its longest
+            // workgroup, one of many keys a stream that more and shorter workgroups only disturb: over batches of 1 to 20
+            // sequences and contexts of 300 to 16 000 keys the best size follows 4 sqrt(total keys) up to 512 (300 keys: 64,
+            // 1100: 128, 4 x 1100: 192 to 256, 8 x 1100: 384, 16 x 1100, 4 x 8000: 512).  At least what fills the chip once, total / (resident
+            // workgroups per head group - a remainder of half a piece per sequence), and no more pieces of a sequence than
+            // the launch has room for (the "+ 1" keeps the longest within nsplit pieces whatever the rounding of the
+            // reciprocals; every workgroup makes the same estimate).  Sequences are only cut if that takes more off the longest
+            // workgroup than the partials of them all cost (8 x 300 and 16 x 600 keys stay whole).
             const int total = wave_sum(ctx_l), longest = wave_max(ctx_l), live = wave_sum(ctx_l > 0 ? 1 : 0);
             const float per_group = (float)P.fit_slots * __builtin_amdgcn_rcpf((float)gridDim.x);      // resident workgroups per head group and query tile
             const float room = fmaxf(1.f, per_group - 0.5f * (float)live);
-            const float least = (float)total * (1.f / 256.f) + (float)live <= 0.5f * per_group ? 256.f : 512.f;
-            const float depth = __builtin_amdgcn_sqrtf(27.6f * (float)longest);
-            const float want = fmaxf(fmaxf(least, (float)total * __builtin_amdgcn_rcpf(room)),
-                                     fmaxf((float)longest * __builtin_amdgcn_rcpf((float)P.nsplit) + 1.f, depth));
-            const int fill = ((int)want + 63) & ~63;
-            if (min(longest, span) - fill >= (longest > span ? 64 : 256)) span = fill;
-            span = max(span, ((int)depth + 63) & ~63);
+            const int best = min(512, ((int)(4.f * __builtin_amdgcn_sqrtf((float)total)) + 32) & ~63);
+            const float least = fmaxf((float)total * __builtin_amdgcn_rcpf(room), (float)longest * __builtin_amdgcn_rcpf((float)P.nsplit) + 1.f);
+            span = max(max(64, best), ((int)least + 63) & ~63);
+            if (longest - span < 64 + 12 * live) span = max(span, longest);
             n = splits_of_lane();
             // a tile more per step (24 steps double the smallest split); a few workgroups beyond what is resident
             // may stay: the last to start are remainders, which fill the tail
@@ -491,13 +477,12 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
             }
         }
         if (kw == 0 && H == 0) {
-            float* ml = P.part_ml + (slot * 2 + 0) * kQTile + r;
+            float* ml = P.part_ml + (slot * kQTile + r) * 2;
             if (P.arrive) {
                 __hip_atomic_store(ml, st.m[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(ml + kQTile, st.l[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(ml + 1, st.l[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             } else {
-                ml[0] = st.m[0];
-                ml[kQTile] = st.l[0];
+                *reinterpret_cast<float2*>(ml) = float2{st.m[0], st.l[0]};
             }
         }
     }
@@ -517,27 +502,68 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
     if (!i_am_last) return;
     for (int e = tid; e < HPW * 256; e += kThreads) {
         const int s = (e & 255) >> 3;
-        if (qt * kQTile + s < P.sq) combine_query<E, true>(P, b, hg * HPW + (e >> 8), qt, s, e & 7, [&]() { return n_valid_splits; });
+        if (qt * kQTile + s < P.sq) combine_query<E>(P, b, hg * HPW + (e >> 8), qt, s, e & 7, n_valid_splits);
     }
     if (tid == 0) __hip_atomic_store(counter, 0.f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // ready for the next launch
 }
 
-// One workgroup per (sequence, head): merges the split partials of its 32 queries; thread t takes
-// 16 consecutive d values of query t / 8.  A sequence that was not split leaves after one load, and
-// there are only bs * Hq workgroups to launch, which is what the common case costs when the
-// attention kernel decided that nothing had to be cut.  The kernel is a chain of memory latencies
-// (length -> partials -> output), not of bytes: the loads of four splits are issued together.
-template <typename E>
+// Folds the split partials: a workgroup takes 8 QUERIES queries of a (sequence, head), a thread four columns of QUERIES of them.  The
+// kernel is a chain of memory latencies (length -> partials -> output), not of bytes: the loads of the first slots are
+// on their way before the lengths say how many of them exist (where a slot lies does not depend on it; what lies
+// beyond is masked out), and a thread's share of a slot is one load.  Few heads (QUERIES = 1) get eight slots in flight and
+// more workgroups; with more of them there are workgroups enough, fewer pieces per sequence, and the workgroups of whole
+// sequences, which leave at once, still have to be launched.  (A workgroup per head with 16 columns per thread, the form this
+// replaced, took 0.6 us per four pieces of a sequence, which kept the pieces long.)
+template <typename E, int QUERIES>
 __global__ __launch_bounds__(256) void paged_combine_kernel(const PagedParams P)
 {
-    const int qt = blockIdx.x % P.nqt, hq = (blockIdx.x / P.nqt) % P.num_q_heads, b = blockIdx.x / P.nqt / P.num_q_heads;
-    const int s = threadIdx.x >> 3, c = threadIdx.x & 7;
-    if (qt * kQTile + s >= P.sq) return;
-    combine_query<E, false>(P, b, hq, qt, s, c, [&]() {
-        const int ctx = min(P.context_lens[b], P.max_pages * P.page_size);
-        const int span = P.span_out ? (int)*P.span_out : P.chunk;     // the attention kernel's choice
-        return (ctx + span - 1) / span;
-    });
+    constexpr int kAhead = 8 / QUERIES, kParts = 4 / QUERIES;
+    const int part = blockIdx.x % kParts, rest = blockIdx.x / kParts;
+    const int qt = rest % P.nqt, hq = (rest / P.nqt) % P.num_q_heads, b = rest / P.nqt / P.num_q_heads;
+    const int c = (threadIdx.x & 31) * 4, s0 = part * 8 * QUERIES + (threadIdx.x >> 5);         // queries s0, s0 + 8
+    if (c >= P.head_dim || qt * kQTile + s0 >= P.sq) return;
+    const int64_t slot0 = (((int64_t)b * P.num_q_heads + hq) * P.nqt + qt) * P.nsplit;
+    const float* part_o = P.part_o + (slot0 * kQTile + s0) * kHeadDim + c;
+    const float2* part_ml = reinterpret_cast<const float2*>(P.part_ml) + slot0 * kQTile + s0;
+    int nv = P.nsplit;                         // until the lengths are in: every slot that exists
+    Fold<4> F[QUERIES];
+#pragma unroll
+    for (int q = 0; q < QUERIES; ++q) F[q].init();
+    for (int i0 = 0; i0 < nv; i0 += kAhead) {
+        float m[QUERIES][kAhead / 4][4], l[QUERIES][kAhead / 4][4];
+        f32x4 po[QUERIES][kAhead / 4][4][1];
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i)
+#pragma unroll
+            for (int q = 0; q < QUERIES; ++q) {
+                const int slot = min(i0 + i, P.nsplit - 1);
+                const float2 ml = part_ml[slot * kQTile + 8 * q];
+                m[q][i / 4][i % 4] = ml.x;
+                l[q][i / 4][i % 4] = ml.y;
+                po[q][i / 4][i % 4][0] = *reinterpret_cast<const f32x4*>(part_o + ((int64_t)slot * kQTile + 8 * q) * kHeadDim);
+            }
+        if (i0 == 0) {
+            const int ctx = min(P.context_lens[b], P.max_pages * P.page_size);
+            const int span = P.span_out ? (int)*P.span_out : P.chunk;     // the attention kernel's choice
+            nv = (ctx + span - 1) / span;
+            if (nv <= 1) return;               // written directly by the attention kernel
+        }
+#pragma unroll
+        for (int g = 0; g < kAhead / 4; ++g)
+#pragma unroll
+            for (int q = 0; q < QUERIES; ++q)
+                if (i0 + 4 * g < nv) F[q].take4(m[q][g], l[q][g], po[q][g], nv - i0 - 4 * g);
+    }
+#pragma unroll
+    for (int q = 0; q < QUERIES; ++q) {
+        const int s = s0 + 8 * q;
+        if (qt * kQTile + s >= P.sq) return;
+        const float inv = F[q].inverse();
+        typename Elem16<E>::vec4 out;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) out[e] = (E)(F[q].acc[e] * inv);
+        *reinterpret_cast<typename Elem16<E>::vec4*>(P.o + (int64_t)b * P.o_sb + (int64_t)(qt * kQTile + s) * P.o_ss + (int64_t)hq * P.o_sh + c) = out;
+    }
 }
 
 // Keys per split.  Measured over batches of 4 to 64 sequences and contexts of 300 to 8000 keys, the
@@ -575,9 +601,20 @@ int pick_chunk(int bs, int head_groups, int max_pages, int page_size, bool* devi
     return (int)chunk;
 }
 
-int nsplit_of(int max_pages, int page_size, int chunk) {
+// Partial slots per sequence: what the host's split needs and, where the kernel cuts by the lengths (up to 64 sequences, not
+// device_span), what its own choice of 4 sqrt(total keys) can need, sqrt(longest) / 4 (beyond 16 K keys the pieces grow) -- as far as that keeps the launch's partials
+// below 17 MB (1024 slots).
+int nsplit_of(int bs, int64_t heads_and_tiles, int max_pages, int page_size, int chunk, bool device_span) {
     const int64_t max_keys = (int64_t)max_pages * page_size;
-    return (int)((max_keys + chunk - 1) / chunk);
+    const int64_t n = (max_keys + chunk - 1) / chunk;
+    if (device_span || bs > 64) return (int)n;
+    // sequences that the kernel would leave whole even in tables that are 65 % full need no slots, and no combine launch
+    const double longest = 0.65 * (double)max_keys, best = 4.0 * sqrt(longest * bs);
+    if (n == 1 && longest - (best > 64.0 ? best : 64.0) < 64.0 + 12.0 * bs) return 1;
+    int64_t own = 2;
+    while ((own - 1) * (own - 1) * 16 < max_keys) ++own;
+    if (own > 1024 / (bs * heads_and_tiles)) own = 1024 / (bs * heads_and_tiles);
+    return (int)(own > n ? own : n);
 }
 
 }  // namespace
@@ -593,7 +630,7 @@ extern "C" int64_t mdx_paged_block_attn_workspace_bytes(int32_t bs, int32_t sq, 
     const int nqt = sq <= kQTile ? 1 : (sq + kQTile - 1) / kQTile;
     bool device_span;
     const int chunk = pick_chunk(bs, num_q_heads / HPW * nqt, max_pages, page_size, &device_span);
-    const int nsplit = nsplit_of(max_pages, page_size, chunk);
+    const int nsplit = nsplit_of(bs, (int64_t)num_q_heads * nqt, max_pages, page_size, chunk, device_span);
     if (nsplit <= 1) return 0;
     return (int64_t)bs * num_q_heads * nqt * nsplit * kQTile * (kHeadDim + 2) * (int64_t)sizeof(float) + 16;   // + the split size
 }
@@ -665,7 +702,7 @@ int launch_paged(const void* q, void* o, const void* k_cache, const void* v_cach
     const int64_t wg_per_pair = (int64_t)(num_q_heads / HPW) * P.nqt;               // workgroups of one (sequence, split)
     const int cus = cu_count();
     P.chunk = pick_chunk(bs, (int)wg_per_pair, max_pages, page_size, &device_span);
-    P.nsplit = nsplit_of(max_pages, page_size, P.chunk);
+    P.nsplit = nsplit_of(bs, (int64_t)num_q_heads * P.nqt, max_pages, page_size, P.chunk, device_span);
     P.num_q_heads = num_q_heads;
     P.head_dim = head_dim;
     P.c = scale * kLog2e;
@@ -706,7 +743,7 @@ int launch_paged(const void* q, void* o, const void* k_cache, const void* v_cach
     // CU that holds a single workgroup still has two wavefronts per SIMD (batch 32 x 8 KV heads: 79 -> 69 us
     // on equal lengths); with more pairs than CUs the second round costs more than that gains.
     const bool eight = device_span && (int64_t)bs * wg_per_pair <= cus;
-    const unsigned n_combine = (unsigned)(bs * num_q_heads * P.nqt);
+    const unsigned n_heads = (unsigned)(bs * num_q_heads * P.nqt);
     const bool two_launches = P.nsplit > 1 && !P.arrive;
     if (dtype == MDX_F16) {
         if (HPW == 2 && eight) paged_block_attn_kernel<_Float16, 2, 2, 8><<<grid, 512, 0, stream>>>(P);
@@ -719,8 +756,9 @@ int launch_paged(const void* q, void* o, const void* k_cache, const void* v_cach
     }
     int rc = mdx::check_launch("paged_block_attn");
     if (rc != MDX_OK || !two_launches) return rc;
-    if (dtype == MDX_F16) paged_combine_kernel<_Float16><<<n_combine, 256, 0, stream>>>(P);
-    else                  paged_combine_kernel<__bf16><<<n_combine, 256, 0, stream>>>(P);
+    const bool few = n_heads <= 128;
+    if (dtype == MDX_F16) { if (few) paged_combine_kernel<_Float16, 1><<<4 * n_heads, 256, 0, stream>>>(P); else paged_combine_kernel<_Float16, 2><<<2 * n_heads, 256, 0, stream>>>(P); }
+    else                  { if (few) paged_combine_kernel<__bf16, 1><<<4 * n_heads, 256, 0, stream>>>(P);   else paged_combine_kernel<__bf16, 2><<<2 * n_heads, 256, 0, stream>>>(P); }
     return mdx::check_launch("paged_combine");
 }
 
