@@ -17,8 +17,8 @@
 //    four lanes of a row cover a line with two loads.
 //
 // QKV (4096 x 2048), output (2048 x 2048), gate/up (12288 x 2048, with SiLU) and down (2048 x 6144) projections, cold weights, us, as
-// here / library product (+ SiLU kernel): 32 rows 6.5 4.8 14.9 8.6 / 11.7 8.4 18.8 16.6, 64 rows 7.8 5.7 17.6 10.0 / 12.1 8.8
-// 20.3 19.4, 128 rows 10.2 7.4 23.9 12.6 / 14.8 8.4 22.3 17.8.  Beyond 128 rows the library's tiles win (256 rows: 15 10 37 20 /
+// here / library product (+ SiLU kernel): 32 rows 6.5 4.6 15.2 8.6 / 11.7 8.4 18.8 16.6, 64 rows 7.8 5.2 17.9 10.0 / 12.1 8.8
+// 20.3 19.4, 128 rows 10.0 6.8 23.7 12.5 / 14.8 8.4 22.3 17.8.  Beyond 128 rows the library's tiles win (256 rows: 15 10 37 20 /
 // 14 10 31 23), for gate/up beyond 64.  Bound: the HBM read of W, about 4.5 TB/s in bursts this short, behind 3 us of launch.
 #include "mdx_common.h"
 #include <atomic>
@@ -81,7 +81,7 @@ __global__ __launch_bounds__(64 * WN * WK, 1) void decode_linear_kernel(const Li
         for (int p = 0; p < kPairs; ++p)
 #pragma unroll
             for (int h = 0; h < 2; ++h)
-                w[p][h] = __builtin_bit_cast(bf16x8, __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wp + t * KC + p * 64 + h * 8)));
+                w[p][h] = *reinterpret_cast<const bf16x8*>(wp + t * KC + p * 64 + h * 8);
     };
     f32x4 acc[MT];
 #pragma unroll

@@ -13,10 +13,12 @@
 // vocab tile sit 8 workgroups apart, so that the dispatcher, which deals consecutive workgroups round-robin
 // to the 8 XCDs, puts them on the same XCD next to each other in time and its L2 fetches that tile of W from
 // HBM once.
-#include "mdx_common.h"
+#include "lm_head.h"
 #include <atomic>
 
 namespace {
+
+using namespace mdx_head;
 
 #include "lm_head_core.inc"
 
@@ -24,20 +26,7 @@ constexpr int kThreads = 256;
 constexpr int kTile = 256;                     // vocab rows and x rows per workgroup
 constexpr int kSlice = 128;                    // vocab rows per record (one wavefront's share)
 constexpr int kLdsBytes = 2 * 2 * kTile * 128; // two stages of (W tile + x tile), 128-byte rows
-constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kClamp = -1.0e30f;
-
-struct Record { float m, s; int idx, pad; };   // max logit, sum of exp2((x - m) c), first index of the max
-
-struct LmHeadParams {
-    const __bf16* x; const __bf16* w;
-    int64_t x_stride, w_stride;                // elements between rows
-    const float* temperatures; int rows_per_temp; const int64_t* row_ids;
-    int rows, vocab, hidden;
-    int n_row_tiles, n_vocab_tiles, n_slices;
-    Record* records;                           // [rows, n_slices]
-    int64_t* x0; float* x0_p;
-};
 
 // 32-bit LDS byte address of a pointer into shared memory (what ds_* instructions and M0 take).
 typedef __attribute__((address_space(3))) char lds_char;
@@ -48,12 +37,6 @@ __device__ __forceinline__ const void* uniform(const void* p) {
     const uint64_t v = (uint64_t)p;
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
     return (const void*)(((uint64_t)hi << 32) | lo);
-}
-
-__device__ __forceinline__ float row_scale(const LmHeadParams& P, int row) {
-    if (!P.temperatures || row >= P.rows) return kLog2e;
-    const int64_t id = P.row_ids ? P.row_ids[row] : row;
-    return kLog2e / P.temperatures[id / P.rows_per_temp];
 }
 
 __global__ __launch_bounds__(kThreads, 1) void lm_head_confidence_kernel(const LmHeadParams P)
@@ -150,6 +133,23 @@ __global__ __launch_bounds__(kThreads) void lm_head_finalize_kernel(const LmHead
 
 int slices_of(int64_t vocab) { return (int)((vocab + kTile - 1) / kTile) * (kTile / kSlice); }
 
+int launch_tiles(const LmHeadParams& P, hipStream_t stream)
+{
+    // the kernel's LDS limit is raised once per device
+    static std::atomic<bool> lds_limit_raised[64];
+    int device = 0;
+    hipError_t e = hipGetDevice(&device);
+    MDX_REQUIRE(e == hipSuccess && device >= 0 && device < 64, MDX_ELAUNCH, "lm_head_confidence: no current device (%s)", hipGetErrorString(e));
+    if (!lds_limit_raised[device].load(std::memory_order_acquire)) {
+        e = hipFuncSetAttribute(reinterpret_cast<const void*>(lm_head_confidence_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+        MDX_REQUIRE(e == hipSuccess, MDX_ELAUNCH, "lm_head_confidence: cannot reserve %d bytes of LDS (%s)", kLdsBytes, hipGetErrorString(e));
+        lds_limit_raised[device].store(true, std::memory_order_release);
+    }
+    const int64_t grid = (int64_t)((P.n_vocab_tiles + 7) / 8) * 8 * P.n_row_tiles;
+    lm_head_confidence_kernel<<<(unsigned)grid, kThreads, kLdsBytes, stream>>>(P);
+    return mdx::check_launch("lm_head_confidence");
+}
+
 }  // namespace
 
 extern "C" int64_t mdx_lm_head_confidence_workspace_bytes(int64_t rows, int64_t vocab)
@@ -194,19 +194,8 @@ extern "C" int mdx_lm_head_confidence(const void* x, int64_t x_row_stride, const
     P.records = static_cast<Record*>(workspace);
     P.x0 = x0; P.x0_p = x0_p;
 
-    // the kernel's LDS limit is raised once per device
-    static std::atomic<bool> lds_limit_raised[64];
-    int device = 0;
-    hipError_t e = hipGetDevice(&device);
-    MDX_REQUIRE(e == hipSuccess && device >= 0 && device < 64, MDX_ELAUNCH, "lm_head_confidence: no current device (%s)", hipGetErrorString(e));
-    if (!lds_limit_raised[device].load(std::memory_order_acquire)) {
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(lm_head_confidence_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
-        MDX_REQUIRE(e == hipSuccess, MDX_ELAUNCH, "lm_head_confidence: cannot reserve %d bytes of LDS (%s)", kLdsBytes, hipGetErrorString(e));
-        lds_limit_raised[device].store(true, std::memory_order_release);
-    }
-    const int64_t grid = (int64_t)((P.n_vocab_tiles + 7) / 8) * 8 * P.n_row_tiles;
-    lm_head_confidence_kernel<<<(unsigned)grid, kThreads, kLdsBytes, stream>>>(P);
-    int rc = mdx::check_launch("lm_head_confidence");
+    // up to 128 rows the tiles of 256 rows are mostly padding
+    const int rc = few_rows_covered(rows, hidden) ? launch_few_rows(P, stream) : launch_tiles(P, stream);
     if (rc != MDX_OK) return rc;
     lm_head_finalize_kernel<<<(unsigned)((rows + kThreads / 64 - 1) / (kThreads / 64)), kThreads, 0, stream>>>(P);
     return mdx::check_launch("lm_head_finalize");

@@ -650,9 +650,9 @@ class BlockDiffusionEngine:
 
     def _fused_head(self, rows: int) -> bool:
         """Projection and confidence in one pass that never writes the logits (mdx_lm_head_confidence): taken where it
-        is the faster of the two (from a few hundred rows on; below that the library GEMM + the vocabulary pass
-        win), for bf16 weights without sampling noise."""
-        return (self.fused_head and self.gumbel_seed is None and rows >= self.fused_head_min_rows
+        is the faster of the two (from a few hundred rows on, and up to 256 rows: one tile of the kernel, or its form for
+        up to 128; between them the library GEMM + the vocabulary pass win), for bf16 weights without sampling noise."""
+        return (self.fused_head and self.gumbel_seed is None and (rows <= 256 or rows >= self.fused_head_min_rows)
                 and self.model.lm_head.dtype == torch.bfloat16 and self.model.lm_head.shape[1] % 128 == 0)
 
     def _draw(self, g, rows):

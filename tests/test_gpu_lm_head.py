@@ -115,3 +115,21 @@ def test_lm_head_confidence_when_the_last_vocab_tile_holds_one_entry(dev, vocab,
     ex0, ep, logits = _reference(x, w, temps.numpy(), rows, None)
     _check(x0, p, ex0, ep, logits, T=np.full(rows, T))
     assert vocab == 1 or (x0 == vocab - 1).any()
+
+
+@pytest.mark.parametrize("rows", [1, 16, 31, 32, 33, 64, 65, 127, 128])
+@pytest.mark.parametrize("vocab,hidden", [(1, 512), (127, 512), (129, 1024), (5003, 2048), (33000, 512), (3000, 2560), (700, 768)])
+def test_lm_head_confidence_of_few_rows(dev, rows, vocab, hidden):
+    """The forms for up to 128 rows: edges of the row tiles and of the vocabulary tiles, less and more than one tile per
+    workgroup, x whole in LDS and step by step, with temperatures."""
+    import mdx
+    g = torch.Generator().manual_seed(rows + vocab)
+    x = torch.randn(rows, hidden, generator=g).bfloat16()
+    w = (torch.randn(vocab, hidden, generator=g) * (3.0 / hidden ** 0.5)).bfloat16()
+    temps = 0.5 + torch.rand(rows, generator=g)
+    padded = torch.zeros(rows, hidden + 8, dtype=torch.bfloat16, device=dev)
+    padded[:, :hidden] = x.to(dev)
+    x0, p = mdx.lm_head_confidence(padded[:, :hidden], w.to(dev), temps.to(dev))
+    torch.cuda.synchronize()
+    ex0, ep, logits = _reference(x, w, temps)
+    _check(x0, p, ex0, ep, logits, temps)
