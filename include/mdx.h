@@ -115,6 +115,23 @@ int mdx_staircase_attn_varlen(const void* q, const void* k, const void* v, void*
                               mdx_stream_t stream);
 
 /*
+ * mdx_store_kvcache of k and v (dense rows, one slot per token) and mdx_staircase_attn_varlen, in either order: the two halves of
+ * the attention layer's prefill (engines/nano_dvlm/nanovllm/layers/sdar_attention.py:37-47), which do not depend on each
+ * other.  One launch where the prompts are short (up to 560 tokens, 16-bit tensors), else two.
+ */
+int mdx_staircase_attn_store(const void* q, const void* k, const void* v, void* o,
+                             int64_t q_stride_t, int64_t q_stride_h,
+                             int64_t k_stride_t, int64_t k_stride_h,
+                             int64_t v_stride_t, int64_t v_stride_h,
+                             int64_t o_stride_t, int64_t o_stride_h,
+                             const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                             int32_t batch, int32_t max_seqlen, int64_t total_tokens,
+                             int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                             int32_t staircase_size, float scale, int32_t dtype,
+                             void* k_cache, void* v_cache, const int32_t* slot_mapping, int64_t num_slots,
+                             mdx_stream_t stream);
+
+/*
  * Paged single-block ("decode") attention -- replaces the call
  * flash_attn_with_kvcache(q, k_cache, v_cache, cache_seqlens=, block_table=,
  * softmax_scale=, causal=False) of

@@ -138,9 +138,8 @@ Tensor token_rows(const Tensor& t) {
     return t.flatten(0, 1);
 }
 
-void store(const Tensor& key4, const Tensor& value4, const Tensor& k_cache, const Tensor& v_cache, const Tensor& slot_mapping, void* stream) {
-    need_gpu({&key4, &value4, &k_cache, &v_cache, &slot_mapping});
-    const Tensor key = token_rows(key4), value = token_rows(value4);
+// What store() asks of its arguments; the slots as a dense int32 tensor.
+Tensor check_store(const Tensor& key, const Tensor& value, const Tensor& k_cache, const Tensor& v_cache, const Tensor& slot_mapping) {
     NEED(key.dim() == 3 && value.dim() == 3);
     const int64_t N = key.size(0), heads = key.size(1), d = key.size(2), D = heads * d;
     NEED(key.stride(2) == 1 && value.stride(2) == 1);
@@ -149,7 +148,14 @@ void store(const Tensor& key4, const Tensor& value4, const Tensor& k_cache, cons
     NEED(slot_mapping.numel() == N);
     NEED(key.scalar_type() == value.scalar_type() && key.scalar_type() == k_cache.scalar_type() && key.scalar_type() == v_cache.scalar_type());
     NEED(k_cache.is_contiguous() && v_cache.is_contiguous());
-    const Tensor slots = int32_list(slot_mapping, "slot_mapping");
+    return int32_list(slot_mapping, "slot_mapping");
+}
+
+void store(const Tensor& key4, const Tensor& value4, const Tensor& k_cache, const Tensor& v_cache, const Tensor& slot_mapping, void* stream) {
+    need_gpu({&key4, &value4, &k_cache, &v_cache, &slot_mapping});
+    const Tensor key = token_rows(key4), value = token_rows(value4);
+    const Tensor slots = check_store(key, value, k_cache, v_cache, slot_mapping);
+    const int64_t N = key.size(0), D = key.size(1) * key.size(2);
     check(mdx_store_kvcache(ptr(key), ptr(value), key.stride(0), value.stride(0), ptr(k_cache), ptr(v_cache),
                             static_cast<const int32_t*>(ptr(slots)), N, D, (int32_t)key.element_size(), k_cache.numel() / D, stream),
           "store_kvcache");
@@ -345,9 +351,10 @@ PyObject* qk_norm_rope_store_partials(PyObject*, PyObject* const* a, Py_ssize_t 
 }
 
 // ---- staircase prefill ------------------------------------------------------------------------------
-// The result as [N, Hq, d], or flattened to [N, Hq * d].
+// The result as [N, Hq, d], or flattened to [N, Hq * d].  With caches, k and v are stored into them too.
+struct Caches { const Tensor &k, &v, &slot_mapping; };
 Tensor staircase(const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& cu_q_, const Tensor& cu_k_, int64_t S, int64_t max_seqlen,
-                 PyObject* scale, bool flat) {
+                 PyObject* scale, bool flat, const Caches* caches = nullptr) {
     need_gpu({&q_, &k_, &v_, &cu_q_, &cu_k_});
     NEED(q_.dim() == 3 && k_.dim() == 3 && v_.dim() == 3);
     NEED(q_.size(0) == k_.size(0) && q_.size(0) == v_.size(0));
@@ -361,10 +368,20 @@ Tensor staircase(const Tensor& q_, const Tensor& k_, const Tensor& v_, const Ten
     const Tensor q = q_.stride(2) == 1 ? q_ : q_.contiguous(), k = k_.stride(2) == 1 ? k_ : k_.contiguous(), v = v_.stride(2) == 1 ? v_ : v_.contiguous();
     Tensor o = flat ? make(q, q.scalar_type(), total, hq * d) : make(q, q.scalar_type(), total, hq, d);
     const Tensor cu_q = int32_list(cu_q_, "cu_seqlens_q"), cu_k = int32_list(cu_k_, "cu_seqlens_k");
-    check(mdx_staircase_attn_varlen(ptr(q), ptr(k), ptr(v), ptr(o), q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
-                                    hq * d, d, static_cast<const int32_t*>(ptr(cu_q)), static_cast<const int32_t*>(ptr(cu_k)),
-                                    (int32_t)(cu_k.numel() - 1), (int32_t)(max_seqlen > 0 ? max_seqlen : total), total, (int32_t)hq, (int32_t)hkv,
-                                    (int32_t)d, (int32_t)S, scale_or_default(scale, d), dtype_of(q), stream_of(q)),
+    auto call = [&](auto fn, auto... more) {
+        return fn(ptr(q), ptr(k), ptr(v), ptr(o), q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1), hq * d, d,
+                  static_cast<const int32_t*>(ptr(cu_q)), static_cast<const int32_t*>(ptr(cu_k)), (int32_t)(cu_k.numel() - 1),
+                  (int32_t)(max_seqlen > 0 ? max_seqlen : total), total, (int32_t)hq, (int32_t)hkv, (int32_t)d, (int32_t)S, scale_or_default(scale, d),
+                  dtype_of(q), more...);
+    };
+    if (caches) {
+        need_gpu({&caches->k, &caches->v, &caches->slot_mapping});
+        const Tensor slots = check_store(k_, v_, caches->k, caches->v, caches->slot_mapping);
+        check(call(mdx_staircase_attn_store, ptr(caches->k), ptr(caches->v), static_cast<const int32_t*>(ptr(slots)), caches->k.numel() / (hkv * d), stream_of(q)),
+              "attention");
+        return o;
+    }
+    check(call(mdx_staircase_attn_varlen, stream_of(q)),
           "sparse_attn_varlen");
     return o;
 }
@@ -452,7 +469,7 @@ PyObject* flash_attn_with_kvcache(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // The prefill store runs beside the attention launch, on one extra stream per device (default priority), from this many
 // tokens on: its small workgroups fill the gaps between the attention kernel's, which own whole CUs (38 690 tokens,
 // store + attention: 0.820 -> 0.808 ms).  Two event records and two waits, 8 us of host time and as much of the GPU's
-// between the launches, are what that costs, so short prompts store on the caller's stream.
+// between the launches, are what that costs, so fewer tokens are stored on the caller's stream (short prompts in the attention launch).
 constexpr int64_t kSideStoreTokens = 16384;
 
 struct Side {
@@ -483,25 +500,25 @@ PyObject* attention_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const Tensor &q = tensor(a[0]), &k = tensor(a[1]), &v = tensor(a[2]), &k_cache = tensor(a[3]), &v_cache = tensor(a[4]);
         const bool have_cache = k_cache.numel() > 0 && v_cache.numel() > 0;
         need_gpu({&q});
-        Side* side = nullptr;
-        hipStream_t main = static_cast<hipStream_t>(stream_of(q));
-        if (have_cache) {
-            hipStream_t stream = main;
-            if (q.dim() == 3 && q.size(0) >= kSideStoreTokens) {
-                side = side_of(q.device().index());
-                chain(main, side->fork, side->stream);
-                stream = side->stream;
-            }
-            store(k, v, k_cache, v_cache, tensor(a[5]), stream);
+        const Tensor &cu_q = tensor(a[6]), &cu_k = tensor(a[7]);
+        const int64_t S = integer(a[8]), max_seqlen = integer(a[9]);
+        if (!have_cache) return wrap(staircase(q, k, v, cu_q, cu_k, S, max_seqlen, a[10], true));
+        if (q.dim() != 3 || q.size(0) < kSideStoreTokens) {
+            const Caches caches{k_cache, v_cache, tensor(a[5])};
+            return wrap(staircase(q, k, v, cu_q, cu_k, S, max_seqlen, a[10], true, &caches));
         }
+        Side* side = side_of(q.device().index());
+        hipStream_t main = static_cast<hipStream_t>(stream_of(q));
+        chain(main, side->fork, side->stream);
         Tensor o;
         try {
-            o = staircase(q, k, v, tensor(a[6]), tensor(a[7]), integer(a[8]), integer(a[9]), a[10], true);
+            store(k, v, k_cache, v_cache, tensor(a[5]), side->stream);
+            o = staircase(q, k, v, cu_q, cu_k, S, max_seqlen, a[10], true);
         } catch (...) {
-            if (side) chain(side->stream, side->join, main);
+            chain(side->stream, side->join, main);
             throw;
         }
-        if (side) chain(side->stream, side->join, main);
+        chain(side->stream, side->join, main);
         return wrap(std::move(o));
     });
 }

@@ -37,6 +37,19 @@ constexpr int kThreads = 256;      // 4 wavefronts, 2 workgroups per CU
 constexpr int kRowsPerWg = 128;    // 4 wavefronts x 32 query rows
 constexpr int kTileBytes = kTileKeys * kLdsPitch;
 
+// The K/V rows of a short prompt's layer go to the paged cache in the attention launch itself (mdx_staircase_attn_store): the
+// attention reads k and v, not the cache, so the rows are copied by workgroups behind the attention's, which find the chip
+// far from full (109 tokens are 16 attention workgroups), and the launch of the store, 2.4 us of an 11-us layer, is saved.
+constexpr int kStoreTokens = 16;                               // tokens per workgroup at most: 16 loads of 16 bytes in flight per lane
+struct StoreParams {
+    const u32x4* key; const u32x4* value;
+    int64_t k_stride16, v_stride16;                            // 16-byte units between tokens
+    u32x4* k_cache; u32x4* v_cache;
+    const int32_t* slot_mapping; int64_t num_slots;
+    int n_tokens, row16, tokens_per_wg;                        // row16: 16-byte units of a token's row, a divisor of kThreads / 2
+    int first_wg;                                              // workgroups from here on copy rows
+};
+
 struct StaircaseParams {
     const __bf16* q; const __bf16* k; const __bf16* v; __bf16* o;
     int64_t q_st, q_sh, k_st, k_sh, v_st, v_sh, o_st, o_sh;   // element strides: token, head
@@ -47,7 +60,31 @@ struct StaircaseParams {
     int head_dim;                                              // <= 128, a multiple of 16
     int o_rows16;                                              // rows of o take 16-byte stores (aligned, strides multiples of 8 elements)
     float c;                                                   // scale * log2(e)
+    StoreParams store;
 };
+
+// Workgroup `wg` of the store: half of the lanes take K rows, half V rows.
+__device__ __forceinline__ void store_rows(const StoreParams& S, int wg, int tid)
+{
+    const bool is_v = tid >= kThreads / 2;
+    const int lane = tid & (kThreads / 2 - 1), at_once = kThreads / 2 / S.row16;              // rows that half of the lanes cover
+    const int sub = lane / S.row16, col = lane % S.row16;
+    const int begin = wg * S.tokens_per_wg, end = min(S.n_tokens, begin + S.tokens_per_wg);
+    const u32x4* src = is_v ? S.value : S.key;
+    const int64_t stride = is_v ? S.v_stride16 : S.k_stride16;
+    u32x4* cache = is_v ? S.v_cache : S.k_cache;
+    u32x4 row[kStoreTokens];
+    int64_t slot[kStoreTokens];
+#pragma unroll
+    for (int i = 0; i < kStoreTokens; ++i) {
+        const int t = begin + i * at_once + sub;
+        slot[i] = t < end ? S.slot_mapping[t] : -1;
+        if (t < end) row[i] = __builtin_nontemporal_load(src + t * stride + col);
+    }
+#pragma unroll
+    for (int i = 0; i < kStoreTokens; ++i)
+        if (slot[i] >= 0 && slot[i] < S.num_slots) __builtin_nontemporal_store(row[i], cache + slot[i] * S.row16 + col);
+}
 
 // Sequence b's first token and length.  Bounds that do not describe a range inside the packed
 // tensors (decreasing, negative, past total_tokens) are clipped to one, so that no row outside
@@ -178,6 +215,8 @@ __global__ __launch_bounds__(kThreads, 2) void staircase_attn_kernel(const Stair
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int H = lane >> 5, r = lane & 31;
+
+    if ((int)blockIdx.x >= P.store.first_wg) { store_rows(P.store, (int)blockIdx.x - P.store.first_wg, tid); return; }
 
     // ---- workgroup -> (head slot, sequence b, row group rg) ------------------------------------
     const int hslot = blockIdx.x % P.num_q_heads;
@@ -434,7 +473,10 @@ int launch_staircase_f32(const void* q, const void* k, const void* v, void* o,
                          int32_t log2_s, float scale, int32_t dtype, hipStream_t stream);      // staircase_attn_f32.hip
 }
 
-extern "C" int mdx_staircase_attn_varlen(const void* q, const void* k, const void* v, void* o,
+namespace {
+
+// `store`: rows to copy in the same launch, or null; *stored says whether the launch took them along.
+int staircase(const void* q, const void* k, const void* v, void* o,
                                          int64_t q_stride_t, int64_t q_stride_h,
                                          int64_t k_stride_t, int64_t k_stride_h,
                                          int64_t v_stride_t, int64_t v_stride_h,
@@ -443,7 +485,7 @@ extern "C" int mdx_staircase_attn_varlen(const void* q, const void* k, const voi
                                          int32_t batch, int32_t max_seqlen, int64_t total_tokens,
                                          int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
                                          int32_t staircase_size, float scale, int32_t dtype,
-                                         mdx_stream_t stream_)
+                                         mdx_stream_t stream_, const StoreParams* store, bool* stored)
 {
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     MDX_REQUIRE(batch >= 0 && total_tokens >= 0 && max_seqlen >= 0, MDX_EINVAL, "staircase_attn: negative size");
@@ -505,7 +547,18 @@ extern "C" int mdx_staircase_attn_varlen(const void* q, const void* k, const voi
     const bool pairs = !narrow && max_l > 560 && o_stride_t % 8 == 0 && o_stride_h % 8 == 0 && o_stride_t > 0 &&
                        o_stride_t * 2 * 128 < ((int64_t)1 << 31) && (num_q_heads / num_kv_heads) % 2 == 0 && k_stride_t > 0 && v_stride_t > 0 &&
                        (max_l + 2 * rows_per_wg) * row_elems * 2 < ((int64_t)1 << 31) && row_elems * 2 < (1 << 24) && max_l + 2 * rows_per_wg < (1 << 24);
-    const int64_t grid = n_pairs * (pairs ? num_q_heads / 2 : num_q_heads);
+    int64_t grid = n_pairs * (pairs ? num_q_heads / 2 : num_q_heads);
+    P.store = StoreParams{};
+    P.store.first_wg = 0x7fffffff;
+    if (store && !pairs && grid < ((int64_t)1 << 30)) {
+        P.store = *store;
+        // one token per workgroup while that leaves them few, up to kStoreTokens rounds of rows
+        const int rounds = (store->n_tokens + 511) / 512 < kStoreTokens ? (store->n_tokens + 511) / 512 : kStoreTokens;
+        P.store.tokens_per_wg = rounds * (kThreads / 2 / store->row16);
+        P.store.first_wg = (int)grid;
+        grid += (store->n_tokens + P.store.tokens_per_wg - 1) / P.store.tokens_per_wg;
+        *stored = true;
+    }
     MDX_REQUIRE(grid < ((int64_t)1 << 31), MDX_EUNSUPPORTED, "staircase_attn: grid too large");
     if (pairs) {
         // the kernel's LDS limit is raised once per device (the attribute belongs to the device's copy of the kernel)
@@ -531,4 +584,54 @@ extern "C" int mdx_staircase_attn_varlen(const void* q, const void* k, const voi
         else        staircase_attn_kernel<__bf16, false><<<(unsigned)grid, kThreads, 0, stream>>>(P);
     }
     return mdx::check_launch("staircase_attn");
+}
+
+}  // namespace
+
+extern "C" int mdx_staircase_attn_varlen(const void* q, const void* k, const void* v, void* o,
+                                         int64_t q_stride_t, int64_t q_stride_h,
+                                         int64_t k_stride_t, int64_t k_stride_h,
+                                         int64_t v_stride_t, int64_t v_stride_h,
+                                         int64_t o_stride_t, int64_t o_stride_h,
+                                         const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                                         int32_t batch, int32_t max_seqlen, int64_t total_tokens,
+                                         int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                                         int32_t staircase_size, float scale, int32_t dtype,
+                                         mdx_stream_t stream_)
+{
+    return staircase(q, k, v, o, q_stride_t, q_stride_h, k_stride_t, k_stride_h, v_stride_t, v_stride_h, o_stride_t, o_stride_h,
+                     cu_seqlens_q, cu_seqlens_k, batch, max_seqlen, total_tokens, num_q_heads, num_kv_heads, head_dim, staircase_size, scale,
+                     dtype, stream_, nullptr, nullptr);
+}
+
+extern "C" int mdx_staircase_attn_store(const void* q, const void* k, const void* v, void* o,
+                                        int64_t q_stride_t, int64_t q_stride_h,
+                                        int64_t k_stride_t, int64_t k_stride_h,
+                                        int64_t v_stride_t, int64_t v_stride_h,
+                                        int64_t o_stride_t, int64_t o_stride_h,
+                                        const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                                        int32_t batch, int32_t max_seqlen, int64_t total_tokens,
+                                        int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                                        int32_t staircase_size, float scale, int32_t dtype,
+                                        void* k_cache, void* v_cache, const int32_t* slot_mapping, int64_t num_slots,
+                                        mdx_stream_t stream)
+{
+    const int elem = dtype == MDX_F32 ? 4 : 2;
+    const int64_t row = (int64_t)num_kv_heads * head_dim, row_bytes = row * elem;
+    MDX_REQUIRE(k_stride_h == head_dim && v_stride_h == head_dim, MDX_EUNSUPPORTED, "staircase_attn_store: rows of k and v must be dense");
+    const int row16 = (int)(row_bytes / 16);
+    const bool along = total_tokens > 0 && total_tokens < ((int64_t)1 << 30) && k && v && k_cache && v_cache && slot_mapping && num_slots >= 0 &&
+                       row_bytes % 16 == 0 && row_bytes <= 16 * (kThreads / 2) && kThreads / 2 % row16 == 0 &&
+                       (k_stride_t * elem) % 16 == 0 && (v_stride_t * elem) % 16 == 0 && k_stride_t >= 0 && v_stride_t >= 0 &&
+                       mdx::aligned16(k) && mdx::aligned16(v) && mdx::aligned16(k_cache) && mdx::aligned16(v_cache);
+    StoreParams S{};
+    if (along)
+        S = StoreParams{(const u32x4*)k, (const u32x4*)v, k_stride_t * elem / 16, v_stride_t * elem / 16, (u32x4*)k_cache, (u32x4*)v_cache,
+                        slot_mapping, num_slots, (int)total_tokens, row16, 0, 0};
+    bool stored = false;
+    const int rc = staircase(q, k, v, o, q_stride_t, q_stride_h, k_stride_t, k_stride_h, v_stride_t, v_stride_h, o_stride_t, o_stride_h,
+                             cu_seqlens_q, cu_seqlens_k, batch, max_seqlen, total_tokens, num_q_heads, num_kv_heads, head_dim, staircase_size,
+                             scale, dtype, stream, along ? &S : nullptr, &stored);
+    if (rc != MDX_OK || stored) return rc;
+    return mdx_store_kvcache(k, v, k_stride_t, v_stride_t, k_cache, v_cache, slot_mapping, total_tokens, row, elem, num_slots, stream);
 }

@@ -26,6 +26,8 @@ SIGNATURES = {
     "mdx_store_kvcache": (c_int32, [_P, _P, _I64, _I64, _P, _P, _P, _I64, _I64, _I32, _I64, _P]),
     "mdx_staircase_attn_varlen": (c_int32, [_P, _P, _P, _P] + [_I64] * 8 + [_P, _P, _I32, _I32, _I64,
                                                                            _I32, _I32, _I32, _I32, _F, _I32, _P]),
+    "mdx_staircase_attn_store": (c_int32, [_P, _P, _P, _P] + [_I64] * 8 + [_P, _P, _I32, _I32, _I64, _I32, _I32, _I32, _I32, _F, _I32,
+                                                                          _P, _P, _P, _I64, _P]),
     "mdx_paged_block_attn_workspace_bytes": (c_int64, [_I32] * 7),
     "mdx_paged_block_attn_f32_workspace_bytes": (c_int64, [_I32] * 6),
     "mdx_paged_block_attn": (c_int32, [_P, _P, _P, _P] + [_I64] * 9 + [_P, _I64, _P] + [_I32] * 7 + [_I64, _F, _I32,

@@ -239,3 +239,34 @@ def test_attention_forward_decode_context(dev):
     got = o.view(bs, S, HQ, D).float().cpu()
     assert (got - ref).abs().max().item() < 2e-2
     assert got[2].abs().max().item() == 0
+
+
+@pytest.mark.parametrize("lens", [[1], [33, 7], [109], [560, 300], [500] * 20, [561]])
+@pytest.mark.parametrize("hkv,d,dtype", [(8, 128, torch.bfloat16), (2, 64, torch.float16), (1, 16, torch.bfloat16), (3, 128, torch.bfloat16), (8, 128, torch.float32)])
+def test_attention_prefill_is_the_store_and_the_attention(dev, lens, hkv, d, dtype):
+    """The layer's prefill, which takes the rows of short prompts along in the attention launch, against the two calls: same
+    output, same cache (slots -1 and beyond the cache are skipped), at few and many rows and row widths with and without that form."""
+    import mdx
+    if dtype == torch.float32 and sum(lens) > 1000:
+        pytest.skip("covered by the 16-bit cases")
+    g = torch.Generator(device=dev).manual_seed(sum(lens) + d)
+    N, hq = sum(lens), 2 * hkv
+    q, k = (torch.randn(N, h, d, generator=g, device=dev).to(dtype) for h in (hq, hkv))
+    v = torch.randn(N, 2 * hkv, d, generator=g, device=dev).to(dtype)[:, hkv:]
+    cu = torch.tensor([0] + list(np.cumsum(lens)), dtype=torch.int32, device=dev)
+    pages = N // PAGE + 2
+    slots = torch.randperm(pages * PAGE, generator=g, device=dev)[:N].int()
+    slots[::7] = -1
+    slots[3::11] = pages * PAGE + 5
+    attn = mdx.Attention(hq, d, d ** -0.5, hkv)
+    attn.k_cache = torch.zeros(pages, PAGE, hkv, d, dtype=dtype, device=dev)
+    attn.v_cache = torch.zeros_like(attn.k_cache)
+    kc, vc = torch.zeros_like(attn.k_cache), torch.zeros_like(attn.k_cache)
+    mdx.set_context(True, cu, cu, max(lens), max(lens), slots, None, None, block_size=S)
+    try:
+        o = attn(q, k, v)
+    finally:
+        mdx.reset_context()
+    mdx.store_kvcache(k, v, kc, vc, slots)
+    want = mdx.sparse_attn_varlen(q, k, v, cu, cu, S, max_seqlen=max(lens), softmax_scale=d ** -0.5)
+    assert torch.equal(o, want.flatten(1)) and torch.equal(attn.k_cache, kc) and torch.equal(attn.v_cache, vc)
