@@ -70,14 +70,41 @@ __device__ __forceinline__ void load_q(float (&q)[D / 2], const T* row, int H, i
     }
 }
 
-// Row `row` of the K and V tiles, columns 4 c4 .. 4 c4 + 3 (null pointers: zeros).
-template <typename T, int D>
-__device__ __forceinline__ void stage4(float* lds, int row, int c4, const T* k4, const T* v4) {
-    f32x4 kx = f32x4{0.f, 0.f, 0.f, 0.f}, vx = kx;
-    if (k4) { kx = load4(k4); vx = load4(v4); }
-    *reinterpret_cast<f32x4*>(Lds<D>::k_tile(lds) + row * Lds<D>::kPitchK + 4 * c4) = kx;
-    *reinterpret_cast<f32x4*>(Lds<D>::v_tile(lds) + row * Lds<D>::kPitchV + 4 * c4) = vx;
-}
+// A tile's K and V rows on their way to LDS: (part of) a thread's share of them, as loaded (16-bit elements are widened when they
+// are written).  Fetching a batch of up to kBatch rows before writing any keeps their loads in flight together; loading and
+// writing row by row had cost a trip to memory per row.
+constexpr int kBatch = 4;
+template <typename T> struct Raw4;
+template <> struct Raw4<float> { typedef f32x4 type; };
+template <> struct Raw4<__bf16> { typedef uint2 type; };
+template <> struct Raw4<_Float16> { typedef uint2 type; };
+
+template <typename T, int D, int THREADS> struct TileRegs {
+    static constexpr int kAll = kTileKeys * (D / 4) / THREADS, kPasses = kAll < kBatch ? kAll : kBatch, kBatches = kAll / kPasses;
+    typename Raw4<T>::type k[kPasses], v[kPasses];
+    // row_ptr(row): element offset of that row of the tile, the same for K and V's bases; any row may be asked for.
+    template <typename KRow, typename VRow>
+    __device__ __forceinline__ void fetch(int batch, int tid, int width, KRow k_row, VRow v_row) {
+#pragma unroll
+        for (int p = 0; p < kPasses; ++p) {
+            const int u = tid + THREADS * (batch * kPasses + p), row = u / (D / 4), col = min(4 * (u % (D / 4)), width - 4);
+            k[p] = *reinterpret_cast<const typename Raw4<T>::type*>(k_row(row) + col);
+            v[p] = *reinterpret_cast<const typename Raw4<T>::type*>(v_row(row) + col);
+        }
+    }
+    // real(row): whether the row holds a key (else, and beyond the head's width: zeros)
+    template <typename Real>
+    __device__ __forceinline__ void write(int batch, float* lds, int tid, int width, Real real) const {
+#pragma unroll
+        for (int p = 0; p < kPasses; ++p) {
+            const int u = tid + THREADS * (batch * kPasses + p), row = u / (D / 4), c4 = u % (D / 4);
+            f32x4 kx = load4(reinterpret_cast<const T*>(&k[p])), vx = load4(reinterpret_cast<const T*>(&v[p]));
+            if (!real(row) || 4 * c4 >= width) { kx = f32x4{0.f, 0.f, 0.f, 0.f}; vx = kx; }
+            *reinterpret_cast<f32x4*>(Lds<D>::k_tile(lds) + row * Lds<D>::kPitchK + 4 * c4) = kx;
+            *reinterpret_cast<f32x4*>(Lds<D>::v_tile(lds) + row * Lds<D>::kPitchV + 4 * c4) = vx;
+        }
+    }
+};
 
 // Running softmax state of a wavefront's 32 queries: l is this half-wavefront's share of the row sum.
 template <int D> struct State {

@@ -31,7 +31,7 @@ struct PagedWideParams {
     int64_t c_sp, c_st, c_sh;                       // cache strides: page, token, head
     const int32_t* block_table; int64_t bt_stride;
     const int32_t* context_lens;
-    int bs, sq, nqt, num_q_heads, heads_per_kv, page_size, max_pages, head_dim;
+    int bs, sq, nqt, num_q_heads, heads_per_kv, page_size, page_shift, max_pages, head_dim;   // page_shift: log2(page_size) or -1
     int64_t num_pages;
     float c;                                        // scale * log2(e)
     int nsplit, pieces;                             // partial slots per sequence; pieces the whole launch should be cut into per (head group, query tile)
@@ -93,24 +93,23 @@ __global__ __launch_bounds__(64 * HPW * KW, D <= 128 ? 2 : 1) void paged_attn_f3
     State<D> st;
     st.init();
     for (int t0 = 0; t0 < n_tiles; t0 += KW) {
-        if (t0) __syncthreads();                               // the previous tiles have been read by everybody
-        // ---- tiles t0 .. t0 + KW - 1 into LDS, all threads on each (a tile never straddles a page: page_size % 32 == 0) ----
+        // ---- tiles t0 .. t0 + KW - 1 into LDS, all threads on each (a tile never straddles a page: page_size % 32 == 0, so that all
+        //      its rows exist in memory, whatever they hold) ----
         unsigned tile_ok = 0;                                  // bit i: tile t0 + i exists and lies on a valid page (uniform)
+        TileRegs<T, D, kThreads> regs;
 #pragma unroll
         for (int i = 0; i < KW; ++i) {
             const int key0 = key_begin + (t0 + i) * kTileKeys;
-            if (key0 >= key_end) break;
-            const int64_t page = bt[key0 / P.page_size];
-            if (page < 0 || page >= P.num_pages) continue;
-            tile_ok |= 1u << i;
-            const int64_t base = page * P.c_sp + (int64_t)(key0 % P.page_size) * P.c_st;
-#pragma unroll
-            for (int p = 0; p < kTileKeys * (D / 4) / kThreads; ++p) {
-                const int u = tid + kThreads * p;
-                const int row = u / (D / 4), c4 = u % (D / 4);
-                const bool real = key0 + row < key_end && 4 * c4 < width;
-                const int64_t off = base + (int64_t)row * P.c_st + 4 * c4;
-                stage4<T, D>(lds + i * kTileFloats, row, c4, real ? kc + off : nullptr, real ? vc + off : nullptr);
+            const int page_slot = P.page_shift >= 0 ? key0 >> P.page_shift : key0 / P.page_size;
+            const int64_t page = key0 < key_end ? bt[page_slot] : -1;
+            const bool ok = page >= 0 && page < P.num_pages;
+            if (ok) tile_ok |= 1u << i;
+            const int64_t base = page * P.c_sp + (int64_t)(key0 - page_slot * P.page_size) * P.c_st;
+#pragma unroll 1
+            for (int b = 0; b < regs.kBatches; ++b) {
+                if (ok) regs.fetch(b, tid, width, [&](int row) { return kc + base + (int64_t)row * P.c_st; }, [&](int row) { return vc + base + (int64_t)row * P.c_st; });
+                if (i == 0 && b == 0 && t0) __syncthreads();   // the previous tiles have been read by everybody
+                if (ok) regs.write(b, lds + i * kTileFloats, tid, width, [&](int row) { return key0 + row < key_end; });
             }
         }
         __syncthreads();
@@ -307,6 +306,8 @@ int launch_paged_f32(const void* q, void* o, const void* k_cache, const void* v_
     P.bs = bs; P.sq = sq; P.nqt = (sq + 31) / 32;
     P.num_q_heads = num_q_heads; P.heads_per_kv = num_q_heads / num_kv_heads;
     P.page_size = page_size; P.max_pages = max_pages; P.head_dim = head_dim;
+    P.page_shift = -1;
+    for (int i = 0; i < 31; ++i) if (page_size == (1 << i)) P.page_shift = i;
     P.num_pages = num_pages;
     P.c = scale * kLog2e;
     // as many partial slots as the launch wants and the caller's workspace holds; none: whole contexts

@@ -73,19 +73,23 @@ __global__ __launch_bounds__(kThreads, D <= 128 ? 2 : 1) void staircase_attn_f32
 
     State<D> st;
     st.init();
+    // the next tile is on its way (its first batch, in registers) while this one is multiplied; rows outside the sequence: its
+    // first one, zeroed later
+    TileRegs<T, D, kThreads> regs;
+    auto fetch = [&](int t, int batch) {
+        auto tok_of = [&](int row) { const int jp = t * kTileKeys + row; return (int64_t)seq0 + (jp >= pad && jp < Lp ? jp - pad : 0); };
+        regs.fetch(batch, tid, width, [&](int row) { return kb + tok_of(row) * P.k_st; }, [&](int row) { return vb + tok_of(row) * P.v_st; });
+    };
+    fetch(0, 0);
     for (int t = 0; t < n_tiles; ++t) {
         const int key0 = t * kTileKeys;
         __syncthreads();                                       // the previous tile has been read by everybody
-        // ---- K and V rows key0 .. key0 + 31 into LDS as fp32 (rows outside the sequence and padding columns: zeros) ----
 #pragma unroll
-        for (int p = 0; p < kTileKeys * (D / 4) / kThreads; ++p) {
-            const int u = tid + kThreads * p;
-            const int row = u / (D / 4), c4 = u % (D / 4);
-            const int jp = key0 + row;
-            const bool real = jp >= pad && jp < Lp && 4 * c4 < width;
-            const int64_t ktok = (int64_t)seq0 + (jp - pad);
-            stage4<T, D>(lds, row, c4, real ? kb + ktok * P.k_st + 4 * c4 : nullptr, real ? vb + ktok * P.v_st + 4 * c4 : nullptr);
+        for (int batch = 0; batch < regs.kBatches; ++batch) {
+            if (batch > 0) fetch(t, batch);
+            regs.write(batch, lds, tid, width, [&](int row) { const int jp = key0 + row; return jp >= pad && jp < Lp; });
         }
+        if (t + 1 < n_tiles) fetch(t + 1, 0);
         __syncthreads();
         if (key0 >= wave_hi || key0 + kTileKeys <= pad) continue;        // nothing of this tile is visible to this wavefront
         tile_step<D>(lds, q, st, P.c, width, lane, [&](int key) { const int kj = key0 + key; return kj >= pad && kj < key_hi; });
