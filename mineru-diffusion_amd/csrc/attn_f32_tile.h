@@ -173,19 +173,54 @@ __device__ __forceinline__ void tile_step(const float* lds, const float (&q)[D /
     }
 }
 
-// O = O^T / l into this lane's query row (4 consecutive d per (d tile, register group)); a row that saw no key: zeros.
-template <typename T, int D>
-__device__ __forceinline__ void store_o(T* orow, const State<D>& st, int H, int width) {
-    const float l_all = st.l + __shfl_xor(st.l, 32);
-    const float inv = l_all > 0.f ? 1.0f / l_all : 0.f;
-    if (!orow) return;
+// Folds, through LDS, the states of the KW wavefronts (wave, wave + 1, ... of a multiple of KW) that shared a query tile's keys, and
+// hands out the columns: emit(d, O's columns d .. d + 3 of this lane's query, not yet divided by l); each wavefront gets every
+// KW-th column tile.  m and l come back whole before the first emit.  Called by all wavefronts; the region must hold their states.
+template <int D, int KW, typename Emit>
+__device__ __forceinline__ void fold_states(float* lds, State<D>& st, int wave, int lane, int width, Emit emit) {
+    constexpr int kMl = (D / 32) * 16 * 64, kStateFloats = kMl + 2 * 64;       // O as [d tile][register][lane], then m, l
+    const int H = lane >> 5, kw = wave % KW;
+    st.l += __shfl_xor(st.l, 32);                                              // a state is now (m, l, O) per query
+    const float* states = lds + (wave - kw) * kStateFloats;
+    float w[KW];
+    if (KW > 1) {
+        __syncthreads();                                                       // the last tiles have been read by everybody
+        float* dst = lds + wave * kStateFloats;
 #pragma unroll
-    for (int dt = 0; dt < D / 32; ++dt)
+        for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) dst[(dt * 16 + i) * 64 + lane] = st.o[dt][i];
+        dst[kMl + lane] = st.m;
+        dst[kMl + 64 + lane] = st.l;
+        __syncthreads();
+        float M = kMinusBig, l_all = 0.f;
+#pragma unroll
+        for (int s = 0; s < KW; ++s) { w[s] = states[s * kStateFloats + kMl + lane]; M = fmaxf(M, w[s]); }
+#pragma unroll
+        for (int s = 0; s < KW; ++s) {
+            w[s] = __builtin_amdgcn_exp2f(w[s] - M);
+            l_all += states[s * kStateFloats + kMl + 64 + lane] * w[s];
+        }
+        st.m = M;
+        st.l = l_all;
+    }
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt) {
+        if (dt % KW != kw || dt * 32 >= width) continue;                       // (uniform per wavefront)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
+            f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (KW == 1) acc[e] = st.o[dt][4 * g + e];
+#pragma unroll
+                for (int s = 0; KW > 1 && s < KW; ++s) acc[e] += states[s * kStateFloats + (dt * 16 + 4 * g + e) * 64 + lane] * w[s];
+            }
             const int d = dt * 32 + 8 * g + 4 * H;
-            if (d < width) store4(orow + d, f32x4{st.o[dt][4 * g] * inv, st.o[dt][4 * g + 1] * inv, st.o[dt][4 * g + 2] * inv, st.o[dt][4 * g + 3] * inv});
+            if (d < width) emit(d, acc);
         }
+    }
 }
+template <int D> constexpr int kStateBytes = ((D / 32) * 16 * 64 + 2 * 64) * (int)sizeof(float);
 
 }  // namespace mdx_attn_f32

@@ -119,59 +119,20 @@ __global__ __launch_bounds__(64 * HPW * KW, D <= 128 ? 2 : 1) void paged_attn_f3
         }
     }
 
-    // ---- merge the KW states of a head through LDS: each of its wavefronts folds, and stores, every KW-th column tile ----
-    constexpr int kStateFloats = (D / 32) * 16 * 64 + 2 * 64;                  // O as [dt][register][lane], then m, l
-    static_assert(HPW * KW * kStateFloats <= KW * kTileFloats, "merge buffer exceeds the tile region");
-    st.l += __shfl_xor(st.l, 32);                                              // a state is now (m, l, O) per query
-    float w[KW];
-    float M = st.m, l_all = st.l;
-    const float* states = lds + hw * KW * kStateFloats;
-    if (KW > 1) {
-        __syncthreads();                                                       // the last tiles have been read by everybody
-        float* dst = lds + wave * kStateFloats;
-#pragma unroll
-        for (int dt = 0; dt < D / 32; ++dt)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) dst[(dt * 16 + i) * 64 + lane] = st.o[dt][i];
-        dst[(D / 32) * 16 * 64 + lane] = st.m;
-        dst[(D / 32) * 16 * 64 + 64 + lane] = st.l;
-        __syncthreads();
-        M = kMinusBig;
-        l_all = 0.f;
-#pragma unroll
-        for (int s = 0; s < KW; ++s) { w[s] = states[s * kStateFloats + (D / 32) * 16 * 64 + lane]; M = fmaxf(M, w[s]); }
-#pragma unroll
-        for (int s = 0; s < KW; ++s) {
-            w[s] = __builtin_amdgcn_exp2f(w[s] - M);
-            l_all += states[s * kStateFloats + (D / 32) * 16 * 64 + 64 + lane] * w[s];
-        }
-    }
-    if (!row_ok) return;
-    const float inv = l_all > 0.f ? 1.0f / l_all : 0.f;                        // no key at all: zeros
+    // ---- the KW states of a head fold through LDS; one piece: the result, else a partial ----
+    static_assert(HPW * KW * kStateBytes<D> <= KW * Lds<D>::kBytes, "merge buffer exceeds the tile region");
     T* orow = static_cast<T*>(P.o) + (int64_t)b * P.o_sb + (int64_t)qrow * P.o_ss + (int64_t)head * P.o_sh;
     const int64_t slot = (((int64_t)b * P.num_q_heads + head) * P.nqt + qt) * P.nsplit + split;
     float* prow = P.part_o + (slot * 32 + r) * D;
-#pragma unroll
-    for (int dt = 0; dt < D / 32; ++dt) {
-        if (dt % KW != kw || dt * 32 >= width) continue;                       // (uniform per wavefront)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                if (KW == 1) acc[e] = st.o[dt][4 * g + e];
-#pragma unroll
-                for (int s = 0; KW > 1 && s < KW; ++s) acc[e] += states[s * kStateFloats + (dt * 16 + 4 * g + e) * 64 + lane] * w[s];
-            }
-            const int d = dt * 32 + 8 * g + 4 * H;
-            if (d >= width) continue;
-            if (n_pieces == 1) store4(orow + d, f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv});
-            else *reinterpret_cast<f32x4*>(prow + d) = acc;
-        }
-    }
-    if (n_pieces > 1 && kw == 0 && H == 0) {
-        P.part_ml[(slot * 2 + 0) * 32 + r] = M;
-        P.part_ml[(slot * 2 + 1) * 32 + r] = l_all;
+    fold_states<D, KW>(lds, st, wave, lane, width, [&](int d, f32x4 acc) {
+        if (!row_ok) return;
+        if (n_pieces > 1) { *reinterpret_cast<f32x4*>(prow + d) = acc; return; }
+        const float inv = st.l > 0.f ? 1.0f / st.l : 0.f;                      // no key at all: zeros
+        store4(orow + d, f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv});
+    });
+    if (row_ok && n_pieces > 1 && kw == 0 && H == 0) {
+        P.part_ml[(slot * 2 + 0) * 32 + r] = st.m;
+        P.part_ml[(slot * 2 + 1) * 32 + r] = st.l;
     }
 }
 

@@ -5,8 +5,10 @@
 // BLOCK_DMODEL = head_dim, o = empty_like(q)); the model itself runs bf16 with d = 128, so this is the path
 // for callers outside the model's own configuration.  Arithmetic and layout: attn_f32_tile.h.
 //
-// Same decomposition as the 16-bit kernels: a workgroup of 4 wavefronts owns 128 padded query rows of one
-// (sequence, head), a wavefront 32 of them; K and V tiles of 32 keys are staged through LDS as fp32, one at a time.
+// A workgroup of 4 wavefronts owns 128 / KW padded query rows of one (sequence, head), KW wavefronts every 32 of them: each takes
+// every KW-th tile of 32 keys, KW tiles (K and V as fp32) are staged through LDS at a time, and the KW states fold at the end.
+// The matrix instruction bounds it, 8192 cycles per wavefront and tile, and its last row group sees all keys, so a launch
+// that does not fill the chip lasts as long as that group's chain of tiles: KW divides the chain.
 //
 // The mask is the reference's (:98-102,137-139): with nb = ceil(L / S) blocks right-aligned, pad = nb S - L,
 // query row i sees key j iff j <= ((i + pad) / S + 1) S - 1 - pad.
@@ -18,7 +20,7 @@ namespace {
 using namespace mdx_attn_f32;
 
 constexpr int kThreads = 256;
-constexpr int kRowsPerWg = 128;
+constexpr int kWaves = kThreads / 64;
 
 struct WideParams {
     const void* q; const void* k; const void* v; void* o;
@@ -29,12 +31,13 @@ struct WideParams {
 };
 
 // T: element type of q/k/v/o.  D: 128 or 256, the head width that registers and LDS are laid out for.
-template <typename T, int D>
-__global__ __launch_bounds__(kThreads, D <= 128 ? 2 : 1) void staircase_attn_f32_kernel(const WideParams P)
+template <typename T, int D, int KW>
+__global__ __launch_bounds__(kThreads, D <= 128 && KW <= 2 ? 2 : 1) void staircase_attn_f32_kernel(const WideParams P)
 {
+    constexpr int kRowsPerWg = 32 * kWaves / KW;
     extern __shared__ __attribute__((aligned(16))) float lds[];
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, kw = wave % KW;
     const int H = lane >> 5, r = lane & 31;
     const int head = blockIdx.x;
     const int rg = P.n_row_groups - 1 - (int)blockIdx.y;       // the heaviest row groups start first
@@ -57,7 +60,7 @@ __global__ __launch_bounds__(kThreads, D <= 128 ? 2 : 1) void staircase_attn_f32
     const T* vb = static_cast<const T*>(P.v) + (int64_t)kvh * P.v_sh;
 
     // ---- this lane's query ----
-    const int row_w0 = row_g0 + wave * 32;
+    const int row_w0 = row_g0 + wave / KW * 32;
     const int ip = row_w0 + r;                                 // padded query row
     const bool row_ok = ip >= pad && ip < Lp;
     const int64_t tok = (int64_t)seq0 + (ip - pad);
@@ -81,38 +84,68 @@ __global__ __launch_bounds__(kThreads, D <= 128 ? 2 : 1) void staircase_attn_f32
         regs.fetch(batch, tid, width, [&](int row) { return kb + tok_of(row) * P.k_st; }, [&](int row) { return vb + tok_of(row) * P.v_st; });
     };
     fetch(0, 0);
-    for (int t = 0; t < n_tiles; ++t) {
-        const int key0 = t * kTileKeys;
-        __syncthreads();                                       // the previous tile has been read by everybody
+    for (int t = 0; t < n_tiles; t += KW) {
+        __syncthreads();                                       // the previous tiles have been read by everybody
 #pragma unroll
-        for (int batch = 0; batch < regs.kBatches; ++batch) {
-            if (batch > 0) fetch(t, batch);
-            regs.write(batch, lds, tid, width, [&](int row) { const int jp = key0 + row; return jp >= pad && jp < Lp; });
+        for (int i = 0; i < KW; ++i) {
+#pragma unroll
+            for (int batch = 0; batch < regs.kBatches; ++batch) {
+                if (i + batch > 0) fetch(t + i, batch);
+                regs.write(batch, lds + i * Lds<D>::kFloats, tid, width, [&](int row) { const int jp = (t + i) * kTileKeys + row; return jp >= pad && jp < Lp; });
+            }
         }
-        if (t + 1 < n_tiles) fetch(t + 1, 0);
+        if (t + KW < n_tiles) fetch(t + KW, 0);
         __syncthreads();
+        const int key0 = (t + kw) * kTileKeys;
         if (key0 >= wave_hi || key0 + kTileKeys <= pad) continue;        // nothing of this tile is visible to this wavefront
-        tile_step<D>(lds, q, st, P.c, width, lane, [&](int key) { const int kj = key0 + key; return kj >= pad && kj < key_hi; });
+        tile_step<D>(lds + kw * Lds<D>::kFloats, q, st, P.c, width, lane, [&](int key) { const int kj = key0 + key; return kj >= pad && kj < key_hi; });
     }
-    store_o<T, D>(row_ok ? static_cast<T*>(P.o) + tok * P.o_st + (int64_t)head * P.o_sh : nullptr, st, H, width);
+    static_assert(KW == 1 || kWaves * kStateBytes<D> <= KW * Lds<D>::kBytes, "merge buffer exceeds the tile region");
+    T* orow = static_cast<T*>(P.o) + tok * P.o_st + (int64_t)head * P.o_sh;
+    fold_states<D, KW>(lds, st, wave, lane, width, [&](int d, f32x4 acc) {
+        const float inv = st.l > 0.f ? 1.0f / st.l : 0.f;
+        if (row_ok) store4(orow + d, f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv});
+    });
 }
 
-template <typename T, int D>
-int launch(const WideParams& P, hipStream_t stream)
+template <typename T, int D, int KW>
+int launch_split(WideParams P, int64_t max_l, hipStream_t stream)
 {
+    constexpr int kRowsPerWg = 32 * kWaves / KW, kLdsBytes = KW * Lds<D>::kBytes;
+    max_l = max_l < P.total_tokens ? max_l : P.total_tokens;
+    P.n_row_groups = (int)((max_l + (1 << P.log2_s) - 1 + kRowsPerWg - 1) / kRowsPerWg);
+    MDX_REQUIRE(P.batch <= 65535 && P.n_row_groups <= 65535, MDX_EUNSUPPORTED,
+                "staircase_attn: fp32 arithmetic takes up to 65535 sequences of up to 8 M tokens");
     // the kernel's LDS limit is raised once per device
     static std::atomic<bool> raised[64];
     int device = 0;
     hipError_t e = hipGetDevice(&device);
     MDX_REQUIRE(e == hipSuccess && device >= 0 && device < 64, MDX_ELAUNCH, "staircase_attn: no current device (%s)", hipGetErrorString(e));
     if (!raised[device].load(std::memory_order_acquire)) {
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(staircase_attn_f32_kernel<T, D>), hipFuncAttributeMaxDynamicSharedMemorySize, Lds<D>::kBytes);
-        MDX_REQUIRE(e == hipSuccess, MDX_ELAUNCH, "staircase_attn: cannot reserve %d bytes of LDS (%s)", Lds<D>::kBytes, hipGetErrorString(e));
+        e = hipFuncSetAttribute(reinterpret_cast<const void*>(staircase_attn_f32_kernel<T, D, KW>), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+        MDX_REQUIRE(e == hipSuccess, MDX_ELAUNCH, "staircase_attn: cannot reserve %d bytes of LDS (%s)", kLdsBytes, hipGetErrorString(e));
         raised[device].store(true, std::memory_order_release);
     }
     const dim3 grid((unsigned)P.num_q_heads, (unsigned)P.n_row_groups, (unsigned)P.batch);
-    staircase_attn_f32_kernel<T, D><<<grid, kThreads, Lds<D>::kBytes, stream>>>(P);
+    staircase_attn_f32_kernel<T, D, KW><<<grid, kThreads, kLdsBytes, stream>>>(P);
     return mdx::check_launch("staircase_attn (fp32 arithmetic)");
+}
+
+// How many wavefronts share a row tile's keys, from the number of row tiles R (all heads) and the longest prompt.  While the
+// launch leaves compute units idle the longest chain of tiles counts: four, as soon as there are tiles for them and their
+// workgroups (135 KB of LDS, one per CU) come in one round, or in three if the chain is long enough to pay for those.  Then
+// two, as long as the row groups' unequal chains leave a ragged end (to 16 row tiles per CU); prompts of two tiles have nothing
+// to share once the chip is full, and the fold at the end costs about one tile.  Measured (1 / 2 / 4 wavefronts, 16 query
+// heads, us): 100 tokens 29 / 21 / 15, 500 98 / 61 / 39, 1024 189 / 114 / 84, 2000 362 / 270 / 289, 4096 931 / 733 / 1077,
+// 8192 2680 / 2703 / 4130, 8 x 250 66 / 52 / 81, 16 x 64 18 / 23 / 29, 4 x 2048 838 / 731 / 1153, 4 x 4096 2605 / 2738 / 4358.
+template <typename T>
+int launch(const WideParams& P, int64_t max_l, hipStream_t stream)
+{
+    if (P.head_dim > 128) return launch_split<T, 256, 1>(P, max_l, stream);
+    const int64_t row_tiles = ((int64_t)P.total_tokens / 32 + P.batch) * P.num_q_heads, cus = mdx::compute_units();
+    if (max_l > 64 && row_tiles <= (max_l < 384 ? cus : 3 * cus)) return launch_split<T, 128, 4>(P, max_l, stream);
+    if (row_tiles <= (max_l <= 64 ? cus : 16 * cus)) return launch_split<T, 128, 2>(P, max_l, stream);
+    return launch_split<T, 128, 1>(P, max_l, stream);
 }
 
 }  // namespace
@@ -142,16 +175,13 @@ int launch_staircase_f32(const void* q, const void* k, const void* v, void* o,
     P.cu_seqlens = cu_seqlens;
     P.batch = batch;
     P.total_tokens = (int)total_tokens;
-    P.n_row_groups = (int)((max_l + (1 << log2_s) - 1 + kRowsPerWg - 1) / kRowsPerWg);
+    P.n_row_groups = 0;                                        // with the split
     P.num_q_heads = num_q_heads; P.num_kv_heads = num_kv_heads; P.head_dim = head_dim; P.log2_s = log2_s;
     P.c = scale * kLog2e;
-    MDX_REQUIRE(batch <= 65535 && P.n_row_groups <= 65535, MDX_EUNSUPPORTED,
-                "staircase_attn: fp32 arithmetic takes up to 65535 sequences of up to 8 M tokens");
-    const bool wide = head_dim > 128;
     switch (dtype) {
-    case MDX_F32:  return wide ? launch<float, 256>(P, stream) : launch<float, 128>(P, stream);
-    case MDX_F16:  return wide ? launch<_Float16, 256>(P, stream) : launch<_Float16, 128>(P, stream);
-    case MDX_BF16: return wide ? launch<__bf16, 256>(P, stream) : launch<__bf16, 128>(P, stream);
+    case MDX_F32:  return launch<float>(P, max_l, stream);
+    case MDX_F16:  return launch<_Float16>(P, max_l, stream);
+    case MDX_BF16: return launch<__bf16>(P, max_l, stream);
     }
     return mdx::fail(MDX_EUNSUPPORTED, "staircase_attn: dtype %d", dtype);
 }

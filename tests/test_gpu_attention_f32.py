@@ -279,3 +279,10 @@ def test_paged_fp32_contexts_cut_into_pieces(dev, ctxs, room):
     ref = oracle.paged_block_attn(q.cpu(), kc.cpu(), vc.cpu(), bt.cpu(), lens.cpu(), scale)
     assert (o.cpu() - ref).abs().max().item() < TOL_F32
     assert (ws[n_bytes:] == 255).all()
+
+
+@pytest.mark.parametrize("lens", [[64, 33, 1] * 14, [65] * 20 + [1, 32], [390, 31, 65, 7], [129, 300] * 3, [1100, 5, 260]])
+def test_fp32_prefill_keys_shared_by_one_two_or_four_wavefronts(dev, lens):
+    """Both sides of the rule that splits a row tile's keys: full launches of short prompts, ragged ones in between, long chains."""
+    _check(dev, lens, 32, 16, 8, 128, torch.float32, seed=sum(lens))
+    _check(dev, lens[:4], 8, 4, 2, 96, torch.float32, seed=sum(lens) + 1)
