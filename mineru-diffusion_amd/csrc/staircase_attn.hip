@@ -32,10 +32,11 @@ namespace {
 
 using namespace mdx_attn;
 
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
 constexpr int kTileKeys = 64;      // keys staged in LDS per iteration
 constexpr int kThreads = 256;      // 4 wavefronts, 2 workgroups per CU
 constexpr int kRowsPerWg = 128;    // 4 wavefronts x 32 query rows
-constexpr int kTileBytes = kTileKeys * kLdsPitch;
 
 // The K/V rows of a short prompt's layer go to the paged cache in the attention launch itself (mdx_staircase_attn_store): the
 // attention reads k and v, not the cache, so the rows are copied by workgroups behind the attention's, which find the chip
@@ -123,15 +124,16 @@ __device__ __forceinline__ int wave_prefix_sum(int x)
 
 // `hist`: 65 ints of LDS that belong to the calling wavefront alone (unused when there are more than 64 row groups).
 constexpr int kDenseMaxBatch = 1024;   // sequences per launch that the histogram numbering walks (64 per step)
-__device__ __forceinline__ bool locate_row_group(const StaircaseParams& P, int j, int lane, int* hist, int& b, int& rg)
+template <int ROWS>
+__device__ __forceinline__ bool locate_row_group(const StaircaseParams& P, int j, int lane, int* hist, int& b, int& rg, int& seq0, int& L)
 {
     // row groups of sequence s (0 for an empty or absent one); never more than the launch has levels for
+    int first = 0, len = 0;                                    // of the sequence that groups_of was last asked about
     auto groups_of = [&](int s) {
         int g = 0;
         if (s < P.batch) {
-            int first, len;
             seq_bounds(P, s, first, len);
-            if (len > 0) g = min(P.n_row_groups, ((((len + (1 << P.log2_s) - 1) >> P.log2_s) << P.log2_s) + kRowsPerWg - 1) / kRowsPerWg);
+            if (len > 0) g = min(P.n_row_groups, ((((len + (1 << P.log2_s) - 1) >> P.log2_s) << P.log2_s) + ROWS - 1) / ROWS);
         }
         return g;
     };
@@ -144,7 +146,7 @@ __device__ __forceinline__ bool locate_row_group(const StaircaseParams& P, int j
         // backwards over the lanes (lane l = level 63 - l).
         hist[lane] = 0;
         if (lane == 0) hist[64] = 0;
-        const int g0 = groups_of(lane);
+        const int g0 = groups_of(lane), first0 = first, len0 = len;
         if (lane < P.batch) atomicAdd(&hist[g0], 1);
         for (int s0 = 64; s0 < P.batch; s0 += 64)
             if (s0 + lane < P.batch) atomicAdd(&hist[groups_of(s0 + lane)], 1);
@@ -165,7 +167,10 @@ __device__ __forceinline__ bool locate_row_group(const StaircaseParams& P, int j
             if (nth < here) {
                 const int before = __popcll(owners & ((1ull << lane) - 1ull));
                 const unsigned long long hit = __ballot(((owners >> lane) & 1ull) != 0 && before == nth);
-                b = s0 + __ffsll((long long)hit) - 1;
+                const int at = __ffsll((long long)hit) - 1;
+                b = s0 + at;
+                seq0 = __builtin_amdgcn_readlane(s0 == 0 ? first0 : first, at);
+                L = __builtin_amdgcn_readlane(s0 == 0 ? len0 : len, at);
                 break;
             }
             nth -= here;
@@ -195,48 +200,57 @@ __device__ __forceinline__ bool locate_row_group(const StaircaseParams& P, int j
         const unsigned long long hit = __ballot(((owners >> lane) & 1ull) != 0 && before == nth);
         b = __ffsll((long long)hit) - 1;
         rg = level;
-        return b >= 0;
+        if (b < 0) return false;
+        seq0 = __builtin_amdgcn_readlane(first, b);
+        L = __builtin_amdgcn_readlane(len, b);
+        return true;
     }
     // more than 64 sequences with more than 64 row groups each: the full (level x sequence) rectangle
     b = j % P.batch;
     rg = P.n_row_groups - 1 - j / P.batch;
+    seq_bounds(P, b, seq0, L);
     return true;
 }
 
+// KW: wavefronts that share a row tile of 32 queries.  2: each takes half of every tile of 64 keys, the workgroup owns 64 rows, and
+// the two states fold through LDS at the end.  A launch of few row groups is a chain of tiles, 1.4 us each from the load to
+// the last product, of which half is the wavefront's own arithmetic; with half the keys it is 1.15 us.  (Four wavefronts, 32
+// rows per workgroup, and steps of 128 keys measured no better: then the staging bounds it, which a compute unit takes in at
+// 12-20 bytes per cycle.)
 // NARROW: head_dim below 128 (a multiple of 16).  Rows of q, k, v are then padded with zeros on their way into
 // registers and LDS, products over the padding are skipped, and only head_dim columns of o are written.
-template <typename E, bool NARROW>
+template <typename E, bool NARROW, int KW>
 __global__ __launch_bounds__(kThreads, 2) void staircase_attn_kernel(const StaircaseParams P)
 {
+    constexpr int kRows = kRowsPerWg / KW, kTileBytes = kTileKeys * kLdsPitch;
+    constexpr int kSub = kTileKeys / KW / 32;                  // sub-tiles of 32 keys that a wavefront takes of a tile
     const int width = NARROW ? P.head_dim : kHeadDim;
-    __shared__ __attribute__((aligned(16))) char lds_kbuf[2][kTileBytes];   // double-buffered K and V tiles
-    __shared__ __attribute__((aligned(16))) char lds_vbuf[2][kTileBytes];
+    __shared__ __attribute__((aligned(16))) char lds[4 * kTileBytes];        // double-buffered K and V tiles
+    auto lds_kbuf = [&](int i) { return lds + i * kTileBytes; };
+    auto lds_vbuf = [&](int i) { return lds + (2 + i) * kTileBytes; };
     __shared__ int lds_hist[kThreads / 64][80];                // per wavefront: scratch of the workgroup numbering (no barrier separates it from the first tile store)
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, kw = wave % KW;
     const int H = lane >> 5, r = lane & 31;
 
     if ((int)blockIdx.x >= P.store.first_wg) { store_rows(P.store, (int)blockIdx.x - P.store.first_wg, tid); return; }
 
     // ---- workgroup -> (head slot, sequence b, row group rg) ------------------------------------
     const int hslot = blockIdx.x % P.num_q_heads;
-    int b, rg;
-    if (!locate_row_group(P, blockIdx.x / P.num_q_heads, lane, lds_hist[wave], b, rg)) return;
-
-    int seq0, L;
-    seq_bounds(P, b, seq0, L);
+    int b, rg, seq0, L;
+    if (!locate_row_group<kRows>(P, blockIdx.x / P.num_q_heads, lane, lds_hist[wave], b, rg, seq0, L)) return;
     if (L <= 0) return;
     const int S = 1 << P.log2_s;
     const int Lp = ((L + S - 1) >> P.log2_s) << P.log2_s;     // padded length
     const int pad = Lp - L;
-    const int row_g0 = rg * kRowsPerWg;                        // first padded row of the workgroup
+    const int row_g0 = rg * kRows;                        // first padded row of the workgroup
     if (row_g0 >= Lp) return;
 
     const int kvh = hslot % P.num_kv_heads;                    // launch order: KV head fastest
     const int head = kvh * (P.num_q_heads / P.num_kv_heads) + hslot / P.num_kv_heads;
 
     // ---- this wavefront's 32 rows ----
-    const int row_w0 = row_g0 + wave * 32;
+    const int row_w0 = row_g0 + wave / KW * 32;
     const int ip = row_w0 + r;                                 // this lane's padded query row
     const bool row_ok = ip >= pad && ip < Lp;
     const int64_t tok = (int64_t)seq0 + (ip - pad);
@@ -248,7 +262,7 @@ __global__ __launch_bounds__(kThreads, 2) void staircase_attn_kernel(const Stair
     const int key_hi = limit_of(ip);
     const int wave_hi = (row_w0 < Lp) ? limit_of(min(row_w0 + 31, Lp - 1)) : 0;   // 0: idle wavefront
     const int wave_hi_min = limit_of(row_w0);
-    const int wg_hi = limit_of(min(row_g0 + kRowsPerWg - 1, Lp - 1));
+    const int wg_hi = limit_of(min(row_g0 + kRows - 1, Lp - 1));
     const int n_tiles = (wg_hi + kTileKeys - 1) / kTileKeys;
 
     WaveState<1> st;
@@ -284,25 +298,25 @@ __global__ __launch_bounds__(kThreads, 2) void staircase_attn_kernel(const Stair
     };
 
     fetch(0);
-    store_tile<kTileKeys, kThreads>(lds_kbuf[0], lds_vbuf[0], regs, tid);
+    store_tile<kTileKeys, kThreads>(lds_kbuf(0), lds_vbuf(0), regs, tid);
     if (n_tiles > 1) fetch(1);
     __syncthreads();
     for (int t = 0; t < n_tiles; ++t) {
-        const char* lds_k = lds_kbuf[t & 1];
-        const char* lds_v = lds_vbuf[t & 1];
-        const int key0 = t * kTileKeys;
-        if (key0 < wave_hi) {
-            if (key0 >= pad && key0 + kTileKeys <= wave_hi_min) {
-                attn_step<E, 1, 2, false>(lds_k, lds_v, 0, q, st, P.c, lane, key0, pad, key_hi, width);
-            } else if (key0 + 32 < wave_hi) {
-                attn_step<E, 1, 2, true>(lds_k, lds_v, 0, q, st, P.c, lane, key0, pad, key_hi, width);
+        const char* lds_k = lds_kbuf(t & 1);
+        const char* lds_v = lds_vbuf(t & 1);
+        const int n0 = kw * kSub * 32, key0 = t * kTileKeys + n0;
+        if (key0 < wave_hi && key0 + kSub * 32 > pad) {
+            if (key0 >= pad && key0 + kSub * 32 <= wave_hi_min) {
+                attn_step<E, 1, kSub, false>(lds_k, lds_v, n0, q, st, P.c, lane, key0, pad, key_hi, width);
+            } else if (kSub == 2 && key0 + 32 < wave_hi) {
+                attn_step<E, 1, kSub, true>(lds_k, lds_v, n0, q, st, P.c, lane, key0, pad, key_hi, width);
             } else {
-                attn_step<E, 1, 1, true>(lds_k, lds_v, 0, q, st, P.c, lane, key0, pad, key_hi, width);
+                attn_step<E, 1, 1, true>(lds_k, lds_v, n0, q, st, P.c, lane, key0, pad, key_hi, width);
             }
         }
         if (t + 1 < n_tiles) {
             // the other buffer was last read in iteration t-1, which every wavefront has left
-            store_tile<kTileKeys, kThreads>(lds_kbuf[(t + 1) & 1], lds_vbuf[(t + 1) & 1], regs, tid);
+            store_tile<kTileKeys, kThreads>(lds_kbuf((t + 1) & 1), lds_vbuf((t + 1) & 1), regs, tid);
             if (t + 2 < n_tiles) fetch(t + 2);
         }
         __syncthreads();
@@ -314,11 +328,60 @@ __global__ __launch_bounds__(kThreads, 2) void staircase_attn_kernel(const Stair
     // hundred tokens).  Each wavefront therefore turns its 32 x 128 tile around through one of the four K / V tile
     // buffers (the loop's last barrier has retired them) and writes whole rows: 16 lanes x 16 bytes per row, four rows
     // per instruction.  LDS operations of a wavefront complete in order, so its reads see all of its writes.
-    const float inv = 1.0f / both_halves_sum(st.l[0]);          // rows outside the sequence: never stored
-    if (P.o_rows16) {
-        char* tile = (wave & 2) ? lds_vbuf[wave & 1] : lds_kbuf[wave & 1];
+    float l_all = both_halves_sum(st.l[0]);
+    if constexpr (KW > 1) {
+        // the KW wavefronts of a row tile exchange their states: each keeps, folded, the d tiles kw, kw + KW, ...
+        constexpr int kSlots = 2;                              // d tiles that a wavefront hands out: the other one's half of the four
+        static_assert(KW == 2, "the exchange is written for two wavefronts");
+        float* xch = reinterpret_cast<float*>(lds);            // per wavefront: kSlots x [group][lane] of four floats, then m, l per lane
+        constexpr int kXch = kSlots * 16 * 64 + 2 * 64;
+        static_assert(4 * kXch * (int)sizeof(float) + (4 / KW) * 32 * kLdsPitch <= 4 * kTileBytes, "no room for the exchange");
+        float* mine = xch + wave * kXch;
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
+        for (int dt = 0; dt < 4; ++dt) {
+            if (dt % KW == kw) continue;
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                *reinterpret_cast<f32x4*>(mine + (((dt >> 1) * 4 + g) * 64 + lane) * 4) =
+                    f32x4{st.o[0][dt][4 * g], st.o[0][dt][4 * g + 1], st.o[0][dt][4 * g + 2], st.o[0][dt][4 * g + 3]};
+        }
+        mine[kSlots * 16 * 64 + lane] = st.m[0];
+        mine[kSlots * 16 * 64 + 64 + lane] = l_all;
+        __syncthreads();
+        float w[KW], M = kMinusBig;
+#pragma unroll
+        for (int s = 0; s < KW; ++s) { w[s] = xch[(wave - kw + s) * kXch + kSlots * 16 * 64 + lane]; M = fmaxf(M, w[s]); }
+        l_all = 0.f;
+#pragma unroll
+        for (int s = 0; s < KW; ++s) {
+            w[s] = __builtin_amdgcn_exp2f(w[s] - M);
+            l_all += w[s] * xch[(wave - kw + s) * kXch + kSlots * 16 * 64 + 64 + lane];
+        }
+        const float own = __builtin_amdgcn_exp2f(st.m[0] - M);
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) {
+            if (dt % KW != kw) continue;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) st.o[0][dt][i] *= own;
+#pragma unroll
+            for (int s = 0; s < KW; ++s) {
+                if (s == kw) continue;
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const f32x4 x = *reinterpret_cast<const f32x4*>(xch + (wave - kw + s) * kXch + (((dt >> 1) * 4 + g) * 64 + lane) * 4);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) st.o[0][dt][4 * g + e] += w[s] * x[e];
+                }
+            }
+        }
+    }
+    const float inv = 1.0f / l_all;                             // rows outside the sequence: never stored
+    if (P.o_rows16) {
+        // KW == 1: one of the four K / V tile buffers per wavefront; else behind the exchange
+        char* tile = KW == 1 ? lds + wave * kTileBytes : lds + 4 * kTileBytes - (wave / KW + 1) * 32 * kLdsPitch;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) {
+            if (dt % KW != kw) continue;
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 typename Elem16<E>::vec4 out;
@@ -326,12 +389,14 @@ __global__ __launch_bounds__(kThreads, 2) void staircase_attn_kernel(const Stair
                 for (int e = 0; e < 4; ++e) out[e] = (E)(st.o[0][dt][4 * g + e] * inv);
                 *reinterpret_cast<typename Elem16<E>::vec4*>(tile + r * kLdsPitch + d_of_reg(dt, 4 * g, H) * 2) = out;
             }
-        __builtin_amdgcn_wave_barrier();
+        }
+        if (KW > 1) __syncthreads();
+        else __builtin_amdgcn_wave_barrier();
         const int chunk16 = lane & 15, sub = lane >> 4;
         if (!NARROW || chunk16 * 8 < width) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int rho = 4 * j + sub;                    // row of the wavefront's tile
+            for (int j = 0; j < 8 / KW; ++j) {
+                const int rho = 4 * (KW * j + kw) + sub;        // row of the row tile
                 const int jp = row_w0 + rho;
                 const u32x4 v = *reinterpret_cast<const u32x4*>(tile + rho * kLdsPitch + chunk16 * 16);
                 if (jp >= pad && jp < Lp)
@@ -343,7 +408,8 @@ __global__ __launch_bounds__(kThreads, 2) void staircase_attn_kernel(const Stair
     if (!row_ok) return;
     __bf16* orow = P.o + tok * P.o_st + (int64_t)head * P.o_sh;
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
+    for (int dt = 0; dt < 4; ++dt) {
+        if (dt % KW != kw) continue;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             typename Elem16<E>::vec4 out;
@@ -351,6 +417,7 @@ __global__ __launch_bounds__(kThreads, 2) void staircase_attn_kernel(const Stair
             for (int e = 0; e < 4; ++e) out[e] = (E)(st.o[0][dt][4 * g + e] * inv);
             if (!NARROW || d_of_reg(dt, 4 * g, H) < width) *reinterpret_cast<typename Elem16<E>::vec4*>(orow + d_of_reg(dt, 4 * g, H)) = out;
         }
+    }
 }
 
 
@@ -391,12 +458,9 @@ __global__ __launch_bounds__(kThreads, 1) void staircase_pair_kernel(const Stair
     // slower although it saves the launch gap between two workgroups of a CU).
     const int item = blockIdx.x;
     const int hslot = item % n_hslots;
-    int b, rg;
+    int b, rg, seq0, L;
     // (scratch for the numbering: in slot 4, which no K/V load targets before every wavefront has passed the core's first barrier)
-    if (!locate_row_group(P, item / n_hslots, lane, reinterpret_cast<int*>(lds_pair + 4 * (2 * kTileKeys * kRowBytes)) + wave * 80, b, rg)) return;
-
-    int seq0, L;
-    seq_bounds(P, b, seq0, L);
+    if (!locate_row_group<kRowsPerWg>(P, item / n_hslots, lane, reinterpret_cast<int*>(lds_pair + 4 * (2 * kTileKeys * kRowBytes)) + wave * 80, b, rg, seq0, L)) return;
     if (L <= 0) return;
     const int S = 1 << P.log2_s;
     const int Lp = ((L + S - 1) >> P.log2_s) << P.log2_s;
@@ -475,6 +539,14 @@ int launch_staircase_f32(const void* q, const void* k, const void* v, void* o,
 
 namespace {
 
+template <typename E>
+void launch_one_head(const StaircaseParams& P, bool narrow, int kw, unsigned grid, hipStream_t stream)
+{
+    if (narrow)       staircase_attn_kernel<E, true, 1><<<grid, kThreads, 0, stream>>>(P);
+    else if (kw == 1) staircase_attn_kernel<E, false, 1><<<grid, kThreads, 0, stream>>>(P);
+    else              staircase_attn_kernel<E, false, 2><<<grid, kThreads, 0, stream>>>(P);
+}
+
 // `store`: rows to copy in the same launch, or null; *stored says whether the launch took them along.
 int staircase(const void* q, const void* k, const void* v, void* o,
                                          int64_t q_stride_t, int64_t q_stride_h,
@@ -516,7 +588,15 @@ int staircase(const void* q, const void* k, const void* v, void* o,
                 v_stride_t % 8 == 0 && v_stride_h % 8 == 0 && o_stride_t % 4 == 0 && o_stride_h % 4 == 0,
                 MDX_EUNSUPPORTED, "staircase_attn: q/k/v/o must be 16-byte aligned with strides that are multiples of 8 elements");
 
-    const int rows_per_wg = kRowsPerWg;
+    const bool narrow = head_dim < kHeadDim;                   // one-head kernel, rows padded with zeros
+    // workgroups that row groups of `rows` rows come to, at most: ceil((L_b + S - 1) / rows) row groups per sequence
+    const int64_t max_l = max_seqlen < total_tokens ? max_seqlen : total_tokens;
+    auto groups_in = [&](int rows) { return (total_tokens + (int64_t)batch * (staircase_size + rows - 2)) / rows; };
+    // Two wavefronts per row tile while their workgroups (half the rows) are all on the chip at once, two per CU: such a launch
+    // lasts as long as the longest chain of key tiles, which the split shortens (us, without / with: 200 tokens 10.6 / 8.6, 500
+    // 17.4 / 13.0, 1000 28 / 21, 2000 46 / 39, 2 x 1000 28 / 23, 4 x 300 12.0 / 11.3); beyond, it only stages the keys more often
+    // (4 x 1000 30 / 37, 8 x 300 13 / 16, 32 x 100 11 / 15).
+    const int kw = !narrow && groups_in(kRowsPerWg / 2) * num_q_heads <= 2 * (int64_t)mdx::compute_units() ? 2 : 1, rows_per_wg = kRowsPerWg / kw;
     StaircaseParams P;
     P.q = (const __bf16*)q; P.k = (const __bf16*)k; P.v = (const __bf16*)v; P.o = (__bf16*)o;
     P.q_st = q_stride_t; P.q_sh = q_stride_h; P.k_st = k_stride_t; P.k_sh = k_stride_h;
@@ -524,7 +604,6 @@ int staircase(const void* q, const void* k, const void* v, void* o,
     P.cu_seqlens = cu_seqlens_k;
     P.total_tokens = (int)total_tokens;
     P.batch = batch;
-    const int64_t max_l = max_seqlen < total_tokens ? max_seqlen : total_tokens;
     P.n_row_groups = (int)((max_l + staircase_size - 1 + rows_per_wg - 1) / rows_per_wg);
     P.num_q_heads = num_q_heads;
     P.num_kv_heads = num_kv_heads;
@@ -532,9 +611,8 @@ int staircase(const void* q, const void* k, const void* v, void* o,
     P.o_rows16 = (o_stride_t % 8 == 0 && o_stride_h % 8 == 0) ? 1 : 0;
     P.log2_s = log2_s;
     P.c = scale * kLog2e;
-    // dense numbering: at most ceil((L_b + S - 1) / rows) row groups per sequence
     const bool dense = batch <= 64 || (P.n_row_groups <= 64 && batch <= kDenseMaxBatch);
-    const int64_t n_pairs = dense ? (total_tokens + (int64_t)batch * (staircase_size + rows_per_wg - 2)) / rows_per_wg
+    const int64_t n_pairs = dense ? groups_in(rows_per_wg)
                                   : (int64_t)P.n_row_groups * batch;
     // Two query heads per wavefront when the heads of a KV head pair up and 32-bit row offsets suffice.
     const int64_t row_elems = k_stride_t > v_stride_t ? k_stride_t : v_stride_t;
@@ -542,9 +620,8 @@ int staircase(const void* q, const void* k, const void* v, void* o,
     // prologue, epilogue: 10 us) is then most of its time, while two one-head workgroups share a CU and hide each
     // other's (one-head against pair, ms: 64 x 300 tokens 0.088 / 0.103, 32 x 500 0.074 / 0.081, 64 x 600 0.222 / 0.216,
     // 32 x 700 0.130 / 0.128, 32 x 800 0.162 / 0.155, 32 x 1000 0.230 / 0.204, 16 x 2048 0.383 / 0.304).
-    const bool narrow = head_dim < kHeadDim;                   // one-head kernel, rows padded with zeros
     // (its epilogue writes rows of o in 16-byte pieces, through 32-bit byte offsets from the wavefront's first row)
-    const bool pairs = !narrow && max_l > 560 && o_stride_t % 8 == 0 && o_stride_h % 8 == 0 && o_stride_t > 0 &&
+    const bool pairs = kw == 1 && !narrow && max_l > 560 && o_stride_t % 8 == 0 && o_stride_h % 8 == 0 && o_stride_t > 0 &&
                        o_stride_t * 2 * 128 < ((int64_t)1 << 31) && (num_q_heads / num_kv_heads) % 2 == 0 && k_stride_t > 0 && v_stride_t > 0 &&
                        (max_l + 2 * rows_per_wg) * row_elems * 2 < ((int64_t)1 << 31) && row_elems * 2 < (1 << 24) && max_l + 2 * rows_per_wg < (1 << 24);
     int64_t grid = n_pairs * (pairs ? num_q_heads / 2 : num_q_heads);
@@ -577,11 +654,9 @@ int staircase(const void* q, const void* k, const void* v, void* o,
         if (half) staircase_pair_kernel<_Float16><<<(unsigned)grid, kThreads, kPairLdsBytes, stream>>>(P);
         else      staircase_pair_kernel<__bf16><<<(unsigned)grid, kThreads, kPairLdsBytes, stream>>>(P);
     } else if (dtype == MDX_F16) {
-        if (narrow) staircase_attn_kernel<_Float16, true><<<(unsigned)grid, kThreads, 0, stream>>>(P);
-        else        staircase_attn_kernel<_Float16, false><<<(unsigned)grid, kThreads, 0, stream>>>(P);
+        launch_one_head<_Float16>(P, narrow, kw, (unsigned)grid, stream);
     } else {
-        if (narrow) staircase_attn_kernel<__bf16, true><<<(unsigned)grid, kThreads, 0, stream>>>(P);
-        else        staircase_attn_kernel<__bf16, false><<<(unsigned)grid, kThreads, 0, stream>>>(P);
+        launch_one_head<__bf16>(P, narrow, kw, (unsigned)grid, stream);
     }
     return mdx::check_launch("staircase_attn");
 }

@@ -51,6 +51,15 @@ def test_prefill_all_staircase_sizes(dev, S):
     _check_prefill(dev, [203, 77, 1, 160], S, seed=S)
 
 
+@pytest.mark.parametrize("S", [1, 8, 32, 128])
+@pytest.mark.parametrize("lens,bound", [([63, 64, 65, 1, 129, 500], None), ([2047], None), ([1, 31, 33, 63, 64, 65, 127, 128, 129, 257] * 4, None),
+                                        ([1, 31, 33, 63, 64, 65, 127, 128, 129, 257] * 4, 1024), ([203, 77, 1, 160] * 6, 1024)])
+def test_prefill_row_tiles_of_one_and_two_wavefronts(dev, lens, bound, S):
+    """Few row groups: two wavefronts share a row tile's keys.  Many: the one-head kernel with a wavefront per row tile, and, with
+    a large enough (still valid) bound, the kernel for pairs of heads."""
+    _check_prefill(dev, lens, S, seed=sum(lens) + S, max_seqlen=bound)
+
+
 @pytest.mark.parametrize("hq,hkv", [(16, 8), (8, 8), (4, 1), (3, 1), (2, 2)])
 def test_prefill_gqa_ratios(dev, hq, hkv):
     _check_prefill(dev, [150, 97], 32, hq=hq, hkv=hkv, seed=hq * 10 + hkv)
