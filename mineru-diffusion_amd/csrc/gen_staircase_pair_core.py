@@ -373,26 +373,45 @@ def qk0_block(out):
             rg.read(out, n + RING_DEPTH, items[n + RING_DEPTH], n + RING_DEPTH)
 
 
-def prologue():
+def issue(slot):
+    """A tile's loads, with what has to stand between the M0 writes and the loads, then the addresses of the next tile."""
     out = []
-    out += [f"v_mov_b32_e32 {NEG_INF}, 0xff800000", f"v_mov_b32_e32 {VPAD}, %[pad]", f"v_mov_b32_e32 {VLPM1}, %[lpm1]",
-            f"v_mov_b32_e32 {MREL}, %[mrel]", f"v_mov_b32_e32 {JPL}, %[jpl]"]
+    for first, last in dma_ops(slot):
+        out += first + ["s_nop 0"] + last
+    return out + load_offset_ops()
+
+
+def start_program():
+    """What the wavefront waits for first, on its way at once: its rows of Q (to registers, in the caller's hands from here), then
+    tile 0.  Returns when Q has landed; the caller scales it while tile 0 arrives."""
+    out = [f"v_mov_b32_e32 {VPAD}, %[pad]", f"v_mov_b32_e32 {VLPM1}, %[lpm1]", f"v_mov_b32_e32 {JPL}, %[jpl]", f"s_mov_b32 {S_R0}, 0"]
+    out += load_offset_ops()
+    for h in range(2):
+        for ks in range(8):
+            out.append(f"global_load_dwordx4 %[q{h}{ks}], %[qp{h}], off" + (f" offset:{32 * ks}" if ks else ""))
+    for first, last in dma_ops(S_R0):
+        out += first + ["s_nop 0"] + last
+    out.append(f"s_waitcnt vmcnt({DMA_PER_TILE})")
+    return out
+
+
+def prologue():
+    out = [f"v_mov_b32_e32 {NEG_INF}, 0xff800000", f"v_mov_b32_e32 {VPAD}, %[pad]", f"v_mov_b32_e32 {VLPM1}, %[lpm1]",
+            f"v_mov_b32_e32 {MREL}, %[mrel]", f"v_add_u32_e32 {JPL}, 64, %[jpl]"]
     out += [f"s_mov_b32 {S_T}, 0", f"s_mov_b32 {S_KEY0}, 0", f"s_mov_b32 {S_R0}, 0", f"s_mov_b32 {S_R1}, {SLOT}",
             f"s_mov_b32 {S_R2}, {2 * SLOT}", f"s_mov_b32 {S_R3}, {3 * SLOT}", f"s_mov_b32 {S_R4}, {4 * SLOT}"]
-    # tiles 0..3 -> slots 0..3; addresses of tile 4 prepared
-    for slot in (S_R0, S_R1, S_R2, S_R3):
-        out += load_offset_ops()
-        for first, last in dma_ops(slot):
-            out += first + ["s_nop 0"] + last
-    out += load_offset_ops()
+    # Tile 0 is on its way (start_program); the others follow one stage ahead of their use: a compute unit takes in about 20 bytes
+    # per cycle, so that four tiles at once would hold up the first by 6000 cycles.
+    out += load_offset_ops() + issue(S_R1)
     for i in range(2):
         out.append(f"v_mov_b32_e32 v{52 + i}, {ONE_PAIR}")
     for i in list(range(128)) + [192 + 16 * h + j for h in range(2) for j in range(L_REGS)]:
         out.append(f"v_accvgpr_write_b32 a{i}, 0")
-    out += [f"s_waitcnt vmcnt({2 * DMA_PER_TILE})", "s_barrier"]      # tiles 0 and 1 have landed
+    out += [f"s_waitcnt vmcnt({DMA_PER_TILE})", "s_barrier"]          # tile 0 has landed
     # QK(0) with C = 0, then m = row max of tile 0: -m tuples and S[0] -= m
     out += k_address_ops(S_R0)
     qk0_block(out)
+    out += issue(S_R2)
     out.append("s_nop 15")
     # m starts as the maximum over the keys each query may see: when the wavefront's first limit lies
     # inside tile 0 the hidden keys are taken out first (keys before the sequence are copies of its
@@ -411,6 +430,8 @@ def prologue():
         out.append(f"v_mov_b32_e32 {MX[h]}, 0")
     # iteration 0 starts with its first K fragments (tile 1) in flight
     out += k_address_ops(S_R1) + v_address_ops(S_R0)
+    out += issue(S_R3)                                                  # leaves the addresses of tile 4
+    out += [f"s_waitcnt vmcnt({2 * DMA_PER_TILE})", "s_barrier"]      # tile 1 has landed
     items = qk_items(1)
     for n in range(RING_DEPTH):
         out += items[n][0](ring(n))
@@ -635,10 +656,11 @@ def program():
 HEADER = '''// GENERATED by gen_staircase_pair_core.py -- do not edit; change the generator and regenerate.
 //
 // Key loop of the staircase attention kernel for a pair of query heads (see the generator's
-// docstring for the schedule, the LDS layout and the register map).  Everything between the loads
-// of Q and the stores of O happens inside this one asm statement; the physical registers it uses
-// are declared as clobbers, the operands are read-only.
-@@STRUCT@@__device__ __forceinline__ void @@NAME@@(const PairCoreArgs& A, const @@VEC@@ (&q)[2][8])
+// docstring for the schedule, the LDS layout and the register map).  The first asm statement issues the
+// loads of Q and of the first tile and waits for Q, which comes back as loaded; everything from there to the
+// stores of O happens inside the second one, which counts on the first's loads being the only ones in flight.  The physical
+// registers that they use are declared as clobbers, the operands are read-only.
+@@STRUCT@@@@START@@__device__ __forceinline__ void @@NAME@@(const PairCoreArgs& A, const @@VEC@@ (&q)[2][8])
 {
     asm volatile(
 '''
@@ -670,6 +692,20 @@ def main():
     vclob = ", ".join(f'"v{r}"' for r in range(16, 256))
     aclob = ", ".join(f'"a{r}"' for r in list(range(0, 128)) + list(range(192, 224)))
     sclob = ", ".join(f'"s{r}"' for r in range(40, 56))
+    start = "\n".join(f'        "{line}\\n"' for line in start_program())
+    start_out = ", ".join(f'[q{h}{ks}] "=&v"(q[{h}][{ks}])' for h in range(2) for ks in range(8))
+    start_clob = ", ".join(f'"v{r}"' for r in [22, 40, 41, 42, *range(56, 64)])
+    begin = f'''__device__ __forceinline__ void @@NAME@@_start(const PairCoreArgs& A, const void* q0, const void* q1, u32x4 (&q)[2][8])
+{{
+    asm volatile(
+{start}
+        : {start_out}
+        : [qp0] "v"(q0), [qp1] "v"(q1), [jpl] "v"(A.jpl), [ch] "v"(A.ch), [kb] "s"(A.kb), [vb] "s"(A.vb), [krb] "s"(A.krb), [vrb] "s"(A.vrb),
+          [wrow] "s"(A.wrow), [pad] "s"(A.pad), [lpm1] "s"(A.lpm1)
+        : "memory", "scc", "m0", {sclob}, {start_clob});
+}}
+
+'''
     tail = f'''
         :
         : [ka] "v"(A.ka), [val] "v"(A.val), [vah] "v"(A.vah), [jpl] "v"(A.jpl), [ch] "v"(A.ch),
@@ -684,6 +720,7 @@ def main():
 }}
 '''
     header = HEADER.replace("@@STRUCT@@", STRUCT if DT == "bf16" else "// (PairCoreArgs: see staircase_pair_core.inc, which is included first)\n\n")
+    header = header.replace("@@START@@", begin if DT == "bf16" else "")
     header = header.replace("@@NAME@@", "staircase_pair_core" if DT == "bf16" else "staircase_pair_core_f16").replace("@@VEC@@", "bf16x8" if DT == "bf16" else "f16x8")
     if DT != "bf16":
         header = header.replace("gen_staircase_pair_core.py --", "gen_staircase_pair_core.py f16 --")

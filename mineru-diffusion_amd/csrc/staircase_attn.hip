@@ -475,18 +475,6 @@ __global__ __launch_bounds__(kThreads, 1) void staircase_pair_kernel(const Stair
     const int row_w0 = row_g0 + wave * 32;
     const int ip = row_w0 + r;
     const bool row_ok = ip >= pad && ip < Lp;
-    const int64_t tok = (int64_t)seq0 + (ip - pad);
-    // Q^T fragments, pre-multiplied by scale * log2(e) (the MFMA then yields scores in log2 units)
-    typename Elem16<E>::vec8 q[2][8];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        load_q(q[h], row_ok ? P.q + tok * P.q_st + (int64_t)(head0 + h) * P.q_sh : nullptr, H);
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) q[h][ks][j] = (E)((float)q[h][ks][j] * P.c);
-    }
-
     auto limit_of = [&](int row) { return min(Lp, ((row >> P.log2_s) + 1) << P.log2_s); };
     const int wg_hi = limit_of(min(row_g0 + kRowsPerWg - 1, Lp - 1));
 
@@ -523,6 +511,20 @@ __global__ __launch_bounds__(kThreads, 1) void staircase_pair_kernel(const Stair
     A.nt = uniform((wg_hi + kTileKeys - 1) / kTileKeys);
     A.whm = uniform(limit_of(min(row_w0, Lp - 1)));
     A.whx = uniform(row_w0 < Lp ? limit_of(min(row_w0 + 31, Lp - 1)) : 0);   // tiles from here on hold nothing this wavefront may see
+    // Q^T fragments, pre-multiplied by scale * log2(e) (the MFMA then yields scores in log2 units); rows outside the sequence: zeros
+    u32x4 raw[2][8];
+    const __bf16* qrow = P.q + ((int64_t)seq0 + min(max(ip - pad, 0), L - 1)) * P.q_st + (int64_t)head0 * P.q_sh + H * 8;
+    staircase_pair_core_start(A, qrow, qrow + P.q_sh, raw);
+    const float c = row_ok ? P.c : 0.f;
+    typename Elem16<E>::vec8 q[2][8];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks) {
+            q[h][ks] = __builtin_bit_cast(typename Elem16<E>::vec8, raw[h][ks]);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) q[h][ks][j] = (E)((float)q[h][ks][j] * c);
+        }
     pair_core(A, q);
 }
 
