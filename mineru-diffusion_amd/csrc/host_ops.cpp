@@ -466,33 +466,6 @@ PyObject* flash_attn_with_kvcache(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // ---- the attention layer --------------------------------------------------------------------------
-// The prefill store runs beside the attention launch, on one extra stream per device (default priority), from this many
-// tokens on: its small workgroups fill the gaps between the attention kernel's, which own whole CUs (38 690 tokens,
-// store + attention: 0.820 -> 0.808 ms).  Two event records and two waits, 8 us of host time and as much of the GPU's
-// between the launches, are what that costs, so fewer tokens are stored on the caller's stream (short prompts in the attention launch).
-constexpr int64_t kSideStoreTokens = 16384;
-
-struct Side {
-    hipStream_t stream;
-    hipEvent_t fork, join;
-};
-
-Side* side_of(int device) {
-    // per thread: an event is recorded and waited for in one call, and calls of different threads must not share it
-    thread_local std::map<int, Side> sides;
-    auto it = sides.find(device);
-    if (it != sides.end()) return &it->second;
-    Side s;
-    s.stream = c10::hip::getStreamFromPool(false, (c10::DeviceIndex)device).stream();
-    if (hipEventCreateWithFlags(&s.fork, hipEventDisableTiming) != hipSuccess || hipEventCreateWithFlags(&s.join, hipEventDisableTiming) != hipSuccess)
-        raise_mdx("attention: cannot create an event");
-    return &sides.emplace(device, s).first->second;
-}
-
-void chain(hipStream_t from, hipEvent_t event, hipStream_t to) {
-    if (hipEventRecord(event, from) != hipSuccess || hipStreamWaitEvent(to, event, 0) != hipSuccess) raise_mdx("attention: cannot order two streams");
-}
-
 // q, k, v, k_cache, v_cache, slot_mapping, cu_seqlens_q, cu_seqlens_k, block_size, max_seqlen, scale -> o [N, Hq * d]
 PyObject* attention_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
     ARGS(11);
@@ -503,23 +476,8 @@ PyObject* attention_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const Tensor &cu_q = tensor(a[6]), &cu_k = tensor(a[7]);
         const int64_t S = integer(a[8]), max_seqlen = integer(a[9]);
         if (!have_cache) return wrap(staircase(q, k, v, cu_q, cu_k, S, max_seqlen, a[10], true));
-        if (q.dim() != 3 || q.size(0) < kSideStoreTokens) {
-            const Caches caches{k_cache, v_cache, tensor(a[5])};
-            return wrap(staircase(q, k, v, cu_q, cu_k, S, max_seqlen, a[10], true, &caches));
-        }
-        Side* side = side_of(q.device().index());
-        hipStream_t main = static_cast<hipStream_t>(stream_of(q));
-        chain(main, side->fork, side->stream);
-        Tensor o;
-        try {
-            store(k, v, k_cache, v_cache, tensor(a[5]), side->stream);
-            o = staircase(q, k, v, cu_q, cu_k, S, max_seqlen, a[10], true);
-        } catch (...) {
-            chain(side->stream, side->join, main);
-            throw;
-        }
-        chain(side->stream, side->join, main);
-        return wrap(std::move(o));
+        const Caches caches{k_cache, v_cache, tensor(a[5])};
+        return wrap(staircase(q, k, v, cu_q, cu_k, S, max_seqlen, a[10], true, &caches));
     });
 }
 

@@ -38,9 +38,10 @@ constexpr int kTileKeys = 64;      // keys staged in LDS per iteration
 constexpr int kThreads = 256;      // 4 wavefronts, 2 workgroups per CU
 constexpr int kRowsPerWg = 128;    // 4 wavefronts x 32 query rows
 
-// The K/V rows of a short prompt's layer go to the paged cache in the attention launch itself (mdx_staircase_attn_store): the
+// The K/V rows of a layer go to the paged cache in the attention launch itself (mdx_staircase_attn_store): the
 // attention reads k and v, not the cache, so the rows are copied by workgroups behind the attention's, which find the chip
-// far from full (109 tokens are 16 attention workgroups), and the launch of the store, 2.4 us of an 11-us layer, is saved.
+// far from full (109 tokens are 16 attention workgroups), and the launch of the store, 2.4 us of an 11-us layer, is saved.  (The pair
+// kernel on a full chip: store_own_rows.)
 constexpr int kStoreTokens = 16;                               // tokens per workgroup at most: 16 loads of 16 bytes in flight per lane
 struct StoreParams {
     const u32x4* key; const u32x4* value;
@@ -49,6 +50,7 @@ struct StoreParams {
     const int32_t* slot_mapping; int64_t num_slots;
     int n_tokens, row16, tokens_per_wg;                        // row16: 16-byte units of a token's row, a divisor of kThreads / 2
     int first_wg;                                              // workgroups from here on copy rows
+    int own_rows;                                              // pair kernel: 1 each workgroup copies its own rows, 0 those from first_wg on do
 };
 
 struct StaircaseParams {
@@ -96,6 +98,64 @@ __device__ __forceinline__ void seq_bounds(const StaircaseParams& P, int b, int&
     const int hi = min(max(P.cu_seqlens[b + 1], lo), P.total_tokens);
     seq0 = lo;
     L = hi - lo;
+}
+
+// Tokens that no row group of the pair kernel owns: before the first sequence, behind the last one, and past max_seqlen.
+// Mostly there are none, and a few workgroups that look are enough.
+constexpr int kUnownedWgs = 8;
+__device__ __forceinline__ void store_unowned_rows(const StaircaseParams& P, int wg, int tid)
+{
+    const int S = 1 << P.log2_s, row16 = P.store.row16;
+    for (int b = wg; b < P.batch + 2; b += kUnownedWgs) {
+        int begin = 0, end = P.total_tokens;
+        if (b == P.batch) end = min(max(P.cu_seqlens[0], 0), end);
+        else if (b == P.batch + 1) begin = min(max(P.cu_seqlens[P.batch], 0), end);
+        else {
+            int seq0, L;
+            seq_bounds(P, b, seq0, L);
+            const int pad = (((L + S - 1) >> P.log2_s) << P.log2_s) - L;
+            begin = seq0 + min(L, P.n_row_groups * kRowsPerWg - pad);
+            end = seq0 + L;
+        }
+        for (int64_t i = tid; i < (int64_t)(end - begin) * row16; i += kThreads) {
+            const int64_t tok = begin + i / row16, slot = P.store.slot_mapping[tok];
+            const int col = (int)(i % row16);
+            if (slot < 0 || slot >= P.store.num_slots) continue;
+            P.store.k_cache[slot * row16 + col] = P.store.key[tok * P.store.k_stride16 + col];
+            P.store.v_cache[slot * row16 + col] = P.store.value[tok * P.store.v_stride16 + col];
+        }
+    }
+}
+
+// The same for the pair kernel, whose workgroups own whole CUs: store workgroups behind them would hold a CU each and start when the
+// attention is done, and cost what a launch of their own costs.  But the K / V rows of a row group's own tokens are the last that
+// its key loop has read, so the workgroup of the KV head's first pair copies them (64 KB, from L2) when it is through: 1.5 us a
+// workgroup.  Store + attention, us, as two launches / here: 6 prompts of 900-1500 tokens 63.5 / 58.3, 6 x 1167 58.5 / 52.5, 4 x 2000
+// 83.7 / 77, 20 x 800 115 / 108, 8 x 1800 154 / 144; against a store on a second stream beside the attention: 32 x 800 193 / 188, 8
+// prompts of 1024-8192 level at 744.
+__device__ __forceinline__ void store_own_rows(const StoreParams& S, int kvh, int seq0, int begin, int end, int tid)
+{
+    constexpr int kRounds = kRowsPerWg / (kThreads / 16);
+    const int col = kvh * (kHeadDim / 8) + (tid & 15);
+    u32x4 k[kRounds], v[kRounds];
+    int64_t slot[kRounds];
+#pragma unroll
+    for (int i = 0; i < kRounds; ++i) {
+        const int t = begin + i * (kThreads / 16) + (tid >> 4);
+        slot[i] = -1;
+        if (t < end) {
+            const int64_t tok = (int64_t)seq0 + t;
+            slot[i] = S.slot_mapping[tok];
+            k[i] = S.key[tok * S.k_stride16 + col];
+            v[i] = S.value[tok * S.v_stride16 + col];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < kRounds; ++i) {
+        if (slot[i] < 0 || slot[i] >= S.num_slots) continue;
+        __builtin_nontemporal_store(k[i], S.k_cache + slot[i] * S.row16 + col);
+        __builtin_nontemporal_store(v[i], S.v_cache + slot[i] * S.row16 + col);
+    }
 }
 
 // Workgroup -> (sequence b, row group rg) for the j-th (sequence, row group) pair in launch order.
@@ -453,6 +513,13 @@ __global__ __launch_bounds__(kThreads, 1) void staircase_pair_kernel(const Stair
     const int H = lane >> 5, r = lane & 31;
     const int n_hslots = P.num_q_heads / 2;
 
+    if ((int)blockIdx.x >= P.store.first_wg) {
+        const int wg = (int)blockIdx.x - P.store.first_wg;
+        if (P.store.own_rows) store_unowned_rows(P, wg, tid);
+        else store_rows(P.store, wg, tid);
+        return;
+    }
+
     // One work item per workgroup: the dispatcher hands the next item to whichever CU frees up
     // first, which balances the ragged item lengths (a fixed item -> CU assignment measured 10%
     // slower although it saves the launch gap between two workgroups of a CU).
@@ -526,6 +593,7 @@ __global__ __launch_bounds__(kThreads, 1) void staircase_pair_kernel(const Stair
             for (int j = 0; j < 8; ++j) q[h][ks][j] = (E)((float)q[h][ks][j] * c);
         }
     pair_core(A, q);
+    if (P.store.own_rows && hslot < P.num_kv_heads) store_own_rows(P.store, kvh, seq0, max(0, row_g0 - pad), min(L, row_g0 - pad + kRowsPerWg), tid);
 }
 
 }  // namespace
@@ -629,13 +697,17 @@ int staircase(const void* q, const void* k, const void* v, void* o,
     int64_t grid = n_pairs * (pairs ? num_q_heads / 2 : num_q_heads);
     P.store = StoreParams{};
     P.store.first_wg = 0x7fffffff;
-    if (store && !pairs && grid < ((int64_t)1 << 30)) {
+    if (store && grid < ((int64_t)1 << 30)) {
         P.store = *store;
-        // one token per workgroup while that leaves them few, up to kStoreTokens rounds of rows
-        const int rounds = (store->n_tokens + 511) / 512 < kStoreTokens ? (store->n_tokens + 511) / 512 : kStoreTokens;
-        P.store.tokens_per_wg = rounds * (kThreads / 2 / store->row16);
         P.store.first_wg = (int)grid;
-        grid += (store->n_tokens + P.store.tokens_per_wg - 1) / P.store.tokens_per_wg;
+        // one token per workgroup while that leaves them few, up to kStoreTokens rounds of rows (as many at once beside the pair kernel, which leaves few CUs)
+        const int rounds = !pairs && (store->n_tokens + 511) / 512 < kStoreTokens ? (store->n_tokens + 511) / 512 : kStoreTokens;
+        P.store.tokens_per_wg = rounds * (kThreads / 2 / store->row16);
+        const int64_t wgs = (store->n_tokens + P.store.tokens_per_wg - 1) / P.store.tokens_per_wg;
+        // Pairs: while the attention leaves CUs idle the rows go there (2 x 1000 tokens, 136 workgroups of 256: 29.8 us for the layer,
+        // 31.2 with own rows, which lengthen every chain), as long as those CUs get through them in a few rounds (2 us each).
+        P.store.own_rows = pairs && wgs > 4 * (mdx::compute_units() - grid);
+        grid += P.store.own_rows ? kUnownedWgs : wgs;
         *stored = true;
     }
     MDX_REQUIRE(grid < ((int64_t)1 << 31), MDX_EUNSUPPORTED, "staircase_attn: grid too large");
@@ -704,7 +776,7 @@ extern "C" int mdx_staircase_attn_store(const void* q, const void* k, const void
     StoreParams S{};
     if (along)
         S = StoreParams{(const u32x4*)k, (const u32x4*)v, k_stride_t * elem / 16, v_stride_t * elem / 16, (u32x4*)k_cache, (u32x4*)v_cache,
-                        slot_mapping, num_slots, (int)total_tokens, row16, 0, 0};
+                        slot_mapping, num_slots, (int)total_tokens, row16, 0, 0, 0};
     bool stored = false;
     const int rc = staircase(q, k, v, o, q_stride_t, q_stride_h, k_stride_t, k_stride_h, v_stride_t, v_stride_h, o_stride_t, o_stride_h,
                              cu_seqlens_q, cu_seqlens_k, batch, max_seqlen, total_tokens, num_q_heads, num_kv_heads, head_dim, staircase_size,

@@ -24,7 +24,7 @@ class Attention(nn.Module):
     def forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor):
         context = get_context()
         if context.is_prefill:
-            # the prefill attention reads k / v, not the cache: for long prompts the store runs beside it on a second stream
+            # the prefill attention reads k / v, not the cache: the store rides in its launch where the rows allow it
             return _host().attention_prefill(q, k, v, self.k_cache, self.v_cache, context.slot_mapping, context.cu_seqlens_q,
                                              context.cu_seqlens_k, context.block_size, context.max_seqlen_k or 0, self.scale)
         return _host().attention_decode(q, k, v, self.k_cache, self.v_cache, context.slot_mapping, context.context_lens,

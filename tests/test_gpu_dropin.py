@@ -270,3 +270,40 @@ def test_attention_prefill_is_the_store_and_the_attention(dev, lens, hkv, d, dty
     mdx.store_kvcache(k, v, kc, vc, slots)
     want = mdx.sparse_attn_varlen(q, k, v, cu, cu, S, max_seqlen=max(lens), softmax_scale=d ** -0.5)
     assert torch.equal(o, want.flatten(1)) and torch.equal(attn.k_cache, kc) and torch.equal(attn.v_cache, vc)
+
+
+@pytest.mark.parametrize("lens,hkv,ratio,dtype,before,behind,longest", [
+    ([561], 8, 2, torch.bfloat16, 0, 0, None),                                  # copied by workgroups on idle CUs
+    ([700] * 5, 8, 2, torch.bfloat16, 0, 0, None),                              # from here on by the row groups' workgroups
+    ([1001, 1, 561, 33, 900, 128, 97, 640], 8, 2, torch.float16, 0, 0, None),
+    ([640] * 20, 2, 4, torch.bfloat16, 0, 0, None),                             # two pairs of query heads per KV head
+    ([700, 0, 900, 650, 831, 777], 8, 2, torch.bfloat16, 130, 77, None),        # tokens outside every sequence
+    ([700, 1300, 650, 831, 777, 1025], 8, 2, torch.float16, 1, 3, 850),         # sequences longer than max_seqlen says
+])
+def test_pair_prefill_stores_every_row(dev, lens, hkv, ratio, dtype, before, behind, longest):
+    """Prompts beyond 560 tokens (the kernel for pairs of heads): the rows that ride in its launch, against the store on its own."""
+    import mdx
+    d, N = 128, before + sum(lens) + behind
+    g = torch.Generator(device=dev).manual_seed(N)
+    q, k = (torch.randn(N, h, d, generator=g, device=dev).to(dtype) for h in (ratio * hkv, hkv))
+    v = torch.randn(N, 2 * hkv, d, generator=g, device=dev).to(dtype)[:, hkv:]
+    cu = torch.tensor([before] + [before + int(n) for n in np.cumsum(lens)], dtype=torch.int32, device=dev)
+    pages = N // PAGE + 2
+    slots = torch.randperm(pages * PAGE, generator=g, device=dev)[:N].int()
+    slots[::7] = -1
+    slots[3::11] = pages * PAGE + 5
+    attn = mdx.Attention(ratio * hkv, d, d ** -0.5, hkv)
+    attn.k_cache = torch.zeros(pages, PAGE, hkv, d, dtype=dtype, device=dev)
+    attn.v_cache = torch.zeros_like(attn.k_cache)
+    kc, vc = torch.zeros_like(attn.k_cache), torch.zeros_like(attn.k_cache)
+    longest = longest or max(lens)
+    mdx.set_context(True, cu, cu, longest, longest, slots, None, None, block_size=S)
+    try:
+        o = attn(q, k, v)
+    finally:
+        mdx.reset_context()
+    mdx.store_kvcache(k, v, kc, vc, slots)
+    assert torch.equal(attn.k_cache, kc) and torch.equal(attn.v_cache, vc)
+    if longest == max(lens):
+        want = mdx.sparse_attn_varlen(q, k, v, cu, cu, S, max_seqlen=longest, softmax_scale=d ** -0.5)
+        assert torch.equal(o[before:N - behind], want.flatten(1)[before:N - behind])
