@@ -316,7 +316,8 @@ __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
             // bulk of a peaked row; what is skipped could not have been picked.  (A noise tensor may hold
             // anything: mode 1 reads all of it.)
             if (NOISE == 2) {
-                if ((++since_look & 7) == 0)           // the others' news every eighth chunk: an LDS read per chunk would cost what it saves
+                ++since_look;                          // the others' news at chunks 1, 2, 4, 8, 16, 24, ...: an LDS read per chunk would cost what it saves
+                if ((since_look & min(since_look - 1, 7)) == 0)
                     seen = fmaxf(seen, __hip_atomic_load(&lead_seen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
                 const bool may_lead = (unit_T ? cmx : cmx / T_) + kGumbelMax >= fmaxf(best, seen);
                 if (__builtin_amdgcn_ballot_w64(may_lead) == 0) continue;
@@ -351,13 +352,19 @@ __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
                 uint32_t top = 0;
 #pragma unroll
                 for (int q = 0; q < EPC / 4; ++q) top = max(max(top, max(r[q].x, r[q].y)), max(r[q].z, r[q].w));
-                if (__builtin_amdgcn_ballot_w64((~top >> 9) <= (uint32_t)reach + 1u) == 0) continue;
+                const uint32_t bound = (uint32_t)reach + 1u;
+                if (__builtin_amdgcn_ballot_w64((~top >> 9) <= bound) == 0) continue;
+                // and element by element, since mostly one draw of the wavefront's 512 has passed: two logarithms and a
+                // division instead of sixteen and eight
+                auto offer_draw = [&](float x_, int index, uint32_t bits) {
+                    if ((~bits >> 9) <= bound) offer(x_, index, gumbel_of(bits));
+                };
 #pragma unroll
                 for (int q = 0; q < EPC / 4; ++q) {
-                    offer(x[4 * q + 0], c0 + 4 * q + 0, gumbel_of(r[q].x));
-                    offer(x[4 * q + 1], c0 + 4 * q + 1, gumbel_of(r[q].y));
-                    offer(x[4 * q + 2], c0 + 4 * q + 2, gumbel_of(r[q].z));
-                    offer(x[4 * q + 3], c0 + 4 * q + 3, gumbel_of(r[q].w));
+                    offer_draw(x[4 * q + 0], c0 + 4 * q + 0, r[q].x);
+                    offer_draw(x[4 * q + 1], c0 + 4 * q + 1, r[q].y);
+                    offer_draw(x[4 * q + 2], c0 + 4 * q + 2, r[q].z);
+                    offer_draw(x[4 * q + 3], c0 + 4 * q + 3, r[q].w);
                 }
             } else {
 #pragma unroll
@@ -617,6 +624,23 @@ int pick_nsplit(int64_t rows, int64_t vocab) {
     return (int)n;
 }
 
+// With noise from the generator a launch is bound by arithmetic, and lasts as long as the CUs with the most workgroups do:
+// among the splits from half of pick_nsplit's on (never more: the workspace is sized for those) the largest that leaves the
+// CUs most evenly loaded.  (96 rows: 9 splits put four workgroups on some CUs and three on others, 8 put three on each.)
+// With the logarithms of the few draws that passed only, the sampled step at N(0, 3^2), us, before / after both: 32 rows
+// 24.1 / 19.6, 96 rows 33.7 / 27.1, 256 rows 53.5 / 45.9, 384 rows 75.6 / 62.1, 1024 rows 139.8 / 128.2.
+int pick_nsplit_sampled(int64_t rows, int64_t vocab) {
+    const int most = pick_nsplit(rows, vocab);
+    const int64_t cus = mdx::compute_units();
+    int best = most;
+    double best_load = 0;
+    for (int n = most; n >= 1 && 2 * n >= most; --n) {
+        const double load = (double)((rows * n + cus - 1) / cus) / n;      // the fullest CU's share of the work, up to a constant
+        if (best_load == 0 || load < best_load * 0.97) { best = n; best_load = load; }
+    }
+    return best;
+}
+
 template <typename T, bool FLOOR>
 int launch_confidence(const void* logits, int64_t row_stride, const float* temperatures, int rows_per_temp,
                       const NoiseSpec& N, const float* floors, int64_t* x0, float* x0_p,
@@ -683,7 +707,7 @@ int confidence_pass(const void* logits, int64_t row_stride, int32_t dtype,
     MDX_REQUIRE(!N.noise || N.noise_row_stride >= vocab, MDX_EINVAL, "confidence_argmax: noise_row_stride < vocab");
     const int esz = dtype == MDX_F32 ? 4 : 2;
     MDX_REQUIRE((reinterpret_cast<uintptr_t>(logits) % esz) == 0, MDX_EUNSUPPORTED, "confidence_argmax: logits not element-aligned");
-    const int nsplit = pick_nsplit(rows, vocab);
+    const int nsplit = N.philox ? pick_nsplit_sampled(rows, vocab) : pick_nsplit(rows, vocab);
     if (nsplit_out) *nsplit_out = nsplit;
     const int64_t need = nsplit > 1 ? rows * nsplit * (int64_t)sizeof(Partial) : 0;
     MDX_REQUIRE(need == 0 || (workspace && workspace_bytes >= need), MDX_EWORKSPACE,

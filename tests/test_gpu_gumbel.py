@@ -201,3 +201,18 @@ def test_seeded_sampling_inside_a_graph_steps_with_the_device_offset(dev):
         assert torch.equal(x0, ex0) and torch.equal(p, ep)
         seen.append(x0.clone())
     assert not torch.equal(seen[0], seen[1])
+
+
+@pytest.mark.parametrize("bs,S", [(1, 1), (1, 5), (3, 32), (5, 32), (9, 33)])
+def test_seeded_sampling_with_every_split_count(dev, bs, S):
+    """Splits of a row are chosen from the row count where the noise is drawn in the kernel, differently from where it is read:
+    the same tokens, all of them, and the same confidences but for the order of the sums."""
+    import mdx
+    V = 151936
+    g = torch.Generator(device=dev).manual_seed(bs * S)
+    logits = (torch.randn(bs, S, V, generator=g, device=dev) * 3).to(torch.bfloat16)
+    temps = torch.linspace(0.7, 1.0, bs, device=dev)
+    x0, p = mdx.confidence_argmax(logits, temps, seed=11, offset=3)
+    x0n, pn = mdx.confidence_argmax(logits, temps, noise=mdx.gumbel_noise(bs * S, V, 11, 3, device=dev).view(bs, S, V))
+    assert torch.equal(x0, x0n)
+    torch.testing.assert_close(p, pn, rtol=3e-6, atol=0)
