@@ -196,3 +196,25 @@ def test_filtered_step_is_the_filter_and_the_step(dev, dtype, V, k, p, noise):
         assert torch.equal(got[0], want[0])
         np.testing.assert_allclose(got[1].cpu().numpy(), want[1].cpu().numpy(), rtol=5e-6)
         assert torch.equal(got[2], want[2]) and torch.equal(got[3], want[3]) and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("V", [700, 151936])
+@pytest.mark.parametrize("k", [63, 64, 65, 128, 400, 511, 512])
+@pytest.mark.parametrize("p", [0.5, 0.97, 1.0])
+def test_filtered_step_at_the_edges_of_a_lane_and_a_register(dev, V, k, p):
+    """Kept elements one per lane (up to 64, ties at the cut-off included), eight registers of them (up to 512) and more, from few
+    candidates and many: as above, against the step on the filtered copy."""
+    import mdx
+    g = torch.Generator(device=dev).manual_seed(V + k)
+    logits = (torch.randn(1, 8, V, generator=g, device=dev) * 3).to(torch.bfloat16)
+    logits[0, 1] = (logits[0, 1] * 8).round() / 8
+    logits[0, 2, ::3] = logits[0, 2].max()                   # more ties than are kept
+    logits[0, 3, 5 : 5 + k - 1] = 30.0                       # k - 1 ahead of the rest
+    logits[0, 4, 70 : 70 + k] = 30.0                         # k
+    a = torch.full((1, 8), 9, dtype=torch.int64, device=dev)
+    b = a.clone()
+    got = mdx.unmask_step(logits, a, 9, 0.9, 2, temperatures=None, top_k=k, top_p=p, seed=5, offset=1)
+    want = mdx.unmask_step(mdx.filter_logits(logits, k, p, None), b, 9, 0.9, 2, temperatures=None, seed=5, offset=1)
+    assert torch.equal(got[0], want[0])
+    np.testing.assert_allclose(got[1].cpu().numpy(), want[1].cpu().numpy(), rtol=5e-6)    # as above: fp32 sums in another order
+    assert torch.equal(a, b) and torch.equal(got[3], want[3])
