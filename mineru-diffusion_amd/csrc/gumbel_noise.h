@@ -19,6 +19,10 @@ struct NoiseSpec {
 
 struct U4 { uint32_t x, y, z, w; };
 
+// a ^ b ^ c as one instruction (the compiler makes two of it); 0x96 is the truth table of the three-way exclusive or.  The sampled step,
+// us, with two / one: 96 rows 27.5 / 26.1, 256 rows 46.2 / 42.5, 384 rows 62.1 / 56.5, 1024 rows 127.5 / 114.
+__device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) { return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96); }
+
 __device__ __forceinline__ U4 philox4x32_10(U4 c, uint32_t k0, uint32_t k1) {
 #pragma unroll
     for (int r = 0; r < 10; ++r) {
@@ -26,7 +30,7 @@ __device__ __forceinline__ U4 philox4x32_10(U4 c, uint32_t k0, uint32_t k1) {
         // multiplies are what this generator costs, and the full-width form is 6.5 % faster over a logits pass
         const uint64_t p0 = (uint64_t)0xD2511F53u * (uint64_t)c.x, p1 = (uint64_t)0xCD9E8D57u * (uint64_t)c.z;
         const uint32_t hi0 = (uint32_t)(p0 >> 32), lo0 = (uint32_t)p0, hi1 = (uint32_t)(p1 >> 32), lo1 = (uint32_t)p1;
-        c = U4{hi1 ^ c.y ^ k0, lo1, hi0 ^ c.w ^ k1, lo0};
+        c = U4{xor3(hi1, c.y, k0), lo1, xor3(hi0, c.w, k1), lo0};
         k0 += 0x9E3779B9u;
         k1 += 0xBB67AE85u;
     }
