@@ -666,7 +666,12 @@ int staircase(const void* q, const void* k, const void* v, void* o,
     // lasts as long as the longest chain of key tiles, which the split shortens (us, without / with: 200 tokens 10.6 / 8.6, 500
     // 17.4 / 13.0, 1000 28 / 21, 2000 46 / 39, 2 x 1000 28 / 23, 4 x 300 12.0 / 11.3); beyond, it only stages the keys more often
     // (4 x 1000 30 / 37, 8 x 300 13 / 16, 32 x 100 11 / 15).
-    const int kw = !narrow && groups_in(kRowsPerWg / 2) * num_q_heads <= 2 * (int64_t)mdx::compute_units() ? 2 : 1, rows_per_wg = kRowsPerWg / kw;
+    // Against the kernel for pairs of heads (below), which such prompts of more than 560 tokens take otherwise, it pays a third further,
+    // while the workgroups that wait for a place are light ones: 2 x 1000 29.1 / 26.0, 2 x 1100 31.5 / 29.3, 1 x 2300 51.7 / 45.3, 1 x
+    // 2600 58.2 / 51.9, 3 x 700 23.6 / 20.9, 400 to 1200 30.6 / 26.8; past that 2 x 1500 39 / 41, 3 x 1000 30.7 / 32.4, 1 x 3500 76 / 86.
+    const bool long_pairs = max_l > 560 && (num_q_heads / num_kv_heads) % 2 == 0;
+    const int64_t split_room = (int64_t)mdx::compute_units() * (long_pairs ? 27 : 20) / 10;
+    const int kw = !narrow && groups_in(kRowsPerWg / 2) * num_q_heads <= split_room ? 2 : 1, rows_per_wg = kRowsPerWg / kw;
     StaircaseParams P;
     P.q = (const __bf16*)q; P.k = (const __bf16*)k; P.v = (const __bf16*)v; P.o = (__bf16*)o;
     P.q_st = q_stride_t; P.q_sh = q_stride_h; P.k_st = k_stride_t; P.k_sh = k_stride_h;

@@ -60,6 +60,12 @@ def test_prefill_row_tiles_of_one_and_two_wavefronts(dev, lens, bound, S):
     _check_prefill(dev, lens, S, seed=sum(lens) + S, max_seqlen=bound)
 
 
+@pytest.mark.parametrize("lens", [[1100, 1100], [2663], [300, 1000, 650], [561, 1, 1403], [1300, 1331]])
+def test_prefill_around_the_room_for_two_wavefronts(dev, lens):
+    """Long prompts whose workgroups of two wavefronts per row tile are a third more than the chip holds at once, and just beyond."""
+    _check_prefill(dev, lens, 32, seed=sum(lens))
+
+
 @pytest.mark.parametrize("hq,hkv", [(16, 8), (8, 8), (4, 1), (3, 1), (2, 2)])
 def test_prefill_gqa_ratios(dev, hq, hkv):
     _check_prefill(dev, [150, 97], 32, hq=hq, hkv=hkv, seed=hq * 10 + hkv)
