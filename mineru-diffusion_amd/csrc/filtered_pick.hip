@@ -157,25 +157,31 @@ __device__ __forceinline__ void pick_from_kept(uint32_t (&key)[N], const int (&c
     for (int off = 32; off >= 1; off >>= 1) mk = max(mk, (uint32_t)__shfl_xor((int)mk, off));
     if (mk == 0) { x0 = 0; x0_p = 0.f; return; }                            // no finite logit
     const float m = value_of_key<T>(mk);
-    float term[N];
-    float Z = 0.f;
+    // The kept elements come in no order, so their masses are summed in fixed point: the same logits give the same cut-off and
+    // the same confidence, whichever wavefront listed its candidates first.  (384 rows, top-k 50, top-p 0.9: 35.0 -> 35.3 us.)
+    const bool fixed = has_masses(m, c);
+    Mass mass[N], total = 0;
+    float plain = 0.f;                                                       // (no fixed point for what is not at most 1: all but always NaN)
 #pragma unroll
     for (int i = 0; i < N; ++i) {
-        term[i] = key[i] ? __builtin_amdgcn_exp2f((value_of_key<T>(key[i]) - m) * c) : 0.f;
-        Z += term[i];
+        const float term = key[i] ? __builtin_amdgcn_exp2f((value_of_key<T>(key[i]) - m) * c) : 0.f;
+        mass[i] = mass_of(term);
+        total += mass[i];
+        plain += term;
     }
-    Z = wave_total(Z);
-    if (top_p < 1.0f && m > -INFINITY && m < INFINITY) {
-        const float target = top_p * Z;
+    total = wave_total(total);
+    if (top_p < 1.0f && fixed) {
+        const Mass target = share_of(total, top_p);
         uint32_t floor_key = 0;
         if (N == 1) {
             // the mass at and above this lane's key, lane by lane: shorter than sixteen sums over the wavefront, one behind the other
-            float above = 0.f;
+            Mass above = 0;
 #pragma unroll
             for (int j = 0; j < 64; ++j) {
                 const uint32_t other = (uint32_t)__builtin_amdgcn_readlane((int)key[0], j);
-                const float its = __uint_as_float((uint32_t)__builtin_amdgcn_readlane(__float_as_int(term[0]), j));
-                above += other >= key[0] ? its : 0.f;
+                const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)mass[0], j);
+                const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(mass[0] >> 32), j);
+                above += other >= key[0] ? ((Mass)hi << 32) | lo : 0ull;
             }
             floor_key = above > target ? key[0] : 0;
 #pragma unroll
@@ -184,19 +190,20 @@ __device__ __forceinline__ void pick_from_kept(uint32_t (&key)[N], const int (&c
         for (int bit = 15; N > 1 && bit >= 0; --bit) {
             const uint32_t trial = floor_key | (1u << bit);
             if (trial > mk) continue;
-            float a = 0.f;
+            Mass a = 0;
 #pragma unroll
-            for (int i = 0; i < N; ++i) a += key[i] >= trial ? term[i] : 0.f;
+            for (int i = 0; i < N; ++i) a += key[i] >= trial ? mass[i] : 0ull;
             if (wave_total(a) > target) floor_key = trial;
         }
-        Z = 0.f;
+        total = 0;
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-            if (key[i] < floor_key) { key[i] = 0; term[i] = 0.f; }
-            Z += term[i];
+            if (key[i] < floor_key) { key[i] = 0; mass[i] = 0; }
+            total += mass[i];
         }
-        Z = wave_total(Z);
+        total = wave_total(total);
     }
+    const float Z = fixed ? (float)total * (1.0f / kMassScale) : wave_total(plain);
     Pick best{-INFINITY, 0.f, 0x7fffffff};
 #pragma unroll
     for (int i = 0; i < N; ++i) {

@@ -62,6 +62,17 @@ __device__ __forceinline__ void scan_row(const RowView& r, int tid, F f) {
     for (int e = r.tail0 + tid; e < r.vocab; e += THREADS) f((uint32_t)r.p[e], e);
 }
 
+// Softmax terms relative to the row's maximum, at most 1 each, are summed as 64-bit integers in units of 2^-40: the sum does not
+// depend on the order of the additions (candidate lists have none), is exact for rows of up to 2^23 elements, and a row of 2^18
+// loses at most 2^-23 of its largest term to the rounding of its smallest.  NaN weighs nothing.
+constexpr float kMassScale = 1099511627776.f;        // 2^40
+typedef unsigned long long Mass;
+__device__ __forceinline__ Mass mass_of(float term) { return term > 0.f ? (Mass)__builtin_rintf(term * kMassScale) : 0ull; }
+// What a cumulative mass has to exceed for a share of the whole.
+__device__ __forceinline__ Mass share_of(Mass total, float share) { return (Mass)((double)share * (double)total); }
+// The terms are at most 1: neither an unbounded maximum nor a temperature that is zero, negative or not a number.
+__device__ __forceinline__ bool has_masses(float m, float c) { return m > -INFINITY && m < INFINITY && c >= 0.f && c < INFINITY; }
+
 template <typename V> __device__ __forceinline__ V wave_total(V v) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off);

@@ -218,3 +218,27 @@ def test_filtered_step_at_the_edges_of_a_lane_and_a_register(dev, V, k, p):
     assert torch.equal(got[0], want[0])
     np.testing.assert_allclose(got[1].cpu().numpy(), want[1].cpu().numpy(), rtol=5e-6)    # as above: fp32 sums in another order
     assert torch.equal(a, b) and torch.equal(got[3], want[3])
+
+
+@pytest.mark.parametrize("k", [3, 50, 400])
+def test_filtered_step_does_not_depend_on_the_order_of_its_candidates(dev, k):
+    """The candidates of a row are listed in whatever order its wavefronts come: rows that hold the same logits at other columns
+    get the same confidence, and a seeded step repeats, both bit for bit."""
+    import mdx
+    g = torch.Generator(device=dev).manual_seed(k)
+    V = 151936
+    base = (torch.randn(V, generator=g, device=dev) * 3).bfloat16()
+    base[:8] = torch.arange(8, device=dev).bfloat16() / 8 + base.max()                    # one row maximum, whatever the order
+    rows = torch.stack([base[torch.randperm(V, generator=g, device=dev)] for _ in range(96)]).view(3, 32, V)
+    masks = torch.full((3, 32), 9, dtype=torch.int64, device=dev)
+    for p in (1.0, 0.9):
+        conf = mdx.unmask_step(rows, masks.clone(), 9, 0.9, 2, top_k=k, top_p=p)[1]
+        assert len(set(conf.flatten().view(torch.int32).tolist())) == 1
+    temps = torch.tensor([0.7, 1.0, 1.3], device=dev)
+    first = None
+    for _ in range(10):
+        tokens = masks.clone()
+        got = [*mdx.unmask_step(rows, tokens, 9, 0.02, 2, temperatures=temps, top_k=k, top_p=0.9, seed=11, offset=4), tokens]
+        got[1] = got[1].view(torch.int32)
+        first = first or got
+        assert all(torch.equal(a, b) for a, b in zip(got, first))
