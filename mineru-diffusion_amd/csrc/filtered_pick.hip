@@ -322,9 +322,10 @@ __global__ __launch_bounds__(kPickThreads) void filtered_pick_kernel(
     // ---- too many ties for a list: the row itself, pass by pass ----
     __shared__ float fslot[kPickThreads / 64];
     __shared__ int islot[kPickThreads / 64];
+    __shared__ Mass mslot[kPickThreads / 64];
     __shared__ Pick bests[kPickThreads / 64];
     const RowView row = row_view(logits + r * row_stride, vocab);
-    const uint32_t floor_key = floor_by_bisection<T, kPickThreads>(row, tid, top_k, top_p, c, fslot, islot);
+    const uint32_t floor_key = floor_by_bisection<T, kPickThreads>(row, tid, top_k, top_p, c, mslot, islot);
     Pick best{-INFINITY, 0.f, 0x7fffffff};
     float m = -INFINITY, Z = 0.f;
     auto kept = [&](uint32_t b) { return b != Bits16<T>::kNegInf && key_of(b) >= floor_key; };

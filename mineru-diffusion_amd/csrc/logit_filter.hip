@@ -16,7 +16,7 @@
 // 344 us, top-p alone 314.)
 //
 // Where the reference's sort leaves the order of equal values open, all elements equal to the crossing
-// value are kept.  The masses are fp32 sums in an order that the row's contents fix; against a computation in higher
+// value are kept.  The masses are 64-bit fixed-point sums of fp32 softmax terms; against a computation in higher
 // precision, a target that falls within fp32 rounding of a cumulative probability can resolve either way.
 #include "logit_keys.h"
 #include "filtered_pick.h"
@@ -33,9 +33,8 @@ constexpr int kWordsPerThread = kWords / kFilterThreads;
 constexpr int kHistBytes = kWords * 4;
 
 struct Scratch {
-    float fslot[kWaves];
+    Mass mslot[kWaves];
     int islot[kWaves];
-    int first;               // the first thread (from the largest keys) whose keys cross a target
     uint32_t floor_key;
 };
 
@@ -83,7 +82,7 @@ __device__ uint32_t floor_from_counts(const RowView& row, uint32_t* hist, Scratc
     int total;
     const int upto = block_prefix(cnt, sh.islot, tid, &total);
     // a counter that ran over has lost 65536, or carried 1 into its neighbour for them: the total shows it
-    if (total + n_inf != row.vocab) return floor_by_bisection<T, kFilterThreads>(row, tid, top_k, top_p, c, sh.fslot, sh.islot);
+    if (total + n_inf != row.vocab) return floor_by_bisection<T, kFilterThreads>(row, tid, top_k, top_p, c, sh.mslot, sh.islot);
 
     uint32_t floor_key = 0;
     if (with_k && total >= top_k) {
@@ -107,42 +106,37 @@ __device__ uint32_t floor_from_counts(const RowView& row, uint32_t* hist, Scratc
     for (int off = 32; off >= 1; off >>= 1) top = max(top, __shfl_xor(top, off));
     __syncthreads();
     if (lane == 0) sh.islot[tid >> 6] = top;
-    if (tid == 0) sh.first = kFilterThreads;
     __syncthreads();
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) top = max(top, sh.islot[w]);
     // a row whose largest element is not finite has no softmax to take a share of: left as it is
     if (top < 0) return floor_key;
     const float m = value_of_key<T>((uint32_t)top);
-    if (!(m > -INFINITY && m < INFINITY)) return floor_key;
+    if (!has_masses(m, c)) return floor_key;
 
-    auto mass_of = [&](uint32_t key, uint32_t n) {
-        return n && key >= floor_key ? (float)n * __builtin_amdgcn_exp2f((value_of_key<T>(key) - m) * c) : 0.f;
+    auto mass_at = [&](uint32_t key, uint32_t n) {
+        return n && key >= floor_key ? n * mass_of(__builtin_amdgcn_exp2f((value_of_key<T>(key) - m) * c)) : 0ull;
     };
-    float mass = 0.f;
+    Mass mass = 0;
     if (2 * (base + kWordsPerThread) > (int)floor_key && 2 * base <= top)
         for (int j = 0; j < kWordsPerThread; ++j) {
             const int at = base + ((j + lane) & (kWordsPerThread - 1));
             const uint32_t w = hist[at];
-            if (w) mass += mass_of(2 * at, w & 0xffffu) + mass_of(2 * at + 1, w >> 16);
+            if (w) mass += mass_at(2 * at, w & 0xffffu) + mass_at(2 * at + 1, w >> 16);
         }
-    float Z;
-    const float mass_upto = block_prefix(mass, sh.fslot, tid, &Z), target = top_p * Z;
-    if (mass > 0.f && mass_upto > target) atomicMin(&sh.first, tid);
-    __syncthreads();
-    if (sh.first == kFilterThreads) return floor_key;                // (the share rounded onto the whole)
-    if (tid == sh.first) {
-        float a = mass_upto - mass;
+    Mass total_mass;
+    const Mass mass_upto = block_prefix(mass, sh.mslot, tid, &total_mass), target = share_of(total_mass, top_p);
+    if (mass_upto > target && mass_upto - mass <= target) {          // exactly one thread (the share is less than the whole)
+        Mass a = mass_upto - mass;
         uint32_t key = 0;
-        for (int at = base + kWordsPerThread - 1; at >= base; --at) {
+        for (int at = base + kWordsPerThread - 1; at >= base && !key; --at) {
             const uint32_t w = hist[at];
-            const float hi = mass_of(2 * at + 1, w >> 16), lo = mass_of(2 * at, w & 0xffffu);
-            a += hi;
-            if (hi > 0.f) { key = 2 * at + 1; if (a > target) break; }
-            a += lo;
-            if (lo > 0.f) { key = 2 * at; if (a > target) break; }
+            a += mass_at(2 * at + 1, w >> 16);
+            if (a > target) { key = 2 * at + 1; break; }
+            a += mass_at(2 * at, w & 0xffffu);
+            if (a > target) key = 2 * at;
         }
-        sh.floor_key = max(floor_key, key);                          // (none crosses, by the rounding of the prefix: its lowest)
+        sh.floor_key = key;
     }
     __syncthreads();
     return sh.floor_key;

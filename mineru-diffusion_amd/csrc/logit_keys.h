@@ -96,7 +96,7 @@ template <int THREADS, typename V> __device__ __forceinline__ V block_total(V v,
 // elements at or above a trial key: the k-th largest key is the largest that k elements reach, the top-p cut-off the largest
 // whose elements weigh more than the share asked for.  0 = everything is kept.
 template <typename T, int THREADS>
-__device__ uint32_t floor_by_bisection(const RowView& row, int tid, int top_k, float top_p, float c, float* fslot, int* islot) {
+__device__ uint32_t floor_by_bisection(const RowView& row, int tid, int top_k, float top_p, float c, Mass* mslot, int* islot) {
     uint32_t floor_key = 0, mk = 0;
     if (top_k > 0 && top_k < row.vocab) {
         for (int bit = 15; bit >= 0; --bit) {
@@ -115,13 +115,13 @@ __device__ uint32_t floor_by_bisection(const RowView& row, int tid, int top_k, f
         __syncthreads();
         for (int w = 0; w < THREADS / 64; ++w) mk = max(mk, (uint32_t)islot[w]);
         const float m = value_of_key<T>(mk);
-        if (m > -INFINITY && m < INFINITY) {                    // a row whose largest element is not finite has no softmax to take a share of
+        if (has_masses(m, c)) {                                 // a row whose largest element is not finite has no softmax to take a share of
             auto mass_from = [&](uint32_t from) {
-                float a = 0.f;
-                scan_row<THREADS>(row, tid, [&](uint32_t b, int) { if (key_of(b) >= from) a += __builtin_amdgcn_exp2f((Bits16<T>::value(b) - m) * c); });
-                return block_total<THREADS>(a, fslot, tid);
+                Mass a = 0;
+                scan_row<THREADS>(row, tid, [&](uint32_t b, int) { if (key_of(b) >= from) a += mass_of(__builtin_amdgcn_exp2f((Bits16<T>::value(b) - m) * c)); });
+                return block_total<THREADS>(a, mslot, tid);
             };
-            const float target = top_p * mass_from(floor_key);
+            const Mass target = share_of(mass_from(floor_key), top_p);
             uint32_t key = 0;
             for (int bit = 15; bit >= 0; --bit) {
                 const uint32_t trial = key | (1u << bit);

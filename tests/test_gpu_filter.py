@@ -242,3 +242,35 @@ def test_filtered_step_does_not_depend_on_the_order_of_its_candidates(dev, k):
         got[1] = got[1].view(torch.int32)
         first = first or got
         assert all(torch.equal(a, b) for a, b in zip(got, first))
+
+
+@pytest.mark.parametrize("form", ["counters", "bisection", "lists", "lists_run_over"])
+@pytest.mark.parametrize("call", ["filter", "step"])
+def test_filter_top_p_cut_off_is_exact_where_the_masses_are(dev, form, call):
+    """Logits 0, -1, -2, .. at the temperature 1 / ln 2 weigh 2^0, 2^-1, 2^-2, ..: cumulative masses that 64-bit sums hold exactly,
+    so the cut-off is right for every p, the fp32 values next to the cumulative shares included."""
+    import mdx
+    from fractions import Fraction
+    rng = np.random.default_rng(3)
+    n, k = [int(c) << (i // 2) for i, c in enumerate(rng.integers(300, 900, 14))], 0
+    if form == "bisection":
+        n[7], n[9] = 66000, 70001                                        # more than a 16-bit counter holds
+    if form.startswith("lists"):
+        n, k = [3, 5, 20, 60, 200, 150 if form == "lists" else 66000], 400     # more ties at the k-th largest than a list holds
+    values = rng.permutation(np.repeat(-np.arange(len(n)), n))
+    logits = torch.from_numpy(values).to(torch.bfloat16).to(dev).view(1, 1, -1)
+    if form == "lists":
+        logits = torch.nn.functional.pad(logits, (0, 5000), value=-300.0)
+    temps = torch.tensor([1.4426950408889634], device=dev)
+    upto = list(np.cumsum([Fraction(c, 2 ** i) for i, c in enumerate(n)]))
+    masks = torch.full((1, 1), 9, dtype=torch.int64, device=dev)
+    for i in range(len(n) - 1):
+        near = np.float32(float(upto[i] / upto[-1]))
+        for p in (np.nextafter(near, np.float32(0)), near, np.nextafter(near, np.float32(1))):
+            last = next(j for j in range(len(n)) if upto[j] > Fraction(float(p)) * upto[-1])
+            if call == "filter":
+                kept = torch.isfinite(mdx.filter_logits(logits, top_k=k, top_p=float(p), temperatures=temps)).sum().item()
+                assert kept == sum(n[: last + 1]), (i, p)
+            else:
+                conf = mdx.unmask_step(logits, masks.clone(), 9, 0.9, 1, temperatures=temps, top_k=k, top_p=float(p))[1].item()
+                assert abs(conf * float(upto[last]) - 1) < 1e-5, (i, p)       # (every level is 5e-4 of the sum or more)
