@@ -211,6 +211,7 @@ __device__ __forceinline__ void pick_from_kept(uint32_t (&key)[N], const int (&c
         if (key[i]) { const float x = value_of_key<T>(key[i]); better(best, drawn(x, column[i]), x, column[i]); }
     }
     best = wave_best(best);
+    if (best.column == 0x7fffffff || !(best.x > kNoConfidence)) { x0 = 0; x0_p = 0.f; return; }      // nothing but NaN, or the type's lowest values
     x0 = best.column;
     x0_p = NOISE == 0 ? fminf(1.0f / Z, 1.0f) : __builtin_amdgcn_exp2f((best.x - m) * c) / Z;
 }
@@ -348,7 +349,7 @@ __global__ __launch_bounds__(kPickThreads) void filtered_pick_kernel(
     __syncthreads();
     if (tid != 0) return;
     for (int w = 1; w < kPickThreads / 64; ++w) better(best, bests[w].v, bests[w].x, bests[w].column);
-    const bool any = best.column != 0x7fffffff;
+    const bool any = best.column != 0x7fffffff && best.x > kNoConfidence;
     x0[r] = any ? best.column : 0;
     x0_p[r] = !any ? 0.f : NOISE == 0 ? fminf(1.0f / Z, 1.0f) : __builtin_amdgcn_exp2f((best.x - m) * c) / Z;
 }

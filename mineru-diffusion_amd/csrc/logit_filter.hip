@@ -61,7 +61,8 @@ __device__ uint32_t floor_from_counts(const RowView& row, uint32_t* hist, Scratc
     for (int i = tid; i < kWords / 4; i += kFilterThreads) reinterpret_cast<u32x4*>(hist)[i] = u32x4{0, 0, 0, 0};
     if (tid == 0) sh.floor_key = 0;
     __syncthreads();
-    // -inf is never kept on account of a filter and often fills most of a row: counted in a register
+    // -inf, which often fills most of a row, is counted in a register
+    constexpr uint32_t kInfKey = Bits16<T>::kNegInf ^ 0xffffu;       // (odd: the high half of its word)
     int n_inf = 0;
     scan_row<kFilterThreads>(row, tid, [&](uint32_t b, int) {
         if (b == Bits16<T>::kNegInf) { ++n_inf; return; }
@@ -79,18 +80,19 @@ __device__ uint32_t floor_from_counts(const RowView& row, uint32_t* hist, Scratc
         cnt += (int)((w & 0xffffu) + (w >> 16));
         if (w) top = max(top, 2 * at + (w >> 16 ? 1 : 0));
     }
+    if (base <= (int)(kInfKey >> 1) && (int)(kInfKey >> 1) < base + kWordsPerThread) cnt += n_inf;
     int total;
     const int upto = block_prefix(cnt, sh.islot, tid, &total);
     // a counter that ran over has lost 65536, or carried 1 into its neighbour for them: the total shows it
-    if (total + n_inf != row.vocab) return floor_by_bisection<T, kFilterThreads>(row, tid, top_k, top_p, c, sh.mslot, sh.islot);
+    if (total != row.vocab) return floor_by_bisection<T, kFilterThreads>(row, tid, top_k, top_p, c, sh.mslot, sh.islot);
 
     uint32_t floor_key = 0;
-    if (with_k && total >= top_k) {
+    if (with_k) {
         if (upto >= top_k && upto - cnt < top_k) {                   // exactly one thread: the k-th largest is among its keys
             int n = upto - cnt;
             uint32_t key = 0;
             for (int at = base + kWordsPerThread - 1; at >= base && !key; --at) {
-                n += (int)(hist[at] >> 16);
+                n += (int)(hist[at] >> 16) + (at == (int)(kInfKey >> 1) ? n_inf : 0);
                 if (n >= top_k) { key = 2 * at + 1; break; }
                 n += (int)(hist[at] & 0xffffu);
                 if (n >= top_k) key = 2 * at;
@@ -157,7 +159,8 @@ __global__ __launch_bounds__(kFilterThreads) void logit_filter_kernel(
     const float c = kLog2e / (temperatures ? temperatures[r / rows_per_temp] : 1.0f);
     const uint32_t floor_key = floor_from_counts<T>(row, hist, sh, tid, top_k, top_p, c);
     if (!WRITE) {
-        if (tid == 0) floors[r] = floor_key ? value_of_key<T>(floor_key) : -INFINITY;
+        // (a cut-off below -inf is a NaN's; one above +inf drops every number, as it should)
+        if (tid == 0) floors[r] = floor_key > (Bits16<T>::kNegInf ^ 0xffffu) ? value_of_key<T>(floor_key) : -INFINITY;
         return;
     }
     uint16_t* op = out + r * out_row_stride;

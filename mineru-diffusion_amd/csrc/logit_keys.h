@@ -25,6 +25,9 @@ __device__ __forceinline__ uint32_t key_of(uint32_t b) {
 __device__ __forceinline__ uint32_t bits_of(uint32_t k) { return (k & 0x8000u) ? (k & 0x7fffu) : (~k & 0xffffu); }
 template <typename T> __device__ __forceinline__ float value_of_key(uint32_t k) { return Bits16<T>::value(bits_of(k)); }
 
+// The vocabulary pass takes no element at or below this for a row's largest: a row that holds no other has no confidence.
+constexpr float kNoConfidence = -3.0e38f;
+
 struct RowView {                        // a row as scalar head, aligned 16-byte chunks, scalar tail
     const uint16_t* p;
     const u32x4* chunks;

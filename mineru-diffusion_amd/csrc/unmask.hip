@@ -15,6 +15,7 @@
 #include "mdx_common.h"
 #include "gumbel_noise.h"
 #include "filtered_pick.h"
+#include "logit_keys.h"
 #include <hip/hip_fp16.h>
 
 namespace {
@@ -24,7 +25,7 @@ using namespace mdx_noise;
 constexpr int kThreads = 256;
 constexpr int kUnroll = 2;               // 16-byte loads in flight per lane
 constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kNegBig = -3.0e38f;      // finite stand-in for -inf: keeps (m - m) away from inf - inf
+constexpr float kNegBig = mdx_keys::kNoConfidence;   // finite stand-in for -inf: keeps (m - m) away from inf - inf
 constexpr int kNoIndex = 0x7fffffff;
 
 struct Partial {                         // one row's (or row split's) running state

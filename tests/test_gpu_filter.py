@@ -274,3 +274,58 @@ def test_filter_top_p_cut_off_is_exact_where_the_masses_are(dev, form, call):
             else:
                 conf = mdx.unmask_step(logits, masks.clone(), 9, 0.9, 1, temperatures=temps, top_k=k, top_p=float(p))[1].item()
                 assert abs(conf * float(upto[last]) - 1) < 1e-5, (i, p)       # (every level is 5e-4 of the sum or more)
+
+
+def _kept_by_order(bits, dtype, k):
+    """What a top-k keeps of rows of 16-bit patterns, from the patterns alone: the k-th in order and everything at or above it."""
+    bits = np.where(bits == 0x8000, 0, bits)                                            # (-0 counts as 0)
+    key = np.where(bits & 0x8000, ~bits & 0xffff, bits | 0x8000)
+    return key >= np.sort(key, axis=1)[:, -k][:, None]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("V", [37, 1003, 40000])
+@pytest.mark.parametrize("k,p", [(1, 1.0), (4, 0.9), (30, 0.8), (30, 1.0), (700, 0.9), (700, 1.0), (0, 0.9)])
+@pytest.mark.parametrize("noise", ["none", "seed"])
+def test_filtered_step_on_rows_that_are_not_finite(dev, dtype, V, k, p, noise):
+    """NaN of both signs (ordered above +inf and below -inf), infinities and the type's lowest values, few of them and nothing else:
+    the filter keeps what its order says, and the step without the filtered copy does what the step on that copy does."""
+    import mdx
+    g = torch.Generator(device=dev).manual_seed(V + k)
+    inf, nan, low = float("inf"), float("nan"), torch.finfo(dtype).min
+    rows = 24
+    x = (torch.randn(rows, V, generator=g, device=dev) * 3).to(dtype)
+    fills = [(nan, 1), (nan, 5), (nan, V - 3), (nan, V), ("-nan", 1), ("-nan", V - 3), ("-nan", V), (inf, 1), (inf, 6), (inf, V), (-inf, V - 2), (-inf, V - 9),
+             (-inf, V), (low, V - 2), (low, V)]
+    for r, (value, count) in enumerate(fills):
+        at = torch.randperm(V, generator=g, device=dev)[:count]
+        if value == "-nan":
+            x.view(torch.int16)[r, at] = -1 - 0x3f                                       # sign bit, all exponent bits, a fraction
+        else:
+            x[r, at] = value
+    x[15, : V // 2], x[15, V // 2 :] = nan, -inf
+    x.view(torch.int16)[16, : V // 2] = -0x40
+    x[16, V // 2 :] = -inf
+    x[17, :3], x[17, 3:6] = nan, inf
+    x[18, 0], x[18, 1] = inf, -inf
+    x.view(torch.int16)[19, ::2] = -0x40
+    x[19, 1::2] = nan
+    x[20, :], x[20, 2] = low, nan
+    x[21, V - 1], x.view(torch.int16)[22, V - 1] = nan, -0x40
+    bits = x.view(torch.int16).cpu().numpy().astype(np.int64) & 0xffff
+    filtered = mdx.filter_logits(x, k, p)
+    if 0 < k < V and p == 1.0:
+        got = filtered.view(torch.int16).cpu().numpy().astype(np.int64) & 0xffff
+        minus_inf = int(torch.tensor([-inf], dtype=dtype).view(torch.int16)) & 0xffff
+        assert np.array_equal(got, np.where(_kept_by_order(bits, dtype, k), bits, minus_inf))
+    opts = dict(seed=5, offset=2) if noise == "seed" else {}
+    tokens = torch.full((rows, 1), 9, dtype=torch.int64, device=dev)
+    want_tokens = tokens.clone()
+    got = mdx.unmask_step(x[:, None], tokens, 9, 0.9, 0, top_k=k, top_p=p, **opts)
+    want = mdx.unmask_step(filtered[:, None], want_tokens, 9, 0.9, 0, **opts)
+    assert torch.equal(got[0], want[0])
+    # where the filter keeps a NaN the step's confidence depends on the columns (a lane whose maximum rises after it forgets it)
+    ok = ~torch.isnan(filtered.float()).any(1)
+    assert ok.sum() >= 8
+    np.testing.assert_allclose(got[1][ok].cpu().numpy(), want[1][ok].cpu().numpy(), rtol=5e-6)   # (equal NaN; fp32 sums in another order)
+    assert torch.equal(got[2][ok], want[2][ok]) and torch.equal(got[3][ok], want[3][ok]) and torch.equal(tokens[ok], want_tokens[ok])
