@@ -142,6 +142,7 @@ Tensor token_rows(const Tensor& t) {
 Tensor check_store(const Tensor& key, const Tensor& value, const Tensor& k_cache, const Tensor& v_cache, const Tensor& slot_mapping) {
     NEED(key.dim() == 3 && value.dim() == 3);
     const int64_t N = key.size(0), heads = key.size(1), d = key.size(2), D = heads * d;
+    NEED(D > 0);
     NEED(key.stride(2) == 1 && value.stride(2) == 1);
     NEED(key.stride(1) == d && value.stride(1) == d);
     NEED(k_cache.dim() > 1 && v_cache.dim() > 1 && k_cache.stride(1) == D && v_cache.stride(1) == D);
@@ -199,6 +200,7 @@ PyObject* qk_norm_rope_store(PyObject*, PyObject* const* a, Py_ssize_t n) {
             NEED(v_cache.defined() && k_cache.is_contiguous() && v_cache.is_contiguous());
             NEED(slot_mapping.defined() && slot_mapping.numel() == x.n);
             slots = int32_list(slot_mapping, "slot_mapping");
+            NEED(hkv > 0 && d > 0);
             num_slots = k_cache.numel() / (hkv * d);
         }
         check(mdx_qk_norm_rope_store(ptr(x.t), x.stride, ptr(qw), ptr(kw), (float)real(a[3]), static_cast<const float*>(ptr(cos)),
@@ -333,7 +335,9 @@ PyObject* qk_norm_rope_store_partials(PyObject*, PyObject* const* a, Py_ssize_t 
         const int64_t hq = integer(a[7]), hkv = integer(a[8]), d = integer(a[9]);
         need_gpu({&p, &qw, &kw, &cos, &sin, &positions, &k_cache, &v_cache, &slot_mapping});
         need_partials(p);
-        const int64_t width = (hq + 2 * hkv) * d, rows = p.numel() / p.size(0) / width;
+        const int64_t width = (hq + 2 * hkv) * d;
+        NEED(p.size(0) > 0 && hq >= 0 && hkv > 0 && d > 0);
+        const int64_t rows = p.numel() / p.size(0) / width;
         NEED(p.size(-1) == width && positions.numel() == rows && positions.scalar_type() == at::kLong && cos.scalar_type() == at::kFloat && sin.scalar_type() == at::kFloat);
         NEED(k_cache.is_contiguous() && v_cache.is_contiguous() && k_cache.scalar_type() == qw.scalar_type() && slot_mapping.numel() == rows);
         const Tensor pos = positions.is_contiguous() ? positions : positions.contiguous(), slots = int32_list(slot_mapping, "slot_mapping");

@@ -775,7 +775,7 @@ extern "C" int mdx_staircase_attn_store(const void* q, const void* k, const void
     MDX_REQUIRE(k_stride_h == head_dim && v_stride_h == head_dim, MDX_EUNSUPPORTED, "staircase_attn_store: rows of k and v must be dense");
     const int row16 = (int)(row_bytes / 16);
     const bool along = total_tokens > 0 && total_tokens < ((int64_t)1 << 30) && k && v && k_cache && v_cache && slot_mapping && num_slots >= 0 &&
-                       row_bytes % 16 == 0 && row_bytes <= 16 * (kThreads / 2) && kThreads / 2 % row16 == 0 &&
+                       row16 > 0 && row_bytes % 16 == 0 && row_bytes <= 16 * (kThreads / 2) && kThreads / 2 % row16 == 0 &&
                        (k_stride_t * elem) % 16 == 0 && (v_stride_t * elem) % 16 == 0 && k_stride_t >= 0 && v_stride_t >= 0 &&
                        mdx::aligned16(k) && mdx::aligned16(v) && mdx::aligned16(k_cache) && mdx::aligned16(v_cache);
     StoreParams S{};

@@ -66,6 +66,9 @@ def test_bad_arguments_are_refused_without_a_launch(L):
     assert sa(hq=12) == -1
     assert sa(dtype=3) == -2 and b"dtype" in L.mdx_last_error()     # bf16, fp16 and fp32 are the element types
     assert sa(scale=-1.0) == -1
+    st = lambda hkv, d: L.mdx_staircase_attn_store(                                              # noqa: E731
+        one, one, one, one, 2048, 128, 1024, d, 1024, d, 2048, 128, one, one, 1, 100, 100, 16, hkv, d, 32, 0.1, 0, one, one, one, 10, null)
+    assert st(0, 128) == -1 and st(8, 0) == -2                      # no KV heads, no columns: an error, not a division
     pa = lambda **kw: L.mdx_paged_block_attn(                                                  # noqa: E731
         one, one, one, one, 65536, 2048, 128, 65536, 2048, 128, 262144, 1024, 128, one, 17, one,
         4, kw.get("sq", 32), 16, 8, kw.get("d", 128), 17, kw.get("page", 256), 100, 0.1, 0, kw.get("ws", null), kw.get("ws_bytes", 0), null)

@@ -307,3 +307,22 @@ def test_pair_prefill_stores_every_row(dev, lens, hkv, ratio, dtype, before, beh
     if longest == max(lens):
         want = mdx.sparse_attn_varlen(q, k, v, cu, cu, S, max_seqlen=longest, softmax_scale=d ** -0.5)
         assert torch.equal(o[before:N - behind], want.flatten(1)[before:N - behind])
+
+
+def test_host_functions_refuse_sizes_of_zero(dev):
+    """No KV heads, empty heads or no partial sums: an exception, as the Python divisions raised, and never the end of the process."""
+    import mdx
+    from mdx import ops
+    i64, f32, bf16 = torch.int64, torch.float32, torch.bfloat16
+    new = lambda *s, dtype=bf16: torch.zeros(*s, dtype=dtype, device=dev)                       # noqa: E731
+    cs, pos, slots, cache = new(16, 64, dtype=f32), new(4, dtype=i64), new(4, dtype=torch.int32), new(1, 256, 2, 128)
+    for hq, hkv, d in ((2, 0, 128), (2, 1, 0)):
+        with pytest.raises((AssertionError, RuntimeError)):
+            ops.qk_norm_rope_store(new(4, (hq + 2 * hkv) * d), new(128), new(128), 1e-6, cs, cs, pos, hq, hkv, d, cache, cache, slots)
+    for splits, hq, hkv, d in ((0, 2, 1, 128), (2, 2, 0, 128), (2, 0, 0, 128), (2, 2, 1, 0)):
+        with pytest.raises(AssertionError):
+            ops.qk_norm_rope_store_partials(new(splits, 4, (hq + 2 * hkv) * d, dtype=f32), new(128), new(128), 1e-6, cs, cs, pos, hq, hkv, d,
+                                            cache, cache, slots)
+    rows = new(4, 0, 128).as_strided((4, 0, 128), (0, 128, 1))
+    with pytest.raises(AssertionError):
+        mdx.store_kvcache(rows, rows, new(1, 256, 0, 128).as_strided((1, 256, 0, 128), (0, 0, 128, 1)), new(1, 256, 0, 128), slots)
