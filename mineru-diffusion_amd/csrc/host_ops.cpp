@@ -132,7 +132,6 @@ template <typename F> PyObject* guarded(F f) {
 // ---- store_kvcache --------------------------------------------------------------------------------
 // [b, s, h, d] as rows [(b s), h, d] (a copy where the first two dimensions do not merge)
 Tensor token_rows(const Tensor& t) {
-    if (t.dim() != 4) return t;
     if (t.size(0) == 1 || t.stride(0) == t.size(1) * t.stride(1))
         return t.as_strided({t.size(0) * t.size(1), t.size(2), t.size(3)}, {t.stride(1), t.stride(2), t.stride(3)});
     return t.flatten(0, 1);
@@ -152,9 +151,8 @@ Tensor check_store(const Tensor& key, const Tensor& value, const Tensor& k_cache
     return int32_list(slot_mapping, "slot_mapping");
 }
 
-void store(const Tensor& key4, const Tensor& value4, const Tensor& k_cache, const Tensor& v_cache, const Tensor& slot_mapping, void* stream) {
-    need_gpu({&key4, &value4, &k_cache, &v_cache, &slot_mapping});
-    const Tensor key = token_rows(key4), value = token_rows(value4);
+void store(const Tensor& key, const Tensor& value, const Tensor& k_cache, const Tensor& v_cache, const Tensor& slot_mapping, void* stream) {
+    need_gpu({&key, &value, &k_cache, &v_cache, &slot_mapping});
     const Tensor slots = check_store(key, value, k_cache, v_cache, slot_mapping);
     const int64_t N = key.size(0), D = key.size(1) * key.size(2);
     check(mdx_store_kvcache(ptr(key), ptr(value), key.stride(0), value.stride(0), ptr(k_cache), ptr(v_cache),
@@ -162,11 +160,30 @@ void store(const Tensor& key4, const Tensor& value4, const Tensor& k_cache, cons
           "store_kvcache");
 }
 
+// k of four dimensions, and v with it, as rows
+void store_maybe4d(const Tensor& k, const Tensor& v, const Tensor& k_cache, const Tensor& v_cache, const Tensor& slot_mapping, void* stream) {
+    const bool four = k.dim() == 4;
+    NEED(!four || v.dim() == 4);
+    store(four ? token_rows(k) : k, four ? token_rows(v) : v, k_cache, v_cache, slot_mapping, stream);
+}
+
 PyObject* store_kvcache(PyObject*, PyObject* const* a, Py_ssize_t n) {
     ARGS(5);
     return guarded([&]() -> PyObject* {
         const Tensor& key = tensor(a[0]);
-        store(key, tensor(a[1]), tensor(a[2]), tensor(a[3]), tensor(a[4]), key.is_cuda() ? stream_of(key) : nullptr);
+        need_gpu({&key});
+        if (key.dim() != 3) throw PyRaise{PyExc_ValueError, "store_kvcache: key must be [N, heads, d]"};
+        store(key, tensor(a[1]), tensor(a[2]), tensor(a[3]), tensor(a[4]), stream_of(key));
+        Py_RETURN_NONE;
+    });
+}
+
+PyObject* store_kvcache_maybe4d(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    ARGS(5);
+    return guarded([&]() -> PyObject* {
+        const Tensor& key = tensor(a[0]);
+        need_gpu({&key});
+        store_maybe4d(key, tensor(a[1]), tensor(a[2]), tensor(a[3]), tensor(a[4]), stream_of(key));
         Py_RETURN_NONE;
     });
 }
@@ -492,7 +509,7 @@ PyObject* attention_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const Tensor &q = tensor(a[0]), &k_cache = tensor(a[3]), &v_cache = tensor(a[4]);
         if (k_cache.numel() > 0 && v_cache.numel() > 0) {
             need_gpu({&q});
-            store(tensor(a[1]), tensor(a[2]), k_cache, v_cache, tensor(a[5]), stream_of(q));
+            store_maybe4d(tensor(a[1]), tensor(a[2]), k_cache, v_cache, tensor(a[5]), stream_of(q));
         }
         return wrap(paged(q, k_cache, v_cache, tensor(a[6]), tensor(a[7]), a[8], Py_None, true));
     });
@@ -771,7 +788,7 @@ PyObject* sampler_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 #define ENTRY(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
-    ENTRY(store_kvcache), ENTRY(qk_norm_rope_store), ENTRY(rms_norm), ENTRY(silu_and_mul), ENTRY(linear_partials), ENTRY(linear_silu),
+    ENTRY(store_kvcache), ENTRY(store_kvcache_maybe4d), ENTRY(qk_norm_rope_store), ENTRY(rms_norm), ENTRY(silu_and_mul), ENTRY(linear_partials), ENTRY(linear_silu),
     ENTRY(rms_norm_partials), ENTRY(qk_norm_rope_store_partials), ENTRY(sparse_attn_varlen),
     ENTRY(flash_attn_with_kvcache), ENTRY(attention_prefill), ENTRY(attention_decode), ENTRY(confidence_argmax), ENTRY(lm_head_confidence),
     ENTRY(filter_logits), ENTRY(select_transfer), ENTRY(unmask_step), ENTRY(sampler_step),

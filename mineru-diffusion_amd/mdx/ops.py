@@ -34,7 +34,7 @@ def store_kvcache(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor,
 
 def store_kvcache_maybe4d(k, v, k_cache, v_cache, slot_mapping) -> None:
     """nanovllm/layers/sdar_attention.py:11-16: [b, s, h, d] inputs are flattened to [(b s), h, d]."""
-    _host().store_kvcache(k, v, k_cache, v_cache, slot_mapping)
+    _host().store_kvcache_maybe4d(k, v, k_cache, v_cache, slot_mapping)
 
 
 def qk_norm_rope_store(qkv: torch.Tensor, q_weight: torch.Tensor, k_weight: torch.Tensor, eps: float,

@@ -81,6 +81,20 @@ def test_store_4d_decode_form(dev):
     assert np.array_equal(_bits(dk), ek) and np.array_equal(_bits(dv), ev)
 
 
+def test_store_kvcache_takes_three_dimensions_only(dev):
+    """[b, s, h, d] is for store_kvcache_maybe4d, with k and v alike."""
+    import mdx
+    new = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=dev)                           # noqa: E731
+    cache, slots = new(1, 256, 8, 128), torch.arange(64, dtype=torch.int32, device=dev)
+    for shape in ((2, 32, 8, 128), (64, 1024)):
+        with pytest.raises(ValueError):
+            mdx.store_kvcache(new(*shape), new(*shape), cache, cache, slots)
+    with pytest.raises(AssertionError):
+        mdx.store_kvcache_maybe4d(new(2, 32, 8, 128), new(64, 8, 128), cache, cache, slots)
+    with pytest.raises(AssertionError):
+        mdx.store_kvcache_maybe4d(new(64, 8, 128), new(2, 32, 8, 128), cache, cache, slots)
+
+
 def test_store_out_of_range_slots_are_skipped(dev):
     import mdx
     N, hkv, d = 8, 8, 128
