@@ -58,10 +58,22 @@ int64_t integer(PyObject* o) {
     if (v == -1 && PyErr_Occurred()) throw PyPending{};
     return v;
 }
-uint64_t integer_mod64(PyObject* o) {
-    const unsigned long long v = PyLong_AsUnsignedLongLongMask(o);
-    if (v == (unsigned long long)-1 && PyErr_Occurred()) throw PyPending{};
+// int(o): what has a value as an integer, a float or a tensor of one element say, is taken for it (towards zero)
+template <typename F> auto as_int(PyObject* o, F value) {
+    PyObject* whole = PyNumber_Long(o);
+    if (!whole) throw PyPending{};
+    const auto v = value(whole);
+    Py_DECREF(whole);
+    if (PyErr_Occurred()) throw PyPending{};
     return v;
+}
+int64_t to_int(PyObject* o) { return as_int(o, PyLong_AsLongLong); }
+uint64_t to_int_mod64(PyObject* o) { return as_int(o, PyLong_AsUnsignedLongLongMask); }
+// None or nothing: `otherwise`
+int64_t to_int_or(PyObject* o, int64_t otherwise) {
+    const int given = PyObject_IsTrue(o);
+    if (given < 0) throw PyPending{};
+    return given ? to_int(o) : otherwise;
 }
 double real(PyObject* o) {
     const double v = PyFloat_AsDouble(o);
@@ -374,7 +386,7 @@ PyObject* qk_norm_rope_store_partials(PyObject*, PyObject* const* a, Py_ssize_t 
 // ---- staircase prefill ------------------------------------------------------------------------------
 // The result as [N, Hq, d], or flattened to [N, Hq * d].  With caches, k and v are stored into them too.
 struct Caches { const Tensor &k, &v, &slot_mapping; };
-Tensor staircase(const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& cu_q_, const Tensor& cu_k_, int64_t S, int64_t max_seqlen,
+Tensor staircase(const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& cu_q_, const Tensor& cu_k_, int64_t S, PyObject* max_seqlen,
                  PyObject* scale, bool flat, const Caches* caches = nullptr) {
     need_gpu({&q_, &k_, &v_, &cu_q_, &cu_k_});
     NEED(q_.dim() == 3 && k_.dim() == 3 && v_.dim() == 3);
@@ -392,7 +404,7 @@ Tensor staircase(const Tensor& q_, const Tensor& k_, const Tensor& v_, const Ten
     auto call = [&](auto fn, auto... more) {
         return fn(ptr(q), ptr(k), ptr(v), ptr(o), q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1), hq * d, d,
                   static_cast<const int32_t*>(ptr(cu_q)), static_cast<const int32_t*>(ptr(cu_k)), (int32_t)(cu_k.numel() - 1),
-                  (int32_t)(max_seqlen > 0 ? max_seqlen : total), total, (int32_t)hq, (int32_t)hkv, (int32_t)d, (int32_t)S, scale_or_default(scale, d),
+                  (int32_t)to_int_or(max_seqlen, total), total, (int32_t)hq, (int32_t)hkv, (int32_t)d, (int32_t)S, scale_or_default(scale, d),
                   dtype_of(q), more...);
     };
     if (caches) {
@@ -407,11 +419,11 @@ Tensor staircase(const Tensor& q_, const Tensor& k_, const Tensor& v_, const Ten
     return o;
 }
 
-// q, k, v, cu_seqlens_q, cu_seqlens_k, staircase_size, max_seqlen (0: the token count), softmax_scale | None
+// q, k, v, cu_seqlens_q, cu_seqlens_k, staircase_size, max_seqlen (None or 0: the token count), softmax_scale | None
 PyObject* sparse_attn_varlen(PyObject*, PyObject* const* a, Py_ssize_t n) {
     ARGS(8);
     return guarded([&]() -> PyObject* {
-        return wrap(staircase(tensor(a[0]), tensor(a[1]), tensor(a[2]), tensor(a[3]), tensor(a[4]), integer(a[5]), integer(a[6]), a[7], false));
+        return wrap(staircase(tensor(a[0]), tensor(a[1]), tensor(a[2]), tensor(a[3]), tensor(a[4]), integer(a[5]), a[6], a[7], false));
     });
 }
 
@@ -495,10 +507,10 @@ PyObject* attention_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const bool have_cache = k_cache.numel() > 0 && v_cache.numel() > 0;
         need_gpu({&q});
         const Tensor &cu_q = tensor(a[6]), &cu_k = tensor(a[7]);
-        const int64_t S = integer(a[8]), max_seqlen = integer(a[9]);
-        if (!have_cache) return wrap(staircase(q, k, v, cu_q, cu_k, S, max_seqlen, a[10], true));
+        const int64_t S = integer(a[8]);
+        if (!have_cache) return wrap(staircase(q, k, v, cu_q, cu_k, S, a[9], a[10], true));
         const Caches caches{k_cache, v_cache, tensor(a[5])};
-        return wrap(staircase(q, k, v, cu_q, cu_k, S, max_seqlen, a[10], true, &caches));
+        return wrap(staircase(q, k, v, cu_q, cu_k, S, a[9], a[10], true, &caches));
     });
 }
 
@@ -551,8 +563,8 @@ Noise noise_of(PyObject* const* a, int64_t rows, int64_t vocab) {
         if (!z.tensor.is_contiguous()) z.tensor = z.tensor.contiguous();
     }
     if (z.seeded) {
-        z.seed = integer_mod64(a[1]);
-        z.offset = integer_mod64(a[2]);
+        z.seed = to_int_mod64(a[1]);
+        z.offset = to_int_mod64(a[2]);
         z.offset_dev = optional_tensor(a[3]);
         z.row_ids = optional_tensor(a[4]);
         if (z.offset_dev.defined()) NEED(z.offset_dev.scalar_type() == at::kLong && z.offset_dev.numel() == 1 && z.offset_dev.is_cuda());
@@ -614,7 +626,7 @@ PyObject* lm_head_confidence(PyObject*, PyObject* const* a, Py_ssize_t n) {
                 NEED(t.numel() > 0 && r.n % t.numel() == 0);
                 per_temp = r.n / t.numel();
             } else {
-                per_temp = integer(a[3]);
+                per_temp = to_int(a[3]);
             }
         }
         if (ids.defined()) NEED(ids.scalar_type() == at::kLong && ids.is_contiguous() && ids.numel() >= r.n);
@@ -653,7 +665,7 @@ Tensor filter(const Tensor& logits, int64_t top_k, double top_p, const Tensor& t
 PyObject* filter_logits(PyObject*, PyObject* const* a, Py_ssize_t n) {
     ARGS(5);
     return guarded([&]() -> PyObject* {
-        return wrap(filter(tensor(a[0]), integer(a[1]), real(a[2]), optional_tensor(a[3]), optional_tensor(a[4])));
+        return wrap(filter(tensor(a[0]), to_int(a[1]), real(a[2]), optional_tensor(a[3]), optional_tensor(a[4])));
     });
 }
 
@@ -669,7 +681,7 @@ PyObject* select_transfer(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const int64_t bs = tokens.size(0), S = tokens.size(1);
         Tensor transfer = make(tokens, at::kBool, bs, S), count = make(tokens, at::kInt, bs);
         check(mdx_select_transfer(static_cast<const int64_t*>(ptr(x0)), static_cast<const float*>(ptr(p)), static_cast<int64_t*>(ptr(tokens)),
-                                  integer(a[3]), (float)real(a[4]), (int32_t)integer(a[5]), static_cast<uint8_t*>(ptr(transfer)),
+                                  to_int(a[3]), (float)real(a[4]), (int32_t)to_int(a[5]), static_cast<uint8_t*>(ptr(transfer)),
                                   static_cast<int32_t*>(ptr(count)), (int32_t)bs, (int32_t)S, stream_of(tokens)), "select_transfer");
         return wrap_tuple(std::move(transfer), std::move(count));
     });
@@ -710,14 +722,14 @@ PyObject* unmask_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return guarded([&]() -> PyObject* {
         const Tensor &logits = tensor(a[0]), &tokens = tensor(a[1]), &temps = optional_tensor(a[5]);
         need_gpu({&logits, &tokens, &temps, &optional_tensor(a[8])});
-        const Filter f{integer(a[6]), real(a[7])};
+        const Filter f{to_int(a[6]), real(a[7])};
         NEED(tokens.scalar_type() == at::kLong && tokens.is_contiguous() && tokens.dim() == 2);
         const int64_t bs = tokens.size(0), S = tokens.size(1), vocab = logits.size(-1);
         NEED(logits.numel() == bs * S * vocab);
         Noise z = noise_of(a + 8, bs * S, vocab);
         Tensor x0 = make(tokens, at::kLong, bs, S), x0_p = make(tokens, at::kFloat, bs, S);
         Tensor transfer = make(tokens, at::kBool, bs, S), count = make(tokens, at::kInt, bs);
-        step(logits, bs, S, static_cast<int64_t*>(ptr(tokens)), integer(a[2]), (float)real(a[3]), (int32_t)integer(a[4]), temps, f, z,
+        step(logits, bs, S, static_cast<int64_t*>(ptr(tokens)), to_int(a[2]), (float)real(a[3]), (int32_t)to_int(a[4]), temps, f, z,
              static_cast<int64_t*>(ptr(x0)), static_cast<float*>(ptr(x0_p)), static_cast<uint8_t*>(ptr(transfer)), static_cast<int32_t*>(ptr(count)));
         return wrap_tuple(std::move(x0), std::move(x0_p), std::move(transfer), std::move(count));
     });
@@ -751,7 +763,7 @@ PyObject* sampler_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
         }
         const Noise z = noise_of(a + 8, bs * S, vocab);
         Tensor x0 = make(logits, at::kLong, bs, S), x0_p = make(logits, at::kFloat, bs, S);
-        step(logits, bs, S, reinterpret_cast<int64_t*>(host), integer(a[5]), (float)real(a[6]), (int32_t)integer(a[7]), temps, Filter{0, 1.0}, z,
+        step(logits, bs, S, reinterpret_cast<int64_t*>(host), to_int(a[5]), (float)real(a[6]), (int32_t)to_int(a[7]), temps, Filter{0, 1.0}, z,
              static_cast<int64_t*>(ptr(x0)), static_cast<float*>(ptr(x0_p)), reinterpret_cast<uint8_t*>(host + flags_at),
              reinterpret_cast<int32_t*>(host + counts_at));
         hipError_t rc;
@@ -767,7 +779,7 @@ PyObject* sampler_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
             std::memcpy(&c, host + counts_at + 4 * i, 4);
             total += c;
             const Tensor& map = tensor(PyList_GET_ITEM(a[3], i));
-            const int64_t at_step = integer(PyList_GET_ITEM(a[4], i));
+            const int64_t at_step = to_int(PyList_GET_ITEM(a[4], i));
             NEED(map.numel() == S);
             if (map.is_cpu() && map.scalar_type() == at::kInt && map.is_contiguous()) {
                 int32_t* m = static_cast<int32_t*>(ptr(map));

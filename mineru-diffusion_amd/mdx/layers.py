@@ -26,7 +26,7 @@ class Attention(nn.Module):
         if context.is_prefill:
             # the prefill attention reads k / v, not the cache: the store rides in its launch where the rows allow it
             return _host().attention_prefill(q, k, v, self.k_cache, self.v_cache, context.slot_mapping, context.cu_seqlens_q,
-                                             context.cu_seqlens_k, context.block_size, context.max_seqlen_k or 0, self.scale)
+                                             context.cu_seqlens_k, context.block_size, context.max_seqlen_k, self.scale)
         return _host().attention_decode(q, k, v, self.k_cache, self.v_cache, context.slot_mapping, context.context_lens,
                                         context.block_tables, self.scale)
 

@@ -95,7 +95,7 @@ def sparse_attn_varlen(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_seq
     rows beyond it are not computed, and the lengths live on the device, so this call cannot check
     it.  None (the default) takes the total token count, which is always enough; the engine passes
     the value it computed on the host while building cu_seqlens (Context.max_seqlen_k)."""
-    return _host().sparse_attn_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, staircase_size, max_seqlen or 0, softmax_scale)
+    return _host().sparse_attn_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, staircase_size, max_seqlen, softmax_scale)
 
 
 sparse_attn_varlen_v2 = sparse_attn_varlen

@@ -326,3 +326,34 @@ def test_host_functions_refuse_sizes_of_zero(dev):
     rows = new(4, 0, 128).as_strided((4, 0, 128), (0, 128, 1))
     with pytest.raises(AssertionError):
         mdx.store_kvcache(rows, rows, new(1, 256, 0, 128).as_strided((1, 256, 0, 128), (0, 0, 128, 1)), new(1, 256, 0, 128), slots)
+
+
+def test_whole_number_arguments_are_taken_as_int_takes_them(dev):
+    """int() stood before these arguments: floats and one-element tensors count as the integers they truncate to.  A negative
+    max_seqlen is an error, not the default."""
+    import mdx
+    g = torch.Generator(device=dev).manual_seed(4)
+    logits = (torch.randn(2, 4, 3000, generator=g, device=dev) * 3).bfloat16()
+    masks = torch.full((2, 4), 9, dtype=torch.int64, device=dev)
+
+    def step(as_given):
+        tokens = masks.clone()
+        return [*mdx.unmask_step(logits, tokens, as_given(9), 0.9, as_given(2), top_k=as_given(40), seed=as_given(77), offset=as_given(3)), tokens]
+
+    want = step(int)
+    for as_given in (float, lambda n: n + 0.75, torch.tensor, np.int32):
+        assert all(torch.equal(a, b) for a, b in zip(step(as_given), want))
+    assert torch.equal(mdx.filter_logits(logits, 40.5), mdx.filter_logits(logits, 40))
+    x0, p = mdx.confidence_argmax(logits, seed=77.9, offset=3.0)
+    assert torch.equal(x0, mdx.confidence_argmax(logits, seed=77, offset=3)[0])
+    assert all(torch.equal(a, b) for a, b in zip(mdx.select_transfer(x0, p, masks.clone(), 9.0, 0.9, 2.0), mdx.select_transfer(x0, p, masks.clone(), 9, 0.9, 2)))
+    x, w, temps = torch.randn(8, 128, device=dev).bfloat16(), torch.randn(512, 128, device=dev).bfloat16(), torch.tensor([0.5, 2.0], device=dev)
+    assert torch.equal(mdx.lm_head_confidence(x, w, temps, rows_per_temp=4.0)[1], mdx.lm_head_confidence(x, w, temps, rows_per_temp=4)[1])
+    q, cu = torch.randn(96, 2, 128, device=dev).bfloat16(), torch.tensor([0, 96], dtype=torch.int32, device=dev)
+    whole = mdx.sparse_attn_varlen(q, q, q, cu, cu, 32)
+    for longest in (None, 0, 96, 96.5):
+        assert torch.equal(mdx.sparse_attn_varlen(q, q, q, cu, cu, 32, max_seqlen=longest), whole)
+    with pytest.raises(mdx.MdxError):
+        mdx.sparse_attn_varlen(q, q, q, cu, cu, 32, max_seqlen=-1)
+    with pytest.raises(TypeError):
+        mdx.filter_logits(logits, [4])
