@@ -295,6 +295,11 @@ PyObject* silu_and_mul(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // ---- linear layers of a decode pass -----------------------------------------------------------------
+// The kernels' rows: bf16, 16-byte aligned, dense along k.  (What is not, as a weight that is a view at an odd offset, takes the library's product.)
+bool rows_covered(const Rows& r, int64_t k) {
+    return r.t.scalar_type() == at::kBFloat16 && r.t.stride(-1) == 1 && r.stride >= k && r.stride % 8 == 0 && reinterpret_cast<uintptr_t>(ptr(r.t)) % 16 == 0;
+}
+
 // x [.., k], w [n, k] -> fp32 partial sums [splits, .., n], or None where the shape is not covered
 PyObject* linear_partials(PyObject*, PyObject* const* a, Py_ssize_t n) {
     ARGS(2);
@@ -304,8 +309,9 @@ PyObject* linear_partials(PyObject*, PyObject* const* a, Py_ssize_t n) {
         NEED(x.dim() >= 2 && w.dim() == 2 && x.size(-1) == w.size(1));
         const int64_t k = w.size(1), cols = w.size(0), rows = k ? x.numel() / k : 0;
         const int32_t splits = mdx_decode_linear_splits(rows, cols, k);
-        if (splits == 0 || x.scalar_type() != at::kBFloat16 || w.scalar_type() != at::kBFloat16 || x.stride(-1) != 1 || w.stride(1) != 1) Py_RETURN_NONE;
+        if (splits == 0) Py_RETURN_NONE;
         const Rows r = rows_of(x, k);
+        if (!rows_covered(r, k) || !rows_covered(rows_of(w, k), k)) Py_RETURN_NONE;
         std::vector<int64_t> shape{splits};
         shape.insert(shape.end(), x.sizes().begin(), x.sizes().end() - 1);
         shape.push_back(cols);
@@ -323,9 +329,9 @@ PyObject* linear_silu(PyObject*, PyObject* const* a, Py_ssize_t n) {
         need_gpu({&x, &w});
         NEED(x.dim() >= 2 && w.dim() == 2 && x.size(-1) == w.size(1) && w.size(0) % 2 == 0);
         const int64_t k = w.size(1), cols = w.size(0) / 2, rows = k ? x.numel() / k : 0;
-        if (!mdx_decode_linear_silu_supported(rows, cols, k) || x.scalar_type() != at::kBFloat16 || w.scalar_type() != at::kBFloat16 || x.stride(-1) != 1 || w.stride(1) != 1)
-            Py_RETURN_NONE;
+        if (!mdx_decode_linear_silu_supported(rows, cols, k)) Py_RETURN_NONE;
         const Rows r = rows_of(x, k);
+        if (!rows_covered(r, k) || !rows_covered(rows_of(w, k), k)) Py_RETURN_NONE;
         std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());
         shape.back() = cols;
         Tensor y = at::empty(shape, at::TensorOptions().dtype(at::kBFloat16).device(x.device()));

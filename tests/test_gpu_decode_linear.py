@@ -37,6 +37,17 @@ def test_linear_partials_and_silu_say_what_they_do_not_cover(dev):
     assert ops.linear_silu(z(65, 512), z(48, 512)) is None and ops.linear_silu(z(4, 256), z(48, 256)) is None
 
 
+@pytest.mark.parametrize("x_at,x_pad,w_at,w_pad", [(1, 0, 0, 0), (0, 3, 0, 0), (0, 0, 1, 0), (0, 0, 0, 4), (0, -256, 0, 0)])
+def test_linear_leaves_rows_that_are_not_aligned_to_the_library(dev, x_at, x_pad, w_at, w_pad):
+    """A view off a 16-byte boundary, rows whose stride is no multiple of 8 elements, and rows that overlap: None, not an error."""
+    from mdx import ops
+    k = 512
+    rows = lambda n, at, pad: torch.zeros(n * (k + 8) + 8, dtype=torch.bfloat16, device=dev).as_strided((n, k), (k + pad, 1), at)    # noqa: E731
+    assert ops.linear_partials(rows(4, x_at, x_pad), rows(64, w_at, w_pad)) is None
+    assert ops.linear_silu(rows(4, x_at, x_pad), rows(48, w_at, w_pad)) is None
+    assert ops.linear_partials(rows(4, 8, 8), rows(64, 8, 8)) is not None and ops.linear_silu(rows(4, 8, 8), rows(48, 8, 8)) is not None
+
+
 @pytest.mark.parametrize("rows", [1, 16, 31, 32, 33, 64])
 @pytest.mark.parametrize("inter,k", [(24, 512), (72, 1536), (6144, 2048)])
 def test_linear_silu(dev, rows, inter, k):
