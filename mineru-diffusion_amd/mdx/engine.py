@@ -319,6 +319,7 @@ class Decoder(nn.Module):
 # ----------------------------------------------------------------------------- engine
 IDLE, DENOISING, CACHING = 0, 1, 2      # MDX_PHASE_* of include/mdx.h: the per-lane state of the device loop
 N_STOP = 4                              # stop-token ids per sequence that the device loop can check
+FUSED_HEAD_MIN_ROWS, FUSED_HEAD_FEW_ROWS = 384, 256      # rows of a pass from which, and up to which, the fused vocabulary head is the faster
 
 
 class _PagesShort(Exception):
@@ -342,9 +343,10 @@ class BlockDiffusionEngine:
                  max_num_seqs: int = 512, shuffle_pages_seed: int | None = None, on_logits=None, unmask=None,
                  decode_graphs: bool = False, max_model_len: int = 8192, masked_rows_only: bool = True,
                  replay_ahead: bool = True, gumbel_seed: int | None = None, fused_head: bool = True,
-                 fused_head_min_rows: int = 384):
+                 fused_head_min_rows: int = FUSED_HEAD_MIN_ROWS):
         self.model = model
-        # device loop: vocabulary projection + confidence in one pass without logits in HBM, from this many rows on
+        # device loop: vocabulary projection + confidence in one pass without logits in HBM, from this many rows on (left at its
+        # default: and up to FUSED_HEAD_FEW_ROWS, see _fused_head)
         self.fused_head, self.fused_head_min_rows = fused_head, fused_head_min_rows
         self.decode_graphs = decode_graphs                 # decode through the device loop (HIP graphs per batch size)
         self.max_model_len = max_model_len
@@ -649,10 +651,12 @@ class BlockDiffusionEngine:
             g["x0_p"].copy_(p.view(-1))
 
     def _fused_head(self, rows: int) -> bool:
-        """Projection and confidence in one pass that never writes the logits (mdx_lm_head_confidence): taken where it
-        is the faster of the two (from a few hundred rows on, and up to 256 rows: one tile of the kernel, or its form for
-        up to 128; between them the library GEMM + the vocabulary pass win), for bf16 weights without sampling noise."""
-        return (self.fused_head and self.gumbel_seed is None and (rows <= 256 or rows >= self.fused_head_min_rows)
+        """Projection and confidence in one pass that never writes the logits (mdx_lm_head_confidence), for bf16 weights
+        without sampling noise.  By default taken where it is the faster of the two: from 384 rows on, and up to 256 rows
+        (the kernel's form for up to 128, or one tile of it); between them the library GEMM + the vocabulary pass win.
+        A caller's own fused_head_min_rows is the one limit: never below it, always from it on."""
+        few = self.fused_head_min_rows == FUSED_HEAD_MIN_ROWS and rows <= FUSED_HEAD_FEW_ROWS
+        return (self.fused_head and self.gumbel_seed is None and (few or rows >= self.fused_head_min_rows)
                 and self.model.lm_head.dtype == torch.bfloat16 and self.model.lm_head.shape[1] % 128 == 0)
 
     def _draw(self, g, rows):

@@ -282,3 +282,13 @@ def test_oracle_block_advance_against_a_hand_written_trace():
     t2, _, _, p2, l2, _, s2 = oracle.block_advance(np.array([[5, 8, 7, 9]]), transfer, np.array([[0, 1, 0, 1]], dtype=np.int32),
                                                    np.array([2], dtype=np.int32), np.array([2]), np.array([10]), first, np.array([8]), stop, M)
     assert p2.tolist() == [1] and l2.tolist() == [14] and s2 == [(1, 14, 4, 0)] and t2.tolist() == [[M, M, M, M]]
+
+
+@pytest.mark.parametrize("given,taken", [({}, [1, 128, 256, 384, 1024]), (dict(fused_head_min_rows=500), [500, 1024]),
+                                         (dict(fused_head_min_rows=1), [1, 128, 256, 257, 383, 384, 500, 1024]), (dict(fused_head=False), [])])
+def test_fused_head_row_limits(given, taken):
+    """By default the few-rows form too; a limit that the caller sets is the only one."""
+    model = ScriptedModel()
+    model.lm_head = torch.zeros(64, 128, dtype=torch.bfloat16)
+    eng = BlockDiffusionEngine(model, num_pages=4, **given)
+    assert [r for r in (1, 128, 256, 257, 383, 384, 500, 1024) if eng._fused_head(r)] == taken
