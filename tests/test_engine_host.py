@@ -284,7 +284,7 @@ def test_oracle_block_advance_against_a_hand_written_trace():
     assert p2.tolist() == [1] and l2.tolist() == [14] and s2 == [(1, 14, 4, 0)] and t2.tolist() == [[M, M, M, M]]
 
 
-@pytest.mark.parametrize("given,taken", [({}, [1, 128, 256, 384, 1024]), (dict(fused_head_min_rows=500), [500, 1024]),
+@pytest.mark.parametrize("given,taken", [({}, [1, 128, 256, 384, 500, 1024]), (dict(fused_head_min_rows=500), [500, 1024]),
                                          (dict(fused_head_min_rows=1), [1, 128, 256, 257, 383, 384, 500, 1024]), (dict(fused_head=False), [])])
 def test_fused_head_row_limits(given, taken):
     """By default the few-rows form too; a limit that the caller sets is the only one."""
