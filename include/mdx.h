@@ -158,7 +158,7 @@ int mdx_staircase_attn_store(const void* q, const void* k, const void* v, void* 
  * of up to 256 columns), run in fp32 arithmetic on the fp32 matrix instruction.  Those calls need no workspace (the query
  * below returns 0 for those widths), but cut a context into pieces of keys, which fills the chip with few sequences, only
  * as far as the workspace they are given has room for the pieces' partials: mdx_paged_block_attn_f32_workspace_bytes says
- * what they can use.  (The last bits of a result depend on where a context is cut.)
+ * what they can use.  (The last bits of a result depend on where a context is cut, and so on the workspace given.)
  */
 int64_t mdx_paged_block_attn_f32_workspace_bytes(int32_t bs, int32_t sq, int32_t num_q_heads, int32_t head_dim,
                                                  int32_t max_pages, int32_t page_size);
@@ -208,13 +208,14 @@ int mdx_paged_block_attn_single_launch(const void* q, void* o, const void* k_cac
  * the reference, whose call sites allocate freely.  Same arguments, kernels and results (bit for
  * bit) as mdx_paged_block_attn, without the workspace: the split-KV partials go into a 40 MiB
  * device array that is part of the library image (each GPU the library runs on holds it until
- * the process ends).  Shapes whose partials need more (the size mdx_paged_block_attn_workspace_bytes
+ * the process ends).  Calls in fp32 arithmetic (see there) leave the array alone and cut no context:
+ * the results of mdx_paged_block_attn without a workspace.  Shapes whose partials need more (the size mdx_paged_block_attn_workspace_bytes
  * reports; 32 sequences x 16 heads with page tables of 17 pages need 32.5 MiB, 64 such sequences
  * 65 MiB) are refused with MDX_EWORKSPACE.
  * The call itself allocates and frees nothing; the first call on each device looks the array's
  * address up (hipGetSymbolAddress), so make that call outside graph capture.  All calls on one
  * GPU share the array: calls that may overlap (different streams) race on it; calls on one
- * stream do not.
+ * stream do not, nor do calls in fp32 arithmetic.
  */
 int mdx_paged_block_attn_static(const void* q, void* o, const void* k_cache, const void* v_cache,
                                 int64_t q_stride_b, int64_t q_stride_s, int64_t q_stride_h,

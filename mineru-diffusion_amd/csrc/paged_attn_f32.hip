@@ -62,7 +62,7 @@ __device__ __forceinline__ int keys_per_piece(const PagedWideParams& P, int ctx,
 }
 
 template <typename T, int D, int HPW, int KW>
-__global__ __launch_bounds__(64 * HPW * KW, D <= 128 ? 2 : 1) void paged_attn_f32_kernel(const PagedWideParams P)
+__global__ __launch_bounds__(64 * HPW * KW, D <= 128 && KW <= 2 ? 2 : 1) void paged_attn_f32_kernel(const PagedWideParams P)
 {
     constexpr int kThreads = 64 * HPW * KW;
     constexpr int kTileFloats = Lds<D>::kFloats;
@@ -96,20 +96,30 @@ __global__ __launch_bounds__(64 * HPW * KW, D <= 128 ? 2 : 1) void paged_attn_f3
         // ---- tiles t0 .. t0 + KW - 1 into LDS, all threads on each (a tile never straddles a page: page_size % 32 == 0, so that all
         //      its rows exist in memory, whatever they hold) ----
         unsigned tile_ok = 0;                                  // bit i: tile t0 + i exists and lies on a valid page (uniform)
-        TileRegs<T, D, kThreads> regs;
+        constexpr int kTogether = KW == 4 ? 4 : 1;             // tiles whose loads are in flight together: as registers allow
+        TileRegs<T, D, kThreads> regs[kTogether];
 #pragma unroll
-        for (int i = 0; i < KW; ++i) {
-            const int key0 = key_begin + (t0 + i) * kTileKeys;
-            const int page_slot = P.page_shift >= 0 ? key0 >> P.page_shift : key0 / P.page_size;
-            const int64_t page = key0 < key_end ? bt[page_slot] : -1;
-            const bool ok = page >= 0 && page < P.num_pages;
-            if (ok) tile_ok |= 1u << i;
-            const int64_t base = page * P.c_sp + (int64_t)(key0 - page_slot * P.page_size) * P.c_st;
+        for (int i0 = 0; i0 < KW; i0 += kTogether) {
+            int64_t base[kTogether];
+#pragma unroll
+            for (int j = 0; j < kTogether; ++j) {
+                const int key0 = key_begin + (t0 + i0 + j) * kTileKeys;
+                const int page_slot = P.page_shift >= 0 ? key0 >> P.page_shift : key0 / P.page_size;
+                const int64_t page = key0 < key_end ? bt[page_slot] : -1;
+                if (page >= 0 && page < P.num_pages) tile_ok |= 1u << (i0 + j);
+                base[j] = page * P.c_sp + (int64_t)(key0 - page_slot * P.page_size) * P.c_st;
+            }
 #pragma unroll 1
-            for (int b = 0; b < regs.kBatches; ++b) {
-                if (ok) regs.fetch(b, tid, width, [&](int row) { return kc + base + (int64_t)row * P.c_st; }, [&](int row) { return vc + base + (int64_t)row * P.c_st; });
-                if (i == 0 && b == 0 && t0) __syncthreads();   // the previous tiles have been read by everybody
-                if (ok) regs.write(b, lds + i * kTileFloats, tid, width, [&](int row) { return key0 + row < key_end; });
+            for (int b = 0; b < regs[0].kBatches; ++b) {
+#pragma unroll
+                for (int j = 0; j < kTogether; ++j)
+                    if ((tile_ok >> (i0 + j)) & 1u)
+                        regs[j].fetch(b, tid, width, [&](int row) { return kc + base[j] + (int64_t)row * P.c_st; }, [&](int row) { return vc + base[j] + (int64_t)row * P.c_st; });
+                if (i0 == 0 && b == 0 && t0) __syncthreads();  // the previous tiles have been read by everybody
+#pragma unroll
+                for (int j = 0; j < kTogether; ++j)
+                    if ((tile_ok >> (i0 + j)) & 1u)
+                        regs[j].write(b, lds + (i0 + j) * kTileFloats, tid, width, [&](int row) { return key_begin + (t0 + i0 + j) * kTileKeys + row < key_end; });
             }
         }
         __syncthreads();
@@ -216,10 +226,16 @@ int launch_groups(const PagedWideParams& P, hipStream_t stream)
     return mdx::check_launch("paged_combine (fp32 arithmetic)");
 }
 
-// KW: tiles of 32 keys staged side by side, two workgroups' worth of LDS per CU.
+// KW: tiles of 32 keys staged side by side, two workgroups' worth of LDS per CU.  Whole contexts for no more heads than there are
+// CUs (a caller without a workspace) are chains of tiles with CUs to spare: a workgroup per head, one per CU with all of its LDS, and
+// twice the wavefronts on the chain with the loads of four tiles in flight (us, two heads / one head per workgroup: d = 128, 4 x 2000
+// keys 231 / 154, 16 x 2000 246 / 173, 1 x 1056 119 / 84; d = 256, 4 x 2000 937 / 560, 16 x 1000 499 / 312).  More heads than CUs are
+// more than one round of such workgroups (24 x 2000, d = 128: 477, with two heads each 260).
 template <typename T>
 int launch(const PagedWideParams& P, hipStream_t stream)
 {
+    if (P.nsplit == 1 && (int64_t)P.bs * P.num_q_heads * P.nqt <= mdx::compute_units())
+        return P.head_dim <= 128 ? launch_groups<T, 128, 1, 4>(P, stream) : launch_groups<T, 256, 1, 2>(P, stream);
     const bool pairs = P.heads_per_kv % 2 == 0;
     if (P.head_dim <= 128) return pairs ? launch_groups<T, 128, 2, 2>(P, stream) : launch_groups<T, 128, 1, 2>(P, stream);
     return pairs ? launch_groups<T, 256, 2, 1>(P, stream) : launch_groups<T, 256, 1, 1>(P, stream);

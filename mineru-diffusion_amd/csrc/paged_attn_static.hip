@@ -56,8 +56,10 @@ extern "C" int mdx_paged_block_attn_static(const void* q, void* o, const void* k
     MDX_REQUIRE(need <= kStaticScratchBytes, MDX_EWORKSPACE,
                 "paged_block_attn_static: this shape needs %lld bytes of split partials, the static array holds %lld; "
                 "use mdx_paged_block_attn with a workspace", (long long)need, (long long)kStaticScratchBytes);
+    // fp32 arithmetic (launch_paged's rule) needs no workspace, and without one never touches the array: such calls may overlap
+    const bool partials = need > 0 && dtype != MDX_F32;                      // (need is 0 for the other widths of fp32 arithmetic)
     void* ws = nullptr;
-    if (need > 0) {
+    if (partials) {
         const int rc = static_scratch(&ws);
         if (rc != MDX_OK) return rc;
     }
@@ -66,5 +68,5 @@ extern "C" int mdx_paged_block_attn_static(const void* q, void* o, const void* k
     return mdx::launch_paged(q, o, k_cache, v_cache, q_stride_b, q_stride_s, q_stride_h, o_stride_b, o_stride_s, o_stride_h,
                         cache_stride_page, cache_stride_tok, cache_stride_head, block_table, bt_stride, context_lens,
                         bs, sq, num_q_heads, num_kv_heads, head_dim, max_pages, page_size, num_pages, scale, dtype,
-                        ws, need > 0 ? kStaticScratchBytes : 0, false, nullptr, 0, stream);
+                        ws, partials ? kStaticScratchBytes : 0, false, nullptr, 0, stream);
 }

@@ -78,3 +78,28 @@ def test_static_scratch_entry_point_refuses_what_does_not_fit(dev):
     rc = L.mdx_paged_block_attn_static(one, one, one, one, 65536, 2048, 128, 65536, 2048, 128, 262144, 1024, 128, one, 17, one,
                                        64, S, HQ, HKV, D, 17, PAGE, 100, 0.1, 0, None)
     assert rc == -3 and b"static array" in L.mdx_last_error()
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.float32, 128), (torch.float32, 256), (torch.bfloat16, 72), (torch.float16, 256)])
+@pytest.mark.parametrize("hq,hkv,ctxs", [(16, 8, [1056]), (6, 2, [300, 0, 2100, 33]), (16, 8, [70, 40, 129, 64] * 5)])
+def test_static_entry_point_in_fp32_arithmetic_takes_no_partials(dev, dtype, d, hq, hkv, ctxs):
+    """Such calls leave the static array alone (they may overlap) and walk whole contexts: the bits of mdx_paged_block_attn
+    without a workspace, for fewer heads than CUs and for more."""
+    import mdx
+    import oracle
+    L, g, page = mdx.lib(), torch.Generator().manual_seed(len(ctxs) + d), 64
+    bs, width = len(ctxs), max(1, -(-max(ctxs) // page))
+    q = torch.randn(bs, S, hq, d, generator=g).to(dtype).to(dev)
+    kc, vc = (torch.randn(bs * width, page, hkv, d, generator=g).to(dtype).to(dev) for _ in range(2))
+    bt = torch.randperm(bs * width, generator=g).int().view(bs, width).to(dev)
+    lens = torch.tensor(ctxs, dtype=torch.int32, device=dev)
+    code = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}[dtype]
+    o_ref, o_new = torch.full_like(q, float("nan")), torch.full_like(q, float("nan"))
+    rest = (kc.data_ptr(), vc.data_ptr(), *q.stride()[:3], *q.stride()[:3], *kc.stride()[:3], bt.data_ptr(), bt.stride(0), lens.data_ptr(),
+            bs, S, hq, hkv, d, width, page, kc.shape[0], 1 / math.sqrt(d), code)
+    stream = torch.cuda.current_stream().cuda_stream
+    assert L.mdx_paged_block_attn(q.data_ptr(), o_ref.data_ptr(), *rest, None, 0, stream) == 0
+    assert L.mdx_paged_block_attn_static(q.data_ptr(), o_new.data_ptr(), *rest, stream) == 0
+    assert torch.equal(o_ref, o_new)
+    ref = oracle.paged_block_attn(q.cpu(), kc.cpu(), vc.cpu(), bt.cpu(), lens.cpu(), 1 / math.sqrt(d))
+    assert (o_new.float().cpu() - ref).abs().max().item() < (2e-4 if dtype == torch.float32 else 2e-2)
