@@ -117,7 +117,7 @@ int mdx_staircase_attn_varlen(const void* q, const void* k, const void* v, void*
 /*
  * mdx_store_kvcache of k and v (dense rows, one slot per token) and mdx_staircase_attn_varlen, in either order: the two halves of
  * the attention layer's prefill (engines/nano_dvlm/nanovllm/layers/sdar_attention.py:37-47), which do not depend on each
- * other.  One launch for 16-bit tensors whose rows are aligned (16 bytes; rows of 2 KiB or a part of that by a power of two), else two.
+ * other.  One launch for 16-bit tensors whose rows are aligned to 16 bytes, else two.
  */
 int mdx_staircase_attn_store(const void* q, const void* k, const void* v, void* o,
                              int64_t q_stride_t, int64_t q_stride_h,

@@ -41,14 +41,16 @@ constexpr int kRowsPerWg = 128;    // 4 wavefronts x 32 query rows
 // The K/V rows of a layer go to the paged cache in the attention launch itself (mdx_staircase_attn_store): the
 // attention reads k and v, not the cache, so the rows are copied by workgroups behind the attention's, which find the chip
 // far from full (109 tokens are 16 attention workgroups), and the launch of the store, 2.4 us of an 11-us layer, is saved.  (The pair
-// kernel on a full chip: store_own_rows.)
-constexpr int kStoreTokens = 16;                               // tokens per workgroup at most: 16 loads of 16 bytes in flight per lane
+// kernel on a full chip: store_own_rows.)  Rows of any multiple of 16 bytes: store + attention as two launches / as one, 32 query heads
+// on 16 KV heads, 4 x 2000 tokens 162 / 155 us, 12 on 6, 8 x 2000 120 / 112, 16 on 16, 4 x 1000 46 / 43.  What this costs against a store
+// on a second stream: 16 heads on 16, where no pairs of heads fill the chip and the copies come last, 4 x 4000 338 / 348.
+constexpr int kStoreRounds = 16;                               // loads of 16 bytes in flight per lane at most
 struct StoreParams {
     const u32x4* key; const u32x4* value;
     int64_t k_stride16, v_stride16;                            // 16-byte units between tokens
     u32x4* k_cache; u32x4* v_cache;
     const int32_t* slot_mapping; int64_t num_slots;
-    int n_tokens, row16, tokens_per_wg;                        // row16: 16-byte units of a token's row, a divisor of kThreads / 2
+    int n_tokens, row16, units_per_wg;                         // row16: 16-byte units of a token's row
     int first_wg;                                              // workgroups from here on copy rows
     int own_rows;                                              // pair kernel: 1 each workgroup copies its own rows, 0 those from first_wg on do
 };
@@ -66,26 +68,35 @@ struct StaircaseParams {
     StoreParams store;
 };
 
-// Workgroup `wg` of the store: half of the lanes take K rows, half V rows.
+// Workgroup `wg` of the store: half of the lanes take units of K rows, half the same of V rows, row after row.
 __device__ __forceinline__ void store_rows(const StoreParams& S, int wg, int tid)
 {
-    const bool is_v = tid >= kThreads / 2;
-    const int lane = tid & (kThreads / 2 - 1), at_once = kThreads / 2 / S.row16;              // rows that half of the lanes cover
-    const int sub = lane / S.row16, col = lane % S.row16;
-    const int begin = wg * S.tokens_per_wg, end = min(S.n_tokens, begin + S.tokens_per_wg);
+    constexpr int kHalf = kThreads / 2;
+    const bool is_v = tid >= kHalf;
+    const int begin = wg * S.units_per_wg, end = min(S.n_tokens * S.row16, begin + S.units_per_wg);      // (below 2^30: the host)
     const u32x4* src = is_v ? S.value : S.key;
     const int64_t stride = is_v ? S.v_stride16 : S.k_stride16;
     u32x4* cache = is_v ? S.v_cache : S.k_cache;
-    u32x4 row[kStoreTokens];
-    int64_t slot[kStoreTokens];
+    const int unit = begin + (tid & (kHalf - 1)), first = unit / S.row16, first_col = unit - first * S.row16;
+    const int next = kHalf / S.row16, next_col = kHalf % S.row16;                                         // kHalf units further
+    u32x4 row[kStoreRounds];
+    int64_t slot[kStoreRounds];
+    int t = first, col = first_col;
+    auto advance = [&]() {
+        t += next;
+        col += next_col;
+        if (col >= S.row16) { col -= S.row16; ++t; }
+    };
 #pragma unroll
-    for (int i = 0; i < kStoreTokens; ++i) {
-        const int t = begin + i * at_once + sub;
-        slot[i] = t < end ? S.slot_mapping[t] : -1;
-        if (t < end) row[i] = __builtin_nontemporal_load(src + t * stride + col);
+    for (int i = 0; i < kStoreRounds; ++i, advance()) {
+        const bool on = unit + i * kHalf < end;
+        slot[i] = on ? S.slot_mapping[t] : -1;
+        if (on) row[i] = __builtin_nontemporal_load(src + t * stride + col);
     }
+    t = first;
+    col = first_col;
 #pragma unroll
-    for (int i = 0; i < kStoreTokens; ++i)
+    for (int i = 0; i < kStoreRounds; ++i, advance())
         if (slot[i] >= 0 && slot[i] < S.num_slots) __builtin_nontemporal_store(row[i], cache + slot[i] * S.row16 + col);
 }
 
@@ -705,10 +716,11 @@ int staircase(const void* q, const void* k, const void* v, void* o,
     if (store && grid < ((int64_t)1 << 30)) {
         P.store = *store;
         P.store.first_wg = (int)grid;
-        // one token per workgroup while that leaves them few, up to kStoreTokens rounds of rows (as many at once beside the pair kernel, which leaves few CUs)
-        const int rounds = !pairs && (store->n_tokens + 511) / 512 < kStoreTokens ? (store->n_tokens + 511) / 512 : kStoreTokens;
-        P.store.tokens_per_wg = rounds * (kThreads / 2 / store->row16);
-        const int64_t wgs = (store->n_tokens + P.store.tokens_per_wg - 1) / P.store.tokens_per_wg;
+        // one round per workgroup while that leaves them few, up to kStoreRounds (as many at once beside the pair kernel, which leaves few CUs)
+        const int64_t units = (int64_t)store->n_tokens * store->row16, wanted = units / (kThreads / 2) > store->n_tokens ? units / (kThreads / 2) : store->n_tokens;
+        const int rounds = !pairs && (wanted + 511) / 512 < kStoreRounds ? (int)((wanted + 511) / 512) : kStoreRounds;
+        P.store.units_per_wg = rounds * (kThreads / 2);
+        const int64_t wgs = (units + P.store.units_per_wg - 1) / P.store.units_per_wg;
         // Pairs: while the attention leaves CUs idle the rows go there (2 x 1000 tokens, 136 workgroups of 256: 29.8 us for the layer,
         // 31.2 with own rows, which lengthen every chain), as long as those CUs get through them in a few rounds (2 us each).
         P.store.own_rows = pairs && wgs > 4 * (mdx::compute_units() - grid);
@@ -773,15 +785,15 @@ extern "C" int mdx_staircase_attn_store(const void* q, const void* k, const void
     const int elem = dtype == MDX_F32 ? 4 : 2;
     const int64_t row = (int64_t)num_kv_heads * head_dim, row_bytes = row * elem;
     MDX_REQUIRE(k_stride_h == head_dim && v_stride_h == head_dim, MDX_EUNSUPPORTED, "staircase_attn_store: rows of k and v must be dense");
-    const int row16 = (int)(row_bytes / 16);
-    const bool along = total_tokens > 0 && total_tokens < ((int64_t)1 << 30) && k && v && k_cache && v_cache && slot_mapping && num_slots >= 0 &&
-                       row16 > 0 && row_bytes % 16 == 0 && row_bytes <= 16 * (kThreads / 2) && kThreads / 2 % row16 == 0 &&
+    const int64_t row16 = row_bytes / 16;
+    const bool along = total_tokens > 0 && total_tokens < ((int64_t)1 << 30) && row16 < ((int64_t)1 << 30) / total_tokens && k && v && k_cache && v_cache && slot_mapping && num_slots >= 0 &&
+                       row16 > 0 && row_bytes % 16 == 0 &&
                        (k_stride_t * elem) % 16 == 0 && (v_stride_t * elem) % 16 == 0 && k_stride_t >= 0 && v_stride_t >= 0 &&
                        mdx::aligned16(k) && mdx::aligned16(v) && mdx::aligned16(k_cache) && mdx::aligned16(v_cache);
     StoreParams S{};
     if (along)
         S = StoreParams{(const u32x4*)k, (const u32x4*)v, k_stride_t * elem / 16, v_stride_t * elem / 16, (u32x4*)k_cache, (u32x4*)v_cache,
-                        slot_mapping, num_slots, (int)total_tokens, row16, 0, 0, 0};
+                        slot_mapping, num_slots, (int)total_tokens, (int)row16, 0, 0, 0};
     bool stored = false;
     const int rc = staircase(q, k, v, o, q_stride_t, q_stride_h, k_stride_t, k_stride_h, v_stride_t, v_stride_h, o_stride_t, o_stride_h,
                              cu_seqlens_q, cu_seqlens_k, batch, max_seqlen, total_tokens, num_q_heads, num_kv_heads, head_dim, staircase_size,

@@ -242,13 +242,12 @@ def test_attention_forward_decode_context(dev):
 
 
 @pytest.mark.parametrize("lens", [[1], [33, 7], [109], [560, 300], [500] * 20, [561]])
-@pytest.mark.parametrize("hkv,d,dtype", [(8, 128, torch.bfloat16), (2, 64, torch.float16), (1, 16, torch.bfloat16), (3, 128, torch.bfloat16), (8, 128, torch.float32)])
+@pytest.mark.parametrize("hkv,d,dtype", [(8, 128, torch.bfloat16), (2, 64, torch.float16), (1, 16, torch.bfloat16), (3, 128, torch.bfloat16), (8, 128, torch.float32),
+                                         (16, 128, torch.bfloat16), (5, 112, torch.float16), (33, 16, torch.bfloat16)])     # 2, 0.55 and 0.52 of half a workgroup
 def test_attention_prefill_is_the_store_and_the_attention(dev, lens, hkv, d, dtype):
     """The layer's prefill, which takes the rows of short prompts along in the attention launch, against the two calls: same
     output, same cache (slots -1 and beyond the cache are skipped), at few and many rows and row widths with and without that form."""
     import mdx
-    if dtype == torch.float32 and sum(lens) > 1000:
-        pytest.skip("covered by the 16-bit cases")
     g = torch.Generator(device=dev).manual_seed(sum(lens) + d)
     N, hq = sum(lens), 2 * hkv
     q, k = (torch.randn(N, h, d, generator=g, device=dev).to(dtype) for h in (hq, hkv))
@@ -279,6 +278,8 @@ def test_attention_prefill_is_the_store_and_the_attention(dev, lens, hkv, d, dty
     ([640] * 20, 2, 4, torch.bfloat16, 0, 0, None),                             # two pairs of query heads per KV head
     ([700, 0, 900, 650, 831, 777], 8, 2, torch.bfloat16, 130, 77, None),        # tokens outside every sequence
     ([700, 1300, 650, 831, 777, 1025], 8, 2, torch.float16, 1, 3, 850),         # sequences longer than max_seqlen says
+    ([700] * 2, 3, 2, torch.bfloat16, 5, 0, None),                              # rows that are no part of half a workgroup, on idle CUs
+    ([900] * 5, 16, 2, torch.bfloat16, 0, 9, None),                             # rows of two of them, with the row groups
 ])
 def test_pair_prefill_stores_every_row(dev, lens, hkv, ratio, dtype, before, behind, longest):
     """Prompts beyond 560 tokens (the kernel for pairs of heads): the rows that ride in its launch, against the store on its own."""
