@@ -45,6 +45,13 @@ constexpr int kQTile = 32;          // queries per workgroup (one per lane pair 
 constexpr int kMaxSq = 128;         // queries per sequence: up to four query tiles
 constexpr int kChunkAlign = 256;   // the host's split sizes are multiples of this many keys
 
+// Few sequences: the kernel's choice of pieces (PagedParams::fit_slots says why), and with the same figures the host's guess of it.
+constexpr float kPieceRoot = 4.f;                       // keys of a piece: this times the root of the launch's keys, from kLeastPiece on
+constexpr int kLeastPiece = 64;
+// Sequences are only cut if that takes more off the longest workgroup than the partials of them all cost (8 x 300 and 16 x 600
+// keys stay whole).
+template <typename T> __host__ __device__ __forceinline__ bool stay_whole(T longest, T piece, int sequences) { return longest - piece < T(64 + 12 * sequences); }
+
 // Sum over the 64 lanes: DPP shifts inside the rows of 16 lanes, the two row broadcasts, the total from lane 63
 // (six additions, no LDS traffic: the butterfly of cross-lane LDS permutes it replaces sat in every workgroup's start).
 __device__ __forceinline__ int wave_sum(int x) {
@@ -232,15 +239,14 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
             // 1100: 128, 4 x 1100: 192 to 256, 8 x 1100: 384, 16 x 1100, 4 x 8000: 512).  At least what fills the chip once, total / (resident
             // workgroups per head group - a remainder of half a piece per sequence), and no more pieces of a sequence than
             // the launch has room for (the "+ 1" keeps the longest within nsplit pieces whatever the rounding of the
-            // reciprocals; every workgroup makes the same estimate).  Sequences are only cut if that takes more off the longest
-            // workgroup than the partials of them all cost (8 x 300 and 16 x 600 keys stay whole).
+            // reciprocals; every workgroup makes the same estimate).
             const int total = wave_sum(ctx_l), longest = wave_max(ctx_l), live = wave_sum(ctx_l > 0 ? 1 : 0);
             const float per_group = (float)P.fit_slots * __builtin_amdgcn_rcpf((float)gridDim.x);      // resident workgroups per head group and query tile
             const float room = fmaxf(1.f, per_group - 0.5f * (float)live);
-            const int best = min(512, ((int)(4.f * __builtin_amdgcn_sqrtf((float)total)) + 32) & ~63);
+            const int best = min(512, ((int)(kPieceRoot * __builtin_amdgcn_sqrtf((float)total)) + 32) & ~63);
             const float least = fmaxf((float)total * __builtin_amdgcn_rcpf(room), (float)longest * __builtin_amdgcn_rcpf((float)P.nsplit) + 1.f);
-            span = max(max(64, best), ((int)least + 63) & ~63);
-            if (longest - span < 64 + 12 * live) span = max(span, longest);
+            span = max(max(kLeastPiece, best), ((int)least + 63) & ~63);
+            if (stay_whole(longest, span, live)) span = max(span, longest);
             n = splits_of_lane();
             // a tile more per step (24 steps double the smallest split); a few workgroups beyond what is resident
             // may stay: the last to start are remainders, which fill the tail
@@ -609,8 +615,8 @@ int nsplit_of(int bs, int64_t heads_and_tiles, int max_pages, int page_size, int
     const int64_t n = (max_keys + chunk - 1) / chunk;
     if (device_span || bs > 64) return (int)n;
     // sequences that the kernel would leave whole even in tables that are 65 % full need no slots, and no combine launch
-    const double longest = 0.65 * (double)max_keys, best = 4.0 * sqrt(longest * bs);
-    if (n == 1 && longest - (best > 64.0 ? best : 64.0) < 64.0 + 12.0 * bs) return 1;
+    const double longest = 0.65 * (double)max_keys, best = kPieceRoot * sqrt(longest * bs);
+    if (n == 1 && stay_whole(longest, best > kLeastPiece ? best : (double)kLeastPiece, bs)) return 1;
     int64_t own = 2;
     while ((own - 1) * (own - 1) * 16 < max_keys) ++own;
     if (own > 1024 / (bs * heads_and_tiles)) own = 1024 / (bs * heads_and_tiles);
