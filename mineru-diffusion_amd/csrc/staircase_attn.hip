@@ -673,16 +673,26 @@ int staircase(const void* q, const void* k, const void* v, void* o,
     // workgroups that row groups of `rows` rows come to, at most: ceil((L_b + S - 1) / rows) row groups per sequence
     const int64_t max_l = max_seqlen < total_tokens ? max_seqlen : total_tokens;
     auto groups_in = [&](int rows) { return (total_tokens + (int64_t)batch * (staircase_size + rows - 2)) / rows; };
+    // Two query heads per wavefront when the heads of a KV head pair up and 32-bit row offsets suffice.
+    const int64_t row_elems = k_stride_t > v_stride_t ? k_stride_t : v_stride_t;
+    // Sequences of a few hundred tokens are left to the one-head kernel: a pair workgroup owns a whole CU and its fixed cost (set-up,
+    // prologue, epilogue: 10 us) is then most of its time, while two one-head workgroups share a CU and hide each
+    // other's (one-head against pair, ms: 64 x 300 tokens 0.088 / 0.103, 32 x 500 0.074 / 0.081, 64 x 600 0.222 / 0.216,
+    // 32 x 700 0.130 / 0.128, 32 x 800 0.162 / 0.155, 32 x 1000 0.230 / 0.204, 16 x 2048 0.383 / 0.304).
+    // (its epilogue writes rows of o in 16-byte pieces, through 32-bit byte offsets from the wavefront's first row)
+    const bool may_pair = !narrow && max_l > 560 && o_stride_t % 8 == 0 && o_stride_h % 8 == 0 && o_stride_t > 0 &&
+                       o_stride_t * 2 * 128 < ((int64_t)1 << 31) && (num_q_heads / num_kv_heads) % 2 == 0 && k_stride_t > 0 && v_stride_t > 0 &&
+                       (max_l + 2 * kRowsPerWg) * row_elems * 2 < ((int64_t)1 << 31) && row_elems * 2 < (1 << 24) && max_l + 2 * kRowsPerWg < (1 << 24);
     // Two wavefronts per row tile while their workgroups (half the rows) are all on the chip at once, two per CU: such a launch
     // lasts as long as the longest chain of key tiles, which the split shortens (us, without / with: 200 tokens 10.6 / 8.6, 500
     // 17.4 / 13.0, 1000 28 / 21, 2000 46 / 39, 2 x 1000 28 / 23, 4 x 300 12.0 / 11.3); beyond, it only stages the keys more often
     // (4 x 1000 30 / 37, 8 x 300 13 / 16, 32 x 100 11 / 15).
-    // Against the kernel for pairs of heads (below), which such prompts of more than 560 tokens take otherwise, it pays a third further,
+    // Against the kernel for pairs of heads, where a launch would take that otherwise, it pays a third further,
     // while the workgroups that wait for a place are light ones: 2 x 1000 29.1 / 26.0, 2 x 1100 31.5 / 29.3, 1 x 2300 51.7 / 45.3, 1 x
     // 2600 58.2 / 51.9, 3 x 700 23.6 / 20.9, 400 to 1200 30.6 / 26.8; past that 2 x 1500 39 / 41, 3 x 1000 30.7 / 32.4, 1 x 3500 76 / 86.
-    const bool long_pairs = max_l > 560 && (num_q_heads / num_kv_heads) % 2 == 0;
-    const int64_t split_room = (int64_t)mdx::compute_units() * (long_pairs ? 27 : 20) / 10;
+    const int64_t split_room = (int64_t)mdx::compute_units() * (may_pair ? 27 : 20) / 10;
     const int kw = !narrow && groups_in(kRowsPerWg / 2) * num_q_heads <= split_room ? 2 : 1, rows_per_wg = kRowsPerWg / kw;
+    const bool pairs = may_pair && kw == 1;
     StaircaseParams P;
     P.q = (const __bf16*)q; P.k = (const __bf16*)k; P.v = (const __bf16*)v; P.o = (__bf16*)o;
     P.q_st = q_stride_t; P.q_sh = q_stride_h; P.k_st = k_stride_t; P.k_sh = k_stride_h;
@@ -700,16 +710,6 @@ int staircase(const void* q, const void* k, const void* v, void* o,
     const bool dense = batch <= 64 || (P.n_row_groups <= 64 && batch <= kDenseMaxBatch);
     const int64_t n_pairs = dense ? groups_in(rows_per_wg)
                                   : (int64_t)P.n_row_groups * batch;
-    // Two query heads per wavefront when the heads of a KV head pair up and 32-bit row offsets suffice.
-    const int64_t row_elems = k_stride_t > v_stride_t ? k_stride_t : v_stride_t;
-    // Sequences of a few hundred tokens are left to the one-head kernel: a pair workgroup owns a whole CU and its fixed cost (set-up,
-    // prologue, epilogue: 10 us) is then most of its time, while two one-head workgroups share a CU and hide each
-    // other's (one-head against pair, ms: 64 x 300 tokens 0.088 / 0.103, 32 x 500 0.074 / 0.081, 64 x 600 0.222 / 0.216,
-    // 32 x 700 0.130 / 0.128, 32 x 800 0.162 / 0.155, 32 x 1000 0.230 / 0.204, 16 x 2048 0.383 / 0.304).
-    // (its epilogue writes rows of o in 16-byte pieces, through 32-bit byte offsets from the wavefront's first row)
-    const bool pairs = kw == 1 && !narrow && max_l > 560 && o_stride_t % 8 == 0 && o_stride_h % 8 == 0 && o_stride_t > 0 &&
-                       o_stride_t * 2 * 128 < ((int64_t)1 << 31) && (num_q_heads / num_kv_heads) % 2 == 0 && k_stride_t > 0 && v_stride_t > 0 &&
-                       (max_l + 2 * rows_per_wg) * row_elems * 2 < ((int64_t)1 << 31) && row_elems * 2 < (1 << 24) && max_l + 2 * rows_per_wg < (1 << 24);
     int64_t grid = n_pairs * (pairs ? num_q_heads / 2 : num_q_heads);
     P.store = StoreParams{};
     P.store.first_wg = 0x7fffffff;
