@@ -120,6 +120,64 @@ def test_fused_head_and_calibration_arguments_are_validated(L):
     assert L.mdx_calib_mfma_loop_flops(16, 256, 3) == 256 * 4 * 8 * 16 * 16 * 16 * 32 * 2              # iterations rounded up to 8
 
 
+def test_calls_that_join_two_steps_refuse_what_either_does(L):
+    """mdx_staircase_attn_store and mdx_unmask_step_filtered."""
+    null, one, big = None, ctypes.c_void_p(16), ctypes.c_void_p(1 << 20)
+    st = lambda **kw: L.mdx_staircase_attn_store(                                                # noqa: E731
+        kw.get("q", one), one, one, one, 2048, 128, 1024, kw.get("ksh", 128), 1024, kw.get("vsh", 128), 2048, 128, one, one, kw.get("batch", 1),
+        kw.get("longest", 100), 100, kw.get("hq", 16), kw.get("hkv", 8), kw.get("d", 128), kw.get("S", 32), kw.get("scale", 0.1), kw.get("dtype", 0),
+        kw.get("kc", one), one, kw.get("slots", one), kw.get("num_slots", 10), null)
+    assert st(ksh=64) == -2 and b"dense" in L.mdx_last_error() and st(vsh=256) == -2
+    assert st(q=null) == -1 and st(batch=-1) == -1 and st(longest=-1) == -1 and st(hq=12) == -1 and st(S=48) == -1 and st(scale=0.0) == -1
+    assert st(dtype=7) == -2
+    fs = lambda **kw: L.mdx_unmask_step_filtered(                                                # noqa: E731
+        kw.get("logits", one), kw.get("stride", 1000), kw.get("dtype", 0), null, kw.get("top_k", 50), kw.get("top_p", 0.9), kw.get("noise", null),
+        kw.get("noise_stride", 0), kw.get("seeded", 0), 1, 2, null, kw.get("tokens", one), 7, 0.9, kw.get("k", 1), kw.get("x0", one), one, one,
+        kw.get("count", one), kw.get("bs", 4), kw.get("S", 32), kw.get("vocab", 1000), kw.get("ws", big), kw.get("ws_bytes", 1 << 30), null)
+    for bad in ("logits", "tokens", "x0", "count"):
+        assert fs(**{bad: null}) == -1 and b"null" in L.mdx_last_error()
+    assert fs(noise=one, noise_stride=1000, seeded=1) == -1 and b"seed" in L.mdx_last_error()
+    assert fs(noise=one, noise_stride=999) == -1
+    assert fs(k=-1) == -1 and fs(bs=-1) == -1 and fs(S=1025) == -2 and fs(stride=999) == -2 and fs(dtype=2) == -2 and fs(vocab=0) == -1
+    assert fs(top_k=-1) == -1 and fs(top_p=-0.1) == -1 and fs(top_p=float("nan")) == -1
+    assert fs(bs=0) == 0 and fs(S=0) == 0
+    for top_k in (50, 0):                                                                        # candidate lists; row cut-offs
+        need = L.mdx_unmask_step_filtered_workspace_bytes(4 * 32, 1000, top_k)
+        assert need > 0
+        assert fs(top_k=top_k, ws=null) == -3 and fs(top_k=top_k, ws_bytes=need - 1) == -3 and b"workspace" in L.mdx_last_error()
+        assert fs(top_k=top_k, ws=ctypes.c_void_p((1 << 20) + 8), ws_bytes=need) == -3
+    assert L.mdx_unmask_step_filtered_workspace_bytes(0, 1000, 50) == 0 and L.mdx_unmask_step_filtered_workspace_bytes(4, 0, 50) == 0
+
+
+def test_decode_linear_arguments_are_validated(L):
+    """The products of few rows and the two calls that take their partial sums."""
+    null, one, odd = None, ctypes.c_void_p(16), ctypes.c_void_p(24)
+    assert L.mdx_decode_linear_splits(32, 2048, 2048) > 0 and 2048 // 256 % L.mdx_decode_linear_splits(32, 2048, 2048) == 0
+    for rows, n, k in ((0, 64, 256), (129, 64, 256), (-1, 64, 256), (4, 72, 256), (4, 0, 256), (4, -64, 256), (4, 64, 320), (4, 64, 0), (4, 1 << 30, 256)):
+        assert L.mdx_decode_linear_splits(rows, n, k) == 0
+    pl = lambda **kw: L.mdx_decode_linear_partials(kw.get("x", one), kw.get("xs", 256), kw.get("w", one), kw.get("ws", 256), kw.get("p", one),    # noqa: E731
+                                                   kw.get("rows", 4), 64, 256, null)
+    sl = lambda **kw: L.mdx_decode_linear_silu(kw.get("x", one), kw.get("xs", 512), kw.get("w", one), kw.get("ws", 512), kw.get("y", one),        # noqa: E731
+                                               kw.get("ys", 24), kw.get("rows", 4), kw.get("n", 24), 512, null)
+    for call in (pl, sl):
+        assert call(x=null) == -1 and call(w=null) == -1 and b"null" in L.mdx_last_error()
+        assert call(x=odd) == -2 and call(w=odd) == -2 and call(xs=100) == -2 and call(ws=515) == -2 and call(xs=516) == -2
+        assert call(rows=129) == -2
+    assert pl(p=null) == -1 and pl(p=odd) == -2
+    assert sl(y=null) == -1 and sl(y=odd) == -2 and sl(ys=20) == -2 and sl(ys=26) == -2 and sl(rows=65) == -2 and sl(n=32) == -2
+    for rows, n, k in ((0, 24, 512), (65, 24, 512), (4, 16, 512), (4, 24, 256), (4, 0, 512)):
+        assert L.mdx_decode_linear_silu_supported(rows, n, k) == 0
+    rn = lambda **kw: L.mdx_add_rms_norm_partials(kw.get("p", one), kw.get("splits", 2), kw.get("res", one), kw.get("rs", 64), kw.get("res_out", one), 64,  # noqa: E731
+                                                  one, kw.get("eps", 1e-6), kw.get("out", one), 64, kw.get("rows", 4), kw.get("hidden", 64), kw.get("dtype", 0), null)
+    assert rn(p=null) == -1 and rn(out=null) == -1 and rn(res=null) == -1 and rn(splits=0) == -1 and rn(rs=56) == -1 and rn(eps=-1.0) == -1
+    assert rn(p=odd) == -2 and rn(hidden=60) == -2 and rn(dtype=2) == -2 and rn(rows=0) == 0
+    qk = lambda **kw: L.mdx_qk_norm_rope_store_partials(kw.get("p", one), kw.get("splits", 2), one, one, 1e-6, one, one, 64, kw.get("pos", one), one, 256,  # noqa: E731
+                                                        kw.get("kc", one), one, kw.get("slots", one), 10, kw.get("n", 4), kw.get("hq", 2), kw.get("hkv", 1),
+                                                        kw.get("d", 128), kw.get("dtype", 0), null)
+    assert qk(p=null) == -1 and qk(pos=null) == -1 and qk(kc=null) == -1 and qk(slots=null) == -1 and qk(splits=0) == -1 and qk(hq=0) == -1 and qk(hkv=0) == -1
+    assert qk(p=odd) == -2 and qk(d=64) == -2 and qk(dtype=1) == -2 and qk(n=0) == 0
+
+
 def test_ops_fail_loudly_off_gpu():
     import torch
     import mdx
