@@ -156,7 +156,7 @@ __global__ __launch_bounds__(2 * D) void paged_combine_f32_kernel(const PagedWid
     const int s = quarter * 8 + threadIdx.x / (D / 4), d = threadIdx.x % (D / 4) * 4;
     const int ctx = keys_of(P, b);
     const int span = keys_per_piece(P, ctx, threadIdx.x & 63);
-    const int n = (ctx + span - 1) / span;
+    const int n = __builtin_amdgcn_readfirstlane((ctx + span - 1) / span);
     const int qrow = qt * 32 + s;
     if (n <= 1 || qrow >= P.sq || d >= P.head_dim) return;      // one piece: written by the attention kernel
     const int64_t slot0 = (((int64_t)b * P.num_q_heads + head) * P.nqt + qt) * P.nsplit;
@@ -182,7 +182,8 @@ __global__ __launch_bounds__(2 * D) void paged_combine_f32_kernel(const PagedWid
         M = Mn;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const float w = i0 + i < n ? __builtin_amdgcn_exp2f(m[i] - M) : 0.f;
+            if (i0 + i >= n) break;                             // (nothing of the others: 0 x infinity is not 0)
+            const float w = __builtin_amdgcn_exp2f(m[i] - M);
             L += w * l[i];
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[e] += w * po[i][e];

@@ -281,6 +281,23 @@ def test_paged_fp32_contexts_cut_into_pieces(dev, ctxs, room):
     assert (ws[n_bytes:] == 255).all()
 
 
+@pytest.mark.parametrize("ctx,key", [(300, 1.0), (1056, 0.3), (1056, 1.0), (2000, 1.0)])
+@pytest.mark.parametrize("dtype,d", [(torch.float32, 128), (torch.bfloat16, 128), (torch.float32, 256)])
+def test_paged_infinite_values_stay_in_their_column(dev, ctx, key, dtype, d):
+    """An infinity in V is one in its column of every query's output, however the context is cut, and nowhere else."""
+    import mdx
+    g = torch.Generator().manual_seed(ctx)
+    q, kc, vc, bt, lens = _paged_inputs(g, [ctx], 32, 4, 2, d, dtype)
+    page, key = kc.shape[1], int(key * (ctx - 1))
+    vc[bt[0, key // page].item(), key % page, 0, 3] = float("inf")
+    o = mdx.flash_attn_with_kvcache(*(t.to(dev) for t in (q, kc, vc)), cache_seqlens=lens.to(dev), block_table=bt.to(dev), softmax_scale=0.1).float().cpu()
+    assert (o[0, :, :2, 3] == float("inf")).all()
+    vc[bt[0, key // page].item(), key % page, 0, 3] = 0.0
+    ref = oracle.paged_block_attn(q, kc, vc, bt, lens, 0.1)
+    o[0, :, :2, 3] = ref[0, :, :2, 3]
+    assert (o - ref).abs().max().item() < (TOL_F32 if dtype == torch.float32 else TOL_16)
+
+
 @pytest.mark.parametrize("lens", [[64, 33, 1] * 14, [65] * 20 + [1, 32], [390, 31, 65, 7], [129, 300] * 3, [1100, 5, 260]])
 def test_fp32_prefill_keys_shared_by_one_two_or_four_wavefronts(dev, lens):
     """Both sides of the rule that splits a row tile's keys: full launches of short prompts, ragged ones in between, long chains."""
