@@ -785,10 +785,14 @@ extern "C" int mdx_staircase_attn_store(const void* q, const void* k, const void
     const int elem = dtype == MDX_F32 ? 4 : 2;
     const int64_t row = (int64_t)num_kv_heads * head_dim, row_bytes = row * elem;
     MDX_REQUIRE(k_stride_h == head_dim && v_stride_h == head_dim, MDX_EUNSUPPORTED, "staircase_attn_store: rows of k and v must be dense");
+    // what the store would refuse, before the attention is launched
+    MDX_REQUIRE(total_tokens <= 0 || (k_cache && v_cache && slot_mapping), MDX_EINVAL, "staircase_attn_store: null pointer");
+    MDX_REQUIRE(num_slots >= 0, MDX_EINVAL, "staircase_attn_store: negative size");
+    MDX_REQUIRE(k_stride_t >= 0 && v_stride_t >= 0, MDX_EUNSUPPORTED, "staircase_attn_store: negative row stride");
     const int64_t row16 = row_bytes / 16;
-    const bool along = total_tokens > 0 && total_tokens < ((int64_t)1 << 30) && row16 < ((int64_t)1 << 30) / total_tokens && k && v && k_cache && v_cache && slot_mapping && num_slots >= 0 &&
+    const bool along = total_tokens > 0 && total_tokens < ((int64_t)1 << 30) && row16 < ((int64_t)1 << 30) / total_tokens && k && v &&
                        row16 > 0 && row_bytes % 16 == 0 &&
-                       (k_stride_t * elem) % 16 == 0 && (v_stride_t * elem) % 16 == 0 && k_stride_t >= 0 && v_stride_t >= 0 &&
+                       (k_stride_t * elem) % 16 == 0 && (v_stride_t * elem) % 16 == 0 &&
                        mdx::aligned16(k) && mdx::aligned16(v) && mdx::aligned16(k_cache) && mdx::aligned16(v_cache);
     StoreParams S{};
     if (along)

@@ -124,12 +124,14 @@ def test_calls_that_join_two_steps_refuse_what_either_does(L):
     """mdx_staircase_attn_store and mdx_unmask_step_filtered."""
     null, one, big = None, ctypes.c_void_p(16), ctypes.c_void_p(1 << 20)
     st = lambda **kw: L.mdx_staircase_attn_store(                                                # noqa: E731
-        kw.get("q", one), one, one, one, 2048, 128, 1024, kw.get("ksh", 128), 1024, kw.get("vsh", 128), 2048, 128, one, one, kw.get("batch", 1),
+        kw.get("q", one), one, one, one, 2048, 128, kw.get("kst", 1024), kw.get("ksh", 128), 1024, kw.get("vsh", 128), 2048, 128, one, one, kw.get("batch", 1),
         kw.get("longest", 100), 100, kw.get("hq", 16), kw.get("hkv", 8), kw.get("d", 128), kw.get("S", 32), kw.get("scale", 0.1), kw.get("dtype", 0),
         kw.get("kc", one), one, kw.get("slots", one), kw.get("num_slots", 10), null)
     assert st(ksh=64) == -2 and b"dense" in L.mdx_last_error() and st(vsh=256) == -2
     assert st(q=null) == -1 and st(batch=-1) == -1 and st(longest=-1) == -1 and st(hq=12) == -1 and st(S=48) == -1 and st(scale=0.0) == -1
     assert st(dtype=7) == -2
+    # the store's own refusals come before the attention's launch (which would end in a launch error here)
+    assert st(kc=null) == -1 and st(slots=null) == -1 and st(num_slots=-1) == -1 and st(kst=-1024) == -2
     fs = lambda **kw: L.mdx_unmask_step_filtered(                                                # noqa: E731
         kw.get("logits", one), kw.get("stride", 1000), kw.get("dtype", 0), null, kw.get("top_k", 50), kw.get("top_p", 0.9), kw.get("noise", null),
         kw.get("noise_stride", 0), kw.get("seeded", 0), 1, 2, null, kw.get("tokens", one), 7, 0.9, kw.get("k", 1), kw.get("x0", one), one, one,
