@@ -731,7 +731,7 @@ def main():
             gf_ms, _ = time_kernel(unmask_gumbel_filtered, 2, max(3, K // 4), graph=True, before_timed=remask)
             result_ops["filter_logits"] = op_entry(fl_ms, fl_min, "hbm", 2 * c4["bytes"], 1e6, PEAK_HBM_GBS, "GB/s",
                                                    dict(top_k=50, top_p=0.9, sampled_step_on_the_filtered_logits_ms=round(gf_ms, 4),
-                                                        note="off by default in the reference; with both filters on a row is read five times (four counting passes and the writing pass)"))
+                                                        note="off by default in the reference; a row is read twice (one pass that counts its values, bound by LDS atomics, and the writing pass)"))
             del flt_out
         del c4
         torch.cuda.empty_cache()

@@ -218,7 +218,8 @@ __device__ __forceinline__ void pick_from_kept(uint32_t (&key)[N], const int (&c
 
 // The same from n candidates, of which the top-k keeps its own: moved together, to one per lane mostly, they take one draw of the
 // generator per 64, where N registers with a few kept elements each take N.  (384 rows, top-k 50 and top-p 0.9 of about 210
-// candidates, whole step: 38.5 -> 34.4 us, with the early lists and the lane-by-lane mass; 32 rows 21.2 -> 17.2; 384 rows, top-k 400: 73.3 -> 67.9.)
+// candidates, whole step: 38.5 -> 34.4 us, with the early lists and the lane-by-lane mass; 32 rows 21.2 -> 17.2; 384 rows, top-k 400: 73.3 -> 67.9; 0.3 and
+// 0.8 more since the masses are 64-bit.)
 constexpr int kManyKept = 8;
 template <typename T, int NOISE, int N>
 __device__ void pick_from_candidates(uint2* cand, int n, int lane, int top_k, float top_p, float c, const Drawn<NOISE>& drawn, int64_t& x0, float& x0_p)

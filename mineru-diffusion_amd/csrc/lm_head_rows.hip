@@ -10,7 +10,7 @@
 //  * otherwise x goes through LDS K step by K step with a barrier per step, W one step ahead.
 //
 // W is read with ordinary loads: marked nontemporal, the two loads that share a 128-byte line fetch it twice now and then (139
-// against 129 us at 32 rows).  Bound: HBM.  us at 16 / 32 / 64 / 128 rows: 119 / 120 / 139 / 166 (5.2 TB/s at 32 rows); the tiles of 256 rows of
+// against 129 us at 32 rows).  Bound: HBM.  us at 16 / 32 / 64 / 128 rows: 119 / 120 / 140 / 170 (5.2 TB/s at 32 rows); the tiles of 256 rows of
 // lm_head_unmask.hip 200 / 199 / 208 / 200, the library's product and a vocabulary pass 213 / 155 / 161 / 175.
 #include "lm_head.h"
 #include <atomic>
