@@ -429,17 +429,30 @@ int mdx_silu_and_mul(const void* x, int64_t x_row_stride, void* out, int64_t out
                      int64_t rows, int32_t intermediate, int32_t dtype, mdx_stream_t stream);
 
 /*
- * Linear layers of a decode pass, x . w^T for few rows (nanovllm/layers/linear.py as called at nanovllm/models/sdar.py:73-112);
- * x [rows, k], w [n, k], MDX_BF16, row strides in elements (multiples of 8), 16-byte aligned.
+ * Linear layers, x . w^T (nanovllm/layers/linear.py as called at nanovllm/models/sdar.py:73-112);
+ * x [rows, k], w [n, k], MDX_BF16, row strides in elements (multiples of 8), 16-byte aligned; n a multiple of 8, k of 128
+ * and at least 256, sizes and strides below 2^28.
  *
- * mdx_decode_linear_partials leaves the product as fp32 partial sums over slices of K, partials [splits, rows, n] (dense),
- * for one of the two kernels below that add them up and round the sum to bf16 as the layer's output; splits =
- * mdx_decode_linear_splits(rows, n, k), 0 where the shape is not covered (rows up to 128, n a multiple of 64, k of 256).
- * mdx_decode_linear_silu: w [2 n, k], gate rows then up rows; y [rows, n] = mdx_silu_and_mul of the product, with its
- * rounding points (rows up to 64, n a multiple of 24, k of 512: mdx_decode_linear_silu_supported).
+ * mdx_linear rounds the product to bf16, y [rows, n] (row stride a multiple of 4).  mdx_linear_partials leaves it as fp32
+ * partial sums over slices of K, partials [splits, rows, n] (dense), for one of the two kernels below that add them up and
+ * round the sum to bf16 as the layer's output.  mdx_linear_splits(rows, n, k): the number of slices where that is the faster
+ * of the two, 0 where mdx_linear is, -1 where a library's product is the better choice (more than 1536 rows) or the shape
+ * is not covered.  mdx_linear_silu: w [2 n, k], gate rows then up rows; y [rows, n] = mdx_silu_and_mul of the product, with
+ * its rounding points; mdx_linear_silu_supported: covered, and up to 8192 rows.
+ * mdx_decode_linear_partials and mdx_decode_linear_silu: the same for the few rows of a decode pass, always as partial sums
+ * (rows up to 128, n a multiple of 64, k of 256; splits = mdx_decode_linear_splits, 0 where not covered) and with the SiLU
+ * (rows up to 64, n a multiple of 24, k of 512: mdx_decode_linear_silu_supported).
  * mdx_add_rms_norm_partials and mdx_qk_norm_rope_store_partials are mdx_add_rms_norm and mdx_qk_norm_rope_store with
  * x / qkv given as such partial sums ([splits, rows, hidden], [splits, n_tokens, (Hq + 2 Hkv) * d]).
  */
+int32_t mdx_linear_splits(int64_t rows, int64_t n, int64_t k);
+int mdx_linear(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride,
+               void* y, int64_t y_row_stride, int64_t rows, int64_t n, int64_t k, mdx_stream_t stream);
+int mdx_linear_partials(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride,
+                        float* partials, int64_t rows, int64_t n, int64_t k, mdx_stream_t stream);
+int32_t mdx_linear_silu_supported(int64_t rows, int64_t n, int64_t k);
+int mdx_linear_silu(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride,
+                    void* y, int64_t y_row_stride, int64_t rows, int64_t n, int64_t k, mdx_stream_t stream);
 int32_t mdx_decode_linear_splits(int64_t rows, int64_t n, int64_t k);
 int mdx_decode_linear_partials(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride,
                                float* partials, int64_t rows, int64_t n, int64_t k, mdx_stream_t stream);

@@ -340,6 +340,50 @@ PyObject* linear_silu(PyObject*, PyObject* const* a, Py_ssize_t n) {
     });
 }
 
+// x [.., k], w [n, k], partials_ok -> the product [.., n] in bf16, or (partials_ok, where that is the faster) its fp32 partial sums
+// [splits, .., n]; None where the library's product is the better one or the shape is not covered
+PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    ARGS(3);
+    return guarded([&]() -> PyObject* {
+        const Tensor &x = tensor(a[0]), &w = tensor(a[1]);
+        need_gpu({&x, &w});
+        NEED(x.dim() >= 2 && w.dim() == 2 && x.size(-1) == w.size(1));
+        const int64_t k = w.size(1), cols = w.size(0), rows = k ? x.numel() / k : 0;
+        const int32_t splits = mdx_linear_splits(rows, cols, k);
+        if (splits < 0) Py_RETURN_NONE;
+        const Rows r = rows_of(x, k);
+        if (!rows_covered(r, k) || !rows_covered(rows_of(w, k), k)) Py_RETURN_NONE;
+        const bool cut = splits > 0 && PyObject_IsTrue(a[2]) == 1;
+        std::vector<int64_t> shape;
+        if (cut) shape.push_back(splits);
+        shape.insert(shape.end(), x.sizes().begin(), x.sizes().end() - 1);
+        shape.push_back(cols);
+        Tensor y = at::empty(shape, at::TensorOptions().dtype(cut ? at::kFloat : at::kBFloat16).device(x.device()));
+        if (cut) check(mdx_linear_partials(ptr(r.t), r.stride, ptr(w), w.stride(0), static_cast<float*>(ptr(y)), rows, cols, k, stream_of(x)), "linear");
+        else check(mdx_linear(ptr(r.t), r.stride, ptr(w), w.stride(0), ptr(y), cols, rows, cols, k, stream_of(x)), "linear");
+        return wrap(std::move(y));
+    });
+}
+
+// x [.., k], w [2 n, k] -> silu_and_mul(x . w^T) [.., n], or None as above
+PyObject* linear_gated(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    ARGS(2);
+    return guarded([&]() -> PyObject* {
+        const Tensor &x = tensor(a[0]), &w = tensor(a[1]);
+        need_gpu({&x, &w});
+        NEED(x.dim() >= 2 && w.dim() == 2 && x.size(-1) == w.size(1) && w.size(0) % 2 == 0);
+        const int64_t k = w.size(1), cols = w.size(0) / 2, rows = k ? x.numel() / k : 0;
+        if (!mdx_linear_silu_supported(rows, cols, k)) Py_RETURN_NONE;
+        const Rows r = rows_of(x, k);
+        if (!rows_covered(r, k) || !rows_covered(rows_of(w, k), k)) Py_RETURN_NONE;
+        std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());
+        shape.back() = cols;
+        Tensor y = at::empty(shape, at::TensorOptions().dtype(at::kBFloat16).device(x.device()));
+        check(mdx_linear_silu(ptr(r.t), r.stride, ptr(w), w.stride(0), ptr(y), cols, rows, cols, k, stream_of(x)), "linear_gated");
+        return wrap(std::move(y));
+    });
+}
+
 void need_partials(const Tensor& p) { NEED(p.dim() >= 3 && p.scalar_type() == at::kFloat && p.is_contiguous()); }
 
 // partials [splits, .., hidden], weight, eps, residual [.., hidden] -> normed, new residual
@@ -806,7 +850,7 @@ PyObject* sampler_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 #define ENTRY(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
-    ENTRY(store_kvcache), ENTRY(store_kvcache_maybe4d), ENTRY(qk_norm_rope_store), ENTRY(rms_norm), ENTRY(silu_and_mul), ENTRY(linear_partials), ENTRY(linear_silu),
+    ENTRY(store_kvcache), ENTRY(store_kvcache_maybe4d), ENTRY(qk_norm_rope_store), ENTRY(rms_norm), ENTRY(silu_and_mul), ENTRY(linear), ENTRY(linear_gated), ENTRY(linear_partials), ENTRY(linear_silu),
     ENTRY(rms_norm_partials), ENTRY(qk_norm_rope_store_partials), ENTRY(sparse_attn_varlen),
     ENTRY(flash_attn_with_kvcache), ENTRY(attention_prefill), ENTRY(attention_decode), ENTRY(confidence_argmax), ENTRY(lm_head_confidence),
     ENTRY(filter_logits), ENTRY(select_transfer), ENTRY(unmask_step), ENTRY(sampler_step),

@@ -47,6 +47,11 @@ SIGNATURES = {
                                          _I64, _I32, _I32, _I32, _I32, _P]),
     "mdx_add_rms_norm": (c_int32, [_P, _I64, _P, _I64, _P, _I64, _P, _F, _P, _I64, _I64, _I32, _I32, _P]),
     "mdx_silu_and_mul": (c_int32, [_P, _I64, _P, _I64, _I64, _I32, _I32, _P]),
+    "mdx_linear_splits": (c_int32, [_I64] * 3),
+    "mdx_linear": (c_int32, [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _P]),
+    "mdx_linear_partials": (c_int32, [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _P]),
+    "mdx_linear_silu_supported": (c_int32, [_I64] * 3),
+    "mdx_linear_silu": (c_int32, [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _P]),
     "mdx_decode_linear_splits": (c_int32, [_I64] * 3),
     "mdx_decode_linear_partials": (c_int32, [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _P]),
     "mdx_decode_linear_silu_supported": (c_int32, [_I64] * 3),

@@ -32,7 +32,7 @@ from torch import nn
 from . import _lib
 from .context import get_context, reset_context, set_context
 from .layers import Attention
-from .ops import (confidence_argmax, lm_head_confidence, flash_attn_with_kvcache, linear_partials, linear_silu, qk_norm_rope_store,
+from .ops import (confidence_argmax, lm_head_confidence, flash_attn_with_kvcache, linear, linear_gated, qk_norm_rope_store,
                   qk_norm_rope_store_partials, rms_norm, rms_norm_partials, select_transfer, silu_and_mul, sparse_attn_varlen, unmask_step)
 
 PAGE = 256                      # tokens per KV page (Sequence.kvcache_block_size, sequence.py:17)
@@ -224,7 +224,7 @@ class DecoderLayer(nn.Module):
             o = self.attn(q, k, v)
         h, residual = self._norm(self._linear(o, self.o_proj), residual, self.post_attention_layernorm)
         if c.fused_layer_ops:
-            act = linear_silu(h, self.gate_up_proj)
+            act = linear_gated(h, self.gate_up_proj)
             if act is None:
                 act = silu_and_mul(F.linear(h, self.gate_up_proj))
         else:
@@ -233,23 +233,24 @@ class DecoderLayer(nn.Module):
         return self._linear(act, self.down_proj), residual
 
     def _linear(self, x, w):
-        """A linear layer whose output the next norm takes in: the partial sums of libmdx's product for the few rows of a
-        small decode batch, else the library's product."""
-        partials = linear_partials(x, w) if self.c.fused_layer_ops else None
-        return F.linear(x, w) if partials is None else partials
+        """A linear layer whose output the next norm takes in: libmdx's product, perhaps as partial sums, or the library's where
+        that is the better one."""
+        y = linear(x, w, True) if self.c.fused_layer_ops else None
+        return F.linear(x, w) if y is None else y
 
     def _attend_fused(self, h, positions, cos_table, sin_table):
         """sdar.py:73-83 + sdar_attention.py:34-57 with the q/k norm, RoPE and cache store done by
         one libmdx launch; the attention calls are the same two as in `Attention.forward`."""
         c, attn, ctx = self.c, self.attn, get_context()
         have_cache = attn.k_cache.numel() > 0
-        qkv = linear_partials(h, self.qkv_proj) if have_cache and not ctx.is_prefill else None
-        if qkv is not None:
+        qkv = linear(h, self.qkv_proj, have_cache and not ctx.is_prefill)
+        if qkv is None:
+            qkv = F.linear(h, self.qkv_proj)
+        if qkv.dim() > h.dim():
             q = qk_norm_rope_store_partials(qkv, self.q_norm, self.k_norm, c.rms_norm_eps, cos_table, sin_table, positions, c.num_heads,
                                             c.num_kv_heads, c.head_dim, attn.k_cache, attn.v_cache, ctx.slot_mapping)
             return flash_attn_with_kvcache(q, attn.k_cache, attn.v_cache, cache_seqlens=ctx.context_lens, block_table=ctx.block_tables,
                                            softmax_scale=attn.scale, causal=False).flatten(2)
-        qkv = F.linear(h, self.qkv_proj)
         q, k, v = qk_norm_rope_store(qkv, self.q_norm, self.k_norm, c.rms_norm_eps, cos_table, sin_table, positions,
                                      c.num_heads, c.num_kv_heads, c.head_dim,
                                      attn.k_cache if have_cache else None, attn.v_cache if have_cache else None,

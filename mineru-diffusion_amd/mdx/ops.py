@@ -60,27 +60,39 @@ def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
     return _host().silu_and_mul(x)
 
 
-# --------------------------------------------------------------------------- linear layers of a decode pass
-# x . weight^T for up to 128 rows as fp32 partial sums over slices of K ([splits, ..., n]), which the two functions after it add up
-# on their way; None where the shape is not covered (more rows, other widths), and the caller takes the library's product.
+# --------------------------------------------------------------------------- linear layers
+# Partial sums ([splits, ..., n] fp32) are the product's sums over slices of K, which rms_norm_partials and
+# qk_norm_rope_store_partials add up on their way.  None where the library's product is the better one (many rows) or the
+# shape is not covered.
+def linear(x: torch.Tensor, weight: torch.Tensor, partials: bool = False) -> torch.Tensor | None:
+    """x . weight^T (nanovllm/layers/linear.py) for up to 1536 rows: bf16 [..., n], or with `partials` what is the faster of
+    that and partial sums (one dimension more than x)."""
+    return _host().linear(x, weight, partials)
+
+
+def linear_gated(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor | None:
+    """silu_and_mul(x . weight^T) for up to 8192 rows in one launch (nanovllm/models/sdar.py:105-111)."""
+    return _host().linear_gated(x, weight)
+
+
 def linear_partials(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor | None:
-    """The product of a linear layer (nanovllm/layers/linear.py) for rms_norm_partials or qk_norm_rope_store_partials."""
+    """The partial sums of up to 128 rows, also where there is one slice only."""
     return _host().linear_partials(x, weight)
 
 
 def linear_silu(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor | None:
-    """silu_and_mul(x . weight^T) for up to 64 rows in one launch (nanovllm/models/sdar.py:105-111); None as above."""
+    """linear_gated for up to 64 rows (weight rows a multiple of 48, k of 512)."""
     return _host().linear_silu(x, weight)
 
 
 def rms_norm_partials(partials: torch.Tensor, weight: torch.Tensor, eps: float, residual: torch.Tensor):
-    """rms_norm(x, weight, eps, residual) with x given by linear_partials."""
+    """rms_norm(x, weight, eps, residual) with x given as partial sums."""
     return _host().rms_norm_partials(partials, weight, eps, residual)
 
 
 def qk_norm_rope_store_partials(partials, q_weight, k_weight, eps, cos, sin, positions, num_q_heads, num_kv_heads, head_dim,
                                 k_cache, v_cache, slot_mapping) -> torch.Tensor:
-    """The decode form of qk_norm_rope_store with qkv given by linear_partials: returns q; k and v go to the caches."""
+    """The decode form of qk_norm_rope_store with qkv given as partial sums: returns q; k and v go to the caches."""
     return _host().qk_norm_rope_store_partials(partials, q_weight, k_weight, eps, cos, sin, positions, num_q_heads, num_kv_heads, head_dim,
                                                k_cache, v_cache, slot_mapping)
 

@@ -212,3 +212,19 @@ def test_generated_kernel_core_is_current():
     # the core of the fused vocabulary projection
     out = subprocess.run([sys.executable, str(csrc / "gen_lm_head_core.py")], capture_output=True, text=True, check=True)
     assert out.stdout == (csrc / "lm_head_core.inc").read_text()
+
+
+def test_linear_arguments_are_validated(L):
+    null, one, odd = None, ctypes.c_void_p(16), ctypes.c_void_p(24)
+    for rows, n, k in ((0, 64, 256), (-1, 64, 256), (1537, 64, 256), (4, 68, 256), (4, 0, 256), (4, -64, 256), (4, 64, 320), (4, 64, 128), (4, 1 << 28, 256)):
+        assert L.mdx_linear_splits(rows, n, k) == -1
+    assert L.mdx_linear_splits(32, 2048, 6144) > 1 and L.mdx_linear_splits(1024, 4096, 2048) == 0
+    assert L.mdx_linear_silu_supported(8192, 64, 256) == 1 and L.mdx_linear_silu_supported(8193, 64, 256) == 0 and L.mdx_linear_silu_supported(4, 60, 256) == 0
+    li = lambda f: lambda **kw: f(kw.get("x", one), kw.get("xs", 256), kw.get("w", one), kw.get("ws", 256), kw.get("y", one), kw.get("ys", 64),    # noqa: E731
+                                  kw.get("rows", 4), kw.get("n", 64), kw.get("k", 256), null)
+    for call in (li(L.mdx_linear), li(L.mdx_linear_silu)):
+        assert call(x=null) == -1 and call(w=null) == -1 and call(y=null) == -1 and b"null" in L.mdx_last_error()
+        assert call(x=odd) == -2 and call(w=odd) == -2 and call(y=odd) == -2 and call(xs=100) == -2 and call(ws=264 - 1) == -2 and call(xs=248) == -2
+        assert call(xs=1 << 28) == -2 and call(ys=60) == -2 and call(ys=66) == -2 and call(rows=0) == -2 and call(n=68) == -2 and call(k=192) == -2
+    pl = lambda **kw: L.mdx_linear_partials(kw.get("x", one), 6144, one, 6144, kw.get("p", one), kw.get("rows", 32), 2048, 6144, null)             # noqa: E731
+    assert pl(x=null) == -1 and pl(p=null) == -1 and pl(p=odd) == -2 and pl(rows=1537) == -2
