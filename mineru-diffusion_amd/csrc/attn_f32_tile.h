@@ -58,15 +58,20 @@ template <int D> struct Lds {
     static __device__ __forceinline__ float* v_tile(float* lds) { return lds + kTileKeys * kPitchK; }
 };
 
-// One query's row of Q^T for lane (H, r): the elements d = 2 j + H (row may be null: zeros).
+// Each half-wavefront contracts over a half of the head's columns: H over the columns from H * half_width(width) on.
+__device__ __forceinline__ int half_width(int width) { return (width + 7) / 8 * 4; }
+
+// One query's row of Q^T for lane (H, r): its half of the columns (row may be null: zeros, as beyond the head's width).
 template <typename T, int D>
 __device__ __forceinline__ void load_q(float (&q)[D / 2], const T* row, int H, int width) {
+    const int half = half_width(width);
 #pragma unroll
-    for (int m = 0; m < D / 4; ++m) {
+    for (int m = 0; m < D / 8; ++m) {
+        const int col = H * half + 4 * m;
         f32x4 x = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (row && 4 * m < width) x = load4(row + 4 * m);
-        q[2 * m] = H ? x[1] : x[0];
-        q[2 * m + 1] = H ? x[3] : x[2];
+        if (row && 4 * m < half && col < width) x = load4(row + col);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q[4 * m + e] = x[e];
     }
 }
 
@@ -124,18 +129,21 @@ template <int D, typename Visible>
 __device__ __forceinline__ void tile_step(const float* lds, const float (&q)[D / 2], State<D>& st, float c, int width, int lane, Visible visible)
 {
     const int H = lane >> 5, r = lane & 31;
-    // ---- S^T = K Q^T: rows = keys, columns = queries; k-step j covers d = 2 j, 2 j + 1 (half-wavefront H holds d = 2 j + H);
-    //      a 16-byte read of key r's columns 4 m .. 4 m + 3 feeds the k-steps 2 m and 2 m + 1 ----
+    // ---- S^T = K Q^T: rows = keys, columns = queries; k-step j covers the columns j and half + j (the order of a contraction is
+    //      free), so that a lane's 16-byte read of key r feeds four k-steps.  (With the columns 2 j and 2 j + 1 half of every read
+    //      of K and of Q was the other half-wavefront's: us, before / after, paged 1 x 1056 keys 23.9 / 21.3, 2 x 900-2000 36.8 / 32.9,
+    //      4 x 1000-3000 62.0 / 55.2; prompts of 60 tokens 16.8 / 13.7, 300 32.5 / 27.9, 1024 107 / 91, 4000 722 / 687) ----
     f32x16 s;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = 0.f;
-    const float* krow = Lds<D>::k_tile(const_cast<float*>(lds)) + r * Lds<D>::kPitchK;
+    const int half = half_width(width);
+    const float* krow = Lds<D>::k_tile(const_cast<float*>(lds)) + r * Lds<D>::kPitchK + H * half;
 #pragma unroll
-    for (int m = 0; m < D / 4; ++m) {
-        if (4 * m >= width) continue;
+    for (int m = 0; m < D / 8; ++m) {
+        if (4 * m >= half) continue;
         const f32x4 kx = *reinterpret_cast<const f32x4*>(krow + 4 * m);
-        s = __builtin_amdgcn_mfma_f32_32x32x2f32(H ? kx[1] : kx[0], q[2 * m], s, 0, 0, 0);
-        s = __builtin_amdgcn_mfma_f32_32x32x2f32(H ? kx[3] : kx[2], q[2 * m + 1], s, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kx[e], q[4 * m + e], s, 0, 0, 0);
     }
 
     // ---- online softmax over the keys, base 2 ----

@@ -230,8 +230,8 @@ int launch_groups(const PagedWideParams& P, hipStream_t stream)
 // KW: tiles of 32 keys staged side by side, two workgroups' worth of LDS per CU.  Whole contexts for no more heads than there are
 // CUs (a caller without a workspace) are chains of tiles with CUs to spare: a workgroup per head, one per CU with all of its LDS, and
 // twice the wavefronts on the chain with the loads of four tiles in flight (us, two heads / one head per workgroup: d = 128, 4 x 2000
-// keys 231 / 154, 16 x 2000 246 / 173, 1 x 1056 119 / 84; d = 256, 4 x 2000 937 / 560, 16 x 1000 499 / 312).  More heads than CUs are
-// more than one round of such workgroups (24 x 2000, d = 128: 477, with two heads each 260).
+// keys 199 / 132, 16 x 2000 220 / 156, 1 x 1056 100 / 69; d = 256, 4 x 2000 746 / 455, 16 x 1000 408 / 252).  More heads than CUs are
+// more than one round of such workgroups (24 x 2000, d = 128: 315, with two heads each 238).
 template <typename T>
 int launch(const PagedWideParams& P, hipStream_t stream)
 {

@@ -136,8 +136,8 @@ int launch_split(WideParams P, int64_t max_l, hipStream_t stream)
 // workgroups (135 KB of LDS, one per CU) come in one round, or in three if the chain is long enough to pay for those.  Then
 // two, as long as the row groups' unequal chains leave a ragged end (to 16 row tiles per CU); prompts of two tiles have nothing
 // to share once the chip is full, and the fold at the end costs about one tile.  Measured (1 / 2 / 4 wavefronts, 16 query
-// heads, us): 100 tokens 29 / 21 / 15, 500 98 / 61 / 39, 1024 189 / 114 / 84, 2000 362 / 270 / 289, 4096 931 / 733 / 1077,
-// 8192 2680 / 2703 / 4130, 8 x 250 66 / 52 / 81, 16 x 64 18 / 23 / 29, 4 x 2048 838 / 731 / 1153, 4 x 4096 2605 / 2738 / 4358.
+// heads, us): 100 tokens 25 / 16 / 12, 500 85 / 50 / 33, 1024 164 / 94 / 71, 2000 320 / 235 / 244, 4096 855 / 694 / 916,
+// 8192 2539 / 2452 / 3527, 8 x 250 59 / 44 / 64, 16 x 64 15 / 18 / 23, 4 x 2048 788 / 680 / 970, 4 x 4096 2438 / 2519 / 3680.
 template <typename T>
 int launch(const WideParams& P, int64_t max_l, hipStream_t stream)
 {
