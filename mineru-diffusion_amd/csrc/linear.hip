@@ -3,23 +3,9 @@
 // layers/activation.py:7-16).  The result is rounded to bf16, or left as fp32 partial sums over slices of K that the next
 // kernel adds up (residual + RMSNorm; q/k norm + RoPE + store: they read every element once anyway).
 //
-// What bounds it.  A CU takes in at most 70 GB/s from its XCD's L2 (8 wavefronts, loads to LDS, whatever is in flight; 59
-// with 4, 78 with 16), all of them 18 TB/s, so a tile of BM x BN costs (BM + BN) x 128 bytes per step of 64 elements of K
-// against BM x BN x 128 operations, and only tiles of about 256 x 256 are bound by the matrix pipe (1.3 PFLOP/s of them under
-// the board's power limit).  With 32 to 1500 rows the chip's 256 CUs can't all have such a tile; the plan below takes the
-// largest tiles that still give every CU one, cutting K where that makes them larger.  Below 100 rows the read of W from HBM
-// is the floor.  From timing builds at 2048 rows, down projection, tiles of 128 x 128, us: whole 60, loads alone 58, without
-// loads 40, matrix instructions alone 34, LDS reads alone 23.
-//
-// The kernel:
-//  * S steps of x and W rows in LDS (128 bytes of a row per step), filled by loads that pass by the registers
-//    (global_load_lds); the 16-byte chunk c of row r sits at c ^ (r / 2 % 8), so that the 16 rows of a fragment read cover all
-//    banks once.  One barrier per step: behind it the next step is in LDS for everybody and nobody reads this one any more.
-//  * the fragments of the next half step are on their way from LDS while this one is multiplied (two register sets).
-//  * small and middle tiles are shared by two groups of four wavefronts, each taking one half of every step (WK = 2): tiles
-//    of (BM / 2) x (BN / 2) per wavefront need half of the LDS reads that eight tiles of half the size would, and the two
-//    wavefronts of a SIMD cover each other's waits.  The sums meet in LDS at the end.
-//  * W is the first operand, so that a lane ends with four consecutive columns of one row.
+// With 32 to 1500 rows the chip's 256 CUs can't all have a tile that the matrix pipe bounds (linear_tile.h); the plan below takes the
+// largest tiles that still give every CU one, cutting K where that makes them larger.  Below 100 rows the read of W from HBM is
+// the floor.
 //
 // Cold weights, us, here / the library's product (gate/up: with the SiLU kernel), QKV (4096 x 2048), output (2048 x 2048), gate/up
 // (12288 x 2048) and down (2048 x 6144) projection:
@@ -31,185 +17,77 @@
 //   rows  1536  27.2 16.8  81.0  40.8 /  26.2 18.3  94.1 46.7
 //   rows  4096  56.8 33.3 167.6 101.4 /  48.8 31.6 178.6 87.4
 //   rows 16384 225  110   679   296   / 187   94.5 669  268
-// Touching lines of W and x ahead of their loads (as the vocabulary head does), starting the workgroups at different steps, other
-// bands of tiles per XCD and six steps in LDS instead of four change nothing or cost 1 us.
-#include "mdx_common.h"
-#include <atomic>
-#include <utility>
+#include "linear_tile.h"
 
 namespace {
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+using namespace mdx_tile;
+
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-typedef __attribute__((address_space(3))) char lds_char;
 
 struct LinearParams {
-    const __bf16* x; const __bf16* w;
+    Operands in;
     __bf16* y; float* partials;                    // y: [M, N]; partials: [splits, M, N]
-    int64_t x_stride, w_stride, y_stride;          // elements between rows
-    int M, N, K;                                   // N: columns of the result (SiLU: W has 2 N rows, gate then up)
-    int m_tiles, n_tiles, splits;
+    int64_t y_stride;                              // elements between rows
+    int K, m_tiles, n_tiles, splits;
 };
 
 enum Form { kRounded = 0, kPartials = 1, kSilu = 2 };
 
-constexpr int kStepK = 64, kRowBytes = 2 * kStepK; // one step of K: 128 bytes of every row
-constexpr int kBand = 8;                           // row tiles that share a column tile of W one after the other
-
-template <typename F, int... J>
-__device__ __forceinline__ void for_each(F f, std::integer_sequence<int, J...>) { (f(std::integral_constant<int, J>{}), ...); }
-
-// This wavefront's loads up to the newest N and all of its LDS reads are done, then everybody's.
-template <int N> __device__ __forceinline__ void wait_loads_and_meet() {
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory");
-    __builtin_amdgcn_sched_barrier(0);
-}
-
-template <int BM, int BN, int WM, int WN, int WK, int S, int FORM>
-__global__ __launch_bounds__(64 * WM * WN * WK, WM * WN * WK / 4) void linear_kernel(const LinearParams A)
+template <typename T, int FORM>
+__global__ __launch_bounds__(T::kThreads, T::kWaves / 4) void linear_kernel(const LinearParams A)
 {
     extern __shared__ __attribute__((aligned(1024))) char lds[];
-    constexpr int kWaves = WM * WN * WK;
-    constexpr int TM = BM / (16 * WM), TN = BN / (16 * WN);  // a wavefront's share, in matrix tiles of 16 x 16
-    constexpr int kStage = (BM + BN) * kRowBytes, kLoads = (BM + BN) / 8 / kWaves;
-    static_assert(BM % (8 * kWaves) == 0 && BN % (8 * kWaves) == 0 && (WK == 1 || (WK == 2 && TM % 2 == 0)), "tile shape");
-    static_assert((FORM != kSilu || TN % 2 == 0) && S % 2 == 0, "pairs of gate and up tiles, pairs of steps");
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int l16 = lane & 15, g = lane >> 4;
-    const int wm = wave % WM, wn = wave / WM % WN, wk = wave / (WM * WN);
-
-    // Consecutive workgroups go to the eight XCDs in turn; each XCD takes a run of the tiles in the order (slice of K, band of
-    // row tiles, column tile, row tile): what it has in flight together shares its rows of x and of W in its L2.
-    const int xcd = blockIdx.x & 7, per_xcd = gridDim.x >> 3, more = gridDim.x & 7;
-    int at = xcd * per_xcd + min(xcd, more) + (int)(blockIdx.x >> 3);
-    const int per_split = A.m_tiles * A.n_tiles, split = at / per_split;
-    at -= split * per_split;
-    const int m_first = at / (kBand * A.n_tiles) * kBand, m_band = min(kBand, A.m_tiles - m_first);
-    at -= m_first * A.n_tiles;
-    constexpr int kCols = FORM == kSilu ? BN / 2 : BN;      // columns of the result
-    const int m0 = (m_first + at % m_band) * BM, n0 = at / m_band * kCols;
-    const int k_split = A.K / A.splits, n_steps = k_split / kStepK;         // (the host's choice: an even number, at least S)
-
-    // Load i of this wavefront fills 8 rows of the tile, x rows first, then rows of W (SiLU: 16 gate rows, the 16 up rows of
-    // the same columns, and so on).  Rows beyond the last are the last one again; their products are not stored.
-    const unsigned lds0 = (unsigned)(uintptr_t)(lds_char*)lds;
-    const char* base[kLoads];                               // the first of the 8 rows, at this slice of K
-    unsigned offset[kLoads];                                // this lane's row and chunk from there
-#pragma unroll
-    for (int i = 0; i < kLoads; ++i) {
-        const int r0 = 8 * (wave + kWaves * i), r = lane >> 3, chunk = (lane & 7) ^ (((r0 + r) >> 1) & 7);
-        const bool of_x = r0 < BM;                          // (known when compiled: BM is a multiple of 8 kWaves)
-        const int b = r0 - BM;
-        const int first = of_x ? m0 + r0 : FORM == kSilu ? n0 + (b >> 5) * 16 + (b & 15) : n0 + b, last = (of_x ? A.M : A.N) - 1;
-        const int64_t stride = (of_x ? A.x_stride : A.w_stride) * 2;
-        const int64_t up = FORM == kSilu && !of_x && ((b >> 4) & 1) ? A.N : 0;
-        base[i] = reinterpret_cast<const char*>((of_x ? A.x : A.w) + split * k_split) + (min(first, last) + up) * stride;
-        offset[i] = (unsigned)(min(first + r, last) - min(first, last)) * (unsigned)stride + chunk * 16;
-    }
-    int64_t k_bytes = 0;                                    // where the step to ask for next begins
-    auto issue = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < kLoads; ++i)
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                         :: "s"(lds0 + buf * kStage + (wave + kWaves * i) * 1024), "v"(offset[i]), "s"(base[i] + k_bytes) : "memory");
-        k_bytes += kRowBytes;
-    };
-    const char* xr = lds + (wm * (BM / WM) + l16) * kRowBytes;
-    const char* wr = lds + (BM + wn * (BN / WN) + l16) * kRowBytes;
-    bf16x8 fx[2][TM], fw[2][TN];
-    auto read = [&](int set, int buf, int half) {            // a half of a step: 32 elements of K
-        const int pos = ((half * 4 + g) ^ ((l16 >> 1) & 7)) * 16 + buf * kStage;
-#pragma unroll
-        for (int i = 0; i < TM; ++i) fx[set][i] = *reinterpret_cast<const bf16x8*>(xr + pos + i * 16 * kRowBytes);
-#pragma unroll
-        for (int i = 0; i < TN; ++i) fw[set][i] = *reinterpret_cast<const bf16x8*>(wr + pos + i * 16 * kRowBytes);
-    };
-    f32x4 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    auto multiply = [&](int half) {
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int i = 0; i < TM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[half][j], fx[half][i], acc[i][j], 0, 0, 0);
-    };
-
-#pragma unroll
-    for (int s = 0; s < S; ++s) issue(s);
-    wait_loads_and_meet<(S - 1) * kLoads>();
-    read(0, 0, WK == 2 ? wk : 0);
-    int buf = 0;                                             // t % S
-    auto next = [&](int b) { return b + 1 == S ? 0 : b + 1; };
-    for (int t = 0; t < n_steps - S; t += 2) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            if constexpr (WK == 1) { read(1, buf, 1); multiply(0); }
-            wait_loads_and_meet<(S - 2) * kLoads>();
-            issue(buf);
-            buf = next(buf);
-            if constexpr (WK == 1) { read(0, buf, 0); multiply(1); }
-            else { read(1 - h, buf, wk); multiply(h); }
-        }
-    }
-    // the last S steps: nothing more to load
-    for_each([&](auto step) {
-        constexpr int J = decltype(step)::value;
-        if constexpr (WK == 1) { read(1, buf, 1); multiply(0); }
-        if constexpr (J + 1 < S) {
-            wait_loads_and_meet<(S - 2 - J) * kLoads>();
-            buf = next(buf);
-            if constexpr (WK == 1) read(0, buf, 0); else read(1 - (J & 1), buf, wk);
-        }
-        if constexpr (WK == 1) multiply(1); else multiply(J & 1);
-    }, std::make_integer_sequence<int, S>{});
+    constexpr int TM = T::TM, TN = T::TN;
+    const T tile;
+    const Place at = place_of(A.m_tiles, A.n_tiles);
+    const int m0 = at.m * T::BM, n0 = at.n * T::kCols, k_split = A.K / A.splits;
+    typename T::Sums acc;
+    tile.product(A.in, m0, n0, (int64_t)at.split * k_split, k_split / kStepK, lds, acc);
 
     // where two wavefronts share a tile, each holds the sums over its halves of the steps, and finishes half of the rows
-    constexpr int H = TM / WK;
+    constexpr int H = TM / T::WK;
     f32x4* sums = reinterpret_cast<f32x4*>(lds);             // [wave][H][TN][lane]
-    if constexpr (WK == 2) {
+    if constexpr (T::WK == 2) {
         wait_loads_and_meet<0>();
-        f32x4* mine = sums + wave * H * TN * 64 + lane;
+        f32x4* mine = sums + tile.wave * H * TN * 64 + tile.lane;
 #pragma unroll
         for (int i = 0; i < H; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) mine[(i * TN + j) * 64] = wk ? acc[i][j] : acc[H + i][j];
+            for (int j = 0; j < TN; ++j) mine[(i * TN + j) * 64] = tile.wk ? acc[i][j] : acc[H + i][j];
         __syncthreads();
     }
-    const f32x4* theirs = sums + (wave ^ (WM * WN)) * H * TN * 64 + lane;
-    const int mb = m0 + wm * (BM / WM) + (WK == 2 ? wk * H * 16 : 0) + l16;
+    const f32x4* theirs = sums + (tile.wave ^ (T::WM * T::WN)) * H * TN * 64 + tile.lane;
+    const int mb = m0 + tile.wm * (T::BM / T::WM) + (T::WK == 2 ? tile.wk * H * 16 : 0) + tile.l16;
 #pragma unroll
     for (int i = 0; i < H; ++i) {
         const int m = mb + i * 16;
         f32x4 sum[TN];
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-            if constexpr (WK == 2) sum[j] = (wk ? acc[H + i][j] : acc[i][j]) + theirs[(i * TN + j) * 64];
+            if constexpr (T::WK == 2) sum[j] = (tile.wk ? acc[H + i][j] : acc[i][j]) + theirs[(i * TN + j) * 64];
             else sum[j] = acc[i][j];
         }
-        if (m >= A.M) continue;
+        if (m >= A.in.M) continue;
         if (FORM == kSilu) {
 #pragma unroll
             for (int j = 0; j < TN; j += 2) {
-                const int n = n0 + (wn * TN + j) * 8 + 4 * g;
+                const int n = n0 + (tile.wn * TN + j) * 8 + 4 * tile.g;
                 bf16x4 out;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const float gate = (float)(__bf16)sum[j][e];      // the projection's own rounding, then SiLU's
                     out[e] = (__bf16)((float)(__bf16)(gate / (1.0f + __expf(-gate))) * (float)(__bf16)sum[j + 1][e]);
                 }
-                if (n < A.N) *reinterpret_cast<bf16x4*>(A.y + (int64_t)m * A.y_stride + n) = out;
+                if (n < A.in.N) *reinterpret_cast<bf16x4*>(A.y + (int64_t)m * A.y_stride + n) = out;
             }
         } else {
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
-                const int n = n0 + (wn * TN + j) * 16 + 4 * g;
-                if (n >= A.N) continue;
+                const int n = n0 + (tile.wn * TN + j) * 16 + 4 * tile.g;
+                if (n >= A.in.N) continue;
                 if (FORM == kPartials) {
-                    *reinterpret_cast<f32x4*>(A.partials + ((int64_t)split * A.M + m) * A.N + n) = sum[j];
+                    *reinterpret_cast<f32x4*>(A.partials + ((int64_t)at.split * A.in.M + m) * A.in.N + n) = sum[j];
                 } else {
                     bf16x4 out;
 #pragma unroll
@@ -221,58 +99,54 @@ __global__ __launch_bounds__(64 * WM * WN * WK, WM * WN * WK / 4) void linear_ke
     }
 }
 
-template <int BM, int BN, int WM, int WN, int WK, int S, int FORM>
+template <int BM, int BN, int WM, int WN, int WK, int S, int SX, int FORM>
 int launch(LinearParams A, hipStream_t stream)
 {
-    constexpr int kTiles = S * (BM + BN) * kRowBytes, kSums = WK == 2 ? BM * BN * 4 : 0, kLdsBytes = kTiles > kSums ? kTiles : kSums;
+    typedef Tile<BM, BN, WM, WN, WK, S, SX, FORM == kSilu> T;
+    constexpr int kSums = WK == 2 ? BM * BN * 4 : 0, kLdsBytes = T::kStepsBytes > kSums ? T::kStepsBytes : kSums;
     static_assert(kLdsBytes <= 160 * 1024, "LDS");
-    if (kLdsBytes > 65536) {
-        // the kernel's LDS limit is raised once per device
-        static std::atomic<bool> raised[64];
-        int device = 0;
-        hipError_t e = hipGetDevice(&device);
-        MDX_REQUIRE(e == hipSuccess && device >= 0 && device < 64, MDX_ELAUNCH, "linear: no current device (%s)", hipGetErrorString(e));
-        if (!raised[device].load(std::memory_order_acquire)) {
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(linear_kernel<BM, BN, WM, WN, WK, S, FORM>), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
-            MDX_REQUIRE(e == hipSuccess, MDX_ELAUNCH, "linear: cannot reserve %d bytes of LDS (%s)", kLdsBytes, hipGetErrorString(e));
-            raised[device].store(true, std::memory_order_release);
-        }
-    }
-    constexpr int kCols = FORM == kSilu ? BN / 2 : BN;
-    A.m_tiles = (A.M + BM - 1) / BM;
-    A.n_tiles = (A.N + kCols - 1) / kCols;
+    static std::atomic<bool> raised[64];
+    const int rc = reserve_lds(reinterpret_cast<const void*>(linear_kernel<T, FORM>), kLdsBytes, raised, "linear");
+    if (rc != MDX_OK) return rc;
+    A.m_tiles = (A.in.M + BM - 1) / BM;
+    A.n_tiles = (A.in.N + T::kCols - 1) / T::kCols;
     const int64_t grid = (int64_t)A.m_tiles * A.n_tiles * A.splits;
     MDX_REQUIRE(grid < ((int64_t)1 << 31), MDX_EUNSUPPORTED, "linear: %lld tiles", (long long)grid);
-    linear_kernel<BM, BN, WM, WN, WK, S, FORM><<<(unsigned)grid, 64 * WM * WN * WK, kLdsBytes, stream>>>(A);
+    linear_kernel<T, FORM><<<(unsigned)grid, T::kThreads, kLdsBytes, stream>>>(A);
     return mdx::check_launch("linear");
 }
 
 // The tiles there are, and what a round of them costs: a step of K and what stands before and behind the steps, us, fitted to
 // 4900 timings (four projections of the decoder, 16 to 8192 rows, every tile, 1 to 24 slices of K).
-struct Tile {
-    int bm, bn, stages;
+struct TileCost {
+    int bm, bn, least_steps, steps_multiple;                // steps of 64 elements of K: at least, and a multiple of
     float step, around;
     int (*rounded)(LinearParams, hipStream_t);
     int (*partials)(LinearParams, hipStream_t);             // none for the tiles that only many rows fill
     int (*silu)(LinearParams, hipStream_t);
 };
-#define MDX_TILE(BM, BN, WM, WN, WK, S) launch<BM, BN, WM, WN, WK, S, kRounded>, launch<BM, BN, WM, WN, WK, S, kPartials>, launch<BM, BN, WM, WN, WK, S, kSilu>
-#define MDX_LARGE_TILE(BM, BN, WM, WN, WK, S) launch<BM, BN, WM, WN, WK, S, kRounded>, nullptr, launch<BM, BN, WM, WN, WK, S, kSilu>
-const Tile kTileTable[] = {
-    {32, 64, 4, 0.150f, 0.2f, MDX_TILE(32, 64, 2, 2, 1, 4)},
-    {64, 64, 4, 0.200f, 0.5f, MDX_TILE(64, 64, 2, 2, 2, 4)},
-    {128, 64, 4, 0.302f, 1.3f, MDX_TILE(128, 64, 2, 2, 2, 4)},
-    {192, 64, 4, 0.395f, 1.6f, MDX_TILE(192, 64, 2, 2, 2, 4)},
-    {128, 128, 4, 0.470f, 1.8f, MDX_TILE(128, 128, 2, 2, 2, 4)},
-    {192, 128, 4, 0.606f, 2.6f, MDX_TILE(192, 128, 2, 2, 2, 4)},
-    {128, 192, 4, 0.677f, 1.5f, MDX_TILE(128, 192, 4, 2, 1, 4)},
-    {256, 192, 2, 1.166f, 1.2f, MDX_LARGE_TILE(256, 192, 4, 2, 1, 2)},
-    {256, 256, 2, 1.432f, 1.3f, MDX_LARGE_TILE(256, 256, 2, 4, 1, 2)},
+template <int BM, int BN, int WM, int WN, int WK, int S, int SX, bool PARTIALS>
+constexpr TileCost tile(float step, float around) {
+    typedef Tile<BM, BN, WM, WN, WK, S, SX, false> T;
+    if constexpr (PARTIALS) return TileCost{BM, BN, T::kLeastSteps, T::kStepsMultiple, step, around, launch<BM, BN, WM, WN, WK, S, SX, kRounded>,
+                                            launch<BM, BN, WM, WN, WK, S, SX, kPartials>, launch<BM, BN, WM, WN, WK, S, SX, kSilu>};
+    else return TileCost{BM, BN, T::kLeastSteps, T::kStepsMultiple, step, around, launch<BM, BN, WM, WN, WK, S, SX, kRounded>, nullptr,
+                         launch<BM, BN, WM, WN, WK, S, SX, kSilu>};
+}
+const TileCost kTiles[] = {
+    tile<32, 64, 2, 2, 1, 4, 4, true>(0.150f, 0.2f),
+    tile<64, 64, 2, 2, 2, 4, 4, true>(0.200f, 0.5f),
+    tile<128, 64, 2, 2, 2, 4, 4, true>(0.302f, 1.3f),
+    tile<192, 64, 2, 2, 2, 4, 4, true>(0.395f, 1.6f),
+    tile<128, 128, 2, 2, 2, 4, 4, true>(0.470f, 1.8f),
+    tile<192, 128, 2, 2, 2, 4, 4, true>(0.606f, 2.6f),
+    tile<128, 192, 4, 2, 1, 4, 4, true>(0.677f, 1.5f),
+    tile<192, 192, 4, 2, 1, 3, 3, false>(0.900f, 2.0f),
+    tile<256, 192, 4, 2, 1, 2, 3, false>(1.140f, 1.2f),
+    tile<256, 256, 4, 2, 1, 2, 3, false>(1.410f, 1.3f),
 };
-#undef MDX_TILE
-#undef MDX_LARGE_TILE
 
-struct Plan { const Tile* tile; int splits; };
+struct Plan { const TileCost* tile; int splits; };
 
 // The cheapest tile and number of slices by the costs above, in rounds of one workgroup per CU (the small tiles' second one
 // per CU is worth little: they share its intake).  Partial sums cost their writing and the next kernel's reading, 0.35 us per
@@ -284,10 +158,10 @@ Plan plan_of(int64_t rows, int64_t n, int64_t k, bool rounded, bool partials, bo
     double least = 0;
     const int cus = mdx::compute_units();
     const double mb = (double)rows * (double)n * 4e-6;
-    for (const Tile& t : kTileTable) {
+    for (const TileCost& t : kTiles) {
         const int64_t cols = silu ? t.bn / 2 : t.bn, tiles = ((rows + t.bm - 1) / t.bm) * ((n + cols - 1) / cols);
-        for (int64_t s = 1; s <= k / (kStepK * t.stages) && s <= 32; ++s) {
-            if (k % (2 * kStepK * s) != 0 || (s > 1 && !partials)) continue;      // whole pairs of steps
+        for (int64_t s = 1; s <= k / (kStepK * t.least_steps) && s <= 32; ++s) {
+            if (k % (kStepK * t.steps_multiple * s) != 0 || (s > 1 && !partials)) continue;
             const double steps = (double)(k / kStepK / s), rounds = (double)((tiles * s + cus - 1) / cus);
             for (int form = 0; form < 2; ++form) {                                  // 0: rounded or SiLU, 1: partial sums
                 if (form == 0 ? (s > 1 || !(rounded || silu)) : (!partials || !t.partials)) continue;
@@ -319,9 +193,8 @@ int check_linear(const char* what, const void* x, int64_t x_row_stride, const vo
 LinearParams params_of(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride, int64_t rows, int64_t n, int64_t k)
 {
     LinearParams A{};
-    A.x = (const __bf16*)x; A.w = (const __bf16*)w;
-    A.x_stride = x_row_stride; A.w_stride = w_row_stride;
-    A.M = (int)rows; A.N = (int)n; A.K = (int)k; A.splits = 1;
+    A.in = Operands{(const __bf16*)x, (const __bf16*)w, x_row_stride, w_row_stride, (int)rows, (int)n};
+    A.K = (int)k; A.splits = 1;
     return A;
 }
 

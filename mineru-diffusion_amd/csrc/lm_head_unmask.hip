@@ -7,29 +7,106 @@
 // (engines/nano_dvlm/nanovllm/layers/embed_head.py:61-67) followed by Sampler.prepare's softmax
 // confidence and argmax without noise (layers/sampler.py:11-22).
 //
-// A workgroup computes a 256-vocab x 256-row tile over the whole hidden dimension (the hand-scheduled core
-// of lm_head_core.inc) and leaves two 16-byte records per x row, one per 128-vocab slice; a second, small
-// kernel folds a row's records (vocab / 128 of them) into x0 / x0_p.  Launch order: the row tiles of one
-// vocab tile sit 8 workgroups apart, so that the dispatcher, which deals consecutive workgroups round-robin
-// to the 8 XCDs, puts them on the same XCD next to each other in time and its L2 fetches that tile of W from
-// HBM once.
+// A workgroup computes a tile of 256 x 256, 128 x 256 or 192 x 192 (x rows by vocabulary rows) over the whole hidden dimension
+// (linear_tile.h) and leaves one 16-byte record per x row; a second, small kernel folds a row's records (about vocab / 256 of them) into x0 /
+// x0_p.  The matrix pipe bounds it, under the board's power limit.
 #include "lm_head.h"
-#include <atomic>
+#include "linear_tile.h"
 
 namespace {
 
 using namespace mdx_head;
+using namespace mdx_tile;
 
+constexpr int kFoldThreads = 256;
+constexpr float kClamp = -1.0e30f;
+
+struct Best { float m, s; int idx; };                     // max logit, sum of exp2((x - m) c), first index of the max
+
+// (0 where a lane saw nothing: its stand-in maximum must not meet an infinite factor)
+__device__ __forceinline__ Best merge(const Best& a, const Best& b, float c) {
+    const float A = fmaxf(a.m, kClamp), B = fmaxf(b.m, kClamp), M = fmaxf(A, B);
+    Best r;
+    r.m = fmaxf(a.m, b.m);
+    r.s = a.s * __builtin_amdgcn_exp2f((A - M) * c) + b.s * __builtin_amdgcn_exp2f((B - M) * c);
+    r.idx = a.m > b.m ? a.idx : b.m > a.m ? b.idx : min(a.idx, b.idx);
+    return r;
+}
+
+__device__ __forceinline__ float max3(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
+template <typename T>
+__global__ __launch_bounds__(T::kThreads, T::kWaves / 4) void lm_head_confidence_kernel(const LmHeadParams P)
+{
+    extern __shared__ __attribute__((aligned(1024))) char lds[];
+    const T tile;
+    const Place at = place_of(P.n_row_tiles, P.n_vocab_tiles);
+    const int xr0 = at.m * T::BM, v0 = at.n * T::BN;
+    const int row0 = tile.wm * (T::BM / T::WM) + tile.l16;        // this lane's first x row in the tile
+    float c[T::TM];
+#pragma unroll
+    for (int i = 0; i < T::TM; ++i) c[i] = row_scale(P, xr0 + row0 + 16 * i);
+    typename T::Sums acc;
+    tile.product(Operands{P.x, P.w, P.x_stride, P.w_stride, P.rows, P.vocab}, xr0, v0, 0, P.hidden / kStepK, lds, acc);
+
+    wait_loads_and_meet<0>();                              // the tile's steps have been read by everybody
+    Best* parts = reinterpret_cast<Best*>(lds);            // [WN][BM]
+    const int v_lane = v0 + tile.wn * (T::BN / T::WN) + 4 * tile.g;                 // vocabulary index of this lane's first logit
+    const bool edge = v0 + T::BN > P.vocab;
+#pragma unroll
+    for (int i = 0; i < T::TM; ++i) {
+        // the lane's logits in ascending vocabulary order, rounded to the projection's bf16; beyond the vocabulary: -inf
+        float v[4 * T::TN];
+#pragma unroll
+        for (int j = 0; j < T::TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[4 * j + e] = (float)(__bf16)acc[i][j][e];
+                if (edge && v_lane + 16 * j + e >= P.vocab) v[4 * j + e] = -INFINITY;
+            }
+        float m = v[0];
+#pragma unroll
+        for (int k = 1; k < 4 * T::TN; k += 2) m = max3(m, v[k], v[k + 1 < 4 * T::TN ? k + 1 : k]);
+        int first = 0;
+#pragma unroll
+        for (int k = 4 * T::TN - 1; k >= 0; --k) first = v[k] == m ? k : first;
+        // one FMA per exponent: the product m c is rounded once and its error taken out of the sum afterwards
+        const float ms = fmaxf(m, kClamp), h = ms * c[i];
+        float s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < 4 * T::TN; ++k) s[k & 3] += __builtin_amdgcn_exp2f(__builtin_fmaf(v[k], c[i], -h));
+        float sum = ((s[0] + s[1]) + (s[2] + s[3])) * __builtin_amdgcn_exp2f(-__builtin_fmaf(ms, c[i], -h));
+        if (!(m > -INFINITY)) sum = 0.f;                   // all of it beyond the vocabulary: 0, not 0 x the correction's infinity
+        Best b = Best{m, sum, v_lane + 16 * (first >> 2) + (first & 3)};
+#pragma unroll
+        for (int off = 16; off <= 32; off <<= 1)
+            b = merge(b, Best{__shfl_xor(b.m, off), __shfl_xor(b.s, off), __shfl_xor(b.idx, off)}, c[i]);
+        if (tile.g == 0) parts[tile.wn * T::BM + row0 + 16 * i] = b;
+    }
+    __syncthreads();
+    const int r = threadIdx.x, row = xr0 + r;
+    if (r >= T::BM || row >= P.rows) return;
+    const float cr = row_scale(P, row);
+    Best b = parts[r];
+#pragma unroll
+    for (int w = 1; w < T::WN; ++w) b = merge(b, parts[w * T::BM + r], cr);
+    P.records[(int64_t)row * P.n_slices + at.n] = Record{b.m, b.s, b.idx, 0};
+}
+
+// ---- 128 columns: two steps, less than the tiles above want in flight.  Tiles of 256 x 256 on the generated core of lm_head_core.inc
+//      (one wavefront per SIMD; over 2048 columns 200 us up to 256 rows, 306-314 up to 512, 577 at 1024), two records per row and tile. ----
 #include "lm_head_core.inc"
 
 constexpr int kThreads = 256;
 constexpr int kTile = 256;                     // vocab rows and x rows per workgroup
 constexpr int kSlice = 128;                    // vocab rows per record (one wavefront's share)
 constexpr int kLdsBytes = 2 * 2 * kTile * 128; // two stages of (W tile + x tile), 128-byte rows
-constexpr float kClamp = -1.0e30f;
 
 // 32-bit LDS byte address of a pointer into shared memory (what ds_* instructions and M0 take).
-typedef __attribute__((address_space(3))) char lds_char;
 __device__ __forceinline__ unsigned lds_address(const void* p) { return (unsigned)(uintptr_t)(const lds_char*)p; }
 
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
@@ -39,7 +116,7 @@ __device__ __forceinline__ const void* uniform(const void* p) {
     return (const void*)(((uint64_t)hi << 32) | lo);
 }
 
-__global__ __launch_bounds__(kThreads, 1) void lm_head_confidence_kernel(const LmHeadParams P)
+__global__ __launch_bounds__(kThreads, 1) void lm_head_two_steps_kernel(const LmHeadParams P)
 {
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -89,9 +166,9 @@ __global__ __launch_bounds__(kThreads, 1) void lm_head_confidence_kernel(const L
 }
 
 // One wavefront per x row: folds the row's records (ascending vocabulary slices) into token and confidence.
-__global__ __launch_bounds__(kThreads) void lm_head_finalize_kernel(const LmHeadParams P)
+__global__ __launch_bounds__(kFoldThreads) void lm_head_finalize_kernel(const LmHeadParams P)
 {
-    const int row = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
+    const int row = blockIdx.x * (kFoldThreads / 64) + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (row >= P.rows) return;
     const float c = row_scale(P, row);
@@ -131,23 +208,51 @@ __global__ __launch_bounds__(kThreads) void lm_head_finalize_kernel(const LmHead
     }
 }
 
-int slices_of(int64_t vocab) { return (int)((vocab + kTile - 1) / kTile) * (kTile / kSlice); }
+// Records per row that the workspace has room for: the form for few rows and every tile below stay under it.
+int slices_of(int64_t vocab) { return (int)((vocab + 255) / 256) * 2; }
 
-int launch_tiles(const LmHeadParams& P, hipStream_t stream)
+template <int BM, int BN, int S, int SX>
+int launch_tiles(LmHeadParams& P, hipStream_t stream)
 {
-    // the kernel's LDS limit is raised once per device
-    static std::atomic<bool> lds_limit_raised[64];
-    int device = 0;
-    hipError_t e = hipGetDevice(&device);
-    MDX_REQUIRE(e == hipSuccess && device >= 0 && device < 64, MDX_ELAUNCH, "lm_head_confidence: no current device (%s)", hipGetErrorString(e));
-    if (!lds_limit_raised[device].load(std::memory_order_acquire)) {
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(lm_head_confidence_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
-        MDX_REQUIRE(e == hipSuccess, MDX_ELAUNCH, "lm_head_confidence: cannot reserve %d bytes of LDS (%s)", kLdsBytes, hipGetErrorString(e));
-        lds_limit_raised[device].store(true, std::memory_order_release);
-    }
-    const int64_t grid = (int64_t)((P.n_vocab_tiles + 7) / 8) * 8 * P.n_row_tiles;
-    lm_head_confidence_kernel<<<(unsigned)grid, kThreads, kLdsBytes, stream>>>(P);
+    typedef Tile<BM, BN, 4, 2, 1, S, SX, false> T;
+    static_assert(T::kStepsBytes <= 160 * 1024 && T::WN * BM * (int)sizeof(Best) <= T::kStepsBytes && BM <= T::kThreads, "LDS, a thread per row");
+    static std::atomic<bool> raised[64];
+    const int rc = reserve_lds(reinterpret_cast<const void*>(lm_head_confidence_kernel<T>), T::kStepsBytes, raised, "lm_head_confidence");
+    if (rc != MDX_OK) return rc;
+    P.n_row_tiles = (P.rows + BM - 1) / BM;
+    P.n_vocab_tiles = P.n_slices = (P.vocab + BN - 1) / BN;
+    lm_head_confidence_kernel<T><<<(unsigned)(P.n_row_tiles * P.n_vocab_tiles), T::kThreads, T::kStepsBytes, stream>>>(P);
     return mdx::check_launch("lm_head_confidence");
+}
+
+int launch_two_steps(LmHeadParams& P, hipStream_t stream)
+{
+    static std::atomic<bool> raised[64];
+    const int rc = reserve_lds(reinterpret_cast<const void*>(lm_head_two_steps_kernel), kLdsBytes, raised, "lm_head_confidence");
+    if (rc != MDX_OK) return rc;
+    P.n_row_tiles = (P.rows + kTile - 1) / kTile;
+    P.n_vocab_tiles = (P.vocab + kTile - 1) / kTile;
+    P.n_slices = slices_of(P.vocab);
+    const int64_t grid = (int64_t)((P.n_vocab_tiles + 7) / 8) * 8 * P.n_row_tiles;
+    lm_head_two_steps_kernel<<<(unsigned)grid, kThreads, kLdsBytes, stream>>>(P);
+    return mdx::check_launch("lm_head_confidence");
+}
+
+// Which tile: rounds of one workgroup per CU times what a round takes (us over 2048 columns: 256 x 256 56, 128 x 256 and 192 x 192
+// 34.5).  151 936 entries, us, 256 x 256 / 128 x 256 / 192 x 192: 129 rows 197 / 182 / 177, 192 192 / 188 / 184, 256 196 / 201 / 238,
+// 320 286 / 250 / 257, 500 300 / 348 / 345, 768 421 / 473 / 468.  The call, generated core / these tiles: 129 rows 212 / 187, 192 206 / 186,
+// 256 212 / 198, 320 296 / 261, 500 307 / 299, 640 438 / 412, 1024 577 / 567, 4096 2168 / 2092.
+int launch_product(LmHeadParams& P, hipStream_t stream)
+{
+    if (P.hidden < 3 * kStepK) return launch_two_steps(P, stream);
+    const int cus = mdx::compute_units();
+    auto cost = [&](int bm, int bn, float round) {
+        const int64_t tiles = (int64_t)((P.rows + bm - 1) / bm) * ((P.vocab + bn - 1) / bn);
+        return (float)((tiles + cus - 1) / cus) * round;
+    };
+    const float large = cost(256, 256, 56.f), half = cost(128, 256, 34.5f), square = cost(192, 192, 34.5f);
+    if (half < large && half <= square) return launch_tiles<128, 256, 3, 3>(P, stream);
+    return square < large ? launch_tiles<192, 192, 3, 3>(P, stream) : launch_tiles<256, 256, 2, 3>(P, stream);
 }
 
 }  // namespace
@@ -188,15 +293,13 @@ extern "C" int mdx_lm_head_confidence(const void* x, int64_t x_row_stride, const
     P.x = (const __bf16*)x; P.w = (const __bf16*)w; P.x_stride = x_row_stride; P.w_stride = w_row_stride;
     P.temperatures = temperatures; P.rows_per_temp = rows_per_temp; P.row_ids = row_ids;
     P.rows = (int)rows; P.vocab = (int)vocab; P.hidden = (int)hidden;
-    P.n_row_tiles = (int)((rows + kTile - 1) / kTile);
-    P.n_vocab_tiles = (int)((vocab + kTile - 1) / kTile);
-    P.n_slices = slices_of(vocab);
+    P.n_row_tiles = P.n_vocab_tiles = P.n_slices = 0;      // with the launch
     P.records = static_cast<Record*>(workspace);
     P.x0 = x0; P.x0_p = x0_p;
 
     // up to 128 rows the tiles of 256 rows are mostly padding
-    const int rc = few_rows_covered(rows, hidden) ? launch_few_rows(P, stream) : launch_tiles(P, stream);
+    const int rc = few_rows_covered(rows, hidden) ? launch_few_rows(P, stream) : launch_product(P, stream);
     if (rc != MDX_OK) return rc;
-    lm_head_finalize_kernel<<<(unsigned)((rows + kThreads / 64 - 1) / (kThreads / 64)), kThreads, 0, stream>>>(P);
+    lm_head_finalize_kernel<<<(unsigned)((rows + kFoldThreads / 64 - 1) / (kFoldThreads / 64)), kFoldThreads, 0, stream>>>(P);
     return mdx::check_launch("lm_head_finalize");
 }

@@ -133,3 +133,18 @@ def test_lm_head_confidence_of_few_rows(dev, rows, vocab, hidden):
     torch.cuda.synchronize()
     ex0, ep, logits = _reference(x, w, temps)
     _check(x0, p, ex0, ep, logits, temps)
+
+
+@pytest.mark.parametrize("rows,vocab,hidden", [(150, 100003, 256), (250, 100003, 256), (320, 100003, 256), (129, 191, 384), (385, 193, 256), (513, 257, 384), (200, 600, 128)])
+def test_lm_head_confidence_tiles(dev, rows, vocab, hidden):
+    """Each of the tiles for more than 128 rows (192 x 192, 256 x 256, 128 x 256 by the rounds they come to), last tiles of few rows
+    and few entries, the fewest steps of each and the form for 128 columns, with temperatures."""
+    import mdx
+    g = torch.Generator().manual_seed(rows + vocab)
+    x = torch.randn(rows, hidden, generator=g).bfloat16()
+    w = (torch.randn(vocab, hidden, generator=g) * (3.0 / hidden ** 0.5)).bfloat16()
+    temps = 0.5 + torch.rand(rows, generator=g)
+    x0, p = mdx.lm_head_confidence(x.to(dev), w.to(dev), temps.to(dev))
+    torch.cuda.synchronize()
+    ex0, ep, logits = _reference(x, w, temps)
+    _check(x0, p, ex0, ep, logits, temps)
