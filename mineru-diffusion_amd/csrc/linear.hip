@@ -7,16 +7,16 @@
 // largest tiles that still give every CU one, cutting K where that makes them larger.  Below 100 rows the read of W from HBM is
 // the floor.
 //
-// Cold weights, us, here / the library's product (gate/up: with the SiLU kernel), QKV (4096 x 2048), output (2048 x 2048), gate/up
+// Weights from HBM, us, here / the library's product (gate/up: with the SiLU kernel), QKV (4096 x 2048), output (2048 x 2048), gate/up
 // (12288 x 2048) and down (2048 x 6144) projection:
-//   rows    32   4.8  3.8  12.4   7.1 /  11.7  8.4  18.8 16.6      (a kernel with W straight in registers: 6.5  4.6 15.2  8.6)
-//   rows   128   6.9  5.0  18.4  10.8 /  12.1  8.6  22.0 17.8      (                                      10.0  6.8 23.7 12.5)
-//   rows   256   9.0  6.3  24.0  15.1 /  11.3  9.7  31.1 22.5
-//   rows   512  12.5  8.6  28.7  20.7 /  15.2 11.1  35.9 27.7
-//   rows  1024  19.3 12.7  46.1  33.2 /  20.9 15.1  54.4 40.6
-//   rows  1536  27.2 16.8  81.0  40.8 /  26.2 18.3  94.1 46.7
-//   rows  4096  56.8 33.3 167.6 101.4 /  48.8 31.6 178.6 87.4
-//   rows 16384 225  110   679   296   / 187   94.5 669  268
+//   rows    32   5.6  4.3  12.9   7.2 /  11.8 11.2  18.0 16.4      (a kernel with W straight in registers: 6.2  4.4 14.9  8.1)
+//   rows   128   8.6  6.6  18.7  11.5 /  14.7 11.3  21.8 17.6      (                                       9.4  6.7  -   12.1)
+//   rows   256  12.4  8.2  24.4  15.3 /  13.4 11.8  31.3 22.5
+//   rows   512  16.4 11.8  31.0  21.4 /  17.7 12.6  36.4 27.6
+//   rows  1024  22.9 16.1  49.6  33.9 /  24.8 16.7  57.6 42.0
+//   rows  1536  29.8 21.0  79.9  42.3 /  29.9 21.6  99.1 48.7
+//   rows  4096  60.6 35.2 175.1  94.1 /  51.3 35.4 177.7 91.3
+//   rows  8192 119.3 59.0 349.7 167.8 /  99.7 53.3 350.6 145.0
 #include "linear_tile.h"
 
 namespace {
@@ -117,7 +117,7 @@ int launch(LinearParams A, hipStream_t stream)
 }
 
 // The tiles there are, and what a round of them costs: a step of K and what stands before and behind the steps, us, fitted to
-// 4900 timings (four projections of the decoder, 16 to 8192 rows, every tile, 1 to 24 slices of K).
+// 3200 timings with cold weights (four projections of the decoder, 16 to 8192 rows, every tile, 1 to 24 slices of K).
 struct TileCost {
     int bm, bn, least_steps, steps_multiple;                // steps of 64 elements of K: at least, and a multiple of
     float step, around;
@@ -134,24 +134,24 @@ constexpr TileCost tile(float step, float around) {
                          launch<BM, BN, WM, WN, WK, S, SX, kSilu>};
 }
 const TileCost kTiles[] = {
-    tile<32, 64, 2, 2, 1, 4, 4, true>(0.150f, 0.2f),
-    tile<64, 64, 2, 2, 2, 4, 4, true>(0.200f, 0.5f),
-    tile<128, 64, 2, 2, 2, 4, 4, true>(0.302f, 1.3f),
-    tile<192, 64, 2, 2, 2, 4, 4, true>(0.395f, 1.6f),
-    tile<128, 128, 2, 2, 2, 4, 4, true>(0.470f, 1.8f),
-    tile<192, 128, 2, 2, 2, 4, 4, true>(0.606f, 2.6f),
-    tile<128, 192, 4, 2, 1, 4, 4, true>(0.677f, 1.5f),
-    tile<192, 192, 4, 2, 1, 3, 3, false>(0.900f, 2.0f),
-    tile<256, 192, 4, 2, 1, 2, 3, false>(1.140f, 1.2f),
-    tile<256, 256, 4, 2, 1, 2, 3, false>(1.410f, 1.3f),
+    tile<32, 64, 2, 2, 1, 4, 4, true>(0.173f, 0.4f),
+    tile<64, 64, 2, 2, 2, 4, 4, true>(0.233f, 0.7f),
+    tile<128, 64, 2, 2, 2, 4, 4, true>(0.336f, 1.7f),
+    tile<192, 64, 2, 2, 2, 4, 4, true>(0.425f, 2.1f),
+    tile<128, 128, 2, 2, 2, 4, 4, true>(0.499f, 2.6f),
+    tile<192, 128, 2, 2, 2, 4, 4, true>(0.602f, 3.5f),
+    tile<128, 192, 4, 2, 1, 4, 4, true>(0.672f, 2.3f),
+    tile<192, 192, 4, 2, 1, 3, 3, false>(0.805f, 5.0f),
+    tile<256, 192, 4, 2, 1, 2, 3, false>(1.117f, 3.7f),
+    tile<256, 256, 4, 2, 1, 2, 3, false>(1.344f, 5.9f),
 };
 
 struct Plan { const TileCost* tile; int splits; };
 
 // The cheapest tile and number of slices by the costs above, in rounds of one workgroup per CU (the small tiles' second one
 // per CU is worth little: they share its intake).  Partial sums cost their writing and the next kernel's reading, 0.35 us per
-// MB together (5.7 TB/s), a rounded result a quarter of that per element.  Against the best of all timed choices this
-// costs 1 % on average and 10 % at most.
+// MB together (5.7 TB/s), a rounded result less than half of that per element.  Against the best of all timed choices this
+// costs 1 % on average and 15 % at most.
 Plan plan_of(int64_t rows, int64_t n, int64_t k, bool rounded, bool partials, bool silu)
 {
     Plan best{nullptr, 0};
@@ -165,7 +165,7 @@ Plan plan_of(int64_t rows, int64_t n, int64_t k, bool rounded, bool partials, bo
             const double steps = (double)(k / kStepK / s), rounds = (double)((tiles * s + cus - 1) / cus);
             for (int form = 0; form < 2; ++form) {                                  // 0: rounded or SiLU, 1: partial sums
                 if (form == 0 ? (s > 1 || !(rounded || silu)) : (!partials || !t.partials)) continue;
-                const double cost = 2.0 + rounds * (steps * t.step + t.around) + (form ? 0.35 * (double)s : 0.09) * mb;
+                const double cost = rounds * (steps * t.step + t.around) + (form ? 0.35 * (double)s : 0.15) * mb;
                 if (!best.tile || cost < least) { best = Plan{&t, form ? (int)s : 0}; least = cost; }
             }
         }
