@@ -439,6 +439,9 @@ int mdx_silu_and_mul(const void* x, int64_t x_row_stride, void* out, int64_t out
  * of the two, 0 where mdx_linear is, -1 where a library's product is the better choice (more than 1536 rows) or the shape
  * is not covered.  mdx_linear_silu: w [2 n, k], gate rows then up rows; y [rows, n] = mdx_silu_and_mul of the product, with
  * its rounding points; mdx_linear_silu_supported: covered, and up to 8192 rows.
+ * mdx_linear_qk_norm_rope_store: the product of a QKV projection with mdx_qk_norm_rope_store on it in one launch; w holds the q
+ * rows, then k, then v; k_out / v_out (the rotated k and the raw v, [rows, Hkv * d]) and the caches may be null;
+ * mdx_linear_qk_norm_rope_store_supported: 384 to 1536 rows, d = 128.
  * mdx_decode_linear_partials and mdx_decode_linear_silu: the same for the few rows of a decode pass, always as partial sums
  * (rows up to 128, n a multiple of 64, k of 256; splits = mdx_decode_linear_splits, 0 where not covered) and with the SiLU
  * (rows up to 64, n a multiple of 24, k of 512: mdx_decode_linear_silu_supported).
@@ -453,6 +456,14 @@ int mdx_linear_partials(const void* x, int64_t x_row_stride, const void* w, int6
 int32_t mdx_linear_silu_supported(int64_t rows, int64_t n, int64_t k);
 int mdx_linear_silu(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride,
                     void* y, int64_t y_row_stride, int64_t rows, int64_t n, int64_t k, mdx_stream_t stream);
+int32_t mdx_linear_qk_norm_rope_store_supported(int64_t rows, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int64_t k);
+int mdx_linear_qk_norm_rope_store(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride,
+                                  const void* q_weight, const void* k_weight, float eps,
+                                  const float* cos_table, const float* sin_table, int64_t max_positions, const int64_t* positions,
+                                  void* q_out, int64_t q_out_row_stride, void* k_out, int64_t k_out_row_stride,
+                                  void* v_out, int64_t v_out_row_stride,
+                                  void* k_cache, void* v_cache, const int32_t* slot_mapping, int64_t num_slots,
+                                  int64_t rows, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int64_t k, mdx_stream_t stream);
 int32_t mdx_decode_linear_splits(int64_t rows, int64_t n, int64_t k);
 int mdx_decode_linear_partials(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride,
                                float* partials, int64_t rows, int64_t n, int64_t k, mdx_stream_t stream);

@@ -384,6 +384,54 @@ PyObject* linear_gated(PyObject*, PyObject* const* a, Py_ssize_t n) {
     });
 }
 
+// x [.., k], w [(hq + 2 hkv) d, k], q/k weights, eps, cos, sin, positions, hq, hkv, d, caches and slots (or None), want_kv
+// -> (q [.., hq, d], k, v [.., hkv, d] or None), or None where the shape is not covered
+PyObject* linear_qk_norm_rope_store(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    ARGS(15);
+    return guarded([&]() -> PyObject* {
+        const Tensor &x = tensor(a[0]), &w = tensor(a[1]), &qw = tensor(a[2]), &kw = tensor(a[3]), &cos = tensor(a[5]), &sin = tensor(a[6]), &positions = tensor(a[7]);
+        const int64_t hq = integer(a[8]), hkv = integer(a[9]), d = integer(a[10]);
+        const Tensor &k_cache = optional_tensor(a[11]), &v_cache = optional_tensor(a[12]), &slot_mapping = optional_tensor(a[13]);
+        const bool want_kv = PyObject_IsTrue(a[14]) == 1;
+        need_gpu({&x, &w, &qw, &kw, &cos, &sin, &positions, &k_cache, &v_cache, &slot_mapping});
+        NEED(x.dim() >= 2 && w.dim() == 2 && x.size(-1) == w.size(1) && hq > 0 && hkv > 0 && d > 0 && w.size(0) == (hq + 2 * hkv) * d);
+        const int64_t k = w.size(1), rows = k ? x.numel() / k : 0;
+        if (!mdx_linear_qk_norm_rope_store_supported(rows, (int32_t)hq, (int32_t)hkv, (int32_t)d, k)) Py_RETURN_NONE;
+        const Rows r = rows_of(x, k);
+        if (!rows_covered(r, k) || !rows_covered(rows_of(w, k), k)) Py_RETURN_NONE;
+        NEED(qw.scalar_type() == at::kBFloat16 && kw.scalar_type() == at::kBFloat16 && qw.numel() == d && kw.numel() == d && qw.is_contiguous() && kw.is_contiguous());
+        NEED(positions.numel() == rows && positions.scalar_type() == at::kLong && cos.scalar_type() == at::kFloat && sin.scalar_type() == at::kFloat);
+        const Tensor pos = positions.is_contiguous() ? positions : positions.contiguous();
+        const bool caches = k_cache.defined() && k_cache.numel() > 0;
+        Tensor slots;
+        if (caches) {
+            NEED(v_cache.defined() && k_cache.is_contiguous() && v_cache.is_contiguous() && k_cache.scalar_type() == at::kBFloat16 && v_cache.scalar_type() == at::kBFloat16);
+            NEED(slot_mapping.defined() && slot_mapping.numel() == rows);
+            slots = int32_list(slot_mapping, "slot_mapping");
+        }
+        std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end() - 1);
+        shape.push_back(hq);
+        shape.push_back(d);
+        const auto options = at::TensorOptions().dtype(at::kBFloat16).device(x.device());
+        Tensor q = at::empty(shape, options), ko, vo;
+        shape[shape.size() - 2] = hkv;
+        if (want_kv) { ko = at::empty(shape, options); vo = at::empty(shape, options); }
+        check(mdx_linear_qk_norm_rope_store(ptr(r.t), r.stride, ptr(w), w.stride(0), ptr(qw), ptr(kw), (float)real(a[4]), static_cast<const float*>(ptr(cos)),
+                                            static_cast<const float*>(ptr(sin)), cos.size(0), static_cast<const int64_t*>(ptr(pos)), ptr(q), hq * d,
+                                            ptr_or_null(ko), hkv * d, ptr_or_null(vo), hkv * d, caches ? ptr(k_cache) : nullptr, caches ? ptr(v_cache) : nullptr,
+                                            static_cast<const int32_t*>(ptr_or_null(slots)), caches ? k_cache.numel() / (hkv * d) : 0, rows, (int32_t)hq,
+                                            (int32_t)hkv, (int32_t)d, k, stream_of(x)),
+              "linear_qk_norm_rope_store");
+        PyObject* t = PyTuple_New(3);
+        PyTuple_SET_ITEM(t, 0, wrap(std::move(q)));
+        for (int i = 1; i < 3; ++i) {
+            if (want_kv) PyTuple_SET_ITEM(t, i, wrap(std::move(i == 1 ? ko : vo)));
+            else { Py_INCREF(Py_None); PyTuple_SET_ITEM(t, i, Py_None); }
+        }
+        return t;
+    });
+}
+
 void need_partials(const Tensor& p) { NEED(p.dim() >= 3 && p.scalar_type() == at::kFloat && p.is_contiguous()); }
 
 // partials [splits, .., hidden], weight, eps, residual [.., hidden] -> normed, new residual
@@ -850,7 +898,7 @@ PyObject* sampler_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 #define ENTRY(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
-    ENTRY(store_kvcache), ENTRY(store_kvcache_maybe4d), ENTRY(qk_norm_rope_store), ENTRY(rms_norm), ENTRY(silu_and_mul), ENTRY(linear), ENTRY(linear_gated), ENTRY(linear_partials), ENTRY(linear_silu),
+    ENTRY(store_kvcache), ENTRY(store_kvcache_maybe4d), ENTRY(qk_norm_rope_store), ENTRY(rms_norm), ENTRY(silu_and_mul), ENTRY(linear), ENTRY(linear_gated), ENTRY(linear_qk_norm_rope_store), ENTRY(linear_partials), ENTRY(linear_silu),
     ENTRY(rms_norm_partials), ENTRY(qk_norm_rope_store_partials), ENTRY(sparse_attn_varlen),
     ENTRY(flash_attn_with_kvcache), ENTRY(attention_prefill), ENTRY(attention_decode), ENTRY(confidence_argmax), ENTRY(lm_head_confidence),
     ENTRY(filter_logits), ENTRY(select_transfer), ENTRY(unmask_step), ENTRY(sampler_step),

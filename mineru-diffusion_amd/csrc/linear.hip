@@ -18,21 +18,28 @@
 //   rows  4096  60.6 35.2 175.1  94.1 /  51.3 35.4 177.7 91.3
 //   rows  8192 119.3 59.0 349.7 167.8 /  99.7 53.3 350.6 145.0
 #include "linear_tile.h"
+#include "qk_row.h"
 
 namespace {
 
 using namespace mdx_tile;
 
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+using mdx_qk::RowParams;
+using mdx_qk::TokenPlace;
 
 struct LinearParams {
     Operands in;
     __bf16* y; float* partials;                    // y: [M, N]; partials: [splits, M, N]
     int64_t y_stride;                              // elements between rows
     int K, m_tiles, n_tiles, splits;
+    RowParams rows;                                // heads
 };
 
-enum Form { kRounded = 0, kPartials = 1, kSilu = 2 };
+enum Form { kRounded = 0, kPartials = 1, kSilu = 2, kHeads = 3 };
+
+template <typename T> constexpr int kSumsBytes = T::WK == 2 ? T::BM * T::BN * 4 : 0;      // where two wavefronts' sums meet
+constexpr int kHeadPitch = mdx_qk::kHeadDim + 8;
 
 template <typename T, int FORM>
 __global__ __launch_bounds__(T::kThreads, T::kWaves / 4) void linear_kernel(const LinearParams A)
@@ -42,6 +49,15 @@ __global__ __launch_bounds__(T::kThreads, T::kWaves / 4) void linear_kernel(cons
     const T tile;
     const Place at = place_of(A.m_tiles, A.n_tiles);
     const int m0 = at.m * T::BM, n0 = at.n * T::kCols, k_split = A.K / A.splits;
+    // heads: a column tile is one head row of every token, eight lanes of this thread's go to a token's; its place in the rotation
+    // and the cache is asked for ahead of the product
+    constexpr int kTokens = T::kThreads / mdx_qk::kLanesPerRow, kPasses = FORM == kHeads ? T::BM / kTokens : 1;
+    const int j8 = threadIdx.x % mdx_qk::kLanesPerRow, tok0 = m0 + (int)threadIdx.x / mdx_qk::kLanesPerRow;
+    TokenPlace places[kPasses];
+    if constexpr (FORM == kHeads) {
+#pragma unroll
+        for (int p = 0; p < kPasses; ++p) places[p] = mdx_qk::place_of_token(A.rows, min(tok0 + p * kTokens, A.in.M - 1), j8);
+    }
     typename T::Sums acc;
     tile.product(A.in, m0, n0, (int64_t)at.split * k_split, k_split / kStepK, lds, acc);
 
@@ -67,6 +83,17 @@ __global__ __launch_bounds__(T::kThreads, T::kWaves / 4) void linear_kernel(cons
         for (int j = 0; j < TN; ++j) {
             if constexpr (T::WK == 2) sum[j] = (tile.wk ? acc[H + i][j] : acc[i][j]) + theirs[(i * TN + j) * 64];
             else sum[j] = acc[i][j];
+        }
+        if constexpr (FORM == kHeads) {                      // the projection's rounding; rows of 128 bf16 and 16 bytes
+            __bf16* row = reinterpret_cast<__bf16*>(lds + kSumsBytes<T>) + (m - m0) * kHeadPitch;
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                bf16x4 out;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) out[e] = (__bf16)sum[j][e];
+                *reinterpret_cast<bf16x4*>(row + (tile.wn * TN + j) * 16 + 4 * tile.g) = out;
+            }
+            continue;
         }
         if (m >= A.in.M) continue;
         if (FORM == kSilu) {
@@ -97,14 +124,25 @@ __global__ __launch_bounds__(T::kThreads, T::kWaves / 4) void linear_kernel(cons
             }
         }
     }
+    if constexpr (FORM == kHeads) {
+        __syncthreads();
+#pragma unroll
+        for (int p = 0; p < kPasses; ++p) {
+            const int tok = tok0 + p * kTokens;
+            if (tok >= A.in.M) break;
+            const __bf16* row = reinterpret_cast<const __bf16*>(lds + kSumsBytes<T>) + (tok - m0) * kHeadPitch;
+            mdx_qk::finish_row(A.rows, tok, at.n, j8, *reinterpret_cast<const bf16x8*>(row + 8 * j8), *reinterpret_cast<const bf16x8*>(row + 64 + 8 * j8), places[p]);
+        }
+    }
 }
 
 template <int BM, int BN, int WM, int WN, int WK, int S, int SX, int FORM>
 int launch(LinearParams A, hipStream_t stream)
 {
     typedef Tile<BM, BN, WM, WN, WK, S, SX, FORM == kSilu> T;
-    constexpr int kSums = WK == 2 ? BM * BN * 4 : 0, kLdsBytes = T::kStepsBytes > kSums ? T::kStepsBytes : kSums;
+    constexpr int kAfter = kSumsBytes<T> + (FORM == kHeads ? BM * kHeadPitch * 2 : 0), kLdsBytes = T::kStepsBytes > kAfter ? T::kStepsBytes : kAfter;
     static_assert(kLdsBytes <= 160 * 1024, "LDS");
+    static_assert(FORM != kHeads || (BN == mdx_qk::kHeadDim && WK == 2 && BM % (T::kThreads / mdx_qk::kLanesPerRow) == 0), "a head per column tile");
     static std::atomic<bool> raised[64];
     const int rc = reserve_lds(reinterpret_cast<const void*>(linear_kernel<T, FORM>), kLdsBytes, raised, "linear");
     if (rc != MDX_OK) return rc;
@@ -173,6 +211,20 @@ Plan plan_of(int64_t rows, int64_t n, int64_t k, bool rounded, bool partials, bo
     return best;                                                                    // splits 0: not partial sums
 }
 
+// The QKV projection with what follows it: tiles of one head, by the same costs.  Two launches / one, us per decoder layer: 160 rows
+// 85.6 / 87.5, 256 94.5 / 96.4, 384 117.9 / 115.5, 512 124.1 / 121.3, 768 153.0 / 150.8, 1024 179.6 / 176.5, 1504 241.5 / 238.4.
+int launch_heads(const LinearParams& A, hipStream_t stream)
+{
+    const int cus = mdx::compute_units();
+    auto cost = [&](int bm, float step, float around) {
+        const int64_t tiles = (int64_t)((A.in.M + bm - 1) / bm) * (A.in.N / mdx_qk::kHeadDim);
+        return (float)((tiles + cus - 1) / cus) * ((float)(A.K / kStepK) * step + around);
+    };
+    const float c64 = cost(64, 0.345f, 1.7f), c128 = cost(128, 0.499f, 2.6f), c192 = cost(192, 0.602f, 3.5f);
+    if (c64 <= c128 && c64 <= c192) return launch<64, 128, 2, 2, 2, 4, 4, kHeads>(A, stream);
+    return c128 <= c192 ? launch<128, 128, 2, 2, 2, 4, 4, kHeads>(A, stream) : launch<192, 128, 2, 2, 2, 4, 4, kHeads>(A, stream);
+}
+
 constexpr int64_t kSizeLimit = (int64_t)1 << 28;
 
 bool sizes_covered(int64_t rows, int64_t n, int64_t k)
@@ -225,6 +277,9 @@ int run_rows(const char* what, bool silu, const void* x, int64_t x_row_stride, c
 // Where the kernel is the better one (table at the top of this file): up to 1536 rows; with the SiLU in the epilogue, which
 // saves writing and reading twice the result, up to 8192.
 constexpr int64_t kMaxRows = 1536, kMaxSiluRows = 8192;
+// With the head rows finished in the epilogue (launch_heads): from where tiles of 128 columns are enough to fill most CUs; fewer rows
+// are bound by what a CU takes in, and the product in narrower tiles or slices of K with a second launch is the faster.
+constexpr int64_t kMinHeadRows = 384;
 constexpr int64_t kMaxDecodeRows = 128, kMaxDecodeSiluRows = 64;
 
 Plan decode_plan(int64_t rows, int64_t n, int64_t k)
@@ -265,6 +320,40 @@ extern "C" int mdx_linear_silu(const void* x, int64_t x_row_stride, const void* 
     MDX_REQUIRE(sizes_covered(rows, n, k), MDX_EUNSUPPORTED, "linear_silu: %lld rows, n %lld (a multiple of 8), k %lld (a multiple of 128, at least 256)",
                 (long long)rows, (long long)n, (long long)k);
     return run_rows("linear_silu", true, x, x_row_stride, w, w_row_stride, y, y_row_stride, rows, n, k, stream);
+}
+
+extern "C" int32_t mdx_linear_qk_norm_rope_store_supported(int64_t rows, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int64_t k)
+{
+    return num_q_heads > 0 && num_kv_heads > 0 && head_dim == mdx_qk::kHeadDim && rows >= kMinHeadRows && rows <= kMaxRows &&
+           sizes_covered(rows, ((int64_t)num_q_heads + 2 * (int64_t)num_kv_heads) * head_dim, k);
+}
+
+extern "C" int mdx_linear_qk_norm_rope_store(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride,
+                                             const void* q_weight, const void* k_weight, float eps,
+                                             const float* cos_table, const float* sin_table, int64_t max_positions, const int64_t* positions,
+                                             void* q_out, int64_t q_out_row_stride, void* k_out, int64_t k_out_row_stride,
+                                             void* v_out, int64_t v_out_row_stride,
+                                             void* k_cache, void* v_cache, const int32_t* slot_mapping, int64_t num_slots,
+                                             int64_t rows, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int64_t k, mdx_stream_t stream)
+{
+    const char* what = "linear_qk_norm_rope_store";
+    MDX_REQUIRE(mdx_linear_qk_norm_rope_store_supported(rows, num_q_heads, num_kv_heads, head_dim, k), MDX_EUNSUPPORTED,
+                "%s: %lld rows (%lld to %lld), head_dim %d (only %d), k %lld (a multiple of 128, at least 256)", what, (long long)rows,
+                (long long)kMinHeadRows, (long long)kMaxRows, head_dim, mdx_qk::kHeadDim, (long long)k);
+    const int64_t n = ((int64_t)num_q_heads + 2 * (int64_t)num_kv_heads) * head_dim;
+    const int rc = check_linear(what, x, x_row_stride, w, w_row_stride, q_out, rows, n, k);
+    if (rc != MDX_OK) return rc;
+    MDX_REQUIRE(q_weight && k_weight && cos_table && sin_table && positions, MDX_EINVAL, "%s: null pointer", what);
+    MDX_REQUIRE((k_cache == nullptr) == (v_cache == nullptr), MDX_EINVAL, "%s: give both caches or neither", what);
+    MDX_REQUIRE(!k_cache || slot_mapping, MDX_EINVAL, "%s: caches without slot_mapping", what);
+    MDX_REQUIRE(mdx::aligned16(q_weight) && mdx::aligned16(k_weight) && mdx::aligned16(k_out) && mdx::aligned16(v_out) &&
+                mdx::aligned16(k_cache) && mdx::aligned16(v_cache) && q_out_row_stride % 8 == 0 && k_out_row_stride % 8 == 0 && v_out_row_stride % 8 == 0,
+                MDX_EUNSUPPORTED, "%s: tensors must be 16-byte aligned with row strides that are multiples of 8", what);
+    LinearParams A = params_of(x, x_row_stride, w, w_row_stride, rows, n, k);
+    A.rows = RowParams{(const __bf16*)q_weight, (const __bf16*)k_weight, eps, cos_table, sin_table, max_positions, positions,
+                       (__bf16*)q_out, q_out_row_stride, (__bf16*)k_out, k_out_row_stride, (__bf16*)v_out, v_out_row_stride,
+                       (__bf16*)k_cache, (__bf16*)v_cache, slot_mapping, num_slots, num_q_heads, num_kv_heads};
+    return launch_heads(A, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int32_t mdx_decode_linear_splits(int64_t rows, int64_t n, int64_t k) { return decode_plan(rows, n, k).splits; }

@@ -52,6 +52,9 @@ SIGNATURES = {
     "mdx_linear_partials": (c_int32, [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _P]),
     "mdx_linear_silu_supported": (c_int32, [_I64] * 3),
     "mdx_linear_silu": (c_int32, [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _P]),
+    "mdx_linear_qk_norm_rope_store_supported": (c_int32, [_I64] + [_I32] * 3 + [_I64]),
+    "mdx_linear_qk_norm_rope_store": (c_int32, [_P, _I64, _P, _I64, _P, _P, _F, _P, _P, _I64, _P] + [_P, _I64] * 3 + [_P, _P, _P, _I64, _I64] +
+                                      [_I32] * 3 + [_I64, _P]),
     "mdx_decode_linear_splits": (c_int32, [_I64] * 3),
     "mdx_decode_linear_partials": (c_int32, [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _P]),
     "mdx_decode_linear_silu_supported": (c_int32, [_I64] * 3),

@@ -32,7 +32,7 @@ from torch import nn
 from . import _lib
 from .context import get_context, reset_context, set_context
 from .layers import Attention
-from .ops import (confidence_argmax, lm_head_confidence, flash_attn_with_kvcache, linear, linear_gated, qk_norm_rope_store,
+from .ops import (confidence_argmax, lm_head_confidence, flash_attn_with_kvcache, linear, linear_gated, linear_qk_norm_rope_store, qk_norm_rope_store,
                   qk_norm_rope_store_partials, rms_norm, rms_norm_partials, select_transfer, silu_and_mul, sparse_attn_varlen, unmask_step)
 
 PAGE = 256                      # tokens per KV page (Sequence.kvcache_block_size, sequence.py:17)
@@ -243,18 +243,21 @@ class DecoderLayer(nn.Module):
         one libmdx launch; the attention calls are the same two as in `Attention.forward`."""
         c, attn, ctx = self.c, self.attn, get_context()
         have_cache = attn.k_cache.numel() > 0
-        qkv = linear(h, self.qkv_proj, have_cache and not ctx.is_prefill)
-        if qkv is None:
-            qkv = F.linear(h, self.qkv_proj)
-        if qkv.dim() > h.dim():
-            q = qk_norm_rope_store_partials(qkv, self.q_norm, self.k_norm, c.rms_norm_eps, cos_table, sin_table, positions, c.num_heads,
-                                            c.num_kv_heads, c.head_dim, attn.k_cache, attn.v_cache, ctx.slot_mapping)
-            return flash_attn_with_kvcache(q, attn.k_cache, attn.v_cache, cache_seqlens=ctx.context_lens, block_table=ctx.block_tables,
-                                           softmax_scale=attn.scale, causal=False).flatten(2)
-        q, k, v = qk_norm_rope_store(qkv, self.q_norm, self.k_norm, c.rms_norm_eps, cos_table, sin_table, positions,
-                                     c.num_heads, c.num_kv_heads, c.head_dim,
-                                     attn.k_cache if have_cache else None, attn.v_cache if have_cache else None,
-                                     ctx.slot_mapping if have_cache else None, want_k=ctx.is_prefill)
+        caches = (attn.k_cache, attn.v_cache, ctx.slot_mapping) if have_cache else (None, None, None)
+        done = linear_qk_norm_rope_store(h, self.qkv_proj, self.q_norm, self.k_norm, c.rms_norm_eps, cos_table, sin_table, positions,
+                                         c.num_heads, c.num_kv_heads, c.head_dim, *caches, want_kv=ctx.is_prefill)
+        if done is not None:
+            q, k, v = done
+        else:
+            qkv = linear(h, self.qkv_proj, have_cache and not ctx.is_prefill)
+            if qkv is None:
+                qkv = F.linear(h, self.qkv_proj)
+            if qkv.dim() > h.dim():
+                q = qk_norm_rope_store_partials(qkv, self.q_norm, self.k_norm, c.rms_norm_eps, cos_table, sin_table, positions, c.num_heads,
+                                                c.num_kv_heads, c.head_dim, *caches)
+            else:
+                q, k, v = qk_norm_rope_store(qkv, self.q_norm, self.k_norm, c.rms_norm_eps, cos_table, sin_table, positions,
+                                             c.num_heads, c.num_kv_heads, c.head_dim, *caches, want_k=ctx.is_prefill)
         if ctx.is_prefill:
             o = sparse_attn_varlen(q, k, v, cu_seqlens_q=ctx.cu_seqlens_q, cu_seqlens_k=ctx.cu_seqlens_k,
                                    staircase_size=ctx.block_size, max_seqlen=ctx.max_seqlen_k or None, softmax_scale=attn.scale)

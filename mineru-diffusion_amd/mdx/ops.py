@@ -75,6 +75,14 @@ def linear_gated(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor | None:
     return _host().linear_gated(x, weight)
 
 
+def linear_qk_norm_rope_store(x, weight, q_weight, k_weight, eps, cos, sin, positions, num_q_heads, num_kv_heads, head_dim,
+                              k_cache=None, v_cache=None, slot_mapping=None, want_kv: bool = True):
+    """qk_norm_rope_store(x . weight^T, ...) for 384 to 1536 rows and heads of 128 columns in one launch (nanovllm/models/sdar.py:73-83
+    and the cache store): (q, k, v), k and v None unless wanted."""
+    return _host().linear_qk_norm_rope_store(x, weight, q_weight, k_weight, eps, cos, sin, positions, num_q_heads, num_kv_heads, head_dim,
+                                             k_cache, v_cache, slot_mapping, want_kv)
+
+
 def linear_partials(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor | None:
     """The partial sums of up to 128 rows, also where there is one slice only."""
     return _host().linear_partials(x, weight)

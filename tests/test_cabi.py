@@ -228,3 +228,9 @@ def test_linear_arguments_are_validated(L):
         assert call(xs=1 << 28) == -2 and call(ys=60) == -2 and call(ys=66) == -2 and call(rows=0) == -2 and call(n=68) == -2 and call(k=192) == -2
     pl = lambda **kw: L.mdx_linear_partials(kw.get("x", one), 6144, one, 6144, kw.get("p", one), kw.get("rows", 32), 2048, 6144, null)             # noqa: E731
     assert pl(x=null) == -1 and pl(p=null) == -1 and pl(p=odd) == -2 and pl(rows=1537) == -2
+
+    hd = lambda **kw: L.mdx_linear_qk_norm_rope_store(kw.get("x", one), kw.get("xs", 256), one, 256, kw.get("qw", one), one, 1e-6, one, one, 8, kw.get("pos", one),   # noqa: E731
+                                                      kw.get("q", one), kw.get("qs", 256), null, 0, null, 0, kw.get("kc", null), kw.get("vc", null), kw.get("slots", null), 0,
+                                                      kw.get("rows", 400), 2, 1, kw.get("d", 128), 256, null)
+    assert hd(x=null) == -1 and hd(qw=null) == -1 and hd(pos=null) == -1 and hd(q=null) == -1 and hd(kc=one) == -1 and hd(kc=one, vc=one) == -1
+    assert hd(rows=383) == -2 and hd(rows=1537) == -2 and hd(d=64) == -2 and hd(q=odd) == -2 and hd(qs=260) == -2 and hd(qw=odd) == -2 and hd(xs=248) == -2

@@ -53,3 +53,43 @@ def test_linear_says_what_it_does_not_cover(dev):
         assert ops.linear(x, w) is None and ops.linear(x, w, True) is None
     assert ops.linear_gated(z(8193, 256), z(64, 256)) is None and ops.linear_gated(z(4, 256), z(72, 256)) is None
     assert ops.linear(z(2, 3, 256), z(64, 256)).shape == (2, 3, 64) and ops.linear_gated(z(2, 3, 256), z(64, 256)).shape == (2, 3, 32)
+
+
+@pytest.mark.parametrize("rows,hq,hkv,k", [(384, 16, 8, 384), (385, 2, 1, 256), (513, 4, 2, 512), (1000, 16, 8, 256), (1100, 16, 8, 256), (1536, 6, 3, 256)])
+@pytest.mark.parametrize("caches", [True, False])
+def test_linear_qk_norm_rope_store(dev, rows, hq, hkv, k, caches):
+    """Each of the tiles with head rows finished in the epilogue against qk_norm_rope_store on the rounded product: last row tiles of
+    few rows, positions beyond the table, slots that are skipped or out of range, with and without caches and k / v."""
+    import mdx
+    from mdx import ops
+    d, n = 128, (hq + 2 * hkv) * 128
+    _, x, w = _xw(dev, rows, n, k)
+    g = torch.Generator().manual_seed(rows)
+    qw, kw = torch.randn(d, generator=g).bfloat16().to(dev), torch.randn(d, generator=g).bfloat16().to(dev)
+    cos, sin = torch.rand(2000, d // 2, generator=g).to(dev), torch.rand(2000, d // 2, generator=g).to(dev)
+    pos = torch.randint(0, 2000, (rows,), generator=g)
+    pos[::17], pos[5] = 2000, -1
+    slots = torch.randperm(2048, generator=g)[:rows].int()
+    slots[::7], slots[3] = -1, 4096
+    pos, slots = pos.to(dev), slots.to(dev)
+    store = lambda: (torch.zeros(8, 256, hkv, d, dtype=torch.bfloat16, device=dev), torch.zeros(8, 256, hkv, d, dtype=torch.bfloat16, device=dev), slots)   # noqa: E731
+    one, two = store(), store()
+    q, kk, v = ops.linear_qk_norm_rope_store(x, w, qw, kw, 1e-6, cos, sin, pos, hq, hkv, d, *(one if caches else (None,) * 3), want_kv=True)
+    q2, k2, v2 = mdx.qk_norm_rope_store(ops.linear(x, w), qw, kw, 1e-6, cos, sin, pos, hq, hkv, d, *(two if caches else (None,) * 3))
+    pairs = [(q, q2), (kk, k2), (v, v2)] + list(zip(one[:2], two[:2])) * caches
+    for a, b in pairs:                        # the same roundings; the two products' orders of summation may round apart
+        assert a.shape == b.shape and (a.float() - b.float()).norm() < 3e-3 * b.float().norm()
+    if caches:
+        assert all(torch.equal(a == 0, b == 0) for a, b in zip(one[:2], two[:2]))
+    q3, none, nothing = ops.linear_qk_norm_rope_store(x, w, qw, kw, 1e-6, cos, sin, pos, hq, hkv, d, *(one if caches else (None,) * 3), want_kv=False)
+    assert none is None and nothing is None and torch.equal(q3, q)
+
+
+def test_linear_qk_norm_rope_store_says_what_it_does_not_cover(dev):
+    from mdx import ops
+    z = lambda *s, dtype=torch.bfloat16: torch.zeros(*s, dtype=dtype, device=dev)                # noqa: E731
+    call = lambda x, w, hq, hkv, d: ops.linear_qk_norm_rope_store(x, w, z(d), z(d), 1e-6, z(8, d // 2, dtype=torch.float32), z(8, d // 2, dtype=torch.float32),   # noqa: E731
+                                                                  z(x.shape[0], dtype=torch.int64), hq, hkv, d)
+    assert call(z(383, 256), z(512, 256), 2, 1, 128) is None and call(z(1537, 256), z(512, 256), 2, 1, 128) is None
+    assert call(z(400, 256), z(256, 256), 2, 1, 64) is None and call(z(400, 320), z(512, 320), 2, 1, 128) is None
+    assert call(z(400, 264)[:, 1:257], z(512, 256), 2, 1, 128) is None and call(z(400, 256), z(512, 256), 2, 1, 128) is not None
