@@ -54,9 +54,11 @@ __global__ __launch_bounds__(T::kThreads, T::kWaves / 4) void linear_kernel(cons
     constexpr int kTokens = T::kThreads / mdx_qk::kLanesPerRow, kPasses = FORM == kHeads ? T::BM / kTokens : 1;
     const int j8 = threadIdx.x % mdx_qk::kLanesPerRow, tok0 = m0 + (int)threadIdx.x / mdx_qk::kLanesPerRow;
     TokenPlace places[kPasses];
+    mdx_qk::RowWeight weight;
     if constexpr (FORM == kHeads) {
 #pragma unroll
         for (int p = 0; p < kPasses; ++p) places[p] = mdx_qk::place_of_token(A.rows, min(tok0 + p * kTokens, A.in.M - 1), j8);
+        weight = mdx_qk::weight_of_row(A.rows, at.n, j8);
     }
     typename T::Sums acc;
     tile.product(A.in, m0, n0, (int64_t)at.split * k_split, k_split / kStepK, lds, acc);
@@ -131,7 +133,7 @@ __global__ __launch_bounds__(T::kThreads, T::kWaves / 4) void linear_kernel(cons
             const int tok = tok0 + p * kTokens;
             if (tok >= A.in.M) break;
             const __bf16* row = reinterpret_cast<const __bf16*>(lds + kSumsBytes<T>) + (tok - m0) * kHeadPitch;
-            mdx_qk::finish_row(A.rows, tok, at.n, j8, *reinterpret_cast<const bf16x8*>(row + 8 * j8), *reinterpret_cast<const bf16x8*>(row + 64 + 8 * j8), places[p]);
+            mdx_qk::finish_row(A.rows, tok, at.n, j8, *reinterpret_cast<const bf16x8*>(row + 8 * j8), *reinterpret_cast<const bf16x8*>(row + 64 + 8 * j8), places[p], weight);
         }
     }
 }

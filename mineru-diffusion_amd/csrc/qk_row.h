@@ -46,8 +46,21 @@ __device__ __forceinline__ TokenPlace place_of_token(const RowParams& P, int64_t
     return t;
 }
 
+struct RowWeight { bf16x8 a, b; };      // the norm's weight for lane j's columns; of a v row, nothing
+
+__device__ __forceinline__ RowWeight weight_of_row(const RowParams& P, int row, int j) {
+    RowWeight w;
+    if (row < P.hq + P.hkv) {
+        const __bf16* src = (row < P.hq ? P.q_w : P.k_w) + 8 * j;
+        w.a = *reinterpret_cast<const bf16x8*>(src);
+        w.b = *reinterpret_cast<const bf16x8*>(src + 64);
+    }
+    return w;
+}
+
 // row: head row of the token, q | k | v.  The 8 lanes of a row call it together.
-__device__ __forceinline__ void finish_row(const RowParams& P, int64_t tok, int row, int j, bf16x8 a, bf16x8 b, const TokenPlace& t) {
+__device__ __forceinline__ void finish_row(const RowParams& P, int64_t tok, int row, int j, bf16x8 a, bf16x8 b, const TokenPlace& t,
+                                           const RowWeight& w) {
     const bool is_q = row < P.hq, is_k = !is_q && row < P.hq + P.hkv;
     if (is_q || is_k) {
         float ss = 0.f;
@@ -57,13 +70,10 @@ __device__ __forceinline__ void finish_row(const RowParams& P, int64_t tok, int 
         ss += __shfl_xor(ss, 2);
         ss += __shfl_xor(ss, 4);
         const float inv = rsqrtf(ss * (1.0f / kHeadDim) + P.eps);
-        const __bf16* w = is_q ? P.q_w : P.k_w;
-        const bf16x8 wa = *reinterpret_cast<const bf16x8*>(w + 8 * j);
-        const bf16x8 wb = *reinterpret_cast<const bf16x8*>(w + 64 + 8 * j);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const float x1 = (float)(__bf16)((float)(__bf16)((float)a[e] * inv) * (float)wa[e]);
-            const float x2 = (float)(__bf16)((float)(__bf16)((float)b[e] * inv) * (float)wb[e]);
+            const float x1 = (float)(__bf16)((float)(__bf16)((float)a[e] * inv) * (float)w.a[e]);
+            const float x2 = (float)(__bf16)((float)(__bf16)((float)b[e] * inv) * (float)w.b[e]);
             a[e] = (__bf16)(x1 * t.cs[e] - x2 * t.sn[e]);
             b[e] = (__bf16)(x2 * t.cs[e] + x1 * t.sn[e]);
         }

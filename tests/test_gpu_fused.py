@@ -167,3 +167,57 @@ def test_silu_and_mul_matches_oracle(dev, rows, inter):
     # rows taken out of a wider matrix
     wide = (torch.randn(rows, 2 * inter + 64, generator=g)).bfloat16().to(dev)
     _ulp_close(mdx.silu_and_mul(wide[:, 64:]), oracle.silu_and_mul(wide[:, 64:].cpu()), frac_equal=0.97)
+
+
+@pytest.mark.parametrize("slices", [1, 2, 4, 5, 8])
+@pytest.mark.parametrize("rows,hidden", [(1, 2048), (3, 8), (256, 2040), (257, 2048), (5, 2056), (300, 4096), (4, 8192)])
+def test_norm_of_partial_sums(dev, slices, rows, hidden):
+    """rms_norm_partials on every number of slices it has a kernel for and on others, on both sides of its rules on rows and widths.
+    The sum is formed in the order of the slices, so the residual is the same to the bit.  Of the norm, the mean's order of summation can
+    turn the first rounding to the next bf16, up to 2^-7 of the value away (8 significant bits), and the product with the weight is
+    rounded by up to 2^-8 on either side: 2^-6 in all."""
+    from mdx import ops
+    g = torch.Generator().manual_seed(slices * rows + hidden)
+    p, res = torch.randn(slices, rows, hidden, generator=g), torch.randn(rows, hidden, generator=g).bfloat16()
+    w = torch.randn(hidden, generator=g).bfloat16()
+    total = p[0].clone()
+    for s in range(1, slices):
+        total += p[s]
+    x = total.bfloat16().float() + res.float()
+    y = (x * torch.rsqrt(x.double().square().mean(1, keepdim=True) + 1e-6).float()).bfloat16() * w
+    out, new = ops.rms_norm_partials(p.to(dev), w.to(dev), 1e-6, res.to(dev))
+    assert torch.equal(new.cpu(), x.bfloat16())
+    assert ((out.cpu().float() - y.float()).abs() <= 2 ** -6 * y.float().abs()).all()
+
+
+@pytest.mark.parametrize("slices", [0, 1, 2, 4, 5, 8])
+@pytest.mark.parametrize("hq,hkv", [(16, 8), (3, 1), (70, 5)])
+def test_fused_does_not_depend_on_the_number_of_tokens(dev, slices, hq, hkv):
+    """Few tokens are spread over several workgroups each, many take one: the same rows in either, as partial sums or (slices 0) not,
+    give the same bits; with more head rows than a workgroup takes at a time."""
+    import mdx
+    from mdx import ops
+    g = torch.Generator().manual_seed(slices + hq)
+    n, d, slots = 300, 128, 512
+    qkv = torch.randn(max(slices, 1), n, (hq + 2 * hkv) * d, generator=g).to(dev)
+    qw, kw = (torch.randn(d, generator=g).bfloat16().to(dev) for _ in range(2))
+    cos, sin = (torch.rand(64, d // 2, generator=g).to(dev) for _ in range(2))
+    pos, slot = torch.randint(0, 64, (n,), generator=g).to(dev), torch.randperm(slots, generator=g)[:n].int().to(dev)
+    total = qkv[0].clone()
+    for s in range(1, slices):
+        total += qkv[s]
+
+    def run(ranges, partials):
+        caches = [torch.zeros(1, slots, hkv, d, dtype=torch.bfloat16, device=dev) for _ in range(2)]
+        q = []
+        for a, b in ranges:
+            if partials:
+                q.append(ops.qk_norm_rope_store_partials(qkv[:, a:b].contiguous(), qw, kw, 1e-6, cos, sin, pos[a:b], hq, hkv, d, *caches, slot[a:b]))
+            else:
+                q.append(mdx.qk_norm_rope_store(total[a:b].bfloat16(), qw, kw, 1e-6, cos, sin, pos[a:b], hq, hkv, d, *caches, slot[a:b])[0])
+        return [torch.cat(q), *caches]
+
+    whole = run([(0, n)], False)
+    for ranges in ([(0, n)], [(0, 1), (1, 45), (45, n)]):
+        for a, b in zip(run(ranges, slices > 0), whole):
+            assert torch.equal(a, b)
