@@ -516,14 +516,14 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
 // Folds the split partials: a workgroup takes 8 QUERIES queries of a (sequence, head), a thread four columns of QUERIES of them.  The
 // kernel is a chain of memory latencies (length -> partials -> output), not of bytes: the loads of the first slots are
 // on their way before the lengths say how many of them exist (where a slot lies does not depend on it; what lies
-// beyond is masked out), and a thread's share of a slot is one load.  Few heads (QUERIES = 1) get eight slots in flight and
+// beyond is masked out), and a thread's share of a slot is one load.  Few heads (QUERIES = 1) get eight or twelve slots in flight and
 // more workgroups; with more of them there are workgroups enough, fewer pieces per sequence, and the workgroups of whole
 // sequences, which leave at once, still have to be launched.  (A workgroup per head with 16 columns per thread, the form this
 // replaced, took 0.6 us per four pieces of a sequence, which kept the pieces long.)
-template <typename E, int QUERIES>
+template <typename E, int QUERIES, int AHEAD>
 __global__ __launch_bounds__(256) void paged_combine_kernel(const PagedParams P)
 {
-    constexpr int kAhead = 8 / QUERIES, kParts = 4 / QUERIES;
+    constexpr int kAhead = AHEAD, kParts = 4 / QUERIES;
     const int part = blockIdx.x % kParts, rest = blockIdx.x / kParts;
     const int qt = rest % P.nqt, hq = (rest / P.nqt) % P.num_q_heads, b = rest / P.nqt / P.num_q_heads;
     const int c = (threadIdx.x & 31) * 4, s0 = part * 8 * QUERIES + (threadIdx.x >> 5);         // queries s0, s0 + 8
@@ -762,9 +762,17 @@ int launch_paged(const void* q, void* o, const void* k_cache, const void* v_cach
     }
     int rc = mdx::check_launch("paged_block_attn");
     if (rc != MDX_OK || !two_launches) return rc;
-    const bool few = n_heads <= 128;
-    if (dtype == MDX_F16) { if (few) paged_combine_kernel<_Float16, 1><<<4 * n_heads, 256, 0, stream>>>(P); else paged_combine_kernel<_Float16, 2><<<2 * n_heads, 256, 0, stream>>>(P); }
-    else                  { if (few) paged_combine_kernel<__bf16, 1><<<4 * n_heads, 256, 0, stream>>>(P);   else paged_combine_kernel<__bf16, 2><<<2 * n_heads, 256, 0, stream>>>(P); }
+    // The slots asked for at once: eight, or twelve where the sequences of tables that are 65 % full have about as many pieces or up to
+    // half as many again.  (One sequence of 1337 keys, twelve against eight: 14.8 and 15.3 us, 1000: 14.2 and 14.7, two of 3000 to 3500:
+    // 21.4 and 21.9, three of 3000 to 5000: 25.3 and 25.9; but one of 300: 12.3 and 12.1, of 2500: 17.2 and 16.9.)
+    const double pieces = sqrt(0.65 * max_pages * page_size / bs) / kPieceRoot;
+    auto combine = [&](auto element) {
+        typedef decltype(element) E;
+        if (n_heads > 128) paged_combine_kernel<E, 2, 4><<<2 * n_heads, 256, 0, stream>>>(P);
+        else if (pieces > 7 && pieces <= 9.5) paged_combine_kernel<E, 1, 12><<<4 * n_heads, 256, 0, stream>>>(P);
+        else paged_combine_kernel<E, 1, 8><<<4 * n_heads, 256, 0, stream>>>(P);
+    };
+    if (dtype == MDX_F16) combine(_Float16()); else combine(__bf16());
     return mdx::check_launch("paged_combine");
 }
 

@@ -29,3 +29,9 @@ def test_pieces(dev, ctxs, wide):
     o = mdx.flash_attn_with_kvcache(q.to(dev), kc.to(dev), vc.to(dev), cache_seqlens=lens.to(dev), block_table=bt.to(dev), softmax_scale=1 / math.sqrt(d))
     ref = oracle.paged_block_attn(q, kc, vc, bt, lens, 1 / math.sqrt(d))
     assert (o.float().cpu() - ref).abs().max().item() < 2e-2
+
+
+@pytest.mark.parametrize("ctxs", [[1030], [1400], [2048], [1, 3500], [3500, 200], [3584, 3584]])
+def test_pieces_folded_twelve_at_a_time(dev, ctxs):
+    """Tables wide enough for 8 to 14 pieces of a sequence: fewer, as many and more than the fold asks for at once."""
+    test_pieces(dev, ctxs, 0)
