@@ -75,7 +75,11 @@ __global__ __launch_bounds__(64 * HPW * KW, D <= 128 && KW <= 2 ? 2 : 1) void pa
     const int kvh = (blockIdx.x / P.nqt) * HPW / P.heads_per_kv;
     const int width = P.head_dim;
 
+    // The workgroup's queries come through LDS too: a lane's own row, 16 bytes at a time, would touch every line eight times.
+    QueryRegs<T, D, HPW, kThreads> queries;
     const int ctx = keys_of(P, b);
+    queries.fetch(static_cast<const T*>(P.q) + (int64_t)b * P.q_sb + (int64_t)(qt * 32) * P.q_ss + (int64_t)(head - hw) * P.q_sh, P.q_ss, P.q_sh,
+                  P.sq - qt * 32, tid, width);
     const int span = P.nsplit > 1 ? keys_per_piece(P, ctx, lane) : max(1, ctx);
     const int n_pieces = max(1, (ctx + span - 1) / span);
     if (split >= n_pieces) return;
@@ -89,7 +93,9 @@ __global__ __launch_bounds__(64 * HPW * KW, D <= 128 && KW <= 2 ? 2 : 1) void pa
     const T* vc = static_cast<const T*>(P.v_cache) + (int64_t)kvh * P.c_sh;
 
     float q[D / 2];
-    load_q<T, D>(q, row_ok ? static_cast<const T*>(P.q) + (int64_t)b * P.q_sb + (int64_t)qrow * P.q_ss + (int64_t)head * P.q_sh : nullptr, H, width);
+    queries.write(lds, tid);
+    __syncthreads();
+    queries.read(q, lds, hw, H, r, width);
     State<D> st;
     st.init();
     for (int t0 = 0; t0 < n_tiles; t0 += KW) {
@@ -115,7 +121,7 @@ __global__ __launch_bounds__(64 * HPW * KW, D <= 128 && KW <= 2 ? 2 : 1) void pa
                 for (int j = 0; j < kTogether; ++j)
                     if ((tile_ok >> (i0 + j)) & 1u)
                         regs[j].fetch(b, tid, width, [&](int row) { return kc + base[j] + (int64_t)row * P.c_st; }, [&](int row) { return vc + base[j] + (int64_t)row * P.c_st; });
-                if (i0 == 0 && b == 0 && t0) __syncthreads();  // the previous tiles have been read by everybody
+                if (i0 == 0 && b == 0) __syncthreads();        // the queries or the previous tiles have been read by everybody
 #pragma unroll
                 for (int j = 0; j < kTogether; ++j)
                     if ((tile_ok >> (i0 + j)) & 1u)
@@ -131,6 +137,7 @@ __global__ __launch_bounds__(64 * HPW * KW, D <= 128 && KW <= 2 ? 2 : 1) void pa
 
     // ---- the KW states of a head fold through LDS; one piece: the result, else a partial ----
     static_assert(HPW * KW * kStateBytes<D> <= KW * Lds<D>::kBytes, "merge buffer exceeds the tile region");
+    static_assert(QueryRegs<T, D, HPW, kThreads>::kBytes <= KW * Lds<D>::kBytes, "queries exceed the tile region");
     T* orow = static_cast<T*>(P.o) + (int64_t)b * P.o_sb + (int64_t)qrow * P.o_ss + (int64_t)head * P.o_sh;
     const int64_t slot = (((int64_t)b * P.num_q_heads + head) * P.nqt + qt) * P.nsplit + split;
     float* prow = P.part_o + (slot * 32 + r) * D;
@@ -146,47 +153,60 @@ __global__ __launch_bounds__(64 * HPW * KW, D <= 128 && KW <= 2 ? 2 : 1) void pa
     }
 }
 
-// Folds the pieces of a sequence: grid (head x query tile x 4, sequence), a thread takes four columns of one of the eight
-// queries of a quarter tile, eight pieces' loads in flight at a time.
-template <typename T, int D>
-__global__ __launch_bounds__(2 * D) void paged_combine_f32_kernel(const PagedWideParams P)
+// Folds the pieces of a sequence: grid (head x query tile x 16, sequence), a thread takes four columns of one of two queries.
+// A chain of memory latencies: the loads of the first AHEAD pieces are on their way before the lengths say how many there are
+// (slots beyond them exist and are not used), the next AHEAD behind them; and a sequence's partials come in through many
+// CUs.  (Eight queries per workgroup and eight pieces at a time, behind the lengths: 1 x 1056 keys 5.2 us of 20.8 for the whole call, which is
+// 18.8 now together with the queries through LDS; 1 x 4000 37.3 -> 35.2, 1 x 12 000 58.5 -> 53.8, 2 x 900-2000 33.6 -> 31.1, 8 x 4000-9000
+// 198 -> 190.)
+constexpr int kFoldRows = 2, kFoldParts = 32 / kFoldRows;
+template <typename T, int D, int AHEAD>
+__global__ __launch_bounds__(kFoldRows * D / 4) void paged_combine_f32_kernel(const PagedWideParams P)
 {
-    const int quarter = blockIdx.x & 3, hq = blockIdx.x >> 2, b = blockIdx.y;
+    const int part = blockIdx.x % kFoldParts, hq = blockIdx.x / kFoldParts, b = blockIdx.y;
     const int qt = hq % P.nqt, head = hq / P.nqt;
-    const int s = quarter * 8 + threadIdx.x / (D / 4), d = threadIdx.x % (D / 4) * 4;
-    const int ctx = keys_of(P, b);
-    const int span = keys_per_piece(P, ctx, threadIdx.x & 63);
-    const int n = __builtin_amdgcn_readfirstlane((ctx + span - 1) / span);
+    const int s = part * kFoldRows + threadIdx.x / (D / 4), d = threadIdx.x % (D / 4) * 4;
     const int qrow = qt * 32 + s;
-    if (n <= 1 || qrow >= P.sq || d >= P.head_dim) return;      // one piece: written by the attention kernel
     const int64_t slot0 = (((int64_t)b * P.num_q_heads + head) * P.nqt + qt) * P.nsplit;
-    float M = kMinusBig, L = 0.f;
-    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int i0 = 0; i0 < n; i0 += 8) {
-        float m[8], l[8];
-        f32x4 po[8];
+    float m[AHEAD], l[AHEAD];
+    f32x4 po[AHEAD];
+    auto load = [&](int i0, int n) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < AHEAD; ++i) {
             const int64_t slot = slot0 + min(i0 + i, n - 1);
-            m[i] = i0 + i < n ? P.part_ml[(slot * 2 + 0) * 32 + s] : kMinusBig;
+            m[i] = P.part_ml[(slot * 2 + 0) * 32 + s];
             l[i] = P.part_ml[(slot * 2 + 1) * 32 + s];
             po[i] = *reinterpret_cast<const f32x4*>(P.part_o + (slot * 32 + s) * D + d);
         }
-        float Mn = M;
+    };
+    load(0, P.nsplit);
+    const int ctx = keys_of(P, b);
+    const int span = keys_per_piece(P, ctx, threadIdx.x & 63);
+    const int n = __builtin_amdgcn_readfirstlane((ctx + span - 1) / span);
+    if (n <= 1 || qrow >= P.sq || d >= P.head_dim) return;      // one piece: written by the attention kernel
+    float M = kMinusBig, L = 0.f;
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i0 = 0; i0 < n; i0 += AHEAD) {
+        if (i0 > 0) load(i0, n);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) Mn = fmaxf(Mn, m[i]);
-        const float keep = __builtin_amdgcn_exp2f(M - Mn);
-        L *= keep;
+        for (int g = 0; g < AHEAD; g += 8) {
+            if (i0 + g >= n) break;
+            float Mn = M;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[e] *= keep;
-        M = Mn;
+            for (int i = g; i < g + 8; ++i) Mn = fmaxf(Mn, i0 + i < n ? m[i] : kMinusBig);
+            const float keep = __builtin_amdgcn_exp2f(M - Mn);
+            L *= keep;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            if (i0 + i >= n) break;                             // (nothing of the others: 0 x infinity is not 0)
-            const float w = __builtin_amdgcn_exp2f(m[i] - M);
-            L += w * l[i];
+            for (int e = 0; e < 4; ++e) acc[e] *= keep;
+            M = Mn;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[e] += w * po[i][e];
+            for (int i = g; i < g + 8; ++i) {
+                if (i0 + i >= n) break;                         // (nothing of the others: 0 x infinity is not 0)
+                const float w = __builtin_amdgcn_exp2f(m[i] - M);
+                L += w * l[i];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[e] += w * po[i][e];
+            }
         }
     }
     const float inv = L > 0.f ? 1.0f / L : 0.f;                 // every key on an invalid page: zeros
@@ -223,7 +243,11 @@ int launch_groups(const PagedWideParams& P, hipStream_t stream)
     paged_attn_f32_kernel<T, D, HPW, KW><<<grid, 64 * HPW * KW, kLdsBytes, stream>>>(P);
     const int rc = mdx::check_launch("paged_block_attn (fp32 arithmetic)");
     if (rc != MDX_OK || P.nsplit == 1) return rc;
-    paged_combine_f32_kernel<T, D><<<dim3((unsigned)(P.num_q_heads * P.nqt * 4), (unsigned)P.bs), 2 * D, 0, stream>>>(P);
+    const dim3 fold((unsigned)(P.num_q_heads * P.nqt * kFoldParts), (unsigned)P.bs);
+    constexpr int kFoldThreads = kFoldRows * D / 4;
+    if (P.nsplit <= 8)       paged_combine_f32_kernel<T, D, 8><<<fold, kFoldThreads, 0, stream>>>(P);
+    else if (P.nsplit <= 16) paged_combine_f32_kernel<T, D, 16><<<fold, kFoldThreads, 0, stream>>>(P);
+    else                     paged_combine_f32_kernel<T, D, 24><<<fold, kFoldThreads, 0, stream>>>(P);     // (sixteen at a time: 1 x 4000 keys 36.8, 24: 35.2)
     return mdx::check_launch("paged_combine (fp32 arithmetic)");
 }
 

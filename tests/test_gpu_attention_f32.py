@@ -303,3 +303,9 @@ def test_fp32_prefill_keys_shared_by_one_two_or_four_wavefronts(dev, lens):
     """Both sides of the rule that splits a row tile's keys: full launches of short prompts, ragged ones in between, long chains."""
     _check(dev, lens, 32, 16, 8, 128, torch.float32, seed=sum(lens))
     _check(dev, lens[:4], 8, 4, 2, 96, torch.float32, seed=sum(lens) + 1)
+
+
+@pytest.mark.parametrize("ctx", [511, 513, 1024, 1030, 1536, 1540, 3100])
+def test_paged_fp32_as_many_pieces_as_are_folded_at_once_and_more(dev, ctx):
+    """Pieces of 64 keys: 8, 9, 16, 17, 24, 25 and 49 of them."""
+    _check_paged(dev, [ctx], 32, 4, 2, 128, torch.float32, seed=ctx)
