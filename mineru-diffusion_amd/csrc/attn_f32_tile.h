@@ -111,18 +111,19 @@ template <typename T, int D, int THREADS> struct TileRegs {
     }
 };
 
-// The 32 queries of each of HEADS heads on their way to LDS, where rows lie like those of a K tile, and from there to the lanes
-// as load_q has them.
-template <typename T, int D, int HEADS, int THREADS> struct QueryRegs {
-    static constexpr int kPasses = HEADS * 32 * (D / 4) / THREADS, kBytes = HEADS * 32 * Lds<D>::kPitchK * (int)sizeof(float);
+// TILES tiles of 32 queries on their way to LDS, where rows lie like those of a K tile, and from there to the lanes as load_q has them
+// (a lane's own row, 16 bytes at a time, touches every line eight times).
+template <typename T, int D, int TILES, int THREADS> struct QueryRegs {
+    static constexpr int kPasses = TILES * 32 * (D / 4) / THREADS, kBytes = TILES * 32 * Lds<D>::kPitchK * (int)sizeof(float);
     f32x4 x[kPasses];
-    // q: row 0 of the first head; rows_left: rows that there are (the others are zeros, as beyond the head's width)
-    __device__ __forceinline__ void fetch(const T* q, int64_t row_stride, int64_t head_stride, int rows_left, int tid, int width) {
+    // row_ptr(row): that row, or null (zeros, as beyond the head's width)
+    template <typename Row> __device__ __forceinline__ void fetch(int tid, int width, Row row_ptr) {
 #pragma unroll
         for (int p = 0; p < kPasses; ++p) {
-            const int u = tid + THREADS * p, row = u / (D / 4), col = 4 * (u % (D / 4));
+            const int u = tid + THREADS * p, col = 4 * (u % (D / 4));
+            const T* row = row_ptr(u / (D / 4));
             x[p] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (row % 32 < rows_left && col < width) x[p] = load4(q + (int64_t)(row % 32) * row_stride + (int64_t)(row / 32) * head_stride + col);
+            if (row && col < width) x[p] = load4(row + col);
         }
     }
     __device__ __forceinline__ void write(float* lds, int tid) const {
@@ -132,9 +133,9 @@ template <typename T, int D, int HEADS, int THREADS> struct QueryRegs {
             *reinterpret_cast<f32x4*>(lds + u / (D / 4) * Lds<D>::kPitchK + 4 * (u % (D / 4))) = x[p];
         }
     }
-    static __device__ __forceinline__ void read(float (&q)[D / 2], const float* lds, int head, int H, int r, int width) {
+    static __device__ __forceinline__ void read(float (&q)[D / 2], const float* lds, int tile, int H, int r, int width) {
         const int half = half_width(width);
-        const float* row = lds + (head * 32 + r) * Lds<D>::kPitchK + H * half;
+        const float* row = lds + (tile * 32 + r) * Lds<D>::kPitchK + H * half;
 #pragma unroll
         for (int m = 0; m < D / 8; ++m) {
             const f32x4 v = 4 * m < half ? *reinterpret_cast<const f32x4*>(row + 4 * m) : f32x4{0.f, 0.f, 0.f, 0.f};

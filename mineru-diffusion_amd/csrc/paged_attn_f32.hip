@@ -75,11 +75,10 @@ __global__ __launch_bounds__(64 * HPW * KW, D <= 128 && KW <= 2 ? 2 : 1) void pa
     const int kvh = (blockIdx.x / P.nqt) * HPW / P.heads_per_kv;
     const int width = P.head_dim;
 
-    // The workgroup's queries come through LDS too: a lane's own row, 16 bytes at a time, would touch every line eight times.
     QueryRegs<T, D, HPW, kThreads> queries;
     const int ctx = keys_of(P, b);
-    queries.fetch(static_cast<const T*>(P.q) + (int64_t)b * P.q_sb + (int64_t)(qt * 32) * P.q_ss + (int64_t)(head - hw) * P.q_sh, P.q_ss, P.q_sh,
-                  P.sq - qt * 32, tid, width);
+    const T* q0 = static_cast<const T*>(P.q) + (int64_t)b * P.q_sb + (int64_t)(qt * 32) * P.q_ss + (int64_t)(head - hw) * P.q_sh;
+    queries.fetch(tid, width, [&](int row) { return qt * 32 + row % 32 < P.sq ? q0 + (int64_t)(row % 32) * P.q_ss + (int64_t)(row / 32) * P.q_sh : nullptr; });
     const int span = P.nsplit > 1 ? keys_per_piece(P, ctx, lane) : max(1, ctx);
     const int n_pieces = max(1, (ctx + span - 1) / span);
     if (split >= n_pieces) return;

@@ -65,7 +65,10 @@ __global__ __launch_bounds__(kThreads, D <= 128 && KW <= 2 ? 2 : 1) void stairca
     const bool row_ok = ip >= pad && ip < Lp;
     const int64_t tok = (int64_t)seq0 + (ip - pad);
     float q[D / 2];
-    load_q<T, D>(q, row_ok ? static_cast<const T*>(P.q) + tok * P.q_st + (int64_t)head * P.q_sh : nullptr, H, width);
+    const T* qb = static_cast<const T*>(P.q) + ((int64_t)seq0 - pad) * P.q_st + (int64_t)head * P.q_sh;      // padded row 0
+    QueryRegs<T, D, kWaves / KW, kThreads> queries;
+    if constexpr (KW == 1) load_q<T, D>(q, row_ok ? qb + ip * P.q_st : nullptr, H, width);                   // (more of them than tiles in LDS)
+    else queries.fetch(tid, width, [&](int row) { const int i = row_g0 + row; return i >= pad && i < Lp ? qb + i * P.q_st : nullptr; });
 
     // exclusive key limit (padded coordinates) of a row
     auto limit_of = [&](int row) { return min(Lp, ((row >> P.log2_s) + 1) << P.log2_s); };
@@ -84,6 +87,12 @@ __global__ __launch_bounds__(kThreads, D <= 128 && KW <= 2 ? 2 : 1) void stairca
         regs.fetch(batch, tid, width, [&](int row) { return kb + tok_of(row) * P.k_st; }, [&](int row) { return vb + tok_of(row) * P.v_st; });
     };
     fetch(0, 0);
+    if constexpr (KW > 1) {
+        static_assert(queries.kBytes <= KW * Lds<D>::kBytes, "queries exceed the tile region");
+        queries.write(lds, tid);
+        __syncthreads();
+        queries.read(q, lds, wave / KW, H, r, width);
+    }
     for (int t = 0; t < n_tiles; t += KW) {
         __syncthreads();                                       // the previous tiles have been read by everybody
 #pragma unroll
