@@ -206,7 +206,7 @@ __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
     // 2^-24 |m c|, into every term (1e-3 at logits of thousands).
     float m = kNegBig, s = 0.f, h = 0.f;
     int first_at = -1;           // element (counted from the first aligned chunk) that first held m
-    auto take_values = [&](const float (&x)[EPC], int64_t chunk) -> float {     // returns the chunk's largest element
+    auto take_values = [&](const float (&x)[EPC], int first) -> float {         // of the chunk from element `first` on; returns the largest
         float cm = x[EPC - 1];
 #pragma unroll
         for (int i = 0; i + 2 < EPC; i += 2) cm = max3(cm, x[i], x[i + 1]);
@@ -217,7 +217,7 @@ __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
             int j = EPC - 1;
 #pragma unroll
             for (int i = EPC - 2; i >= 0; --i) if (x[i] == cm) j = i;
-            first_at = (int)chunk * EPC + j;
+            first_at = first + j;
             const float h_new = -(cm * c);
             s = s > 0.f ? s * fast_exp2(h_new - h) : 0.f;   // h_new <= h once a finite maximum exists
             m = cm;
@@ -240,7 +240,7 @@ __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
         auto take = [&](const u32x4 u, int64_t chunk) {
             float x[EPC];
             unpack(u, x);
-            take_values(x, chunk);
+            take_values(x, (int)chunk * EPC);
         };
         int64_t ch = cbeg + tid;
         // Main loop: the next group's kUnroll loads are issued before this group is reduced, so a lane
@@ -294,21 +294,33 @@ __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
             const float v = (unit_T ? x : x / T_) + g;
             if (v > best || (v == best && index < best_idx)) { best = v; best_x = x; best_idx = index; }
         };
+        // No less than x / T, for the tests below: the reciprocal and the product are off by 2^-24 of it each.  (One instruction per
+        // chunk more than the product instead of the ten of a division; with 32-bit counts in the loop, which is bound by its
+        // instructions from 256 rows on: 768 rows 89.5 -> 87.3 us for the step, 1024 114 -> 111.5; 32 to 160 rows level.)
+        const float inv_T = 1.0f / T_;
+        const bool plain_T = inv_T > 1e-30f && inv_T < 1e30f;
+        auto at_most = [&](float x) {
+            const float l = plain_T ? x * inv_T : x / T_;
+            return __builtin_fmaf(fabsf(l), 4.76837158203125e-07f, l);
+        };
         auto noise_at = [&](int64_t e) { return NOISE == 1 ? np[e] : rn.at((int)e); };
         // The chunks after this one are on their way while it is worked on: few wavefronts share a SIMD here (96 rows:
         // three), and where the noise of a chunk is skipped there is little else to hide a trip to HBM behind.
+        const u32x4* part = cp + cbeg;
+        const uint32_t chunks = (uint32_t)max(cend - cbeg, (int64_t)0);
+        const int e0 = (int)cbeg * EPC;                          // element, counted from the first aligned chunk, that the part begins with
         u32x4 next[kUnroll];
 #pragma unroll
         for (int k = 0; k < kUnroll; ++k)
-            if (cbeg + tid + k * kThreads < cend) next[k] = __builtin_nontemporal_load(cp + cbeg + tid + k * kThreads);
-        for (int64_t ch = cbeg + tid; ch < cend; ch += kThreads) {
+            if (tid + k * kThreads < chunks) next[k] = __builtin_nontemporal_load(part + tid + k * kThreads);
+        for (uint32_t at = (uint32_t)tid; at < chunks; at += kThreads) {
             float x[EPC];
             unpack(next[0], x);
 #pragma unroll
             for (int k = 0; k + 1 < kUnroll; ++k) next[k] = next[k + 1];
-            if (ch + kUnroll * kThreads < cend) next[kUnroll - 1] = __builtin_nontemporal_load(cp + ch + kUnroll * kThreads);
-            const float cmx = take_values(x, ch);
-            const int c0 = (int)(lead + ch * EPC);
+            if (at + kUnroll * kThreads < chunks) next[kUnroll - 1] = __builtin_nontemporal_load(part + at + kUnroll * kThreads);
+            const float cmx = take_values(x, e0 + (int)at * EPC);
+            const int c0 = (int)lead + e0 + (int)at * EPC;
             // No draw of the generator exceeds kGumbelMax, and rounding is monotonic: an element of this chunk can
             // take (or tie) the row's lead only if (largest element) / T + kGumbelMax reaches the best noisy logit
             // that anybody in the workgroup has found so far (lead_seen: published by the wavefronts as they go; an
@@ -320,7 +332,7 @@ __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
                 ++since_look;                          // the others' news at chunks 1, 2, 4, 8, 16, 24, ...: an LDS read per chunk would cost what it saves
                 if ((since_look & min(since_look - 1, 7)) == 0)
                     seen = fmaxf(seen, __hip_atomic_load(&lead_seen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
-                const bool may_lead = (unit_T ? cmx : cmx / T_) + kGumbelMax >= fmaxf(best, seen);
+                const bool may_lead = at_most(cmx) + kGumbelMax >= fmaxf(best, seen);
                 if (__builtin_amdgcn_ballot_w64(may_lead) == 0) continue;
             }
             if (NOISE == 1) {
@@ -348,7 +360,7 @@ __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
                 // j <= e^-need 2^23 matter: at need = 10, one in 22 000.  need is taken 0.02 + 2^-22 |lead| lower than
                 // computed, which covers the error of the hardware logarithms (2e-6) and every rounding on the way.
                 const float lim = fmaxf(best, seen);
-                const float need = lim - (unit_T ? cmx : cmx / T_) - __builtin_fmaf(fabsf(lim), 2.384185791015625e-07f, 0.02f);
+                const float need = lim - at_most(cmx) - __builtin_fmaf(fabsf(lim), 2.384185791015625e-07f, 0.02f);
                 const float reach = fminf(fast_exp2(__builtin_fmaf(-kLog2e, need, 23.f)), 8388608.f);    // NaN (lead and element both infinite) -> the other operand
                 uint32_t top = 0;
 #pragma unroll

@@ -216,3 +216,19 @@ def test_seeded_sampling_with_every_split_count(dev, bs, S):
     x0n, pn = mdx.confidence_argmax(logits, temps, noise=mdx.gumbel_noise(bs * S, V, 11, 3, device=dev).view(bs, S, V))
     assert torch.equal(x0, x0n)
     torch.testing.assert_close(p, pn, rtol=3e-6, atol=0)
+
+
+@pytest.mark.parametrize("scale,temps", [(1e-6, [1e-6, 3e-7, 0.9e-30]), (3e4, [0.3, 1.7, 1e4]), (1e30, [3.3e29, 1.1e30, 0.7]), (1.0, [1e-38, 1e31, 3e38])])
+def test_seeded_sampling_at_any_temperature(dev, scale, temps):
+    """The tests that spare the generator compare with (largest element) / T from a reciprocal, rounded up; temperatures whose
+    reciprocal is huge or tiny are divided by.  Picks must be those of the tensor-noise path, which divides and skips nothing."""
+    import mdx
+    g = torch.Generator().manual_seed(5)
+    bs, S, V = 3, 8, 30000
+    logits = (torch.randn(bs, S, V, generator=g) * scale).to(dev)
+    t = torch.tensor(temps, device=dev)
+    for offset in range(3):
+        x0, _ = mdx.confidence_argmax(logits, t, seed=3, offset=offset)
+        noise = mdx.gumbel_noise(bs * S, V, 3, offset, device=dev)
+        x0n, _ = mdx.confidence_argmax(logits, t, noise=noise.view(bs, S, V))
+        assert torch.equal(x0, x0n)
