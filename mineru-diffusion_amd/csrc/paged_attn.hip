@@ -513,41 +513,36 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
     if (tid == 0) __hip_atomic_store(counter, 0.f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // ready for the next launch
 }
 
-// Folds the split partials: a workgroup takes 8 QUERIES queries of a (sequence, head), a thread four columns of QUERIES of them.  The
-// kernel is a chain of memory latencies (length -> partials -> output), not of bytes: the loads of the first slots are
+// Folds the split partials: a workgroup takes ROWS queries of a (sequence, head), a thread four columns of one of them.  The
+// kernel is a chain of memory latencies (length -> partials -> output), not of bytes: the loads of the first AHEAD slots are
 // on their way before the lengths say how many of them exist (where a slot lies does not depend on it; what lies
-// beyond is masked out), and a thread's share of a slot is one load.  Few heads (QUERIES = 1) get eight or twelve slots in flight and
-// more workgroups; with more of them there are workgroups enough, fewer pieces per sequence, and the workgroups of whole
-// sequences, which leave at once, still have to be launched.  (A workgroup per head with 16 columns per thread, the form this
+// beyond is masked out), and a thread's share of a slot is one load.  (A workgroup per head with 16 columns per thread, the form this
 // replaced, took 0.6 us per four pieces of a sequence, which kept the pieces long.)
-template <typename E, int QUERIES, int AHEAD>
-__global__ __launch_bounds__(256) void paged_combine_kernel(const PagedParams P)
+template <typename E, int AHEAD, int ROWS>
+__global__ __launch_bounds__(32 * ROWS) void paged_combine_kernel(const PagedParams P)
 {
-    constexpr int kAhead = AHEAD, kParts = 4 / QUERIES;
+    constexpr int kParts = kQTile / ROWS;
     const int part = blockIdx.x % kParts, rest = blockIdx.x / kParts;
     const int qt = rest % P.nqt, hq = (rest / P.nqt) % P.num_q_heads, b = rest / P.nqt / P.num_q_heads;
-    const int c = (threadIdx.x & 31) * 4, s0 = part * 8 * QUERIES + (threadIdx.x >> 5);         // queries s0, s0 + 8
-    if (c >= P.head_dim || qt * kQTile + s0 >= P.sq) return;
+    const int c = (threadIdx.x & 31) * 4, s = part * ROWS + (threadIdx.x >> 5);
+    if (c >= P.head_dim || qt * kQTile + s >= P.sq) return;
     const int64_t slot0 = (((int64_t)b * P.num_q_heads + hq) * P.nqt + qt) * P.nsplit;
-    const float* part_o = P.part_o + (slot0 * kQTile + s0) * kHeadDim + c;
-    const float2* part_ml = reinterpret_cast<const float2*>(P.part_ml) + slot0 * kQTile + s0;
+    const float* part_o = P.part_o + (slot0 * kQTile + s) * kHeadDim + c;
+    const float2* part_ml = reinterpret_cast<const float2*>(P.part_ml) + slot0 * kQTile + s;
     int nv = P.nsplit;                         // until the lengths are in: every slot that exists
-    Fold<4> F[QUERIES];
+    Fold<4> F;
+    F.init();
+    for (int i0 = 0; i0 < nv; i0 += AHEAD) {
+        float m[AHEAD / 4][4], l[AHEAD / 4][4];
+        f32x4 po[AHEAD / 4][4][1];
 #pragma unroll
-    for (int q = 0; q < QUERIES; ++q) F[q].init();
-    for (int i0 = 0; i0 < nv; i0 += kAhead) {
-        float m[QUERIES][kAhead / 4][4], l[QUERIES][kAhead / 4][4];
-        f32x4 po[QUERIES][kAhead / 4][4][1];
-#pragma unroll
-        for (int i = 0; i < kAhead; ++i)
-#pragma unroll
-            for (int q = 0; q < QUERIES; ++q) {
-                const int slot = min(i0 + i, P.nsplit - 1);
-                const float2 ml = part_ml[slot * kQTile + 8 * q];
-                m[q][i / 4][i % 4] = ml.x;
-                l[q][i / 4][i % 4] = ml.y;
-                po[q][i / 4][i % 4][0] = *reinterpret_cast<const f32x4*>(part_o + ((int64_t)slot * kQTile + 8 * q) * kHeadDim);
-            }
+        for (int i = 0; i < AHEAD; ++i) {
+            const int slot = min(i0 + i, P.nsplit - 1);
+            const float2 ml = part_ml[slot * kQTile];
+            m[i / 4][i % 4] = ml.x;
+            l[i / 4][i % 4] = ml.y;
+            po[i / 4][i % 4][0] = *reinterpret_cast<const f32x4*>(part_o + (int64_t)slot * kQTile * kHeadDim);
+        }
         if (i0 == 0) {
             const int ctx = min(P.context_lens[b], P.max_pages * P.page_size);
             const int span = P.span_out ? (int)*P.span_out : P.chunk;     // the attention kernel's choice
@@ -555,21 +550,14 @@ __global__ __launch_bounds__(256) void paged_combine_kernel(const PagedParams P)
             if (nv <= 1) return;               // written directly by the attention kernel
         }
 #pragma unroll
-        for (int g = 0; g < kAhead / 4; ++g)
-#pragma unroll
-            for (int q = 0; q < QUERIES; ++q)
-                if (i0 + 4 * g < nv) F[q].take4(m[q][g], l[q][g], po[q][g], nv - i0 - 4 * g);
+        for (int g = 0; g < AHEAD / 4; ++g)
+            if (i0 + 4 * g < nv) F.take4(m[g], l[g], po[g], nv - i0 - 4 * g);
     }
+    const float inv = F.inverse();
+    typename Elem16<E>::vec4 out;
 #pragma unroll
-    for (int q = 0; q < QUERIES; ++q) {
-        const int s = s0 + 8 * q;
-        if (qt * kQTile + s >= P.sq) return;
-        const float inv = F[q].inverse();
-        typename Elem16<E>::vec4 out;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) out[e] = (E)(F[q].acc[e] * inv);
-        *reinterpret_cast<typename Elem16<E>::vec4*>(P.o + (int64_t)b * P.o_sb + (int64_t)(qt * kQTile + s) * P.o_ss + (int64_t)hq * P.o_sh + c) = out;
-    }
+    for (int e = 0; e < 4; ++e) out[e] = (E)(F.acc[e] * inv);
+    *reinterpret_cast<typename Elem16<E>::vec4*>(P.o + (int64_t)b * P.o_sb + (int64_t)(qt * kQTile + s) * P.o_ss + (int64_t)hq * P.o_sh + c) = out;
 }
 
 // Keys per split.  Measured over batches of 4 to 64 sequences and contexts of 300 to 8000 keys, the
@@ -762,15 +750,25 @@ int launch_paged(const void* q, void* o, const void* k_cache, const void* v_cach
     }
     int rc = mdx::check_launch("paged_block_attn");
     if (rc != MDX_OK || !two_launches) return rc;
-    // The slots asked for at once: eight, or twelve where the sequences of tables that are 65 % full have about as many pieces or up to
+    // The slots asked for at once.  Many heads: four (sequences of so many have few pieces, and workgroups enough to wait beside each other;
+    // with two queries per thread and half the workgroups, 9 x 1000-3000 keys took 34.8 us, this way 33.7, 16 x 512-4096 43.9 and 42.8).
+    // Few: eight, or twelve where the sequences of tables that are 65 % full have about as many pieces or up to
     // half as many again.  (One sequence of 1337 keys, twelve against eight: 14.8 and 15.3 us, 1000: 14.2 and 14.7, two of 3000 to 3500:
     // 21.4 and 21.9, three of 3000 to 5000: 25.3 and 25.9; but one of 300: 12.3 and 12.1, of 2500: 17.2 and 16.9.)
     const double pieces = sqrt(0.65 * max_pages * page_size / bs) / kPieceRoot;
+    // Up to 64 heads: two queries per workgroup, so that the partials come in through many CUs (one sequence of 1337 keys 14.6 -> 14.3 us, of
+    // 4000 19.2 -> 18.5, four of 1000 to 3000 23.5 -> 23.2; eight of those 29.9 and 30.6).
+    const bool twelve = pieces > 7 && pieces <= 9.5;
     auto combine = [&](auto element) {
         typedef decltype(element) E;
-        if (n_heads > 128) paged_combine_kernel<E, 2, 4><<<2 * n_heads, 256, 0, stream>>>(P);
-        else if (pieces > 7 && pieces <= 9.5) paged_combine_kernel<E, 1, 12><<<4 * n_heads, 256, 0, stream>>>(P);
-        else paged_combine_kernel<E, 1, 8><<<4 * n_heads, 256, 0, stream>>>(P);
+        if (n_heads <= 64) {
+            if (twelve) paged_combine_kernel<E, 12, 2><<<kQTile / 2 * n_heads, 64, 0, stream>>>(P);
+            else        paged_combine_kernel<E, 8, 2><<<kQTile / 2 * n_heads, 64, 0, stream>>>(P);
+        } else {
+            if (n_heads > 128) paged_combine_kernel<E, 4, 8><<<kQTile / 8 * n_heads, 256, 0, stream>>>(P);
+            else if (twelve)   paged_combine_kernel<E, 12, 8><<<kQTile / 8 * n_heads, 256, 0, stream>>>(P);
+            else               paged_combine_kernel<E, 8, 8><<<kQTile / 8 * n_heads, 256, 0, stream>>>(P);
+        }
     };
     if (dtype == MDX_F16) combine(_Float16()); else combine(__bf16());
     return mdx::check_launch("paged_combine");
