@@ -101,7 +101,9 @@ __global__ __launch_bounds__(64 * HPW * KW, D <= 128 && KW <= 2 ? 2 : 1) void pa
         // ---- tiles t0 .. t0 + KW - 1 into LDS, all threads on each (a tile never straddles a page: page_size % 32 == 0, so that all
         //      its rows exist in memory, whatever they hold) ----
         unsigned tile_ok = 0;                                  // bit i: tile t0 + i exists and lies on a valid page (uniform)
-        constexpr int kTogether = KW == 4 ? 4 : 1;             // tiles whose loads are in flight together: as registers allow
+        // tiles whose loads are in flight together: as registers allow (two instead of one at 128 columns: 8 x 4000-9000 keys
+            // 192 -> 186 us, 1 x 4000 35.2 -> 34.4, 1 x 1056 and shorter level)
+            constexpr int kTogether = KW == 4 ? 4 : D <= 128 ? KW : 1;
         TileRegs<T, D, kThreads> regs[kTogether];
 #pragma unroll
         for (int i0 = 0; i0 < KW; i0 += kTogether) {
