@@ -1,6 +1,6 @@
 // The fused vocabulary projection for few rows (up to 128: a decode pass of one to four sequences, or what is left masked of
 // more): logits x . W^T, rounded to bf16, reduced to (max, sum of exp, first argmax) in registers.  With so few rows it is a read
-// of W (622 MB at 151 936 x 2048), so it is built like the linear layers of decode_linear.hip: fragments of W straight
+// of W (622 MB at 151 936 x 2048): fragments of W straight
 // from memory into registers, x through LDS without passing registers.  One workgroup per CU walks the vocabulary in tiles of
 // 128 rows without a pause between tiles; a lane keeps the running state of its rows of x over all its logits, so that a
 // workgroup leaves one record per row at its end and the fold over the records is short.
@@ -10,8 +10,8 @@
 //  * otherwise x goes through LDS K step by K step with a barrier per step, W one step ahead.
 //
 // W is read with ordinary loads: marked nontemporal, the two loads that share a 128-byte line fetch it twice now and then (139
-// against 129 us at 32 rows).  Bound: HBM.  us at 16 / 32 / 64 / 128 rows: 119 / 120 / 140 / 170 (5.2 TB/s at 32 rows); the tiles of 256 rows of
-// lm_head_unmask.hip 200 / 199 / 208 / 200, the library's product and a vocabulary pass 213 / 155 / 161 / 175.
+// against 129 us at 32 rows).  Bound: HBM.  us at 16 / 32 / 64 / 128 rows: 119 / 120 / 140 / 170 (5.2 TB/s at 32 rows); tiles of 256 rows
+// 200 / 199 / 208 / 200, the library's product and a vocabulary pass 213 / 155 / 161 / 175.
 #include "lm_head.h"
 #include <atomic>
 
