@@ -203,6 +203,23 @@ int mdx_paged_block_attn_single_launch(const void* q, void* o, const void* k_cac
                                        void* counters, int64_t counter_bytes, mdx_stream_t stream);
 
 /*
+ * mdx_paged_block_attn (counters null) or mdx_paged_block_attn_single_launch, in a decode pass: next and then are memory that the launches
+ * behind it read (the weights of the output and of the gate/up projection).  While the attention of up to 256 rows (bs * Sq) leaves
+ * most of the chip idle, workgroups of the same launch read as much of it as pays, which leaves it in the device's cache; nothing depends on it, and
+ * other launches take no notice.  16-byte aligned, sizes multiples of 16 bytes, null with a size of 0; valid and not written while the launch runs.
+ */
+int mdx_paged_block_attn_read_ahead(const void* q, void* o, const void* k_cache, const void* v_cache,
+                                    int64_t q_stride_b, int64_t q_stride_s, int64_t q_stride_h,
+                                    int64_t o_stride_b, int64_t o_stride_s, int64_t o_stride_h,
+                                    int64_t cache_stride_page, int64_t cache_stride_tok, int64_t cache_stride_head,
+                                    const int32_t* block_table, int64_t bt_stride, const int32_t* context_lens,
+                                    int32_t bs, int32_t sq, int32_t num_q_heads, int32_t num_kv_heads,
+                                    int32_t head_dim, int32_t max_pages, int32_t page_size, int64_t num_pages,
+                                    float scale, int32_t dtype,
+                                    void* workspace, int64_t workspace_bytes, void* counters, int64_t counter_bytes,
+                                    const void* next, int64_t next_bytes, const void* then, int64_t then_bytes, mdx_stream_t stream);
+
+/*
  * mdx_paged_block_attn for callers that CANNOT ALLOCATE (code under HIP graph capture without an
  * allocator, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in
  * the reference, whose call sites allocate freely.  Same arguments, kernels and results (bit for

@@ -553,7 +553,7 @@ Tensor counters_for(const Tensor& like, int64_t bytes) {
 // counters: None = single launch with this module's counters, False = two launches, a tensor = the caller's.
 // The result as [bs, Sq, Hq, d], or flattened to [bs, Sq, Hq * d].
 Tensor paged(const Tensor& q_, const Tensor& k_cache, const Tensor& v_cache, const Tensor& lens_, const Tensor& bt_, PyObject* scale,
-             PyObject* counters_arg, bool flat) {
+             PyObject* counters_arg, bool flat, const Tensor* next = nullptr, const Tensor* then = nullptr) {
     need_gpu({&q_, &k_cache, &v_cache, &lens_, &bt_});
     NEED(q_.dim() == 4 && k_cache.dim() == 4 && v_cache.sizes() == k_cache.sizes());
     NEED(q_.scalar_type() == k_cache.scalar_type() && q_.scalar_type() == v_cache.scalar_type());
@@ -582,6 +582,15 @@ Tensor paged(const Tensor& q_, const Tensor& k_cache, const Tensor& v_cache, con
                   static_cast<const int32_t*>(ptr(lens)), (int32_t)bs, (int32_t)sq, (int32_t)hq, (int32_t)hkv, (int32_t)d, (int32_t)bt.size(1),
                   (int32_t)page, num_pages, scale_or_default(scale, d), dtype_of(q), ptr_or_null(ws), bytes, more...);
     };
+    if (next) {                             // (what does not lie in one piece of whole 16 bytes is not read ahead)
+        auto bytes_of = [&](const Tensor& t) -> int64_t {
+            return t.is_contiguous() && t.device() == q.device() && reinterpret_cast<uintptr_t>(ptr(t)) % 16 == 0 ? t.nbytes() / 16 * 16 : 0;
+        };
+        const int64_t n0 = bytes_of(*next), n1 = bytes_of(*then);
+        check(call(mdx_paged_block_attn_read_ahead, ptr_or_null(counters), counters.defined() ? counters.numel() * 4 : 0, n0 ? ptr(*next) : nullptr, n0,
+                   n1 ? ptr(*then) : nullptr, n1, stream_of(q)), "flash_attn_with_kvcache");
+        return o;
+    }
     check(counters.defined() ? call(mdx_paged_block_attn_single_launch, ptr(counters), counters.numel() * 4, stream_of(q))
                              : call(mdx_paged_block_attn, stream_of(q)),
           "flash_attn_with_kvcache");
@@ -593,6 +602,15 @@ PyObject* flash_attn_with_kvcache(PyObject*, PyObject* const* a, Py_ssize_t n) {
     ARGS(7);
     return guarded([&]() -> PyObject* {
         return wrap(paged(tensor(a[0]), tensor(a[1]), tensor(a[2]), tensor(a[3]), tensor(a[4]), a[5], a[6], false));
+    });
+}
+
+// q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale | None, the weights of the two products behind the call
+PyObject* flash_attn_with_kvcache_read_ahead(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    ARGS(8);
+    return guarded([&]() -> PyObject* {
+        const Tensor &next = tensor(a[6]), &then = tensor(a[7]);
+        return wrap(paged(tensor(a[0]), tensor(a[1]), tensor(a[2]), tensor(a[3]), tensor(a[4]), a[5], Py_None, false, &next, &then));
     });
 }
 
@@ -900,7 +918,7 @@ PyObject* sampler_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyMethodDef methods[] = {
     ENTRY(store_kvcache), ENTRY(store_kvcache_maybe4d), ENTRY(qk_norm_rope_store), ENTRY(rms_norm), ENTRY(silu_and_mul), ENTRY(linear), ENTRY(linear_gated), ENTRY(linear_qk_norm_rope_store), ENTRY(linear_partials), ENTRY(linear_silu),
     ENTRY(rms_norm_partials), ENTRY(qk_norm_rope_store_partials), ENTRY(sparse_attn_varlen),
-    ENTRY(flash_attn_with_kvcache), ENTRY(attention_prefill), ENTRY(attention_decode), ENTRY(confidence_argmax), ENTRY(lm_head_confidence),
+    ENTRY(flash_attn_with_kvcache), ENTRY(flash_attn_with_kvcache_read_ahead), ENTRY(attention_prefill), ENTRY(attention_decode), ENTRY(confidence_argmax), ENTRY(lm_head_confidence),
     ENTRY(filter_logits), ENTRY(select_transfer), ENTRY(unmask_step), ENTRY(sampler_step),
     {nullptr, nullptr, 0, nullptr},
 };

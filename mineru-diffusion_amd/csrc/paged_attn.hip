@@ -123,6 +123,34 @@ struct PagedParams {
     float* arrive;
 };
 
+// Weights that the launches behind this one read.  An attention launch of a few sequences leaves most of the chip idle and HBM nearly
+// so for 8 to 15 us, while the products behind it get W from HBM at half of its rate: a CU's loads come back in order, and
+// rows of x from L2 wait behind rows of W.  Read once before, W is in the memory-side cache (256 MB), from where the gate/up projection of 128 rows takes
+// 12.6 us instead of 19.6, of 32 rows 9.6 instead of 14.
+struct ReadAhead {
+    const u32x4* p[2]; int n[2];                    // 16-byte elements
+    int first_y;                                    // blockIdx.y from which workgroups read
+};
+__device__ __forceinline__ bool is_reader(const ReadAhead& A) { return (int)blockIdx.y >= A.first_y; }
+template <int THREADS> __device__ __forceinline__ void read_ahead(const ReadAhead& A) {
+    constexpr int kTogether = 8;
+    const int step = ((int)gridDim.y - A.first_y) * (int)gridDim.x * THREADS;
+    u32x4 all = {0, 0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        int i = (((int)blockIdx.y - A.first_y) * (int)gridDim.x + (int)blockIdx.x) * THREADS + (int)threadIdx.x;
+        for (; i + (kTogether - 1) * step < A.n[k]; i += kTogether * step) {
+            u32x4 x[kTogether];
+#pragma unroll
+            for (int u = 0; u < kTogether; ++u) x[u] = A.p[k][i + u * step];
+#pragma unroll
+            for (int u = 0; u < kTogether; ++u) all ^= x[u];
+        }
+        for (; i < A.n[k]; i += step) all ^= A.p[k][i];
+    }
+    asm volatile("" :: "v"(all));                   // (the loads have a use)
+}
+
 // Running fold of split partials over COLS columns of one query.
 template <int COLS> struct Fold {
     float M, L, acc[COLS];
@@ -200,9 +228,13 @@ __device__ __forceinline__ void combine_query(const PagedParams& P, int b, int h
 // WAVES = 4 (two workgroups per CU) or 8 (one workgroup per CU, 128-key tiles: for launches with about
 // one workgroup per CU, where a CU would otherwise hold four wavefronts only).  Tiles hold 32 keys per
 // key slice (WAVES / HPW slices); two 64-key tile buffers fit a CU twice, two 128-key ones once.
-template <typename E, int HPW, int DEPTH, int WAVES>
-__global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_block_attn_kernel(const PagedParams P)
+// AHEAD: none, or ReadAhead: workgroups behind those of the attention read what the launches behind it need.
+template <typename E, int HPW, int DEPTH, int WAVES, typename... AHEAD>
+__global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_block_attn_kernel(const PagedParams P, const AHEAD... ahead)
 {
+    if constexpr (sizeof...(AHEAD) > 0) {
+        if (is_reader(ahead...)) { read_ahead<64 * WAVES>(ahead...); return; }
+    }
     constexpr int kThreads = 64 * WAVES;
     constexpr int kRowsPerPass = kThreads / 16;     // LDS rows one pass of the workgroup stages
     constexpr int kPassesPerSlice = 32 / kRowsPerPass;
@@ -317,7 +349,13 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
     WaveState<1> st;
     st.init();
 
-    const int32_t* bt = P.block_table + (int64_t)b * P.bt_stride;
+    // (with the readers' loads in the kernel the compiler no longer takes the table for constant by itself)
+    typedef __attribute__((address_space(4))) const int32_t ConstantEntry;
+    auto table_row = [&] {
+        const int32_t* row = P.block_table + (int64_t)b * P.bt_stride;
+        if constexpr (sizeof...(AHEAD) > 0) return (ConstantEntry*)(uintptr_t)row; else return row;
+    };
+    const auto bt = table_row();
     const int chunk = tid & 15, trow = tid >> 4;    // one pass stages kRowsPerPass rows
     const int n_tiles = (key_end - key_begin + kTileKeys - 1) / kTileKeys;
     // kRowsPerPass (16 or 32) consecutive keys starting at a multiple of that never straddle a page (page_size % 32 == 0):
@@ -560,6 +598,10 @@ __global__ __launch_bounds__(32 * ROWS) void paged_combine_kernel(const PagedPar
     *reinterpret_cast<typename Elem16<E>::vec4*>(P.o + (int64_t)b * P.o_sb + (int64_t)(qt * kQTile + s) * P.o_ss + (int64_t)hq * P.o_sh + c) = out;
 }
 
+// Reading ahead: rows of a pass, and what is read at most.
+constexpr int64_t kReadAheadFewRows = 32, kReadAheadRows = 256;
+constexpr int64_t kReadAheadFewBytes = (int64_t)32 << 20, kReadAheadBytes = (int64_t)64 << 20;
+
 // Keys per split.  Measured over batches of 4 to 64 sequences and contexts of 300 to 8000 keys, the
 // kernel is fastest with 1.5 to 1.8 workgroups per CU in total (just under the two per CU that are
 // resident at once: one round, no tail of late workgroups), with splits of at least 512 keys (a
@@ -640,8 +682,8 @@ int launch_paged_f32(const void* q, void* o, const void* k_cache, const void* v_
                      int32_t head_dim, int32_t max_pages, int32_t page_size, int64_t num_pages,
                      float scale, int32_t dtype, void* workspace, int64_t workspace_bytes, hipStream_t stream);   // paged_attn_f32.hip
 
-// The launch behind every paged entry point of the library.
-int launch_paged(const void* q, void* o, const void* k_cache, const void* v_cache,
+// The launch behind every paged entry point of the library.  next, then: what the launches behind it read.
+int launch_paged_ahead(const void* q, void* o, const void* k_cache, const void* v_cache,
                  int64_t q_stride_b, int64_t q_stride_s, int64_t q_stride_h,
                  int64_t o_stride_b, int64_t o_stride_s, int64_t o_stride_h,
                  int64_t cache_stride_page, int64_t cache_stride_tok, int64_t cache_stride_head,
@@ -650,9 +692,12 @@ int launch_paged(const void* q, void* o, const void* k_cache, const void* v_cach
                  int32_t head_dim, int32_t max_pages, int32_t page_size, int64_t num_pages,
                  float scale, int32_t dtype,
                  void* workspace, int64_t workspace_bytes, bool single_launch, void* counters, int64_t counter_bytes,
-                 mdx_stream_t stream_)
+                 const void* next, int64_t next_bytes, const void* then, int64_t then_bytes, mdx_stream_t stream_)
 {
     hipStream_t stream = static_cast<hipStream_t>(stream_);
+    MDX_REQUIRE(next_bytes >= 0 && then_bytes >= 0 && (next || next_bytes == 0) && (then || then_bytes == 0) && next_bytes % 16 == 0 &&
+                then_bytes % 16 == 0 && mdx::aligned16(next) && mdx::aligned16(then), MDX_EINVAL,
+                "paged_block_attn: what is read ahead starts at and is a multiple of 16 bytes");
     MDX_REQUIRE(bs >= 0 && sq >= 0 && max_pages >= 0 && num_pages >= 0, MDX_EINVAL, "paged_block_attn: negative size");
     MDX_REQUIRE(dtype == MDX_BF16 || dtype == MDX_F16 || dtype == MDX_F32, MDX_EUNSUPPORTED, "paged_block_attn: dtype %d (bf16, fp16 or fp32)", dtype);
     // 16-bit elements and heads of 16, 32, ..., 128 columns run on the 16-bit matrix instructions; fp32 tensors and
@@ -738,13 +783,29 @@ int launch_paged(const void* q, void* o, const void* k_cache, const void* v_cach
     // on equal lengths); with more pairs than CUs the second round costs more than that gains.
     const bool eight = device_span && (int64_t)bs * wg_per_pair <= cus;
     const unsigned n_heads = (unsigned)(bs * num_q_heads * P.nqt);
+    // Reading ahead, by rows of the pass (kReadAhead*): engine, ms per generation without / with, contexts of 1088 and more: one request 68.0 / 66.2, two 79.8 /
+    // 78.2, three 96.1 / 91.0, four 100.2 / 95.9, six 121.8 / 119.8, eight 132.8 / 130.7; of 32: one 61.6 / 60.7, four 82.2 / 77.9, eight 98.1 / 96.7.  More
+    // rows: 16 requests 190.3 / 190.7 (the attention streams by itself then, and the products are bound by other things).  32 rows have the
+    // shortest attention: all of 56 MB there 68.6, a workgroup on every other CU and 32 MB 66.2.
+    ReadAhead A{};
+    int64_t budget = 0;
+    int readers = 0;
+    const int64_t pass_rows = (int64_t)bs * sq;
+    if (next_bytes + then_bytes > 0 && dtype == MDX_BF16 && HPW == 2 && !eight && pass_rows <= kReadAheadRows) {
+        budget = pass_rows <= kReadAheadFewRows ? kReadAheadFewBytes : kReadAheadBytes;
+        readers = (int)((pass_rows <= kReadAheadFewRows ? cus / 2 : cus) / wg_per_pair);
+        const int64_t n0 = next_bytes < budget ? next_bytes : budget, n1 = then_bytes < budget - n0 ? then_bytes : budget - n0;
+        A = ReadAhead{{static_cast<const u32x4*>(next), static_cast<const u32x4*>(then)}, {(int)(n0 / 16), (int)(n1 / 16)}, pairs_y};
+    }
+    if (pairs_y + readers > 65535) readers = 0;
     const bool two_launches = P.nsplit > 1 && !P.arrive;
     if (dtype == MDX_F16) {
         if (HPW == 2 && eight) paged_block_attn_kernel<_Float16, 2, 2, 8><<<grid, 512, 0, stream>>>(P);
         else if (HPW == 2)     paged_block_attn_kernel<_Float16, 2, 2, 4><<<grid, 256, 0, stream>>>(P);
         else                   paged_block_attn_kernel<_Float16, 1, 1, 4><<<grid, 256, 0, stream>>>(P);
     } else {
-        if (HPW == 2 && eight) paged_block_attn_kernel<__bf16, 2, 2, 8><<<grid, 512, 0, stream>>>(P);
+        if (readers > 0)       paged_block_attn_kernel<__bf16, 2, 2, 4, ReadAhead><<<dim3(grid.x, grid.y + readers), 256, 0, stream>>>(P, A);
+        else if (HPW == 2 && eight) paged_block_attn_kernel<__bf16, 2, 2, 8><<<grid, 512, 0, stream>>>(P);
         else if (HPW == 2)     paged_block_attn_kernel<__bf16, 2, 2, 4><<<grid, 256, 0, stream>>>(P);
         else                   paged_block_attn_kernel<__bf16, 1, 1, 4><<<grid, 256, 0, stream>>>(P);
     }
@@ -772,6 +833,23 @@ int launch_paged(const void* q, void* o, const void* k_cache, const void* v_cach
     };
     if (dtype == MDX_F16) combine(_Float16()); else combine(__bf16());
     return mdx::check_launch("paged_combine");
+}
+
+int launch_paged(const void* q, void* o, const void* k_cache, const void* v_cache,
+                 int64_t q_stride_b, int64_t q_stride_s, int64_t q_stride_h,
+                 int64_t o_stride_b, int64_t o_stride_s, int64_t o_stride_h,
+                 int64_t cache_stride_page, int64_t cache_stride_tok, int64_t cache_stride_head,
+                 const int32_t* block_table, int64_t bt_stride, const int32_t* context_lens,
+                 int32_t bs, int32_t sq, int32_t num_q_heads, int32_t num_kv_heads,
+                 int32_t head_dim, int32_t max_pages, int32_t page_size, int64_t num_pages,
+                 float scale, int32_t dtype,
+                 void* workspace, int64_t workspace_bytes, bool single_launch, void* counters, int64_t counter_bytes,
+                 mdx_stream_t stream)
+{
+    return launch_paged_ahead(q, o, k_cache, v_cache, q_stride_b, q_stride_s, q_stride_h, o_stride_b, o_stride_s, o_stride_h,
+                              cache_stride_page, cache_stride_tok, cache_stride_head, block_table, bt_stride, context_lens,
+                              bs, sq, num_q_heads, num_kv_heads, head_dim, max_pages, page_size, num_pages, scale, dtype,
+                              workspace, workspace_bytes, single_launch, counters, counter_bytes, nullptr, 0, nullptr, 0, stream);
 }
 
 }  // namespace mdx
@@ -815,4 +893,23 @@ extern "C" int mdx_paged_block_attn_single_launch(const void* q, void* o, const 
                         cache_stride_page, cache_stride_tok, cache_stride_head, block_table, bt_stride, context_lens,
                         bs, sq, num_q_heads, num_kv_heads, head_dim, max_pages, page_size, num_pages, scale, dtype,
                         workspace, workspace_bytes, true, counters, counter_bytes, stream);
+}
+
+extern "C" int mdx_paged_block_attn_read_ahead(const void* q, void* o, const void* k_cache, const void* v_cache,
+                                               int64_t q_stride_b, int64_t q_stride_s, int64_t q_stride_h,
+                                               int64_t o_stride_b, int64_t o_stride_s, int64_t o_stride_h,
+                                               int64_t cache_stride_page, int64_t cache_stride_tok, int64_t cache_stride_head,
+                                               const int32_t* block_table, int64_t bt_stride, const int32_t* context_lens,
+                                               int32_t bs, int32_t sq, int32_t num_q_heads, int32_t num_kv_heads,
+                                               int32_t head_dim, int32_t max_pages, int32_t page_size, int64_t num_pages,
+                                               float scale, int32_t dtype,
+                                               void* workspace, int64_t workspace_bytes, void* counters, int64_t counter_bytes,
+                                               const void* next, int64_t next_bytes, const void* then, int64_t then_bytes,
+                                               mdx_stream_t stream)
+{
+    return mdx::launch_paged_ahead(q, o, k_cache, v_cache, q_stride_b, q_stride_s, q_stride_h, o_stride_b, o_stride_s, o_stride_h,
+                                   cache_stride_page, cache_stride_tok, cache_stride_head, block_table, bt_stride, context_lens,
+                                   bs, sq, num_q_heads, num_kv_heads, head_dim, max_pages, page_size, num_pages, scale, dtype,
+                                   workspace, workspace_bytes, counters != nullptr, counters, counter_bytes,
+                                   next, next_bytes, then, then_bytes, stream);
 }

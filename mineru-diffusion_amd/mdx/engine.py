@@ -32,7 +32,7 @@ from torch import nn
 from . import _lib
 from .context import get_context, reset_context, set_context
 from .layers import Attention
-from .ops import (confidence_argmax, lm_head_confidence, flash_attn_with_kvcache, linear, linear_gated, linear_qk_norm_rope_store, qk_norm_rope_store,
+from .ops import (confidence_argmax, lm_head_confidence, flash_attn_with_kvcache_read_ahead, linear, linear_gated, linear_qk_norm_rope_store, qk_norm_rope_store,
                   qk_norm_rope_store_partials, rms_norm, rms_norm_partials, select_transfer, silu_and_mul, sparse_attn_varlen, unmask_step)
 
 PAGE = 256                      # tokens per KV page (Sequence.kvcache_block_size, sequence.py:17)
@@ -262,8 +262,8 @@ class DecoderLayer(nn.Module):
             o = sparse_attn_varlen(q, k, v, cu_seqlens_q=ctx.cu_seqlens_q, cu_seqlens_k=ctx.cu_seqlens_k,
                                    staircase_size=ctx.block_size, max_seqlen=ctx.max_seqlen_k or None, softmax_scale=attn.scale)
             return o.flatten(1)
-        o = flash_attn_with_kvcache(q, attn.k_cache, attn.v_cache, cache_seqlens=ctx.context_lens,
-                                    block_table=ctx.block_tables, softmax_scale=attn.scale, causal=False)
+        o = flash_attn_with_kvcache_read_ahead(q, attn.k_cache, attn.v_cache, ctx.context_lens, ctx.block_tables, attn.scale,
+                                               self.o_proj, self.gate_up_proj)
         return o.flatten(2)
 
 

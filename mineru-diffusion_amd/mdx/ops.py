@@ -138,6 +138,12 @@ def flash_attn_with_kvcache(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
     return _host().flash_attn_with_kvcache(q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale, counters)
 
 
+def flash_attn_with_kvcache_read_ahead(q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale, next_weight, then_weight) -> torch.Tensor:
+    """flash_attn_with_kvcache in a decode pass, whose launch also reads the weights of the two products behind it where it leaves the
+    chip idle (up to 256 rows): the same result; the products find them in the device's cache."""
+    return _host().flash_attn_with_kvcache_read_ahead(q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale, next_weight, then_weight)
+
+
 # --------------------------------------------------------------------------- unmask step
 def gumbel_noise(rows: int, vocab: int, seed: int, offset: int = 0, device=None,
                  offset_dev: torch.Tensor | None = None, row_ids: torch.Tensor | None = None) -> torch.Tensor:

@@ -214,6 +214,18 @@ def test_generated_kernel_core_is_current():
     assert out.stdout == (csrc / "lm_head_core.inc").read_text()
 
 
+def test_read_ahead_arguments_are_validated(L):
+    """What an attention launch is asked to read ahead: whole 16-byte pieces that exist; all other arguments as in the plain call."""
+    one, null = ctypes.c_void_p(256), ctypes.c_void_p(0)
+    ra = lambda **kw: L.mdx_paged_block_attn_read_ahead(                                       # noqa: E731
+        one, one, one, one, 65536, 2048, 128, 65536, 2048, 128, 262144, 1024, 128, one, 17, one,
+        kw.get("bs", 4), kw.get("sq", 32), 16, 8, 128, 17, 256, 100, 0.1, 0, null, 0, kw.get("counters", null), 0,
+        kw.get("a", one), kw.get("na", 256), kw.get("b", one), kw.get("nb", 256), null)
+    assert ra(na=-16) == -1 and ra(nb=8) == -1 and ra(a=null) == -1 and ra(b=ctypes.c_void_p(264)) == -1 and b"16 bytes" in L.mdx_last_error()
+    assert ra(bs=-1) == -1 and ra(sq=129) == -2 and ra(bs=0) == 0
+    assert ra() == -3 and ra(a=null, na=0, b=null, nb=0) == -3 and b"workspace" in L.mdx_last_error()
+
+
 def test_linear_arguments_are_validated(L):
     null, one, odd = None, ctypes.c_void_p(16), ctypes.c_void_p(24)
     for rows, n, k in ((0, 64, 256), (-1, 64, 256), (1537, 64, 256), (4, 68, 256), (4, 0, 256), (4, -64, 256), (4, 64, 320), (4, 64, 128), (4, 1 << 28, 256)):

@@ -35,3 +35,31 @@ def test_pieces(dev, ctxs, wide):
 def test_pieces_folded_twelve_at_a_time(dev, ctxs):
     """Tables wide enough for 8 to 14 pieces of a sequence: fewer, as many and more than the fold asks for at once."""
     test_pieces(dev, ctxs, 0)
+
+
+@pytest.mark.parametrize("bs,hq,hkv,dtype", [(1, 16, 8, torch.bfloat16), (2, 16, 8, torch.bfloat16), (8, 16, 8, torch.bfloat16), (9, 16, 8, torch.bfloat16),
+                                             (3, 3, 1, torch.bfloat16), (4, 4, 2, torch.float16), (6, 64, 32, torch.bfloat16), (2, 4, 2, torch.float32)])
+def test_reading_ahead_changes_nothing(dev, bs, hq, hkv, dtype):
+    """Rows of a pass with readers behind the attention's workgroups and, beyond the rule or for other types, without: the same bits as the
+    call that reads nothing, eagerly and from a graph, for weights of any size and layout."""
+    import mdx
+    from mdx import ops
+    g = torch.Generator().manual_seed(bs * hq)
+    d, page, ctx = 128, 256, 900
+    pool = bs * 4
+    q = torch.randn(bs, 32, hq, d, generator=g).to(dtype).to(dev)
+    kc, vc = (torch.randn(pool, page, hkv, d, generator=g).to(dtype).to(dev) for _ in range(2))
+    bt = torch.randperm(pool, generator=g).int().view(bs, 4).to(dev)
+    lens = torch.tensor([ctx - 37 * b for b in range(bs)], dtype=torch.int32, device=dev)
+    want = mdx.flash_attn_with_kvcache(q, kc, vc, cache_seqlens=lens, block_table=bt, softmax_scale=d ** -0.5)
+    w = torch.zeros(24 << 20, dtype=torch.bfloat16, device=dev)
+    for a, b in ((w[:8], w[:3]), (w[:1 << 20], w), (w, w), (w[1:9], w[:1 << 20].view(1024, 1024).t()), (w[:0], w[:8200])):
+        assert torch.equal(ops.flash_attn_with_kvcache_read_ahead(q, kc, vc, lens, bt, d ** -0.5, a, b), want)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = ops.flash_attn_with_kvcache_read_ahead(q, kc, vc, lens, bt, d ** -0.5, w[:1 << 22], w)
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
