@@ -448,7 +448,7 @@ int mdx_silu_and_mul(const void* x, int64_t x_row_stride, void* out, int64_t out
 /*
  * Linear layers, x . w^T (nanovllm/layers/linear.py as called at nanovllm/models/sdar.py:73-112);
  * x [rows, k], w [n, k], MDX_BF16, row strides in elements (multiples of 8), 16-byte aligned; n a multiple of 8, k of 128
- * and at least 256, sizes and strides below 2^28.
+ * and at least 256, sizes and strides below 2^28 (the two mdx_decode_linear_*: n and k below 2^30, any strides).
  *
  * mdx_linear rounds the product to bf16, y [rows, n] (row stride a multiple of 4).  mdx_linear_partials leaves it as fp32
  * partial sums over slices of K, partials [splits, rows, n] (dense), for one of the two kernels below that add them up and

@@ -300,6 +300,12 @@ bool rows_covered(const Rows& r, int64_t k) {
     return r.t.scalar_type() == at::kBFloat16 && r.t.stride(-1) == 1 && r.stride >= k && r.stride % 8 == 0 && reinterpret_cast<uintptr_t>(ptr(r.t)) % 16 == 0;
 }
 
+// x and W for the calls whose row strides end below 2^28 elements
+bool operands_covered(const Rows& x, const Rows& w, int64_t k) {
+    constexpr int64_t kStrides = (int64_t)1 << 28;
+    return rows_covered(x, k) && rows_covered(w, k) && x.stride < kStrides && w.stride < kStrides;
+}
+
 // x [.., k], w [n, k] -> fp32 partial sums [splits, .., n], or None where the shape is not covered
 PyObject* linear_partials(PyObject*, PyObject* const* a, Py_ssize_t n) {
     ARGS(2);
@@ -352,7 +358,7 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const int32_t splits = mdx_linear_splits(rows, cols, k);
         if (splits < 0) Py_RETURN_NONE;
         const Rows r = rows_of(x, k);
-        if (!rows_covered(r, k) || !rows_covered(rows_of(w, k), k)) Py_RETURN_NONE;
+        if (!operands_covered(r, rows_of(w, k), k)) Py_RETURN_NONE;
         const bool cut = splits > 0 && PyObject_IsTrue(a[2]) == 1;
         std::vector<int64_t> shape;
         if (cut) shape.push_back(splits);
@@ -375,7 +381,7 @@ PyObject* linear_gated(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const int64_t k = w.size(1), cols = w.size(0) / 2, rows = k ? x.numel() / k : 0;
         if (!mdx_linear_silu_supported(rows, cols, k)) Py_RETURN_NONE;
         const Rows r = rows_of(x, k);
-        if (!rows_covered(r, k) || !rows_covered(rows_of(w, k), k)) Py_RETURN_NONE;
+        if (!operands_covered(r, rows_of(w, k), k)) Py_RETURN_NONE;
         std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());
         shape.back() = cols;
         Tensor y = at::empty(shape, at::TensorOptions().dtype(at::kBFloat16).device(x.device()));
@@ -398,7 +404,7 @@ PyObject* linear_qk_norm_rope_store(PyObject*, PyObject* const* a, Py_ssize_t n)
         const int64_t k = w.size(1), rows = k ? x.numel() / k : 0;
         if (!mdx_linear_qk_norm_rope_store_supported(rows, (int32_t)hq, (int32_t)hkv, (int32_t)d, k)) Py_RETURN_NONE;
         const Rows r = rows_of(x, k);
-        if (!rows_covered(r, k) || !rows_covered(rows_of(w, k), k)) Py_RETURN_NONE;
+        if (!operands_covered(r, rows_of(w, k), k)) Py_RETURN_NONE;
         NEED(qw.scalar_type() == at::kBFloat16 && kw.scalar_type() == at::kBFloat16 && qw.numel() == d && kw.numel() == d && qw.is_contiguous() && kw.is_contiguous());
         NEED(positions.numel() == rows && positions.scalar_type() == at::kLong && cos.scalar_type() == at::kFloat && sin.scalar_type() == at::kFloat);
         const Tensor pos = positions.is_contiguous() ? positions : positions.contiguous();

@@ -138,10 +138,10 @@ __global__ __launch_bounds__(T::kThreads, T::kWaves / 4) void linear_kernel(cons
     }
 }
 
-template <int BM, int BN, int WM, int WN, int WK, int S, int SX, int FORM>
+template <int BM, int BN, int WM, int WN, int WK, int S, int SX, int FORM, bool WIDE = false>
 int launch(LinearParams A, hipStream_t stream)
 {
-    typedef Tile<BM, BN, WM, WN, WK, S, SX, FORM == kSilu> T;
+    typedef Tile<BM, BN, WM, WN, WK, S, SX, FORM == kSilu, WIDE> T;
     constexpr int kAfter = kSumsBytes<T> + (FORM == kHeads ? BM * kHeadPitch * 2 : 0), kLdsBytes = T::kStepsBytes > kAfter ? T::kStepsBytes : kAfter;
     static_assert(kLdsBytes <= 160 * 1024, "LDS");
     static_assert(FORM != kHeads || (BN == mdx_qk::kHeadDim && WK == 2 && BM % (T::kThreads / mdx_qk::kLanesPerRow) == 0), "a head per column tile");
@@ -234,13 +234,19 @@ bool sizes_covered(int64_t rows, int64_t n, int64_t k)
     return rows > 0 && rows < kSizeLimit && n > 0 && n % 8 == 0 && n < kSizeLimit && k >= 256 && k % 128 == 0 && k < kSizeLimit;
 }
 
-int check_linear(const char* what, const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride, const void* out, int64_t rows, int64_t n, int64_t k)
+bool narrow(int64_t x_row_stride, int64_t w_row_stride) { return x_row_stride < kNarrowStride && w_row_stride < kNarrowStride; }
+
+// any_stride: the two mdx_decode_linear_* calls, which have always taken rows however far apart
+int check_linear(const char* what, bool any_stride, const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride, const void* out,
+                 int64_t rows, int64_t n, int64_t k)
 {
     MDX_REQUIRE(rows >= 0 && n >= 0 && k >= 0, MDX_EINVAL, "%s: negative size", what);
     MDX_REQUIRE(x && w && out, MDX_EINVAL, "%s: null pointer", what);
     MDX_REQUIRE(mdx::aligned16(x) && mdx::aligned16(w) && mdx::aligned16(out) && x_row_stride % 8 == 0 && w_row_stride % 8 == 0 &&
-                x_row_stride >= k && w_row_stride >= k && x_row_stride < kSizeLimit && w_row_stride < kSizeLimit, MDX_EUNSUPPORTED,
+                x_row_stride >= k && w_row_stride >= k, MDX_EUNSUPPORTED,
                 "%s: x, W and the result must be 16-byte aligned, row strides multiples of 8 elements and at least k", what);
+    MDX_REQUIRE(any_stride || narrow(x_row_stride, w_row_stride), MDX_EUNSUPPORTED, "%s: row strides %lld and %lld (below %lld elements)", what,
+                (long long)x_row_stride, (long long)w_row_stride, (long long)kNarrowStride);
     return MDX_OK;
 }
 
@@ -252,26 +258,28 @@ LinearParams params_of(const void* x, int64_t x_row_stride, const void* w, int64
     return A;
 }
 
-int run_partials(const char* what, const Plan& plan, const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride, float* partials,
+int run_partials(const char* what, bool any_stride, const Plan& plan, const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride, float* partials,
                  int64_t rows, int64_t n, int64_t k, mdx_stream_t stream)
 {
-    const int rc = check_linear(what, x, x_row_stride, w, w_row_stride, partials, rows, n, k);
+    const int rc = check_linear(what, any_stride, x, x_row_stride, w, w_row_stride, partials, rows, n, k);
     if (rc != MDX_OK) return rc;
     LinearParams A = params_of(x, x_row_stride, w, w_row_stride, rows, n, k);
     A.partials = partials;
     A.splits = plan.splits;
+    if (!narrow(x_row_stride, w_row_stride)) return launch<32, 64, 2, 2, 1, 4, 4, kPartials, true>(A, static_cast<hipStream_t>(stream));
     return plan.tile->partials(A, static_cast<hipStream_t>(stream));
 }
 
-int run_rows(const char* what, bool silu, const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride, void* y, int64_t y_row_stride,
+int run_rows(const char* what, bool any_stride, bool silu, const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride, void* y, int64_t y_row_stride,
              int64_t rows, int64_t n, int64_t k, mdx_stream_t stream)
 {
-    const int rc = check_linear(what, x, x_row_stride, w, w_row_stride, y, rows, n, k);
+    const int rc = check_linear(what, any_stride, x, x_row_stride, w, w_row_stride, y, rows, n, k);
     if (rc != MDX_OK) return rc;
     MDX_REQUIRE(y_row_stride % 4 == 0 && y_row_stride >= n, MDX_EUNSUPPORTED, "%s: row stride of y (a multiple of 4, at least n)", what);
     LinearParams A = params_of(x, x_row_stride, w, w_row_stride, rows, n, k);
     A.y = (__bf16*)y;
     A.y_stride = y_row_stride;
+    if (silu && !narrow(x_row_stride, w_row_stride)) return launch<32, 64, 2, 2, 1, 4, 4, kSilu, true>(A, static_cast<hipStream_t>(stream));
     const Plan plan = plan_of(rows, n, k, !silu, false, silu);
     return (silu ? plan.tile->silu : plan.tile->rounded)(A, static_cast<hipStream_t>(stream));
 }
@@ -282,11 +290,11 @@ constexpr int64_t kMaxRows = 1536, kMaxSiluRows = 8192;
 // With the head rows finished in the epilogue (launch_heads): from where tiles of 128 columns are enough to fill most CUs; fewer rows
 // are bound by what a CU takes in, and the product in narrower tiles or slices of K with a second launch is the faster.
 constexpr int64_t kMinHeadRows = 384;
-constexpr int64_t kMaxDecodeRows = 128, kMaxDecodeSiluRows = 64;
+constexpr int64_t kMaxDecodeRows = 128, kMaxDecodeSiluRows = 64, kDecodeSizeLimit = (int64_t)1 << 30;
 
 Plan decode_plan(int64_t rows, int64_t n, int64_t k)
 {
-    if (!sizes_covered(rows, n, k) || rows > kMaxDecodeRows || n % 64 != 0 || k % 256 != 0) return Plan{nullptr, 0};
+    if (rows <= 0 || rows > kMaxDecodeRows || n <= 0 || n % 64 != 0 || n >= kDecodeSizeLimit || k <= 0 || k % 256 != 0 || k >= kDecodeSizeLimit) return Plan{nullptr, 0};
     return plan_of(rows, n, k, false, true, false);
 }
 
@@ -303,7 +311,7 @@ extern "C" int mdx_linear(const void* x, int64_t x_row_stride, const void* w, in
 {
     MDX_REQUIRE(sizes_covered(rows, n, k), MDX_EUNSUPPORTED, "linear: %lld rows, n %lld (a multiple of 8), k %lld (a multiple of 128, at least 256)",
                 (long long)rows, (long long)n, (long long)k);
-    return run_rows("linear", false, x, x_row_stride, w, w_row_stride, y, y_row_stride, rows, n, k, stream);
+    return run_rows("linear", false, false, x, x_row_stride, w, w_row_stride, y, y_row_stride, rows, n, k, stream);
 }
 
 extern "C" int mdx_linear_partials(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride,
@@ -311,7 +319,7 @@ extern "C" int mdx_linear_partials(const void* x, int64_t x_row_stride, const vo
 {
     MDX_REQUIRE(mdx_linear_splits(rows, n, k) > 0, MDX_EUNSUPPORTED, "linear_partials: %lld rows, n %lld, k %lld are not cut along k",
                 (long long)rows, (long long)n, (long long)k);
-    return run_partials("linear_partials", plan_of(rows, n, k, true, true, false), x, x_row_stride, w, w_row_stride, partials, rows, n, k, stream);
+    return run_partials("linear_partials", false, plan_of(rows, n, k, true, true, false), x, x_row_stride, w, w_row_stride, partials, rows, n, k, stream);
 }
 
 extern "C" int32_t mdx_linear_silu_supported(int64_t rows, int64_t n, int64_t k) { return sizes_covered(rows, n, k) && rows <= kMaxSiluRows; }
@@ -321,7 +329,7 @@ extern "C" int mdx_linear_silu(const void* x, int64_t x_row_stride, const void* 
 {
     MDX_REQUIRE(sizes_covered(rows, n, k), MDX_EUNSUPPORTED, "linear_silu: %lld rows, n %lld (a multiple of 8), k %lld (a multiple of 128, at least 256)",
                 (long long)rows, (long long)n, (long long)k);
-    return run_rows("linear_silu", true, x, x_row_stride, w, w_row_stride, y, y_row_stride, rows, n, k, stream);
+    return run_rows("linear_silu", false, true, x, x_row_stride, w, w_row_stride, y, y_row_stride, rows, n, k, stream);
 }
 
 extern "C" int32_t mdx_linear_qk_norm_rope_store_supported(int64_t rows, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int64_t k)
@@ -343,7 +351,7 @@ extern "C" int mdx_linear_qk_norm_rope_store(const void* x, int64_t x_row_stride
                 "%s: %lld rows (%lld to %lld), head_dim %d (only %d), k %lld (a multiple of 128, at least 256)", what, (long long)rows,
                 (long long)kMinHeadRows, (long long)kMaxRows, head_dim, mdx_qk::kHeadDim, (long long)k);
     const int64_t n = ((int64_t)num_q_heads + 2 * (int64_t)num_kv_heads) * head_dim;
-    const int rc = check_linear(what, x, x_row_stride, w, w_row_stride, q_out, rows, n, k);
+    const int rc = check_linear(what, false, x, x_row_stride, w, w_row_stride, q_out, rows, n, k);
     if (rc != MDX_OK) return rc;
     MDX_REQUIRE(q_weight && k_weight && cos_table && sin_table && positions, MDX_EINVAL, "%s: null pointer", what);
     MDX_REQUIRE((k_cache == nullptr) == (v_cache == nullptr), MDX_EINVAL, "%s: give both caches or neither", what);
@@ -366,12 +374,12 @@ extern "C" int mdx_decode_linear_partials(const void* x, int64_t x_row_stride, c
     const Plan plan = decode_plan(rows, n, k);
     MDX_REQUIRE(plan.tile, MDX_EUNSUPPORTED, "decode_linear: %lld rows (up to %lld), n %lld (a multiple of 64), k %lld (a multiple of 256)",
                 (long long)rows, (long long)kMaxDecodeRows, (long long)n, (long long)k);
-    return run_partials("decode_linear", plan, x, x_row_stride, w, w_row_stride, partials, rows, n, k, stream);
+    return run_partials("decode_linear", true, plan, x, x_row_stride, w, w_row_stride, partials, rows, n, k, stream);
 }
 
 extern "C" int32_t mdx_decode_linear_silu_supported(int64_t rows, int64_t n, int64_t k)
 {
-    return sizes_covered(rows, n, k) && rows <= kMaxDecodeSiluRows && n % 24 == 0 && k % 512 == 0;
+    return rows > 0 && rows <= kMaxDecodeSiluRows && n > 0 && n % 24 == 0 && n < kDecodeSizeLimit / 2 && k > 0 && k % 512 == 0 && k < kDecodeSizeLimit;
 }
 
 extern "C" int mdx_decode_linear_silu(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride,
@@ -380,5 +388,5 @@ extern "C" int mdx_decode_linear_silu(const void* x, int64_t x_row_stride, const
     MDX_REQUIRE(mdx_decode_linear_silu_supported(rows, n, k), MDX_EUNSUPPORTED,
                 "decode_linear_silu: %lld rows (up to %lld), n %lld (a multiple of 24), k %lld (a multiple of 512)", (long long)rows,
                 (long long)kMaxDecodeSiluRows, (long long)n, (long long)k);
-    return run_rows("decode_linear_silu", true, x, x_row_stride, w, w_row_stride, y, y_row_stride, rows, n, k, stream);
+    return run_rows("decode_linear_silu", true, true, x, x_row_stride, w, w_row_stride, y, y_row_stride, rows, n, k, stream);
 }

@@ -22,6 +22,7 @@
 // steps of 32 elements (half lines: slower) and six steps in LDS instead of four of the small tiles gained nothing.
 #pragma once
 #include "mdx_common.h"
+#include <type_traits>
 #include <utility>
 
 namespace mdx_tile {
@@ -49,8 +50,10 @@ template <int N> __device__ __forceinline__ void wait_loads_and_meet() {
 }
 
 // BM rows of x by BN rows of W on WM x WN x WK wavefronts.  PAIRS: W is two matrices one after the other (gate, up), and the
-// tile's rows of W are 16 rows of the first, the same 16 of the second, and so on.
-template <int BM_, int BN_, int WM_, int WN_, int WK_, int S_, int SX_, bool PAIRS> struct Tile {
+// tile's rows of W are 16 rows of the first, the same 16 of the second, and so on.  WIDE: row strides of any size; else below
+// kNarrowStride elements, so that a lane's place among the eight rows of a load is 32 bits beside a scalar address (7 x 2^29 bytes).
+constexpr int64_t kNarrowStride = (int64_t)1 << 28;
+template <int BM_, int BN_, int WM_, int WN_, int WK_, int S_, int SX_, bool PAIRS, bool WIDE = false> struct Tile {
     static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, WK = WK_, S = S_, SX = SX_;
     static constexpr int kWaves = WM * WN * WK, kThreads = 64 * kWaves;
     static constexpr int TM = BM / (16 * WM), TN = BN / (16 * WN);     // a wavefront's share, in matrix tiles of 16 x 16
@@ -82,7 +85,8 @@ template <int BM_, int BN_, int WM_, int WN_, int WK_, int S_, int SX_, bool PAI
         // again; their products are not used.
         const unsigned lds0 = (unsigned)(uintptr_t)(lds_char*)lds;
         const char* base[kLoads];                           // the first of the 8 rows, at this slice of K
-        unsigned offset[kLoads];                            // this lane's row and chunk from there
+        typedef std::conditional_t<WIDE, uint64_t, unsigned> Offset;
+        Offset offset[kLoads];                              // this lane's row and chunk from there
 #pragma unroll
         for (int i = 0; i < kLoads; ++i) {
             const bool of_x = i < kXLoads;
@@ -91,11 +95,12 @@ template <int BM_, int BN_, int WM_, int WN_, int WK_, int S_, int SX_, bool PAI
             const int64_t stride = (of_x ? A.x_stride : A.w_stride) * 2;
             const int64_t second = PAIRS && !of_x && ((r0 >> 4) & 1) ? A.N : 0;
             base[i] = reinterpret_cast<const char*>((of_x ? A.x : A.w) + k0) + (min(first, last) + second) * stride;
-            offset[i] = (unsigned)(min(first + r, last) - min(first, last)) * (unsigned)stride + chunk * 16;
+            offset[i] = (Offset)(min(first + r, last) - min(first, last)) * (Offset)stride + chunk * 16;
         }
         int64_t x_at = 0, w_at = 0;                         // where the step to ask for next begins
         auto load = [&](int i, unsigned dst, int64_t at) {
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(dst), "v"(offset[i]), "s"(base[i] + at) : "memory");
+            if constexpr (WIDE) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" :: "s"(dst), "v"(base[i] + at + offset[i]) : "memory");
+            else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(dst), "v"(offset[i]), "s"(base[i] + at) : "memory");
         };
         auto load_x = [&](int slot) {
 #pragma unroll

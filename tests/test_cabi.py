@@ -157,6 +157,8 @@ def test_decode_linear_arguments_are_validated(L):
     assert L.mdx_decode_linear_splits(32, 2048, 2048) > 0 and 2048 // 256 % L.mdx_decode_linear_splits(32, 2048, 2048) == 0
     for rows, n, k in ((0, 64, 256), (129, 64, 256), (-1, 64, 256), (4, 72, 256), (4, 0, 256), (4, -64, 256), (4, 64, 320), (4, 64, 0), (4, 1 << 30, 256)):
         assert L.mdx_decode_linear_splits(rows, n, k) == 0
+    for n, k in ((1 << 28, 256), (64, 1 << 28), (64, (1 << 30) - 256), ((1 << 30) - 64, 256)):
+        assert L.mdx_decode_linear_splits(4, n, k) > 0 and k // 256 % L.mdx_decode_linear_splits(4, n, k) == 0
     pl = lambda **kw: L.mdx_decode_linear_partials(kw.get("x", one), kw.get("xs", 256), kw.get("w", one), kw.get("ws", 256), kw.get("p", one),    # noqa: E731
                                                    kw.get("rows", 4), 64, 256, null)
     sl = lambda **kw: L.mdx_decode_linear_silu(kw.get("x", one), kw.get("xs", 512), kw.get("w", one), kw.get("ws", 512), kw.get("y", one),        # noqa: E731
@@ -167,8 +169,9 @@ def test_decode_linear_arguments_are_validated(L):
         assert call(rows=129) == -2
     assert pl(p=null) == -1 and pl(p=odd) == -2
     assert sl(y=null) == -1 and sl(y=odd) == -2 and sl(ys=20) == -2 and sl(ys=26) == -2 and sl(rows=65) == -2 and sl(n=32) == -2
-    for rows, n, k in ((0, 24, 512), (65, 24, 512), (4, 16, 512), (4, 24, 256), (4, 0, 512)):
+    for rows, n, k in ((0, 24, 512), (65, 24, 512), (4, 16, 512), (4, 24, 256), (4, 0, 512), (4, 24, 0), (4, 3 << 28, 512), (4, 24, 1 << 30)):
         assert L.mdx_decode_linear_silu_supported(rows, n, k) == 0
+    assert L.mdx_decode_linear_silu_supported(4, 3 << 27, 512) == 1 and L.mdx_decode_linear_silu_supported(4, 24, 1 << 28) == 1
     rn = lambda **kw: L.mdx_add_rms_norm_partials(kw.get("p", one), kw.get("splits", 2), kw.get("res", one), kw.get("rs", 64), kw.get("res_out", one), 64,  # noqa: E731
                                                   one, kw.get("eps", 1e-6), kw.get("out", one), 64, kw.get("rows", 4), kw.get("hidden", 64), kw.get("dtype", 0), null)
     assert rn(p=null) == -1 and rn(out=null) == -1 and rn(res=null) == -1 and rn(splits=0) == -1 and rn(rs=56) == -1 and rn(eps=-1.0) == -1

@@ -55,6 +55,34 @@ def test_linear_says_what_it_does_not_cover(dev):
     assert ops.linear(z(2, 3, 256), z(64, 256)).shape == (2, 3, 64) and ops.linear_gated(z(2, 3, 256), z(64, 256)).shape == (2, 3, 32)
 
 
+def test_rows_far_apart(dev):
+    """Rows 2^28 elements and more apart: computed by the two calls for few rows, left to the library by the others."""
+    import mdx
+    from mdx import ops
+    far = (1 << 28) + 8
+    buffer = torch.empty(63 * far + 2048, dtype=torch.bfloat16, device=dev)               # 32 GB, of which the rows below are written
+
+    def apart(t, offset):
+        view = buffer.as_strided(t.shape, (far, 1), offset)
+        view.copy_(t)
+        return view
+
+    for rows, n, k in ((3, 64, 256), (33, 64, 768), (64, 64, 512)):
+        ref, x, w = _xw(dev, rows, n, k)
+        for a, b in ((apart(x, 0), w), (x, apart(w, 1024)), (apart(x, 0), apart(w, 1024))):
+            p = ops.linear_partials(a, b)
+            assert p.shape == (mdx._lib.lib().mdx_decode_linear_splits(rows, n, k), rows, n) and _close(p.sum(0), ref, 2e-6)
+            assert ops.linear(a, b) is None and ops.linear(a, b, True) is None and ops.linear_gated(a, b) is None
+    for rows, n in ((3, 24), (40, 24)):
+        ref, x, w = _xw(dev, rows, 2 * n, 512)
+        want = mdx.silu_and_mul(ref.bfloat16().to(dev)).float().cpu()
+        for a, b in ((apart(x, 0), w), (x, apart(w, 1024)), (apart(x, 0), apart(w, 1024))):
+            y = ops.linear_silu(a, b)
+            assert y.shape == want.shape and _close(y, want, 3e-3)
+    del buffer
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("rows,hq,hkv,k", [(384, 16, 8, 384), (385, 2, 1, 256), (513, 4, 2, 512), (1000, 16, 8, 256), (1100, 16, 8, 256), (1536, 6, 3, 256)])
 @pytest.mark.parametrize("caches", [True, False])
 def test_linear_qk_norm_rope_store(dev, rows, hq, hkv, k, caches):
