@@ -783,17 +783,23 @@ int launch_paged_ahead(const void* q, void* o, const void* k_cache, const void* 
     // on equal lengths); with more pairs than CUs the second round costs more than that gains.
     const bool eight = device_span && (int64_t)bs * wg_per_pair <= cus;
     const unsigned n_heads = (unsigned)(bs * num_q_heads * P.nqt);
-    // Reading ahead, by rows of the pass (kReadAhead*): engine, ms per generation without / with, contexts of 1088 and more: one request 68.0 / 66.2, two 79.8 /
-    // 78.2, three 96.1 / 91.0, four 100.2 / 95.9, six 121.8 / 119.8, eight 132.8 / 130.7; of 32: one 61.6 / 60.7, four 82.2 / 77.9, eight 98.1 / 96.7.  More
-    // rows: 16 requests 190.3 / 190.7 (the attention streams by itself then, and the products are bound by other things).  32 rows have the
-    // shortest attention: all of 56 MB there 68.6, a workgroup on every other CU and 32 MB 66.2.
+    // Reading ahead, by rows of the pass (kReadAhead*).  Engine, ms per generation without / with, contexts of 1088 and more in tables of 2048: one request
+    // 68.0 / 66.2, two 79.8 / 78.2, three 96.1 / 91.0, four 100.2 / 95.9, six 121.8 / 119.8, eight 132.8 / 130.7; of 32: one 61.6 / 60.7, four 82.2 / 77.9,
+    // eight 98.1 / 96.7.  More rows: 16 requests 190.3 / 190.7 (the attention streams by itself then, and the products are bound by other things).  32 rows have
+    // the shortest attention: all of 56 MB there 68.6, a workgroup on every other CU and 32 MB 66.2, and only where each reader has a CU to itself beside
+    // all workgroups of the attention, with keys or without: us per decode pass without / with, one request of 1088 in tables of 2048 1808 / 1764, of 3072
+    // 1814 / 1775, of 4096 1816 / 1817, of 8192 1817 / 1824 (of 4096 there 1943 / 1952).  Long contexts by themselves do no harm, although their K/V
+    // passes through the same cache behind the readers: two of 4096 to 15000 in 16384 2257 / 2213 to 2724 / 2748, four of 15000 3607 / 3470, six 4605 / 4487, eight
+    // of 8000 in 8192 4126 / 4061; only eight of 12000 to 15000 (390 MB and more per layer) are slower, 5189 / 5212.
     ReadAhead A{};
     int64_t budget = 0;
     int readers = 0;
     const int64_t pass_rows = (int64_t)bs * sq;
     if (next_bytes + then_bytes > 0 && dtype == MDX_BF16 && HPW == 2 && !eight && pass_rows <= kReadAheadRows) {
-        budget = pass_rows <= kReadAheadFewRows ? kReadAheadFewBytes : kReadAheadBytes;
-        readers = (int)((pass_rows <= kReadAheadFewRows ? cus / 2 : cus) / wg_per_pair);
+        const bool few = pass_rows <= kReadAheadFewRows;
+        budget = few ? kReadAheadFewBytes : kReadAheadBytes;
+        const int64_t attending = wg_per_pair * pairs_y, reading = few ? cus / 2 : cus;
+        if (!few || attending + reading <= cus) readers = (int)(reading / wg_per_pair);
         const int64_t n0 = next_bytes < budget ? next_bytes : budget, n1 = then_bytes < budget - n0 ? then_bytes : budget - n0;
         A = ReadAhead{{static_cast<const u32x4*>(next), static_cast<const u32x4*>(then)}, {(int)(n0 / 16), (int)(n1 / 16)}, pairs_y};
     }

@@ -63,3 +63,18 @@ def test_reading_ahead_changes_nothing(dev, bs, hq, hkv, dtype):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("bs,pages", [(1, 14), (1, 15), (2, 15), (2, 32)])
+def test_reading_ahead_in_wide_tables(dev, bs, pages):
+    """Tables on both sides of what leaves each reader of 32 rows a CU (16 heads on 8: 14 pages do, 15 do not), and 64 rows, which do not ask: the same bits."""
+    import mdx
+    from mdx import ops
+    g = torch.Generator().manual_seed(pages)
+    q = torch.randn(bs, 32, 16, 128, generator=g).bfloat16().to(dev)
+    kc, vc = (torch.randn(pages, 256, 8, 128, generator=g).bfloat16().to(dev) for _ in range(2))
+    bt = torch.stack([torch.randperm(pages, generator=g).int() for _ in range(bs)]).to(dev)
+    lens = torch.tensor([pages * 256, 1088][:bs], dtype=torch.int32, device=dev)
+    w = torch.zeros(24 << 20, dtype=torch.bfloat16, device=dev)
+    want = mdx.flash_attn_with_kvcache(q, kc, vc, cache_seqlens=lens, block_table=bt, softmax_scale=128 ** -0.5)
+    assert torch.equal(ops.flash_attn_with_kvcache_read_ahead(q, kc, vc, lens, bt, 128 ** -0.5, w[:4 << 20], w), want)
