@@ -285,8 +285,13 @@ int run_rows(const char* what, bool any_stride, bool silu, const void* x, int64_
 }
 
 // Where the kernel is the better one (table at the top of this file): up to 1536 rows; with the SiLU in the epilogue, which
-// saves writing and reading twice the result, up to 8192.
+// saves writing and reading twice the result, up to 8192.  Other widths, us, here / library's product: 5120 x 5120, 1024 rows (54 GFLOP) 58.1 / 61.1, 1280 77.1 / 71.7;
+// 7168 x 5120, 512 (38) 51.3 / 49.4, 1280 (94) 101 / 85; 8192 x 8192, 384 (52) 59.6 / 64.3, 768 (103) 94.4 / 97.4, 1024 (137) 141 / 116; 6144 x 4096, 1024 (52) 52.5 / 51.7, 1280 (64)
+// 68.2 / 57.3: from 52 GFLOP on the library's tiles come to their rate.  Where K is long beside n they do not: 5120 x 17408, 1024 rows (183) 173 / 244, 4096 x 12288, 768 (77) 77 / 90.
+// With the SiLU both sides lie within 15 % of each other from 200 GFLOP on, now one and now the other ahead.
 constexpr int64_t kMaxRows = 1536, kMaxSiluRows = 8192;
+constexpr double kMaxWork = 52e9;
+bool linear_pays(int64_t rows, int64_t n, int64_t k) { return rows <= kMaxRows && (2.0 * (double)rows * (double)n * (double)k <= kMaxWork || k >= 3 * n); }
 // With the head rows finished in the epilogue (launch_heads): from where tiles of 128 columns are enough to fill most CUs; fewer rows
 // are bound by what a CU takes in, and the product in narrower tiles or slices of K with a second launch is the faster.
 constexpr int64_t kMinHeadRows = 384;
@@ -302,7 +307,7 @@ Plan decode_plan(int64_t rows, int64_t n, int64_t k)
 
 extern "C" int32_t mdx_linear_splits(int64_t rows, int64_t n, int64_t k)
 {
-    if (!sizes_covered(rows, n, k) || rows > kMaxRows) return -1;
+    if (!sizes_covered(rows, n, k) || !linear_pays(rows, n, k)) return -1;
     return plan_of(rows, n, k, true, true, false).splits;
 }
 
@@ -317,9 +322,10 @@ extern "C" int mdx_linear(const void* x, int64_t x_row_stride, const void* w, in
 extern "C" int mdx_linear_partials(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride,
                                    float* partials, int64_t rows, int64_t n, int64_t k, mdx_stream_t stream)
 {
-    MDX_REQUIRE(mdx_linear_splits(rows, n, k) > 0, MDX_EUNSUPPORTED, "linear_partials: %lld rows, n %lld, k %lld are not cut along k",
-                (long long)rows, (long long)n, (long long)k);
-    return run_partials("linear_partials", false, plan_of(rows, n, k, true, true, false), x, x_row_stride, w, w_row_stride, partials, rows, n, k, stream);
+    Plan plan{nullptr, 0};
+    if (sizes_covered(rows, n, k) && rows <= kMaxRows) plan = plan_of(rows, n, k, true, true, false);
+    MDX_REQUIRE(plan.splits > 0, MDX_EUNSUPPORTED, "linear_partials: %lld rows, n %lld, k %lld are not cut along k", (long long)rows, (long long)n, (long long)k);
+    return run_partials("linear_partials", false, plan, x, x_row_stride, w, w_row_stride, partials, rows, n, k, stream);
 }
 
 extern "C" int32_t mdx_linear_silu_supported(int64_t rows, int64_t n, int64_t k) { return sizes_covered(rows, n, k) && rows <= kMaxSiluRows; }

@@ -234,6 +234,9 @@ def test_linear_arguments_are_validated(L):
     for rows, n, k in ((0, 64, 256), (-1, 64, 256), (1537, 64, 256), (4, 68, 256), (4, 0, 256), (4, -64, 256), (4, 64, 320), (4, 64, 128), (4, 1 << 28, 256)):
         assert L.mdx_linear_splits(rows, n, k) == -1
     assert L.mdx_linear_splits(32, 2048, 6144) > 1 and L.mdx_linear_splits(1024, 4096, 2048) == 0
+    # wide layers: beyond 52 GFLOP only those whose K is long beside n
+    assert L.mdx_linear_splits(512, 7168, 5120) >= 0 and L.mdx_linear_splits(1280, 7168, 5120) == -1 and L.mdx_linear_splits(1024, 8192, 8192) == -1
+    assert L.mdx_linear_splits(1536, 2048, 6144) >= 0 and L.mdx_linear_splits(1024, 5120, 17408) >= 0
     assert L.mdx_linear_silu_supported(8192, 64, 256) == 1 and L.mdx_linear_silu_supported(8193, 64, 256) == 0 and L.mdx_linear_silu_supported(4, 60, 256) == 0
     li = lambda f: lambda **kw: f(kw.get("x", one), kw.get("xs", 256), kw.get("w", one), kw.get("ws", 256), kw.get("y", one), kw.get("ys", 64),    # noqa: E731
                                   kw.get("rows", 4), kw.get("n", 64), kw.get("k", 256), null)
