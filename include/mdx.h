@@ -458,7 +458,7 @@ int mdx_silu_and_mul(const void* x, int64_t x_row_stride, void* out, int64_t out
  * its rounding points; mdx_linear_silu_supported: covered, and up to 8192 rows.
  * mdx_linear_qk_norm_rope_store: the product of a QKV projection with mdx_qk_norm_rope_store on it in one launch; w holds the q
  * rows, then k, then v; k_out / v_out (the rotated k and the raw v, [rows, Hkv * d]) and the caches may be null;
- * mdx_linear_qk_norm_rope_store_supported: 384 to 1536 rows, d = 128.
+ * covered: 384 to 1536 rows, d = 128; mdx_linear_qk_norm_rope_store_supported: and the faster of one launch and two.
  * mdx_decode_linear_partials and mdx_decode_linear_silu: the same for the few rows of a decode pass, always as partial sums
  * (rows up to 128, n a multiple of 64, k of 256; splits = mdx_decode_linear_splits, 0 where not covered) and with the SiLU
  * (rows up to 64, n a multiple of 24, k of 512: mdx_decode_linear_silu_supported).

@@ -186,7 +186,7 @@ const TileCost kTiles[] = {
     tile<256, 256, 4, 2, 1, 2, 3, false>(1.344f, 5.9f),
 };
 
-struct Plan { const TileCost* tile; int splits; };
+struct Plan { const TileCost* tile; int splits; double cost; };
 
 // The cheapest tile and number of slices by the costs above, in rounds of one workgroup per CU (the small tiles' second one
 // per CU is worth little: they share its intake).  Partial sums cost their writing and the next kernel's reading, 0.35 us per
@@ -194,8 +194,7 @@ struct Plan { const TileCost* tile; int splits; };
 // costs 1 % on average and 15 % at most.
 Plan plan_of(int64_t rows, int64_t n, int64_t k, bool rounded, bool partials, bool silu)
 {
-    Plan best{nullptr, 0};
-    double least = 0;
+    Plan best{nullptr, 0, 0};
     const int cus = mdx::compute_units();
     const double mb = (double)rows * (double)n * 4e-6;
     for (const TileCost& t : kTiles) {
@@ -206,7 +205,7 @@ Plan plan_of(int64_t rows, int64_t n, int64_t k, bool rounded, bool partials, bo
             for (int form = 0; form < 2; ++form) {                                  // 0: rounded or SiLU, 1: partial sums
                 if (form == 0 ? (s > 1 || !(rounded || silu)) : (!partials || !t.partials)) continue;
                 const double cost = rounds * (steps * t.step + t.around) + (form ? 0.35 * (double)s : 0.15) * mb;
-                if (!best.tile || cost < least) { best = Plan{&t, form ? (int)s : 0}; least = cost; }
+                if (!best.tile || cost < best.cost) best = Plan{&t, form ? (int)s : 0, cost};
             }
         }
     }
@@ -215,16 +214,18 @@ Plan plan_of(int64_t rows, int64_t n, int64_t k, bool rounded, bool partials, bo
 
 // The QKV projection with what follows it: tiles of one head, by the same costs.  Two launches / one, us per decoder layer: 160 rows
 // 85.6 / 87.5, 256 94.5 / 96.4, 384 117.9 / 115.5, 512 124.1 / 121.3, 768 153.0 / 150.8, 1024 179.6 / 176.5, 1504 241.5 / 238.4.
-int launch_heads(const LinearParams& A, hipStream_t stream)
+struct HeadsPlan { int (*run)(LinearParams, hipStream_t); float cost; };
+HeadsPlan heads_plan(int64_t rows, int64_t n, int64_t k)
 {
     const int cus = mdx::compute_units();
     auto cost = [&](int bm, float step, float around) {
-        const int64_t tiles = (int64_t)((A.in.M + bm - 1) / bm) * (A.in.N / mdx_qk::kHeadDim);
-        return (float)((tiles + cus - 1) / cus) * ((float)(A.K / kStepK) * step + around);
+        const int64_t tiles = (rows + bm - 1) / bm * (n / mdx_qk::kHeadDim);
+        return (float)((tiles + cus - 1) / cus) * ((float)(k / kStepK) * step + around);
     };
     const float c64 = cost(64, 0.345f, 1.7f), c128 = cost(128, 0.499f, 2.6f), c192 = cost(192, 0.602f, 3.5f);
-    if (c64 <= c128 && c64 <= c192) return launch<64, 128, 2, 2, 2, 4, 4, kHeads>(A, stream);
-    return c128 <= c192 ? launch<128, 128, 2, 2, 2, 4, 4, kHeads>(A, stream) : launch<192, 128, 2, 2, 2, 4, 4, kHeads>(A, stream);
+    if (c64 <= c128 && c64 <= c192) return {launch<64, 128, 2, 2, 2, 4, 4, kHeads>, c64};
+    if (c128 <= c192) return {launch<128, 128, 2, 2, 2, 4, 4, kHeads>, c128};
+    return {launch<192, 128, 2, 2, 2, 4, 4, kHeads>, c192};
 }
 
 constexpr int64_t kSizeLimit = (int64_t)1 << 28;
@@ -292,14 +293,22 @@ int run_rows(const char* what, bool any_stride, bool silu, const void* x, int64_
 constexpr int64_t kMaxRows = 1536, kMaxSiluRows = 8192;
 constexpr double kMaxWork = 52e9;
 bool linear_pays(int64_t rows, int64_t n, int64_t k) { return rows <= kMaxRows && (2.0 * (double)rows * (double)n * (double)k <= kMaxWork || k >= 3 * n); }
-// With the head rows finished in the epilogue (launch_heads): from where tiles of 128 columns are enough to fill most CUs; fewer rows
-// are bound by what a CU takes in, and the product in narrower tiles or slices of K with a second launch is the faster.
+// With the head rows finished in the epilogue (heads_plan): from where tiles of 128 columns are enough to fill most CUs; fewer rows
+// are bound by what a CU takes in, and the product in narrower tiles or slices of K with a second launch is the faster.  So it is where these tiles cost more
+// than the product's own plan by what the second launch takes (2.5 us by the costs above): 32 heads on 8, one launch / two, us: 2560 columns of K, 768 rows 39.2 / 43.1, 1024 (tiles
+// for a round and a half) 59.7 / 46.1; 4096, 640 rows 42.2 / 46.9, 1024 77.0 / 59.6; 64 on 8, 8192, 512 rows 91 / 95, 640 143 / 123; 16 on 2, 2048, 384 rows 17.7 / 16.0, 512 17.6 / 21.1.
 constexpr int64_t kMinHeadRows = 384;
+constexpr double kSecondLaunch = 2.5;
+bool heads_covered(int64_t rows, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int64_t k)
+{
+    return num_q_heads > 0 && num_kv_heads > 0 && head_dim == mdx_qk::kHeadDim && rows >= kMinHeadRows && rows <= kMaxRows &&
+           sizes_covered(rows, ((int64_t)num_q_heads + 2 * (int64_t)num_kv_heads) * head_dim, k);
+}
 constexpr int64_t kMaxDecodeRows = 128, kMaxDecodeSiluRows = 64, kDecodeSizeLimit = (int64_t)1 << 30;
 
 Plan decode_plan(int64_t rows, int64_t n, int64_t k)
 {
-    if (rows <= 0 || rows > kMaxDecodeRows || n <= 0 || n % 64 != 0 || n >= kDecodeSizeLimit || k <= 0 || k % 256 != 0 || k >= kDecodeSizeLimit) return Plan{nullptr, 0};
+    if (rows <= 0 || rows > kMaxDecodeRows || n <= 0 || n % 64 != 0 || n >= kDecodeSizeLimit || k <= 0 || k % 256 != 0 || k >= kDecodeSizeLimit) return Plan{nullptr, 0, 0};
     return plan_of(rows, n, k, false, true, false);
 }
 
@@ -322,7 +331,7 @@ extern "C" int mdx_linear(const void* x, int64_t x_row_stride, const void* w, in
 extern "C" int mdx_linear_partials(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride,
                                    float* partials, int64_t rows, int64_t n, int64_t k, mdx_stream_t stream)
 {
-    Plan plan{nullptr, 0};
+    Plan plan{nullptr, 0, 0};
     if (sizes_covered(rows, n, k) && rows <= kMaxRows) plan = plan_of(rows, n, k, true, true, false);
     MDX_REQUIRE(plan.splits > 0, MDX_EUNSUPPORTED, "linear_partials: %lld rows, n %lld, k %lld are not cut along k", (long long)rows, (long long)n, (long long)k);
     return run_partials("linear_partials", false, plan, x, x_row_stride, w, w_row_stride, partials, rows, n, k, stream);
@@ -340,8 +349,9 @@ extern "C" int mdx_linear_silu(const void* x, int64_t x_row_stride, const void* 
 
 extern "C" int32_t mdx_linear_qk_norm_rope_store_supported(int64_t rows, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int64_t k)
 {
-    return num_q_heads > 0 && num_kv_heads > 0 && head_dim == mdx_qk::kHeadDim && rows >= kMinHeadRows && rows <= kMaxRows &&
-           sizes_covered(rows, ((int64_t)num_q_heads + 2 * (int64_t)num_kv_heads) * head_dim, k);
+    if (!heads_covered(rows, num_q_heads, num_kv_heads, head_dim, k)) return 0;
+    const int64_t n = ((int64_t)num_q_heads + 2 * (int64_t)num_kv_heads) * head_dim;
+    return heads_plan(rows, n, k).cost <= plan_of(rows, n, k, true, true, false).cost + kSecondLaunch;
 }
 
 extern "C" int mdx_linear_qk_norm_rope_store(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride,
@@ -353,7 +363,7 @@ extern "C" int mdx_linear_qk_norm_rope_store(const void* x, int64_t x_row_stride
                                              int64_t rows, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int64_t k, mdx_stream_t stream)
 {
     const char* what = "linear_qk_norm_rope_store";
-    MDX_REQUIRE(mdx_linear_qk_norm_rope_store_supported(rows, num_q_heads, num_kv_heads, head_dim, k), MDX_EUNSUPPORTED,
+    MDX_REQUIRE(heads_covered(rows, num_q_heads, num_kv_heads, head_dim, k), MDX_EUNSUPPORTED,
                 "%s: %lld rows (%lld to %lld), head_dim %d (only %d), k %lld (a multiple of 128, at least 256)", what, (long long)rows,
                 (long long)kMinHeadRows, (long long)kMaxRows, head_dim, mdx_qk::kHeadDim, (long long)k);
     const int64_t n = ((int64_t)num_q_heads + 2 * (int64_t)num_kv_heads) * head_dim;
@@ -369,7 +379,7 @@ extern "C" int mdx_linear_qk_norm_rope_store(const void* x, int64_t x_row_stride
     A.rows = RowParams{(const __bf16*)q_weight, (const __bf16*)k_weight, eps, cos_table, sin_table, max_positions, positions,
                        (__bf16*)q_out, q_out_row_stride, (__bf16*)k_out, k_out_row_stride, (__bf16*)v_out, v_out_row_stride,
                        (__bf16*)k_cache, (__bf16*)v_cache, slot_mapping, num_slots, num_q_heads, num_kv_heads};
-    return launch_heads(A, static_cast<hipStream_t>(stream));
+    return heads_plan(rows, n, k).run(A, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int32_t mdx_decode_linear_splits(int64_t rows, int64_t n, int64_t k) { return decode_plan(rows, n, k).splits; }

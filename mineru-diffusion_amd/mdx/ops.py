@@ -65,8 +65,8 @@ def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
 # qk_norm_rope_store_partials add up on their way.  None where the library's product is the better one (many rows) or the
 # shape is not covered.
 def linear(x: torch.Tensor, weight: torch.Tensor, partials: bool = False) -> torch.Tensor | None:
-    """x . weight^T (nanovllm/layers/linear.py) for up to 1536 rows: bf16 [..., n], or with `partials` what is the faster of
-    that and partial sums (one dimension more than x)."""
+    """x . weight^T (nanovllm/layers/linear.py) for up to 1536 rows (wide layers: up to 52 GFLOP): bf16 [..., n], or with
+    `partials` what is the faster of that and partial sums (one dimension more than x)."""
     return _host().linear(x, weight, partials)
 
 
@@ -78,7 +78,7 @@ def linear_gated(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor | None:
 def linear_qk_norm_rope_store(x, weight, q_weight, k_weight, eps, cos, sin, positions, num_q_heads, num_kv_heads, head_dim,
                               k_cache=None, v_cache=None, slot_mapping=None, want_kv: bool = True):
     """qk_norm_rope_store(x . weight^T, ...) for 384 to 1536 rows and heads of 128 columns in one launch (nanovllm/models/sdar.py:73-83
-    and the cache store): (q, k, v), k and v None unless wanted."""
+    and the cache store): (q, k, v), k and v None unless wanted.  None where two launches are the faster."""
     return _host().linear_qk_norm_rope_store(x, weight, q_weight, k_weight, eps, cos, sin, positions, num_q_heads, num_kv_heads, head_dim,
                                              k_cache, v_cache, slot_mapping, want_kv)
 

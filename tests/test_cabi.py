@@ -250,5 +250,10 @@ def test_linear_arguments_are_validated(L):
     hd = lambda **kw: L.mdx_linear_qk_norm_rope_store(kw.get("x", one), kw.get("xs", 256), one, 256, kw.get("qw", one), one, 1e-6, one, one, 8, kw.get("pos", one),   # noqa: E731
                                                       kw.get("q", one), kw.get("qs", 256), null, 0, null, 0, kw.get("kc", null), kw.get("vc", null), kw.get("slots", null), 0,
                                                       kw.get("rows", 400), 2, 1, kw.get("d", 128), 256, null)
+    # one launch where its tiles of a head cost no more than the product's own and a second launch: the model's heads at all rows, others by their rounds
+    hs = L.mdx_linear_qk_norm_rope_store_supported
+    assert all(hs(rows, 16, 8, 128, 2048) == 1 for rows in range(384, 1537)) and hs(383, 16, 8, 128, 2048) == 0 and hs(1537, 16, 8, 128, 2048) == 0
+    assert hs(512, 64, 8, 128, 8192) == 1 and hs(1536, 64, 8, 128, 8192) == 0 and hs(768, 32, 8, 128, 2560) == 1 and hs(1024, 32, 8, 128, 2560) == 0
+    assert hs(384, 16, 2, 128, 2048) == 0 and hs(512, 16, 2, 128, 2048) == 1
     assert hd(x=null) == -1 and hd(qw=null) == -1 and hd(pos=null) == -1 and hd(q=null) == -1 and hd(kc=one) == -1 and hd(kc=one, vc=one) == -1
     assert hd(rows=383) == -2 and hd(rows=1537) == -2 and hd(d=64) == -2 and hd(q=odd) == -2 and hd(qs=260) == -2 and hd(qw=odd) == -2 and hd(xs=248) == -2
