@@ -80,8 +80,9 @@ __global__ __launch_bounds__(T::kThreads, T::kWaves / 4) void lm_head_confidence
 #pragma unroll
         for (int k = 0; k < 4 * T::TN; ++k) s[k & 3] += __builtin_amdgcn_exp2f(__builtin_fmaf(v[k], c[i], -h));
         float sum = ((s[0] + s[1]) + (s[2] + s[3])) * __builtin_amdgcn_exp2f(-__builtin_fmaf(ms, c[i], -h));
-        if (!(m > -INFINITY)) sum = 0.f;                   // all of it beyond the vocabulary: 0, not 0 x the correction's infinity
-        Best b = Best{m, sum, v_lane + 16 * (first >> 2) + (first & 3)};
+        if (m == -INFINITY) sum = 0.f;                     // all of it beyond the vocabulary: 0, not 0 x the correction's infinity
+        // (nothing but NaN: no maximum, so that no other lane's loses its index to this one's; the sum stays NaN)
+        Best b = Best{fmaxf(m, -INFINITY), sum, v_lane + 16 * (first >> 2) + (first & 3)};
 #pragma unroll
         for (int off = 16; off <= 32; off <<= 1)
             b = merge(b, Best{__shfl_xor(b.m, off), __shfl_xor(b.s, off), __shfl_xor(b.idx, off)}, c[i]);

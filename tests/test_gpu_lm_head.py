@@ -148,3 +148,29 @@ def test_lm_head_confidence_tiles(dev, rows, vocab, hidden):
     torch.cuda.synchronize()
     ex0, ep, logits = _reference(x, w, temps)
     _check(x0, p, ex0, ep, logits, temps)
+
+
+@pytest.mark.parametrize("rows,vocab,hidden", [(40, 1000, 512), (150, 100003, 256), (250, 100003, 256), (320, 100003, 256), (200, 1000, 128)])
+def test_lm_head_confidence_of_values_that_are_not_finite(dev, rows, vocab, hidden):
+    """NaN and infinities in rows of x and in W, in each form of the product (few rows, the three tiles, 128 columns): the tokens of the vocabulary pass on the same logits (small
+    integers: exact in any order), which are the largest number's, and its confidences where the logits hold no NaN."""
+    import mdx
+    g = torch.Generator().manual_seed(rows)
+    inf, nan = float("inf"), float("nan")
+    x = torch.randint(-2, 3, (rows, hidden), generator=g).float()
+    w = torch.randint(-2, 3, (vocab, hidden), generator=g).float()
+    x[1], x[2, 5], x[3:5] = nan, nan, 0.0
+    x[3, 7], x[4, 7] = inf, -inf
+    several = {"nan in one entry": (slice(17, 18), nan), "inf": (slice(vocab - 1, vocab), inf), "-inf": (slice(5, None), -inf), "nan in a tile": (slice(0, 256), nan),
+               # what one lane of the matrix instruction holds: four entries of every sixteen
+               "nan in lanes": ([i for i in range(128) if i // 4 % 4 < 2], nan), "nan at the end": (slice(vocab - 1, None), nan), "all nan": (slice(None), nan)}
+    for name, (where, value) in [("finite", (slice(0, 0), 0.0)), *several.items()]:
+        ww = w.clone()
+        ww[where] = value
+        xd, wd = x.bfloat16().to(dev), ww.bfloat16().to(dev)
+        x0, p = mdx.lm_head_confidence(xd, wd)
+        logits = (xd.float().cpu() @ wd.float().cpu().T).bfloat16()
+        t0, tp = mdx.confidence_argmax(logits.to(dev).unsqueeze(1))
+        assert torch.equal(x0, t0.view(-1)), f"{name}: tokens"
+        whole = ~logits.isnan().any(1).to(dev)
+        torch.testing.assert_close(p[whole], tp.view(-1)[whole], rtol=3e-5, atol=0, msg=lambda m: f"{name}: {m}")
