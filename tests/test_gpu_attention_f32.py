@@ -192,6 +192,14 @@ def test_paged_head_widths_outside_the_16bit_kernel(dev, d, dtype):
     _check_paged(dev, [300, 2100, 64], 32, 4, 2, d, dtype, seed=8000 + d, page=256 if d >= 128 else 32)
 
 
+@pytest.mark.parametrize("d", [4, 12, 20, 100, 132, 252])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_paged_head_widths_that_are_odd_multiples_of_four(dev, d, dtype):
+    """Widths that the two half-wavefronts cannot halve into whole loads: the halves are rounded up, their last columns masked."""
+    _check_paged(dev, [300, 2100, 64], 32, 4, 2, d, dtype, seed=8100 + d, page=256 if d >= 128 else 32)
+    _check_paged(dev, [33, 1], 7, 3, 1, d, dtype, seed=8200 + d)
+
+
 def test_paged_fp32_invalid_pages_are_left_out(dev):
     """Keys on a page id outside the pool are excluded; a sequence without any valid page yields zeros."""
     import mdx

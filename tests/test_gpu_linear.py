@@ -55,6 +55,60 @@ def test_linear_says_what_it_does_not_cover(dev):
     assert ops.linear(z(2, 3, 256), z(64, 256)).shape == (2, 3, 64) and ops.linear_gated(z(2, 3, 256), z(64, 256)).shape == (2, 3, 32)
 
 
+@pytest.mark.parametrize("rows,n,k", [(40, 72, 384), (333, 2056, 512), (1100, 4104, 256)])
+def test_rows_of_w_in_a_wider_matrix(dev, rows, n, k):
+    """W with rows further apart than k, rounded, as partial sums, with the SiLU (whose second half of W begins n such rows on) and with the
+    head rows: the results for dense rows, bit for bit."""
+    from mdx import ops
+    _, x, w = _xw(dev, rows, 2 * n, k)
+    wide = torch.full((2 * n, k + 24), float("nan"), dtype=torch.bfloat16, device=dev)
+    wide[:, :k] = w
+    w2 = wide[:, :k]
+    for partials in (False, True):
+        assert torch.equal(ops.linear(x, w2[:n], partials), ops.linear(x, w[:n], partials))
+    assert torch.equal(ops.linear_gated(x, w2), ops.linear_gated(x, w))
+    if rows >= 384:
+        one, pos = torch.ones(128, dtype=torch.bfloat16, device=dev), torch.arange(rows, device=dev)
+        table = torch.rand(rows, 64, device=dev)
+        heads = lambda w: ops.linear_qk_norm_rope_store(x, w[:4096], one, one, 1e-6, table, table, pos, 16, 8, 128)      # noqa: E731
+        assert all(torch.equal(a, b) for a, b in zip(heads(w2), heads(w)))
+
+
+@pytest.mark.parametrize("rows,n,k", [(1537, 520, 256), (3000, 2056, 384), (9000, 1032, 256)])
+def test_rows_beyond_what_the_dispatch_takes(dev, rows, n, k):
+    """The C entries take more rows than pay, and results in wider matrices, whose other columns stay as they are."""
+    import mdx
+    ref, x, w = _xw(dev, rows, 2 * n, k)
+    L, stream = mdx._lib.lib(), torch.cuda.current_stream().cuda_stream
+    for call, want, rel in ((L.mdx_linear, ref[:, :n], 2.0 ** -8), (L.mdx_linear_silu, mdx.silu_and_mul(ref.bfloat16().to(dev)).float().cpu(), 3e-3)):
+        y = torch.full((rows, n + 12), 7.0, dtype=torch.bfloat16, device=dev)
+        assert call(x.data_ptr(), k, w.data_ptr(), k, y.data_ptr(), n + 12, rows, n, k, stream) == 0
+        torch.cuda.synchronize()
+        assert _close(y[:, :n], want, rel) and bool((y[:, n:] == 7.0).all())
+
+
+@pytest.mark.parametrize("rows,n,k", [(20, 72, 384), (130, 136, 2048), (520, 4104, 384), (1100, 4104, 256)])
+def test_values_that_are_not_finite(dev, rows, n, k):
+    """NaN and infinities in a row of x or of W reach that row's or column's results and no others, in every form."""
+    import mdx
+    from mdx import ops
+    inf, nan = float("inf"), float("nan")
+    _, x, w = _xw(dev, rows, 2 * n, k)
+    x[3, 5], x[rows - 1, k - 1], x[4, 7] = nan, inf, -inf
+    w[6, 9], w[n - 1, 0], w[n + 8, 3] = inf, nan, nan
+    ref = x.float().cpu() @ w.float().cpu().T
+
+    def same(got, want, rel):
+        got, plain = got.float().cpu(), want.isfinite()
+        return torch.equal(got.isnan(), want.isnan()) and torch.equal(got[~plain & ~want.isnan()], want[~plain & ~want.isnan()]) and _close(got[plain], want[plain], rel)
+
+    first = ref[:, :n].contiguous()
+    assert same(ops.linear(x, w[:n]), first.bfloat16().float(), 2.0 ** -8)
+    either = ops.linear(x, w[:n], True)
+    assert either.dim() == 2 or same(either.sum(0), first, 2e-6)
+    assert same(ops.linear_gated(x, w), mdx.silu_and_mul(ref.bfloat16().to(dev)).float().cpu(), 3e-3)
+
+
 def test_rows_far_apart(dev):
     """Rows 2^28 elements and more apart: computed by the two calls for few rows, left to the library by the others."""
     import mdx
