@@ -453,7 +453,7 @@ int mdx_silu_and_mul(const void* x, int64_t x_row_stride, void* out, int64_t out
  * mdx_linear rounds the product to bf16, y [rows, n] (row stride a multiple of 4).  mdx_linear_partials leaves it as fp32
  * partial sums over slices of K, partials [splits, rows, n] (dense), for one of the two kernels below that add them up and
  * round the sum to bf16 as the layer's output.  mdx_linear_splits(rows, n, k): the number of slices where that is the faster
- * of the two, 0 where mdx_linear is, -1 where a library's product is the better choice (more than 1536 rows; wide layers from
+ * of the two (mdx_linear is then slower than a library's product for long k and few columns), 0 where mdx_linear is, -1 where a library's product is the better choice (more than 1536 rows; wide layers from
  * 52 GFLOP on) or the shape is not covered.  mdx_linear_silu: w [2 n, k], gate rows then up rows; y [rows, n] = mdx_silu_and_mul of the product, with
  * its rounding points; mdx_linear_silu_supported: covered, and up to 8192 rows.
  * mdx_linear_qk_norm_rope_store: the product of a QKV projection with mdx_qk_norm_rope_store on it in one launch; w holds the q

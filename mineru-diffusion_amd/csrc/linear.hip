@@ -17,6 +17,9 @@
 //   rows  1536  29.8 21.0  79.9  42.3 /  29.9 21.6  99.1 48.7
 //   rows  4096  60.6 35.2 175.1  94.1 /  51.3 35.4 177.7 91.3
 //   rows  8192 119.3 59.0 349.7 167.8 /  99.7 53.3 350.6 145.0
+// (Up to 1536 rows the better of rounded and partial sums.  Rounded where partial sums would be the faster, for a caller that doesn't take them: QKV 32 rows 10.5, 256 12.2, 383 16.3
+// against the library's 14.9; down, whose chain of 96 steps few tiles share, 32 rows 25 / 17, 512 29.5 / 27.5, 1536 54 / 45: a caller that can't take partial sums
+// there does better with the library.)
 #include "linear_tile.h"
 #include "qk_row.h"
 

@@ -9,7 +9,8 @@
 //
 // A workgroup computes a tile of 256 x 256, 128 x 256 or 192 x 192 (x rows by vocabulary rows) over the whole hidden dimension
 // (linear_tile.h) and leaves one 16-byte record per x row; a second, small kernel folds a row's records (about vocab / 256 of them) into x0 /
-// x0_p.  The matrix pipe bounds it, under the board's power limit.
+// x0_p.  What bounds it: the matrix pipe behind one barrier per step, at which all eight wavefronts wait for their LDS reads and loads; at 1024 rows the pipe is busy
+// 50.5 % of 1.205 M active cycles per SIMD (the generated core below: 56.4 % of 1.078 M, at a lower clock).
 #include "lm_head.h"
 #include "linear_tile.h"
 
@@ -98,8 +99,9 @@ __global__ __launch_bounds__(T::kThreads, T::kWaves / 4) void lm_head_confidence
     P.records[(int64_t)row * P.n_slices + at.n] = Record{b.m, b.s, b.idx, 0};
 }
 
-// ---- 128 columns: two steps, less than the tiles above want in flight.  Tiles of 256 x 256 on the generated core of lm_head_core.inc
-//      (one wavefront per SIMD; over 2048 columns 200 us up to 256 rows, 306-314 up to 512, 577 at 1024), two records per row and tile. ----
+// ---- 128 columns: two steps, which leave a tile's epilogue most of the time.  Tiles of 256 x 256 on the generated core of lm_head_core.inc
+//      (one wavefront per SIMD), two records per row and tile.  151 936 entries, us, this core / a 256 x 256 tile of linear_tile.h with two steps in LDS: 256 rows 38 / 40,
+//      500 57 / 60, 1024 101 / 110, 4096 349 / 392. ----
 #include "lm_head_core.inc"
 
 constexpr int kThreads = 256;

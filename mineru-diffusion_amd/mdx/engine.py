@@ -323,7 +323,9 @@ class Decoder(nn.Module):
 # ----------------------------------------------------------------------------- engine
 IDLE, DENOISING, CACHING = 0, 1, 2      # MDX_PHASE_* of include/mdx.h: the per-lane state of the device loop
 N_STOP = 4                              # stop-token ids per sequence that the device loop can check
-FUSED_HEAD_MIN_ROWS, FUSED_HEAD_FEW_ROWS = 384, 256      # rows of a pass from which, and up to which, the fused vocabulary head is the faster
+# rows of a pass from which, and up to which, the fused vocabulary head is taken.  Fused / library product + vocabulary pass, us: 192 rows 181 / 199, 256 195 / 220,
+# 272 258 / 244, 320 258 / 255, 352 263 / 275, 383 262 / 277, 512 305 / 342
+FUSED_HEAD_MIN_ROWS, FUSED_HEAD_FEW_ROWS = 384, 256
 FUSED_HEAD_WHOLE_ROWS = 32              # rows that it holds whole (8 rows 120 us, 32 rows 119); compacting takes six launches of a pass, 66.4 against 65.5 ms for one request
 
 
@@ -657,8 +659,9 @@ class BlockDiffusionEngine:
 
     def _fused_head(self, rows: int) -> bool:
         """Projection and confidence in one pass that never writes the logits (mdx_lm_head_confidence), for bf16 weights
-        without sampling noise.  By default taken where it is the faster of the two: from 384 rows on, and up to 256 rows
-        (the kernel's form for up to 128, or one tile of it); between them the library GEMM + the vocabulary pass win.
+        without sampling noise.  By default from 384 rows on, where it is the faster of the two, and up to 256 (the form for up to
+        128 rows, then tiles of 128 or 192 rows or one of 256); between them the library GEMM + the vocabulary pass
+        win, or come within 5 %.
         A caller's own fused_head_min_rows is the one limit: never below it, always from it on."""
         few = self.fused_head_min_rows == FUSED_HEAD_MIN_ROWS and rows <= FUSED_HEAD_FEW_ROWS
         return (self.fused_head and self.gumbel_seed is None and (few or rows >= self.fused_head_min_rows)

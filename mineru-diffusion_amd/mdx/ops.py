@@ -66,7 +66,8 @@ def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
 # shape is not covered.
 def linear(x: torch.Tensor, weight: torch.Tensor, partials: bool = False) -> torch.Tensor | None:
     """x . weight^T (nanovllm/layers/linear.py) for up to 1536 rows (wide layers: up to 52 GFLOP): bf16 [..., n], or with
-    `partials` what is the faster of that and partial sums (one dimension more than x)."""
+    `partials` what is the faster of that and partial sums (one dimension more than x).  Without, a layer of long K and few
+    columns is slower than the library's (2048 x 6144: 25 us against 17 at 32 rows, 54 against 45 at 1536)."""
     return _host().linear(x, weight, partials)
 
 
