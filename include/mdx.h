@@ -176,13 +176,11 @@ int mdx_paged_block_attn(const void* q, void* o, const void* k_cache, const void
                          void* workspace, int64_t workspace_bytes, mdx_stream_t stream);
 
 /*
- * The same in ONE launch where that pays: with about a (sequence, head group) pair per CU or
- * more, where only sequences far longer than the rest are split, the last split of a pair to
+ * The same in ONE launch where that pays: the last split of a (sequence, head group) pair to
  * finish merges the pair's partials itself instead of a second (combine) launch; no workgroup
- * waits for another.  In a decode pass whose sequences stay whole (the usual case at batch 32)
- * this saves the launch of a kernel that finds nothing to do, 28 times per forward pass.  With
- * fewer pairs, where every sequence is split, the call makes the same two launches as
- * mdx_paged_block_attn (counting in costs each split workgroup a device-wide release).
+ * waits for another.  With about a pair per CU or more this is always done
+ * (mdx_paged_block_attn_needs_counters: 1), with fewer where sequences come to few splits and the counters
+ * are there; otherwise the call makes the same two launches as mdx_paged_block_attn.
  *
  * counters: mdx_paged_block_attn_counter_bytes(bs, Hq, Hkv) bytes of device memory (one fp32 per
  * sequence, head group and tile of 32 queries, sized for Sq = 128), 4-byte
@@ -191,6 +189,7 @@ int mdx_paged_block_attn(const void* q, void* o, const void* k_cache, const void
  * own.  workspace as above.  Same results bit for bit as mdx_paged_block_attn.
  */
 int64_t mdx_paged_block_attn_counter_bytes(int32_t bs, int32_t num_q_heads, int32_t num_kv_heads);
+int32_t mdx_paged_block_attn_needs_counters(int32_t bs, int32_t sq, int32_t num_q_heads, int32_t num_kv_heads, int32_t max_pages, int32_t page_size);
 int mdx_paged_block_attn_single_launch(const void* q, void* o, const void* k_cache, const void* v_cache,
                                        int64_t q_stride_b, int64_t q_stride_s, int64_t q_stride_h,
                                        int64_t o_stride_b, int64_t o_stride_s, int64_t o_stride_h,

@@ -539,6 +539,10 @@ PyObject* sparse_attn_varlen(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // request does not fit it, or while a graph is being captured and that stream has no buffer yet (it could not be
 // zeroed outside the graph): the caller then takes the two-launch entry point -- run the forward once on the capture
 // stream before capturing.
+bool capturing(const Tensor& like) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(static_cast<hipStream_t>(stream_of(like)), &status) != hipSuccess || status != hipStreamCaptureStatusNone;
+}
 constexpr int64_t kCounterFloats = 64 * 256;   // the single-launch path exists for up to 64 sequences; 256 head groups is far beyond any model
 Tensor counters_for(const Tensor& like, int64_t bytes) {
     static auto* kept = new std::map<std::pair<int, void*>, Tensor>();      // (never destroyed: the driver may be gone at exit)
@@ -549,8 +553,7 @@ Tensor counters_for(const Tensor& like, int64_t bytes) {
     std::lock_guard<std::mutex> guard(lock);
     auto it = kept->find(key);
     if (it != kept->end()) return it->second;
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &status) != hipSuccess || status != hipStreamCaptureStatusNone) return Tensor();
+    if (capturing(like)) return Tensor();
     Tensor t = at::zeros({kCounterFloats}, at::TensorOptions().dtype(at::kFloat).device(like.device()));
     kept->emplace(key, t);
     return t;
@@ -577,7 +580,10 @@ Tensor paged(const Tensor& q_, const Tensor& k_cache, const Tensor& v_cache, con
     const Tensor ws = bytes > 0 ? make(q, at::kByte, bytes) : Tensor();
     Tensor counters;
     if (counters_arg == Py_None) {         // more than 64 sequences never take the single-launch path
-        if (bs <= 64) counters = counters_for(q, mdx_paged_block_attn_counter_bytes((int32_t)bs, (int32_t)hq, (int32_t)hkv));
+        // Launches that may do without (mdx_paged_block_attn_needs_counters) leave the kept buffer out of graphs: two graphs captured on one
+        // stream may be replayed beside each other.
+        if (bs <= 64 && (!capturing(q) || mdx_paged_block_attn_needs_counters((int32_t)bs, (int32_t)sq, (int32_t)hq, (int32_t)hkv, (int32_t)bt.size(1), (int32_t)page)))
+            counters = counters_for(q, mdx_paged_block_attn_counter_bytes((int32_t)bs, (int32_t)hq, (int32_t)hkv));
     } else if (counters_arg != Py_False) {
         counters = tensor(counters_arg);
         NEED(counters.scalar_type() == at::kFloat && counters.is_contiguous() && counters.device() == q.device());
@@ -611,12 +617,12 @@ PyObject* flash_attn_with_kvcache(PyObject*, PyObject* const* a, Py_ssize_t n) {
     });
 }
 
-// q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale | None, the weights of the two products behind the call
+// q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale | None, the weights of the two products behind the call, counters
 PyObject* flash_attn_with_kvcache_read_ahead(PyObject*, PyObject* const* a, Py_ssize_t n) {
-    ARGS(8);
+    ARGS(9);
     return guarded([&]() -> PyObject* {
         const Tensor &next = tensor(a[6]), &then = tensor(a[7]);
-        return wrap(paged(tensor(a[0]), tensor(a[1]), tensor(a[2]), tensor(a[3]), tensor(a[4]), a[5], Py_None, false, &next, &then));
+        return wrap(paged(tensor(a[0]), tensor(a[1]), tensor(a[2]), tensor(a[3]), tensor(a[4]), a[5], a[8], false, &next, &then));
     });
 }
 

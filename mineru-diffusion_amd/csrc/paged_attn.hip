@@ -36,6 +36,7 @@
 //    (m, l, O) that a second, small kernel combines.
 #include "mdx_common.h"
 #include "attn_tile.h"
+#include <type_traits>
 
 namespace {
 
@@ -51,6 +52,15 @@ constexpr int kLeastPiece = 64;
 // Sequences are only cut if that takes more off the longest workgroup than the partials of them all cost (8 x 300 and 16 x 600
 // keys stay whole).
 template <typename T> __host__ __device__ __forceinline__ bool stay_whole(T longest, T piece, int sequences) { return longest - piece < T(64 + 12 * sequences); }
+
+// About a (sequence, head group) pair per CU and more: sequences are left whole -- no partials, nothing to merge -- unless the longest is kWholeFactor
+// times what a resident workgroup's even share of the keys comes to (or 1.2 times the mean, where that is more); then all are cut into pieces
+// of kShareFactor shares and kShareKeys keys.  The layer, us, cut at 1.25 times the mean only / by shares: 24 sequences of 1250-5000 keys 86 / 71, 550-2200
+// 49 / 42, 32 of 375-1500 45 / 38, 825-3300 71 / 64, 33 of 1000-4000 100 / 78, 40 of 500-3500 93 / 76, 48 of 550-2200 85 / 68, 64 of 300-2300 89 / 78;
+// equal lengths stay whole, level.  (Shares of 1.05 without the keys: 33 of 1000-4000 75, but 24 of 375-1500 38 instead of 33, 32 of those 43
+// instead of 38: a second workgroup on a CU that holds one at a time costs its start and end.)
+constexpr float kWholeFactor = 1.33f, kShareFactor = 1.2f;
+constexpr int kShareKeys = 192;
 
 // Sum over the 64 lanes: DPP shifts inside the rows of 16 lanes, the two row broadcasts, the total from lane 63
 // (six additions, no LDS traffic: the butterfly of cross-lane LDS permutes it replaces sat in every workgroup's start).
@@ -117,6 +127,8 @@ struct PagedParams {
     // 1000 to 3000 keys in a table 12 pages wide 51 -> 42 us; no shape of the sweep slower.  Cutting each sequence
     // into equal pieces instead of full splits and a short remainder was measured too and loses: the remainders
     // start last and fill the tail.)
+    // < 0: about a pair per CU or more, minus the workgroups that are resident (kWholeFactor).  (One field for both: with four bytes more of arguments
+    // the launch with readers takes 0.2 us longer.)
     int fit_slots;
     // Single-launch mode: one arrival counter per (sequence, head group), zero between launches.  The
     // last split of a pair to arrive merges the pair's partials itself.  float for the same reason.
@@ -183,53 +195,12 @@ template <int COLS> struct Fold {
     __device__ __forceinline__ float inverse() const { return L > 0.f ? 1.0f / L : 0.f; }   // no valid key at all (every page id invalid): zeros, like a context of 0
 };
 
-// Single-launch merge: folds the nv split partials of query s of (sequence b, head hq), which other workgroups of this launch
-// have just written; the caller's 8 threads c = 0..7 of a query take 16 consecutive d values each.
-template <typename E>
-__device__ __forceinline__ void combine_query(const PagedParams& P, int b, int hq, int qt, int s, int c, int nv)
-{
-    if (c * 16 >= P.head_dim) return;
-    const int64_t slot0 = (((int64_t)b * P.num_q_heads + hq) * P.nqt + qt) * P.nsplit;
-    Fold<16> F;
-    F.init();
-    for (int i0 = 0; i0 < nv; i0 += 4) {
-        float m[4], l[4];
-        f32x4 po[4][4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int64_t slot = slot0 + min(i0 + i, P.nsplit - 1);
-            const float* ml = P.part_ml + (slot * kQTile + s) * 2;
-            const float* src = P.part_o + (slot * kQTile + s) * kHeadDim + c * 16;
-            m[i] = __hip_atomic_load(ml, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            l[i] = __hip_atomic_load(ml + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) po[i][k] = load_agent(src + 4 * k);
-        }
-        // the asm loads are invisible to the compiler's own counting: wait here, and tie every loaded
-        // value to the wait so that no use of it can be scheduled above it
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int k = 0; k < 4; ++k) asm volatile("s_waitcnt vmcnt(0)" : "+v"(po[i][k]) :: "memory");
-        F.take4(m, l, po, nv - i0);
-    }
-    const float inv = F.inverse();
-    typedef typename Elem16<E>::vec8 vec8;
-    __bf16* dst = P.o + (int64_t)b * P.o_sb + (int64_t)(qt * kQTile + s) * P.o_ss + (int64_t)hq * P.o_sh + c * 16;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        vec8 out;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) out[e] = (E)(F.acc[8 * h + e] * inv);
-        *reinterpret_cast<vec8*>(dst + 8 * h) = out;
-    }
-}
-
 // WAVES = 4 (two workgroups per CU) or 8 (one workgroup per CU, 128-key tiles: for launches with about
 // one workgroup per CU, where a CU would otherwise hold four wavefronts only).  Tiles hold 32 keys per
 // key slice (WAVES / HPW slices); two 64-key tile buffers fit a CU twice, two 128-key ones once.
+// MERGE: single launch, the last split of a pair merges them (a kernel of its own: one sequence's launch is 0.3 us longer with that code in it).
 // AHEAD: none, or ReadAhead: workgroups behind those of the attention read what the launches behind it need.
-template <typename E, int HPW, int DEPTH, int WAVES, typename... AHEAD>
+template <typename E, int HPW, int DEPTH, int WAVES, bool MERGE, typename... AHEAD>
 __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_block_attn_kernel(const PagedParams P, const AHEAD... ahead)
 {
     if constexpr (sizeof...(AHEAD) > 0) {
@@ -262,8 +233,9 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
         // lengths beyond the page table name keys that do not exist: clipped here and below
         const int ctx_l = lane < P.bs ? min(max(0, P.context_lens[lane]), P.max_pages * P.page_size) : 0;
         ctx_all = ctx_l;
+        bool cut = true;                            // false: every sequence is known to be one piece
         auto splits_of_lane = [&]() { return lane < P.bs ? max(1, (ctx_l + span - 1) / span) : 0; };   // (padding rows get one)
-        int n;
+        int n = 0;
         if (P.fit_slots > 0) {
             // One size of piece for all sequences.  A launch of few keys is a chain of latencies as long as its longest
             // workgroup, one of many keys a stream that more and shorter workgroups only disturb: over batches of 1 to 20
@@ -288,34 +260,50 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
             }
             if (blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) *P.span_out = (float)span;
         } else {
-            if (P.span_out) {
-                // With a (sequence, head group) pair per CU the sequences are best left whole (no partials,
-                // nothing to combine) -- unless one of them is much longer than the rest and would keep
-                // its CU busy long after the others are done.  Only the device knows the lengths: the
-                // split grows from the host's size to 1.25 x the mean length, so that only sequences
-                // well above the mean are cut, into pieces of about the mean.
-                const int live = wave_sum(ctx_l > 0 ? 1 : 0);
-                const int mean = wave_sum(ctx_l) / max(live, 1);
-                span = max(span, (mean + mean / 4 + kChunkAlign - 1) / kChunkAlign * kChunkAlign);
+            if (P.fit_slots < 0) {
+                // (kWholeFactor above says why; the host's split is what keeps the longest within nsplit pieces)
+                const int total = wave_sum(ctx_l), longest = wave_max(ctx_l), live = wave_sum(ctx_l > 0 ? 1 : 0);
+                const float share = (float)total * (float)gridDim.x * __builtin_amdgcn_rcpf((float)-P.fit_slots);
+                const float mean = (float)total * __builtin_amdgcn_rcpf((float)max(live, 1));
+                span = max(span, ((int)(kShareFactor * share) + kShareKeys + 63) & ~63);
+                if ((float)longest <= kWholeFactor * fmaxf(share, 0.9f * mean)) span = max(span, longest);
+                cut = longest > span;
                 if (blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) *P.span_out = (float)span;
             }
-            n = splits_of_lane();
+            if (!MERGE) n = splits_of_lane();
         }
-        // Launch order: the first split of every sequence, then the second of those that have one, ...
-        // The last split of a sequence is its short remainder, so the workgroups that start late
-        // (when there are more of them than the chip holds at once) are the short ones.
+        // the j-th (sequence, split) pair in launch order; `has`: the lanes (sequences) that own a pair of the kind that is next in it
         int j = blockIdx.y, level = 0;
         b = -1;
-        for (; level < P.nsplit; ++level) {
-            const unsigned long long has = __ballot(n > level);
+        auto among = [&](unsigned long long has) {
             const int c = __popcll(has);
             if (j < c) {
                 const int before = __popcll(has & ((1ull << lane) - 1ull));
                 const unsigned long long hit = __ballot(((has >> lane) & 1ull) != 0 && before == j);
                 b = __ffsll((long long)hit) - 1;
-                break;
+                return true;
             }
             j -= c;
+            return false;
+        };
+        if constexpr (MERGE) {
+            // Heaviest first: all whole pieces, then the remainders (and sequences shorter than a piece) by eighths of a piece, so that
+            // those which start late, when there are more workgroups than the chip holds at once, are the short ones of all.  (16 sequences of
+            // 375-1500 keys 30.3 us in the order below, 26.2 in this one.)
+            const int whole = cut ? ctx_l / span : ctx_l == span && ctx_l > 0, rest = ctx_l - whole * span;
+            if (j >= (cut ? wave_sum(lane < P.bs ? whole + (rest > 0 || whole == 0) : 0) : P.bs)) return;
+            bool found = false;
+            for (; !found && level < P.nsplit; ++level) found = among(__ballot(whole > level));
+            if (found) {
+                --level;
+            } else {
+                const int eighth = lane < P.bs && (rest > 0 || whole == 0) ? min(7, (int)((float)rest * 8.f * __builtin_amdgcn_rcpf((float)span))) : -1;
+                for (int e = 7; !found && e >= 0; --e) found = among(__ballot(eighth == e));
+                if (found) level = __builtin_amdgcn_readlane(whole, b);
+            }
+        } else {
+            // the first split of every sequence, then the second of those that have one, ...: the last split of a sequence is its remainder
+            for (; level < P.nsplit; ++level) if (among(__ballot(n > level))) break;
         }
         if (b < 0) return;                          // past the last (sequence, split) pair
         split = level;
@@ -336,9 +324,10 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
         }
         return;
     }
-    const int key_begin = split * span;
+    // (uniform in the compiler's eyes too, or the page table comes through vector loads)
+    const int key_begin = __builtin_amdgcn_readfirstlane(split * span);
     if (key_begin >= ctx) return;
-    const int key_end = min(ctx, key_begin + span);
+    const int key_end = __builtin_amdgcn_readfirstlane(min(ctx, key_begin + span));
     const int kvh = (hg * HPW) / P.heads_per_kv;
 
     const int qrow = qt * kQTile + r;               // this lane's query of the sequence's block
@@ -444,6 +433,10 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
     // and every slice stores what it folded.  (A tree of pairwise merges with 4-byte LDS accesses and three barriers,
     // all output from one wavefront, took 2.7 us of every workgroup's end.)  All slices sum in the same order, so they
     // agree on the head's m and l bit for bit.
+    // (single launch: how many splits of this pair have counted themselves in -- asked for here, needed behind the merge)
+    __shared__ int counted;
+    float* const counter = MERGE ? P.arrive + ((int64_t)b * n_groups + hg) * P.nqt + qt : nullptr;
+    if (MERGE && n_valid_splits > 1 && tid == 0) counted = (int)__hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     st.l[0] = both_halves_sum(st.l[0]);          // a state is now (m, l, O) per query
     // Exchange layout per wavefront: O as [d tile][group][64 lanes][4] floats, then m, l as [64].
     constexpr int kStateFloats = 4 * 16 * 64 + 2 * 64;
@@ -462,6 +455,7 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
         dst[4 * 16 * 64 + 64 + lane] = st.l[0];
     }
     __syncthreads();
+    f32x4 own[4 / KW][4];                           // what this slice folds: d tiles kw, kw + KW, ...
     {
         float w[KW];                                // weights of the KW states: 2^(m_s - M)
         float M = kMinusBig;
@@ -476,79 +470,131 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
         st.m[0] = M;
         st.l[0] = l;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            if (t % KW != kw) continue;             // (uniform per wavefront)
+        for (int t = 0; t < 4 / KW; ++t)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                own[t][g] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int s = 0; s < KW; ++s)
-                    acc += *reinterpret_cast<const f32x4*>(xch + s * kStateFloats + ((t * 4 + g) * 64 + lane) * 4) * w[s];
-                st.o[0][t][4 * g] = acc.x; st.o[0][t][4 * g + 1] = acc.y; st.o[0][t][4 * g + 2] = acc.z; st.o[0][t][4 * g + 3] = acc.w;
+                    own[t][g] += *reinterpret_cast<const f32x4*>(xch + s * kStateFloats + (((kw + KW * t) * 4 + g) * 64 + lane) * 4) * w[s];
             }
-        }
     }
 
     // ---- output: slice kw holds, and stores, the d tiles kw, kw + KW, ... of its head ----------------
-    if (n_valid_splits == 1) {
+    constexpr int kMine = 4 / KW;                // d tile kw + KW * t is `t` below
+    auto store_rows = [&](const f32x4 (&acc)[kMine][4], float l) {
         if (!row_ok) return;
-        const float inv = st.l[0] > 0.f ? 1.0f / st.l[0] : 0.f;   // no valid key at all: zeros
+        const float inv = l > 0.f ? 1.0f / l : 0.f;              // no valid key at all: zeros
         __bf16* orow = P.o + (int64_t)b * P.o_sb + (int64_t)qrow * P.o_ss + (int64_t)head * P.o_sh;
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-            if (dt % KW != kw) continue;
+        for (int t = 0; t < kMine; ++t)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
+                const int d = d_of_reg(kw + KW * t, 4 * g, H);
                 typename Elem16<E>::vec4 out;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) out[e] = (E)(st.o[0][dt][4 * g + e] * inv);
-                if (d_of_reg(dt, 4 * g, H) < P.head_dim) *reinterpret_cast<typename Elem16<E>::vec4*>(orow + d_of_reg(dt, 4 * g, H)) = out;
+                for (int e = 0; e < 4; ++e) out[e] = (E)(acc[t][g][e] * inv);
+                if (d < P.head_dim) *reinterpret_cast<typename Elem16<E>::vec4*>(orow + d) = out;
             }
-        }
-        return;
-    }
-    if (row_ok) {
-        const int64_t slot = (((int64_t)b * P.num_q_heads + head) * P.nqt + qt) * P.nsplit + split;
-        float* po = P.part_o + (slot * kQTile + r) * kHeadDim;
+    };
+    if (n_valid_splits == 1) { store_rows(own, st.l[0]); return; }
+    const int64_t slot0 = (((int64_t)b * P.num_q_heads + head) * P.nqt + qt) * P.nsplit;
+    if constexpr (!MERGE) {                      // two launches: the combine kernel follows
+        if (row_ok) {
+            float* po = P.part_o + ((slot0 + split) * kQTile + r) * kHeadDim;
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-            if (dt % KW != kw) continue;
+            for (int t = 0; t < kMine; ++t)
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const f32x4 out = {st.o[0][dt][4 * g], st.o[0][dt][4 * g + 1], st.o[0][dt][4 * g + 2], st.o[0][dt][4 * g + 3]};
-                if (P.arrive) store_agent(po + d_of_reg(dt, 4 * g, H), out);
-                else *reinterpret_cast<f32x4*>(po + d_of_reg(dt, 4 * g, H)) = out;
-            }
+                for (int g = 0; g < 4; ++g) *reinterpret_cast<f32x4*>(po + d_of_reg(kw + KW * t, 4 * g, H)) = own[t][g];
+            if (kw == 0 && H == 0) *reinterpret_cast<float2*>(P.part_ml + ((slot0 + split) * kQTile + r) * 2) = float2{st.m[0], st.l[0]};
         }
-        if (kw == 0 && H == 0) {
-            float* ml = P.part_ml + (slot * kQTile + r) * 2;
-            if (P.arrive) {
-                __hip_atomic_store(ml, st.m[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(ml + 1, st.l[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            } else {
-                *reinterpret_cast<float2*>(ml) = float2{st.m[0], st.l[0]};
-            }
-        }
-    }
-    if (!P.arrive) return;                       // two-launch mode: the combine kernel follows
+    } else {
 
-    // ---- single-launch mode: the last split of this (sequence, head group) to arrive merges them ----
-    // Every writer waits until its (written-through) partials have reached memory, then the workgroup
-    // counts itself in; the workgroup that finds itself last reads all partials of the pair with
-    // agent-scope loads.  No cache-wide fence on either side, and nobody waits for anybody: a
-    // workgroup that is not last leaves.
+    // ---- single launch: the last split of this (sequence, head group) to arrive merges them ----
+    // A split that finds all others counted in is the last, keeps its state in its registers and folds theirs into the result.  Any other
+    // writes its partials (in the order of its registers, 1 KB per store: nobody but this kernel reads them), waits until they have reached
+    // memory, and counts itself in; it may still turn out to be the last by that count, and folds then.  No cache-wide
+    // fence on either side, and nobody waits for anybody.  What this costs falls at the end of a launch: one trip to memory for
+    // the other splits' partials, four at a time, by the workgroup that has just finished, where every split used to write its own, wait, count,
+    // and the last to read them all back in two rounds of smaller loads (32 sequences of 375-1500 keys, same cuts: 45 -> 39 us).
     __shared__ int i_am_last;
-    wait_vector_memory();
-    __syncthreads();
-    float* counter = P.arrive + ((int64_t)b * n_groups + hg) * P.nqt + qt;
-    if (tid == 0) i_am_last = atomicAdd(counter, 1.0f) == (float)(n_valid_splits - 1) ? 1 : 0;
-    __syncthreads();
-    if (!i_am_last) return;
-    for (int e = tid; e < HPW * 256; e += kThreads) {
-        const int s = (e & 255) >> 3;
-        if (qt * kQTile + s < P.sq) combine_query<E>(P, b, hg * HPW + (e >> 8), qt, s, e & 7, n_valid_splits);
+    auto part = [&](int sp, int t, int g) { return P.part_o + (((slot0 + sp) * 16 + (kw + KW * t) * 4 + g) * 64 + lane) * 4; };
+    if (counted != n_valid_splits - 1) {
+#pragma unroll
+        for (int t = 0; t < kMine; ++t)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) store_agent(part(split, t, g), own[t][g]);
+        if (kw == 0 && H == 0) {
+            float* ml = P.part_ml + ((slot0 + split) * kQTile + r) * 2;
+            __hip_atomic_store(ml, st.m[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(ml + 1, st.l[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        wait_vector_memory();
+        __syncthreads();
+        if (tid == 0) i_am_last = atomicAdd(counter, 1.0f) == (float)(n_valid_splits - 1) ? 1 : 0;
+        __syncthreads();
+        if (!i_am_last) return;
     }
+    // the arithmetic of Fold::take4, split by split in groups of four, whoever is last: the bits of the combine kernel
+    float M = kMinusBig, L = 0.f;
+    f32x4 acc[kMine][4];
+#pragma unroll
+    for (int t = 0; t < kMine; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) acc[t][g] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i0 = 0; i0 < n_valid_splits; i0 += 4) {
+        float m[4], l[4];
+        f32x4 po[4][kMine][4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int sp = min(i0 + i, n_valid_splits - 1);
+            const float* ml = P.part_ml + ((slot0 + sp) * kQTile + r) * 2;
+            m[i] = __hip_atomic_load(ml, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            l[i] = __hip_atomic_load(ml + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (i0 + i < n_valid_splits && i0 + i != split) {
+#pragma unroll
+                for (int t = 0; t < kMine; ++t)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) po[i][t][g] = load_agent(part(sp, t, g));
+            }
+        }
+        // the asm loads are invisible to the compiler's own counting: wait here, and tie every loaded
+        // value to the wait so that no use of it can be scheduled above it
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int t = 0; t < kMine; ++t)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) asm volatile("s_waitcnt vmcnt(0)" : "+v"(po[i][t][g]) :: "memory");
+        float Mn = M;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (i0 + i == split) { m[i] = st.m[0]; l[i] = st.l[0]; }
+            if (i0 + i < n_valid_splits) Mn = fmaxf(Mn, m[i]);
+        }
+        const float keep = __builtin_amdgcn_exp2f(M - Mn);
+        M = Mn;
+        L *= keep;
+#pragma unroll
+        for (int t = 0; t < kMine; ++t)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) acc[t][g] *= keep;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (i0 + i >= n_valid_splits) break;
+            const float w = __builtin_amdgcn_exp2f(m[i] - M);
+            L = __builtin_fmaf(w, l[i], L);
+#pragma unroll
+            for (int t = 0; t < kMine; ++t)
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[t][g][e] = __builtin_fmaf(w, i0 + i == split ? own[t][g][e] : po[i][t][g][e], acc[t][g][e]);
+        }
+    }
+    store_rows(acc, L);
     if (tid == 0) __hip_atomic_store(counter, 0.f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // ready for the next launch
+    }
 }
 
 // Folds the split partials: a workgroup takes ROWS queries of a (sequence, head), a thread four columns of one of them.  The
@@ -636,6 +682,14 @@ int pick_chunk(int bs, int head_groups, int max_pages, int page_size, bool* devi
     if (2 * chunk >= max_keys && (int64_t)bs * head_groups >= (cus * 25) / 32) chunk = whole;   // two short splits only to fill CUs
     return (int)chunk;
 }
+
+// Where the kernel picks the pieces of few sequences: whether the last split of a pair merges them (single launch) or a combine launch does.  One
+// workgroup reads what the combine launch reads through many, so it is for enough pairs to be done next to each other, and for
+// sequences of few pieces.  The layer, us, combine launch / merging: tables of 768 keys 8 sequences 22.2 / 19.9, 16: 27.1 / 22.8, 20: 30.3 / 25.8; of 1280 keys 16 of
+// a quarter to all of that 29.7 / 24.2; of 2304 keys 8: 31.1 / 28.0, 16: 42.2 / 41.0, 6: 26.8 / 25.5; but 4 of 1280 20.2 / 20.9, one 15.8 / 19.3, 12 of 3328 41.9 / 43.8,
+// 16 of 832-3288 41.7 / 42.8.
+constexpr int64_t kMergeKeys = 2560;
+bool merges_itself(int64_t pairs, int64_t max_keys, int cus) { return pairs >= cus * 3 / 16 && max_keys <= kMergeKeys; }
 
 // Partial slots per sequence: what the host's split needs and, where the kernel cuts by the lengths (up to 64 sequences, not
 // device_span), what its own choice of 4 sqrt(total keys) can need, sqrt(longest) / 4 (beyond 16 K keys the pieces grow) -- as far as that keeps the launch's partials
@@ -746,6 +800,11 @@ int launch_paged_ahead(const void* q, void* o, const void* k_cache, const void* 
     P.head_dim = head_dim;
     P.c = scale * kLog2e;
     P.part_o = nullptr; P.part_ml = nullptr; P.span_out = nullptr; P.arrive = nullptr; P.fit_slots = 0;
+    // Up to one (sequence, head group) pair per CU: workgroups of 8 wavefronts on 128-key tiles, so that a
+    // CU that holds a single workgroup still has two wavefronts per SIMD (batch 32 x 8 KV heads: 79 -> 69 us
+    // on equal lengths); with more pairs than CUs the second round costs more than that gains.
+    const bool eight = device_span && (int64_t)bs * wg_per_pair <= cus;
+    const int resident = cus * (HPW == 2 && !eight ? 2 : 1);           // workgroups at once
     if (P.nsplit > 1) {
         const int64_t n_slots = (int64_t)bs * num_q_heads * P.nqt * P.nsplit;
         const int64_t need = n_slots * kQTile * (kHeadDim + 2) * (int64_t)sizeof(float) + 16;
@@ -754,34 +813,32 @@ int launch_paged_ahead(const void* q, void* o, const void* k_cache, const void* 
         MDX_REQUIRE(mdx::aligned16(workspace), MDX_EWORKSPACE, "paged_block_attn: workspace not 16-byte aligned");
         P.part_o = static_cast<float*>(workspace);
         P.part_ml = P.part_o + n_slots * kQTile * kHeadDim;
-        if (!device_span && bs <= 64) P.fit_slots = cus * (HPW == 2 ? 2 : 1);        // workgroups resident at once
-        if (device_span || P.fit_slots > 0) P.span_out = P.part_ml + n_slots * kQTile * 2;
+        if (device_span) P.fit_slots = -resident;
+        else if (bs <= 64) P.fit_slots = resident;
+        if (P.fit_slots != 0) P.span_out = P.part_ml + n_slots * kQTile * 2;
         // Single launch: the partials are written through with agent-scope stores and read back with
         // agent-scope loads, so counting in costs a workgroup the wait for its own stores and one atomic,
-        // not a device-wide release (a write-back walk of its XCD's L2).  Where only outliers are cut
-        // (device_span) that beats the combine launch (ragged batch of 32: 93 -> 80 us, and a launch
-        // whose sequences stay whole pays nothing).  Where every sequence is split the merges all fall
-        // at the end of the launch, one after the other behind the written-through stores (config 2:
-        // 61 us against 49 with the combine launch; with full release fences it was 145), so those
-        // launches keep the combine kernel.
+        // not a device-wide release (a write-back walk of its XCD's L2).  With about a pair per CU that always beats the combine launch (24 sequences of
+        // 1250-5000 keys 75 / 72 us, 48 of 550-2200 74 / 68, and sequences that stay whole pay nothing); with fewer it does for kMergePairs and more pairs
+        // whose sequences come to few pieces (kMergeKeys).  Those launches take two where there are no counters to use.
+        const int64_t pairs = (int64_t)bs * wg_per_pair, need_c = pairs * (int64_t)sizeof(float);
+        const bool have_counters = counters && counter_bytes >= need_c && ((uintptr_t)counters & 3) == 0;
         if (single_launch && device_span) {
-            const int64_t need_c = (int64_t)bs * wg_per_pair * (int64_t)sizeof(float);
             MDX_REQUIRE(counters && counter_bytes >= need_c, MDX_EWORKSPACE,
                         "paged_block_attn: %lld bytes of arrival counters needed, %lld given", (long long)need_c, (long long)counter_bytes);
             MDX_REQUIRE(((uintptr_t)counters & 3) == 0, MDX_EWORKSPACE, "paged_block_attn: counters not 4-byte aligned");
+            P.arrive = static_cast<float*>(counters);
+        } else if (single_launch && P.fit_slots > 0 && have_counters && merges_itself(pairs, (int64_t)max_pages * page_size, cus)) {
             P.arrive = static_cast<float*>(counters);
         }
     }
     // head group fastest, then the dense (sequence, split) index
     MDX_REQUIRE((int64_t)bs * P.nsplit <= 65535, MDX_EUNSUPPORTED, "paged_block_attn: bs * splits %lld > 65535", (long long)bs * P.nsplit);
-    // With device-chosen splits of at least 1.25 x the mean length, sum_b ceil(len_b / split) <= 1.8 bs:
-    // the dense numbering never needs more than 2 bs (sequence, split) pairs, whatever nsplit allows.
-    const int pairs_y = device_span ? (bs * P.nsplit < 2 * bs ? bs * P.nsplit : 2 * bs) : bs * P.nsplit;
+    // With pieces of kShareFactor shares and more there are at most 1 / kShareFactor cuts per workgroup that is resident of a head group,
+    // whatever nsplit allows.
+    const int64_t most_pairs = bs + (int64_t)((double)resident / (kShareFactor * (double)wg_per_pair)) + 1;
+    const int pairs_y = device_span && most_pairs < (int64_t)bs * P.nsplit ? (int)most_pairs : bs * P.nsplit;
     const dim3 grid((unsigned)(num_q_heads / HPW * P.nqt), (unsigned)pairs_y);
-    // Up to one (sequence, head group) pair per CU: workgroups of 8 wavefronts on 128-key tiles, so that a
-    // CU that holds a single workgroup still has two wavefronts per SIMD (batch 32 x 8 KV heads: 79 -> 69 us
-    // on equal lengths); with more pairs than CUs the second round costs more than that gains.
-    const bool eight = device_span && (int64_t)bs * wg_per_pair <= cus;
     const unsigned n_heads = (unsigned)(bs * num_q_heads * P.nqt);
     // Reading ahead, by rows of the pass (kReadAhead*).  Engine, ms per generation without / with, contexts of 1088 and more in tables of 2048: one request
     // 68.0 / 66.2, two 79.8 / 78.2, three 96.1 / 91.0, four 100.2 / 95.9, six 121.8 / 119.8, eight 132.8 / 130.7; of 32: one 61.6 / 60.7, four 82.2 / 77.9,
@@ -805,16 +862,18 @@ int launch_paged_ahead(const void* q, void* o, const void* k_cache, const void* 
     }
     if (pairs_y + readers > 65535) readers = 0;
     const bool two_launches = P.nsplit > 1 && !P.arrive;
-    if (dtype == MDX_F16) {
-        if (HPW == 2 && eight) paged_block_attn_kernel<_Float16, 2, 2, 8><<<grid, 512, 0, stream>>>(P);
-        else if (HPW == 2)     paged_block_attn_kernel<_Float16, 2, 2, 4><<<grid, 256, 0, stream>>>(P);
-        else                   paged_block_attn_kernel<_Float16, 1, 1, 4><<<grid, 256, 0, stream>>>(P);
-    } else {
-        if (readers > 0)       paged_block_attn_kernel<__bf16, 2, 2, 4, ReadAhead><<<dim3(grid.x, grid.y + readers), 256, 0, stream>>>(P, A);
-        else if (HPW == 2 && eight) paged_block_attn_kernel<__bf16, 2, 2, 8><<<grid, 512, 0, stream>>>(P);
-        else if (HPW == 2)     paged_block_attn_kernel<__bf16, 2, 2, 4><<<grid, 256, 0, stream>>>(P);
-        else                   paged_block_attn_kernel<__bf16, 1, 1, 4><<<grid, 256, 0, stream>>>(P);
-    }
+    auto attend = [&](auto element, auto merge) {
+        typedef decltype(element) E;
+        constexpr bool M = decltype(merge)::value;
+        if constexpr (std::is_same<E, __bf16>::value) {
+            if (readers > 0) { paged_block_attn_kernel<E, 2, 2, 4, M, ReadAhead><<<dim3(grid.x, grid.y + readers), 256, 0, stream>>>(P, A); return; }
+        }
+        if (HPW == 2 && eight) paged_block_attn_kernel<E, 2, 2, 8, M><<<grid, 512, 0, stream>>>(P);
+        else if (HPW == 2)     paged_block_attn_kernel<E, 2, 2, 4, M><<<grid, 256, 0, stream>>>(P);
+        else                   paged_block_attn_kernel<E, 1, 1, 4, M><<<grid, 256, 0, stream>>>(P);
+    };
+    if (dtype == MDX_F16) { if (P.arrive) attend(_Float16(), std::true_type()); else attend(_Float16(), std::false_type()); }
+    else                  { if (P.arrive) attend(__bf16(), std::true_type()); else attend(__bf16(), std::false_type()); }
     int rc = mdx::check_launch("paged_block_attn");
     if (rc != MDX_OK || !two_launches) return rc;
     // The slots asked for at once.  Many heads: four (sequences of so many have few pieces, and workgroups enough to wait beside each other;
@@ -882,6 +941,15 @@ extern "C" int64_t mdx_paged_block_attn_counter_bytes(int32_t bs, int32_t num_q_
     const int G = num_q_heads / num_kv_heads;
     // one counter per (sequence, head group, query tile), sized for the largest block (four tiles of 32 queries)
     return (int64_t)bs * (num_q_heads / ((G % 2 == 0) ? 2 : 1)) * (kMaxSq / kQTile) * (int64_t)sizeof(float);
+}
+
+extern "C" int32_t mdx_paged_block_attn_needs_counters(int32_t bs, int32_t sq, int32_t num_q_heads, int32_t num_kv_heads, int32_t max_pages, int32_t page_size)
+{
+    if (bs <= 0 || num_q_heads <= 0 || num_kv_heads <= 0 || max_pages <= 0 || page_size <= 0) return 0;
+    const int hpw = (num_q_heads / num_kv_heads) % 2 == 0 ? 2 : 1, nqt = sq <= kQTile ? 1 : (sq + kQTile - 1) / kQTile;
+    bool device_span;
+    pick_chunk(bs, num_q_heads / hpw * nqt, max_pages, page_size, &device_span);
+    return device_span;
 }
 
 extern "C" int mdx_paged_block_attn_single_launch(const void* q, void* o, const void* k_cache, const void* v_cache,

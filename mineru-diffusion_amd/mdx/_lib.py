@@ -33,6 +33,7 @@ SIGNATURES = {
     "mdx_paged_block_attn": (c_int32, [_P, _P, _P, _P] + [_I64] * 9 + [_P, _I64, _P] + [_I32] * 7 + [_I64, _F, _I32,
                                                                                                       _P, _I64, _P]),
     "mdx_paged_block_attn_counter_bytes": (c_int64, [_I32] * 3),
+    "mdx_paged_block_attn_needs_counters": (c_int32, [_I32] * 6),
     "mdx_paged_block_attn_read_ahead": (c_int32, [_P, _P, _P, _P] + [_I64] * 9 + [_P, _I64, _P] + [_I32] * 7 + [_I64, _F, _I32, _P, _I64, _P, _I64]
                                         + [_P, _I64] * 2 + [_P]),
     "mdx_paged_block_attn_single_launch": (c_int32, [_P, _P, _P, _P] + [_I64] * 9 + [_P, _I64, _P] + [_I32] * 7 + [_I64, _F, _I32,

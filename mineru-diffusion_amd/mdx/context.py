@@ -18,6 +18,7 @@ class Context:
     context_lens: torch.Tensor | None = None
     block_tables: torch.Tensor | None = None
     block_size: int = 32
+    counters: torch.Tensor | None = None    # decode: arrival counters of the caller's (ops.flash_attn_with_kvcache), not in the reference
 
 
 _CONTEXT = Context()

@@ -263,7 +263,7 @@ class DecoderLayer(nn.Module):
                                    staircase_size=ctx.block_size, max_seqlen=ctx.max_seqlen_k or None, softmax_scale=attn.scale)
             return o.flatten(1)
         o = flash_attn_with_kvcache_read_ahead(q, attn.k_cache, attn.v_cache, ctx.context_lens, ctx.block_tables, attn.scale,
-                                               self.o_proj, self.gate_up_proj)
+                                               self.o_proj, self.gate_up_proj, ctx.counters)
         return o.flatten(2)
 
 
@@ -591,6 +591,8 @@ class BlockDiffusionEngine:
         g["pos"] = torch.zeros(gbs, S, dtype=i64, device=dev)                  # written by mdx_block_prepare every pass
         g["slots"] = torch.full((gbs, S), -1, dtype=i32, device=dev)
         g["ctx"] = torch.zeros(gbs, dtype=i32, device=dev)
+        # the attention's arrival counters: the lanes' own, since their graphs may run beside other graphs captured on this stream
+        g["counters"] = torch.zeros(max(1, _lib.lib().mdx_paged_block_attn_counter_bytes(gbs, self.c.num_heads, self.c.num_kv_heads) // 4), device=dev)
         g["x0"] = torch.zeros(gbs * S, dtype=i64, device=dev)
         g["x0_p"] = torch.zeros(gbs * S, dtype=f32, device=dev)
         g["rows"] = torch.zeros(gbs * S, dtype=i64, device=dev)
@@ -627,6 +629,7 @@ class BlockDiffusionEngine:
                                                 g["width"], PAGE, S, g["pos"].data_ptr(), g["slots"].data_ptr(), g["ctx"].data_ptr(),
                                                 g["bs"], stream), "block_prepare")
         set_context(False, slot_mapping=g["slots"], context_lens=g["ctx"], block_tables=g["bt"], block_size=S)
+        get_context().counters = g["counters"]
         hidden = self.model(self.model.embed(g["ids"]), g["pos"])
         reset_context()
         return hidden

@@ -131,18 +131,19 @@ def flash_attn_with_kvcache(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
     q [bs, Sq, Hq, d], caches [pages, page, Hkv, d], block_table [bs, max_pages] int32,
     cache_seqlens [bs] int32, non-causal.  Returns o like q.
 
-    counters (keyword, not in the reference): None = single launch with this module's arrival
-    counters (one buffer per device and stream); a zeroed fp32 tensor of the caller's = single
-    launch with those; False = attention launch + combine launch."""
+    counters (keyword, not in the reference): None = single launch, where that pays, with this module's arrival
+    counters (one buffer per device and stream; while a graph is captured only for launches that need them); a zeroed fp32
+    tensor of the caller's = the same with those; False = attention launch + combine launch."""
     if causal:
         raise MdxError("flash_attn_with_kvcache: only causal=False (block-diffusion decode) is implemented")
     return _host().flash_attn_with_kvcache(q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale, counters)
 
 
-def flash_attn_with_kvcache_read_ahead(q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale, next_weight, then_weight) -> torch.Tensor:
+def flash_attn_with_kvcache_read_ahead(q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale, next_weight, then_weight,
+                                       counters: torch.Tensor | None | bool = None) -> torch.Tensor:
     """flash_attn_with_kvcache in a decode pass, whose launch also reads the weights of the two products behind it where it leaves the
     chip idle (up to 256 rows): the same result; the products find them in the device's cache."""
-    return _host().flash_attn_with_kvcache_read_ahead(q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale, next_weight, then_weight)
+    return _host().flash_attn_with_kvcache_read_ahead(q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale, next_weight, then_weight, counters)
 
 
 # --------------------------------------------------------------------------- unmask step

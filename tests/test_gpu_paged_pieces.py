@@ -78,3 +78,53 @@ def test_reading_ahead_in_wide_tables(dev, bs, pages):
     w = torch.zeros(24 << 20, dtype=torch.bfloat16, device=dev)
     want = mdx.flash_attn_with_kvcache(q, kc, vc, cache_seqlens=lens, block_table=bt, softmax_scale=128 ** -0.5)
     assert torch.equal(ops.flash_attn_with_kvcache_read_ahead(q, kc, vc, lens, bt, 128 ** -0.5, w[:4 << 20], w), want)
+
+
+def _spread(n, lo, hi):
+    return [lo + (hi - lo) * ((7 * b) % n) // max(1, n - 1) for b in range(n)]
+
+
+@pytest.mark.parametrize("ctxs,hq,hkv,dtype", [
+    (_spread(24, 90, 1500), 16, 8, torch.bfloat16),                        # a pair per CU: cut by shares
+    ([0, 0] + _spread(22, 1, 2100), 16, 8, torch.float16),                 # absent sequences among them
+    ([4000] + [60] * 23, 16, 8, torch.bfloat16),                           # one far above the rest: as many pieces as there is room for
+    ([640] * 24, 16, 8, torch.bfloat16),                                   # whole, all of one length
+    (_spread(64, 30, 1290), 10, 5, torch.bfloat16),                        # more pairs than CUs
+    (_spread(64, 30, 1290), 3, 1, torch.bfloat16),                         # one head per workgroup
+    (_spread(8, 700, 2560), 12, 6, torch.bfloat16),                        # few sequences, 10 pages: five and six pieces merged by the last
+    (_spread(8, 700, 2561), 12, 6, torch.bfloat16),                        # 11 pages: the combine launch
+    (_spread(8, 65, 129), 12, 6, torch.float16),
+])
+def test_pieces_merged_by_the_last_to_arrive(dev, ctxs, hq, hkv, dtype):
+    """One launch whose last split of a pair merges them: the oracle's result and the bits of attention + combine, whichever split is the last, on
+    counters that every launch leaves zero; from a graph too, replayed between eager calls on other counters."""
+    import mdx
+    g = torch.Generator().manual_seed(sum(ctxs) + hq)
+    d, page = 128, 256
+    counts = [-(-c // page) for c in ctxs]
+    pool = sum(counts) + 2
+    q = torch.randn(len(ctxs), 32, hq, d, generator=g).to(dtype)
+    kc, vc = (torch.randn(pool, page, hkv, d, generator=g).to(dtype) for _ in range(2))
+    bt = torch.full((len(ctxs), max(counts)), -1, dtype=torch.int32)
+    order, at = torch.randperm(pool, generator=g).int(), 0
+    for b, n in enumerate(counts):
+        bt[b, :n] = order[at:at + n]
+        at += n
+    lens = torch.tensor(ctxs, dtype=torch.int32)
+    args = (q.to(dev), kc.to(dev), vc.to(dev))
+    kw = dict(cache_seqlens=lens.to(dev), block_table=bt.to(dev), softmax_scale=1 / math.sqrt(d))
+    two = mdx.flash_attn_with_kvcache(*args, **kw, counters=False)
+    assert (two.float().cpu() - oracle.paged_block_attn(q, kc, vc, bt, lens, 1 / math.sqrt(d))).abs().max().item() < 2e-2
+    own, other = (torch.zeros(64 * 64, device=dev) for _ in range(2))
+    for _ in range(4):
+        assert torch.equal(mdx.flash_attn_with_kvcache(*args, **kw, counters=own), two)
+        assert own.abs().sum().item() == 0
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = mdx.flash_attn_with_kvcache(*args, **kw, counters=own)
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        assert torch.equal(mdx.flash_attn_with_kvcache(*args, **kw, counters=other), two)
+        torch.cuda.synchronize()
+        assert torch.equal(got, two) and own.abs().sum().item() == 0
