@@ -93,7 +93,7 @@ struct AdvanceParams {
 
 __global__ __launch_bounds__(64) void block_advance_kernel(const AdvanceParams P)
 {
-    const int b = blockIdx.x, lane = threadIdx.x;
+    const int b = (int)blockIdx.x + mdx::fetch_arguments<sizeof(AdvanceParams)>(), lane = threadIdx.x;
     const int ph = P.phase[b];
     const int S = P.block_len;
     if (ph == kIdle) {

@@ -50,7 +50,7 @@ __global__ __launch_bounds__(T::kThreads, T::kWaves / 4) void linear_kernel(cons
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     constexpr int TM = T::TM, TN = T::TN;
     const T tile;
-    const Place at = place_of(A.m_tiles, A.n_tiles);
+    const Place at = place_of((int)blockIdx.x + mdx::fetch_arguments<sizeof(LinearParams)>(gridDim.x), A.m_tiles, A.n_tiles);
     const int m0 = at.m * T::BM, n0 = at.n * T::kCols, k_split = A.K / A.splits;
     // heads: a column tile is one head row of every token, eight lanes of this thread's go to a token's; its place in the rotation
     // and the cache is asked for ahead of the product

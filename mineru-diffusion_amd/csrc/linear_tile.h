@@ -173,9 +173,9 @@ template <int BM_, int BN_, int WM_, int WN_, int WK_, int S_, int SX_, bool PAI
 // band of row tiles, column tile, row tile): what it has in flight together shares its rows of x and of W in its L2.
 constexpr int kBand = 8;                           // row tiles that share a column tile of W one after the other
 struct Place { int split, m, n; };
-__device__ __forceinline__ Place place_of(int m_tiles, int n_tiles) {
-    const int xcd = blockIdx.x & 7, per_xcd = gridDim.x >> 3, more = gridDim.x & 7;
-    int at = xcd * per_xcd + min(xcd, more) + (int)(blockIdx.x >> 3);
+__device__ __forceinline__ Place place_of(int block, int m_tiles, int n_tiles) {
+    const int xcd = block & 7, per_xcd = gridDim.x >> 3, more = gridDim.x & 7;
+    int at = xcd * per_xcd + min(xcd, more) + (block >> 3);
     const int per_split = m_tiles * n_tiles, split = at / per_split;
     at -= split * per_split;
     const int m_first = at / (kBand * n_tiles) * kBand, m_band = min(kBand, m_tiles - m_first);

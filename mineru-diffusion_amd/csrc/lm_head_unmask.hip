@@ -45,7 +45,7 @@ __global__ __launch_bounds__(T::kThreads, T::kWaves / 4) void lm_head_confidence
 {
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     const T tile;
-    const Place at = place_of(P.n_row_tiles, P.n_vocab_tiles);
+    const Place at = place_of((int)blockIdx.x, P.n_row_tiles, P.n_vocab_tiles);
     const int xr0 = at.m * T::BM, v0 = at.n * T::BN;
     const int row0 = tile.wm * (T::BM / T::WM) + tile.l16;        // this lane's first x row in the tile
     float c[T::TM];
@@ -171,7 +171,7 @@ __global__ __launch_bounds__(kThreads, 1) void lm_head_two_steps_kernel(const Lm
 // One wavefront per x row: folds the row's records (ascending vocabulary slices) into token and confidence.
 __global__ __launch_bounds__(kFoldThreads) void lm_head_finalize_kernel(const LmHeadParams P)
 {
-    const int row = blockIdx.x * (kFoldThreads / 64) + (threadIdx.x >> 6);
+    const int row = ((int)blockIdx.x + mdx::fetch_arguments<sizeof(LmHeadParams)>()) * (kFoldThreads / 64) + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (row >= P.rows) return;
     const float c = row_scale(P, row);

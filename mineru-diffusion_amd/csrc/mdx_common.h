@@ -56,5 +56,29 @@ inline int compute_units() {
 
 }  // namespace mdx
 
+namespace mdx {
+
+// A kernel's arguments come through the scalar cache, 64 bytes at a time, and the compiler asks for them where they are first used: a line that
+// is first used behind other loads puts one more trip to memory (0.1 to 0.2 us) into every workgroup's chain.  This asks for all lines of BYTES bytes of
+// arguments, and for the grid's size if it is given, at once.  Returns 0 in a way that the compiler doesn't see, to be added to something that is
+// used early.  (Not a volatile asm: behind one, the compiler no longer takes page tables and lengths for constant and reads them through vector loads.)
+// One sequence through attention and combine: 14.2 -> 13.8 us.
+template <int BYTES>
+__device__ __forceinline__ int fetch_arguments(int grid = 0)
+{
+    typedef __attribute__((address_space(4))) const int Word;
+    Word* const a = (Word*)__builtin_amdgcn_kernarg_segment_ptr();
+    constexpr int kLines = (BYTES + 63) / 64;
+    static_assert(kLines >= 1 && kLines <= 4, "lines of arguments");
+    int zero;
+    if constexpr (kLines == 1) asm("" : "=s"(zero) : "0"(0), "s"(grid), "s"(a[0]));
+    if constexpr (kLines == 2) asm("" : "=s"(zero) : "0"(0), "s"(grid), "s"(a[0]), "s"(a[16]));
+    if constexpr (kLines == 3) asm("" : "=s"(zero) : "0"(0), "s"(grid), "s"(a[0]), "s"(a[16]), "s"(a[32]));
+    if constexpr (kLines == 4) asm("" : "=s"(zero) : "0"(0), "s"(grid), "s"(a[0]), "s"(a[16]), "s"(a[32]), "s"(a[48]));
+    return zero;
+}
+
+}  // namespace mdx
+
 #define MDX_REQUIRE(cond, code, ...) \
     do { if (!(cond)) return ::mdx::fail(code, __VA_ARGS__); } while (0)

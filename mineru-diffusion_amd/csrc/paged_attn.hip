@@ -143,7 +143,7 @@ struct ReadAhead {
     const u32x4* p[2]; int n[2];                    // 16-byte elements
     int first_y;                                    // blockIdx.y from which workgroups read
 };
-__device__ __forceinline__ bool is_reader(const ReadAhead& A) { return (int)blockIdx.y >= A.first_y; }
+__device__ __forceinline__ bool is_reader(int block_y, const ReadAhead& A) { return block_y >= A.first_y; }
 template <int THREADS> __device__ __forceinline__ void read_ahead(const ReadAhead& A) {
     constexpr int kTogether = 8;
     const int step = ((int)gridDim.y - A.first_y) * (int)gridDim.x * THREADS;
@@ -203,8 +203,10 @@ template <int COLS> struct Fold {
 template <typename E, int HPW, int DEPTH, int WAVES, bool MERGE, typename... AHEAD>
 __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_block_attn_kernel(const PagedParams P, const AHEAD... ahead)
 {
+    const int zero = mdx::fetch_arguments<sizeof(PagedParams)>(gridDim.x);
+    const unsigned block_x = blockIdx.x + zero;
     if constexpr (sizeof...(AHEAD) > 0) {
-        if (is_reader(ahead...)) { read_ahead<64 * WAVES>(ahead...); return; }
+        if (is_reader((int)blockIdx.y + zero, ahead...)) { read_ahead<64 * WAVES>(ahead...); return; }
     }
     constexpr int kThreads = 64 * WAVES;
     constexpr int kRowsPerPass = kThreads / 16;     // LDS rows one pass of the workgroup stages
@@ -221,8 +223,8 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
     // launch order: head group fastest, then the query tiles of a (sequence, split), then the pairs -- the tiles of a
     // block longer than 32 queries stream the same keys, so they start next to each other and on the same XCD
     const int n_groups = P.num_q_heads / HPW;
-    const int hg = blockIdx.x % n_groups;
-    const int qt = blockIdx.x / n_groups;           // this workgroup's tile of 32 queries
+    const int hg = block_x % n_groups;
+    const int qt = block_x / n_groups;           // this workgroup's tile of 32 queries
     const int kw = wave % KW;                       // this wavefront's key slice
     const int head = hg * HPW + wave / KW;          // and query head
 
@@ -341,7 +343,7 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
     // (with the readers' loads in the kernel the compiler no longer takes the table for constant by itself)
     typedef __attribute__((address_space(4))) const int32_t ConstantEntry;
     auto table_row = [&] {
-        const int32_t* row = P.block_table + (int64_t)b * P.bt_stride;
+        const int32_t* row = P.block_table + (int64_t)__builtin_amdgcn_readfirstlane(b) * P.bt_stride;
         if constexpr (sizeof...(AHEAD) > 0) return (ConstantEntry*)(uintptr_t)row; else return row;
     };
     const auto bt = table_row();
@@ -606,7 +608,8 @@ template <typename E, int AHEAD, int ROWS>
 __global__ __launch_bounds__(32 * ROWS) void paged_combine_kernel(const PagedParams P)
 {
     constexpr int kParts = kQTile / ROWS;
-    const int part = blockIdx.x % kParts, rest = blockIdx.x / kParts;
+    const unsigned block = blockIdx.x + mdx::fetch_arguments<sizeof(PagedParams)>();
+    const int part = block % kParts, rest = block / kParts;
     const int qt = rest % P.nqt, hq = (rest / P.nqt) % P.num_q_heads, b = rest / P.nqt / P.num_q_heads;
     const int c = (threadIdx.x & 31) * 4, s = part * ROWS + (threadIdx.x >> 5);
     if (c >= P.head_dim || qt * kQTile + s >= P.sq) return;

@@ -27,7 +27,7 @@ template <int SLICES, int THREADS>
 __global__ __launch_bounds__(THREADS) void qk_norm_rope_store_kernel(const FusedParams P)
 {
     constexpr int kRows = THREADS / kLanesPerRow;
-    const int64_t tok = blockIdx.x;
+    const int64_t tok = (int)blockIdx.x + mdx::fetch_arguments<sizeof(FusedParams)>(gridDim.y);
     const int n_rows = P.rows.hq + 2 * P.rows.hkv;             // head rows of this token: q | k | v
     const int j = threadIdx.x % kLanesPerRow;
     const int64_t width = (int64_t)n_rows * kHeadDim;

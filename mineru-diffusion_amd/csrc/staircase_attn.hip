@@ -304,12 +304,13 @@ __global__ __launch_bounds__(kThreads, 2) void staircase_attn_kernel(const Stair
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, kw = wave % KW;
     const int H = lane >> 5, r = lane & 31;
 
-    if ((int)blockIdx.x >= P.store.first_wg) { store_rows(P.store, (int)blockIdx.x - P.store.first_wg, tid); return; }
+    const int block = (int)blockIdx.x + mdx::fetch_arguments<sizeof(StaircaseParams)>();
+    if (block >= P.store.first_wg) { store_rows(P.store, block - P.store.first_wg, tid); return; }
 
     // ---- workgroup -> (head slot, sequence b, row group rg) ------------------------------------
-    const int hslot = blockIdx.x % P.num_q_heads;
+    const int hslot = (unsigned)block % P.num_q_heads;
     int b, rg, seq0, L;
-    if (!locate_row_group<kRows>(P, blockIdx.x / P.num_q_heads, lane, lds_hist[wave], b, rg, seq0, L)) return;
+    if (!locate_row_group<kRows>(P, (unsigned)block / P.num_q_heads, lane, lds_hist[wave], b, rg, seq0, L)) return;
     if (L <= 0) return;
     const int S = 1 << P.log2_s;
     const int Lp = ((L + S - 1) >> P.log2_s) << P.log2_s;     // padded length
@@ -524,8 +525,9 @@ __global__ __launch_bounds__(kThreads, 1) void staircase_pair_kernel(const Stair
     const int H = lane >> 5, r = lane & 31;
     const int n_hslots = P.num_q_heads / 2;
 
-    if ((int)blockIdx.x >= P.store.first_wg) {
-        const int wg = (int)blockIdx.x - P.store.first_wg;
+    const int item = (int)blockIdx.x + mdx::fetch_arguments<sizeof(StaircaseParams)>();
+    if (item >= P.store.first_wg) {
+        const int wg = item - P.store.first_wg;
         if (P.store.own_rows) store_unowned_rows(P, wg, tid);
         else store_rows(P.store, wg, tid);
         return;
@@ -534,7 +536,6 @@ __global__ __launch_bounds__(kThreads, 1) void staircase_pair_kernel(const Stair
     // One work item per workgroup: the dispatcher hands the next item to whichever CU frees up
     // first, which balances the ragged item lengths (a fixed item -> CU assignment measured 10%
     // slower although it saves the launch gap between two workgroups of a CU).
-    const int item = blockIdx.x;
     const int hslot = item % n_hslots;
     int b, rg, seq0, L;
     // (scratch for the numbering: in slot 4, which no K/V load targets before every wavefront has passed the core's first barrier)

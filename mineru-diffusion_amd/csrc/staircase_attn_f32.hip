@@ -41,7 +41,7 @@ __global__ __launch_bounds__(kThreads, D <= 128 && KW <= 2 ? 2 : 1) void stairca
     const int H = lane >> 5, r = lane & 31;
     const int head = blockIdx.x;
     const int rg = P.n_row_groups - 1 - (int)blockIdx.y;       // the heaviest row groups start first
-    const int b = blockIdx.z;
+    const int b = (int)blockIdx.z + mdx::fetch_arguments<sizeof(WideParams)>();
 
     // bounds that do not describe a range inside the packed tensors (decreasing, negative, past total_tokens) are clipped
     // to one, so that no row outside q/k/v/o is ever touched
