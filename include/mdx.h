@@ -349,6 +349,19 @@ int mdx_unmask_step_gumbel(const void* logits, int64_t row_stride, int32_t dtype
                            int64_t* x0, float* x0_p, uint8_t* transfer, int32_t* count,
                            int32_t bs, int32_t block_len, int64_t vocab,
                            void* workspace, int64_t workspace_bytes, mdx_stream_t stream);
+
+/*
+ * mdx_unmask_step (or, seeded, mdx_unmask_step_gumbel) on blocks in host memory that the GPU reaches (pinned), for a caller that wants the blocks, the flags and the
+ * counts: which positions are masked is read here, and only their rows are computed.  tokens must hold its values when the call is made and may be written by the
+ * GPU until the stream is done.  The workspace (16-byte aligned) holds the confidences as well.
+ */
+int64_t mdx_unmask_step_host_blocks_workspace_bytes(int64_t rows, int64_t vocab);
+int mdx_unmask_step_host_blocks(const void* logits, int64_t row_stride, int32_t dtype,
+                                const float* temperatures, const float* noise, int64_t noise_row_stride,
+                                int32_t seeded, uint64_t seed, uint64_t offset, const int64_t* offset_dev,
+                                int64_t* tokens, int64_t mask_token_id, float threshold, int32_t k,
+                                uint8_t* transfer, int32_t* count, int32_t bs, int32_t block_len, int64_t vocab,
+                                void* workspace, int64_t workspace_bytes, mdx_stream_t stream);
 int mdx_gumbel_noise(float* noise, int64_t noise_row_stride, int64_t rows, int64_t vocab,
                      uint64_t seed, uint64_t offset, const int64_t* offset_dev, const int64_t* row_ids,
                      mdx_stream_t stream);

@@ -919,10 +919,17 @@ PyObject* sampler_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
             std::memcpy(host + i * S * 8, ptr(block), S * 8);
         }
         const Noise z = noise_of(a + 8, bs * S, vocab);
-        Tensor x0 = make(logits, at::kLong, bs, S), x0_p = make(logits, at::kFloat, bs, S);
-        step(logits, bs, S, reinterpret_cast<int64_t*>(host), to_int(a[5]), (float)real(a[6]), (int32_t)to_int(a[7]), temps, Filter{0, 1.0}, z,
-             static_cast<int64_t*>(ptr(x0)), static_cast<float*>(ptr(x0_p)), reinterpret_cast<uint8_t*>(host + flags_at),
-             reinterpret_cast<int32_t*>(host + counts_at));
+        const Logits l = logits_of(logits);
+        NEED(l.rows == bs * S);
+        const Tensor t = temperatures_of(temps);
+        if (t.defined()) NEED(t.numel() == bs);
+        const int64_t ws_bytes = mdx_unmask_step_host_blocks_workspace_bytes(l.rows, l.vocab);
+        const Tensor ws = make(logits, at::kByte, ws_bytes);
+        check(mdx_unmask_step_host_blocks(ptr(l.t), l.stride, dtype_of(logits), static_cast<const float*>(ptr_or_null(t)), z.data(), z.data() ? l.vocab : 0,
+                                          z.seeded ? 1 : 0, z.seed, z.offset, static_cast<const int64_t*>(ptr_or_null(z.offset_dev)),
+                                          reinterpret_cast<int64_t*>(host), to_int(a[5]), (float)real(a[6]), (int32_t)to_int(a[7]),
+                                          reinterpret_cast<uint8_t*>(host + flags_at), reinterpret_cast<int32_t*>(host + counts_at), (int32_t)bs, (int32_t)S, l.vocab,
+                                          ptr(ws), ws_bytes, stream_of(logits)), "unmask_step");
         hipError_t rc;
         Py_BEGIN_ALLOW_THREADS
         rc = hipStreamSynchronize(static_cast<hipStream_t>(stream_of(logits)));

@@ -136,6 +136,28 @@ def test_sampler_with_a_seed_samples_like_the_reference_prepare(dev):
     assert not torch.equal(x0_plain, x0_noisy)
 
 
+@pytest.mark.parametrize("mode", ["plain", "seed", "tensor"])
+@pytest.mark.parametrize("bs,vocab,masked", [(1, 40000, 0), (1, 40000, 1), (3, 40000, 50), (5, 1001, 159), (32, 3000, 700), (32, 3000, 1024), (33, 3000, 5)])
+def test_sampler_computes_masked_rows_only(dev, mode, bs, vocab, masked):
+    """None, one, some and all positions masked, up to the most rows that are picked out and beyond: the committed tokens are those of unmask_step, which computes
+    every row (the same picks bit for bit; confidences are sums in another order, and the ranking of random ones is not that close)."""
+    import mdx
+    g = torch.Generator().manual_seed(bs * vocab + masked)
+    logits = (torch.randn(bs, S, vocab, generator=g) * 3).bfloat16().to(dev)
+    tokens = torch.randint(0, 900, (bs, S), generator=g)
+    tokens.view(-1)[torch.randperm(bs * S, generator=g)[:masked]] = MASK_ID
+    temps = (0.7 + torch.rand(bs, 1, generator=g)).to(dev)
+    noise = torch.rand(bs, S, vocab, generator=g).to(dev) if mode == "tensor" else None
+    want = tokens.clone().to(dev)
+    _, _, transfer, count = mdx.unmask_step(logits, want, MASK_ID, 0.9, 3, temperatures=temps, seed=77 if mode == "seed" else None, offset=0, noise=noise)
+    seqs = _fake_seqs(tokens.clone(), 0.9, [2] * bs)
+    n = mdx.Sampler(k=3, seed=77 if mode == "seed" else None, noise_fn=(lambda _: noise) if mode == "tensor" else None)(logits, temps, seqs)
+    assert n == int(count.sum())
+    for b, s in enumerate(seqs):
+        assert torch.equal(s.current_denoising_block, want[b].cpu())
+        assert torch.equal(s.current_step_map, transfer[b].cpu().int() * 2)
+
+
 def test_sampler_prepare_is_the_confidence_pass(dev):
     import mdx
     logits, _, temps = _sampler_case(seed=8, bs=3)
