@@ -94,10 +94,11 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 __device__ __forceinline__ void store_agent(float* p, f32x4 v) {
     asm volatile("global_store_dwordx4 %0, %1, off sc1" :: "v"(p), "v"(v) : "memory");
 }
-__device__ __forceinline__ f32x4 load_agent(const float* p) {
-    f32x4 v;
-    asm volatile("global_load_dwordx4 %0, %1, off sc1" : "=v"(v) : "v"(p) : "memory");
-    return v;
+// (Not inline asm: the compiler takes such a load's registers for written while it is still on its way, and what it moved or spilled before the wait would be
+// the old contents.  Two atomic loads of eight bytes: 16 sequences of 375-1500 keys 24.9 -> 25.5 us.)
+constexpr int kAgentScope = 16;                      // sc1
+__device__ __forceinline__ f32x4 load_agent(__amdgpu_buffer_rsrc_t from, int offset) {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from, offset, 0, kAgentScope));
 }
 __device__ __forceinline__ void wait_vector_memory() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
@@ -537,6 +538,9 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
         __syncthreads();
         if (!i_am_last) return;
     }
+    const int64_t sequence_floats = (int64_t)P.num_q_heads * P.nqt * P.nsplit * kQTile * kHeadDim;       // (below 2^31 bytes: the launch)
+    const __amdgpu_buffer_rsrc_t of_sequence =
+        __builtin_amdgcn_make_buffer_rsrc(P.part_o + __builtin_amdgcn_readfirstlane(b) * sequence_floats, 0, (int)(sequence_floats * 4), 0x27000);
     // the arithmetic of Fold::take4, split by split in groups of four, whoever is last: the bits of the combine kernel
     float M = kMinusBig, L = 0.f;
     f32x4 acc[kMine][4];
@@ -557,17 +561,9 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
 #pragma unroll
                 for (int t = 0; t < kMine; ++t)
 #pragma unroll
-                    for (int g = 0; g < 4; ++g) po[i][t][g] = load_agent(part(sp, t, g));
+                    for (int g = 0; g < 4; ++g) po[i][t][g] = load_agent(of_sequence, ((((head * P.nqt + qt) * P.nsplit + sp) * 16 + (kw + KW * t) * 4 + g) * 64 + lane) * 16);
             }
         }
-        // the asm loads are invisible to the compiler's own counting: wait here, and tie every loaded
-        // value to the wait so that no use of it can be scheduled above it
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int t = 0; t < kMine; ++t)
-#pragma unroll
-                for (int g = 0; g < 4; ++g) asm volatile("s_waitcnt vmcnt(0)" : "+v"(po[i][t][g]) :: "memory");
         float Mn = M;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -826,12 +822,14 @@ int launch_paged_ahead(const void* q, void* o, const void* k_cache, const void* 
         // whose sequences come to few pieces (kMergeKeys).  Those launches take two where there are no counters to use.
         const int64_t pairs = (int64_t)bs * wg_per_pair, need_c = pairs * (int64_t)sizeof(float);
         const bool have_counters = counters && counter_bytes >= need_c && ((uintptr_t)counters & 3) == 0;
+        // (a sequence's partials: 31 bits of bytes, or two launches)
+        const bool addressable = (int64_t)num_q_heads * P.nqt * P.nsplit * kQTile * kHeadDim * 4 < ((int64_t)1 << 31);
         if (single_launch && device_span) {
             MDX_REQUIRE(counters && counter_bytes >= need_c, MDX_EWORKSPACE,
                         "paged_block_attn: %lld bytes of arrival counters needed, %lld given", (long long)need_c, (long long)counter_bytes);
             MDX_REQUIRE(((uintptr_t)counters & 3) == 0, MDX_EWORKSPACE, "paged_block_attn: counters not 4-byte aligned");
-            P.arrive = static_cast<float*>(counters);
-        } else if (single_launch && P.fit_slots > 0 && have_counters && merges_itself(pairs, (int64_t)max_pages * page_size, cus)) {
+            if (addressable) P.arrive = static_cast<float*>(counters);
+        } else if (single_launch && P.fit_slots > 0 && have_counters && addressable && merges_itself(pairs, (int64_t)max_pages * page_size, cus)) {
             P.arrive = static_cast<float*>(counters);
         }
     }
