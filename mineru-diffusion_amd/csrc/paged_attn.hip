@@ -656,7 +656,7 @@ constexpr int64_t kReadAheadFewBytes = (int64_t)32 << 20, kReadAheadBytes = (int
 // page-table width, not the lengths: tables are taken to be about 65 % full, and the last split of
 // a sequence to be half a split (the attention kernel, which sees the lengths, corrects the split
 // both ways: PagedParams::fit_slots).  In the pair-per-CU case up to four splits per sequence are allowed
-// and the kernel itself, which sees the lengths, cuts only sequences well above the mean
+// and the kernel itself, which sees the lengths, cuts by even shares where the longest is well above one: kWholeFactor
 // (*device_span; the dense workgroup numbering that this needs exists for up to 64 sequences).
 //
 // The counts behind those rules (1.95 workgroups per CU, pairs per CU) are taken from the current device's
@@ -818,8 +818,8 @@ int launch_paged_ahead(const void* q, void* o, const void* k_cache, const void* 
         // Single launch: the partials are written through with agent-scope stores and read back with
         // agent-scope loads, so counting in costs a workgroup the wait for its own stores and one atomic,
         // not a device-wide release (a write-back walk of its XCD's L2).  With about a pair per CU that always beats the combine launch (24 sequences of
-        // 1250-5000 keys 75 / 72 us, 48 of 550-2200 74 / 68, and sequences that stay whole pay nothing); with fewer it does for kMergePairs and more pairs
-        // whose sequences come to few pieces (kMergeKeys).  Those launches take two where there are no counters to use.
+        // 1250-5000 keys 75 / 72 us, 48 of 550-2200 74 / 68, and sequences that stay whole pay nothing); with fewer it does for enough pairs
+        // whose sequences come to few pieces (merges_itself).  Those launches take two where there are no counters to use.
         const int64_t pairs = (int64_t)bs * wg_per_pair, need_c = pairs * (int64_t)sizeof(float);
         const bool have_counters = counters && counter_bytes >= need_c && ((uintptr_t)counters & 3) == 0;
         // (a sequence's partials: 31 bits of bytes, or two launches)
