@@ -247,7 +247,7 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
             // workgroups per head group - a remainder of half a piece per sequence), and no more pieces of a sequence than
             // the launch has room for (the "+ 1" keeps the longest within nsplit pieces whatever the rounding of the
             // reciprocals; every workgroup makes the same estimate).
-            const int total = wave_sum(ctx_l), longest = wave_max(ctx_l), live = wave_sum(ctx_l > 0 ? 1 : 0);
+            const int total = wave_sum(ctx_l), longest = wave_max(ctx_l), live = __popcll(__ballot(ctx_l > 0));
             const float per_group = (float)P.fit_slots * __builtin_amdgcn_rcpf((float)gridDim.x);      // resident workgroups per head group and query tile
             const float room = fmaxf(1.f, per_group - 0.5f * (float)live);
             const int best = min(512, ((int)(kPieceRoot * __builtin_amdgcn_sqrtf((float)total)) + 32) & ~63);
@@ -265,7 +265,7 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
         } else {
             if (P.fit_slots < 0) {
                 // (kWholeFactor above says why; the host's split is what keeps the longest within nsplit pieces)
-                const int total = wave_sum(ctx_l), longest = wave_max(ctx_l), live = wave_sum(ctx_l > 0 ? 1 : 0);
+                const int total = wave_sum(ctx_l), longest = wave_max(ctx_l), live = __popcll(__ballot(ctx_l > 0));
                 const float share = (float)total * (float)gridDim.x * __builtin_amdgcn_rcpf((float)-P.fit_slots);
                 const float mean = (float)total * __builtin_amdgcn_rcpf((float)max(live, 1));
                 span = max(span, ((int)(kShareFactor * share) + kShareKeys + 63) & ~63);
@@ -289,7 +289,13 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
             j -= c;
             return false;
         };
-        if constexpr (MERGE) {
+        if (MERGE && !cut && P.bs * (int)gridDim.x <= -P.fit_slots) {
+            // Whole sequences that are all resident at once: any order will do, and the search for a pair is part of every workgroup's start.  (32 equal
+            // sequences of 1088-3136 keys, average under the profiler: 52.6 us with the search below, 51.6 without; a decode pass of them is 0.9 % shorter.)
+            if (j >= P.bs) return;
+            b = j;
+            level = 0;
+        } else if constexpr (MERGE) {
             // Heaviest first: all whole pieces, then the remainders (and sequences shorter than a piece) by eighths of a piece, so that
             // those which start late, when there are more workgroups than the chip holds at once, are the short ones of all.  (16 sequences of
             // 375-1500 keys 30.3 us in the order below, 26.2 in this one.)

@@ -89,6 +89,9 @@ def _spread(n, lo, hi):
     ([0, 0] + _spread(22, 1, 2100), 16, 8, torch.float16),                 # absent sequences among them
     ([4000] + [60] * 23, 16, 8, torch.bfloat16),                           # one far above the rest: as many pieces as there is room for
     ([640] * 24, 16, 8, torch.bfloat16),                                   # whole, all of one length
+    ([0, 1100, 0] + [1030 + 3 * b for b in range(29)], 16, 8, torch.bfloat16),   # whole, a pair per CU: sequences taken as they come, absent ones too
+    ([1030 + 3 * b for b in range(63)] + [0], 16, 8, torch.float16),       # the most pairs that are resident at once
+    ([1030 + 3 * b for b in range(63)] + [0], 18, 9, torch.bfloat16),      # more than that: whole, the longest first
     (_spread(64, 30, 1290), 10, 5, torch.bfloat16),                        # more pairs than CUs
     (_spread(64, 30, 1290), 3, 1, torch.bfloat16),                         # one head per workgroup
     (_spread(8, 700, 2560), 12, 6, torch.bfloat16),                        # few sequences, 10 pages: five and six pieces merged by the last
