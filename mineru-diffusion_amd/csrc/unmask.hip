@@ -169,7 +169,10 @@ __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
     int64_t* __restrict__ x0, float* __restrict__ x0_p)
 {
     constexpr int EPC = Elem<T>::EPC;
-    const int64_t row = sizeof...(LIVE) > 0 ? live_row(blockIdx.x) : (int)blockIdx.x;
+    // (without LIVE from an unsigned number: from a signed one the compiler forms other code, and the step of 8 sequences takes 19.8 instead of 19.3 us, the
+    // sampled one 42.6 instead of 42.1)
+    const uint32_t row32 = sizeof...(LIVE) > 0 ? (uint32_t)live_row(blockIdx.x) : blockIdx.x;
+    const int64_t row = row32;
     const int split = blockIdx.y;
     const int tid = threadIdx.x;
     const T* rp = logits + row * row_stride;
