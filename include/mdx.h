@@ -474,10 +474,6 @@ int mdx_silu_and_mul(const void* x, int64_t x_row_stride, void* out, int64_t out
  * mdx_decode_linear_partials and mdx_decode_linear_silu: the same for the few rows of a decode pass, always as partial sums
  * (rows up to 128, n a multiple of 64, k of 256; splits = mdx_decode_linear_splits, 0 where not covered) and with the SiLU
  * (rows up to 64, n a multiple of 24, k of 512: mdx_decode_linear_silu_supported).
- * mdx_linear_residual: s = residual_in + round(x . w^T) for up to 64 rows (n and k multiples of 512 up to 4096: mdx_linear_residual_supported), with the norm
- * that follows as far as it goes before a row's sum of squares is known: residual_out = round(s), z = round(s * norm_weight), sums [rows, n / 16]
- * (dense fp32) = the sums of s^2 over 16 columns each; residual_out and z must not overlap what is read.  mdx_linear_scaled_silu: mdx_linear_silu of the rows
- * z / sqrt(sum of the row's sums / k + eps), up to 64 of them, k a multiple of 512 up to 4096 (mdx_linear_scaled_silu_supported).
  * mdx_add_rms_norm_partials and mdx_qk_norm_rope_store_partials are mdx_add_rms_norm and mdx_qk_norm_rope_store with
  * x / qkv given as such partial sums ([splits, rows, hidden], [splits, n_tokens, (Hq + 2 Hkv) * d]).
  */
@@ -502,14 +498,6 @@ int mdx_decode_linear_partials(const void* x, int64_t x_row_stride, const void* 
                                float* partials, int64_t rows, int64_t n, int64_t k, mdx_stream_t stream);
 int32_t mdx_decode_linear_silu_supported(int64_t rows, int64_t n, int64_t k);
 int mdx_decode_linear_silu(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride,
-                           void* y, int64_t y_row_stride, int64_t rows, int64_t n, int64_t k, mdx_stream_t stream);
-int32_t mdx_linear_residual_supported(int64_t rows, int64_t n, int64_t k);
-int mdx_linear_residual(const void* x, int64_t x_row_stride, const void* w, int64_t w_row_stride,
-                        const void* residual_in, int64_t residual_in_row_stride, void* residual_out, int64_t residual_out_row_stride,
-                        const void* norm_weight, void* z, int64_t z_row_stride, float* sums,
-                        int64_t rows, int64_t n, int64_t k, mdx_stream_t stream);
-int32_t mdx_linear_scaled_silu_supported(int64_t rows, int64_t n, int64_t k);
-int mdx_linear_scaled_silu(const void* z, int64_t z_row_stride, const float* sums, float eps, const void* w, int64_t w_row_stride,
                            void* y, int64_t y_row_stride, int64_t rows, int64_t n, int64_t k, mdx_stream_t stream);
 int mdx_add_rms_norm_partials(const float* partials, int32_t splits,
                               const void* residual_in, int64_t residual_in_row_stride,

@@ -390,35 +390,6 @@ PyObject* linear_gated(PyObject*, PyObject* const* a, Py_ssize_t n) {
     });
 }
 
-// x [.., k], w [n, k], residual [.., n], a norm's weight [n], eps, the gate/up weight [2 i, n] -> (silu_and_mul(norm(residual + x . w^T) . gate_up^T)
-// [.., i], the new residual), or None where the shapes are not covered
-PyObject* linear_residual_gated(PyObject*, PyObject* const* a, Py_ssize_t n) {
-    ARGS(6);
-    return guarded([&]() -> PyObject* {
-        const Tensor &x = tensor(a[0]), &w = tensor(a[1]), &residual = tensor(a[2]), &norm = tensor(a[3]), &gate_up = tensor(a[5]);
-        need_gpu({&x, &w, &residual, &norm, &gate_up});
-        NEED(x.dim() >= 2 && w.dim() == 2 && x.size(-1) == w.size(1) && gate_up.dim() == 2 && gate_up.size(1) == w.size(0) && gate_up.size(0) % 2 == 0);
-        const int64_t k = w.size(1), cols = w.size(0), rows = k ? x.numel() / k : 0, inter = gate_up.size(0) / 2;
-        NEED(residual.dim() >= 1 && residual.size(-1) == cols && residual.numel() == rows * cols && norm.dim() == 1 && norm.size(0) == cols && norm.is_contiguous());
-        if (!mdx_linear_residual_supported(rows, cols, k) || !mdx_linear_scaled_silu_supported(rows, inter, cols)) Py_RETURN_NONE;
-        const Rows r = rows_of(x, k), in = rows_of(residual, cols);
-        if (!operands_covered(r, rows_of(w, k), k) || !operands_covered(in, rows_of(gate_up, cols), cols) || norm.scalar_type() != at::kBFloat16 ||
-            reinterpret_cast<uintptr_t>(ptr(norm)) % 16 != 0) Py_RETURN_NONE;
-        const auto options = at::TensorOptions().dtype(at::kBFloat16).device(x.device());
-        std::vector<int64_t> shape(residual.sizes().begin(), residual.sizes().end());
-        Tensor z = make(x, at::kBFloat16, rows, cols), sums = make(x, at::kFloat, rows, cols / 16), out = at::empty(shape, options);
-        check(mdx_linear_residual(ptr(r.t), r.stride, ptr(w), w.stride(0), ptr(in.t), in.stride, ptr(out), cols, ptr(norm), ptr(z), cols, static_cast<float*>(ptr(sums)),
-                                  rows, cols, k, stream_of(x)),
-              "linear_residual");
-        shape.back() = inter;
-        Tensor y = at::empty(shape, options);
-        check(mdx_linear_scaled_silu(ptr(z), cols, static_cast<const float*>(ptr(sums)), (float)real(a[4]), ptr(gate_up), gate_up.stride(0), ptr(y), inter, rows, inter, cols,
-                                     stream_of(x)),
-              "linear_scaled_silu");
-        return wrap_tuple(std::move(y), std::move(out));
-    });
-}
-
 // x [.., k], w [(hq + 2 hkv) d, k], q/k weights, eps, cos, sin, positions, hq, hkv, d, caches and slots (or None), want_kv
 // -> (q [.., hq, d], k, v [.., hkv, d] or None), or None where the shape is not covered
 PyObject* linear_qk_norm_rope_store(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -964,7 +935,7 @@ PyObject* sampler_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 #define ENTRY(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
-    ENTRY(store_kvcache), ENTRY(store_kvcache_maybe4d), ENTRY(qk_norm_rope_store), ENTRY(rms_norm), ENTRY(silu_and_mul), ENTRY(linear), ENTRY(linear_gated), ENTRY(linear_residual_gated), ENTRY(linear_qk_norm_rope_store), ENTRY(linear_partials), ENTRY(linear_silu),
+    ENTRY(store_kvcache), ENTRY(store_kvcache_maybe4d), ENTRY(qk_norm_rope_store), ENTRY(rms_norm), ENTRY(silu_and_mul), ENTRY(linear), ENTRY(linear_gated), ENTRY(linear_qk_norm_rope_store), ENTRY(linear_partials), ENTRY(linear_silu),
     ENTRY(rms_norm_partials), ENTRY(qk_norm_rope_store_partials), ENTRY(sparse_attn_varlen),
     ENTRY(flash_attn_with_kvcache), ENTRY(flash_attn_with_kvcache_read_ahead), ENTRY(attention_prefill), ENTRY(attention_decode), ENTRY(confidence_argmax), ENTRY(lm_head_confidence),
     ENTRY(filter_logits), ENTRY(select_transfer), ENTRY(unmask_step), ENTRY(sampler_step),

@@ -37,7 +37,6 @@ struct LinearParams {
     int64_t y_stride;                              // elements between rows
     int K, m_tiles, n_tiles, splits;
     RowParams rows;                                // heads
-    const float* sums; int n_sums; float eps;      // scaled: sums of squares of the rows [M, n_sums]
 };
 
 enum Form { kRounded = 0, kPartials = 1, kSilu = 2, kHeads = 3 };
@@ -45,10 +44,7 @@ enum Form { kRounded = 0, kPartials = 1, kSilu = 2, kHeads = 3 };
 template <typename T> constexpr int kSumsBytes = T::WK == 2 ? T::BM * T::BN * 4 : 0;      // where two wavefronts' sums meet
 constexpr int kHeadPitch = mdx_qk::kHeadDim + 8;
 
-// SCALED: x as linear_residual.hip leaves it, a row before its norm times the norm's weight; the row's sums of squares are on their way during the
-// product, and the result is divided by their root.
-constexpr int kSumLoads = 8;                                 // of 32 sums: eight lanes of a row, four each
-template <typename T, int FORM, bool SCALED>
+template <typename T, int FORM>
 __global__ __launch_bounds__(T::kThreads, T::kWaves / 4) void linear_kernel(const LinearParams A)
 {
     extern __shared__ __attribute__((aligned(1024))) char lds[];
@@ -67,29 +63,8 @@ __global__ __launch_bounds__(T::kThreads, T::kWaves / 4) void linear_kernel(cons
         for (int p = 0; p < kPasses; ++p) places[p] = mdx_qk::place_of_token(A.rows, min(tok0 + p * kTokens, A.in.M - 1), j8);
         weight = mdx_qk::weight_of_row(A.rows, at.n, j8);
     }
-    f32x4 squares[SCALED ? kSumLoads : 1];
-    if constexpr (SCALED) {
-        static_assert(T::kThreads == 8 * T::BM, "eight lanes per row");
-        const float* of_row = A.sums + (int64_t)min(m0 + (int)threadIdx.x / 8, A.in.M - 1) * A.n_sums + threadIdx.x % 8 * 4;
-#pragma unroll
-        for (int i = 0; i < kSumLoads; ++i) squares[i] = 32 * i < A.n_sums ? *reinterpret_cast<const f32x4*>(of_row + 32 * i) : f32x4{0.f, 0.f, 0.f, 0.f};
-    }
     typename T::Sums acc;
     tile.product(A.in, m0, n0, (int64_t)at.split * k_split, k_split / kStepK, lds, acc);
-    __shared__ float scale[SCALED ? T::BM : 1];
-    if constexpr (SCALED) {
-        // (not before here: the compiler would add them up, and wait for them, ahead of the product)
-#pragma unroll
-        for (int i = 0; i < kSumLoads; ++i) asm volatile("" : "+v"(squares[i]));
-        f32x4 four = squares[0];
-#pragma unroll
-        for (int i = 1; i < kSumLoads; ++i) four += squares[i];
-        float total = (four.x + four.y) + (four.z + four.w);
-#pragma unroll
-        for (int off = 1; off <= 4; off <<= 1) total += __shfl_xor(total, off);
-        if (threadIdx.x % 8 == 0) scale[threadIdx.x / 8] = 1.0f / sqrtf(total / (float)A.K + A.eps);
-        __syncthreads();
-    }
 
     // where two wavefronts share a tile, each holds the sums over its halves of the steps, and finishes half of the rows
     constexpr int H = TM / T::WK;
@@ -113,7 +88,6 @@ __global__ __launch_bounds__(T::kThreads, T::kWaves / 4) void linear_kernel(cons
         for (int j = 0; j < TN; ++j) {
             if constexpr (T::WK == 2) sum[j] = (tile.wk ? acc[H + i][j] : acc[i][j]) + theirs[(i * TN + j) * 64];
             else sum[j] = acc[i][j];
-            if constexpr (SCALED) sum[j] *= scale[m - m0];
         }
         if constexpr (FORM == kHeads) {                      // the projection's rounding; rows of 128 bf16 and 16 bytes
             __bf16* row = reinterpret_cast<__bf16*>(lds + kSumsBytes<T>) + (m - m0) * kHeadPitch;
@@ -167,7 +141,7 @@ __global__ __launch_bounds__(T::kThreads, T::kWaves / 4) void linear_kernel(cons
     }
 }
 
-template <int BM, int BN, int WM, int WN, int WK, int S, int SX, int FORM, bool WIDE = false, bool SCALED = false>
+template <int BM, int BN, int WM, int WN, int WK, int S, int SX, int FORM, bool WIDE = false>
 int launch(LinearParams A, hipStream_t stream)
 {
     typedef Tile<BM, BN, WM, WN, WK, S, SX, FORM == kSilu, WIDE> T;
@@ -175,13 +149,13 @@ int launch(LinearParams A, hipStream_t stream)
     static_assert(kLdsBytes <= 160 * 1024, "LDS");
     static_assert(FORM != kHeads || (BN == mdx_qk::kHeadDim && WK == 2 && BM % (T::kThreads / mdx_qk::kLanesPerRow) == 0), "a head per column tile");
     static std::atomic<bool> raised[64];
-    const int rc = reserve_lds(reinterpret_cast<const void*>(linear_kernel<T, FORM, SCALED>), kLdsBytes, raised, "linear");
+    const int rc = reserve_lds(reinterpret_cast<const void*>(linear_kernel<T, FORM>), kLdsBytes, raised, "linear");
     if (rc != MDX_OK) return rc;
     A.m_tiles = (A.in.M + BM - 1) / BM;
     A.n_tiles = (A.in.N + T::kCols - 1) / T::kCols;
     const int64_t grid = (int64_t)A.m_tiles * A.n_tiles * A.splits;
     MDX_REQUIRE(grid < ((int64_t)1 << 31), MDX_EUNSUPPORTED, "linear: %lld tiles", (long long)grid);
-    linear_kernel<T, FORM, SCALED><<<(unsigned)grid, T::kThreads, kLdsBytes, stream>>>(A);
+    linear_kernel<T, FORM><<<(unsigned)grid, T::kThreads, kLdsBytes, stream>>>(A);
     return mdx::check_launch("linear");
 }
 
@@ -409,34 +383,6 @@ extern "C" int mdx_linear_qk_norm_rope_store(const void* x, int64_t x_row_stride
                        (__bf16*)q_out, q_out_row_stride, (__bf16*)k_out, k_out_row_stride, (__bf16*)v_out, v_out_row_stride,
                        (__bf16*)k_cache, (__bf16*)v_cache, slot_mapping, num_slots, num_q_heads, num_kv_heads};
     return heads_plan(rows, n, k).run(A, static_cast<hipStream_t>(stream));
-}
-
-// The gate/up projection of rows that mdx_linear_residual leaves, on the tiles that the plan has for so few.
-namespace {
-constexpr int64_t kMaxScaledRows = 64, kMaxScaledK = 16 * 32 * kSumLoads;
-}
-
-extern "C" int32_t mdx_linear_scaled_silu_supported(int64_t rows, int64_t n, int64_t k)
-{
-    return sizes_covered(rows, n, k) && rows <= kMaxScaledRows && k % 512 == 0 && k <= kMaxScaledK;
-}
-
-extern "C" int mdx_linear_scaled_silu(const void* z, int64_t z_row_stride, const float* sums, float eps, const void* w, int64_t w_row_stride,
-                                      void* y, int64_t y_row_stride, int64_t rows, int64_t n, int64_t k, mdx_stream_t stream)
-{
-    const char* what = "linear_scaled_silu";
-    MDX_REQUIRE(mdx_linear_scaled_silu_supported(rows, n, k), MDX_EUNSUPPORTED, "%s: %lld rows (up to %lld), n %lld (a multiple of 8), k %lld (a multiple of 512 up to %lld)", what,
-                (long long)rows, (long long)kMaxScaledRows, (long long)n, (long long)k, (long long)kMaxScaledK);
-    const int rc = check_linear(what, false, z, z_row_stride, w, w_row_stride, y, rows, n, k);
-    if (rc != MDX_OK) return rc;
-    MDX_REQUIRE(y_row_stride % 4 == 0 && y_row_stride >= n, MDX_EUNSUPPORTED, "%s: row stride of y (a multiple of 4, at least n)", what);
-    MDX_REQUIRE(sums && mdx::aligned16(sums) && eps >= 0.f, MDX_EINVAL, "%s: the sums of squares (16-byte aligned) and eps", what);
-    LinearParams A = params_of(z, z_row_stride, w, w_row_stride, rows, n, k);
-    A.y = (__bf16*)y; A.y_stride = y_row_stride;
-    A.sums = sums; A.n_sums = (int)(k / 16); A.eps = eps;
-    // (k of 512 and more is steps enough for either; 33 to 64 rows in two tiles of 32 would read W twice)
-    if (rows <= 32) return launch<32, 64, 2, 2, 1, 4, 4, kSilu, false, true>(A, static_cast<hipStream_t>(stream));
-    return launch<64, 64, 2, 2, 2, 4, 4, kSilu, false, true>(A, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int32_t mdx_decode_linear_splits(int64_t rows, int64_t n, int64_t k) { return decode_plan(rows, n, k).splits; }

@@ -64,10 +64,6 @@ SIGNATURES = {
     "mdx_decode_linear_partials": (c_int32, [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _P]),
     "mdx_decode_linear_silu_supported": (c_int32, [_I64] * 3),
     "mdx_decode_linear_silu": (c_int32, [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _I64, _P]),
-    "mdx_linear_residual_supported": (c_int32, [_I64] * 3),
-    "mdx_linear_residual": (c_int32, [_P, _I64] * 4 + [_P, _P, _I64, _P] + [_I64] * 3 + [_P]),
-    "mdx_linear_scaled_silu_supported": (c_int32, [_I64] * 3),
-    "mdx_linear_scaled_silu": (c_int32, [_P, _I64, _P, _F, _P, _I64, _P, _I64] + [_I64] * 3 + [_P]),
     "mdx_add_rms_norm_partials": (c_int32, [_P, _I32, _P, _I64, _P, _I64, _P, _F, _P, _I64, _I64, _I32, _I32, _P]),
     "mdx_qk_norm_rope_store_partials": (c_int32, [_P, _I32, _P, _P, _F, _P, _P, _I64, _P, _P, _I64, _P, _P, _P, _I64,
                                                   _I64, _I32, _I32, _I32, _I32, _P]),

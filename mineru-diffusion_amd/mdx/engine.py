@@ -32,7 +32,7 @@ from torch import nn
 from . import _lib
 from .context import get_context, reset_context, set_context
 from .layers import Attention
-from .ops import (confidence_argmax, lm_head_confidence, flash_attn_with_kvcache_read_ahead, linear, linear_gated, linear_qk_norm_rope_store, linear_residual_gated, qk_norm_rope_store,
+from .ops import (confidence_argmax, lm_head_confidence, flash_attn_with_kvcache_read_ahead, linear, linear_gated, linear_qk_norm_rope_store, qk_norm_rope_store,
                   qk_norm_rope_store_partials, rms_norm, rms_norm_partials, select_transfer, silu_and_mul, sparse_attn_varlen, unmask_step)
 
 PAGE = 256                      # tokens per KV page (Sequence.kvcache_block_size, sequence.py:17)
@@ -222,9 +222,6 @@ class DecoderLayer(nn.Module):
             k = _rms(k, self.k_norm, c.rms_norm_eps)
             q, k = _rope(q, cos, sin), _rope(k, cos, sin)
             o = self.attn(q, k, v)
-        few = linear_residual_gated(o, self.o_proj, residual, self.post_attention_layernorm, c.rms_norm_eps, self.gate_up_proj) if c.fused_layer_ops else None
-        if few is not None:
-            return self._linear(few[0], self.down_proj), few[1]
         h, residual = self._norm(self._linear(o, self.o_proj), residual, self.post_attention_layernorm)
         if c.fused_layer_ops:
             act = linear_gated(h, self.gate_up_proj)

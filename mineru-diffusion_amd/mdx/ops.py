@@ -84,12 +84,6 @@ def linear_qk_norm_rope_store(x, weight, q_weight, k_weight, eps, cos, sin, posi
                                              k_cache, v_cache, slot_mapping, want_kv)
 
 
-def linear_residual_gated(x, weight, residual, norm_weight, eps, gate_up_weight):
-    """(linear_gated(h, gate_up_weight), s) with h, s = rms_norm(x . weight^T, norm_weight, eps, residual), for up to 64 rows in two launches
-    (nanovllm/models/sdar.py:84,150-152,105-111); None where the shapes are not covered."""
-    return _host().linear_residual_gated(x, weight, residual, norm_weight, eps, gate_up_weight)
-
-
 def linear_partials(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor | None:
     """The partial sums of up to 128 rows, also where there is one slice only."""
     return _host().linear_partials(x, weight)

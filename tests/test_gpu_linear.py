@@ -177,42 +177,30 @@ def test_linear_qk_norm_rope_store_says_what_it_does_not_cover(dev):
     assert call(z(400, 264)[:, 1:257], z(512, 256), 2, 1, 128) is None and call(z(400, 256), z(512, 256), 2, 1, 128) is not None
 
 
-@pytest.mark.parametrize("rows,n,k,i", [(1, 512, 512, 264), (16, 2048, 2048, 512), (17, 1024, 1536, 72), (32, 2048, 3584, 264), (32, 4096, 4096, 72), (33, 1536, 4096, 264),
-                                        (50, 2048, 2048, 8), (64, 512, 2560, 520)])
-def test_residual_norm_and_gated(dev, rows, n, k, i):
-    """The two launches of linear_residual_gated at the edges of their row tiles, of a wavefront's ring of steps and of the sums that a lane takes, on rows of
-    wider matrices, against fp64.  s is rounded behind the layer's own rounding (2^-8 of its norm together at most) and passes through the norm and the
-    product as it is; so does the rounding of z; the SiLU's two roundings are those of linear_gated (3e-3)."""
-    import mdx
-    from mdx import ops
-    g = torch.Generator().manual_seed(rows + n + k)
-    rand = lambda *s: torch.randn(*s, generator=g)                                         # noqa: E731
-    x, w, res = rand(rows, k + 8).bfloat16(), (rand(n, k + 16) * 0.05).bfloat16(), (rand(rows, n + 8) * 4).bfloat16()
-    nw, v = (1 + 0.2 * rand(n)).bfloat16(), (rand(2 * i, n + 8) * 0.05).bfloat16()
-    args = (x.to(dev)[:, :k], w.to(dev)[:, :k], res.to(dev)[:, :n], nw.to(dev), 1e-6, v.to(dev)[:, :n])
-    y, new = ops.linear_residual_gated(*args)
-    s = res[:, :n].double() + x[:, :k].double() @ w[:, :k].double().T
-    assert (new.double().cpu() - s).norm() < 2.0 ** -8 * s.norm()
-    h = s * torch.rsqrt(s.square().mean(1, keepdim=True) + 1e-6) * nw.double()
-    gate, up = (h @ v[:, :n].double().T).chunk(2, dim=1)
-    ref = torch.nn.functional.silu(gate) * up
-    err = (y.double().cpu() - ref).norm() / ref.norm()
-    # the launches for more rows, whose norm rounds twice, lie no nearer (5 %: single roundings that fall either way)
-    old_h, old_s = ops.rms_norm_partials(ops.linear_partials(args[0], args[1]), args[3], 1e-6, args[2].contiguous())
-    old = (ops.linear_gated(old_h, args[5]).double().cpu() - ref).norm() / ref.norm()
-    assert err < 3e-3 + 2 * 2.0 ** -8 and err < 1.05 * old
-    assert (new.float() - old_s.float()).norm() < 2.0 ** -9 * old_s.float().norm()         # (a value on a rounding boundary may fall either way)
-    assert all(torch.equal(a, b) for a, b in zip((y, new), ops.linear_residual_gated(*args)))
-    zero = ops.linear_residual_gated(torch.zeros_like(args[0]), args[1], torch.zeros_like(args[2]), *args[3:])
-    assert not zero[0].any() and not zero[1].any()                                         # (rows of zeros: divided by the root of eps)
-
-
-def test_residual_norm_and_gated_says_what_it_does_not_cover(dev):
-    from mdx import ops
-    t = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=dev)                       # noqa: E731
-    for rows, n, k, i in ((65, 512, 512, 64), (4, 528, 512, 64), (4, 512, 768, 64), (4, 4608, 512, 64), (4, 512, 4608, 64), (0, 512, 512, 64), (4, 512, 512, 12)):
-        assert ops.linear_residual_gated(t(rows, k), t(n, k), t(rows, n), t(n), 1e-6, t(2 * i, n)) is None
-    assert ops.linear_residual_gated(t(4, 513)[:, 1:], t(512, 512), t(4, 512), t(512), 1e-6, t(128, 512)) is None
-    assert ops.linear_residual_gated(t(4, 512), t(512, 512), t(4, 512), t(513)[1:], 1e-6, t(128, 512)) is None
-    y, s = ops.linear_residual_gated(t(2, 3, 512), t(512, 512), t(2, 3, 512), t(512), 1e-6, t(128, 512))
-    assert y.shape == (2, 3, 64) and s.shape == (2, 3, 512)
+@pytest.mark.parametrize("rows", [1, 16, 32, 33, 64, 65])
+def test_layer_of_few_rows_rounds_where_the_reference_does(dev, rows):
+    """Behind the attention a decoder layer rounds the normed sum, and again behind the norm's weight (layernorm.py:28-41), however few rows there are.  Small
+    integers and rows of an identity matrix as weights: every product is exact in any order, so that what comes out is the oracle's but for a reciprocal
+    root or a SiLU on a rounding boundary (below 3 % of the values, one step; with one rounding for both, nearly half of them differ)."""
+    import oracle
+    from mdx.engine import DecoderConfig, DecoderLayer
+    h = 512
+    c = DecoderConfig(hidden_size=h, num_heads=4, num_kv_heads=2, intermediate_size=h)
+    layer = DecoderLayer(c).to(dev, torch.bfloat16)
+    g = torch.Generator().manual_seed(rows)
+    o, w = (torch.randint(-2, 3, s, generator=g).bfloat16() for s in ((rows, h), (h, h)))
+    x, nw = (torch.randn(rows, h, generator=g) * 9).bfloat16(), (1 + 0.3 * torch.randn(h, generator=g)).bfloat16()
+    eye = torch.eye(h).bfloat16()
+    with torch.no_grad():
+        layer.o_proj.copy_(w)
+        layer.gate_up_proj.copy_(torch.cat((eye, eye.roll(7, 0))))
+        layer.down_proj.copy_(eye)
+        layer.post_attention_layernorm.copy_(nw)
+        layer._attend_fused = lambda *_: o.to(dev)
+        y, residual = layer(None, x.to(dev), None, None, None)
+    y = (y.sum(0) if y.dim() == 3 else y).bfloat16().cpu()
+    normed, s = oracle.add_rms_norm((o.float() @ w.float().T).bfloat16(), x, nw, c.rms_norm_eps)
+    want = oracle.silu_and_mul(torch.cat((normed, normed.roll(7, 1)), 1))
+    assert torch.equal(residual.cpu(), s)
+    assert (y == want).float().mean() > 0.97
+    assert (y.float() - want.float()).norm() < 2.0 ** -9 * want.float().norm()
