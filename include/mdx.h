@@ -250,7 +250,8 @@ int mdx_paged_block_attn_static(const void* q, void* o, const void* k_cache, con
  *
  * x [rows, hidden] and w [vocab, hidden], MDX_BF16, row strides in elements (multiples of 8, 16-byte
  * aligned bases); hidden a multiple of 128.  The logits x . w^T are accumulated in fp32 and rounded to
- * bf16, as the projection's output is in the reference; then x0[r] = first index of the row's maximum,
+ * bf16, as the projection's output is in the reference (in an order that does not depend on the row of w: equal
+ * rows have equal logits); then x0[r] = first index of the row's maximum,
  * x0_p[r] = softmax(logits / T)[x0[r]].  temperatures (NULL = 1.0): row r uses entry
  * (row_ids ? row_ids[r] : r) / rows_per_temp, so that rows compacted out of [bs, block] keep their
  * sequence's temperature; row_ids may be NULL.  The workspace (mdx_lm_head_confidence_workspace_bytes,

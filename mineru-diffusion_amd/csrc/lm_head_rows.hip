@@ -9,12 +9,12 @@
 //    streams its own rows of W, three steps of 256 columns (24 KB) ahead of the product;
 //  * otherwise x goes through LDS K step by K step with a barrier per step, W one step ahead.
 //
-// Rows of W are as far apart as a power of two, mostly, so that what all workgroups ask for at the same column meets in few of the memory's channels: each workgroup
-// (and, with x whole, each wavefront) begins its rows at another column and comes round.  us, all from column 0 / each XCD's workgroups from another one: 16 rows 118.5 / 111.2, 32
-// 119.8 / 112.5, 64 141.5 / 128.3, 128 171.0 / 165.9 (by wavefront only 116.5, 118.2, 140.8, 169.8; by the workgroup's place in its XCD 112.7, 114.1, 135.2, 164.0).
+// All workgroups sum a row of W from column 0 on, so that equal rows have equal logits and the first of them is taken.  (Beginning at another column each
+// spreads the rows, which are mostly a power of two apart, over more of the memory's channels: 119 / 120 / 141 / 171 us below are 111 / 112 / 128 / 166 then.
+// Equal rows in different tiles then round apart.)
 //
 // W is read with ordinary loads: marked nontemporal, the two loads that share a 128-byte line fetch it twice now and then (139
-// against 129 us at 32 rows).  Bound: HBM.  us at 16 / 32 / 64 / 128 rows: 111 / 112 / 128 / 166 (5.5 TB/s at 32 rows); tiles of 256 rows
+// against 129 us at 32 rows).  Bound: HBM.  us at 16 / 32 / 64 / 128 rows: 119 / 120 / 140 / 170 (5.2 TB/s at 32 rows); tiles of 256 rows
 // 200 / 199 / 208 / 200, the library's product and a vocabulary pass 213 / 155 / 161 / 175.
 #include "lm_head.h"
 #include <atomic>
@@ -157,10 +157,8 @@ __global__ __launch_bounds__(kThreads, 1) void lm_head_whole_kernel(const LmHead
     for (int k = 0; k < P.hidden; k += kPanel) load_x<MT, kPanel>(P, lds0 + k / kPanel * kPanelBytes, k, wave, lane);
     Weights<kSub / 64> ring[kRing];
     int f_tile = blockIdx.x, f_sub = 0, m_tile = blockIdx.x, m_sub = 0;           // the step being fetched, and the one being multiplied
-    const int turn = (wave + (int)blockIdx.x) % subs;
-    auto turned = [&](int sub) { return sub + turn < subs ? sub + turn : sub + turn - subs; };
     auto fetch = [&](Weights<kSub / 64>& d) {
-        load_weights(d, P, f_tile, turned(f_sub) * kSub, wave, lane);
+        load_weights(d, P, f_tile, f_sub * kSub, wave, lane);
         if (++f_sub == subs) { f_sub = 0; f_tile += gridDim.x; }
     };
 #pragma unroll
@@ -172,8 +170,7 @@ __global__ __launch_bounds__(kThreads, 1) void lm_head_whole_kernel(const LmHead
             if (t + r + kRing - 1 < n_steps) fetch(ring[(r + kRing - 1) % kRing]);
             __builtin_amdgcn_sched_barrier(0);
             if (t + r < n_steps) {
-                const int sub = turned(m_sub);
-                multiply<MT, kPanel>(acc, ring[r], lds + sub / 2 * kPanelBytes, (sub & 1) * (kSub / 8), lane);
+                multiply<MT, kPanel>(acc, ring[r], lds + m_sub / 2 * kPanelBytes, (m_sub & 1) * (kSub / 8), lane);
                 if (++m_sub == subs) {
                     rows.take(acc, m_tile * kTileRows + wave * 16 + 4 * (lane >> 4), P.vocab);
                     m_sub = 0;
@@ -203,11 +200,9 @@ __global__ __launch_bounds__(kThreads, 1) void lm_head_rows_kernel(const LmHeadP
 
     Weights<kPairs> a, b;
     int f_tile = blockIdx.x, f_chunk = 0, m_tile = blockIdx.x, m_chunk = 0;       // the step being fetched, and the one being multiplied
-    const int turn = (int)blockIdx.x % chunks;
     auto fetch = [&](Weights<kPairs>& d, int buf) {
-        const int chunk = f_chunk + turn < chunks ? f_chunk + turn : f_chunk + turn - chunks;
-        load_x<MT, KC>(P, lds0 + buf * kBufBytes, chunk * KC, wave, lane);
-        load_weights(d, P, f_tile, chunk * KC, wave, lane);
+        load_x<MT, KC>(P, lds0 + buf * kBufBytes, f_chunk * KC, wave, lane);
+        load_weights(d, P, f_tile, f_chunk * KC, wave, lane);
         if (++f_chunk == chunks) { f_chunk = 0; f_tile += gridDim.x; }
     };
     auto step = [&](const Weights<kPairs>& d, int buf) {

@@ -174,3 +174,19 @@ def test_lm_head_confidence_of_values_that_are_not_finite(dev, rows, vocab, hidd
         assert torch.equal(x0, t0.view(-1)), f"{name}: tokens"
         whole = ~logits.isnan().any(1).to(dev)
         torch.testing.assert_close(p[whole], tp.view(-1)[whole], rtol=3e-5, atol=0, msg=lambda m: f"{name}: {m}")
+
+
+@pytest.mark.parametrize("rows", [1, 32, 33, 64, 65, 128, 129, 250])
+@pytest.mark.parametrize("half,hidden", [(20001, 2048), (1030, 512), (20001, 2560)])
+def test_lm_head_confidence_equal_rows_of_w(dev, rows, half, hidden):
+    """Every row of W twice, `half` rows apart, in another tile, wavefront and lane: equal rows have equal logits, so the first of them is taken.  Two large
+    terms that cancel pass through the sums, so that sums in another order would round to another bf16 value in every few."""
+    import mdx
+    g = torch.Generator().manual_seed(rows + hidden)
+    x, w = torch.randn(rows, hidden, generator=g), torch.randn(half, hidden, generator=g) * (3.0 / hidden ** 0.5)
+    x[:, 5] = x[:, hidden // 2 + 9] = 2.0 ** 14
+    w[:, 5], w[:, hidden // 2 + 9] = 1, -1
+    w = w.bfloat16().repeat(2, 1)
+    x0, p = mdx.lm_head_confidence(x.bfloat16().to(dev), w.to(dev))
+    torch.cuda.synchronize()
+    assert torch.isfinite(p).all() and (x0 < half).all()
