@@ -532,11 +532,12 @@ PyObject* sparse_attn_varlen(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // ---- paged decode -----------------------------------------------------------------------------------
-// The arrival counters of mdx_paged_block_attn_single_launch that this module keeps: one buffer per device and
-// stream, zero when created, left zero by every launch.  Launches on one stream run one after the other, so they can
-// share a buffer; a HIP graph keeps using the buffer of the stream it was captured on wherever it is replayed, which
-// is why a buffer, once handed out, is never replaced or freed: it has its full size from the start.  None (undefined) when the
-// request does not fit it, or while a graph is being captured and that stream has no buffer yet (it could not be
+// The arrival counters of mdx_paged_block_attn_single_launch that this module keeps: two buffers per device and
+// stream, zero when created, left zero by every launch.  Eager launches on one stream run one after the other, so they can
+// share one; a HIP graph keeps using the buffer that it was captured with wherever and beside whatever it is replayed, which
+// is why captured calls have the other one, and why a buffer, once handed out, is never replaced or freed: it has its full size from the
+// start.  (Several graphs captured on one stream share theirs: they run one after the other, or with counters of the caller's.)  None (undefined)
+// when the request does not fit it, or while a graph is being captured and that stream has no buffers yet (they could not be
 // zeroed outside the graph): the caller then takes the two-launch entry point -- run the forward once on the capture
 // stream before capturing.
 bool capturing(const Tensor& like) {
@@ -544,19 +545,33 @@ bool capturing(const Tensor& like) {
     return hipStreamIsCapturing(static_cast<hipStream_t>(stream_of(like)), &status) != hipSuccess || status != hipStreamCaptureStatusNone;
 }
 constexpr int64_t kCounterFloats = 64 * 256;   // the single-launch path exists for up to 64 sequences; 256 head groups is far beyond any model
-Tensor counters_for(const Tensor& like, int64_t bytes) {
-    static auto* kept = new std::map<std::pair<int, void*>, Tensor>();      // (never destroyed: the driver may be gone at exit)
+struct KeptCounters { Tensor eager, captured; };
+KeptCounters kept_counters_of(const Tensor& like, bool create) {
+    static auto* kept = new std::map<std::pair<int, void*>, KeptCounters>();      // (never destroyed: the driver may be gone at exit)
     static std::mutex lock;
-    if (bytes > kCounterFloats * 4) return Tensor();
-    void* stream = stream_of(like);
-    const std::pair<int, void*> key{like.device().index(), stream};
+    const std::pair<int, void*> key{like.device().index(), stream_of(like)};
     std::lock_guard<std::mutex> guard(lock);
     auto it = kept->find(key);
     if (it != kept->end()) return it->second;
-    if (capturing(like)) return Tensor();
-    Tensor t = at::zeros({kCounterFloats}, at::TensorOptions().dtype(at::kFloat).device(like.device()));
-    kept->emplace(key, t);
-    return t;
+    if (!create) return {};
+    const Tensor both = at::zeros({2, kCounterFloats}, at::TensorOptions().dtype(at::kFloat).device(like.device()));
+    return kept->emplace(key, KeptCounters{both[0], both[1]}).first->second;
+}
+Tensor counters_for(const Tensor& like, int64_t bytes, bool captured) {
+    if (bytes > kCounterFloats * 4) return Tensor();
+    const KeptCounters kept = kept_counters_of(like, !captured);
+    return captured ? kept.captured : kept.eager;
+}
+
+// a tensor of the device -> the counters kept for the current stream (eager calls', captured calls'), or None
+PyObject* kept_counters(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    ARGS(1);
+    return guarded([&]() -> PyObject* {
+        need_gpu({&tensor(a[0])});
+        const KeptCounters kept = kept_counters_of(tensor(a[0]), false);
+        if (!kept.eager.defined()) Py_RETURN_NONE;
+        return wrap_tuple(kept.eager, kept.captured);
+    });
 }
 
 // counters: None = single launch with this module's counters, False = two launches, a tensor = the caller's.
@@ -580,10 +595,11 @@ Tensor paged(const Tensor& q_, const Tensor& k_cache, const Tensor& v_cache, con
     const Tensor ws = bytes > 0 ? make(q, at::kByte, bytes) : Tensor();
     Tensor counters;
     if (counters_arg == Py_None) {         // more than 64 sequences never take the single-launch path
-        // Launches that may do without (mdx_paged_block_attn_needs_counters) leave the kept buffer out of graphs: two graphs captured on one
+        // Launches that may do without (mdx_paged_block_attn_needs_counters) leave the kept buffers out of graphs: two graphs captured on one
         // stream may be replayed beside each other.
-        if (bs <= 64 && (!capturing(q) || mdx_paged_block_attn_needs_counters((int32_t)bs, (int32_t)sq, (int32_t)hq, (int32_t)hkv, (int32_t)bt.size(1), (int32_t)page)))
-            counters = counters_for(q, mdx_paged_block_attn_counter_bytes((int32_t)bs, (int32_t)hq, (int32_t)hkv));
+        const bool captured = bs <= 64 && capturing(q);
+        if (bs <= 64 && (!captured || mdx_paged_block_attn_needs_counters((int32_t)bs, (int32_t)sq, (int32_t)hq, (int32_t)hkv, (int32_t)bt.size(1), (int32_t)page)))
+            counters = counters_for(q, mdx_paged_block_attn_counter_bytes((int32_t)bs, (int32_t)hq, (int32_t)hkv), captured);
     } else if (counters_arg != Py_False) {
         counters = tensor(counters_arg);
         NEED(counters.scalar_type() == at::kFloat && counters.is_contiguous() && counters.device() == q.device());
@@ -937,7 +953,7 @@ PyObject* sampler_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyMethodDef methods[] = {
     ENTRY(store_kvcache), ENTRY(store_kvcache_maybe4d), ENTRY(qk_norm_rope_store), ENTRY(rms_norm), ENTRY(silu_and_mul), ENTRY(linear), ENTRY(linear_gated), ENTRY(linear_qk_norm_rope_store), ENTRY(linear_partials), ENTRY(linear_silu),
     ENTRY(rms_norm_partials), ENTRY(qk_norm_rope_store_partials), ENTRY(sparse_attn_varlen),
-    ENTRY(flash_attn_with_kvcache), ENTRY(flash_attn_with_kvcache_read_ahead), ENTRY(attention_prefill), ENTRY(attention_decode), ENTRY(confidence_argmax), ENTRY(lm_head_confidence),
+    ENTRY(flash_attn_with_kvcache), ENTRY(flash_attn_with_kvcache_read_ahead), ENTRY(kept_counters), ENTRY(attention_prefill), ENTRY(attention_decode), ENTRY(confidence_argmax), ENTRY(lm_head_confidence),
     ENTRY(filter_logits), ENTRY(select_transfer), ENTRY(unmask_step), ENTRY(sampler_step),
     {nullptr, nullptr, 0, nullptr},
 };

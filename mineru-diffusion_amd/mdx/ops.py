@@ -132,8 +132,8 @@ def flash_attn_with_kvcache(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
     cache_seqlens [bs] int32, non-causal.  Returns o like q.
 
     counters (keyword, not in the reference): None = single launch, where that pays, with this module's arrival
-    counters (one buffer per device and stream; while a graph is captured only for launches that need them); a zeroed fp32
-    tensor of the caller's = the same with those; False = attention launch + combine launch."""
+    counters (per device and stream, one buffer for eager calls and one for captured ones, which only launches that need them
+    take); a zeroed fp32 tensor of the caller's = the same with those; False = attention launch + combine launch."""
     if causal:
         raise MdxError("flash_attn_with_kvcache: only causal=False (block-diffusion decode) is implemented")
     return _host().flash_attn_with_kvcache(q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale, counters)

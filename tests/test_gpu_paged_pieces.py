@@ -131,3 +131,53 @@ def test_pieces_merged_by_the_last_to_arrive(dev, ctxs, hq, hkv, dtype):
         assert torch.equal(mdx.flash_attn_with_kvcache(*args, **kw, counters=other), two)
         torch.cuda.synchronize()
         assert torch.equal(got, two) and own.abs().sum().item() == 0
+
+
+def _paged_args(dev, ctxs, hq, hkv, seed):
+    g = torch.Generator().manual_seed(seed)
+    d, page = 128, 256
+    counts = [-(-c // page) for c in ctxs]
+    q = torch.randn(len(ctxs), 32, hq, d, generator=g).bfloat16().to(dev)
+    kc, vc = (torch.randn(sum(counts), page, hkv, d, generator=g).bfloat16().to(dev) for _ in range(2))
+    bt, at = torch.full((len(ctxs), max(counts)), -1, dtype=torch.int32), 0
+    for b, n in enumerate(counts):
+        bt[b, :n] = torch.arange(at, at + n)
+        at += n
+    return (q, kc, vc), dict(cache_seqlens=torch.tensor(ctxs, dtype=torch.int32, device=dev), block_table=bt.to(dev), softmax_scale=d ** -0.5)
+
+
+def test_eager_and_captured_calls_count_in_buffers_of_their_own(dev):
+    """A graph may be replayed beside eager calls on the stream that it was captured on, so neither uses the other's arrival counters.  Counters that don't begin at
+    zero merge nothing: with the other kind's set to a half, each call gives the right result and leaves them alone."""
+    import mdx
+    from mdx.ops import _host
+    many, few = _paged_args(dev, _spread(24, 90, 1500), 16, 8, 1), _paged_args(dev, _spread(16, 300, 1280), 16, 8, 2)   # cut by shares; pieces merged where counters are at hand
+    call = lambda case: mdx.flash_attn_with_kvcache(*case[0], **case[1])                               # noqa: E731
+    want = [mdx.flash_attn_with_kvcache(*case[0], **case[1], counters=False) for case in (many, few)]
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        assert torch.equal(call(many), want[0]) and torch.equal(call(few), want[1])
+        eager, captured = _host().kept_counters(many[0][0])
+        torch.cuda.synchronize()
+        assert eager.data_ptr() + 4 * eager.numel() <= captured.data_ptr() or captured.data_ptr() + 4 * captured.numel() <= eager.data_ptr()
+        assert not eager.any() and not captured.any()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        got = [call(many), call(few)]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        captured.fill_(0.5)
+        assert torch.equal(call(many), want[0]) and torch.equal(call(few), want[1])
+        assert not eager.any() and (captured == 0.5).all()
+        captured.zero_()
+        eager.fill_(0.5)
+    torch.cuda.synchronize()
+    for _ in range(3):                       # on the current stream, another than the graph was captured on
+        for t in got:
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want)) and not captured.any() and (eager == 0.5).all()
+    eager.zero_()
+    torch.cuda.synchronize()
