@@ -592,7 +592,8 @@ class BlockDiffusionEngine:
         g["slots"] = torch.full((gbs, S), -1, dtype=i32, device=dev)
         g["ctx"] = torch.zeros(gbs, dtype=i32, device=dev)
         # the attention's arrival counters: the lanes' own, since their graphs may run beside other graphs captured on this stream
-        g["counters"] = torch.zeros(max(1, _lib.lib().mdx_paged_block_attn_counter_bytes(gbs, self.c.num_heads, self.c.num_kv_heads) // 4), device=dev)
+        g["counters"] = torch.zeros(max(1, _lib.lib().mdx_paged_block_attn_counter_bytes(gbs, self.c.num_heads, self.c.num_kv_heads) // 4),
+                                    dtype=f32, device=dev)
         g["x0"] = torch.zeros(gbs * S, dtype=i64, device=dev)
         g["x0_p"] = torch.zeros(gbs * S, dtype=f32, device=dev)
         g["rows"] = torch.zeros(gbs * S, dtype=i64, device=dev)

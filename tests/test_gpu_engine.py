@@ -337,3 +337,24 @@ def test_stop_token_ends_the_sequence_at_its_block(dev):
     eng.generate()
     assert s.num_completion_tokens == end and s.completion_token_ids == tokens[:end]
     assert len(eng.block_manager.free) == 8
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float64])
+def test_device_loop_under_another_default_dtype(dev, dtype):
+    """The lanes' buffers, the attention's fp32 arrival counters among them, don't follow torch's default dtype (16 bits are common where models are built)."""
+    from mdx.engine import BlockDiffusionEngine, SamplingParams
+    _, model = _tiny(dev)
+    sp = SamplingParams(max_new_tokens=64, ignore_eos=True, transfer_count=4, dynamic_threshold=1.0)
+
+    def tokens():
+        eng = BlockDiffusionEngine(model, num_pages=8, decode_graphs=True, max_model_len=512)
+        seq = eng.add_request(list(range(100)), sp)
+        eng.generate()
+        return seq.completion_token_ids
+    want = tokens()
+    before = torch.get_default_dtype()
+    torch.set_default_dtype(dtype)
+    try:
+        assert tokens() == want
+    finally:
+        torch.set_default_dtype(before)
