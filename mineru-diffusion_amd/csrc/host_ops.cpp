@@ -658,16 +658,16 @@ PyObject* attention_prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
     });
 }
 
-// q, k, v, k_cache, v_cache, slot_mapping, context_lens, block_tables, scale -> o [bs, Sq, Hq * d]
+// q, k, v, k_cache, v_cache, slot_mapping, context_lens, block_tables, scale, counters -> o [bs, Sq, Hq * d]
 PyObject* attention_decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
-    ARGS(9);
+    ARGS(10);
     return guarded([&]() -> PyObject* {
         const Tensor &q = tensor(a[0]), &k_cache = tensor(a[3]), &v_cache = tensor(a[4]);
         if (k_cache.numel() > 0 && v_cache.numel() > 0) {
             need_gpu({&q});
             store_maybe4d(tensor(a[1]), tensor(a[2]), k_cache, v_cache, tensor(a[5]), stream_of(q));
         }
-        return wrap(paged(q, k_cache, v_cache, tensor(a[6]), tensor(a[7]), a[8], Py_None, true));
+        return wrap(paged(q, k_cache, v_cache, tensor(a[6]), tensor(a[7]), a[8], a[9], true));
     });
 }
 

@@ -29,10 +29,10 @@ def get_context() -> Context:
 
 
 def set_context(is_prefill, cu_seqlens_q=None, cu_seqlens_k=None, max_seqlen_q=0, max_seqlen_k=0,
-                slot_mapping=None, context_lens=None, block_tables=None, block_size=32) -> None:
+                slot_mapping=None, context_lens=None, block_tables=None, block_size=32, counters=None) -> None:
     global _CONTEXT
     _CONTEXT = Context(is_prefill, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
-                       slot_mapping, context_lens, block_tables, block_size)
+                       slot_mapping, context_lens, block_tables, block_size, counters)
 
 
 def reset_context() -> None:

@@ -629,8 +629,7 @@ class BlockDiffusionEngine:
         _lib.check(_lib.lib().mdx_block_prepare(g["lens"].data_ptr(), g["phase"].data_ptr(), g["bt"].data_ptr(), g["bt"].stride(0),
                                                 g["width"], PAGE, S, g["pos"].data_ptr(), g["slots"].data_ptr(), g["ctx"].data_ptr(),
                                                 g["bs"], stream), "block_prepare")
-        set_context(False, slot_mapping=g["slots"], context_lens=g["ctx"], block_tables=g["bt"], block_size=S)
-        get_context().counters = g["counters"]
+        set_context(False, slot_mapping=g["slots"], context_lens=g["ctx"], block_tables=g["bt"], block_size=S, counters=g["counters"])
         hidden = self.model(self.model.embed(g["ids"]), g["pos"])
         reset_context()
         return hidden

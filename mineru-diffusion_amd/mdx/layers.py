@@ -28,7 +28,7 @@ class Attention(nn.Module):
             return _host().attention_prefill(q, k, v, self.k_cache, self.v_cache, context.slot_mapping, context.cu_seqlens_q,
                                              context.cu_seqlens_k, context.block_size, context.max_seqlen_k, self.scale)
         return _host().attention_decode(q, k, v, self.k_cache, self.v_cache, context.slot_mapping, context.context_lens,
-                                        context.block_tables, self.scale)
+                                        context.block_tables, self.scale, context.counters)
 
 
 class Sampler(nn.Module):

@@ -181,3 +181,41 @@ def test_eager_and_captured_calls_count_in_buffers_of_their_own(dev):
         assert all(torch.equal(a, b) for a, b in zip(got, want)) and not captured.any() and (eager == 0.5).all()
     eager.zero_()
     torch.cuda.synchronize()
+
+
+def test_counters_of_the_context_reach_the_attention(dev):
+    """mdx.Attention in decode mode counts in the buffer that set_context was given, eagerly and from a graph, not in the kept ones."""
+    import mdx
+    from mdx.ops import _host
+    (q, kc, vc), kw = _paged_args(dev, _spread(24, 90, 1500), 16, 8, 3)
+    want = mdx.flash_attn_with_kvcache(q, kc, vc, **kw).flatten(2)
+    attn = mdx.Attention(16, 128, 128 ** -0.5, 8)
+    attn.k_cache, attn.v_cache = kc, vc
+    slots = torch.full((24, 32), -1, dtype=torch.int32, device=dev)                      # (stores nothing)
+    own = torch.zeros(64 * 64, device=dev)
+    kept = _host().kept_counters(q)
+    new = torch.zeros_like(q[:, :, :8])
+
+    def call(counters):
+        mdx.set_context(False, slot_mapping=slots, context_lens=kw["cache_seqlens"], block_tables=kw["block_table"], counters=counters)
+        try:
+            return attn(q, new, new)
+        finally:
+            mdx.reset_context()
+    kept[0].fill_(0.5)                                                                   # (merges nothing)
+    got = call(own)
+    assert torch.equal(got, want) and not own.any()
+    kept[0].zero_()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = call(own)
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        assert torch.equal(call(None), want) and torch.equal(call(False), want)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want) and not own.any()
+    with pytest.raises(AssertionError):
+        call(own.double())
+    assert mdx.get_context().counters is None
