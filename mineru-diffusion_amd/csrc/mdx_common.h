@@ -58,11 +58,12 @@ inline int compute_units() {
 
 namespace mdx {
 
-// A kernel's arguments come through the scalar cache, 64 bytes at a time, and the compiler asks for them where they are first used: a line that
-// is first used behind other loads puts one more trip to memory (0.1 to 0.2 us) into every workgroup's chain.  This asks for all lines of BYTES bytes of
-// arguments, and for the grid's size if it is given, at once.  Returns 0 in a way that the compiler doesn't see, to be added to something that is
-// used early.  (Not a volatile asm: behind one, the compiler no longer takes page tables and lengths for constant and reads them through vector loads.)
-// One sequence through attention and combine: 14.2 -> 13.8 us.
+// A kernel's arguments come through the scalar cache, 64 bytes at a time, and the compiler asks for them where they are first used, some of them behind
+// other loads.  This asks for all lines of BYTES bytes of arguments, and for the grid's size if it is given, at once.  Returns 0 in a way that the
+// compiler doesn't see, to be added to something that is used early.  (Not a volatile asm: behind one, the compiler no longer takes page tables and
+// lengths for constant and reads them through vector loads.)
+// One sequence through attention and combine: 14.2 -> 13.8 us.  Probably a trip to memory less in every workgroup's chain; under the profiler
+// one run differs from the next by as much (attention of one sequence 11.0 to 11.4 us with it, 11.3 without).
 template <int BYTES>
 __device__ __forceinline__ int fetch_arguments(int grid = 0)
 {

@@ -14,9 +14,9 @@
 // rows), so the design goal is to keep the whole chip streaming pages:
 //  * split-KV: a workgroup owns one split of consecutive keys of one sequence
 //    for one group of query heads; the split size is chosen so that there are
-//    one to two workgroups per CU at most (pick_chunk and the rule in the kernel), and with a (sequence, KV head)
-//    pair per CU sequences stay whole unless the kernel finds one far longer
-//    than the mean.  Workgroups are numbered densely over the
+//    one to two workgroups per CU at most (pick_chunk and the rule in the kernel), and with about a (sequence, KV head)
+//    pair per CU sequences stay whole unless the longest is well above what
+//    a resident workgroup's even share of all keys comes to (kWholeFactor).  Workgroups are numbered densely over the
 //    (sequence, split) pairs that exist (lane b of each wavefront holds the
 //    split count of sequence b), so the launch order has no holes: the
 //    dispatcher deals consecutive workgroups round-robin to XCDs and shader
@@ -33,7 +33,8 @@
 //    load queue is not what bounds this kernel.)
 //  * the KW wavefront states of a head are merged through LDS, then either
 //    written as the final output (single split) or as an fp32 partial
-//    (m, l, O) that a second, small kernel combines.
+//    (m, l, O) that the last split of the pair to arrive merges (single launch)
+//    or a second, small kernel combines.
 #include "mdx_common.h"
 #include "attn_tile.h"
 #include <type_traits>
@@ -97,6 +98,7 @@ __device__ __forceinline__ void store_agent(float* p, f32x4 v) {
 // (Not inline asm: the compiler takes such a load's registers for written while it is still on its way, and what it moved or spilled before the wait would be
 // the old contents.  Two atomic loads of eight bytes: 16 sequences of 375-1500 keys 24.9 -> 25.5 us.)
 constexpr int kAgentScope = 16;                      // sc1
+constexpr int kRawBuffer = 0x27000;                  // last word of the descriptor: elements of 32 bits, not swizzled, out of range reads 0
 __device__ __forceinline__ f32x4 load_agent(__amdgpu_buffer_rsrc_t from, int offset) {
     return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from, offset, 0, kAgentScope));
 }
@@ -164,16 +166,17 @@ template <int THREADS> __device__ __forceinline__ void read_ahead(const ReadAhea
     asm volatile("" :: "v"(all));                   // (the loads have a use)
 }
 
-// Running fold of split partials over COLS columns of one query.
-template <int COLS> struct Fold {
-    float M, L, acc[COLS];
+// The combine kernel's running fold of split partials over four columns of one query.  The merge at the end of paged_block_attn_kernel does the same
+// operations in the same order on other columns per lane, and has to: a pair's result has the same bits either way.
+struct Fold {
+    float M, L, acc[4];
     __device__ __forceinline__ void init() {
         M = kMinusBig; L = 0.f;
 #pragma unroll
-        for (int e = 0; e < COLS; ++e) acc[e] = 0.f;
+        for (int e = 0; e < 4; ++e) acc[e] = 0.f;
     }
     // Four slots, of which the first `on` exist (the others hold leftovers).
-    __device__ __forceinline__ void take4(const float (&m_in)[4], const float (&l)[4], const f32x4 (&po)[4][COLS / 4], int on) {
+    __device__ __forceinline__ void take4(const float (&m_in)[4], const float (&l)[4], const f32x4 (&po)[4], int on) {
         float m[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) m[i] = i < on ? m_in[i] : kMinusBig;
@@ -181,16 +184,14 @@ template <int COLS> struct Fold {
         const float keep = __builtin_amdgcn_exp2f(M - Mn);
         L *= keep;
 #pragma unroll
-        for (int e = 0; e < COLS; ++e) acc[e] *= keep;
+        for (int e = 0; e < 4; ++e) acc[e] *= keep;
         M = Mn;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float w = i < on ? __builtin_amdgcn_exp2f(m[i] - M) : 0.f;
-            L = i < on ? __builtin_fmaf(w, l[i], L) : L;                   // (explicit: both users of this fold give the same bits)
+            L = i < on ? __builtin_fmaf(w, l[i], L) : L;                   // (explicit: a contraction that the compiler picked could differ from the merge's)
 #pragma unroll
-            for (int k = 0; k < COLS / 4; ++k)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) acc[4 * k + e] = i < on ? __builtin_fmaf(w, po[i][k][e], acc[4 * k + e]) : acc[4 * k + e];
+            for (int e = 0; e < 4; ++e) acc[e] = i < on ? __builtin_fmaf(w, po[i][e], acc[e]) : acc[e];
         }
     }
     __device__ __forceinline__ float inverse() const { return L > 0.f ? 1.0f / L : 0.f; }   // no valid key at all (every page id invalid): zeros, like a context of 0
@@ -546,8 +547,8 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
     }
     const int64_t sequence_floats = (int64_t)P.num_q_heads * P.nqt * P.nsplit * kQTile * kHeadDim;       // (below 2^31 bytes: the launch)
     const __amdgpu_buffer_rsrc_t of_sequence =
-        __builtin_amdgcn_make_buffer_rsrc(P.part_o + __builtin_amdgcn_readfirstlane(b) * sequence_floats, 0, (int)(sequence_floats * 4), 0x27000);
-    // the arithmetic of Fold::take4, split by split in groups of four, whoever is last: the bits of the combine kernel
+        __builtin_amdgcn_make_buffer_rsrc(P.part_o + __builtin_amdgcn_readfirstlane(b) * sequence_floats, 0, (int)(sequence_floats * 4), kRawBuffer);
+    // the operations of Fold::take4 in its order, split by split in groups of four, whoever is last: the bits of the combine kernel (change both or neither)
     float M = kMinusBig, L = 0.f;
     f32x4 acc[kMine][4];
 #pragma unroll
@@ -619,18 +620,18 @@ __global__ __launch_bounds__(32 * ROWS) void paged_combine_kernel(const PagedPar
     const float* part_o = P.part_o + (slot0 * kQTile + s) * kHeadDim + c;
     const float2* part_ml = reinterpret_cast<const float2*>(P.part_ml) + slot0 * kQTile + s;
     int nv = P.nsplit;                         // until the lengths are in: every slot that exists
-    Fold<4> F;
+    Fold F;
     F.init();
     for (int i0 = 0; i0 < nv; i0 += AHEAD) {
         float m[AHEAD / 4][4], l[AHEAD / 4][4];
-        f32x4 po[AHEAD / 4][4][1];
+        f32x4 po[AHEAD / 4][4];
 #pragma unroll
         for (int i = 0; i < AHEAD; ++i) {
             const int slot = min(i0 + i, P.nsplit - 1);
             const float2 ml = part_ml[slot * kQTile];
             m[i / 4][i % 4] = ml.x;
             l[i / 4][i % 4] = ml.y;
-            po[i / 4][i % 4][0] = *reinterpret_cast<const f32x4*>(part_o + (int64_t)slot * kQTile * kHeadDim);
+            po[i / 4][i % 4] = *reinterpret_cast<const f32x4*>(part_o + (int64_t)slot * kQTile * kHeadDim);
         }
         if (i0 == 0) {
             const int ctx = min(P.context_lens[b], P.max_pages * P.page_size);

@@ -326,7 +326,7 @@ N_STOP = 4                              # stop-token ids per sequence that the d
 # rows of a pass from which, and up to which, the fused vocabulary head is taken.  Fused / library product + vocabulary pass, us: 192 rows 181 / 199, 256 195 / 220,
 # 272 258 / 244, 320 258 / 255, 352 263 / 275, 383 262 / 277, 512 305 / 342
 FUSED_HEAD_MIN_ROWS, FUSED_HEAD_FEW_ROWS = 384, 256
-FUSED_HEAD_WHOLE_ROWS = 32              # rows that it holds whole (8 rows 120 us, 32 rows 119); compacting takes six launches of a pass, 66.4 against 65.5 ms for one request
+FUSED_HEAD_WHOLE_ROWS = 32              # rows that it holds whole (8 rows 120 us, 32 rows 119); compacting takes six launches of a pass, 63.9 against 63.4 ms for one request
 
 
 class _PagesShort(Exception):
