@@ -324,6 +324,23 @@ int mdx_unmask_step(const void* logits, int64_t row_stride, int32_t dtype,
                     void* workspace, int64_t workspace_bytes, mdx_stream_t stream);
 
 /*
+ * mdx_unmask_step (or, seeded, mdx_unmask_step_gumbel) in ONE launch: the last workgroup of a sequence to finish merges its rows and
+ * selects; no workgroup waits for another.  Blocks of more than 64 positions, and calls without room for their counters, make
+ * the two launches of the other calls; same results bit for bit.
+ *
+ * counters: mdx_unmask_step_counter_bytes(bs, block_len) bytes of device memory, 4-byte aligned (or NULL), that MUST BE ZERO before the first call and
+ * are left zero by every call that completes; calls that may run at the same time (different streams) need counters of their own.
+ */
+int64_t mdx_unmask_step_counter_bytes(int32_t bs, int32_t block_len);
+int mdx_unmask_step_single_launch(const void* logits, int64_t row_stride, int32_t dtype,
+                                  const float* temperatures, const float* noise, int64_t noise_row_stride,
+                                  int32_t seeded, uint64_t seed, uint64_t offset, const int64_t* offset_dev,
+                                  int64_t* tokens, int64_t mask_token_id, float threshold, int32_t k,
+                                  int64_t* x0, float* x0_p, uint8_t* transfer, int32_t* count,
+                                  int32_t bs, int32_t block_len, int64_t vocab,
+                                  void* workspace, int64_t workspace_bytes, void* counters, int64_t counter_bytes, mdx_stream_t stream);
+
+/*
  * The same two calls with the Gumbel noise of Sampler.prepare (layers/sampler.py:15-16:
  * gumbel = -log(Exponential(1)), added to logits / T before the argmax) drawn inside the kernel
  * instead of read from a tensor.  The draw is a pure function of (seed, offset, row, column):
@@ -354,7 +371,8 @@ int mdx_unmask_step_gumbel(const void* logits, int64_t row_stride, int32_t dtype
 /*
  * mdx_unmask_step (or, seeded, mdx_unmask_step_gumbel) on blocks in host memory that the GPU reaches (pinned), for a caller that wants the blocks, the flags and the
  * counts: which positions are masked is read here, and only their rows are computed.  tokens must hold its values when the call is made and may be written by the
- * GPU until the stream is done.  The workspace (16-byte aligned) holds the confidences as well.
+ * GPU until the stream is done.  The workspace (16-byte aligned) holds the confidences as well.  _single_launch: with counters as in
+ * mdx_unmask_step_single_launch; a call with a sequence that has nothing masked makes two launches.
  */
 int64_t mdx_unmask_step_host_blocks_workspace_bytes(int64_t rows, int64_t vocab);
 int mdx_unmask_step_host_blocks(const void* logits, int64_t row_stride, int32_t dtype,
@@ -363,6 +381,12 @@ int mdx_unmask_step_host_blocks(const void* logits, int64_t row_stride, int32_t 
                                 int64_t* tokens, int64_t mask_token_id, float threshold, int32_t k,
                                 uint8_t* transfer, int32_t* count, int32_t bs, int32_t block_len, int64_t vocab,
                                 void* workspace, int64_t workspace_bytes, mdx_stream_t stream);
+int mdx_unmask_step_host_blocks_single_launch(const void* logits, int64_t row_stride, int32_t dtype,
+                                              const float* temperatures, const float* noise, int64_t noise_row_stride,
+                                              int32_t seeded, uint64_t seed, uint64_t offset, const int64_t* offset_dev,
+                                              int64_t* tokens, int64_t mask_token_id, float threshold, int32_t k,
+                                              uint8_t* transfer, int32_t* count, int32_t bs, int32_t block_len, int64_t vocab,
+                                              void* workspace, int64_t workspace_bytes, void* counters, int64_t counter_bytes, mdx_stream_t stream);
 int mdx_gumbel_noise(float* noise, int64_t noise_row_stride, int64_t rows, int64_t vocab,
                      uint64_t seed, uint64_t offset, const int64_t* offset_dev, const int64_t* row_ids,
                      mdx_stream_t stream);

@@ -532,7 +532,7 @@ PyObject* sparse_attn_varlen(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // ---- paged decode -----------------------------------------------------------------------------------
-// The arrival counters of mdx_paged_block_attn_single_launch that this module keeps: two buffers per device and
+// The arrival counters of mdx_paged_block_attn_single_launch and of the unmask step that this module keeps: two buffers per device and
 // stream, zero when created, left zero by every launch.  Eager launches on one stream run one after the other, so they can
 // share one; a HIP graph keeps using the buffer that it was captured with wherever and beside whatever it is replayed, which
 // is why captured calls have the other one, and why a buffer, once handed out, is never replaced or freed: it has its full size from the
@@ -550,6 +550,7 @@ KeptCounters kept_counters_of(const Tensor& like, bool create) {
     static auto* kept = new std::map<std::pair<int, void*>, KeptCounters>();      // (never destroyed: the driver may be gone at exit)
     static std::mutex lock;
     const std::pair<int, void*> key{like.device().index(), stream_of(like)};
+    if (key.second == static_cast<void*>(hipStreamPerThread)) return {};          // (one handle for as many streams as there are threads)
     std::lock_guard<std::mutex> guard(lock);
     auto it = kept->find(key);
     if (it != kept->end()) return it->second;
@@ -562,6 +563,9 @@ Tensor counters_for(const Tensor& like, int64_t bytes, bool captured) {
     const KeptCounters kept = kept_counters_of(like, !captured);
     return captured ? kept.captured : kept.eager;
 }
+
+// The kept counters of calls that can do without: eager ones only.
+Tensor eager_counters(const Tensor& like, int64_t bytes) { return capturing(like) ? Tensor() : counters_for(like, bytes, false); }
 
 // a tensor of the device -> the counters kept for the current stream (eager calls', captured calls'), or None
 PyObject* kept_counters(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -850,14 +854,11 @@ void step(const Tensor& logits, int64_t bs, int64_t S, int64_t* tokens, int64_t 
     }
     const int64_t bytes = mdx_confidence_argmax_workspace_bytes(l.rows, l.vocab);
     const Tensor ws = bytes > 0 ? make(logits, at::kByte, bytes) : Tensor();
-    const float* tp = static_cast<const float*>(ptr_or_null(t));
-    if (z.seeded)
-        check(mdx_unmask_step_gumbel(ptr(l.t), l.stride, dtype_of(logits), tp, z.seed, z.offset, static_cast<const int64_t*>(ptr_or_null(z.offset_dev)),
-                                     nullptr, tokens, mask_id, threshold, k, x0, x0_p, transfer, count, (int32_t)bs, (int32_t)S, l.vocab,
-                                     ptr_or_null(ws), bytes, stream_of(logits)), "unmask_step");
-    else
-        check(mdx_unmask_step(ptr(l.t), l.stride, dtype_of(logits), tp, z.data(), z.data() ? l.vocab : 0, tokens, mask_id, threshold, k, x0, x0_p,
-                              transfer, count, (int32_t)bs, (int32_t)S, l.vocab, ptr_or_null(ws), bytes, stream_of(logits)), "unmask_step");
+    const Tensor counters = eager_counters(logits, mdx_unmask_step_counter_bytes((int32_t)bs, (int32_t)S));
+    check(mdx_unmask_step_single_launch(ptr(l.t), l.stride, dtype_of(logits), static_cast<const float*>(ptr_or_null(t)), z.data(), z.data() ? l.vocab : 0,
+                                        z.seeded ? 1 : 0, z.seed, z.offset, static_cast<const int64_t*>(ptr_or_null(z.offset_dev)), tokens, mask_id,
+                                        threshold, k, x0, x0_p, transfer, count, (int32_t)bs, (int32_t)S, l.vocab, ptr_or_null(ws), bytes,
+                                        ptr_or_null(counters), counters.defined() ? counters.nbytes() : 0, stream_of(logits)), "unmask_step");
 }
 
 // logits, tokens, mask_token_id, threshold, k, temperatures | None, top_k, top_p, noise (5: see noise_of) -> x0, x0_p, transfer, count
@@ -912,11 +913,12 @@ PyObject* sampler_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (t.defined()) NEED(t.numel() == bs);
         const int64_t ws_bytes = mdx_unmask_step_host_blocks_workspace_bytes(l.rows, l.vocab);
         const Tensor ws = make(logits, at::kByte, ws_bytes);
-        check(mdx_unmask_step_host_blocks(ptr(l.t), l.stride, dtype_of(logits), static_cast<const float*>(ptr_or_null(t)), z.data(), z.data() ? l.vocab : 0,
+        const Tensor counters = eager_counters(logits, mdx_unmask_step_counter_bytes((int32_t)bs, (int32_t)S));
+        check(mdx_unmask_step_host_blocks_single_launch(ptr(l.t), l.stride, dtype_of(logits), static_cast<const float*>(ptr_or_null(t)), z.data(), z.data() ? l.vocab : 0,
                                           z.seeded ? 1 : 0, z.seed, z.offset, static_cast<const int64_t*>(ptr_or_null(z.offset_dev)),
                                           reinterpret_cast<int64_t*>(host), to_int(a[5]), (float)real(a[6]), (int32_t)to_int(a[7]),
                                           reinterpret_cast<uint8_t*>(host + flags_at), reinterpret_cast<int32_t*>(host + counts_at), (int32_t)bs, (int32_t)S, l.vocab,
-                                          ptr(ws), ws_bytes, stream_of(logits)), "unmask_step");
+                                          ptr(ws), ws_bytes, ptr_or_null(counters), counters.defined() ? counters.nbytes() : 0, stream_of(logits)), "unmask_step");
         hipError_t rc;
         Py_BEGIN_ALLOW_THREADS
         rc = hipStreamSynchronize(static_cast<hipStream_t>(stream_of(logits)));

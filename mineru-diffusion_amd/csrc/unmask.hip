@@ -145,6 +145,44 @@ __device__ __forceinline__ void visit(Partial& p, float x, int index, float c, f
     }
 }
 
+// What the selection needs.  `arrive`: null, or an arrival counter per sequence, zero between launches, and the vocabulary pass selects
+// by itself (select_when_last).  (Arrivals at one cache line take about 3 ns each, one behind the other: with the counters next to each other,
+// 8 sequences of 9 splits took 26 us instead of 18.)
+constexpr int kCounterWords = 64;                            // from one counter to the next
+struct Selection {
+    uint32_t* arrive;
+    int64_t* tokens; int64_t mask_token_id; float threshold; int k;
+    uint8_t* transfer; int32_t* count; int block_len, lanes;
+};
+
+// The rule for a block of up to 64 positions, by ONE wavefront: lane p owns position p, counts are ballots, and the rank among the masked positions
+// comes from reading every lane's confidence in turn -- no LDS, no atomics, no barrier.
+__device__ __forceinline__ void select_by_wave(const Selection& S, int b, int p, bool masked, int64_t pick, float pick_p)
+{
+    const bool on = p < S.block_len;
+    const int64_t at = (int64_t)b * S.block_len + p;
+    const float conf = masked ? pick_p : -INFINITY;
+    const bool hi = conf > S.threshold;
+    bool commit;
+    if (__popcll(__ballot(hi)) >= S.k) {
+        commit = hi;
+    } else {
+        // rank among masked positions: higher confidence first, lower position first on ties
+        int rank = 0;
+        for (int j = 0; j < S.block_len; ++j) {
+            const float cj = __shfl(conf, j);
+            rank += (cj > conf || (cj == conf && j < p)) ? 1 : 0;
+        }
+        commit = masked && rank < S.k && conf > -INFINITY;   // at most min(k, #masked) positions; a confidence of -inf is never committed
+    }
+    const int n_commit = __popcll(__ballot(commit));
+    if (on) {
+        S.transfer[at] = commit ? 1 : 0;
+        if (commit) S.tokens[at] = pick;
+    }
+    if (p == 0) S.count[b] = n_commit;
+}
+
 // The rows that a call asks for, where it does not want all: a kernel's first argument, so that a workgroup's row is one scalar load away.
 constexpr int kMaxLiveRows = 1024;
 struct LiveRows { uint16_t row[kMaxLiveRows]; };
@@ -154,11 +192,130 @@ __device__ __forceinline__ int live_row(int i) {
     return (int)(i & 1 ? two >> 16 : two & 0xffff);
 }
 
+// Between workgroups of one launch: stores that are written through to memory and loads that take no line that this XCD's L2 may still hold.
+template <typename T> __device__ __forceinline__ void put_agent(T* p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+template <typename T> __device__ __forceinline__ T get_agent(const T* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ void store_agent(Partial* to, const Partial& p) {
+    put_agent(&to->m, p.m); put_agent(&to->s, p.s); put_agent(&to->idx, p.idx);
+    put_agent(&to->pick, p.pick); put_agent(&to->pick_x, p.pick_x); put_agent(&to->pick_idx, p.pick_idx);
+}
+template <bool NOISE> __device__ __forceinline__ Partial load_agent(const Partial* from) {
+    return Partial{get_agent(&from->m), get_agent(&from->s), get_agent(&from->idx), NOISE ? get_agent(&from->pick) : kNegBig,
+                   NOISE ? get_agent(&from->pick_x) : 0.f, NOISE ? get_agent(&from->pick_idx) : kNoIndex};
+}
+
+// A row's splits merged by a group of lanes: each takes every lanes-th, then the exchanges.  (One lane per row walking
+// the splits was a chain of dependent trips to memory: 6.2 us for nine splits, a third of what 96 sampled rows take.  Two or
+// three splits are walked all the same: a selection launch of 16 lanes per position takes 0.4 us longer than one of one.)
+constexpr int kMergeLanes = 16;                // at most
+int merge_lanes(int nsplit) { return nsplit <= 3 ? 1 : nsplit <= 8 ? 4 : kMergeLanes; }
+template <bool NOISE> __device__ __forceinline__ Partial merge_lanes_of(Partial r, int lanes, float c) {
+    for (int off = lanes / 2; off >= 1; off >>= 1) combine(r, shfl_xor(r, off, NOISE), c, NOISE);
+    return r;
+}
+template <bool NOISE>
+__device__ __forceinline__ Partial merge_splits(const Partial* __restrict__ partials, int nsplit, int lane, int lanes, float c) {
+    Partial r;
+    r.m = kNegBig; r.s = 0.f; r.idx = kNoIndex; r.pick = kNegBig; r.pick_x = 0.f; r.pick_idx = kNoIndex;
+    for (int s = lane; s < nsplit; s += lanes) combine(r, partials[s], c, NOISE);
+    return merge_lanes_of<NOISE>(r, lanes, c);
+}
+
+// The end of a workgroup of the vocabulary pass that selects by itself: the last one of a sequence to arrive merges its rows' splits and applies
+// the rule.  No workgroup waits for another; what the last one reads of the others was in memory before they arrived.  own: in thread 0, what the workgroup has found.
+// Three trips to memory (store, arrival, merge) take the GPU about as long as a second launch does, and the host 3.5 us less.  The step, us, two launches / one: 1 sequence
+// 15.7 / 13.4, 3 15.7 / 14.5, 5 16.6 / 15.8, 8 19.1 / 18.3, 16 30.0 / 29.5, 32 51.6 / 50.9; sampled, where the pass itself takes longer than the host, 3 25.6 / 25.6, 32 112.0 / 111.8.
+// (A counter per row as well, and a merge per row, was a trip more: 5 sequences 16.2, 8 18.6.)
+template <bool NOISE, bool LIVE>
+__device__ __forceinline__ void select_when_last(const Selection& S, const Partial& own, int row, int split, float c, int nsplit, Partial* partials, int64_t* x0, float* x0_p)
+{
+    __shared__ bool last;
+    __shared__ float conf_s[mdx::kWave];
+    __shared__ int pick_s[mdx::kWave];
+    const int tid = threadIdx.x, b = row / S.block_len;
+    const int64_t first = (int64_t)b * S.block_len;
+    uint32_t* const counter = S.arrive + (int64_t)b * kCounterWords;
+    bool masked = false;
+    if (tid < mdx::kWave) {
+        if (tid == 0) {
+            if (nsplit > 1) {
+                store_agent(partials + (int64_t)row * nsplit + split, own);
+            } else {
+                int64_t tok; float conf;
+                finish_row<NOISE>(own, c, tok, conf);
+                put_agent(x0 + row, tok);
+                put_agent(x0_p + row, conf);
+            }
+        }
+        int rows = S.block_len;
+        if (LIVE) {                          // (the list is in order, and a sequence has at most 64 rows)
+            unsigned long long asked = 0;
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const int e = (int)blockIdx.x - (mdx::kWave - 1) + k * mdx::kWave + tid;
+                const int other = e >= 0 && e < (int)gridDim.x ? live_row(e) - (int)first : -1;
+                if (other >= 0 && other < S.block_len) asked |= 1ull << other;
+            }
+#pragma unroll
+            for (int off = 32; off >= 1; off >>= 1) asked |= __shfl_xor(asked, off);
+            masked = (asked >> tid) & 1;
+            rows = __popcll(asked);
+        } else if (tid < S.block_len) {
+            masked = S.tokens[first + tid] == S.mask_token_id;
+        }
+        if (tid == 0) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(rows * nsplit - 1);
+        }
+    }
+    __syncthreads();
+    if (!last) return;
+    if (nsplit > 1) {
+        // (rows that a call does not ask for: whatever is there, of positions that are in no race)
+        const int lane = tid & (S.lanes - 1), step = kThreads / S.lanes;
+        for (int p = tid / S.lanes; p < S.block_len; p += 2 * step) {
+            Partial r[2];                    // both on their way together
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+                if (p + k * step < S.block_len && lane < nsplit) r[k] = load_agent<NOISE>(partials + (first + p + k * step) * nsplit + lane);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const int64_t at = first + p + k * step;
+                if (p + k * step >= S.block_len) break;      // (whole groups)
+                Partial sum;
+                sum.m = kNegBig; sum.s = 0.f; sum.idx = kNoIndex; sum.pick = kNegBig; sum.pick_x = 0.f; sum.pick_idx = kNoIndex;
+                if (lane < nsplit) combine(sum, r[k], c, NOISE);
+                for (int sp = lane + S.lanes; sp < nsplit; sp += S.lanes) combine(sum, load_agent<NOISE>(partials + at * nsplit + sp), c, NOISE);
+                sum = merge_lanes_of<NOISE>(sum, S.lanes, c);
+                if (lane == 0) {
+                    int64_t tok; float conf;
+                    finish_row<NOISE>(sum, c, tok, conf);
+                    x0[at] = tok;
+                    x0_p[at] = conf;
+                    pick_s[p + k * step] = (int)tok;
+                    conf_s[p + k * step] = conf;
+                }
+            }
+        }
+        __syncthreads();
+    }
+    if (tid >= mdx::kWave) return;
+    int64_t pick = 0;
+    float pick_p = 0.f;
+    if (masked) {
+        pick = nsplit > 1 ? pick_s[tid] : get_agent(x0 + first + tid);
+        pick_p = nsplit > 1 ? conf_s[tid] : get_agent(x0_p + first + tid);
+    }
+    select_by_wave(S, b, tid, masked, pick, pick_p);
+    if (tid == 0) put_agent(counter, 0u);                    // ready for the next launch
+}
+
 // grid = (rows, nsplit).  Each workgroup reduces chunks [split*cps, (split+1)*cps)
 // of one row; split 0 also takes the unaligned head and tail elements.
 // NOISE: 0 = plain argmax, 1 = noise read from a tensor, 2 = noise drawn in the kernel.
 // FLOOR: elements below floors[row] count as -inf (what a top-k / top-p filter would have left of the row).
 // LIVE: none, or LiveRows: only those rows.
+// With S.arrive the launch selects as well.
 template <typename T, int NOISE, bool FLOOR, typename... LIVE>
 __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
     const LIVE... live, const T* __restrict__ logits, int64_t row_stride,
@@ -166,7 +323,7 @@ __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
     const NoiseSpec N, const float* __restrict__ floors,
     int64_t vocab, int nsplit,
     Partial* __restrict__ partials,          // [rows, nsplit] when nsplit > 1
-    int64_t* __restrict__ x0, float* __restrict__ x0_p)
+    int64_t* __restrict__ x0, float* __restrict__ x0_p, const Selection S)
 {
     constexpr int EPC = Elem<T>::EPC;
     // (without LIVE from an unsigned number: from a signed one the compiler forms other code, and the step of 8 sequences takes 19.8 instead of 19.3 us, the
@@ -428,33 +585,21 @@ __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
     __shared__ Partial wave_part[kThreads / mdx::kWave];
     if ((tid & (mdx::kWave - 1)) == 0) wave_part[tid / mdx::kWave] = p;
     __syncthreads();
+    Partial r = wave_part[0];
     if (tid == 0) {
-        Partial r = wave_part[0];
 #pragma unroll
         for (int w = 1; w < kThreads / mdx::kWave; ++w) combine(r, wave_part[w], c, NOISE != 0);
-        if (nsplit > 1) {
-            partials[row * nsplit + split] = r;
-        } else {
-            int64_t tok; float conf;
-            finish_row<(NOISE != 0)>(r, c, tok, conf);
-            x0[row] = tok;
-            x0_p[row] = conf;
-        }
     }
-}
-
-// A row's splits merged by a group of lanes: each takes every lanes-th, then the exchanges.  (One lane per row walking
-// the splits was a chain of dependent trips to memory: 6.2 us for nine splits, a third of what 96 sampled rows take.  Two or
-// three splits are walked all the same: a selection launch of 16 lanes per position takes 0.4 us longer than one of one.)
-constexpr int kMergeLanes = 16;                // at most
-int merge_lanes(int nsplit) { return nsplit <= 3 ? 1 : nsplit <= 8 ? 4 : kMergeLanes; }
-template <bool NOISE>
-__device__ __forceinline__ Partial merge_splits(const Partial* __restrict__ partials, int nsplit, int lane, int lanes, float c) {
-    Partial r;
-    r.m = kNegBig; r.s = 0.f; r.idx = kNoIndex; r.pick = kNegBig; r.pick_x = 0.f; r.pick_idx = kNoIndex;
-    for (int s = lane; s < nsplit; s += lanes) combine(r, partials[s], c, NOISE);
-    for (int off = lanes / 2; off >= 1; off >>= 1) combine(r, shfl_xor(r, off, NOISE), c, NOISE);
-    return r;
+    if (S.arrive) { select_when_last<(NOISE != 0), (sizeof...(LIVE) > 0)>(S, r, (int)row32, split, c, nsplit, partials, x0, x0_p); return; }
+    if (tid != 0) return;
+    if (nsplit > 1) {
+        partials[row * nsplit + split] = r;
+    } else {
+        int64_t tok; float conf;
+        finish_row<(NOISE != 0)>(r, c, tok, conf);
+        x0[row] = tok;
+        x0_p[row] = conf;
+    }
 }
 
 template <bool NOISE>
@@ -562,55 +707,31 @@ __global__ __launch_bounds__(kMaxBlockLen) void select_transfer_kernel(
 }
 
 // The same rule for blocks of up to 64 positions (the engine's blocks hold 32) with ONE wavefront per
-// sequence: lane p owns position p, counts are ballots, and the rank among the masked positions comes
-// from reading every lane's confidence in turn -- no LDS, no atomics, no barrier, so the launch costs
-// little more than its one round trip to memory.  Where the row splits have to be merged first, the sequence gets
-// more lanes per position for that, and its first wavefront goes on alone.
+// sequence (select_by_wave), so that the launch costs little more than its one round trip to memory.  Where the row splits have to be merged first,
+// the sequence gets more lanes per position for that, and its first wavefront goes on alone.
 template <int SOURCE>
 __global__ __launch_bounds__(kMaxSelectThreads) void select_transfer_wave_kernel(
-    int64_t* __restrict__ x0, float* __restrict__ x0_p, int64_t* __restrict__ tokens,
-    const Partial* __restrict__ partials, int nsplit, const float* __restrict__ temperatures,
-    int64_t mask_token_id, float threshold, int k,
-    uint8_t* __restrict__ transfer, int32_t* __restrict__ count, int block_len, int lanes)
+    int64_t* __restrict__ x0, float* __restrict__ x0_p, const Partial* __restrict__ partials, int nsplit, const float* __restrict__ temperatures,
+    const Selection S)
 {
     __shared__ float conf_s[SOURCE == kFromRows ? 1 : mdx::kWave];
     __shared__ int pick_s[SOURCE == kFromRows ? 1 : mdx::kWave];
     const int b = blockIdx.x;
     const int p = threadIdx.x;
-    const bool on = p < block_len;
-    const int64_t at = (int64_t)b * block_len + p;
+    const bool on = p < S.block_len;
+    const int64_t at = (int64_t)b * S.block_len + p;
     int64_t pick = 0;
     float pick_p = 0.f;
-    const int64_t tok = on ? tokens[at] : 0;
+    const int64_t tok = on ? S.tokens[at] : 0;
     if (SOURCE != kFromRows) {
-        gather_block<SOURCE>(conf_s, pick_s, x0, x0_p, partials, nsplit, temperatures, b, block_len, lanes);
+        gather_block<SOURCE>(conf_s, pick_s, x0, x0_p, partials, nsplit, temperatures, b, S.block_len, S.lanes);
         if (p >= mdx::kWave) return;
         if (on) { pick = pick_s[p]; pick_p = conf_s[p]; }
     } else if (on) {
         pick = x0[at];
         pick_p = x0_p[at];
     }
-    const bool masked = on && tok == mask_token_id;
-    const float conf = masked ? pick_p : -INFINITY;
-    const bool hi = conf > threshold;
-    bool commit;
-    if (__popcll(__ballot(hi)) >= k) {
-        commit = hi;
-    } else {
-        // rank among masked positions: higher confidence first, lower position first on ties
-        int rank = 0;
-        for (int j = 0; j < block_len; ++j) {
-            const float cj = __shfl(conf, j);
-            rank += (cj > conf || (cj == conf && j < p)) ? 1 : 0;
-        }
-        commit = masked && rank < k && conf > -INFINITY;     // at most min(k, #masked) positions; a confidence of -inf is never committed
-    }
-    const int n_commit = __popcll(__ballot(commit));
-    if (on) {
-        transfer[at] = commit ? 1 : 0;
-        if (commit) tokens[at] = pick;
-    }
-    if (p == 0) count[b] = n_commit;
+    select_by_wave(S, b, p, on && tok == S.mask_token_id, pick, pick_p);
 }
 
 int launch_select(int64_t* x0, float* x0_p, int64_t* tokens, const Partial* partials, int nsplit, bool noisy, const float* temperatures,
@@ -623,13 +744,14 @@ int launch_select(int64_t* x0, float* x0_p, int64_t* tokens, const Partial* part
     const int lanes = merge_lanes(nsplit), wanted = (block_len * lanes + mdx::kWave - 1) / mdx::kWave * mdx::kWave;
     const int merging = wanted < kMaxSelectThreads ? wanted : kMaxSelectThreads;
     const unsigned threads = source == kFromRows ? whole_waves : (merging > whole_waves ? merging : whole_waves);
+    if (block_len <= mdx::kWave) {
+        const Selection S{nullptr, tokens, mask_token_id, threshold, k, transfer, count, block_len, lanes};
+        if (source == kFromRows)        select_transfer_wave_kernel<kFromRows><<<(unsigned)bs, threads, 0, stream>>>(x0, x0_p, partials, nsplit, temperatures, S);
+        else if (source == kFromSplits) select_transfer_wave_kernel<kFromSplits><<<(unsigned)bs, threads, 0, stream>>>(x0, x0_p, partials, nsplit, temperatures, S);
+        else                            select_transfer_wave_kernel<kFromNoisySplits><<<(unsigned)bs, threads, 0, stream>>>(x0, x0_p, partials, nsplit, temperatures, S);
+    } else {
 #define MDX_SELECT(KERNEL, SOURCE) KERNEL<SOURCE><<<(unsigned)bs, threads, 0, stream>>>( \
         x0, x0_p, tokens, partials, nsplit, temperatures, mask_token_id, threshold, k, transfer, count, block_len, lanes)
-    if (block_len <= mdx::kWave) {
-        if (source == kFromRows)        MDX_SELECT(select_transfer_wave_kernel, kFromRows);
-        else if (source == kFromSplits) MDX_SELECT(select_transfer_wave_kernel, kFromSplits);
-        else                            MDX_SELECT(select_transfer_wave_kernel, kFromNoisySplits);
-    } else {
         if (source == kFromRows)        MDX_SELECT(select_transfer_kernel, kFromRows);
         else if (source == kFromSplits) MDX_SELECT(select_transfer_kernel, kFromSplits);
         else                            MDX_SELECT(select_transfer_kernel, kFromNoisySplits);
@@ -670,14 +792,14 @@ int pick_nsplit_sampled(int64_t rows, int64_t vocab) {
 template <typename T, bool FLOOR>
 int launch_confidence(const void* logits, int64_t row_stride, const float* temperatures, int rows_per_temp,
                       const NoiseSpec& N, const float* floors, int64_t* x0, float* x0_p,
-                      int64_t rows, int64_t vocab, int nsplit, Partial* partials, bool finalize, const LiveRows* live, hipStream_t stream)
+                      int64_t rows, int64_t vocab, int nsplit, Partial* partials, bool finalize, const LiveRows* live, const Selection& S, hipStream_t stream)
 {
     const dim3 grid((unsigned)rows, (unsigned)nsplit);
     const bool noisy = N.noise != nullptr || N.philox;
     if constexpr (!FLOOR) {
         if (live) {
 #define MDX_CONFIDENCE(NOISE) confidence_argmax_kernel<T, NOISE, false, LiveRows><<<grid, kThreads, 0, stream>>>( \
-        *live, (const T*)logits, row_stride, temperatures, rows_per_temp, N, floors, vocab, nsplit, partials, x0, x0_p)
+        *live, (const T*)logits, row_stride, temperatures, rows_per_temp, N, floors, vocab, nsplit, partials, x0, x0_p, S)
             if (N.philox)     MDX_CONFIDENCE(2);
             else if (N.noise) MDX_CONFIDENCE(1);
             else              MDX_CONFIDENCE(0);
@@ -686,7 +808,7 @@ int launch_confidence(const void* logits, int64_t row_stride, const float* tempe
         }
     }
 #define MDX_CONFIDENCE(NOISE) confidence_argmax_kernel<T, NOISE, FLOOR><<<grid, kThreads, 0, stream>>>( \
-        (const T*)logits, row_stride, temperatures, rows_per_temp, N, floors, vocab, nsplit, partials, x0, x0_p)
+        (const T*)logits, row_stride, temperatures, rows_per_temp, N, floors, vocab, nsplit, partials, x0, x0_p, S)
     if (N.philox)     MDX_CONFIDENCE(2);
     else if (N.noise) MDX_CONFIDENCE(1);
     else              MDX_CONFIDENCE(0);
@@ -731,7 +853,7 @@ int confidence_pass(const void* logits, int64_t row_stride, int32_t dtype,
                     const NoiseSpec& N, const float* floors,
                     int64_t* x0, float* x0_p, int64_t rows, int64_t vocab,
                     void* workspace, int64_t workspace_bytes, bool finalize, int* nsplit_out, hipStream_t stream,
-                    const LiveRows* live = nullptr, int n_live = 0)
+                    const LiveRows* live = nullptr, int n_live = 0, Selection* select = nullptr)
 {
     MDX_REQUIRE(rows >= 0 && vocab >= 0, MDX_EINVAL, "confidence_argmax: negative size");
     if (nsplit_out) *nsplit_out = 1;
@@ -753,7 +875,9 @@ int confidence_pass(const void* logits, int64_t row_stride, int32_t dtype,
     MDX_REQUIRE(need == 0 || (workspace && workspace_bytes >= need), MDX_EWORKSPACE,
                 "confidence_argmax: workspace of %lld bytes needed, %lld given", (long long)need, (long long)workspace_bytes);
     Partial* partials = static_cast<Partial*>(workspace);
-#define MDX_PASS(T, FLOOR) launch_confidence<T, FLOOR>(logits, row_stride, temperatures, rows_per_temp, N, floors, x0, x0_p, asked, vocab, nsplit, partials, finalize, live, stream)
+    Selection S{};
+    if (select) { S = *select; S.lanes = merge_lanes(nsplit); }
+#define MDX_PASS(T, FLOOR) launch_confidence<T, FLOOR>(logits, row_stride, temperatures, rows_per_temp, N, floors, x0, x0_p, asked, vocab, nsplit, partials, finalize, live, S, stream)
     switch (dtype) {
         case MDX_BF16: return floors ? MDX_PASS(__bf16, true) : MDX_PASS(__bf16, false);
         case MDX_F16:  return floors ? MDX_PASS(__half, true) : MDX_PASS(__half, false);
@@ -816,26 +940,35 @@ extern "C" int mdx_select_transfer(const int64_t* x0, const float* x0_p, int64_t
                          transfer, count, bs, block_len, stream);
 }
 
+extern "C" int64_t mdx_unmask_step_counter_bytes(int32_t bs, int32_t block_len)
+{
+    if (bs <= 0 || block_len <= 0) return 0;
+    return (int64_t)bs * kCounterWords * (int64_t)sizeof(uint32_t);
+}
+
 namespace {
 
 int unmask_step_impl(const void* logits, int64_t row_stride, int32_t dtype,
                      const float* temperatures, const NoiseSpec& N,
                      int64_t* tokens, int64_t mask_token_id, float threshold, int32_t k,
                      int64_t* x0, float* x0_p, uint8_t* transfer, int32_t* count,
-                     int32_t bs, int32_t block_len, int64_t vocab,
-                     void* workspace, int64_t workspace_bytes, hipStream_t stream, const LiveRows* live = nullptr, int n_live = 0)
+                     int32_t bs, int32_t block_len, int64_t vocab, void* workspace, int64_t workspace_bytes,
+                     void* counters, int64_t counter_bytes, hipStream_t stream, const LiveRows* live = nullptr, int n_live = 0)
 {
     MDX_REQUIRE(bs >= 0 && block_len >= 0, MDX_EINVAL, "unmask_step: negative size");
     MDX_REQUIRE(k >= 0, MDX_EINVAL, "unmask_step: k %d < 0", k);
     MDX_REQUIRE(block_len <= kMaxBlockLen, MDX_EUNSUPPORTED, "unmask_step: block_len %d > %d", block_len, kMaxBlockLen);
     if (bs == 0 || block_len == 0) return MDX_OK;
     MDX_REQUIRE(tokens && transfer && count, MDX_EINVAL, "unmask_step: null pointer");
-    // The selection kernel merges the row splits itself (one launch fewer).
+    // With counters the last workgroup of a sequence selects; otherwise the selection kernel merges the row splits itself (one launch fewer).
     const bool noisy = N.noise != nullptr || N.philox;
+    const bool single = counters && ((uintptr_t)counters & 3) == 0 && counter_bytes >= mdx_unmask_step_counter_bytes(bs, block_len) && block_len <= mdx::kWave && vocab > 0;
+    uint32_t* const arrive = static_cast<uint32_t*>(counters);
+    Selection S{arrive, tokens, mask_token_id, threshold, k, transfer, count, block_len, 1};
     int nsplit = 1;
-    int rc = confidence_pass(logits, row_stride, dtype, temperatures, block_len, N, nullptr,
-                             x0, x0_p, (int64_t)bs * block_len, vocab, workspace, workspace_bytes, false, &nsplit, stream, live, n_live);
-    if (rc != MDX_OK) return rc;
+    int rc = confidence_pass(logits, row_stride, dtype, temperatures, block_len, N, nullptr, x0, x0_p, (int64_t)bs * block_len, vocab,
+                             workspace, workspace_bytes, false, &nsplit, stream, live, n_live, single ? &S : nullptr);
+    if (rc != MDX_OK || single) return rc;
     // (rows that were not asked for: whatever was there, of positions that are not masked and so in no race)
     return launch_select(x0, x0_p, tokens, nsplit > 1 ? static_cast<const Partial*>(workspace) : nullptr, nsplit, noisy, temperatures,
                          mask_token_id, threshold, k, transfer, count, bs, block_len, stream);
@@ -903,7 +1036,7 @@ extern "C" int mdx_unmask_step(const void* logits, int64_t row_stride, int32_t d
                                void* workspace, int64_t workspace_bytes, mdx_stream_t stream)
 {
     return unmask_step_impl(logits, row_stride, dtype, temperatures, tensor_noise(noise, noise_row_stride), tokens, mask_token_id,
-                            threshold, k, x0, x0_p, transfer, count, bs, block_len, vocab, workspace, workspace_bytes,
+                            threshold, k, x0, x0_p, transfer, count, bs, block_len, vocab, workspace, workspace_bytes, nullptr, 0,
                             static_cast<hipStream_t>(stream));
 }
 
@@ -916,9 +1049,25 @@ extern "C" int mdx_unmask_step_gumbel(const void* logits, int64_t row_stride, in
                                       void* workspace, int64_t workspace_bytes, mdx_stream_t stream)
 {
     return unmask_step_impl(logits, row_stride, dtype, temperatures, generator_noise(seed, offset, offset_dev, row_ids), tokens,
-                            mask_token_id, threshold, k, x0, x0_p, transfer, count, bs, block_len, vocab, workspace, workspace_bytes,
+                            mask_token_id, threshold, k, x0, x0_p, transfer, count, bs, block_len, vocab, workspace, workspace_bytes, nullptr, 0,
                             static_cast<hipStream_t>(stream));
 }
+
+extern "C" int mdx_unmask_step_single_launch(const void* logits, int64_t row_stride, int32_t dtype,
+                                             const float* temperatures, const float* noise, int64_t noise_row_stride,
+                                             int32_t seeded, uint64_t seed, uint64_t offset, const int64_t* offset_dev,
+                                             int64_t* tokens, int64_t mask_token_id, float threshold, int32_t k,
+                                             int64_t* x0, float* x0_p, uint8_t* transfer, int32_t* count,
+                                             int32_t bs, int32_t block_len, int64_t vocab,
+                                             void* workspace, int64_t workspace_bytes, void* counters, int64_t counter_bytes, mdx_stream_t stream)
+{
+    MDX_REQUIRE(!(noise && seeded), MDX_EINVAL, "unmask_step: either a noise tensor or a seed");
+    const NoiseSpec N = seeded ? generator_noise(seed, offset, offset_dev, nullptr) : tensor_noise(noise, noise_row_stride);
+    return unmask_step_impl(logits, row_stride, dtype, temperatures, N, tokens, mask_token_id, threshold, k, x0, x0_p, transfer, count, bs, block_len,
+                            vocab, workspace, workspace_bytes, counters, counter_bytes, static_cast<hipStream_t>(stream));
+}
+
+constexpr int kSingleLaunchRows = 128;
 
 // What the step keeps in the caller's workspace: x0, x0_p, and the splits of as many rows as there are, by the most splits that fewer rows are cut into.
 namespace {
@@ -930,12 +1079,13 @@ extern "C" int64_t mdx_unmask_step_host_blocks_workspace_bytes(int64_t rows, int
     return rows <= 0 || vocab <= 0 ? 0 : confidences_bytes(rows) + rows * pick_nsplit(1, vocab) * (int64_t)sizeof(Partial);
 }
 
-extern "C" int mdx_unmask_step_host_blocks(const void* logits, int64_t row_stride, int32_t dtype,
-                                           const float* temperatures, const float* noise, int64_t noise_row_stride,
-                                           int32_t seeded, uint64_t seed, uint64_t offset, const int64_t* offset_dev,
-                                           int64_t* tokens, int64_t mask_token_id, float threshold, int32_t k,
-                                           uint8_t* transfer, int32_t* count, int32_t bs, int32_t block_len, int64_t vocab,
-                                           void* workspace, int64_t workspace_bytes, mdx_stream_t stream)
+extern "C" int mdx_unmask_step_host_blocks_single_launch(const void* logits, int64_t row_stride, int32_t dtype,
+                                                         const float* temperatures, const float* noise, int64_t noise_row_stride,
+                                                         int32_t seeded, uint64_t seed, uint64_t offset, const int64_t* offset_dev,
+                                                         int64_t* tokens, int64_t mask_token_id, float threshold, int32_t k,
+                                                         uint8_t* transfer, int32_t* count, int32_t bs, int32_t block_len, int64_t vocab,
+                                                         void* workspace, int64_t workspace_bytes, void* counters, int64_t counter_bytes,
+                                                         mdx_stream_t stream)
 {
     MDX_REQUIRE(bs >= 0 && block_len >= 0, MDX_EINVAL, "unmask_step: negative size");
     if (bs == 0 || block_len == 0) return MDX_OK;
@@ -947,15 +1097,34 @@ extern "C" int mdx_unmask_step_host_blocks(const void* logits, int64_t row_strid
     // The masked positions are known here, and no other row's confidence reaches a result: a row is 304 KB of reads and 150 000 draws.  The sampler's
     // call, us, all rows / masked rows (three quarters): sampled, 1 sequence 36.3 / 34.6, 3 43.4 / 40.0, 8 63.1 / 57.9, 24 118.4 / 106.2; plain, 3 30.4 / 28.2, 24 73.9 / 65.4.
     LiveRows live;
-    int n_live = 0;
+    int n_live = 0, with_rows = 0;                           // masked rows, and the sequences that have any
     if (rows <= kMaxLiveRows) {
-        for (int64_t i = 0; i < rows; ++i)
-            if (tokens[i] == mask_token_id) live.row[n_live++] = (uint16_t)i;
+        for (int32_t b = 0; b < bs; ++b) {
+            const int before = n_live;
+            for (int64_t i = (int64_t)b * block_len; i < (int64_t)(b + 1) * block_len; ++i)
+                if (tokens[i] == mask_token_id) live.row[n_live++] = (uint16_t)i;
+            with_rows += n_live > before;
+        }
+        // Nobody would select for the sequences without any; and a caller that waits for the result does not see what a launch costs the host, so that few
+        // rows are as quick in two (us, two launches / one: 32 rows 24.5 / 26, 96 40.8 / 41.0, 192 36.1 / 35.4, 576 63.1 / 62.7).
+        if (with_rows < bs || n_live < kSingleLaunchRows) counters = nullptr;
     }
     const NoiseSpec N = seeded ? generator_noise(seed, offset, offset_dev, nullptr) : tensor_noise(noise, noise_row_stride);
     int64_t* x0 = static_cast<int64_t*>(workspace);
     char* splits = static_cast<char*>(workspace) + confidences_bytes(rows);
     return unmask_step_impl(logits, row_stride, dtype, temperatures, N, tokens, mask_token_id, threshold, k, x0, reinterpret_cast<float*>(x0 + rows), transfer, count,
-                            bs, block_len, vocab, splits, workspace_bytes - confidences_bytes(rows), static_cast<hipStream_t>(stream),
+                            bs, block_len, vocab, splits, workspace_bytes - confidences_bytes(rows), counters, counter_bytes, static_cast<hipStream_t>(stream),
                             rows <= kMaxLiveRows && n_live < rows ? &live : nullptr, n_live);
+}
+
+extern "C" int mdx_unmask_step_host_blocks(const void* logits, int64_t row_stride, int32_t dtype,
+                                           const float* temperatures, const float* noise, int64_t noise_row_stride,
+                                           int32_t seeded, uint64_t seed, uint64_t offset, const int64_t* offset_dev,
+                                           int64_t* tokens, int64_t mask_token_id, float threshold, int32_t k,
+                                           uint8_t* transfer, int32_t* count, int32_t bs, int32_t block_len, int64_t vocab,
+                                           void* workspace, int64_t workspace_bytes, mdx_stream_t stream)
+{
+    return mdx_unmask_step_host_blocks_single_launch(logits, row_stride, dtype, temperatures, noise, noise_row_stride, seeded, seed, offset, offset_dev,
+                                                     tokens, mask_token_id, threshold, k, transfer, count, bs, block_len, vocab, workspace, workspace_bytes,
+                                                     nullptr, 0, stream);
 }

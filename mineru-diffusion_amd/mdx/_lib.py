@@ -46,6 +46,11 @@ SIGNATURES = {
                                          _I32, _I32, _I64, _P, _I64, _P]),
     "mdx_unmask_step_host_blocks_workspace_bytes": (c_int64, [_I64, _I64]),
     "mdx_unmask_step_host_blocks": (c_int32, [_P, _I64, _I32, _P, _P, _I64, _I32, _U64, _U64, _P, _P, _I64, _F, _I32, _P, _P, _I32, _I32, _I64, _P, _I64, _P]),
+    "mdx_unmask_step_host_blocks_single_launch": (c_int32, [_P, _I64, _I32, _P, _P, _I64, _I32, _U64, _U64, _P, _P, _I64, _F, _I32, _P, _P, _I32, _I32, _I64,
+                                                            _P, _I64, _P, _I64, _P]),
+    "mdx_unmask_step_counter_bytes": (c_int64, [_I32, _I32]),
+    "mdx_unmask_step_single_launch": (c_int32, [_P, _I64, _I32, _P, _P, _I64, _I32, _U64, _U64, _P, _P, _I64, _F, _I32, _P, _P, _P, _P, _I32, _I32, _I64,
+                                                _P, _I64, _P, _I64, _P]),
     "mdx_gumbel_noise": (c_int32, [_P, _I64, _I64, _I64, _U64, _U64, _P, _P, _P]),
     "mdx_select_transfer": (c_int32, [_P, _P, _P, _I64, _F, _I32, _P, _P, _I32, _I32, _P]),
     "mdx_qk_norm_rope_store": (c_int32, [_P, _I64, _P, _P, _F, _P, _P, _I64, _P, _P, _I64, _P, _I64, _P, _P, _P, _I64,
