@@ -177,16 +177,16 @@ constexpr TileCost tile(float step, float around) {
                          launch<BM, BN, WM, WN, WK, S, SX, kSilu>};
 }
 const TileCost kTiles[] = {
-    tile<32, 64, 2, 2, 1, 4, 4, true>(0.173f, 0.4f),
-    tile<64, 64, 2, 2, 2, 4, 4, true>(0.233f, 0.7f),
-    tile<128, 64, 2, 2, 2, 4, 4, true>(0.336f, 1.7f),
-    tile<192, 64, 2, 2, 2, 4, 4, true>(0.425f, 2.1f),
-    tile<128, 128, 2, 2, 2, 4, 4, true>(0.499f, 2.6f),
-    tile<192, 128, 2, 2, 2, 4, 4, true>(0.602f, 3.5f),
-    tile<128, 192, 4, 2, 1, 4, 4, true>(0.672f, 2.3f),
-    tile<192, 192, 4, 2, 1, 3, 3, false>(0.805f, 5.0f),
-    tile<256, 192, 4, 2, 1, 2, 3, false>(1.117f, 3.7f),
-    tile<256, 256, 4, 2, 1, 2, 3, false>(1.344f, 5.9f),
+    tile<32, 64, 2, 2, 1, 4, 4, true>(0.167f, 0.4f),
+    tile<64, 64, 2, 2, 2, 4, 4, true>(0.231f, 0.7f),
+    tile<128, 64, 2, 2, 2, 4, 4, true>(0.326f, 1.7f),
+    tile<192, 64, 2, 2, 2, 4, 4, true>(0.408f, 2.9f),
+    tile<128, 128, 2, 2, 2, 4, 4, true>(0.487f, 2.6f),
+    tile<192, 128, 2, 2, 2, 4, 4, true>(0.584f, 3.5f),
+    tile<128, 192, 4, 2, 1, 4, 4, true>(0.617f, 2.3f),
+    tile<192, 192, 4, 2, 1, 3, 3, false>(0.741f, 5.0f),
+    tile<256, 192, 4, 2, 1, 3, 2, false>(0.983f, 3.7f),
+    tile<256, 256, 4, 2, 1, 3, 2, false>(1.149f, 5.9f),
 };
 
 struct Plan { const TileCost* tile; int splits; double cost; };
@@ -225,7 +225,7 @@ HeadsPlan heads_plan(int64_t rows, int64_t n, int64_t k)
         const int64_t tiles = (rows + bm - 1) / bm * (n / mdx_qk::kHeadDim);
         return (float)((tiles + cus - 1) / cus) * ((float)(k / kStepK) * step + around);
     };
-    const float c64 = cost(64, 0.345f, 1.7f), c128 = cost(128, 0.499f, 2.6f), c192 = cost(192, 0.602f, 3.5f);
+    const float c64 = cost(64, 0.338f, 1.7f), c128 = cost(128, 0.487f, 2.6f), c192 = cost(192, 0.584f, 3.5f);
     if (c64 <= c128 && c64 <= c192) return {launch<64, 128, 2, 2, 2, 4, 4, kHeads>, c64};
     if (c128 <= c192) return {launch<128, 128, 2, 2, 2, 4, 4, kHeads>, c128};
     return {launch<192, 128, 2, 2, 2, 4, 4, kHeads>, c192};

@@ -7,10 +7,10 @@
 // (engines/nano_dvlm/nanovllm/layers/embed_head.py:61-67) followed by Sampler.prepare's softmax
 // confidence and argmax without noise (layers/sampler.py:11-22).
 //
-// A workgroup computes a tile of 256 x 256, 128 x 256 or 192 x 192 (x rows by vocabulary rows) over the whole hidden dimension
+// A workgroup computes a tile of 256 x 256 or 192 x 256 (x rows by vocabulary rows) over the whole hidden dimension
 // (linear_tile.h) and leaves one 16-byte record per x row; a second, small kernel folds a row's records (about vocab / 256 of them) into x0 /
-// x0_p.  What bounds it: the matrix pipe behind one barrier per step, at which all eight wavefronts wait for their LDS reads and loads; at 1024 rows the pipe is busy
-// 50.5 % of 1.205 M active cycles per SIMD (the generated core below: 56.4 % of 1.078 M, at a lower clock).
+// x0_p.  What bounds it: the matrix pipe under the board's power limit (at 1024 rows 522 us on data, 441 on zeros, whose clock
+// is higher, 380 without loads), 5 us of epilogue per tile, the last round of tiles (500 rows: 4.64 of 5).
 #include "lm_head.h"
 #include "linear_tile.h"
 
@@ -241,10 +241,10 @@ int launch_two_steps(LmHeadParams& P, hipStream_t stream)
     return mdx::check_launch("lm_head_confidence");
 }
 
-// Which tile: rounds of one workgroup per CU times what a round takes (us over 2048 columns: 256 x 256 56, 128 x 256 and 192 x 192
-// 34.5).  151 936 entries, us, 256 x 256 / 128 x 256 / 192 x 192: 129 rows 197 / 182 / 177, 192 192 / 188 / 184, 256 196 / 201 / 238,
-// 320 286 / 250 / 257, 500 300 / 348 / 345, 768 421 / 473 / 468.  The call, generated core / these tiles: 129 rows 212 / 187, 192 206 / 186,
-// 256 212 / 198, 320 296 / 261, 500 307 / 299, 640 438 / 412, 1024 577 / 567, 4096 2168 / 2092.
+// Which tile: rounds of one workgroup per CU times what a round takes (us over 2048 columns: 256 x 256 53.5, 192 x 256 44.5).  151 936 entries, the call, us,
+// 256 x 256 / 192 x 256: 136 rows 186 / 170, 192 188 / 172, 256 188 / 226, 300 270 / 230, 384 270 / 229, 512 274 / 312, 640 373 / 418, 768 383 / 421, 1024
+// 522 / 584.  (128 x 256: 183, 191, 194, 245, 246, 329, 388, 445, 599; 192 x 192: 175, 180, 243, 248, 253, 346, 437, 444, 620; 256 x 192 and 128 x 192 lie above
+// the better of the two everywhere.)  With loads and reads in bursts behind the barriers (linear_tile.h): 136 rows 181, 192 185, 256 198, 384 263, 512 304, 768 418, 1024 560.
 int launch_product(LmHeadParams& P, hipStream_t stream)
 {
     if (P.hidden < 3 * kStepK) return launch_two_steps(P, stream);
@@ -253,9 +253,7 @@ int launch_product(LmHeadParams& P, hipStream_t stream)
         const int64_t tiles = (int64_t)((P.rows + bm - 1) / bm) * ((P.vocab + bn - 1) / bn);
         return (float)((tiles + cus - 1) / cus) * round;
     };
-    const float large = cost(256, 256, 56.f), half = cost(128, 256, 34.5f), square = cost(192, 192, 34.5f);
-    if (half < large && half <= square) return launch_tiles<128, 256, 3, 3>(P, stream);
-    return square < large ? launch_tiles<192, 192, 3, 3>(P, stream) : launch_tiles<256, 256, 2, 3>(P, stream);
+    return cost(192, 256, 44.5f) < cost(256, 256, 53.5f) ? launch_tiles<192, 256, 3, 2>(P, stream) : launch_tiles<256, 256, 3, 2>(P, stream);
 }
 
 }  // namespace

@@ -1,0 +1,48 @@
+"""The tiles of the linear layers and the vocabulary head at the fewest steps of K and at their edges in rows and columns, on small integers: sums are
+exact in any order, so results are those of an fp32 product rounded once, bit for bit."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _integers(rows, n, k):
+    g = torch.Generator().manual_seed(rows * 7 + n + k)
+    return (torch.randint(-2, 3, (rows, k), generator=g).bfloat16(), torch.randint(-2, 3, (n, k), generator=g).bfloat16())
+
+
+@pytest.mark.parametrize("k", [256, 384, 640])
+@pytest.mark.parametrize("rows,n", [(33, 72), (129, 264), (192, 2056), (257, 4104), (577, 2056), (1025, 4104), (1120, 6152), (1536, 8200), (2049, 6152), (4100, 6152)])
+def test_products_at_few_steps(dev, rows, n, k):
+    import mdx
+    x, w = _integers(rows, n, k)
+    want = (x.to(dev).float() @ w.to(dev).float().T).bfloat16()
+    L, stream = mdx._lib.lib(), torch.cuda.current_stream().cuda_stream
+    x, w = x.to(dev), w.to(dev)
+    y = torch.full((rows, n + 4), 7.0, dtype=torch.bfloat16, device=dev)
+    assert L.mdx_linear(x.data_ptr(), k, w.data_ptr(), k, y.data_ptr(), n + 4, rows, n, k, stream) == 0
+    assert torch.equal(y[:, :n], want) and bool((y[:, n:] == 7.0).all())
+    half = n // 2 // 8 * 8
+    act = torch.full((rows, half + 4), 7.0, dtype=torch.bfloat16, device=dev)
+    assert L.mdx_linear_silu(x.data_ptr(), k, w.data_ptr(), k, act.data_ptr(), half + 4, rows, half, k, stream) == 0
+    gated = mdx.silu_and_mul(want[:, :2 * half].contiguous())
+    # the exponential of the two kernels is the same, the result one rounding to bf16 behind the same products
+    assert (act[:, :half].float() - gated.float()).abs().max() <= 2.0 ** -7 * gated.float().abs().max() and bool((act[:, half:] == 7.0).all())
+    splits = L.mdx_linear_splits(rows, n, k)
+    if splits > 0:
+        parts = torch.full((splits, rows, n), 7.0, device=dev)
+        assert L.mdx_linear_partials(x.data_ptr(), k, w.data_ptr(), k, parts.data_ptr(), rows, n, k, stream) == 0
+        assert torch.equal(parts.sum(0).bfloat16(), want)
+
+
+@pytest.mark.parametrize("rows,vocab,hidden", [(129, 511, 256), (192, 30000, 256), (193, 30001, 384), (256, 70000, 256), (384, 40003, 256), (385, 769, 512), (512, 70001, 256)])
+def test_head_at_few_steps(dev, rows, vocab, hidden):
+    import mdx
+    x, w = _integers(rows, vocab, hidden)
+    x, w = x.to(dev), w.to(dev)
+    x0, p = mdx.lm_head_confidence(x, w)
+    logits = (x.float() @ w.float().T).bfloat16()
+    tx0, tp = mdx.confidence_argmax(logits.unsqueeze(0))
+    assert torch.equal(x0, tx0.view(-1))
+    # two sums of the same fp32 terms: 2^-24 per addition and of each exponent's argument
+    assert torch.allclose(p, tp.view(-1), rtol=3e-5, atol=0)
