@@ -492,7 +492,7 @@ int mdx_silu_and_mul(const void* x, int64_t x_row_stride, void* out, int64_t out
  * round the sum to bf16 as the layer's output.  mdx_linear_splits(rows, n, k): the number of slices where that is the faster
  * of the two (mdx_linear is then slower than a library's product for long k and few columns), 0 where mdx_linear is, -1 where a library's product is the better choice (more than 1536 rows; wide layers from
  * 52 GFLOP on) or the shape is not covered.  mdx_linear_silu: w [2 n, k], gate rows then up rows; y [rows, n] = mdx_silu_and_mul of the product, with
- * its rounding points; mdx_linear_silu_supported: covered, and up to 8192 rows.
+ * its rounding points; mdx_linear_silu_supported: covered, and up to 8192 rows, or any number where n is at least 1024 and at least k.
  * mdx_linear_qk_norm_rope_store: the product of a QKV projection with mdx_qk_norm_rope_store on it in one launch; w holds the q
  * rows, then k, then v; k_out / v_out (the rotated k and the raw v, [rows, Hkv * d]) and the caches may be null;
  * covered: 384 to 1536 rows, d = 128; mdx_linear_qk_norm_rope_store_supported: and the faster of one launch and two.

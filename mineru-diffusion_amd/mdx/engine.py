@@ -12,7 +12,7 @@ kernels can be driven exactly as the engine drives them:
                                   layers/rotary_embedding.py:6-48, layers/embed_head.py:61-67
 
 The decoder is a random-init scaffold; attention, the KV store, the norms, the activation, the unmask step and the
-linear layers of up to 1536 rows (gate/up: 8192) go through libmdx, the other GEMMs are stock PyTorch (library) GEMMs.  Decode passes can
+linear layers of up to 1536 rows (gate/up: all) go through libmdx, the other GEMMs are stock PyTorch (library) GEMMs.  Decode passes can
 replay a captured HIP graph (model_runner.py:198-259).  There is no vision tower, tokenizer,
 weight loader or tensor parallelism here.
 """

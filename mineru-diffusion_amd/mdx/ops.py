@@ -72,7 +72,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, partials: bool = False) -> tor
 
 
 def linear_gated(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor | None:
-    """silu_and_mul(x . weight^T) for up to 8192 rows in one launch (nanovllm/models/sdar.py:105-111)."""
+    """silu_and_mul(x . weight^T) in one launch, beyond 8192 rows where weight has 2048 rows or more and twice as many as columns (nanovllm/models/sdar.py:105-111)."""
     return _host().linear_gated(x, weight)
 
 

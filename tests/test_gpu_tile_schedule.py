@@ -35,6 +35,19 @@ def test_products_at_few_steps(dev, rows, n, k):
         assert torch.equal(parts.sum(0).bfloat16(), want)
 
 
+@pytest.mark.parametrize("rows,n,k,taken", [(8193, 1024, 512, True), (8400, 2056, 640, True), (8193, 1016, 512, False), (8193, 1024, 1152, False)])
+def test_gated_product_of_many_rows(dev, rows, n, k, taken):
+    """Beyond 8192 rows the gated product is taken where W's halves are no narrower than 1024 and K: the two steps' result."""
+    import mdx
+    x, w = _integers(rows, 2 * n, k)
+    x, w = x.to(dev), w.to(dev)
+    y = mdx.ops.linear_gated(x, w)
+    assert (y is not None) == taken
+    if taken:
+        want = mdx.silu_and_mul((x.float() @ w.float().T).bfloat16()).float()
+        assert (y.float() - want).abs().max() <= 2.0 ** -7 * want.abs().max()
+
+
 @pytest.mark.parametrize("rows,vocab,hidden", [(129, 511, 256), (192, 30000, 256), (193, 30001, 384), (256, 70000, 256), (384, 40003, 256), (385, 769, 512), (512, 70001, 256)])
 def test_head_at_few_steps(dev, rows, vocab, hidden):
     import mdx
