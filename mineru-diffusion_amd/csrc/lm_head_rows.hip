@@ -9,12 +9,14 @@
 //    streams its own rows of W, three steps of 256 columns (24 KB) ahead of the product;
 //  * otherwise x goes through LDS K step by K step with a barrier per step, W one step ahead.
 //
-// All workgroups sum a row of W from column 0 on, so that equal rows have equal logits and the first of them is taken.  (Beginning at another column each
-// spreads the rows, which are mostly a power of two apart, over more of the memory's channels: 119 / 120 / 141 / 171 us below are 111 / 112 / 128 / 166 then.
-// Equal rows in different tiles then round apart.)
+// Rows of W are mostly a power of two apart, so that what all workgroups ask for at the same column meets in few of the memory's channels.  With x whole and
+// rows of whole quarters (1024 and 2048 columns) workgroup b therefore takes quarter i ^ (b % 4) of its rows as its i-th, and adds the quarters' sums as (0th + 1st) + (2nd +
+// 3rd): the same two meet whatever b is, so that equal rows have equal logits wherever they stand and the first of them is taken.  (us, 2048 columns, all from column 0 on / so: 12 rows
+// 119.1 / 109.0, 32 rows 120.5 / 110.5; 1024 columns level.  Eighths 114; each wavefront in an order of its own 115.  A loop without the fixed quarters, whose sums are
+// moved at run time, 165.  More rows hold too many sums: 64 rows 141 / 172.)
 //
 // W is read with ordinary loads: marked nontemporal, the two loads that share a 128-byte line fetch it twice now and then (139
-// against 129 us at 32 rows).  Bound: HBM.  us at 16 / 32 / 64 / 128 rows: 119 / 120 / 140 / 170 (5.2 TB/s at 32 rows); tiles of 256 rows
+// against 129 us at 32 rows).  Bound: HBM.  us at 16 / 32 / 64 / 128 rows: 109 / 110 / 140 / 170 (5.6 TB/s at 32 rows); tiles of 256 rows
 // 200 / 199 / 208 / 200, the library's product and a vocabulary pass 213 / 155 / 161 / 175.
 #include "lm_head.h"
 #include <atomic>
@@ -183,6 +185,49 @@ __global__ __launch_bounds__(kThreads, 1) void lm_head_whole_kernel(const LmHead
     rows.finish(P, lds, tid);
 }
 
+// The same where a row is SUBS steps, whole quarters: in an order of the workgroup's own.
+constexpr int kParts = 4;
+template <int SUBS>
+__global__ __launch_bounds__(kThreads, 1) void lm_head_parts_kernel(const LmHeadParams P)
+{
+    constexpr int MT = 2, kPanelBytes = 16 * MT * kPanel * 2, kEach = SUBS / kParts, kFar = kRing - 1;
+    static_assert(SUBS % kRing == 0 && SUBS % kParts == 0, "a tile begins with the ring's first");
+    extern __shared__ __attribute__((aligned(1024))) char lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const unsigned lds0 = (unsigned)(uintptr_t)(lds_char*)lds;
+    const int p = ((int)blockIdx.x & (kParts - 1)) * kEach, tiles = tiles_of_workgroup(P);
+    auto sub_of = [&](int i) { return (i / kEach * kEach ^ p) + i % kEach; };
+    Rows<MT> rows;
+    rows.init(P, lane & 15);
+#pragma unroll
+    for (int k = 0; k < SUBS * kSub; k += kPanel) load_x<MT, kPanel>(P, lds0 + k / kPanel * kPanelBytes, k, wave, lane);
+    Weights<kSub / 64> ring[kRing];
+    int tile = blockIdx.x;
+#pragma unroll
+    for (int r = 0; r < kFar; ++r) load_weights(ring[r], P, tile, sub_of(r) * kSub, wave, lane);
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");                // x is in LDS for everybody
+    for (int n = 0; n < tiles; ++n) {
+        const int next = tile + (int)gridDim.x;
+        f32x4 part[kParts][MT];
+#pragma unroll
+        for (int i = 0; i < SUBS; ++i) {
+            if (i + kFar < SUBS || n + 1 < tiles) load_weights(ring[(i + kFar) % kRing], P, i + kFar < SUBS ? tile : next, sub_of((i + kFar) % SUBS) * kSub, wave, lane);
+            __builtin_amdgcn_sched_barrier(0);
+            const int sub = sub_of(i);
+            if (i % kEach == 0)
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) part[i / kEach][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+            multiply<MT, kPanel>(part[i / kEach], ring[i % kRing], lds + sub / 2 * kPanelBytes, (sub & 1) * (kSub / 8), lane);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) part[0][mt] = (part[0][mt] + part[1][mt]) + (part[2][mt] + part[3][mt]);
+        rows.take(part[0], tile * kTileRows + wave * 16 + 4 * (lane >> 4), P.vocab);
+        tile = next;
+    }
+    rows.finish(P, lds, tid);
+}
+
 // MT: tiles of 16 rows of x.  KC: columns per step.
 template <int MT, int KC>
 __global__ __launch_bounds__(kThreads, 1) void lm_head_rows_kernel(const LmHeadParams P)
@@ -267,7 +312,9 @@ int launch_few_rows(LmHeadParams& P, hipStream_t stream)
     const int cus = mdx::compute_units();
     P.n_slices = P.n_vocab_tiles < cus ? P.n_vocab_tiles : cus;
     if (P.rows <= 32 && P.hidden <= kMaxWhole) {
-        static std::atomic<bool> raised[64];
+        static std::atomic<bool> raised[64], raised4[64], raised8[64];
+        if (P.hidden == 4 * kSub) return launch(lm_head_parts_kernel<4>, 32 * 4 * kSub * 2, raised4, P, stream);
+        if (P.hidden == 8 * kSub) return launch(lm_head_parts_kernel<8>, 32 * 8 * kSub * 2, raised8, P, stream);
         return launch(lm_head_whole_kernel, 32 * kMaxWhole * 2, raised, P, stream);
     }
     return P.rows <= 32 ? launch_steps<2, 512>(P, stream) : P.rows <= 64 ? launch_steps<4, 512>(P, stream) : launch_steps<8, 256>(P, stream);
