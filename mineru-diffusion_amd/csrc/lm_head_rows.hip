@@ -1,25 +1,21 @@
-// The fused vocabulary projection for few rows (up to 128: a decode pass of one to four sequences, or what is left masked of
-// more): logits x . W^T, rounded to bf16, reduced to (max, sum of exp, first argmax) in registers.  With so few rows it is a read
-// of W (622 MB at 151 936 x 2048): fragments of W straight
-// from memory into registers, x through LDS without passing registers.  One workgroup per CU walks the vocabulary in tiles of
-// 128 rows without a pause between tiles; a lane keeps the running state of its rows of x over all its logits, so that a
+// The fused vocabulary projection for up to 32 rows of 2048 columns (a decode pass of one sequence, or what is left masked of more): logits x . W^T, rounded to
+// bf16, reduced to (max, sum of exp, first argmax) in registers.  With so few rows it is a read of W (622 MB at 151 936 entries): fragments of W straight
+// from memory into registers, x whole in LDS (128 KB).  One workgroup per CU walks the vocabulary in tiles of
+// 128 rows without a pause between tiles; the wavefronts share nothing but x and need no barrier: each streams its own rows of W, three steps of 256 columns (24 KB)
+// ahead of the product.  A lane keeps the running state of its rows of x over all its logits, so that a
 // workgroup leaves one record per row at its end and the fold over the records is short.
 //
-//  * up to 32 rows and 2048 columns x fits in LDS whole (128 KB), the wavefronts share nothing else and need no barrier: each
-//    streams its own rows of W, three steps of 256 columns (24 KB) ahead of the product;
-//  * otherwise x goes through LDS K step by K step with a barrier per step, W one step ahead.
-//
-// Rows of W are mostly a power of two apart, so that what all workgroups ask for at the same column meets in few of the memory's channels.  With x whole and
-// rows of whole quarters (1024 and 2048 columns) workgroup b therefore takes quarter i ^ (b % 4) of its rows as its i-th, and adds the quarters' sums as (0th + 1st) + (2nd +
-// 3rd): the same two meet whatever b is, so that equal rows have equal logits wherever they stand and the first of them is taken.  (us, 2048 columns, all from column 0 on / so: 12 rows
-// 119.1 / 109.0, 32 rows 120.5 / 110.5; 1024 columns level.  Eighths 114; each wavefront in an order of its own 115.  A loop without the fixed quarters, whose sums are
-// moved at run time, 165.  More rows hold too many sums: 64 rows 141 / 172.)
+// Rows of W are mostly a power of two apart, so that what all workgroups ask for at the same column meets in few of the memory's channels.  Workgroup b therefore takes
+// quarter i ^ (b % 4) of its rows as its i-th, and adds the quarters' sums as (0th + 1st) + (2nd + 3rd): the same two meet whatever b is, so that equal
+// rows have equal logits wherever they stand and the first of them is taken.  (us, all from column 0 on / so: 12 rows 119.1 / 109.0, 32 rows 120.5 / 110.5.  Eighths
+// 114; each wavefront in an order of its own 115; a loop without the fixed quarters, whose sums are moved at run time, 165.)
 //
 // W is read with ordinary loads: marked nontemporal, the two loads that share a 128-byte line fetch it twice now and then (139
-// against 129 us at 32 rows).  Bound: HBM.  us at 16 / 32 / 64 / 128 rows: 109 / 110 / 140 / 170 (5.6 TB/s at 32 rows); tiles of 256 rows
-// 200 / 199 / 208 / 200, the library's product and a vocabulary pass 213 / 155 / 161 / 175.
+// against 129 us at 32 rows).  Bound: HBM.  us at 12 / 32 rows: 109 / 110 (5.6 TB/s); tiles of 64 x 128 (lm_head_unmask.hip) 124 / 124, the library's product and a vocabulary
+// pass 213 / 155.  More rows, and other widths, are better served by those tiles: 1024 columns, 24 rows 58.2 here, 56.9 there; 64 rows of 2048 through LDS step by step, a barrier
+// each, 141 against 127, 128 rows 170 against 154.
 #include "lm_head.h"
-#include <atomic>
+#include "linear_tile.h"
 
 namespace {
 
@@ -143,55 +139,12 @@ __device__ __forceinline__ void multiply(f32x4 (&acc)[MT], const Weights<PAIRS>&
 
 __device__ __forceinline__ int tiles_of_workgroup(const LmHeadParams& P) { return (P.n_vocab_tiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x; }
 
-// Up to 32 rows, x whole in LDS as panels of 512 columns.
-constexpr int kPanel = 512, kSub = 256, kRing = 4, kMaxWhole = 2048;
-__global__ __launch_bounds__(kThreads, 1) void lm_head_whole_kernel(const LmHeadParams P)
+// x in LDS as panels of 512 columns.
+constexpr int kPanel = 512, kSub = 256, kRing = 4, kParts = 4, kColumns = 2048;
+__global__ __launch_bounds__(kThreads, 1) void lm_head_few_rows_kernel(const LmHeadParams P)
 {
-    constexpr int MT = 2, kPanelBytes = 16 * MT * kPanel * 2;
-    extern __shared__ __attribute__((aligned(1024))) char lds[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const unsigned lds0 = (unsigned)(uintptr_t)(lds_char*)lds;
-    const int subs = P.hidden / kSub, n_steps = tiles_of_workgroup(P) * subs;
-    Rows<MT> rows;
-    rows.init(P, lane & 15);
-    f32x4 acc[MT] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-
-    for (int k = 0; k < P.hidden; k += kPanel) load_x<MT, kPanel>(P, lds0 + k / kPanel * kPanelBytes, k, wave, lane);
-    Weights<kSub / 64> ring[kRing];
-    int f_tile = blockIdx.x, f_sub = 0, m_tile = blockIdx.x, m_sub = 0;           // the step being fetched, and the one being multiplied
-    auto fetch = [&](Weights<kSub / 64>& d) {
-        load_weights(d, P, f_tile, f_sub * kSub, wave, lane);
-        if (++f_sub == subs) { f_sub = 0; f_tile += gridDim.x; }
-    };
-#pragma unroll
-    for (int r = 0; r < kRing - 1; ++r) fetch(ring[r]);                          // (a tile has at least two steps, and reading a tile too many is in bounds)
-    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");                // x is in LDS for everybody
-    for (int t = 0; t < n_steps; t += kRing) {
-#pragma unroll
-        for (int r = 0; r < kRing; ++r) {
-            if (t + r + kRing - 1 < n_steps) fetch(ring[(r + kRing - 1) % kRing]);
-            __builtin_amdgcn_sched_barrier(0);
-            if (t + r < n_steps) {
-                multiply<MT, kPanel>(acc, ring[r], lds + m_sub / 2 * kPanelBytes, (m_sub & 1) * (kSub / 8), lane);
-                if (++m_sub == subs) {
-                    rows.take(acc, m_tile * kTileRows + wave * 16 + 4 * (lane >> 4), P.vocab);
-                    m_sub = 0;
-                    m_tile += gridDim.x;
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    }
-    rows.finish(P, lds, tid);
-}
-
-// The same where a row is SUBS steps, whole quarters: in an order of the workgroup's own.
-constexpr int kParts = 4;
-template <int SUBS>
-__global__ __launch_bounds__(kThreads, 1) void lm_head_parts_kernel(const LmHeadParams P)
-{
-    constexpr int MT = 2, kPanelBytes = 16 * MT * kPanel * 2, kEach = SUBS / kParts, kFar = kRing - 1;
-    static_assert(SUBS % kRing == 0 && SUBS % kParts == 0, "a tile begins with the ring's first");
+    constexpr int MT = 2, kPanelBytes = 16 * MT * kPanel * 2, kSubs = kColumns / kSub, kEach = kSubs / kParts, kFar = kRing - 1;
+    static_assert(kSubs % kRing == 0 && kSubs % kParts == 0, "a tile begins with the ring's first");
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const unsigned lds0 = (unsigned)(uintptr_t)(lds_char*)lds;
@@ -200,7 +153,7 @@ __global__ __launch_bounds__(kThreads, 1) void lm_head_parts_kernel(const LmHead
     Rows<MT> rows;
     rows.init(P, lane & 15);
 #pragma unroll
-    for (int k = 0; k < SUBS * kSub; k += kPanel) load_x<MT, kPanel>(P, lds0 + k / kPanel * kPanelBytes, k, wave, lane);
+    for (int k = 0; k < kColumns; k += kPanel) load_x<MT, kPanel>(P, lds0 + k / kPanel * kPanelBytes, k, wave, lane);
     Weights<kSub / 64> ring[kRing];
     int tile = blockIdx.x;
 #pragma unroll
@@ -210,8 +163,8 @@ __global__ __launch_bounds__(kThreads, 1) void lm_head_parts_kernel(const LmHead
         const int next = tile + (int)gridDim.x;
         f32x4 part[kParts][MT];
 #pragma unroll
-        for (int i = 0; i < SUBS; ++i) {
-            if (i + kFar < SUBS || n + 1 < tiles) load_weights(ring[(i + kFar) % kRing], P, i + kFar < SUBS ? tile : next, sub_of((i + kFar) % SUBS) * kSub, wave, lane);
+        for (int i = 0; i < kSubs; ++i) {
+            if (i + kFar < kSubs || n + 1 < tiles) load_weights(ring[(i + kFar) % kRing], P, i + kFar < kSubs ? tile : next, sub_of((i + kFar) % kSubs) * kSub, wave, lane);
             __builtin_amdgcn_sched_barrier(0);
             const int sub = sub_of(i);
             if (i % kEach == 0)
@@ -228,96 +181,23 @@ __global__ __launch_bounds__(kThreads, 1) void lm_head_parts_kernel(const LmHead
     rows.finish(P, lds, tid);
 }
 
-// MT: tiles of 16 rows of x.  KC: columns per step.
-template <int MT, int KC>
-__global__ __launch_bounds__(kThreads, 1) void lm_head_rows_kernel(const LmHeadParams P)
-{
-    extern __shared__ __attribute__((aligned(1024))) char lds[];            // two x tiles of [16 MT][KC]
-    constexpr int kBufBytes = 16 * MT * KC * 2, kPairs = KC / 64;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const unsigned lds0 = (unsigned)(uintptr_t)(lds_char*)lds;
-    const int chunks = P.hidden / KC, n_steps = tiles_of_workgroup(P) * chunks;
-    Rows<MT> rows;
-    rows.init(P, lane & 15);
-    f32x4 acc[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    Weights<kPairs> a, b;
-    int f_tile = blockIdx.x, f_chunk = 0, m_tile = blockIdx.x, m_chunk = 0;       // the step being fetched, and the one being multiplied
-    auto fetch = [&](Weights<kPairs>& d, int buf) {
-        load_x<MT, KC>(P, lds0 + buf * kBufBytes, f_chunk * KC, wave, lane);
-        load_weights(d, P, f_tile, f_chunk * KC, wave, lane);
-        if (++f_chunk == chunks) { f_chunk = 0; f_tile += gridDim.x; }
-    };
-    auto step = [&](const Weights<kPairs>& d, int buf) {
-        multiply<MT, KC>(acc, d, lds + buf * kBufBytes, 0, lane);
-        if (++m_chunk < chunks) return;
-        rows.take(acc, m_tile * kTileRows + wave * 16 + 4 * (lane >> 4), P.vocab);
-        m_chunk = 0;
-        m_tile += gridDim.x;
-    };
-    // A step's x is in LDS for everybody once each wavefront has waited for its own loads; its W, issued after them, may still be on
-    // its way (the compiler waits for that register by register).
-    auto arrived = [&]() {
-        __builtin_amdgcn_sched_barrier(0);
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(2 * kPairs) : "memory");
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    fetch(a, 0);
-    for (int t = 0; t < n_steps; t += 2) {
-        arrived();
-        if (t + 1 < n_steps) fetch(b, 1);
-        __builtin_amdgcn_sched_barrier(0);
-        step(a, 0);
-        if (t + 1 >= n_steps) break;
-        arrived();
-        if (t + 2 < n_steps) fetch(a, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        step(b, 1);
-    }
-    rows.finish(P, lds, tid);
-}
-
-// The kernel's LDS limit is raised once per device.
-int launch(void (*kernel)(const LmHeadParams), int lds_bytes, std::atomic<bool>* raised, const LmHeadParams& P, hipStream_t stream)
-{
-    int device = 0;
-    hipError_t e = hipGetDevice(&device);
-    MDX_REQUIRE(e == hipSuccess && device >= 0 && device < 64, MDX_ELAUNCH, "lm_head_confidence: no current device (%s)", hipGetErrorString(e));
-    if (!raised[device].load(std::memory_order_acquire)) {
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
-        MDX_REQUIRE(e == hipSuccess, MDX_ELAUNCH, "lm_head_confidence: cannot reserve %d bytes of LDS (%s)", lds_bytes, hipGetErrorString(e));
-        raised[device].store(true, std::memory_order_release);
-    }
-    kernel<<<(unsigned)P.n_slices, kThreads, lds_bytes, stream>>>(P);
-    return mdx::check_launch("lm_head_confidence");
-}
-
-template <int MT, int KC> int launch_steps(const LmHeadParams& P, hipStream_t stream)
-{
-    static std::atomic<bool> raised[64];
-    return launch(lm_head_rows_kernel<MT, KC>, 2 * 16 * MT * KC * 2, raised, P, stream);
-}
-
 }  // namespace
 
 namespace mdx_head {
 
-bool few_rows_covered(int64_t rows, int64_t hidden) { return rows <= 128 && hidden % (rows <= 64 ? 512 : 256) == 0; }
+bool few_rows_covered(int64_t rows, int64_t hidden) { return rows <= 32 && hidden == kColumns; }
 
 int launch_few_rows(LmHeadParams& P, hipStream_t stream)
 {
+    static std::atomic<bool> raised[64];
+    constexpr int kLdsBytes = 32 * kColumns * 2;
+    const int rc = mdx_tile::reserve_lds(reinterpret_cast<const void*>(lm_head_few_rows_kernel), kLdsBytes, raised, "lm_head_confidence");
+    if (rc != MDX_OK) return rc;
     P.n_vocab_tiles = (P.vocab + kTileRows - 1) / kTileRows;
     const int cus = mdx::compute_units();
     P.n_slices = P.n_vocab_tiles < cus ? P.n_vocab_tiles : cus;
-    if (P.rows <= 32 && P.hidden <= kMaxWhole) {
-        static std::atomic<bool> raised[64], raised4[64], raised8[64];
-        if (P.hidden == 4 * kSub) return launch(lm_head_parts_kernel<4>, 32 * 4 * kSub * 2, raised4, P, stream);
-        if (P.hidden == 8 * kSub) return launch(lm_head_parts_kernel<8>, 32 * 8 * kSub * 2, raised8, P, stream);
-        return launch(lm_head_whole_kernel, 32 * kMaxWhole * 2, raised, P, stream);
-    }
-    return P.rows <= 32 ? launch_steps<2, 512>(P, stream) : P.rows <= 64 ? launch_steps<4, 512>(P, stream) : launch_steps<8, 256>(P, stream);
+    lm_head_few_rows_kernel<<<(unsigned)P.n_slices, kThreads, kLdsBytes, stream>>>(P);
+    return mdx::check_launch("lm_head_confidence");
 }
 
 }  // namespace mdx_head

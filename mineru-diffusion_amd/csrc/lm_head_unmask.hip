@@ -7,8 +7,8 @@
 // (engines/nano_dvlm/nanovllm/layers/embed_head.py:61-67) followed by Sampler.prepare's softmax
 // confidence and argmax without noise (layers/sampler.py:11-22).
 //
-// A workgroup computes a tile of 256 x 256 or 192 x 256 (x rows by vocabulary rows) over the whole hidden dimension
-// (linear_tile.h) and leaves one 16-byte record per x row; a second, small kernel folds a row's records (about vocab / 256 of them) into x0 /
+// A workgroup computes a tile of 64 x 128 to 256 x 256 (x rows by vocabulary rows) over the whole hidden dimension
+// (linear_tile.h) and leaves one 16-byte record per x row; a second, small kernel folds a row's records (about vocab / 256 or / 128 of them) into x0 /
 // x0_p.  What bounds it: the matrix pipe under the board's power limit (at 1024 rows 522 us on data, 441 on zeros, whose clock
 // is higher, 380 without loads), 5 us of epilogue per tile, the last round of tiles (500 rows: 4.64 of 5).
 #include "lm_head.h"
@@ -241,13 +241,18 @@ int launch_two_steps(LmHeadParams& P, hipStream_t stream)
     return mdx::check_launch("lm_head_confidence");
 }
 
-// Which tile: rounds of one workgroup per CU times what a round takes (us over 2048 columns: 256 x 256 53.5, 192 x 256 44.5).  151 936 entries, the call, us,
-// 256 x 256 / 192 x 256: 136 rows 186 / 170, 192 188 / 172, 256 188 / 226, 300 270 / 230, 384 270 / 229, 512 274 / 312, 640 373 / 418, 768 383 / 421, 1024
-// 522 / 584.  (128 x 256: 183, 191, 194, 245, 246, 329, 388, 445, 599; 192 x 192: 175, 180, 243, 248, 253, 346, 437, 444, 620; 256 x 192 and 128 x 192 lie above
-// the better of the two everywhere.)  With loads and reads in bursts behind the barriers (linear_tile.h): 136 rows 181, 192 185, 256 198, 384 263, 512 304, 768 418, 1024 560.
+// Which tile.  Up to 64 rows 64 x 128, of which two fit a CU (72 KB of LDS each), so that one's epilogue has the other's loads beside it; up to 128 rows 128 x 128.  151 936 entries, us,
+// through LDS step by step, W straight to registers (which these two replaced) / here: 2048 columns, 40 rows 140 / 125, 64 141 / 127, 80 166 / 150, 128 171 / 154; 1024 columns 69 / 58, 71 / 61, 90 /
+// 82, 91 / 85; 4096 256 / 234, 260 / 231, 314 / 258, 318 / 265.  (128 x 256: 40 rows 152, 128 159; 128 x 128 with two steps in LDS, two a CU, 128 rows 163; 64 x 128 with two steps 141.)
+// More rows: rounds of one workgroup per CU times what a round takes (us over 2048 columns: 256 x 256 53.5, 192 x 256 44.5), us, 256 x 256 / 192 x 256: 136 rows 186 / 170, 192 188 / 172, 256
+// 188 / 226, 300 270 / 230, 384 270 / 229, 512 274 / 312, 640 373 / 418, 768 383 / 421, 1024 522 / 584.  (128 x 256: 183, 191, 194, 245, 246, 329, 388, 445, 599; 192 x 192: 175, 180, 243, 248, 253, 346, 437,
+// 444, 620; 192 x 128, 192 rows 172; 256 x 192, 256 x 128 and 128 x 192 lie above the better of the two everywhere.)  With loads and reads in bursts behind the barriers (linear_tile.h): 136 rows 181, 192 185, 256 198,
+// 384 263, 512 304, 768 418, 1024 560.  Whole rounds in the larger tile and the rest of the vocabulary in smaller ones is level (500 rows 273.5 / 274.9): the last round's tiles run faster by themselves.
 int launch_product(LmHeadParams& P, hipStream_t stream)
 {
-    if (P.hidden < 3 * kStepK) return launch_two_steps(P, stream);
+    if (P.hidden < 4 * kStepK) return launch_two_steps(P, stream);       // (128 columns)
+    if (P.rows <= 64) return launch_tiles<64, 128, 3, 3>(P, stream);
+    if (P.rows <= 128) return launch_tiles<128, 128, 4, 4>(P, stream);
     const int cus = mdx::compute_units();
     auto cost = [&](int bm, int bn, float round) {
         const int64_t tiles = (int64_t)((P.rows + bm - 1) / bm) * ((P.vocab + bn - 1) / bn);
@@ -298,7 +303,6 @@ extern "C" int mdx_lm_head_confidence(const void* x, int64_t x_row_stride, const
     P.records = static_cast<Record*>(workspace);
     P.x0 = x0; P.x0_p = x0_p;
 
-    // up to 128 rows the tiles of 256 rows are mostly padding
     const int rc = few_rows_covered(rows, hidden) ? launch_few_rows(P, stream) : launch_product(P, stream);
     if (rc != MDX_OK) return rc;
     lm_head_finalize_kernel<<<(unsigned)((rows + kFoldThreads / 64 - 1) / (kFoldThreads / 64)), kFoldThreads, 0, stream>>>(P);

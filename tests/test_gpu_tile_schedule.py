@@ -48,7 +48,7 @@ def test_gated_product_of_many_rows(dev, rows, n, k, taken):
         assert (y.float() - want).abs().max() <= 2.0 ** -7 * want.abs().max()
 
 
-@pytest.mark.parametrize("rows,vocab,hidden", [(1, 100, 2048), (17, 1000, 1024), (32, 40001, 2048), (31, 70001, 1024), (20, 33000, 2048), (129, 511, 256), (192, 30000, 256), (193, 30001, 384), (256, 70000, 256), (384, 40003, 256), (385, 769, 512), (512, 70001, 256)])
+@pytest.mark.parametrize("rows,vocab,hidden", [(1, 100, 2048), (17, 1000, 1024), (33, 70001, 256), (64, 129, 512), (65, 70001, 256), (100, 40001, 1024), (128, 257, 384), (32, 40001, 2048), (31, 70001, 1024), (20, 33000, 2048), (129, 511, 256), (192, 30000, 256), (193, 30001, 384), (256, 70000, 256), (384, 40003, 256), (385, 769, 512), (512, 70001, 256)])
 def test_head_at_few_steps(dev, rows, vocab, hidden):
     import mdx
     x, w = _integers(rows, vocab, hidden)
