@@ -185,6 +185,7 @@ const TileCost kTiles[] = {
     tile<192, 128, 2, 2, 2, 4, 4, true>(0.584f, 3.5f),
     tile<128, 192, 4, 2, 1, 4, 4, true>(0.617f, 2.3f),
     tile<192, 192, 4, 2, 1, 3, 3, false>(0.741f, 5.0f),
+    tile<256, 128, 4, 2, 1, 3, 3, true>(0.60f, 4.5f),        // slices of long K: 1024 x 2048 x 6144 and the norm behind it 40.0 us as two of 128 x 128 tiles, 37.9 as four
     tile<256, 192, 4, 2, 1, 3, 2, false>(0.983f, 3.7f),
     tile<256, 256, 4, 2, 1, 3, 2, false>(1.149f, 5.9f),
 };

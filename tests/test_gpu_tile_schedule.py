@@ -11,8 +11,8 @@ def _integers(rows, n, k):
     return (torch.randint(-2, 3, (rows, k), generator=g).bfloat16(), torch.randint(-2, 3, (n, k), generator=g).bfloat16())
 
 
-@pytest.mark.parametrize("k", [256, 384, 640])
-@pytest.mark.parametrize("rows,n", [(33, 72), (129, 264), (192, 2056), (257, 4104), (577, 2056), (1025, 4104), (1120, 6152), (1536, 8200), (2049, 6152), (4100, 6152)])
+@pytest.mark.parametrize("k", [256, 384, 640, 6144])
+@pytest.mark.parametrize("rows,n", [(33, 72), (129, 264), (192, 2056), (257, 4104), (577, 2056), (1025, 4104), (1120, 6152), (1536, 8200), (2049, 6152), (4100, 6152), (1000, 2048), (1280, 2048)])
 def test_products_at_few_steps(dev, rows, n, k):
     import mdx
     x, w = _integers(rows, n, k)
