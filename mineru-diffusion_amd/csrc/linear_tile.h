@@ -21,7 +21,7 @@
 //    194 / 186, 500 299 / 282, 1024 551 / 531).
 //  * W is the first operand, so that a lane ends with four consecutive columns of one row of x.
 // Touching lines of W ahead of their loads (a CU's loads come back in order: gate/up 45 -> 49 us), starting the workgroups at different steps of K, other bands of
-// tiles per XCD, steps of 32 elements (half lines: slower), six steps in LDS instead of four of the small tiles, a wavefront priority around the products and a barrier that does not wait for the reads (five steps in LDS)
+// tiles per XCD, steps of 32 elements (half lines: slower), more steps in LDS for the middle tiles, a wavefront priority around the products and a barrier that does not wait for the reads (five steps in LDS)
 // gained nothing; four wavefronts of 128 x 128 instead of eight of 64 x 128 are slower (35 840 rows 1356 -> 1402 us, the head's 1024 528 -> 544).
 #pragma once
 #include "mdx_common.h"
