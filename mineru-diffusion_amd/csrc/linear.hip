@@ -178,7 +178,7 @@ constexpr TileCost tile(float step, float around) {
 }
 const TileCost kTiles[] = {
     tile<32, 64, 2, 2, 1, 6, 6, true>(0.165f, 0.4f),         // (four steps in LDS: gate/up of 32 rows 12.66 us, down 8.33; six 12.30, 8.05)
-    tile<64, 64, 2, 2, 2, 4, 4, true>(0.231f, 0.7f),
+    tile<64, 64, 2, 2, 2, 6, 6, true>(0.223f, 0.7f),         // (four: QKV in two slices, 96 rows 8.52, down 64 rows 8.43; six 8.02, 8.17)
     tile<128, 64, 2, 2, 2, 4, 4, true>(0.326f, 1.7f),
     tile<192, 64, 2, 2, 2, 4, 4, true>(0.408f, 2.9f),
     tile<128, 128, 2, 2, 2, 4, 4, true>(0.487f, 2.6f),
