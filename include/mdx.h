@@ -381,6 +381,7 @@ int mdx_unmask_step_host_blocks(const void* logits, int64_t row_stride, int32_t 
                                 int64_t* tokens, int64_t mask_token_id, float threshold, int32_t k,
                                 uint8_t* transfer, int32_t* count, int32_t bs, int32_t block_len, int64_t vocab,
                                 void* workspace, int64_t workspace_bytes, mdx_stream_t stream);
+int64_t mdx_unmask_step_host_blocks_counter_bytes(int32_t bs, int32_t block_len);   /* 0: counters would not be used */
 int mdx_unmask_step_host_blocks_single_launch(const void* logits, int64_t row_stride, int32_t dtype,
                                               const float* temperatures, const float* noise, int64_t noise_row_stride,
                                               int32_t seeded, uint64_t seed, uint64_t offset, const int64_t* offset_dev,

@@ -913,7 +913,8 @@ PyObject* sampler_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (t.defined()) NEED(t.numel() == bs);
         const int64_t ws_bytes = mdx_unmask_step_host_blocks_workspace_bytes(l.rows, l.vocab);
         const Tensor ws = make(logits, at::kByte, ws_bytes);
-        const Tensor counters = eager_counters(logits, mdx_unmask_step_counter_bytes((int32_t)bs, (int32_t)S));
+        const int64_t counter_bytes = mdx_unmask_step_host_blocks_counter_bytes((int32_t)bs, (int32_t)S);
+        const Tensor counters = counter_bytes > 0 ? eager_counters(logits, counter_bytes) : Tensor();   // (the call waits: 0.15 us of three sequences' 40)
         check(mdx_unmask_step_host_blocks_single_launch(ptr(l.t), l.stride, dtype_of(logits), static_cast<const float*>(ptr_or_null(t)), z.data(), z.data() ? l.vocab : 0,
                                           z.seeded ? 1 : 0, z.seed, z.offset, static_cast<const int64_t*>(ptr_or_null(z.offset_dev)),
                                           reinterpret_cast<int64_t*>(host), to_int(a[5]), (float)real(a[6]), (int32_t)to_int(a[7]),

@@ -1079,6 +1079,11 @@ extern "C" int64_t mdx_unmask_step_host_blocks_workspace_bytes(int64_t rows, int
     return rows <= 0 || vocab <= 0 ? 0 : confidences_bytes(rows) + rows * pick_nsplit(1, vocab) * (int64_t)sizeof(Partial);
 }
 
+extern "C" int64_t mdx_unmask_step_host_blocks_counter_bytes(int32_t bs, int32_t block_len)
+{
+    return (int64_t)bs * block_len < kSingleLaunchRows ? 0 : mdx_unmask_step_counter_bytes(bs, block_len);
+}
+
 extern "C" int mdx_unmask_step_host_blocks_single_launch(const void* logits, int64_t row_stride, int32_t dtype,
                                                          const float* temperatures, const float* noise, int64_t noise_row_stride,
                                                          int32_t seeded, uint64_t seed, uint64_t offset, const int64_t* offset_dev,
