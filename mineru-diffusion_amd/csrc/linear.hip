@@ -9,16 +9,17 @@
 //
 // Weights from HBM, us, here / the library's product (gate/up: with the SiLU kernel), QKV (4096 x 2048), output (2048 x 2048), gate/up
 // (12288 x 2048) and down (2048 x 6144) projection:
-//   rows    32   5.6  4.3  12.9   7.2 /  11.8 11.2  18.0 16.4      (a kernel with W straight in registers: 6.2  4.4 14.9  8.1)
-//   rows   128   8.6  6.6  18.7  11.5 /  14.7 11.3  21.8 17.6      (                                       9.4  6.7  -   12.1)
-//   rows   256  12.4  8.2  24.4  15.3 /  13.4 11.8  31.3 22.5
-//   rows   512  16.4 11.8  31.0  21.4 /  17.7 12.6  36.4 27.6
-//   rows  1024  22.9 16.1  49.6  33.9 /  24.8 16.7  57.6 42.0
-//   rows  1536  29.8 21.0  79.9  42.3 /  29.9 21.6  99.1 48.7
-//   rows  4096  60.6 35.2 175.1  94.1 /  51.3 35.4 177.7 91.3
-//   rows  8192 119.3 59.0 349.7 167.8 /  99.7 53.3 350.6 145.0
-// (Up to 1536 rows the better of rounded and partial sums.  Rounded where partial sums would be the faster, for a caller that doesn't take them: QKV 32 rows 10.5, 256 12.2, 383 16.3
-// against the library's 14.9; down, whose chain of 96 steps few tiles share, 32 rows 25 / 17, 512 29.5 / 27.5, 1536 54 / 45: a caller that can't take partial sums
+//   rows    32    5.7   4.7  11.8   7.6 /   9.3   8.9  16.1  17.1
+//   rows   128    7.8   6.0  16.0  11.7 /  12.6   9.0  20.9  17.9
+//   rows   256    9.6   7.0  21.1  15.5 /  11.5   9.9  29.4  22.7
+//   rows   512   12.9   9.1  27.3  21.4 /  15.7  11.3  34.8  27.6
+//   rows  1024   18.7  13.1  43.6  28.1 /  20.9  15.1  53.1  41.6
+//   rows  1536   25.2  16.6  67.0  40.3 /  25.8  18.3  89.3  47.1
+//   rows  4096   56.5  33.2   154  80.3 /  49.8  33.2   167  81.8
+//   rows  8192    106  55.6   323   140 /  93.5  49.7   337   129
+//   rows 35840    485   262  1385   823 /   434   213  1501   668
+// (Up to 1536 rows the better of rounded and partial sums.  Rounded where partial sums would be the faster, for a caller that doesn't take them, is slower than the library where K is long: down, whose
+// chain of 96 steps few tiles share, 32 rows 25 / 17, 512 38 / 27.6, 1024 40 / 41.6: a caller that can't take partial sums
 // there does better with the library.)
 #include "linear_tile.h"
 #include "qk_row.h"
@@ -160,7 +161,7 @@ int launch(LinearParams A, hipStream_t stream)
 }
 
 // The tiles there are, and what a round of them costs: a step of K and what stands before and behind the steps, us, fitted to
-// 3200 timings with cold weights (four projections of the decoder, 16 to 8192 rows, every tile, 1 to 24 slices of K).
+// 1700 timings with cold weights (four projections of the decoder, 32 to 8192 rows, every tile, 1 to 32 slices of K).
 struct TileCost {
     int bm, bn, least_steps, steps_multiple;                // steps of 64 elements of K: at least, and a multiple of
     float step, around;
@@ -195,7 +196,7 @@ struct Plan { const TileCost* tile; int splits; double cost; };
 // The cheapest tile and number of slices by the costs above, in rounds of one workgroup per CU (the small tiles' second one
 // per CU is worth little: they share its intake).  Partial sums cost their writing and the next kernel's reading, 0.35 us per
 // MB together (5.7 TB/s), a rounded result less than half of that per element.  Against the best of all timed choices this
-// costs 1 % on average and 15 % at most.
+// costs 0.3 % on average and 4 % at most.
 Plan plan_of(int64_t rows, int64_t n, int64_t k, bool rounded, bool partials, bool silu)
 {
     Plan best{nullptr, 0, 0};
