@@ -48,6 +48,27 @@ def test_gated_product_of_many_rows(dev, rows, n, k, taken):
         assert (y.float() - want).abs().max() <= 2.0 ** -7 * want.abs().max()
 
 
+def test_silu_of_every_gate(dev):
+    """Every bf16 value, times powers of two, as the gate of the product's own SiLU and of the kernel that divides: the same bits."""
+    import mdx
+    k, n = 256, 16
+    gates = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    x = torch.zeros(65536, k, dtype=torch.bfloat16)
+    x[:, 0], x[:, 1] = gates, 1.0
+    w = torch.zeros(2 * n, k, dtype=torch.bfloat16)
+    w[:n, 0] = 2.0 ** (torch.arange(n) - 8.0)
+    w[n:, 1] = 1.0 + torch.arange(n) / 16
+    x, w = x.to(dev), w.to(dev)
+    L, stream = mdx._lib.lib(), torch.cuda.current_stream().cuda_stream
+    product = torch.empty(65536, 2 * n, dtype=torch.bfloat16, device=dev)
+    y = torch.empty(65536, n, dtype=torch.bfloat16, device=dev)
+    assert L.mdx_linear(x.data_ptr(), k, w.data_ptr(), k, product.data_ptr(), 2 * n, 65536, 2 * n, k, stream) == 0
+    assert L.mdx_linear_silu(x.data_ptr(), k, w.data_ptr(), k, y.data_ptr(), n, 65536, n, k, stream) == 0
+    want = mdx.silu_and_mul(product)
+    assert torch.equal(y.isnan(), want.isnan())
+    assert torch.equal(y.nan_to_num(nan=7.0).view(torch.int16), want.nan_to_num(nan=7.0).view(torch.int16))
+
+
 @pytest.mark.parametrize("rows,vocab,hidden", [(1, 100, 2048), (17, 1000, 1024), (33, 70001, 256), (64, 129, 512), (65, 70001, 256), (100, 40001, 1024), (128, 257, 384), (32, 40001, 2048), (31, 70001, 1024), (20, 33000, 2048), (129, 511, 256), (192, 30000, 256), (193, 30001, 384), (256, 70000, 256), (384, 40003, 256), (385, 769, 512), (512, 70001, 256)])
 def test_head_at_few_steps(dev, rows, vocab, hidden):
     import mdx
