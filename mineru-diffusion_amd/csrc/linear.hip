@@ -192,7 +192,8 @@ struct TileCost {
 template <int BM, int BN, int WM, int WN, int WK, int S, int SX, bool PARTIALS>
 constexpr TileCost tile(float step, float around) {
     typedef Tile<BM, BN, WM, WN, WK, S, SX, false> T;
-    if constexpr (PARTIALS) return TileCost{BM, BN, T::kLeastSteps, T::kStepsMultiple, step, around, launch<BM, BN, WM, WN, WK, S, SX, kRounded>,
+    // (a slice has four steps at least: rows that are too far apart for the plan's tile go to one that loads four ahead, run_partials)
+    if constexpr (PARTIALS) return TileCost{BM, BN, T::kLeastSteps < 4 ? 4 : T::kLeastSteps, T::kStepsMultiple, step, around, launch<BM, BN, WM, WN, WK, S, SX, kRounded>,
                                             launch<BM, BN, WM, WN, WK, S, SX, kPartials>, launch<BM, BN, WM, WN, WK, S, SX, kSilu>};
     else return TileCost{BM, BN, T::kLeastSteps, T::kStepsMultiple, step, around, launch<BM, BN, WM, WN, WK, S, SX, kRounded>, nullptr,
                          launch<BM, BN, WM, WN, WK, S, SX, kSilu>};

@@ -1,0 +1,19 @@
+"""Slices of K that the linear layers' plans make: whole steps of 64 elements, and never fewer than the four that the tile for rows far apart loads ahead."""
+import random
+
+import mdx
+
+
+def test_slices_have_four_steps_and_more():
+    L, rng = mdx._lib.lib(), random.Random(3)
+    seen = set()
+    for _ in range(20000):
+        rows, k = rng.randint(1, 128), 256 * rng.randint(1, 40)
+        n = 64 * (rng.randint(1, 64) if rng.random() < 0.7 else rng.randint(64, 4000))
+        s = L.mdx_decode_linear_splits(rows, n, k)
+        assert s > 0 and k % (64 * s) == 0 and k // 64 // s >= 4, (rows, n, k, s)
+        seen.add(s)
+        rows, k = rng.randint(1, 1536), 128 * rng.randint(2, 80)
+        s = L.mdx_linear_splits(rows, n, k)
+        assert s <= 0 or (k % (64 * s) == 0 and k // 64 // s >= 4), (rows, n, k, s)
+    assert len(seen) > 4
