@@ -24,14 +24,21 @@ __global__ __launch_bounds__(kThreads) void store_kvcache_vec16(
     const int32_t* __restrict__ slot_mapping,
     int row16, int64_t num_slots)
 {
+    // The row is on its way before its slot is known: one trip to memory instead of two.  (us, the other way round / so: the store and the attention of one
+    // block behind 16 x 2300 keys 43.2 / 43.0, 64 x 800 57.0 / 56.5; 38 434 tokens 51.7 / 50.6.  Both rows of a token in one workgroup: 51.8.)
     const int64_t tok = blockIdx.x;
-    const int64_t s = slot_mapping[tok];
-    if (s < 0 || s >= num_slots) return;
     const bool is_v = blockIdx.y != 0;
     const u32x4* src = is_v ? value + tok * v_stride16 : key + tok * k_stride16;
+    int c = threadIdx.x;
+    u32x4 x = c < row16 ? __builtin_nontemporal_load(src + c) : u32x4{0, 0, 0, 0};
+    const int64_t s = slot_mapping[tok];
+    if (s < 0 || s >= num_slots) return;
     u32x4* dst = (is_v ? v_cache : k_cache) + s * row16;
-    for (int c = threadIdx.x; c < row16; c += blockDim.x)
-        __builtin_nontemporal_store(__builtin_nontemporal_load(src + c), dst + c);
+    while (c < row16) {
+        __builtin_nontemporal_store(x, dst + c);
+        c += blockDim.x;
+        if (c < row16) x = __builtin_nontemporal_load(src + c);
+    }
 }
 
 // Fallback for unaligned bases/strides or odd row sizes: element-wise copy.
