@@ -25,7 +25,7 @@ __device__ __forceinline__ float row_scale(const LmHeadParams& P, int row) {
 }
 
 // The form for few rows: whether it covers the shape, and its launch (records only; n_slices is set to their number per row).
-bool few_rows_covered(int64_t rows, int64_t hidden);
+bool few_rows_covered(int64_t rows, int64_t vocab, int64_t hidden);
 int launch_few_rows(LmHeadParams& P, hipStream_t stream);
 
 }  // namespace mdx_head

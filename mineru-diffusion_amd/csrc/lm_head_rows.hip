@@ -1,19 +1,21 @@
-// The fused vocabulary projection for up to 32 rows of 2048 columns (a decode pass of one sequence, or what is left masked of more): logits x . W^T, rounded to
-// bf16, reduced to (max, sum of exp, first argmax) in registers.  With so few rows it is a read of W (622 MB at 151 936 entries): fragments of W straight
-// from memory into registers, x whole in LDS (128 KB).  One workgroup per CU walks the vocabulary in tiles of
+// The fused vocabulary projection for up to 32 rows of 2048 columns, and of 512 and 1024 for large vocabularies (a decode pass of one sequence, or what is left masked of
+// more): logits x . W^T, rounded to bf16, reduced to (max, sum of exp, first argmax) in registers.  With so few rows it is a read of W (622 MB at 151 936 x 2048): fragments of W straight
+// from memory into registers, x whole in LDS (at most 128 KB).  One workgroup per CU walks the vocabulary in tiles of
 // 128 rows without a pause between tiles; the wavefronts share nothing but x and need no barrier: each streams its own rows of W, three steps of 256 columns (24 KB)
 // ahead of the product.  A lane keeps the running state of its rows of x over all its logits, so that a
 // workgroup leaves one record per row at its end and the fold over the records is short.
 //
 // Rows of W are mostly a power of two apart, so that what all workgroups ask for at the same column meets in few of the memory's channels.  Workgroup b therefore takes
-// quarter i ^ (b % 4) of its rows as its i-th, and adds the quarters' sums as (0th + 1st) + (2nd + 3rd): the same two meet whatever b is, so that equal
-// rows have equal logits wherever they stand and the first of them is taken.  (us, all from column 0 on / so: 12 rows 119.1 / 109.0, 32 rows 120.5 / 110.5.  Eighths
-// 114; each wavefront in an order of its own 115; a loop without the fixed quarters, whose sums are moved at run time, 165.)
+// part i ^ (b % parts) of its rows as its i-th (four parts of 2048 columns, two of the others: parts of 1 KB, or half a row), and adds the parts' sums as (0th + 1st) + (2nd + 3rd): the
+// same two meet whatever b is, so that equal rows have equal logits wherever they stand and the first of them is taken.  (us, all from column 0 on / so: 12 rows 119.1 / 109.0, 32 rows
+// 120.5 / 110.5.  Eighths 114; each wavefront in an order of its own 115; a loop without the fixed parts, whose sums are moved at run time, 165; 1024 columns in four parts of 512
+// bytes 69, in two 60.)  The loads ahead are asked for without a condition: behind one that might not have been, the compiler waits for all of them (512 columns 68 us, so 36).
 //
 // W is read with ordinary loads: marked nontemporal, the two loads that share a 128-byte line fetch it twice now and then (139
 // against 129 us at 32 rows).  Bound: HBM.  us at 12 / 32 rows: 109 / 110 (5.6 TB/s); tiles of 64 x 128 (lm_head_unmask.hip) 124 / 124, the library's product and a vocabulary
-// pass 213 / 155.  More rows, and other widths, are better served by those tiles: 1024 columns, 24 rows 58.2 here, 56.9 there; 64 rows of 2048 through LDS step by step, a barrier
-// each, 141 against 127, 128 rows 170 against 154.
+// pass 213 / 155.  More rows are better served by those tiles: 64 rows of 2048 through LDS step by step, a barrier each, 141 against 127, 128 rows 170 against 154.  So are other widths,
+// but where a workgroup has more than four tiles of 512 or 1024 columns (32 rows, here / there, us: 151 936 entries, 512 columns 35.6 / 38.3, 1024 60.2 / 64.1; 100 000 31 / 30, 50 / 49;
+// 48 000 21.6 / 18.0, 31 / 28.5; 32 000 16 / 13.4, 22.7 / 19.7).  1536 columns: level at 151 936 (90 / 91), 70 / 68 at 100 000, 29.8 / 27.3 at 32 000.
 #include "lm_head.h"
 #include "linear_tile.h"
 
@@ -139,12 +141,14 @@ __device__ __forceinline__ void multiply(f32x4 (&acc)[MT], const Weights<PAIRS>&
 
 __device__ __forceinline__ int tiles_of_workgroup(const LmHeadParams& P) { return (P.n_vocab_tiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x; }
 
-// x in LDS as panels of 512 columns.
-constexpr int kPanel = 512, kSub = 256, kRing = 4, kParts = 4, kColumns = 2048;
+// x in LDS as panels of 512 columns.  The ring's slots are fixed in the code, so that where a tile's steps are no multiple of the ring two tiles make one pass of the loop.
+constexpr int kPanel = 512, kSub = 256, kRing = 4, kLeastRounds = 4;
+template <int COLUMNS>
 __global__ __launch_bounds__(kThreads, 1) void lm_head_few_rows_kernel(const LmHeadParams P)
 {
-    constexpr int MT = 2, kPanelBytes = 16 * MT * kPanel * 2, kSubs = kColumns / kSub, kEach = kSubs / kParts, kFar = kRing - 1;
-    static_assert(kSubs % kRing == 0 && kSubs % kParts == 0, "a tile begins with the ring's first");
+    constexpr int MT = 2, kPanelBytes = 16 * MT * kPanel * 2, kSubs = COLUMNS / kSub, kParts = kSubs == 8 ? 4 : 2, kEach = kSubs / kParts, kFar = kRing - 1;
+    constexpr int kTiles = kSubs % kRing == 0 ? 1 : 2;
+    static_assert(kSubs % kParts == 0 && kTiles * kSubs % kRing == 0, "whole parts; a pass of the loop begins with the ring's first");
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const unsigned lds0 = (unsigned)(uintptr_t)(lds_char*)lds;
@@ -153,51 +157,67 @@ __global__ __launch_bounds__(kThreads, 1) void lm_head_few_rows_kernel(const LmH
     Rows<MT> rows;
     rows.init(P, lane & 15);
 #pragma unroll
-    for (int k = 0; k < kColumns; k += kPanel) load_x<MT, kPanel>(P, lds0 + k / kPanel * kPanelBytes, k, wave, lane);
+    for (int k = 0; k < COLUMNS; k += kPanel) load_x<MT, kPanel>(P, lds0 + k / kPanel * kPanelBytes, k, wave, lane);
     Weights<kSub / 64> ring[kRing];
     int tile = blockIdx.x;
+    auto load_step = [&](int slot, int i) { load_weights(ring[slot], P, tile + i / kSubs * (int)gridDim.x, sub_of(i % kSubs) * kSub, wave, lane); };      // step i from this tile's first on
 #pragma unroll
-    for (int r = 0; r < kFar; ++r) load_weights(ring[r], P, tile, sub_of(r) * kSub, wave, lane);
+    for (int r = 0; r < kFar; ++r) load_step(r, r);                              // (reading a tile too many is in bounds)
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");                // x is in LDS for everybody
-    for (int n = 0; n < tiles; ++n) {
-        const int next = tile + (int)gridDim.x;
-        f32x4 part[kParts][MT];
+    for (int n = 0; n < tiles; n += kTiles) {
 #pragma unroll
-        for (int i = 0; i < kSubs; ++i) {
-            if (i + kFar < kSubs || n + 1 < tiles) load_weights(ring[(i + kFar) % kRing], P, i + kFar < kSubs ? tile : next, sub_of((i + kFar) % kSubs) * kSub, wave, lane);
-            __builtin_amdgcn_sched_barrier(0);
-            const int sub = sub_of(i);
-            if (i % kEach == 0)
+        for (int u = 0; u < kTiles; ++u) {
+            if (n + u >= tiles) break;
+            f32x4 part[kParts][MT];
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) part[i / kEach][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-            multiply<MT, kPanel>(part[i / kEach], ring[i % kRing], lds + sub / 2 * kPanelBytes, (sub & 1) * (kSub / 8), lane);
-            __builtin_amdgcn_sched_barrier(0);
+            for (int i = 0; i < kSubs; ++i) {
+                const int step = u * kSubs + i, sub = sub_of(i);
+                load_step((step + kFar) % kRing, i + kFar);
+                __builtin_amdgcn_sched_barrier(0);
+                if (i % kEach == 0)
+#pragma unroll
+                    for (int mt = 0; mt < MT; ++mt) part[i / kEach][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+                multiply<MT, kPanel>(part[i / kEach], ring[step % kRing], lds + sub / 2 * kPanelBytes, (sub & 1) * (kSub / 8), lane);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                part[0][mt] += part[1][mt];
+                if constexpr (kParts == 4) part[0][mt] += part[2][mt] + part[3][mt];
+            }
+            rows.take(part[0], tile * kTileRows + wave * 16 + 4 * (lane >> 4), P.vocab);
+            tile += gridDim.x;
         }
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) part[0][mt] = (part[0][mt] + part[1][mt]) + (part[2][mt] + part[3][mt]);
-        rows.take(part[0], tile * kTileRows + wave * 16 + 4 * (lane >> 4), P.vocab);
-        tile = next;
     }
     rows.finish(P, lds, tid);
+}
+
+template <int COLUMNS> int launch(const LmHeadParams& P, hipStream_t stream)
+{
+    static std::atomic<bool> raised[64];
+    constexpr int kLdsBytes = 32 * COLUMNS * 2;
+    const int rc = mdx_tile::reserve_lds(reinterpret_cast<const void*>(lm_head_few_rows_kernel<COLUMNS>), kLdsBytes, raised, "lm_head_confidence");
+    if (rc != MDX_OK) return rc;
+    lm_head_few_rows_kernel<COLUMNS><<<(unsigned)P.n_slices, kThreads, kLdsBytes, stream>>>(P);
+    return mdx::check_launch("lm_head_confidence");
 }
 
 }  // namespace
 
 namespace mdx_head {
 
-bool few_rows_covered(int64_t rows, int64_t hidden) { return rows <= 32 && hidden == kColumns; }
+bool few_rows_covered(int64_t rows, int64_t vocab, int64_t hidden)
+{
+    if (rows > 32) return false;
+    return hidden == 2048 || ((hidden == 512 || hidden == 1024) && vocab > (int64_t)kLeastRounds * kTileRows * mdx::compute_units());
+}
 
 int launch_few_rows(LmHeadParams& P, hipStream_t stream)
 {
-    static std::atomic<bool> raised[64];
-    constexpr int kLdsBytes = 32 * kColumns * 2;
-    const int rc = mdx_tile::reserve_lds(reinterpret_cast<const void*>(lm_head_few_rows_kernel), kLdsBytes, raised, "lm_head_confidence");
-    if (rc != MDX_OK) return rc;
     P.n_vocab_tiles = (P.vocab + kTileRows - 1) / kTileRows;
     const int cus = mdx::compute_units();
     P.n_slices = P.n_vocab_tiles < cus ? P.n_vocab_tiles : cus;
-    lm_head_few_rows_kernel<<<(unsigned)P.n_slices, kThreads, kLdsBytes, stream>>>(P);
-    return mdx::check_launch("lm_head_confidence");
+    return P.hidden == 512 ? launch<512>(P, stream) : P.hidden == 1024 ? launch<1024>(P, stream) : launch<2048>(P, stream);
 }
 
 }  // namespace mdx_head

@@ -303,7 +303,7 @@ extern "C" int mdx_lm_head_confidence(const void* x, int64_t x_row_stride, const
     P.records = static_cast<Record*>(workspace);
     P.x0 = x0; P.x0_p = x0_p;
 
-    const int rc = few_rows_covered(rows, hidden) ? launch_few_rows(P, stream) : launch_product(P, stream);
+    const int rc = few_rows_covered(rows, vocab, hidden) ? launch_few_rows(P, stream) : launch_product(P, stream);
     if (rc != MDX_OK) return rc;
     lm_head_finalize_kernel<<<(unsigned)((rows + kFoldThreads / 64 - 1) / (kFoldThreads / 64)), kFoldThreads, 0, stream>>>(P);
     return mdx::check_launch("lm_head_finalize");

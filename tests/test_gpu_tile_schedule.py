@@ -80,3 +80,20 @@ def test_head_at_few_steps(dev, rows, vocab, hidden):
     assert torch.equal(x0, tx0.view(-1))
     # two sums of the same fp32 terms: 2^-24 per addition and of each exponent's argument
     assert torch.allclose(p, tp.view(-1), rtol=3e-5, atol=0)
+
+
+# up to 32 rows and rows of 512 and 1024 columns that the workgroups stream past x: from five tiles of 128 entries per CU on (131 072 entries and more), an odd number of
+# tiles in a workgroup's turn, a last tile of one entry; and both sides of that line, of 32 rows and of the widths
+@pytest.mark.parametrize("rows,vocab,hidden", [(1, 131073, 512), (17, 151936, 512), (32, 163841, 512), (16, 131073, 1024), (32, 151936, 1024), (31, 200001, 1024),
+                                               (32, 131072, 512), (33, 131073, 512), (5, 131073, 1536), (32, 300, 2048), (9, 131073, 2048)])
+def test_head_of_few_rows_at_other_widths(dev, rows, vocab, hidden):
+    import mdx
+    x, w = _integers(rows, vocab, hidden)
+    w[vocab // 2] = w[vocab - 1] = w[3]                    # equal rows: equal logits wherever they stand
+    x[0] = w[3]                                            # and of row 0 the largest: the first of them is taken
+    x, w = x.to(dev), w.to(dev)
+    x0, p = mdx.lm_head_confidence(x, w)
+    logits = (x.float() @ w.float().T).bfloat16()
+    tx0, tp = mdx.confidence_argmax(logits.unsqueeze(0))
+    assert int(x0[0]) == 3 and torch.equal(x0, tx0.view(-1))
+    assert torch.allclose(p, tp.view(-1), rtol=3e-5, atol=0)
