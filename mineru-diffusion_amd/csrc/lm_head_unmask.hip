@@ -244,21 +244,29 @@ int launch_two_steps(LmHeadParams& P, hipStream_t stream)
 // Which tile.  Up to 64 rows 64 x 128, of which two fit a CU (72 KB of LDS each), so that one's epilogue has the other's loads beside it; up to 128 rows 128 x 128.  151 936 entries, us,
 // through LDS step by step, W straight to registers (which these two replaced) / here: 2048 columns, 40 rows 140 / 125, 64 141 / 127, 80 166 / 150, 128 171 / 154; 1024 columns 69 / 58, 71 / 61, 90 /
 // 82, 91 / 85; 4096 256 / 234, 260 / 231, 314 / 258, 318 / 265.  (128 x 256: 40 rows 152, 128 159; 128 x 128 with two steps in LDS, two a CU, 128 rows 163; 64 x 128 with two steps 141.)
+// Of 65 to 128 rows, 128 x 256 where it halves the rounds (100 rows, us, 128 x 128 / so: 50 000 entries, 512 columns 26.1 / 20.8, 2048 63.9 / 59.6; 100 000, 2048 114 / 104; 4096 191 / 172), and
+// below kLongK columns, where the epilogue counts, 128 x 128 with two steps in LDS if there is more than a round of them (151 936, 100 rows, four steps / two: 256 columns 42.7 / 35.5, 384
+// 51.1 / 43.4, 640 65.1 / 59.6, 1152 92.7 / 89.8, 1280 105.7 / 106.3, 2048 154 / 165; 32 000 entries, 512 columns 15.1 / 15.9, 1024 22.9 / 26.0).
 // More rows: rounds of one workgroup per CU times what a round takes (us over 2048 columns: 256 x 256 53.5, 192 x 256 44.5), us, 256 x 256 / 192 x 256: 136 rows 186 / 170, 192 188 / 172, 256
 // 188 / 226, 300 270 / 230, 384 270 / 229, 512 274 / 312, 640 373 / 418, 768 383 / 421, 1024 522 / 584.  (128 x 256: 183, 191, 194, 245, 246, 329, 388, 445, 599; 192 x 192: 175, 180, 243, 248, 253, 346, 437,
 // 444, 620; 192 x 128, 192 rows 172; 256 x 192, 256 x 128 and 128 x 192 lie above the better of the two everywhere.)  With loads and reads in bursts behind the barriers (linear_tile.h): 136 rows 181, 192 185, 256 198,
 // 384 263, 512 304, 768 418, 1024 560.  Whole rounds in the larger tile and the rest of the vocabulary in smaller ones is level (500 rows 273.5 / 274.9): the last round's tiles run faster by themselves.
+constexpr int kLongK = 1280;
 int launch_product(LmHeadParams& P, hipStream_t stream)
 {
     if (P.hidden < 4 * kStepK) return launch_two_steps(P, stream);       // (128 columns)
     if (P.rows <= 64) return launch_tiles<64, 128, 3, 3>(P, stream);
-    if (P.rows <= 128) return launch_tiles<128, 128, 4, 4>(P, stream);
     const int cus = mdx::compute_units();
-    auto cost = [&](int bm, int bn, float round) {
+    auto rounds = [&](int bm, int bn) {
         const int64_t tiles = (int64_t)((P.rows + bm - 1) / bm) * ((P.vocab + bn - 1) / bn);
-        return (float)((tiles + cus - 1) / cus) * round;
+        return (int)((tiles + cus - 1) / cus);
     };
-    return cost(192, 256, 44.5f) < cost(256, 256, 53.5f) ? launch_tiles<192, 256, 3, 2>(P, stream) : launch_tiles<256, 256, 3, 2>(P, stream);
+    if (P.rows <= 128) {
+        const int narrow = rounds(128, 128);
+        if (narrow >= 2 * rounds(128, 256)) return launch_tiles<128, 256, 3, 3>(P, stream);
+        return narrow > 1 && P.hidden < kLongK ? launch_tiles<128, 128, 2, 2>(P, stream) : launch_tiles<128, 128, 4, 4>(P, stream);
+    }
+    return 44.5f * rounds(192, 256) < 53.5f * rounds(256, 256) ? launch_tiles<192, 256, 3, 2>(P, stream) : launch_tiles<256, 256, 3, 2>(P, stream);
 }
 
 }  // namespace

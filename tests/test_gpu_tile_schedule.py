@@ -97,3 +97,11 @@ def test_head_of_few_rows_at_other_widths(dev, rows, vocab, hidden):
     tx0, tp = mdx.confidence_argmax(logits.unsqueeze(0))
     assert int(x0[0]) == 3 and torch.equal(x0, tx0.view(-1))
     assert torch.allclose(p, tp.view(-1), rtol=3e-5, atol=0)
+
+
+# the tiles of 65 to 128 rows: two steps in LDS (a round of tiles of 128 entries and one more, widths of two whole steps of the pipeline and up to the limit), twice as wide
+# where that halves the rounds, four steps otherwise; one and two row tiles of the others
+@pytest.mark.parametrize("rows,vocab,hidden", [(65, 70001, 256), (128, 70001, 384), (100, 131073, 1152), (128, 131073, 1280), (65, 32769, 256), (128, 50001, 512), (77, 65536, 2048),
+                                               (100, 32768, 256), (128, 511, 1024)])
+def test_head_tiles_of_up_to_128_rows(dev, rows, vocab, hidden):
+    test_head_at_few_steps(dev, rows, vocab, hidden)
