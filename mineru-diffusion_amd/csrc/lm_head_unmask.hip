@@ -247,7 +247,9 @@ int launch_two_steps(LmHeadParams& P, hipStream_t stream)
 // Of 65 to 128 rows, 128 x 256 where it halves the rounds (100 rows, us, 128 x 128 / so: 50 000 entries, 512 columns 26.1 / 20.8, 2048 63.9 / 59.6; 100 000, 2048 114 / 104; 4096 191 / 172), and
 // below kLongK columns, where the epilogue counts, 128 x 128 with two steps in LDS if there is more than a round of them (151 936, 100 rows, four steps / two: 256 columns 42.7 / 35.5, 384
 // 51.1 / 43.4, 640 65.1 / 59.6, 1152 92.7 / 89.8, 1280 105.7 / 106.3, 2048 154 / 165; 32 000 entries, 512 columns 15.1 / 15.9, 1024 22.9 / 26.0).
-// More rows: rounds of one workgroup per CU times what a round takes (us over 2048 columns: 256 x 256 53.5, 192 x 256 44.5), us, 256 x 256 / 192 x 256: 136 rows 186 / 170, 192 188 / 172, 256
+// More rows: rounds of one workgroup per CU times what a round takes (us over 2048 columns: 256 x 256 53.5, 192 x 256 44.5, 128 x 256 33, 192 x 192 34; of other widths about the same to each
+// other).  The two smaller ones are for vocabularies that the larger tiles have too few of for every CU (us, without / with them: 32 000 entries, 144 rows of 512 columns 19.9 / 18.6, 192 of
+// 2048 51.1 / 44.2, 192 of 4096 87.2 / 75.5; 16 000, 192 of 2048 44.8 / 37.1).  151 936 entries, us, 256 x 256 / 192 x 256: 136 rows 186 / 170, 192 188 / 172, 256
 // 188 / 226, 300 270 / 230, 384 270 / 229, 512 274 / 312, 640 373 / 418, 768 383 / 421, 1024 522 / 584.  (128 x 256: 183, 191, 194, 245, 246, 329, 388, 445, 599; 192 x 192: 175, 180, 243, 248, 253, 346, 437,
 // 444, 620; 192 x 128, 192 rows 172; 256 x 192, 256 x 128 and 128 x 192 lie above the better of the two everywhere.)  With loads and reads in bursts behind the barriers (linear_tile.h): 136 rows 181, 192 185, 256 198,
 // 384 263, 512 304, 768 418, 1024 560.  Whole rounds in the larger tile and the rest of the vocabulary in smaller ones is level (500 rows 273.5 / 274.9): the last round's tiles run faster by themselves.
@@ -266,7 +268,10 @@ int launch_product(LmHeadParams& P, hipStream_t stream)
         if (narrow >= 2 * rounds(128, 256)) return launch_tiles<128, 256, 3, 3>(P, stream);
         return narrow > 1 && P.hidden < kLongK ? launch_tiles<128, 128, 2, 2>(P, stream) : launch_tiles<128, 128, 4, 4>(P, stream);
     }
-    return 44.5f * rounds(192, 256) < 53.5f * rounds(256, 256) ? launch_tiles<192, 256, 3, 2>(P, stream) : launch_tiles<256, 256, 3, 2>(P, stream);
+    const float large = 53.5f * rounds(256, 256), middle = 44.5f * rounds(192, 256), half = 33.f * rounds(128, 256), square = 34.f * rounds(192, 192);
+    if (half < large && half < middle && half <= square) return launch_tiles<128, 256, 3, 3>(P, stream);
+    if (square < large && square < middle) return launch_tiles<192, 192, 3, 3>(P, stream);
+    return middle < large ? launch_tiles<192, 256, 3, 2>(P, stream) : launch_tiles<256, 256, 3, 2>(P, stream);
 }
 
 }  // namespace

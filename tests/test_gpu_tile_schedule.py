@@ -105,3 +105,10 @@ def test_head_of_few_rows_at_other_widths(dev, rows, vocab, hidden):
                                                (100, 32768, 256), (128, 511, 1024)])
 def test_head_tiles_of_up_to_128_rows(dev, rows, vocab, hidden):
     test_head_at_few_steps(dev, rows, vocab, hidden)
+
+
+# vocabularies that tiles of 256 entries leave CUs empty with: 128 x 256 and 192 x 192, at their edges in rows, and both sides of a full round
+@pytest.mark.parametrize("rows,vocab,hidden", [(129, 32000, 256), (192, 32000, 2048), (256, 16001, 384), (300, 16000, 512), (150, 48000, 256), (192, 48129, 1024), (250, 65536, 256),
+                                               (193, 257, 640), (500, 8000, 256)])
+def test_head_tiles_of_small_vocabularies(dev, rows, vocab, hidden):
+    test_head_at_few_steps(dev, rows, vocab, hidden)
