@@ -199,8 +199,13 @@ constexpr TileCost tile(float step, float around) {
                          launch<BM, BN, WM, WN, WK, S, SX, kSilu>};
 }
 const TileCost kTiles[] = {
-    tile<32, 64, 2, 2, 1, 6, 6, true>(0.165f, 0.4f),         // (four steps in LDS: gate/up of 32 rows 12.66 us, down 8.33; six 12.30, 8.05)
-    tile<64, 64, 2, 2, 2, 6, 6, true>(0.223f, 0.7f),         // (four: QKV in two slices, 96 rows 8.52, down 64 rows 8.43; six 8.02, 8.17)
+    // The two smallest hold four steps in LDS or six.  Six are the faster where a slice has as many and W comes from HBM (us, four / six: gate/up of 32 rows 12.66 / 12.30, down 8.33 / 8.05,
+    // QKV of 96 rows in two slices 8.52 / 8.02; W from the memory-side cache, 512 columns of K, 3.7 / 3.8), but K of 256, and K cut into slices of four steps, would go to larger tiles without four:
+    // 32 rows x 1024 x 256 3.1 / 4.1, 128 rows 3.1 / 4.8; 32 rows x 1024 x 1024 with the reading of the sums 3.2 / 3.8, 32 rows x 2048 x 2048 4.7 / 5.0.
+    tile<32, 64, 2, 2, 1, 4, 4, true>(0.173f, 0.4f),
+    tile<32, 64, 2, 2, 1, 6, 6, true>(0.165f, 0.4f),
+    tile<64, 64, 2, 2, 2, 4, 4, true>(0.233f, 0.7f),
+    tile<64, 64, 2, 2, 2, 6, 6, true>(0.223f, 0.7f),
     tile<128, 64, 2, 2, 2, 4, 4, true>(0.326f, 1.7f),
     tile<192, 64, 2, 2, 2, 4, 4, true>(0.408f, 2.9f),
     tile<128, 128, 2, 2, 2, 4, 4, true>(0.487f, 2.6f),

@@ -35,6 +35,13 @@ def test_products_at_few_steps(dev, rows, n, k):
         assert torch.equal(parts.sum(0).bfloat16(), want)
 
 
+# slices of four and five steps, six and more: both depths of the two smallest tiles, at their edges in rows
+@pytest.mark.parametrize("rows,n,k", [(1, 64, 256), (32, 72, 256), (33, 1024, 256), (64, 520, 256), (128, 512, 512), (17, 1024, 640), (32, 2048, 2048), (64, 1032, 1024), (65, 512, 1280),
+                                      (160, 512, 384), (48, 1024, 3072)])
+def test_products_of_the_small_tiles(dev, rows, n, k):
+    test_products_at_few_steps(dev, rows, n, k)
+
+
 @pytest.mark.parametrize("rows,n,k,taken", [(8193, 1024, 512, True), (8400, 2056, 640, True), (8193, 1016, 512, False), (8193, 1024, 1152, False)])
 def test_gated_product_of_many_rows(dev, rows, n, k, taken):
     """Beyond 8192 rows the gated product is taken where W's halves are no narrower than 1024 and K: the two steps' result."""
