@@ -181,31 +181,33 @@ int launch(LinearParams A, hipStream_t stream)
 }
 
 // The tiles there are, and what a round of them costs: a step of K and what stands before and behind the steps, us, fitted to
-// 1700 timings with cold weights (four projections of the decoder, 32 to 8192 rows, every tile, 1 to 32 slices of K).
+// 1700 timings with cold weights (four projections of the decoder, 32 to 8192 rows, every tile, 1 to 32 slices of K) and held against 1486 shapes of other widths (K of 256 to 6144,
+// 1024 to 12 288 columns, 16 to 1536 rows).  Small tiles that leave no room on the CU for the next round's, or share its intake with them, cost more from the second round
+// on: 320 rows x 6144 x 2048 as 480 tiles of 64 x 64 with six steps 22.5 us, as 192 of 192 x 64 18.6; 160 x 6144 x 6144 as 480 of 32 x 64 42.3, as 192 of 128 x 64 35.0.
 struct TileCost {
     int bm, bn, least_steps, steps_multiple;                // steps of 64 elements of K: at least, and a multiple of
-    float step, around;
+    float step, around, again;                              // again: how much more every round costs where there are several
     int (*rounded)(LinearParams, hipStream_t);
     int (*partials)(LinearParams, hipStream_t);             // none for the tiles that only many rows fill
     int (*silu)(LinearParams, hipStream_t);
 };
 template <int BM, int BN, int WM, int WN, int WK, int S, int SX, bool PARTIALS>
-constexpr TileCost tile(float step, float around) {
+constexpr TileCost tile(float step, float around, float again = 1.f) {
     typedef Tile<BM, BN, WM, WN, WK, S, SX, false> T;
     // (a slice has four steps at least: rows that are too far apart for the plan's tile go to one that loads four ahead, run_partials)
-    if constexpr (PARTIALS) return TileCost{BM, BN, T::kLeastSteps < 4 ? 4 : T::kLeastSteps, T::kStepsMultiple, step, around, launch<BM, BN, WM, WN, WK, S, SX, kRounded>,
+    if constexpr (PARTIALS) return TileCost{BM, BN, T::kLeastSteps < 4 ? 4 : T::kLeastSteps, T::kStepsMultiple, step, around, again, launch<BM, BN, WM, WN, WK, S, SX, kRounded>,
                                             launch<BM, BN, WM, WN, WK, S, SX, kPartials>, launch<BM, BN, WM, WN, WK, S, SX, kSilu>};
-    else return TileCost{BM, BN, T::kLeastSteps, T::kStepsMultiple, step, around, launch<BM, BN, WM, WN, WK, S, SX, kRounded>, nullptr,
+    else return TileCost{BM, BN, T::kLeastSteps, T::kStepsMultiple, step, around, again, launch<BM, BN, WM, WN, WK, S, SX, kRounded>, nullptr,
                          launch<BM, BN, WM, WN, WK, S, SX, kSilu>};
 }
 const TileCost kTiles[] = {
     // The two smallest hold four steps in LDS or six.  Six are the faster where a slice has as many and W comes from HBM (us, four / six: gate/up of 32 rows 12.66 / 12.30, down 8.33 / 8.05,
     // QKV of 96 rows in two slices 8.52 / 8.02; W from the memory-side cache, 512 columns of K, 3.7 / 3.8), but K of 256, and K cut into slices of four steps, would go to larger tiles without four:
     // 32 rows x 1024 x 256 3.1 / 4.1, 128 rows 3.1 / 4.8; 32 rows x 1024 x 1024 with the reading of the sums 3.2 / 3.8, 32 rows x 2048 x 2048 4.7 / 5.0.
-    tile<32, 64, 2, 2, 1, 4, 4, true>(0.173f, 0.4f),
-    tile<32, 64, 2, 2, 1, 6, 6, true>(0.165f, 0.4f),
+    tile<32, 64, 2, 2, 1, 4, 4, true>(0.173f, 0.4f, 1.1f),
+    tile<32, 64, 2, 2, 1, 6, 6, true>(0.165f, 0.4f, 1.1f),
     tile<64, 64, 2, 2, 2, 4, 4, true>(0.233f, 0.7f),
-    tile<64, 64, 2, 2, 2, 6, 6, true>(0.223f, 0.7f),
+    tile<64, 64, 2, 2, 2, 6, 6, true>(0.223f, 0.7f, 1.1f),
     tile<128, 64, 2, 2, 2, 4, 4, true>(0.326f, 1.7f),
     tile<192, 64, 2, 2, 2, 4, 4, true>(0.408f, 2.9f),
     tile<128, 128, 2, 2, 2, 4, 4, true>(0.487f, 2.6f),
@@ -222,7 +224,7 @@ struct Plan { const TileCost* tile; int splits; double cost; };
 // The cheapest tile and number of slices by the costs above, in rounds of one workgroup per CU (the small tiles' second one
 // per CU is worth little: they share its intake).  Partial sums cost their writing and the next kernel's reading, 0.35 us per
 // MB together (5.7 TB/s), a rounded result less than half of that per element.  Against the best of all timed choices this
-// costs 0.3 % on average and 4 % at most.
+// costs 0.3 % on average and 4 % at most at the decoder's widths, 0.6 % on average and 16 % at most at the others.
 Plan plan_of(int64_t rows, int64_t n, int64_t k, bool rounded, bool partials, bool silu)
 {
     Plan best{nullptr, 0, 0};
@@ -235,7 +237,7 @@ Plan plan_of(int64_t rows, int64_t n, int64_t k, bool rounded, bool partials, bo
             const double steps = (double)(k / kStepK / s), rounds = (double)((tiles * s + cus - 1) / cus);
             for (int form = 0; form < 2; ++form) {                                  // 0: rounded or SiLU, 1: partial sums
                 if (form == 0 ? (s > 1 || !(rounded || silu)) : (!partials || !t.partials)) continue;
-                const double cost = rounds * (steps * t.step + t.around) + (form ? 0.35 * (double)s : 0.15) * mb;
+                const double cost = rounds * (steps * t.step + t.around) * (rounds > 1 ? t.again : 1.f) + (form ? 0.35 * (double)s : 0.15) * mb;
                 if (!best.tile || cost < best.cost) best = Plan{&t, form ? (int)s : 0, cost};
             }
         }

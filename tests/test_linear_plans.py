@@ -25,3 +25,8 @@ def test_small_tiles_keep_slices_of_four_steps():
     for rows, n, k, slices in ((32, 512, 512, 2), (8, 1024, 1024, 4), (32, 1024, 2048, 8), (64, 512, 1024, 4), (32, 2048, 2048, 8), (128, 512, 512, 2)):
         assert L.mdx_decode_linear_splits(rows, n, k) == slices, (rows, n, k)
         assert L.mdx_linear_splits(rows, n, k) == slices, (rows, n, k)
+
+
+def test_second_rounds_of_small_tiles_are_not_taken_for_free():
+    """480 tiles of 32 x 64 would be two rounds on 256 CUs: two slices of K in larger tiles, which are one."""
+    assert mdx._lib.lib().mdx_linear_splits(160, 6144, 2048) == 2
