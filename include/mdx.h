@@ -332,6 +332,7 @@ int mdx_unmask_step(const void* logits, int64_t row_stride, int32_t dtype,
  * are left zero by every call that completes; calls that may run at the same time (different streams) need counters of their own.
  */
 int64_t mdx_unmask_step_counter_bytes(int32_t bs, int32_t block_len);
+int32_t mdx_unmask_step_single_launch_pays(int32_t bs, int32_t block_len, int64_t vocab, int32_t seeded);   /* 0: the two launches are faster, and mdx.unmask_step makes those */
 int mdx_unmask_step_single_launch(const void* logits, int64_t row_stride, int32_t dtype,
                                   const float* temperatures, const float* noise, int64_t noise_row_stride,
                                   int32_t seeded, uint64_t seed, uint64_t offset, const int64_t* offset_dev,
@@ -372,7 +373,7 @@ int mdx_unmask_step_gumbel(const void* logits, int64_t row_stride, int32_t dtype
  * mdx_unmask_step (or, seeded, mdx_unmask_step_gumbel) on blocks in host memory that the GPU reaches (pinned), for a caller that wants the blocks, the flags and the
  * counts: which positions are masked is read here, and only their rows are computed.  tokens must hold its values when the call is made and may be written by the
  * GPU until the stream is done.  The workspace (16-byte aligned) holds the confidences as well.  _single_launch: with counters as in
- * mdx_unmask_step_single_launch; a call with a sequence that has nothing masked makes two launches.
+ * mdx_unmask_step_single_launch; a call with a sequence that has nothing masked, or where two are faster, makes two launches.
  */
 int64_t mdx_unmask_step_host_blocks_workspace_bytes(int64_t rows, int64_t vocab);
 int mdx_unmask_step_host_blocks(const void* logits, int64_t row_stride, int32_t dtype,

@@ -854,7 +854,8 @@ void step(const Tensor& logits, int64_t bs, int64_t S, int64_t* tokens, int64_t 
     }
     const int64_t bytes = mdx_confidence_argmax_workspace_bytes(l.rows, l.vocab);
     const Tensor ws = bytes > 0 ? make(logits, at::kByte, bytes) : Tensor();
-    const Tensor counters = eager_counters(logits, mdx_unmask_step_counter_bytes((int32_t)bs, (int32_t)S));
+    const bool one = mdx_unmask_step_single_launch_pays((int32_t)bs, (int32_t)S, l.vocab, z.seeded ? 1 : 0) != 0;
+    const Tensor counters = one ? eager_counters(logits, mdx_unmask_step_counter_bytes((int32_t)bs, (int32_t)S)) : Tensor();
     check(mdx_unmask_step_single_launch(ptr(l.t), l.stride, dtype_of(logits), static_cast<const float*>(ptr_or_null(t)), z.data(), z.data() ? l.vocab : 0,
                                         z.seeded ? 1 : 0, z.seed, z.offset, static_cast<const int64_t*>(ptr_or_null(z.offset_dev)), tokens, mask_id,
                                         threshold, k, x0, x0_p, transfer, count, (int32_t)bs, (int32_t)S, l.vocab, ptr_or_null(ws), bytes,

@@ -223,8 +223,7 @@ __device__ __forceinline__ Partial merge_splits(const Partial* __restrict__ part
 
 // The end of a workgroup of the vocabulary pass that selects by itself: the last one of a sequence to arrive merges its rows' splits and applies
 // the rule.  No workgroup waits for another; what the last one reads of the others was in memory before they arrived.  own: in thread 0, what the workgroup has found.
-// Three trips to memory (store, arrival, merge) take the GPU about as long as a second launch does, and the host 3.5 us less.  The step, us, two launches / one: 1 sequence
-// 15.7 / 13.4, 3 15.7 / 14.5, 5 16.6 / 15.8, 8 19.1 / 18.3, 16 30.0 / 29.5, 32 51.6 / 50.9; sampled, where the pass itself takes longer than the host, 3 25.6 / 25.6, 32 112.0 / 111.8.
+// Three trips to memory (store, arrival, merge) take the GPU about as long as a second launch does, and the host 2 to 3.5 us less (one_launch_pays has where they don't).
 // (A counter per row as well, and a merge per row, was a trip more: 5 sequences 16.2, 8 18.6.)
 template <bool NOISE, bool LIVE>
 __device__ __forceinline__ void select_when_last(const Selection& S, const Partial& own, int row, int split, float c, int nsplit, Partial* partials, int64_t* x0, float* x0_p)
@@ -940,6 +939,27 @@ extern "C" int mdx_select_transfer(const int64_t* x0, const float* x0_p, int64_t
                          transfer, count, bs, block_len, stream);
 }
 
+namespace {
+
+// Whether the vocabulary pass of so many rows better selects by itself.  Not where the rows are many and short: the ends of the workgroups, three trips to memory, then hold up those
+// that wait for their place (blocks of 32, us on the GPU, two launches / one: 200 blocks of 1000 entries 14.6 / 16.9, of 16 000 40.2 / 41.5, 64 of 1000 sampled 13.3 / 15.1; 64 of 4000
+// 9.9 / 9.9, of 151 936 100.8 / 99.1).  Nor where a counter has more arrivals than the pass itself covers (151 936 entries in 9 splits: 1 block of 32, 288 arrivals, 9.6 / 12.6, 2 10.8 / 13.1,
+// 3 12.3 / 14.0; of 64, 576, 10.9 / 18.2; in 8, 256 arrivals, 4 blocks of 32 12.4 / 12.2); draws take longer than their arrivals (1 block of 32 18.5 / 17.8, of 64 21.7 / 20.6).
+// Elsewhere: 8 blocks of 32 18.5 / 18.2, 16 30.0 / 29.3, 32 51.8 / 51.4; 64 000 entries 1 block 9.2 / 9.5, and with the host's part, which the step of few rows waits for, 11.4 / 9.3.
+constexpr int kMostArrivals = 256, kFewRows = 1024, kManyRows = 2048, kShortRow = 4096;
+bool one_launch_pays(int64_t rows, int32_t block_len, int64_t vocab, bool seeded)
+{
+    if (rows < 1 || rows > kManyRows || (rows > kFewRows && vocab < kShortRow)) return false;
+    return seeded || (int64_t)block_len * pick_nsplit(rows, vocab) <= kMostArrivals;
+}
+
+}  // namespace
+
+extern "C" int32_t mdx_unmask_step_single_launch_pays(int32_t bs, int32_t block_len, int64_t vocab, int32_t seeded)
+{
+    return bs > 0 && block_len > 0 && block_len <= mdx::kWave && vocab > 0 && one_launch_pays((int64_t)bs * block_len, block_len, vocab, seeded != 0);
+}
+
 extern "C" int64_t mdx_unmask_step_counter_bytes(int32_t bs, int32_t block_len)
 {
     if (bs <= 0 || block_len <= 0) return 0;
@@ -1081,7 +1101,7 @@ extern "C" int64_t mdx_unmask_step_host_blocks_workspace_bytes(int64_t rows, int
 
 extern "C" int64_t mdx_unmask_step_host_blocks_counter_bytes(int32_t bs, int32_t block_len)
 {
-    return (int64_t)bs * block_len < kSingleLaunchRows ? 0 : mdx_unmask_step_counter_bytes(bs, block_len);
+    return (int64_t)bs * block_len < kSingleLaunchRows || (int64_t)bs * block_len > kManyRows ? 0 : mdx_unmask_step_counter_bytes(bs, block_len);
 }
 
 extern "C" int mdx_unmask_step_host_blocks_single_launch(const void* logits, int64_t row_stride, int32_t dtype,
@@ -1114,6 +1134,7 @@ extern "C" int mdx_unmask_step_host_blocks_single_launch(const void* logits, int
         // rows are as quick in two (us, two launches / one: 32 rows 24.5 / 26, 96 40.8 / 41.0, 192 36.1 / 35.4, 576 63.1 / 62.7).
         if (with_rows < bs || n_live < kSingleLaunchRows) counters = nullptr;
     }
+    if (!one_launch_pays(rows <= kMaxLiveRows ? n_live : rows, block_len, vocab, seeded != 0)) counters = nullptr;
     const NoiseSpec N = seeded ? generator_noise(seed, offset, offset_dev, nullptr) : tensor_noise(noise, noise_row_stride);
     int64_t* x0 = static_cast<int64_t*>(workspace);
     char* splits = static_cast<char*>(workspace) + confidences_bytes(rows);

@@ -49,6 +49,7 @@ SIGNATURES = {
     "mdx_unmask_step_host_blocks_single_launch": (c_int32, [_P, _I64, _I32, _P, _P, _I64, _I32, _U64, _U64, _P, _P, _I64, _F, _I32, _P, _P, _I32, _I32, _I64,
                                                             _P, _I64, _P, _I64, _P]),
     "mdx_unmask_step_counter_bytes": (c_int64, [_I32, _I32]),
+    "mdx_unmask_step_single_launch_pays": (c_int32, [_I32, _I32, _I64, _I32]),
     "mdx_unmask_step_host_blocks_counter_bytes": (c_int64, [_I32, _I32]),
     "mdx_unmask_step_single_launch": (c_int32, [_P, _I64, _I32, _P, _P, _I64, _I32, _U64, _U64, _P, _P, _I64, _F, _I32, _P, _P, _P, _P, _I32, _I32, _I64,
                                                 _P, _I64, _P, _I64, _P]),

@@ -103,3 +103,28 @@ def test_captured_step_keeps_no_counters(dev):
         assert torch.equal(block, want)
         for a, b in zip(out, eager):
             assert torch.equal(a, b)
+
+
+# counters that a call is given are used whatever mdx.unmask_step would choose: many arrivals at one, many rows, and what lies between
+@pytest.mark.parametrize("bs, S, V", [(1, 32, 151936), (1, 64, 151936), (3, 48, 151936), (80, 32, 1000), (70, 32, 5000), (4, 64, 151936)])
+@pytest.mark.parametrize("seed", [None, 5])
+def test_given_counters_are_used(dev, bs, S, V, seed):
+    import mdx
+    L = mdx.lib()
+    counters = torch.zeros(L.mdx_unmask_step_counter_bytes(bs, S) // 4, dtype=torch.int32, device=dev)
+    for call in range(2):
+        logits, tokens, temps = _data(bs, S, V, torch.bfloat16, 50 * call + bs)
+        logits, temps = logits.to(dev), temps.to(dev)
+        one, two = tokens.to(dev), tokens.to(dev)
+        x0, p = torch.empty(bs, S, dtype=torch.int64, device=dev), torch.empty(bs, S, device=dev)
+        transfer, count = torch.empty(bs, S, dtype=torch.bool, device=dev), torch.empty(bs, dtype=torch.int32, device=dev)
+        n = L.mdx_confidence_argmax_workspace_bytes(bs * S, V)
+        ws = torch.empty(max(n, 16), dtype=torch.uint8, device=dev)
+        rc = L.mdx_unmask_step_single_launch(logits.data_ptr(), V, 0, temps.data_ptr(), None, 0, int(seed is not None), seed or 0, 3, None, one.data_ptr(), MASK_ID, 0.9, 2,
+                                             x0.data_ptr(), p.data_ptr(), transfer.data_ptr(), count.data_ptr(), bs, S, V, ws.data_ptr(), n,
+                                             counters.data_ptr(), counters.nbytes, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, L.mdx_last_error()
+        ex0, ep, et, ec = _two_launches(logits, two, temps, seed, 3, 0.9, 2)
+        torch.cuda.synchronize()
+        assert torch.equal(x0, ex0) and torch.equal(p, ep) and torch.equal(transfer, et) and torch.equal(count, ec) and torch.equal(one, two)
+        assert not bool(counters.any())
