@@ -314,7 +314,7 @@ __device__ __forceinline__ void select_when_last(const Selection& S, const Parti
 // NOISE: 0 = plain argmax, 1 = noise read from a tensor, 2 = noise drawn in the kernel.
 // FLOOR: elements below floors[row] count as -inf (what a top-k / top-p filter would have left of the row).
 // LIVE: none, or LiveRows: only those rows.
-// With S.arrive the launch selects as well.
+// With S.arrive the launch selects as well (never with floors: the filtered step selects in a launch of its own).
 template <typename T, int NOISE, bool FLOOR, typename... LIVE>
 __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
     const LIVE... live, const T* __restrict__ logits, int64_t row_stride,
@@ -589,7 +589,9 @@ __global__ __launch_bounds__(kThreads) void confidence_argmax_kernel(
 #pragma unroll
         for (int w = 1; w < kThreads / mdx::kWave; ++w) combine(r, wave_part[w], c, NOISE != 0);
     }
-    if (S.arrive) { select_when_last<(NOISE != 0), (sizeof...(LIVE) > 0)>(S, r, (int)row32, split, c, nsplit, partials, x0, x0_p); return; }
+    if constexpr (!FLOOR) {
+        if (S.arrive) { select_when_last<(NOISE != 0), (sizeof...(LIVE) > 0)>(S, r, (int)row32, split, c, nsplit, partials, x0, x0_p); return; }
+    }
     if (tid != 0) return;
     if (nsplit > 1) {
         partials[row * nsplit + split] = r;
