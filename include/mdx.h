@@ -61,7 +61,8 @@ const char* mdx_last_error(void);  /* thread-local; valid until the next failing
  * elements; rows themselves are dense (attention.py:36-38).  elem_size is in
  * bytes (2 for bf16/f16).  Slots outside [0, num_slots) are skipped instead
  * of written (the reference leaves them undefined); num_slots = pages*page.
- * If two tokens name the same slot the result holds one of the two rows.
+ * If two tokens name the same slot the result holds one of the two rows.  key
+ * and value hold n_tokens rows; those of skipped tokens may be read as well.
  */
 int mdx_store_kvcache(const void* key, const void* value,
                       int64_t k_row_stride, int64_t v_row_stride,

@@ -17,6 +17,12 @@ constexpr int kThreads = 256;
 
 // Fast path: rows are multiples of 16 B, all bases and strides 16-B aligned.
 // grid = (tokens, 2): blockIdx.y 0 copies the token's K row, 1 its V row.
+// EARLY: the row is on its way before its slot is known, one trip to memory instead of two; rows that no slot takes are read in vain.  For launches whose workgroups
+// are all on the chip at once, where that trip is what counts and such rows keep nobody waiting.  (us, the slot first / so: the store and the attention of one block behind 16 x 2300
+// keys 43.2 / 43.0, fp32, 1056 keys 20.1 / 19.8; 1024 tokens 3.36 / 3.25, half of them without a slot 2.83 / 2.90, none with one 2.16 / 2.25; but 2048 tokens 4.73 / 4.56,
+// 3.74 / 3.78, 2.50 / 2.84, and 38 434 57.9 / 58.2, 31.4 / 44.7, 17.8 / 26.2.)
+constexpr int64_t kEarlyTokens = 1024;
+template <bool EARLY>
 __global__ __launch_bounds__(kThreads) void store_kvcache_vec16(
     const u32x4* __restrict__ key, const u32x4* __restrict__ value,
     int64_t k_stride16, int64_t v_stride16,
@@ -24,15 +30,15 @@ __global__ __launch_bounds__(kThreads) void store_kvcache_vec16(
     const int32_t* __restrict__ slot_mapping,
     int row16, int64_t num_slots)
 {
-    // The row is on its way before its slot is known: one trip to memory instead of two.  (us, the other way round / so: the store and the attention of one
-    // block behind 16 x 2300 keys 43.2 / 43.0, 64 x 800 57.0 / 56.5; 38 434 tokens 51.7 / 50.6.  Both rows of a token in one workgroup: 51.8.)
     const int64_t tok = blockIdx.x;
     const bool is_v = blockIdx.y != 0;
     const u32x4* src = is_v ? value + tok * v_stride16 : key + tok * k_stride16;
     int c = threadIdx.x;
-    u32x4 x = c < row16 ? __builtin_nontemporal_load(src + c) : u32x4{0, 0, 0, 0};
+    u32x4 x{0, 0, 0, 0};
+    if (EARLY && c < row16) x = __builtin_nontemporal_load(src + c);
     const int64_t s = slot_mapping[tok];
     if (s < 0 || s >= num_slots) return;
+    if (!EARLY && c < row16) x = __builtin_nontemporal_load(src + c);
     u32x4* dst = (is_v ? v_cache : k_cache) + s * row16;
     while (c < row16) {
         __builtin_nontemporal_store(x, dst + c);
@@ -91,7 +97,7 @@ extern "C" int mdx_store_kvcache(const void* key, const void* value,
         // one lane per 16-byte chunk of the row, in whole wavefronts, up to 256 lanes (longer rows loop)
         int threads = (row16 + mdx::kWave - 1) / mdx::kWave * mdx::kWave;
         if (threads > kThreads) threads = kThreads;
-        store_kvcache_vec16<<<dim3((unsigned)n_tokens, 2), threads, 0, stream>>>(
+        (n_tokens <= kEarlyTokens ? store_kvcache_vec16<true> : store_kvcache_vec16<false>)<<<dim3((unsigned)n_tokens, 2), threads, 0, stream>>>(
             (const u32x4*)key, (const u32x4*)value, ks16, vs16, (u32x4*)k_cache, (u32x4*)v_cache,
             slot_mapping, row16, num_slots);
     } else {

@@ -125,3 +125,11 @@ def test_store_full_size_round_trip(dev):
     assert torch.equal(kc.view(-1, hkv, d)[slots.long()], key)
     assert torch.equal(vc.view(-1, hkv, d)[slots.long()], value)
     assert int((kc.view(-1, hkv * d).float().abs().sum(1) > 0).sum()) <= N   # nothing else touched
+
+
+# both sides of the number of tokens up to which a row is read before its slot is known; rows of one lane, of a workgroup's lanes, and beyond them; none, some and all skipped
+@pytest.mark.parametrize("N", [1024, 1025])
+@pytest.mark.parametrize("hkv,d", [(1, 8), (8, 128), (3, 1000)])
+@pytest.mark.parametrize("skipped", [0.0, 0.5, 1.1])
+def test_store_row_before_its_slot(dev, N, hkv, d, skipped):
+    _case(dev, N, hkv, d, pages=9, page=256, seed=N + d, frac_skip=skipped)
