@@ -203,8 +203,9 @@ constexpr TileCost tile(float step, float around, float again = 1.f) {
 const TileCost kTiles[] = {
     // The two smallest hold four steps in LDS or six.  Six are the faster where a slice has as many and W comes from HBM (us, four / six: gate/up of 32 rows 12.66 / 12.30, down 8.33 / 8.05,
     // QKV of 96 rows in two slices 8.52 / 8.02; W from the memory-side cache, 512 columns of K, 3.7 / 3.8), but K of 256, and K cut into slices of four steps, would go to larger tiles without four:
-    // 32 rows x 1024 x 256 3.1 / 4.1, 128 rows 3.1 / 4.8; 32 rows x 1024 x 1024 with the reading of the sums 3.2 / 3.8, 32 rows x 2048 x 2048 4.7 / 5.0.
-    tile<32, 64, 2, 2, 1, 4, 4, true>(0.173f, 0.4f, 1.1f),
+    // 32 rows x 1024 x 256 3.1 / 4.1, 128 rows 3.1 / 4.8.  Slices of four steps are for few sums: with the norm behind them, us, half as many with six / so: 32 rows x 1024 x 1024 6.50 / 6.06, x 2048
+    // 6.65 / 6.39, 16 rows less; but 32 rows x 2048 x 2048 7.98 / 8.15, 64 rows 8.42 / 9.39 (the first tile's 0.7).
+    tile<32, 64, 2, 2, 1, 4, 4, true>(0.173f, 0.7f, 1.04f),
     tile<32, 64, 2, 2, 1, 6, 6, true>(0.165f, 0.4f, 1.1f),
     tile<64, 64, 2, 2, 2, 4, 4, true>(0.233f, 0.7f),
     tile<64, 64, 2, 2, 2, 6, 6, true>(0.223f, 0.7f, 1.1f),

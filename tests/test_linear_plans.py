@@ -22,7 +22,7 @@ def test_slices_have_four_steps_and_more():
 def test_small_tiles_keep_slices_of_four_steps():
     """Few rows and columns fill few CUs: K is cut down to the four steps that the smaller depth of the small tiles takes."""
     L = mdx._lib.lib()
-    for rows, n, k, slices in ((32, 512, 512, 2), (8, 1024, 1024, 4), (32, 1024, 2048, 8), (64, 512, 1024, 4), (32, 2048, 2048, 8), (128, 512, 512, 2)):
+    for rows, n, k, slices in ((32, 512, 512, 2), (8, 1024, 1024, 4), (32, 1024, 2048, 8), (64, 512, 1024, 4), (16, 2048, 2048, 8), (128, 512, 512, 2), (32, 2048, 2048, 4)):
         assert L.mdx_decode_linear_splits(rows, n, k) == slices, (rows, n, k)
         assert L.mdx_linear_splits(rows, n, k) == slices, (rows, n, k)
 
