@@ -328,7 +328,7 @@ def run_cfg5(dev, layers=28, batch=32, new_tokens=2048, steps_per_block=8, maske
                ms_per_decode_pass=round(st["decode_s"] / max(1, st["decode_passes"]) * 1e3, 3), layers=layers,
                vocabulary_projection=("rows of still-masked positions only (the unmask rule reads no others; same tokens)"
                                       if masked_rows_only else "all 32 positions of every block, as the reference computes them"),
-               model="random-init 28-layer SDAR-shaped decoder, libmdx attention, KV store, unmask, norms and linear layers (of more than 1536 rows the gate/up projection; the others: stock PyTorch-ROCm GEMMs)")
+               model="random-init 28-layer SDAR-shaped decoder, libmdx attention, KV store, unmask, norms and linear layers (of more than 1536 rows, at these widths, the gate/up projection; the others: stock PyTorch-ROCm GEMMs)")
     del eng, model
     torch.cuda.empty_cache()
     return out

@@ -320,10 +320,10 @@ int run_rows(const char* what, bool any_stride, bool silu, const void* x, int64_
 }
 
 // Where the kernel is the better one (table at the top of this file): up to 1536 rows; with the SiLU in the epilogue, which
-// saves writing and reading twice the result, all of them.  Other widths, us, here / library's product: 5120 x 5120, 1024 rows (54 GFLOP) 58.1 / 61.1, 1280 77.1 / 71.7;
+// saves writing and reading twice the result, up to 8192, and beyond where W is wide.  Other widths, us, here / library's product: 5120 x 5120, 1024 rows (54 GFLOP) 58.1 / 61.1, 1280 77.1 / 71.7;
 // 7168 x 5120, 512 (38) 51.3 / 49.4, 1280 (94) 101 / 85; 8192 x 8192, 384 (52) 59.6 / 64.3, 768 (103) 94.4 / 97.4, 1024 (137) 141 / 116; 6144 x 4096, 1024 (52) 52.5 / 51.7, 1280 (64)
 // 68.2 / 57.3: from 52 GFLOP on the library's tiles come to their rate.  Where K is long beside n they do not: 5120 x 17408, 1024 rows (183) 173 / 244, 4096 x 12288, 768 (77) 77 / 90.
-// With the SiLU, beyond 8192 rows as well where W's halves are no narrower than K and 1024 (n x k, here / library's product and SiLU, us): 35 840 rows, 6144 x 2048 1410 / 1494, 1024 x 512
+// Beyond 8192 rows it is where W's halves are no narrower than K and 1024 (n x k, here / library's product and SiLU, us): 35 840 rows, 6144 x 2048 1410 / 1494, 1024 x 512
 // 102 / 166, 3072 x 1024 428 / 486, 8960 x 1536 1600 / 1819, 8192 x 3072 2608 / 2676, 12288 x 4096 5205 / 5281; 16 384 rows, 17408 x 5120 4000 / 4466; but 2048 x 8192 787 / 741.
 constexpr int64_t kMaxRows = 1536, kMaxSiluRows = 8192, kLeastSiluWidth = 1024;
 bool silu_pays(int64_t rows, int64_t n, int64_t k) { return rows <= kMaxSiluRows || (n >= kLeastSiluWidth && n >= k); }

@@ -10,7 +10,7 @@
 //    (global_load_lds); the 16-byte chunk c of row r sits at c ^ (r / 2 % 8), so that the 16 rows of a fragment read cover all
 //    banks once.  One barrier per step: behind it the next step is in LDS for everybody and nobody reads this one any more.
 //  * the fragments of the next half step are on their way from LDS while this one is multiplied (two register sets).
-//  * loads and fragment reads stand between the products, each at its place (sched_barrier): as a burst behind the barrier, where the compiler leaves them, 64 loads
+//  * loads and fragment reads stand between the products, each at its place (sched_barrier; with fewer than eight products per wavefront and half step all of them before the first): as a burst behind the barrier, where the compiler leaves them, 64 loads
 //    of 1 KB keep the CU's address unit busy for over 1000 cycles, and the products behind them wait to be issued, in all wavefronts at once.  In bursts / between the
 //    products, with W from HBM, us: gate/up projection with its SiLU, 1024 rows 51.5 / 45.1, 2048 102 / 88, 4096 183 / 163, 35 840 1480 / 1360; 128 x 128 tiles, 1024 x 2048 x 6144
 //    34.5 / 30; smaller tiles 0 to 5 % less; the head's 500 rows 304 / 277.

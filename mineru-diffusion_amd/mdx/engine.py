@@ -12,7 +12,7 @@ kernels can be driven exactly as the engine drives them:
                                   layers/rotary_embedding.py:6-48, layers/embed_head.py:61-67
 
 The decoder is a random-init scaffold; attention, the KV store, the norms, the activation, the unmask step and the
-linear layers of up to 1536 rows (gate/up: all) go through libmdx, the other GEMMs are stock PyTorch (library) GEMMs.  Decode passes can
+linear layers of up to 1536 rows (gate/up: 8192, and any number at these widths) go through libmdx, the other GEMMs are stock PyTorch (library) GEMMs.  Decode passes can
 replay a captured HIP graph (model_runner.py:198-259).  There is no vision tower, tokenizer,
 weight loader or tensor parallelism here.
 """
@@ -323,10 +323,10 @@ class Decoder(nn.Module):
 # ----------------------------------------------------------------------------- engine
 IDLE, DENOISING, CACHING = 0, 1, 2      # MDX_PHASE_* of include/mdx.h: the per-lane state of the device loop
 N_STOP = 4                              # stop-token ids per sequence that the device loop can check
-# rows of a pass from which, and up to which, the fused vocabulary head is taken.  Fused / library product + vocabulary pass, us: 192 rows 181 / 199, 256 195 / 220,
-# 272 258 / 244, 320 258 / 255, 352 263 / 275, 383 262 / 277, 512 305 / 342
+# rows of a pass from which, and up to which, the fused vocabulary head is taken.  Fused / library product + vocabulary pass, us: 192 rows 172 / 199, 256 188 / 220,
+# 272 230 / 244, 320 230 / 255, 352 230 / 275, 383 229 / 277, 512 280 / 342: between them the fused head is the faster as well since its tiles are those of linear_tile.h
 FUSED_HEAD_MIN_ROWS, FUSED_HEAD_FEW_ROWS = 384, 256
-FUSED_HEAD_WHOLE_ROWS = 32              # rows that it holds whole (8 rows 120 us, 32 rows 119); compacting takes six launches of a pass, 63.9 against 63.4 ms for one request
+FUSED_HEAD_WHOLE_ROWS = 32              # rows that it holds whole (12 rows 109 us, 32 rows 110); compacting takes six launches of a pass, 63.9 against 63.4 ms for one request
 
 
 class _PagesShort(Exception):
@@ -662,8 +662,8 @@ class BlockDiffusionEngine:
 
     def _fused_head(self, rows: int) -> bool:
         """Projection and confidence in one pass that never writes the logits (mdx_lm_head_confidence), for bf16 weights
-        without sampling noise.  By default from 384 rows on and up to 256; between them the library GEMM + the vocabulary pass
-        (272 to 383 rows 0.244 to 0.277 ms against 0.23: the limits are older than the head's present tiles).
+        without sampling noise.  By default from 384 rows on and up to 256; between them the library GEMM + the vocabulary pass run, whose
+        0.244 to 0.277 ms were less than the fused head's when the limits were set (now 0.23).
         A caller's own fused_head_min_rows is the one limit: never below it, always from it on."""
         few = self.fused_head_min_rows == FUSED_HEAD_MIN_ROWS and rows <= FUSED_HEAD_FEW_ROWS
         return (self.fused_head and self.gumbel_seed is None and (few or rows >= self.fused_head_min_rows)
