@@ -224,7 +224,8 @@ __device__ __forceinline__ Partial merge_splits(const Partial* __restrict__ part
 // The end of a workgroup of the vocabulary pass that selects by itself: the last one of a sequence to arrive merges its rows' splits and applies
 // the rule.  No workgroup waits for another; what the last one reads of the others was in memory before they arrived.  own: in thread 0, what the workgroup has found.
 // Three trips to memory (store, arrival, merge) take the GPU about as long as a second launch does, and the host 2 to 3.5 us less (one_launch_pays has where they don't).
-// (A counter per row as well, and a merge per row, was a trip more: 5 sequences 16.2, 8 18.6.)
+// (A counter per row as well, and a merge per row, was a trip more: 5 sequences 16.2, 8 18.6.  Arrivals at 16 counters of a sequence first, the last of each at the sequence's own: 1 block of 32 in
+// 9 splits 12.5 / 10.9, 2 13.2 / 12.2, 3 14.0 / 13.6, 5 15.1 / 15.5; two launches 9.6, 10.9, 12.3, 15.0.)
 template <bool NOISE, bool LIVE>
 __device__ __forceinline__ void select_when_last(const Selection& S, const Partial& own, int row, int split, float c, int nsplit, Partial* partials, int64_t* x0, float* x0_p)
 {
