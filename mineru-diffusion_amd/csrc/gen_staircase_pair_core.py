@@ -30,7 +30,14 @@ reads of the first fragments of iteration t+1 are issued during the last items o
   items 0..15:  32 MFMAs of QK(t+1) -> S[1-cb]   ||  rescale check(t), P(t) = exp2(S[cb]) in place
   wait until tile t+2 (loaded two iterations ago) has landed, barrier (publishes it; everyone has left tile t-1)
   items 16..31: 32 MFMAs of PV(t) + 16 small ones (row sums)    ||  loads of tile t+4 -> slot of
-                tile t-1, row max of S[1-cb], fragment addresses of iteration t+1, addresses of tile t+5
+                tile t-1, row max of S[1-cb], fragment addresses of iteration t+1, addresses of tile t+5,
+                and behind the last two products what the next iteration starts with
+What stands between the last product of an iteration and the first of the next is not hidden by either: one comparison decides
+for the plain body, and the slots' rotation and the rescale's comparison are ahead of it (us: with seven comparisons, the rotation and
+the rescale's there 8 x 1024-8192 tokens 740, 32 x 1088 258, six of 900-1500 57; so, and without the loads beyond the last tile, 721, 243, 54).
+Nothing is loaded beyond the last tile: those loads held up the stores of O, and took the slot of the last tile but one, which the
+kernel's copies to the cache read.  The last iterations have plain bodies of their own for that (as switched-off loads in the common one they cost
+every iteration 3 %: 8 x 1024-8192 768).
 
 Physical registers (all clobbered; the compiler keeps v0..v15 and a128..a191, a224..a255 for operands):
   v16..v23  temporaries                  v24..v39  K / V^T fragment addresses
@@ -72,6 +79,8 @@ S_T, S_KEY0, S_R0, S_R1, S_R2, S_R3, S_TMP = "s40", "s41", "s42", "s43", "s44", 
 S_R4 = "s51"
 S_SAVE = "s[48:49]"
 S_DST = "s50"
+S_MASK = "s[52:53]"
+S_REL, S_PLAIN = "s54", "s55"                    # first key of the tile beyond pad; from where on (beyond pad) a tile is not for the plain body
 
 
 def sreg(b, h, u, i):
@@ -228,6 +237,18 @@ def dma_ops(slot_sreg):
     return groups
 
 
+def landed(uid):
+    """Iteration t: tile t + 2 has landed.  Tile t + 3, where there is one, may still be in flight; behind the last tile nothing is, and the
+    newest loads are those of tile t + 2.  Then the barrier, and whether there is a tile t + 4 to ask for."""
+    return [f"s_add_i32 {S_TMP}, {S_T}, 3", f"s_cmp_lt_i32 {S_TMP}, %[nt]", f"s_cbranch_scc1 .Lmore_{uid}_%=", "s_waitcnt vmcnt(0)", f".Lmore_{uid}_%=:",
+            f"s_waitcnt vmcnt({DMA_PER_TILE})", "s_barrier",
+            f"s_add_i32 {S_TMP}, {S_T}, 4", f"s_cmp_lt_i32 {S_TMP}, %[nt]", f"s_cselect_b64 {S_MASK}, -1, 0"]
+
+
+def if_more(load):
+    return [f"s_mov_b64 exec, {S_MASK}", *load, "s_mov_b64 exec, -1"]
+
+
 def k_address_ops(slot_sreg):
     """K fragment addresses (one per k-step: the swizzle is an XOR) for the slot in slot_sreg."""
     ops = [f"v_add_u32_e32 {KA[0]}, {slot_sreg}, %[ka]"]
@@ -260,6 +281,16 @@ def mask_ops(b):
     return ops
 
 
+def ask_rescale():
+    """vcc: the queries for which check_rescale of the next iteration has to move the maximum (asked for between the last products of this one)."""
+    return [f"v_max_f32_e32 {T[0]}, {MX[0]}, {MX[1]}", f"v_cmp_lt_f32_e32 vcc, 0x41000000, {T[0]}"]
+
+
+def rotate_slots():
+    return [f"s_mov_b32 {S_TMP}, {S_R0}", f"s_mov_b32 {S_R0}, {S_R1}", f"s_mov_b32 {S_R1}, {S_R2}", f"s_mov_b32 {S_R2}, {S_R3}",
+            f"s_mov_b32 {S_R3}, {S_R4}", f"s_mov_b32 {S_R4}, {S_TMP}"]
+
+
 def check_rescale(uid, cb, masked):
     """Lazy running-max update from MX = row max of S' = c s - m: only when some query of either
     head exceeds the stale max by more than 2^8.  The rare path moves m up by delta = max(MX, 0):
@@ -271,9 +302,7 @@ def check_rescale(uid, cb, masked):
     a hidden key with a score far above every visible one must not raise m (the visible terms, and
     everything accumulated so far, would be scaled to zero)."""
     lab = f".Lskip_{uid}_%="
-    out = [f"v_max_f32_e32 {T[0]}, {MX[0]}, {MX[1]}",
-           f"v_cmp_lt_f32_e32 vcc, 0x41000000, {T[0]}",
-           f"s_cbranch_vccz {lab}"]
+    out = [f"s_cbranch_vccz {lab}"]
     if masked:
         out += mask_ops(cb) + rowmax_ops(cb)
     for h in range(2):
@@ -386,6 +415,7 @@ def start_program():
     tile 0.  Returns when Q has landed; the caller scales it while tile 0 arrives."""
     out = [f"v_mov_b32_e32 {VPAD}, %[pad]", f"v_mov_b32_e32 {VLPM1}, %[lpm1]", f"v_mov_b32_e32 {JPL}, %[jpl]", f"s_mov_b32 {S_R0}, 0"]
     out += load_offset_ops()
+    out += ["global_load_dword %[slot0], %[sp0], off", "global_load_dword %[slot1], %[sp1], off"]
     for h in range(2):
         for ks in range(8):
             out.append(f"global_load_dwordx4 %[q{h}{ks}], %[qp{h}], off" + (f" offset:{32 * ks}" if ks else ""))
@@ -398,7 +428,7 @@ def start_program():
 def prologue():
     out = [f"v_mov_b32_e32 {NEG_INF}, 0xff800000", f"v_mov_b32_e32 {VPAD}, %[pad]", f"v_mov_b32_e32 {VLPM1}, %[lpm1]",
             f"v_mov_b32_e32 {MREL}, %[mrel]", f"v_add_u32_e32 {JPL}, 64, %[jpl]"]
-    out += [f"s_mov_b32 {S_T}, 0", f"s_mov_b32 {S_KEY0}, 0", f"s_mov_b32 {S_R0}, 0", f"s_mov_b32 {S_R1}, {SLOT}",
+    out += [f"s_mov_b32 {S_R0}, 0", f"s_mov_b32 {S_R1}, {SLOT}",
             f"s_mov_b32 {S_R2}, {2 * SLOT}", f"s_mov_b32 {S_R3}, {3 * SLOT}", f"s_mov_b32 {S_R4}, {4 * SLOT}"]
     # Tile 0 is on its way (start_program); the others follow one stage ahead of their use: a compute unit takes in about 20 bytes
     # per cycle, so that four tiles at once would hold up the first by 6000 cycles.
@@ -428,6 +458,11 @@ def prologue():
                 r = sreg(0, h, u, i)
                 out.append(f"v_sub_f32_e32 v{r}, v{r}, {MX[h]}")
         out.append(f"v_mov_b32_e32 {MX[h]}, 0")
+    out.append("s_mov_b64 vcc, 0")
+    # plain tiles: key0 + 64 <= whm, key0 + 64 < whx, key0 + 4 * 64 < 64 nt; from pad on
+    out += [f"s_add_i32 {S_PLAIN}, %[whm], -63", f"s_add_i32 {S_TMP}, %[whx], -64", f"s_min_i32 {S_PLAIN}, {S_PLAIN}, {S_TMP}",
+            f"s_lshl_b32 {S_TMP}, %[nt], 6", f"s_add_i32 {S_TMP}, {S_TMP}, -256", f"s_min_i32 {S_PLAIN}, {S_PLAIN}, {S_TMP}",
+            f"s_sub_i32 {S_PLAIN}, {S_PLAIN}, %[pad]", f"s_max_i32 {S_PLAIN}, {S_PLAIN}, 0", f"s_sub_i32 {S_REL}, 0, %[pad]"]
     # iteration 0 starts with its first K fragments (tile 1) in flight
     out += k_address_ops(S_R1) + v_address_ops(S_R0)
     out += issue(S_R3)                                                  # leaves the addresses of tile 4
@@ -438,10 +473,10 @@ def prologue():
     return out
 
 
-def body(cb, masked):
+def body(cb, masked, loads):
     """One iteration.  On entry the reads of items 0..RING_DEPTH-1 are in flight; on exit those of
-    the next iteration are."""
-    uid = f"{cb}{int(masked)}"
+    the next iteration are.  loads: always (there is a tile t+4), never (there is none), or as it turns out."""
+    uid = f"{cb}{int(masked)}{loads}"
     out = []
     nb = 1 - cb
     items = qk_items(nb) + pv_items(cb)
@@ -458,10 +493,11 @@ def body(cb, masked):
     per = -(-len(rm) // 8)
     for i in range(8):
         plan[18 + i] += rm[per * i:per * (i + 1)]
-    tail = v_address_ops(S_R1) + load_offset_ops()
+    tail = v_address_ops(S_R1) + (load_offset_ops() if loads != "never" else [])
     per = -(-len(tail) // 6)
     for i in range(6):
         plan[26 + i] += tail[per * i:per * (i + 1)]
+    plan[31] += rotate_slots() + [f"s_add_i32 {S_REL}, {S_REL}, 64"] + ask_rescale()
     dma = dma_ops(S_R4)
     rg = Ring()
     for n in range(RING_DEPTH):
@@ -473,18 +509,15 @@ def body(cb, masked):
             # tile t+2 (loaded two iterations ago; tile t+3 may still be in flight) has landed; after
             # the barrier every wavefront sees it and has left tile t-1, whose slot the loads below
             # (tile t+4) overwrite
-            out += [f"s_waitcnt vmcnt({DMA_PER_TILE})", "s_barrier"]
+            out += [f"s_waitcnt vmcnt({DMA_PER_TILE})", "s_barrier"] if loads == "always" else landed(uid)
         if n % 2 == 0:
             rg.wait(out, n + 1)
-        first, last = dma[n - 17] if 17 <= n < 17 + DMA_PER_TILE else ([], [])
+        first, last = dma[n - 17] if loads != "never" and 17 <= n < 17 + DMA_PER_TILE else ([], [])
         out.extend(first)
         spread(out, items[n][1](ring(n)), plan[n])
         k = n + RING_DEPTH
         rg.read(out, k, items[k] if k < 32 else nxt[k - 32], k)
-        out.extend(last)
-    out += [f"s_mov_b32 {S_TMP}, {S_R0}", f"s_mov_b32 {S_R0}, {S_R1}", f"s_mov_b32 {S_R1}, {S_R2}", f"s_mov_b32 {S_R2}, {S_R3}",
-            f"s_mov_b32 {S_R3}, {S_R4}", f"s_mov_b32 {S_R4}, {S_TMP}",
-            f"s_add_i32 {S_T}, {S_T}, 1", f"s_add_i32 {S_KEY0}, {S_KEY0}, 64", f"v_add_u32_e32 {MREL}, 64, {MREL}"]
+        out.extend(if_more(last) if last and loads == "maybe" else last)
     return out
 
 
@@ -497,18 +530,13 @@ def body_last(cb):
     out = []
     items = [None] * 16 + pv_items(cb)
     plan = softmax_plan(cb, True)
-    tail = load_offset_ops()
-    per = -(-len(tail) // 6)
-    for i in range(6):
-        plan[26 + i] += tail[per * i:per * (i + 1)]
-    dma = dma_ops(S_R4)
     rg = Ring()
     rg.issued = RING_DEPTH                              # the K reads in flight on entry: they complete first, in order
     out += check_rescale(uid, cb, True)
     out += v_address_ops(S_R0)                          # V^T addresses of tile t (the previous iteration set them too; kept explicit)
     for n in range(32):
         if n == 16:
-            out += [f"s_waitcnt vmcnt({DMA_PER_TILE})", "s_barrier"]
+            out += landed(uid)
         if n < 16:
             out.extend(plan[n])
             out.append("s_nop 1")                       # no MFMAs here to space a v_exp from the conversion that reads it
@@ -518,16 +546,11 @@ def body_last(cb):
             continue
         if n % 2 == 0:
             rg.wait(out, n + 1)
-        first, last = dma[n - 17] if 17 <= n < 17 + DMA_PER_TILE else ([], [])
-        out.extend(first)
         spread(out, items[n][1](ring(n)), plan[n])
         k = n + RING_DEPTH
         if k < 32:
             rg.read(out, k, items[k], k)
-        out.extend(last)
-    out += [f"s_mov_b32 {S_TMP}, {S_R0}", f"s_mov_b32 {S_R0}, {S_R1}", f"s_mov_b32 {S_R1}, {S_R2}", f"s_mov_b32 {S_R2}, {S_R3}",
-            f"s_mov_b32 {S_R3}, {S_R4}", f"s_mov_b32 {S_R4}, {S_TMP}",
-            f"s_add_i32 {S_T}, {S_T}, 1",
+    out += rotate_slots() + [f"s_add_i32 {S_T}, {S_T}, 1",
             f"s_cmp_ge_i32 {S_T}, %[nt]",
             "s_cbranch_scc1 .Lend_%=",
             "s_branch .Lidle_%="]
@@ -535,8 +558,18 @@ def body_last(cb):
 
 
 def select(cb):
-    """Top of iteration t: leave after the last tile; tiles that need the key mask go out of line."""
+    """Top of iteration t.  One comparison for the tiles of the plain body: all of their keys visible to every query of the wavefront, and a tile t+4 to ask for."""
     return [f".Ltop_{cb}_%=:",
+            f"s_cmp_ge_u32 {S_REL}, {S_PLAIN}",
+            f"s_cbranch_scc1 .Lother_{cb}_%="]
+
+
+def select_other(cb):
+    """Leave after the last tile; tiles that need the key mask, and the last ones, go out of line."""
+    return [f".Lother_{cb}_%=:",
+            f"s_add_i32 {S_KEY0}, {S_REL}, %[pad]",
+            f"v_add_u32_e32 {MREL}, {S_KEY0}, %[mrel]",
+            f"s_lshr_b32 {S_T}, {S_KEY0}, 6",
             f"s_cmp_ge_i32 {S_T}, %[nt]",
             "s_cbranch_scc1 .Lend_%=",
             f"s_cmp_ge_i32 {S_KEY0}, %[whx]",
@@ -555,14 +588,11 @@ def idle_loop():
     wavefronts of the workgroup own later rows and still need the tile): nothing to compute -- every probability
     would be zero -- but the wavefront keeps loading its quarter of every tile and meets the others at the barrier.
     Entered from the top of an iteration, left only through the end of the loop."""
-    out = [".Lidle_%=:",
-           f"s_waitcnt vmcnt({DMA_PER_TILE})", "s_barrier"]
+    out = [".Lidle_%=:"] + landed("idle")
     for first, last in dma_ops(S_R4):
-        out += first + ["s_nop 0"] + last
+        out += first + ["s_nop 0"] + if_more(last)
     out += load_offset_ops()
-    out += [f"s_mov_b32 {S_TMP}, {S_R0}", f"s_mov_b32 {S_R0}, {S_R1}", f"s_mov_b32 {S_R1}, {S_R2}", f"s_mov_b32 {S_R2}, {S_R3}",
-            f"s_mov_b32 {S_R3}, {S_R4}", f"s_mov_b32 {S_R4}, {S_TMP}",
-            f"s_add_i32 {S_T}, {S_T}, 1",
+    out += rotate_slots() + [f"s_add_i32 {S_T}, {S_T}, 1",
             f"s_cmp_ge_i32 {S_T}, %[nt]",
             "s_cbranch_scc0 .Lidle_%="]
     return out
@@ -573,9 +603,8 @@ def epilogue():
     d group): stored from there, a store instruction touches 32 rows with 16 bytes each.  Instead every wavefront
     turns its 32 x 128 tile of one head around through 8 KB of LDS and writes whole rows: 16 lanes x 16 bytes per
     row, four rows per instruction, 8 instructions per head (before: 16 of half the width, and they cost a tenth
-    of a launch of 1000-token sequences).  The LDS comes from the slot of tile nt + 1: that tile was loaded ahead
-    of need and landed, for every wavefront, before the barrier of the last iteration; nobody reads it and no
-    load still in flight targets it (those are tiles nt + 2 and nt + 3).  Rows use the K / V swizzle (16-byte
+    of a launch of 1000-token sequences).  The LDS comes from the slot of tile nt + 1, which nobody reads any more and no load
+    is on its way to (the prologue's of tiles up to 3 have landed before the last iteration's barrier).  Rows use the K / V swizzle (16-byte
     chunk c of row r at position c ^ (r % 16)), which keeps the 8-byte writes of a (d tile, group) off each
     other's banks; the reads are linear."""
     LN, X, WB, RB, L4, OFFL, C0, RV = (f"v{80 + i}" for i in range(8))
@@ -643,11 +672,15 @@ def epilogue():
 def program():
     # the common path falls through: top 0, plain body 0, top 1, plain body 1, one branch back
     out = prologue()
-    out += select(0) + body(0, False) + select(1) + body(1, False) + ["s_branch .Ltop_0_%="]
-    out += [".Lmasked_0_%=:"] + body(0, True) + ["s_branch .Ltop_1_%="]
-    out += [".Lmasked_1_%=:"] + body(1, True) + ["s_branch .Ltop_0_%="]
-    out += [".Llast_0_%=:"] + body_last(0)
-    out += [".Llast_1_%=:"] + body_last(1)
+    for cb in range(2):
+        out += select(cb) + body(cb, False, "always")
+    out += ["s_branch .Ltop_0_%="]
+    for cb in range(2):
+        out += select_other(cb) + body(cb, False, "never") + [f"s_branch .Ltop_{1 - cb}_%="]
+    for cb in range(2):
+        out += [f".Lmasked_{cb}_%=:"] + body(cb, True, "maybe") + [f"s_branch .Ltop_{1 - cb}_%="]
+    for cb in range(2):
+        out += [f".Llast_{cb}_%=:"] + body_last(cb)
     out += idle_loop()
     out += epilogue()
     return out
@@ -695,12 +728,13 @@ def main():
     start = "\n".join(f'        "{line}\\n"' for line in start_program())
     start_out = ", ".join(f'[q{h}{ks}] "=&v"(q[{h}][{ks}])' for h in range(2) for ks in range(8))
     start_clob = ", ".join(f'"v{r}"' for r in [22, 40, 41, 42, *range(56, 64)])
-    begin = f'''__device__ __forceinline__ void @@NAME@@_start(const PairCoreArgs& A, const void* q0, const void* q1, u32x4 (&q)[2][8])
+    begin = f'''__device__ __forceinline__ void @@NAME@@_start(const PairCoreArgs& A, const void* q0, const void* q1, u32x4 (&q)[2][8],
+                                                          const int* s0, const int* s1, int (&slot)[2])
 {{
     asm volatile(
 {start}
-        : {start_out}
-        : [qp0] "v"(q0), [qp1] "v"(q1), [jpl] "v"(A.jpl), [ch] "v"(A.ch), [kb] "s"(A.kb), [vb] "s"(A.vb), [krb] "s"(A.krb), [vrb] "s"(A.vrb),
+        : {start_out}, [slot0] "=&v"(slot[0]), [slot1] "=&v"(slot[1])
+        : [sp0] "v"(s0), [sp1] "v"(s1), [qp0] "v"(q0), [qp1] "v"(q1), [jpl] "v"(A.jpl), [ch] "v"(A.ch), [kb] "s"(A.kb), [vb] "s"(A.vb), [krb] "s"(A.krb), [vrb] "s"(A.vrb),
           [wrow] "s"(A.wrow), [pad] "s"(A.pad), [lpm1] "s"(A.lpm1)
         : "memory", "scc", "m0", {sclob}, {start_clob});
 }}

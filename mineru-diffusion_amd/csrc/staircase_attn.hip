@@ -138,37 +138,6 @@ __device__ __forceinline__ void store_unowned_rows(const StaircaseParams& P, int
     }
 }
 
-// The same for the pair kernel, whose workgroups own whole CUs: store workgroups behind them would hold a CU each and start when the
-// attention is done, and cost what a launch of their own costs.  But the K / V rows of a row group's own tokens are the last that
-// its key loop has read, so the workgroup of the KV head's first pair copies them (64 KB, from L2) when it is through: 1.5 us a
-// workgroup.  Store + attention, us, as two launches / here: 6 prompts of 900-1500 tokens 63.5 / 58.3, 6 x 1167 58.5 / 52.5, 4 x 2000
-// 83.7 / 77, 20 x 800 115 / 108, 8 x 1800 154 / 144; against a store on a second stream beside the attention: 32 x 800 193 / 188, 8
-// prompts of 1024-8192 level at 744.
-__device__ __forceinline__ void store_own_rows(const StoreParams& S, int kvh, int seq0, int begin, int end, int tid)
-{
-    constexpr int kRounds = kRowsPerWg / (kThreads / 16);
-    const int col = kvh * (kHeadDim / 8) + (tid & 15);
-    u32x4 k[kRounds], v[kRounds];
-    int64_t slot[kRounds];
-#pragma unroll
-    for (int i = 0; i < kRounds; ++i) {
-        const int t = begin + i * (kThreads / 16) + (tid >> 4);
-        slot[i] = -1;
-        if (t < end) {
-            const int64_t tok = (int64_t)seq0 + t;
-            slot[i] = S.slot_mapping[tok];
-            k[i] = S.key[tok * S.k_stride16 + col];
-            v[i] = S.value[tok * S.v_stride16 + col];
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < kRounds; ++i) {
-        if (slot[i] < 0 || slot[i] >= S.num_slots) continue;
-        __builtin_nontemporal_store(k[i], S.k_cache + slot[i] * S.row16 + col);
-        __builtin_nontemporal_store(v[i], S.v_cache + slot[i] * S.row16 + col);
-    }
-}
-
 // Workgroup -> (sequence b, row group rg) for the j-th (sequence, row group) pair in launch order.
 // Row groups are handed out heaviest-first (the last row group of a sequence attends to the most
 // keys).  The dispatcher deals consecutive workgroups round-robin to XCDs and shader engines and
@@ -517,6 +486,29 @@ __device__ __forceinline__ const void* uniform(const void* p) {
     return (const void*)(((uint64_t)hi << 32) | lo);
 }
 
+// The store of the pair kernel, whose workgroups own whole CUs: store workgroups behind them would hold a CU each and start when the
+// attention is done, and cost what a launch of their own costs.  But the K / V rows of a row group's own tokens are its last two tiles (its
+// key limit is its last row's block's end, and a block is at most as long as the group), which the core leaves in LDS, so the workgroup of the KV head's first pair
+// copies them when it is through.  64 stores of 1 KB: 1.3 us a workgroup (2.9 with the rows read again from L2: a CU's address unit takes a load or store of
+// 1 KB in 50 cycles, 57.0 -> 54.3 us for 6 prompts of 900-1500 tokens together with the core's part of it).  Store + attention, us, as two launches /
+// here: 6 of 900-1500 63.5 / 54.3, 8 x 1800 154 / 127; against a store on a second stream beside the attention (with the rows from L2): 32 x 800 193 / 188, 8
+// prompts of 1024-8192 level at 744.
+__device__ __forceinline__ void store_own_rows(const StoreParams& S, const char* lds, int kvh, int row_g0, int pad, int L, const int (&slots)[2], int tid)
+{
+    constexpr int kRounds = kRowsPerWg / (kThreads / 16);
+    const int chunk = tid & 15, col = kvh * (kHeadDim / 8) + chunk;
+#pragma unroll
+    for (int i = 0; i < kRounds; ++i) {
+        const int row = i * (kThreads / 16) + (tid >> 4), t = row_g0 + row - pad, r = row % kTileKeys;
+        const int slot = __shfl(slots[i / (kRounds / 2)], r);
+        const char* at = lds + (row_g0 + row) / kTileKeys % kPairSlots * (2 * kTileKeys * kRowBytes) + r * kRowBytes + ((chunk ^ (r & 15)) << 4);
+        const u32x4 k = *reinterpret_cast<const u32x4*>(at), v = *reinterpret_cast<const u32x4*>(at + kTileKeys * kRowBytes);
+        if (t < 0 || t >= L || slot < 0 || slot >= S.num_slots) continue;
+        __builtin_nontemporal_store(k, S.k_cache + slot * (int64_t)S.row16 + col);
+        __builtin_nontemporal_store(v, S.v_cache + slot * (int64_t)S.row16 + col);
+    }
+}
+
 template <typename E>
 __global__ __launch_bounds__(kThreads, 1) void staircase_pair_kernel(const StaircaseParams P)
 {
@@ -593,7 +585,12 @@ __global__ __launch_bounds__(kThreads, 1) void staircase_pair_kernel(const Stair
     // Q^T fragments, pre-multiplied by scale * log2(e) (the MFMA then yields scores in log2 units); rows outside the sequence: zeros
     u32x4 raw[2][8];
     const __bf16* qrow = P.q + ((int64_t)seq0 + min(max(ip - pad, 0), L - 1)) * P.q_st + (int64_t)head0 * P.q_sh + H * 8;
-    staircase_pair_core_start(A, qrow, qrow + P.q_sh, raw);
+    // (the cache slots of the row group's tokens come along, row `lane` and row 64 + lane; any address that exists where nothing is stored)
+    auto slot_of = [&](int row) {
+        return P.store.own_rows ? P.store.slot_mapping + seq0 + min(max(row_g0 + row - pad, 0), L - 1) : reinterpret_cast<const int32_t*>(qrow);
+    };
+    int slots[2];
+    staircase_pair_core_start(A, qrow, qrow + P.q_sh, raw, slot_of(lane), slot_of(64 + lane), slots);
     const float c = row_ok ? P.c : 0.f;
     typename Elem16<E>::vec8 q[2][8];
 #pragma unroll
@@ -605,7 +602,8 @@ __global__ __launch_bounds__(kThreads, 1) void staircase_pair_kernel(const Stair
             for (int j = 0; j < 8; ++j) q[h][ks][j] = (E)((float)q[h][ks][j] * c);
         }
     pair_core(A, q);
-    if (P.store.own_rows && hslot < P.num_kv_heads) store_own_rows(P.store, kvh, seq0, max(0, row_g0 - pad), min(L, row_g0 - pad + kRowsPerWg), tid);
+    if (!P.store.own_rows || hslot >= P.num_kv_heads) return;
+    store_own_rows(P.store, lds_pair, kvh, row_g0, pad, L, slots, tid);
 }
 
 }  // namespace

@@ -332,6 +332,35 @@ def test_pair_prefill_stores_every_row(dev, lens, hkv, ratio, dtype, before, beh
         assert torch.equal(o[before:N - behind], want.flatten(1)[before:N - behind])
 
 
+@pytest.mark.parametrize("block", [1, 16, 32, 64, 128])
+def test_pair_prefill_at_the_edges_of_key_tiles(dev, block):
+    """Sequences that end one short of, at and one past each of the first key tiles, in one launch with a long one: outputs against the oracle,
+    and the stored rows, which come from the last two tiles, against the tensors."""
+    import mdx
+    import oracle
+    hq, hkv, d = 4, 2, 128
+    lens = [1400, 640] + [n + e for n in (32, 64, 128, 192, 256, 320, 384) for e in (-1, 0, 1)] * 2
+    N = sum(lens)
+    g = torch.Generator().manual_seed(block)
+    q, k, v = (torch.randn(N, h, d, generator=g).bfloat16() for h in (hq, hkv, hkv))
+    cu = torch.tensor([0] + [int(n) for n in np.cumsum(lens)], dtype=torch.int32)
+    pages = N // PAGE + 1
+    slots = torch.randperm(pages * PAGE, generator=g)[:N].int()
+    attn = mdx.Attention(hq, d, d ** -0.5, hkv)
+    attn.k_cache = torch.zeros(pages, PAGE, hkv, d, dtype=torch.bfloat16, device=dev)
+    attn.v_cache = torch.zeros_like(attn.k_cache)
+    mdx.set_context(True, cu.to(dev), cu.to(dev), max(lens), max(lens), slots.to(dev), None, None, block_size=block)
+    try:
+        o = attn(q.to(dev), k.to(dev), v.to(dev))
+    finally:
+        mdx.reset_context()
+    assert torch.equal(attn.k_cache.view(-1, hkv, d)[slots.long().to(dev)].cpu(), k)
+    assert torch.equal(attn.v_cache.view(-1, hkv, d)[slots.long().to(dev)].cpu(), v)
+    want = oracle.staircase_attn_varlen(q, k, v, cu, block)
+    # 16-bit outputs of size one: half a unit in the last place, and probabilities of 8 bits, whose errors average out over the keys
+    assert (o.float().cpu().view(N, hq, d) - want.float()).abs().max() < 2e-2
+
+
 def test_host_functions_refuse_sizes_of_zero(dev):
     """No KV heads, empty heads or no partial sums: an exception, as the Python divisions raised, and never the end of the process."""
     import mdx
