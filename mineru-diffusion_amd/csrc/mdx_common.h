@@ -58,6 +58,11 @@ inline int compute_units() {
 
 namespace mdx {
 
+// n / d of wavefront-uniform numbers for a d that the compiler doesn't know and that is mostly a power of two (heads, groups of heads, tiles): the general
+// sequence goes through a float reciprocal in the vector unit and back, in every workgroup's start.  Attention calls, us, by that sequence / so: paged, one sequence of 1337 keys 14.6 / 14.35, four of 1000-3000
+// 23.0 / 22.7, 32 of 600-2400 55.9 / 55.5; prompts 3 x 40-150 7.75 / 7.6, 500 13.4 / 13.2.  (In fp32 arithmetic 20.2 / 20.4: not there.)
+__device__ __forceinline__ unsigned quotient(unsigned n, unsigned d) { return (d & (d - 1)) == 0 ? n >> __builtin_ctz(d) : n / d; }
+
 // A kernel's arguments come through the scalar cache, 64 bytes at a time, and the compiler asks for them where they are first used, some of them behind
 // other loads.  This asks for all lines of BYTES bytes of arguments, and for the grid's size if it is given, at once.  Returns 0 in a way that the
 // compiler doesn't see, to be added to something that is used early.  (Not a volatile asm: behind one, the compiler no longer takes page tables and

@@ -225,8 +225,8 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
     // launch order: head group fastest, then the query tiles of a (sequence, split), then the pairs -- the tiles of a
     // block longer than 32 queries stream the same keys, so they start next to each other and on the same XCD
     const int n_groups = P.num_q_heads / HPW;
-    const int hg = block_x % n_groups;
-    const int qt = block_x / n_groups;           // this workgroup's tile of 32 queries
+    const int qt = mdx::quotient(block_x, n_groups);           // this workgroup's tile of 32 queries
+    const int hg = block_x - qt * n_groups;
     const int kw = wave % KW;                       // this wavefront's key slice
     const int head = hg * HPW + wave / KW;          // and query head
 
@@ -338,7 +338,7 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
     const int key_begin = __builtin_amdgcn_readfirstlane(split * span);
     if (key_begin >= ctx) return;
     const int key_end = __builtin_amdgcn_readfirstlane(min(ctx, key_begin + span));
-    const int kvh = (hg * HPW) / P.heads_per_kv;
+    const int kvh = mdx::quotient(hg * HPW, P.heads_per_kv);
 
     const int qrow = qt * kQTile + r;               // this lane's query of the sequence's block
     const bool row_ok = qrow < P.sq;
@@ -613,7 +613,7 @@ __global__ __launch_bounds__(32 * ROWS) void paged_combine_kernel(const PagedPar
     constexpr int kParts = kQTile / ROWS;
     const unsigned block = blockIdx.x + mdx::fetch_arguments<sizeof(PagedParams)>();
     const int part = block % kParts, rest = block / kParts;
-    const int qt = rest % P.nqt, hq = (rest / P.nqt) % P.num_q_heads, b = rest / P.nqt / P.num_q_heads;
+    const int row_tile = mdx::quotient(rest, P.nqt), qt = rest - row_tile * P.nqt, b = mdx::quotient(row_tile, P.num_q_heads), hq = row_tile - b * P.num_q_heads;
     const int c = (threadIdx.x & 31) * 4, s = part * ROWS + (threadIdx.x >> 5);
     if (c >= P.head_dim || qt * kQTile + s >= P.sq) return;
     const int64_t slot0 = (((int64_t)b * P.num_q_heads + hq) * P.nqt + qt) * P.nsplit;

@@ -277,9 +277,9 @@ __global__ __launch_bounds__(kThreads, 2) void staircase_attn_kernel(const Stair
     if (block >= P.store.first_wg) { store_rows(P.store, block - P.store.first_wg, tid); return; }
 
     // ---- workgroup -> (head slot, sequence b, row group rg) ------------------------------------
-    const int hslot = (unsigned)block % P.num_q_heads;
+    const int pair = mdx::quotient(block, P.num_q_heads), hslot = block - pair * P.num_q_heads;
     int b, rg, seq0, L;
-    if (!locate_row_group<kRows>(P, (unsigned)block / P.num_q_heads, lane, lds_hist[wave], b, rg, seq0, L)) return;
+    if (!locate_row_group<kRows>(P, pair, lane, lds_hist[wave], b, rg, seq0, L)) return;
     if (L <= 0) return;
     const int S = 1 << P.log2_s;
     const int Lp = ((L + S - 1) >> P.log2_s) << P.log2_s;     // padded length
@@ -287,8 +287,8 @@ __global__ __launch_bounds__(kThreads, 2) void staircase_attn_kernel(const Stair
     const int row_g0 = rg * kRows;                        // first padded row of the workgroup
     if (row_g0 >= Lp) return;
 
-    const int kvh = hslot % P.num_kv_heads;                    // launch order: KV head fastest
-    const int head = kvh * (P.num_q_heads / P.num_kv_heads) + hslot / P.num_kv_heads;
+    const int of_kvh = mdx::quotient(hslot, P.num_kv_heads), kvh = hslot - of_kvh * P.num_kv_heads;      // launch order: KV head fastest
+    const int head = kvh * mdx::quotient(P.num_q_heads, P.num_kv_heads) + of_kvh;
 
     // ---- this wavefront's 32 rows ----
     const int row_w0 = row_g0 + wave / KW * 32;
@@ -528,10 +528,10 @@ __global__ __launch_bounds__(kThreads, 1) void staircase_pair_kernel(const Stair
     // One work item per workgroup: the dispatcher hands the next item to whichever CU frees up
     // first, which balances the ragged item lengths (a fixed item -> CU assignment measured 10%
     // slower although it saves the launch gap between two workgroups of a CU).
-    const int hslot = item % n_hslots;
+    const int at = mdx::quotient(item, n_hslots), hslot = item - at * n_hslots;
     int b, rg, seq0, L;
     // (scratch for the numbering: in slot 4, which no K/V load targets before every wavefront has passed the core's first barrier)
-    if (!locate_row_group<kRowsPerWg>(P, item / n_hslots, lane, reinterpret_cast<int*>(lds_pair + 4 * (2 * kTileKeys * kRowBytes)) + wave * 80, b, rg, seq0, L)) return;
+    if (!locate_row_group<kRowsPerWg>(P, at, lane, reinterpret_cast<int*>(lds_pair + 4 * (2 * kTileKeys * kRowBytes)) + wave * 80, b, rg, seq0, L)) return;
     if (L <= 0) return;
     const int S = 1 << P.log2_s;
     const int Lp = ((L + S - 1) >> P.log2_s) << P.log2_s;
@@ -539,9 +539,9 @@ __global__ __launch_bounds__(kThreads, 1) void staircase_pair_kernel(const Stair
     const int row_g0 = rg * kRowsPerWg;
     if (row_g0 >= Lp) return;
 
-    const int heads_per_kv = P.num_q_heads / P.num_kv_heads;
-    const int kvh = hslot % P.num_kv_heads;                    // launch order: KV head fastest
-    const int head0 = kvh * heads_per_kv + 2 * (hslot / P.num_kv_heads);
+    const int heads_per_kv = mdx::quotient(P.num_q_heads, P.num_kv_heads);
+    const int of_kvh = mdx::quotient(hslot, P.num_kv_heads), kvh = hslot - of_kvh * P.num_kv_heads;      // launch order: KV head fastest
+    const int head0 = kvh * heads_per_kv + 2 * of_kvh;
 
     const int row_w0 = row_g0 + wave * 32;
     const int ip = row_w0 + r;
