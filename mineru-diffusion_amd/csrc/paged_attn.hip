@@ -117,7 +117,7 @@ struct PagedParams {
     int num_q_heads;
     int head_dim;                                   // <= 128, a multiple of 16: columns beyond it are zeros in LDS and never stored
     float c;                                        // scale * log2(e)
-    float* part_o; float* part_ml;                  // [bs, Hq, nqt, nsplit, 32, 128] and [bs, Hq, nqt, nsplit, 32, (m, l)]
+    float* part_o; float* part_ml;                  // [bs, Hq, nqt, nsplit, (d tile, register quad), lane, 4] and [bs, Hq, nqt, nsplit, 32, (m, l)]
     // non-null: the attention kernel picks the split size (>= chunk) from the lengths and leaves it
     // here for the combine kernel.  A float on purpose: an int store in the attention kernel could
     // alias the int page table and lengths for the compiler, which would then stop fetching those
@@ -232,6 +232,7 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
 
     // ---- workgroup -> (sequence b, split) ------------------------------------------------------
     int b, split, span = P.chunk;
+    bool paced = false;
     int ctx_all = 0;                                // (up to 64 sequences) the clipped length of sequence `lane`
     if (P.bs <= 64) {
         // lengths beyond the page table name keys that do not exist: clipped here and below
@@ -262,6 +263,9 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
                 span += 64;
                 n = splits_of_lane();
             }
+            // more than three quarters of the resident workgroups have a whole piece (fetch_by says why; launches that merge themselves have no more than 2560 keys a
+            // sequence and were level)
+            paced = !MERGE && 4.f * (float)total * (float)gridDim.x > 3.f * (float)P.fit_slots * (float)span;
             if (blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) *P.span_out = (float)span;
         } else {
             if (P.fit_slots < 0) {
@@ -313,6 +317,9 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
             }
         } else {
             // the first split of every sequence, then the second of those that have one, ...: the last split of a sequence is its remainder
+            // (from the level that the pair would have if all of them had that many: those below it hold a sum)
+            level = mdx::quotient(j, P.bs);
+            j -= level > 0 ? wave_sum(min(n, level)) : 0;
             for (; level < P.nsplit; ++level) if (among(__ballot(n > level))) break;
         }
         if (b < 0) return;                          // past the last (sequence, split) pair
@@ -340,26 +347,24 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
     const int key_end = __builtin_amdgcn_readfirstlane(min(ctx, key_begin + span));
     const int kvh = mdx::quotient(hg * HPW, P.heads_per_kv);
 
-    const int qrow = qt * kQTile + r;               // this lane's query of the sequence's block
-    const bool row_ok = qrow < P.sq;
-    typename Elem16<E>::vec8 q[1][8];
-    load_q(q[0], row_ok ? P.q + (int64_t)b * P.q_sb + (int64_t)qrow * P.q_ss + (int64_t)head * P.q_sh : nullptr, H, P.head_dim);
-
-    WaveState<1> st;
-    st.init();
-
     // (with the readers' loads in the kernel the compiler no longer takes the table for constant by itself)
     typedef __attribute__((address_space(4))) const int32_t ConstantEntry;
     auto table_row = [&] {
         const int32_t* row = P.block_table + (int64_t)__builtin_amdgcn_readfirstlane(b) * P.bt_stride;
-        if constexpr (sizeof...(AHEAD) > 0) return (ConstantEntry*)(uintptr_t)row; else return row;
+        return (ConstantEntry*)(uintptr_t)row;
     };
     const auto bt = table_row();
     const int chunk = tid & 15, trow = tid >> 4;    // one pass stages kRowsPerPass rows
     const int n_tiles = (key_end - key_begin + kTileKeys - 1) / kTileKeys;
-    // kRowsPerPass (16 or 32) consecutive keys starting at a multiple of that never straddle a page (page_size % 32 == 0):
-    // each pass looks its page up once.  The loads of a fetch are unconditional (rows past the context
-    // or on an invalid page id read row `trow` of page 0 instead and are zeroed when they reach LDS).
+    // The loads of a fetch are unconditional (rows past the context or on an invalid page id read a row of the page, or of page 0, instead and are zeroed when they
+    // reach LDS).  Where a tile lies in one page (tile_in_page) its page comes from a register that holds the piece's first 64, and its loads stand one
+    // behind the other; else each pass of kRowsPerPass keys, which never straddles a page (page_size % 32 == 0), looks its page up.  A lookup is 500 to 1700 cycles, waited for before
+    // the pass's loads: with one per pass the first two tiles' loads took 4800 cycles of a workgroup's start, and the first had landed before the last was asked
+    // for.  The layer, us, before / now: one sequence of 1337 keys 14.4 / 14.0, 4000 19.2 / 18.3, 12 000 27.7 / 25.1, four of 1000-3000 22.7 / 22.0, eight 30.3 / 28.8, 12 of 500-2500 34.8 / 32.5.
+    // Not everywhere (`paced`): where the launch fills most of the resident workgroups HBM is the bound, and workgroups that ask for their tiles as soon as they can crowd out
+    // each other; there a lookup per pass spreads the loads behind the first two tiles (16 of 512-4096 44.4 / 41.9, start 42.6, 8 of 3000-6000 42.2 / 41.4).  K's rows of a tile before V's is
+    // the better order there too, and with a pair per CU (32 of 600-2400 56.5 / 56.1), at the start as well, while few workgroups do best with K and V in turn at the start.  And not beside readers:
+    // that launch lasts as long as those do (generating with one request 61.7 ms, 62.1 with tiles looked up at once, eight 57.5 / 58.5).
     struct Staged {
         TileRegs<kTileKeys, kThreads> regs;
         unsigned row_ok;       // bit p: this thread's row of pass p holds a real key
@@ -368,25 +373,53 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
     // (a thread whose 16-byte chunk lies beyond a narrow head reads the head's last chunk instead; zeroed like a row past the end)
     const bool col_ok = chunk * 8 < P.head_dim;
     const int64_t safe_off = (int64_t)trow * P.c_st + (int64_t)kvh * P.c_sh + min(chunk * 8, P.head_dim - 8);
-    auto fetch = [&](Staged& sg, int t) {
+    const bool tile_in_page = sizeof...(AHEAD) == 0 && P.page_shift >= 0 && P.page_size >= kTileKeys && (key_begin & (kTileKeys - 1)) == 0;
+    const bool paged_tiles = tile_in_page && !paced;
+    auto slot_of = [&](int key) { return P.page_shift >= 0 ? key >> P.page_shift : key / P.page_size; };
+    const int first_slot = slot_of(key_begin);
+    const int pages = bt[min(first_slot + lane, P.max_pages - 1)];
+    auto load_k = [&](Staged& sg, int p, int64_t off) { sg.regs.k[p] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(P.k_cache + off)); };
+    auto load_v = [&](Staged& sg, int p, int64_t off, bool ok, int key0) {
+        sg.regs.v[p] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(P.v_cache + off));
+        sg.pass_ok |= (ok ? 1u : 0u) << p;
+        sg.row_ok |= ((ok && col_ok && key0 + kRowsPerPass * p + trow < key_end) ? 1u : 0u) << p;
+    };
+    auto fetch_by = [&](auto first, Staged& sg, int t) {
         const int key0 = key_begin + t * kTileKeys;
         sg.row_ok = 0;
         sg.pass_ok = 0;
+        if (first ? tile_in_page : paged_tiles) {
+            const int ahead = slot_of(key0) - first_slot, page = ahead < 64 ? __builtin_amdgcn_readlane(pages, ahead) : bt[first_slot + ahead];
+            const bool valid = page >= 0 && page < P.num_pages;
+            const int64_t base = valid ? page * P.c_sp + (int64_t)(key0 & (P.page_size - 1)) * P.c_st : 0;
+            auto offset = [&](int p) { return base + (int64_t)(kRowsPerPass * p) * P.c_st + safe_off; };
+            auto ok = [&](int p) { return valid && key0 + kRowsPerPass * p < key_end; };
 #pragma unroll
-        for (int p = 0; p < kPasses; ++p) {
-            const int kp = key0 + kRowsPerPass * p;
-            const int page_slot = P.page_shift >= 0 ? kp >> P.page_shift : kp / P.page_size;
-            const int in_page = P.page_shift >= 0 ? kp & (P.page_size - 1) : kp % P.page_size;
-            const bool inside = kp < key_end && page_slot < P.max_pages;
-            const int64_t page = bt[inside ? page_slot : 0];
-            const bool ok = inside && page >= 0 && page < P.num_pages;             // uniform
-            const int64_t off = ok ? page * P.c_sp + (int64_t)in_page * P.c_st + safe_off : safe_off;
-            sg.regs.k[p] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(P.k_cache + off));
-            sg.regs.v[p] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(P.v_cache + off));
-            sg.pass_ok |= (ok ? 1u : 0u) << p;
-            sg.row_ok |= ((ok && col_ok && kp + trow < key_end) ? 1u : 0u) << p;
+            for (int p = 0; p < kPasses; ++p) {
+                load_k(sg, p, offset(p));
+                if (first && !MERGE) load_v(sg, p, offset(p), ok(p), key0);
+            }
+            if (!first || MERGE) {
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int p = 0; p < kPasses; ++p) load_v(sg, p, offset(p), ok(p), key0);
+            }
+        } else {
+#pragma unroll
+            for (int p = 0; p < kPasses; ++p) {
+                const int kp = key0 + kRowsPerPass * p, page_slot = slot_of(kp);
+                const bool inside = kp < key_end && page_slot < P.max_pages;
+                const int64_t page = bt[inside ? page_slot : 0];
+                const bool ok = inside && page >= 0 && page < P.num_pages;             // uniform
+                const int64_t off = ok ? page * P.c_sp + (int64_t)(kp - page_slot * P.page_size) * P.c_st + safe_off : safe_off;
+                load_k(sg, p, off);
+                load_v(sg, p, off, ok, key0);
+            }
         }
     };
+    typename Elem16<E>::vec8 q[1][8];
+    WaveState<1> st;
+    auto fetch = [&](Staged& sg, int t) { fetch_by(std::false_type(), sg, t); };
     unsigned tile_pass_ok[2] = {0, 0};                 // pass_ok of the tile sitting in LDS buffer 0 / 1
     auto stage = [&](int buf, Staged& sg) {
 #pragma unroll
@@ -409,8 +442,13 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
 
     // Register sets ra / rb hold the tiles after the one in LDS; tile t+1 sits in set (t+1)%2.
     Staged ra, rb;
-    fetch(ra, 0);
-    if (DEPTH == 2 && n_tiles > 1) fetch(rb, 1);
+    const int qrow = qt * kQTile + r;               // this lane's query of the sequence's block
+    const bool row_ok = qrow < P.sq;
+    load_q(q[0], row_ok ? P.q + (int64_t)b * P.q_sb + (int64_t)qrow * P.q_ss + (int64_t)head * P.q_sh : nullptr, H, P.head_dim);
+
+    st.init();
+    fetch_by(std::true_type(), ra, 0);
+    if (DEPTH == 2 && n_tiles > 1) fetch_by(std::true_type(), rb, 1);
     stage(0, ra);
     if (DEPTH == 2) { if (n_tiles > 2) fetch(ra, 2); } else { if (n_tiles > 1) fetch(ra, 1); }
     __syncthreads();
@@ -511,11 +549,11 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
     const int64_t slot0 = (((int64_t)b * P.num_q_heads + head) * P.nqt + qt) * P.nsplit;
     if constexpr (!MERGE) {                      // two launches: the combine kernel follows
         if (row_ok) {
-            float* po = P.part_o + ((slot0 + split) * kQTile + r) * kHeadDim;
+            float* po = P.part_o + ((slot0 + split) * 16 * 64 + lane) * 4;
 #pragma unroll
             for (int t = 0; t < kMine; ++t)
 #pragma unroll
-                for (int g = 0; g < 4; ++g) *reinterpret_cast<f32x4*>(po + d_of_reg(kw + KW * t, 4 * g, H)) = own[t][g];
+                for (int g = 0; g < 4; ++g) *reinterpret_cast<f32x4*>(po + ((kw + KW * t) * 4 + g) * 64 * 4) = own[t][g];
             if (kw == 0 && H == 0) *reinterpret_cast<float2*>(P.part_ml + ((slot0 + split) * kQTile + r) * 2) = float2{st.m[0], st.l[0]};
         }
     } else {
@@ -614,10 +652,11 @@ __global__ __launch_bounds__(32 * ROWS) void paged_combine_kernel(const PagedPar
     const unsigned block = blockIdx.x + mdx::fetch_arguments<sizeof(PagedParams)>();
     const int part = block % kParts, rest = block / kParts;
     const int row_tile = mdx::quotient(rest, P.nqt), qt = rest - row_tile * P.nqt, b = mdx::quotient(row_tile, P.num_q_heads), hq = row_tile - b * P.num_q_heads;
-    const int c = (threadIdx.x & 31) * 4, s = part * ROWS + (threadIdx.x >> 5);
+    const int unit = part * (ROWS / 2) + (threadIdx.x >> 6), lane = threadIdx.x & 63;       // a register quad of the attention's wavefronts, and the lane that held it
+    const int c = d_of_reg(unit >> 2, 4 * (unit & 3), lane >> 5), s = lane & 31;
     if (c >= P.head_dim || qt * kQTile + s >= P.sq) return;
     const int64_t slot0 = (((int64_t)b * P.num_q_heads + hq) * P.nqt + qt) * P.nsplit;
-    const float* part_o = P.part_o + (slot0 * kQTile + s) * kHeadDim + c;
+    const float* part_o = P.part_o + ((slot0 * 16 + unit) * 64 + lane) * 4;
     const float2* part_ml = reinterpret_cast<const float2*>(P.part_ml) + slot0 * kQTile + s;
     int nv = P.nsplit;                         // until the lengths are in: every slot that exists
     Fold F;

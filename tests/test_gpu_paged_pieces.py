@@ -37,6 +37,45 @@ def test_pieces_folded_twelve_at_a_time(dev, ctxs):
     test_pieces(dev, ctxs, 0)
 
 
+@pytest.mark.parametrize("ctxs,page,hq,hkv", [
+    ([700, 64, 65, 63, 1], 32, 4, 2),                       # pages smaller than a tile of 64 keys
+    ([700, 300, 96], 96, 4, 2),                             # not a power of two
+    ([700, 64, 127, 128, 129], 64, 4, 2),                   # a tile per page
+    ([1000, 511, 200], 128, 2, 2), ([900, 511, 200], 64, 2, 2),      # one head per workgroup: tiles of 128 keys, as long as a page and longer
+    ([5000] * 2 + [300] * 30, 64, 16, 8),                   # pieces of more pages than a wavefront has lanes
+    ([2600] * 16, 256, 16, 8), ([2200] * 16, 256, 16, 8),   # most resident workgroups used: one lookup per pass after the first tiles; with a merging last workgroup
+])
+def test_tiles_and_pages(dev, ctxs, page, hq, hkv):
+    """A tile's keys looked up by page: rows behind the context hold NaN, and one page in the middle of every longer context has an id that does not
+    exist, so that its keys are left out."""
+    import mdx
+    g = torch.Generator(device=dev).manual_seed(sum(ctxs) + page)
+    d, scale = 128, 128 ** -0.5
+    counts = [-(-c // page) for c in ctxs]
+    pool = sum(counts) + 2
+    q = torch.randn(len(ctxs), 32, hq, d, generator=g, device=dev).bfloat16()
+    kc, vc = (torch.randn(pool, page, hkv, d, generator=g, device=dev).bfloat16() for _ in range(2))
+    bt = torch.full((len(ctxs), max(counts)), -1, dtype=torch.int32)
+    order, at = torch.randperm(pool, generator=g, device=dev).int().cpu(), 0
+    for b, n in enumerate(counts):
+        bt[b, :n] = order[at:at + n]
+        at += n
+        kc[bt[b, n - 1], ctxs[b] - (n - 1) * page:] = float("nan")
+        vc[bt[b, n - 1], ctxs[b] - (n - 1) * page:] = float("nan")
+    holes = [n // 2 if n > 2 else None for n in counts]
+    want = torch.empty(len(ctxs), 32, hq, d)
+    for b, n in enumerate(counts):
+        rows = [r for r in range(n) if r != holes[b]]
+        k, v = (x[bt[b, rows].long().to(dev)].float().flatten(0, 1)[:ctxs[b] - (n - len(rows)) * page].repeat_interleave(hq // hkv, 1) for x in (kc, vc))
+        p = torch.softmax(torch.bmm(q[b].float().transpose(0, 1).contiguous(), k.permute(1, 2, 0).contiguous()) * scale, -1)
+        want[b] = torch.bmm(p, v.transpose(0, 1).contiguous()).transpose(0, 1).cpu()
+        if holes[b] is not None:
+            bt[b, holes[b]] = -1 if b % 2 else pool + 3
+    lens = torch.tensor(ctxs, dtype=torch.int32, device=dev)
+    o = mdx.flash_attn_with_kvcache(q, kc, vc, cache_seqlens=lens, block_table=bt.to(dev), softmax_scale=scale)
+    assert (o.float().cpu() - want).abs().max().item() < 2e-2
+
+
 @pytest.mark.parametrize("bs,hq,hkv,dtype", [(1, 16, 8, torch.bfloat16), (2, 16, 8, torch.bfloat16), (8, 16, 8, torch.bfloat16), (9, 16, 8, torch.bfloat16),
                                              (3, 3, 1, torch.bfloat16), (4, 4, 2, torch.float16), (6, 64, 32, torch.bfloat16), (2, 4, 2, torch.float32)])
 def test_reading_ahead_changes_nothing(dev, bs, hq, hkv, dtype):
