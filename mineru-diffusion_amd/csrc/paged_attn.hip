@@ -63,29 +63,8 @@ template <typename T> __host__ __device__ __forceinline__ bool stay_whole(T long
 constexpr float kWholeFactor = 1.33f, kShareFactor = 1.2f;
 constexpr int kShareKeys = 192;
 
-// Sum over the 64 lanes: DPP shifts inside the rows of 16 lanes, the two row broadcasts, the total from lane 63
-// (six additions, no LDS traffic: the butterfly of cross-lane LDS permutes it replaces sat in every workgroup's start).
-__device__ __forceinline__ int wave_sum(int x) {
-    int v = x;
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);   // row_shr:2
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);   // row_shr:4
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);   // row_shr:8
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
-    return __builtin_amdgcn_readlane(v, 63);
-}
-
-__device__ __forceinline__ int wave_max(int x) {                         // same pattern; x >= 0
-    int v = x;
-    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));
-    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
-    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));
-    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));
-    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));
-    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));
-    return __builtin_amdgcn_readlane(v, 63);
-}
+using mdx::wave_sum;
+using mdx::wave_max;
 
 // Partials that another workgroup of the same launch reads (single-launch merge) travel with
 // agent-scope accesses: such a store is written through to memory and such a load does not take a line
@@ -233,9 +212,17 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
     // ---- workgroup -> (sequence b, split) ------------------------------------------------------
     int b, split, span = P.chunk;
     bool paced = false;
+    typedef __attribute__((address_space(4))) const int32_t ConstantEntry;
+    constexpr bool kGuesses = sizeof...(AHEAD) == 0 && !MERGE;
+    int b_guessed = -1, pages_guessed = 0;
     int ctx_all = 0;                                // (up to 64 sequences) the clipped length of sequence `lane`
     if (P.bs <= 64) {
         // lengths beyond the page table name keys that do not exist: clipped here and below
+        // the first pages of the sequence that this is if all before it in launch order have as many pieces: on their way with the lengths
+        if (kGuesses) {
+            b_guessed = (int)blockIdx.y - mdx::quotient(blockIdx.y, P.bs) * P.bs;
+            pages_guessed = ((ConstantEntry*)(uintptr_t)P.block_table)[(int64_t)b_guessed * P.bt_stride + min(lane, P.max_pages - 1)];
+        }
         const int ctx_l = lane < P.bs ? min(max(0, P.context_lens[lane]), P.max_pages * P.page_size) : 0;
         ctx_all = ctx_l;
         bool cut = true;                            // false: every sequence is known to be one piece
@@ -347,8 +334,7 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
     const int key_end = __builtin_amdgcn_readfirstlane(min(ctx, key_begin + span));
     const int kvh = mdx::quotient(hg * HPW, P.heads_per_kv);
 
-    // (with the readers' loads in the kernel the compiler no longer takes the table for constant by itself)
-    typedef __attribute__((address_space(4))) const int32_t ConstantEntry;
+    // (with the readers' loads in the kernel, or two ways to look pages up, the compiler no longer takes the table for constant by itself)
     auto table_row = [&] {
         const int32_t* row = P.block_table + (int64_t)__builtin_amdgcn_readfirstlane(b) * P.bt_stride;
         return (ConstantEntry*)(uintptr_t)row;
@@ -373,11 +359,12 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
     // (a thread whose 16-byte chunk lies beyond a narrow head reads the head's last chunk instead; zeroed like a row past the end)
     const bool col_ok = chunk * 8 < P.head_dim;
     const int64_t safe_off = (int64_t)trow * P.c_st + (int64_t)kvh * P.c_sh + min(chunk * 8, P.head_dim - 8);
-    const bool tile_in_page = sizeof...(AHEAD) == 0 && P.page_shift >= 0 && P.page_size >= kTileKeys && (key_begin & (kTileKeys - 1)) == 0;
+    const bool tile_in_page = sizeof...(AHEAD) == 0 && WAVES == 4 && P.page_shift >= 0 && P.page_size >= kTileKeys && (key_begin & (kTileKeys - 1)) == 0;
     const bool paged_tiles = tile_in_page && !paced;
     auto slot_of = [&](int key) { return P.page_shift >= 0 ? key >> P.page_shift : key / P.page_size; };
-    const int first_slot = slot_of(key_begin);
-    const int pages = bt[min(first_slot + lane, P.max_pages - 1)];
+    const bool guessed = kGuesses && b == b_guessed && slot_of(key_end - 1) < 64;
+    const int first_slot = guessed ? 0 : slot_of(key_begin);
+    const int pages = guessed ? pages_guessed : bt[min(first_slot + lane, P.max_pages - 1)];
     auto load_k = [&](Staged& sg, int p, int64_t off) { sg.regs.k[p] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(P.k_cache + off)); };
     auto load_v = [&](Staged& sg, int p, int64_t off, bool ok, int key0) {
         sg.regs.v[p] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(P.v_cache + off));
@@ -490,21 +477,21 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
     constexpr int kStateFloats = 4 * 16 * 64 + 2 * 64;
     static_assert(HPW * KW * kStateFloats * 4 <= (int)sizeof(lds), "merge buffer exceeds the tile region");
     float* xch = reinterpret_cast<float*>(&lds[0][0]) + (wave / KW) * KW * kStateFloats;   // this head's slots
-    // (the loop's last barrier already separates the tile reads from these writes)
-    {
-        float* dst = xch + kw * kStateFloats;
+    // (the loop's last barrier already separates the tile reads from these writes; what a slice folds itself stays in its registers: with all of every state written and read,
+    // 128 KB through LDS, the merge took 1960 cycles of a workgroup's 14 500 of one sequence, so 1400)
+    f32x4 own[4 / KW][4];                           // what this slice folds: d tiles kw, kw + KW, ...
+    auto exchange = [&](auto slice) {
+        constexpr int MINE = decltype(slice)::value;
+        auto quad = [&](int t, int g) { return f32x4{st.o[0][t][4 * g], st.o[0][t][4 * g + 1], st.o[0][t][4 * g + 2], st.o[0][t][4 * g + 3]}; };
+        float* dst = xch + MINE * kStateFloats;
 #pragma unroll
         for (int t = 0; t < 4; ++t)
 #pragma unroll
             for (int g = 0; g < 4; ++g)
-                *reinterpret_cast<f32x4*>(dst + ((t * 4 + g) * 64 + lane) * 4) =
-                    f32x4{st.o[0][t][4 * g], st.o[0][t][4 * g + 1], st.o[0][t][4 * g + 2], st.o[0][t][4 * g + 3]};
+                if (t % KW != MINE) *reinterpret_cast<f32x4*>(dst + ((t * 4 + g) * 64 + lane) * 4) = quad(t, g);
         dst[4 * 16 * 64 + lane] = st.m[0];
         dst[4 * 16 * 64 + 64 + lane] = st.l[0];
-    }
-    __syncthreads();
-    f32x4 own[4 / KW][4];                           // what this slice folds: d tiles kw, kw + KW, ...
-    {
+        __syncthreads();
         float w[KW];                                // weights of the KW states: 2^(m_s - M)
         float M = kMinusBig;
 #pragma unroll
@@ -524,8 +511,50 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
                 own[t][g] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int s = 0; s < KW; ++s)
-                    own[t][g] += *reinterpret_cast<const f32x4*>(xch + s * kStateFloats + (((kw + KW * t) * 4 + g) * 64 + lane) * 4) * w[s];
+                    own[t][g] += (s == MINE ? quad(MINE + KW * t, g) : *reinterpret_cast<const f32x4*>(xch + s * kStateFloats + (((MINE + KW * t) * 4 + g) * 64 + lane) * 4)) * w[s];
             }
+    };
+    // (kw is the same throughout a wavefront; each meets one barrier, whichever branch it takes.  Of four slices each keeps a quarter only: 32 sequences of 1150 keys,
+    // whose merge is all through LDS, 42.6 us, with four branches 42.9.)
+    if constexpr (KW == 2) {
+        if (__builtin_amdgcn_readfirstlane(kw) == 0) exchange(std::integral_constant<int, 0>());
+        else exchange(std::integral_constant<int, 1>());
+    } else {
+        {
+            float* dst = xch + kw * kStateFloats;
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    *reinterpret_cast<f32x4*>(dst + ((t * 4 + g) * 64 + lane) * 4) =
+                        f32x4{st.o[0][t][4 * g], st.o[0][t][4 * g + 1], st.o[0][t][4 * g + 2], st.o[0][t][4 * g + 3]};
+            dst[4 * 16 * 64 + lane] = st.m[0];
+            dst[4 * 16 * 64 + 64 + lane] = st.l[0];
+        }
+        __syncthreads();
+        {
+            float w[KW];                                // weights of the KW states: 2^(m_s - M)
+            float M = kMinusBig;
+#pragma unroll
+            for (int s = 0; s < KW; ++s) { w[s] = xch[s * kStateFloats + 4 * 16 * 64 + lane]; M = fmaxf(M, w[s]); }
+            float l = 0.f;
+#pragma unroll
+            for (int s = 0; s < KW; ++s) {
+                w[s] = __builtin_amdgcn_exp2f(w[s] - M);
+                l += xch[s * kStateFloats + 4 * 16 * 64 + 64 + lane] * w[s];
+            }
+            st.m[0] = M;
+            st.l[0] = l;
+#pragma unroll
+            for (int t = 0; t < 4 / KW; ++t)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    own[t][g] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int s = 0; s < KW; ++s)
+                        own[t][g] += *reinterpret_cast<const f32x4*>(xch + s * kStateFloats + (((kw + KW * t) * 4 + g) * 64 + lane) * 4) * w[s];
+                }
+        }
     }
 
     // ---- output: slice kw holds, and stores, the d tiles kw, kw + KW, ... of its head ----------------
