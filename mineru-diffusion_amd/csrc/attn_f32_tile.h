@@ -10,6 +10,7 @@
 // in LDS as fp32.
 #pragma once
 #include "mdx_common.h"
+#include <type_traits>
 
 namespace mdx_attn_f32 {
 
@@ -220,48 +221,59 @@ __device__ __forceinline__ void tile_step(const float* lds, const float (&q)[D /
 // KW-th column tile.  m and l come back whole before the first emit.  Called by all wavefronts; the region must hold their states.
 template <int D, int KW, typename Emit>
 __device__ __forceinline__ void fold_states(float* lds, State<D>& st, int wave, int lane, int width, Emit emit) {
-    constexpr int kMl = (D / 32) * 16 * 64, kStateFloats = kMl + 2 * 64;       // O as [d tile][register][lane], then m, l
+    constexpr int kMl = (D / 32) * 16 * 64, kStateFloats = kMl + 2 * 64;       // O as [d tile][register quad][lane][4], then m, l
     const int H = lane >> 5, kw = wave % KW;
     st.l += __shfl_xor(st.l, 32);                                              // a state is now (m, l, O) per query
     const float* states = lds + (wave - kw) * kStateFloats;
-    float w[KW];
-    if (KW > 1) {
-        __syncthreads();                                                       // the last tiles have been read by everybody
-        float* dst = lds + wave * kStateFloats;
+    auto quad = [&](int dt, int g) { return f32x4{st.o[dt][4 * g], st.o[dt][4 * g + 1], st.o[dt][4 * g + 2], st.o[dt][4 * g + 3]}; };
+    // MINE: this wavefront's kw.  What it hands out itself stays in its registers.  (All of every state through LDS, four bytes at a time: 3600 cycles of a workgroup's
+    // 24 900 of one sequence of 1056 keys.)
+    auto fold = [&](auto mine) {
+        constexpr int MINE = decltype(mine)::value;
+        float w[KW];
+        if (KW > 1) {
+            __syncthreads();                                                   // the last tiles have been read by everybody
+            float* dst = lds + wave * kStateFloats;
 #pragma unroll
-        for (int dt = 0; dt < D / 32; ++dt)
+            for (int dt = 0; dt < D / 32; ++dt)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) dst[(dt * 16 + i) * 64 + lane] = st.o[dt][i];
-        dst[kMl + lane] = st.m;
-        dst[kMl + 64 + lane] = st.l;
-        __syncthreads();
-        float M = kMinusBig, l_all = 0.f;
+                for (int g = 0; g < 4; ++g)
+                    if (dt % KW != MINE) *reinterpret_cast<f32x4*>(dst + ((dt * 4 + g) * 64 + lane) * 4) = quad(dt, g);
+            dst[kMl + lane] = st.m;
+            dst[kMl + 64 + lane] = st.l;
+            __syncthreads();
+            float M = kMinusBig, l_all = 0.f;
 #pragma unroll
-        for (int s = 0; s < KW; ++s) { w[s] = states[s * kStateFloats + kMl + lane]; M = fmaxf(M, w[s]); }
+            for (int s = 0; s < KW; ++s) { w[s] = states[s * kStateFloats + kMl + lane]; M = fmaxf(M, w[s]); }
 #pragma unroll
-        for (int s = 0; s < KW; ++s) {
-            w[s] = __builtin_amdgcn_exp2f(w[s] - M);
-            l_all += states[s * kStateFloats + kMl + 64 + lane] * w[s];
-        }
-        st.m = M;
-        st.l = l_all;
-    }
-#pragma unroll
-    for (int dt = 0; dt < D / 32; ++dt) {
-        if (dt % KW != kw || dt * 32 >= width) continue;                       // (uniform per wavefront)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                if (KW == 1) acc[e] = st.o[dt][4 * g + e];
-#pragma unroll
-                for (int s = 0; KW > 1 && s < KW; ++s) acc[e] += states[s * kStateFloats + (dt * 16 + 4 * g + e) * 64 + lane] * w[s];
+            for (int s = 0; s < KW; ++s) {
+                w[s] = __builtin_amdgcn_exp2f(w[s] - M);
+                l_all += states[s * kStateFloats + kMl + 64 + lane] * w[s];
             }
-            const int d = dt * 32 + 8 * g + 4 * H;
-            if (d < width) emit(d, acc);
+            st.m = M;
+            st.l = l_all;
         }
-    }
+#pragma unroll
+        for (int dt = MINE; dt < D / 32; dt += KW) {
+            if (dt * 32 >= width) continue;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+                if (KW == 1) acc = quad(dt, g);
+#pragma unroll
+                for (int s = 0; KW > 1 && s < KW; ++s)
+                    acc += (s == MINE ? quad(dt, g) : *reinterpret_cast<const f32x4*>(states + s * kStateFloats + ((dt * 4 + g) * 64 + lane) * 4)) * w[s];
+                const int d = dt * 32 + 8 * g + 4 * H;
+                if (d < width) emit(d, acc);
+            }
+        }
+    };
+    // (the same throughout a wavefront; each meets the same barriers, whichever branch it takes)
+    const int slice = __builtin_amdgcn_readfirstlane(kw);
+    if (KW == 1 || slice == 0) fold(std::integral_constant<int, 0>());
+    else if (slice == 1) fold(std::integral_constant<int, 1 % KW>());
+    else if (slice == 2) fold(std::integral_constant<int, 2 % KW>());
+    else fold(std::integral_constant<int, 3 % KW>());
 }
 template <int D> constexpr int kStateBytes = ((D / 32) * 16 * 64 + 2 * 64) * (int)sizeof(float);
 

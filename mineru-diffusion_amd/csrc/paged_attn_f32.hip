@@ -50,18 +50,25 @@ __device__ __forceinline__ int keys_of(const PagedWideParams& P, int b) {
 // Keys per piece of sequence b (all wavefronts of both kernels find the same).  Pieces of one size for all sequences, so that a
 // long sequence gets more of them and all workgroups run equally long: total keys / pieces, but never more pieces of a
 // sequence than it has slots.  Beyond 64 sequences, whose lengths no wavefront holds, a sequence is cut evenly.
+// QUICK: the sum by DPP shifts, 1200 cycles less of a workgroup's start.  Not in launches of several rounds per piece: there it is up to 2 % slower where all workgroups are equal
+// (us, by shuffles / by shifts: 1 x 16 300 keys 65.4 / 67.2, 1 x 14 000 63.8 / 64.9, 4 x 4000 73.6 / 74.5; but 8 x 300-2000 64.2 / 62.4).  Probably the two
+// workgroups of a CU stay in step then, stage at the same time and multiply at the same time; a wave priority for one of them undid that there and cost 1 % elsewhere.
+template <bool QUICK>
 __device__ __forceinline__ int keys_per_piece(const PagedWideParams& P, int ctx, int lane) {
     int want = (ctx + P.nsplit - 1) / P.nsplit;
     if (P.bs <= 64) {
         int total = lane < P.bs ? keys_of(P, lane) : 0;
+        if (QUICK) total = mdx::wave_sum(total);
 #pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) total += __shfl_xor(total, off);
+        for (int off = 32; !QUICK && off >= 1; off >>= 1) total += __shfl_xor(total, off);
         want = max(want, (total + P.pieces - 1) / P.pieces);
     }
     return max(1, (want + kLeastKeys - 1) / kLeastKeys) * kLeastKeys;
 }
 
-template <typename T, int D, int HPW, int KW>
+// ONE_ROUND: pieces of KW tiles at most, whose loads are on their way before the queries go through LDS and their pages are looked up in a register.  (Where there
+// are more rounds the same start, or the next round's loads ahead of the products, is slower: 1 x 4000 keys 34.9 -> 35.5 us, 1 x 16 000 66 -> 67.5 and 70.)
+template <typename T, int D, int HPW, int KW, bool ONE_ROUND>
 __global__ __launch_bounds__(64 * HPW * KW, D <= 128 && KW <= 2 ? 2 : 1) void paged_attn_f32_kernel(const PagedWideParams P)
 {
     constexpr int kThreads = 64 * HPW * KW;
@@ -79,7 +86,7 @@ __global__ __launch_bounds__(64 * HPW * KW, D <= 128 && KW <= 2 ? 2 : 1) void pa
     const int ctx = keys_of(P, b);
     const T* q0 = static_cast<const T*>(P.q) + (int64_t)b * P.q_sb + (int64_t)(qt * 32) * P.q_ss + (int64_t)(head - hw) * P.q_sh;
     queries.fetch(tid, width, [&](int row) { return qt * 32 + row % 32 < P.sq ? q0 + (int64_t)(row % 32) * P.q_ss + (int64_t)(row / 32) * P.q_sh : nullptr; });
-    const int span = P.nsplit > 1 ? keys_per_piece(P, ctx, lane) : max(1, ctx);
+    const int span = P.nsplit > 1 ? keys_per_piece<ONE_ROUND>(P, ctx, lane) : max(1, ctx);
     const int n_pieces = max(1, (ctx + span - 1) / span);
     if (split >= n_pieces) return;
     const int key_begin = split * span, key_end = min(ctx, key_begin + span);
@@ -92,18 +99,24 @@ __global__ __launch_bounds__(64 * HPW * KW, D <= 128 && KW <= 2 ? 2 : 1) void pa
     const T* vc = static_cast<const T*>(P.v_cache) + (int64_t)kvh * P.c_sh;
 
     float q[D / 2];
-    queries.write(lds, tid);
-    __syncthreads();
-    queries.read(q, lds, hw, H, r, width);
+    auto hand_out_queries = [&] {
+        queries.write(lds, tid);
+        __syncthreads();
+        queries.read(q, lds, hw, H, r, width);
+    };
+    if (!ONE_ROUND) hand_out_queries();
+    const int first_slot = P.page_shift >= 0 ? key_begin >> P.page_shift : key_begin / P.page_size;
+    const int pages = ONE_ROUND ? bt[min(first_slot + lane, P.max_pages - 1)] : 0;
     State<D> st;
     st.init();
-    for (int t0 = 0; t0 < n_tiles; t0 += KW) {
+    for (int t0 = 0; t0 < (ONE_ROUND ? 1 : n_tiles); t0 += KW) {
         // ---- tiles t0 .. t0 + KW - 1 into LDS, all threads on each (a tile never straddles a page: page_size % 32 == 0, so that all
         //      its rows exist in memory, whatever they hold) ----
         unsigned tile_ok = 0;                                  // bit i: tile t0 + i exists and lies on a valid page (uniform)
         // tiles whose loads are in flight together: as registers allow (two instead of one at 128 columns: 8 x 4000-9000 keys
             // 192 -> 186 us, 1 x 4000 35.2 -> 34.4, 1 x 1056 and shorter level)
             constexpr int kTogether = KW == 4 ? 4 : D <= 128 ? KW : 1;
+            static_assert(!ONE_ROUND || (kTogether == KW && TileRegs<T, D, kThreads>::kBatches == 1), "a round in registers");
         TileRegs<T, D, kThreads> regs[kTogether];
 #pragma unroll
         for (int i0 = 0; i0 < KW; i0 += kTogether) {
@@ -112,7 +125,7 @@ __global__ __launch_bounds__(64 * HPW * KW, D <= 128 && KW <= 2 ? 2 : 1) void pa
             for (int j = 0; j < kTogether; ++j) {
                 const int key0 = key_begin + (t0 + i0 + j) * kTileKeys;
                 const int page_slot = P.page_shift >= 0 ? key0 >> P.page_shift : key0 / P.page_size;
-                const int64_t page = key0 < key_end ? bt[page_slot] : -1;
+                const int64_t page = key0 >= key_end ? -1 : ONE_ROUND ? __builtin_amdgcn_readlane(pages, page_slot - first_slot) : bt[page_slot];
                 if (page >= 0 && page < P.num_pages) tile_ok |= 1u << (i0 + j);
                 base[j] = page * P.c_sp + (int64_t)(key0 - page_slot * P.page_size) * P.c_st;
             }
@@ -122,6 +135,7 @@ __global__ __launch_bounds__(64 * HPW * KW, D <= 128 && KW <= 2 ? 2 : 1) void pa
                 for (int j = 0; j < kTogether; ++j)
                     if ((tile_ok >> (i0 + j)) & 1u)
                         regs[j].fetch(b, tid, width, [&](int row) { return kc + base[j] + (int64_t)row * P.c_st; }, [&](int row) { return vc + base[j] + (int64_t)row * P.c_st; });
+                if (ONE_ROUND) hand_out_queries();
                 if (i0 == 0 && b == 0) __syncthreads();        // the queries or the previous tiles have been read by everybody
 #pragma unroll
                 for (int j = 0; j < kTogether; ++j)
@@ -182,7 +196,7 @@ __global__ __launch_bounds__(kFoldRows * D / 4) void paged_combine_f32_kernel(co
     };
     load(0, P.nsplit);
     const int ctx = keys_of(P, b);
-    const int span = keys_per_piece(P, ctx, threadIdx.x & 63);
+    const int span = keys_per_piece<true>(P, ctx, threadIdx.x & 63);
     const int n = __builtin_amdgcn_readfirstlane((ctx + span - 1) / span);
     if (n <= 1 || qrow >= P.sq || d >= P.head_dim) return;      // one piece: written by the attention kernel
     float M = kMinusBig, L = 0.f;
@@ -226,7 +240,7 @@ int splits_wanted(int64_t bs, int nqt, int num_q_heads, int64_t max_keys) {
     return n < 1 ? 1 : (int)n;
 }
 
-template <typename T, int D, int HPW, int KW>
+template <typename T, int D, int HPW, int KW, bool ONE_ROUND = false>
 int launch_groups(const PagedWideParams& P, hipStream_t stream)
 {
     constexpr int kLdsBytes = KW * Lds<D>::kBytes;
@@ -236,12 +250,12 @@ int launch_groups(const PagedWideParams& P, hipStream_t stream)
     hipError_t e = hipGetDevice(&device);
     MDX_REQUIRE(e == hipSuccess && device >= 0 && device < 64, MDX_ELAUNCH, "paged_block_attn: no current device (%s)", hipGetErrorString(e));
     if (!raised[device].load(std::memory_order_acquire)) {
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(paged_attn_f32_kernel<T, D, HPW, KW>), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+        e = hipFuncSetAttribute(reinterpret_cast<const void*>(paged_attn_f32_kernel<T, D, HPW, KW, ONE_ROUND>), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
         MDX_REQUIRE(e == hipSuccess, MDX_ELAUNCH, "paged_block_attn: cannot reserve %d bytes of LDS (%s)", kLdsBytes, hipGetErrorString(e));
         raised[device].store(true, std::memory_order_release);
     }
     const dim3 grid((unsigned)(P.num_q_heads / HPW * P.nqt), (unsigned)P.nsplit, (unsigned)P.bs);
-    paged_attn_f32_kernel<T, D, HPW, KW><<<grid, 64 * HPW * KW, kLdsBytes, stream>>>(P);
+    paged_attn_f32_kernel<T, D, HPW, KW, ONE_ROUND><<<grid, 64 * HPW * KW, kLdsBytes, stream>>>(P);
     const int rc = mdx::check_launch("paged_block_attn (fp32 arithmetic)");
     if (rc != MDX_OK || P.nsplit == 1) return rc;
     const dim3 fold((unsigned)(P.num_q_heads * P.nqt * kFoldParts), (unsigned)P.bs);
@@ -263,6 +277,11 @@ int launch(const PagedWideParams& P, hipStream_t stream)
     if (P.nsplit == 1 && (int64_t)P.bs * P.num_q_heads * P.nqt <= mdx::compute_units())
         return P.head_dim <= 128 ? launch_groups<T, 128, 1, 4>(P, stream) : launch_groups<T, 256, 1, 2>(P, stream);
     const bool pairs = P.heads_per_kv % 2 == 0;
+    // pieces of the least size, whatever the lengths: no more keys in the tables than the pieces and the slots hold of it.  (Us: 1 x 1024 keys 20.0 / 19.4, 3 x 100-400
+    // 19.0 / 18.4; a head per workgroup loads its tiles in two batches.)
+    const int64_t max_keys = (int64_t)P.max_pages * P.page_size;
+    const bool one_round = P.bs <= 64 && P.bs * max_keys <= (int64_t)kLeastKeys * P.pieces && max_keys <= (int64_t)kLeastKeys * P.nsplit;
+    if (P.head_dim <= 128 && pairs && one_round && P.nsplit > 1) return launch_groups<T, 128, 2, 2, true>(P, stream);
     if (P.head_dim <= 128) return pairs ? launch_groups<T, 128, 2, 2>(P, stream) : launch_groups<T, 128, 1, 2>(P, stream);
     return pairs ? launch_groups<T, 256, 2, 1>(P, stream) : launch_groups<T, 256, 1, 1>(P, stream);
 }

@@ -266,6 +266,30 @@ def test_fp32_sequence_bounds_are_clipped_to_the_tensors(dev):
     assert (o[:60].cpu() - ref[:60]).abs().max().item() < TOL_F32
 
 
+@pytest.mark.parametrize("hq,hkv,page,width", [(4, 2, 32, 0), (4, 2, 96, 0), (16, 8, 64, 0),      # every piece one round: two tiles on one page, on two, on either side of its end
+                                               (16, 8, 256, 14), (16, 8, 256, 40), (3, 3, 64, 0)])    # ... and, by the tables' width or the heads, not
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_paged_fp32_pieces_of_one_round(dev, hq, hkv, page, width, dtype):
+    """Lengths at the edges of tiles and pieces, NaN behind the context and a page in the middle that does not exist (its keys are left out)."""
+    import mdx
+    ctxs, d, g = [1, 33, 64, 65, 300, 700], 100 if dtype == torch.bfloat16 else 128, torch.Generator().manual_seed(page + width)
+    q, kc, vc, bt, lens = _paged_inputs(g, ctxs, 32, hq, hkv, d, dtype, page=page, pool=80)
+    bt = torch.cat([bt, torch.full((len(ctxs), max(0, width - bt.shape[1])), -1, dtype=torch.int32)], 1)
+    for b, c in enumerate(ctxs):
+        if c % page:
+            kc[bt[b, c // page], c % page:] = float("nan")
+            vc[bt[b, c // page], c % page:] = float("nan")
+    ref = oracle.paged_block_attn(q, kc, vc, bt, lens, d ** -0.5)
+    n = 700 // page // 2
+    keep = [i for i in range(-(-700 // page)) if i != n]
+    short = torch.full_like(bt[:1], -1)
+    short[0, :len(keep)] = bt[5, keep]
+    ref[5] = oracle.paged_block_attn(q[5:], kc, vc, short, lens[5:] - page, d ** -0.5)[0]
+    bt[5, n] = 80
+    o = mdx.flash_attn_with_kvcache(q.to(dev), kc.to(dev), vc.to(dev), cache_seqlens=lens.to(dev), block_table=bt.to(dev), softmax_scale=d ** -0.5)
+    assert (o.float().cpu() - ref).abs().max().item() < (TOL_F32 if dtype == torch.float32 else TOL_16)
+
+
 @pytest.mark.parametrize("ctxs", [[63, 64, 65, 127, 129], [3000] + [40] * 9, [70] * 70])
 @pytest.mark.parametrize("room", [0.0, 0.4, 1.0])
 def test_paged_fp32_contexts_cut_into_pieces(dev, ctxs, room):
