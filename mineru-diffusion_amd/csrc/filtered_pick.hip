@@ -132,8 +132,8 @@ __device__ __forceinline__ void better(Pick& a, float v, float x, int column) {
 __device__ __forceinline__ Pick wave_best(Pick p) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
-        const float v = __shfl_xor(p.v, off), x = __shfl_xor(p.x, off);
-        const int column = __shfl_xor(p.column, off);
+        const float v = mdx::xor_lanes(p.v, off), x = mdx::xor_lanes(p.x, off);
+        const int column = mdx::xor_lanes(p.column, off);
         better(p, v, x, column);
     }
     return p;
@@ -157,7 +157,7 @@ __device__ __forceinline__ void pick_from_kept(uint32_t (&key)[N], const int (&c
 #pragma unroll
     for (int i = 0; i < N; ++i) mk = max(mk, key[i]);
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) mk = max(mk, (uint32_t)__shfl_xor((int)mk, off));
+    for (int off = 32; off >= 1; off >>= 1) mk = max(mk, (uint32_t)mdx::xor_lanes((int)mk, off));
     if (mk == 0) { x0 = 0; x0_p = 0.f; return; }                            // no finite logit
     const float m = value_of_key<T>(mk);
     // The kept elements come in no order, so their masses are summed in fixed point: the same logits give the same cut-off and
@@ -188,7 +188,7 @@ __device__ __forceinline__ void pick_from_kept(uint32_t (&key)[N], const int (&c
             }
             floor_key = above > target ? key[0] : 0;
 #pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) floor_key = max(floor_key, (uint32_t)__shfl_xor((int)floor_key, off));
+            for (int off = 32; off >= 1; off >>= 1) floor_key = max(floor_key, (uint32_t)mdx::xor_lanes((int)floor_key, off));
         }
         for (int bit = 15; N > 1 && bit >= 0; --bit) {
             const uint32_t trial = floor_key | (1u << bit);
@@ -336,7 +336,7 @@ __global__ __launch_bounds__(kPickThreads) void filtered_pick_kernel(
     auto kept = [&](uint32_t b) { return b != Bits16<T>::kNegInf && key_of(b) >= floor_key; };
     scan_row<kPickThreads>(row, tid, [&](uint32_t b, int) { if (kept(b)) m = fmaxf(m, Bits16<T>::value(b)); });
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+    for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, mdx::xor_lanes(m, off));
     __syncthreads();
     if (lane == 0) fslot[tid >> 6] = m;
     __syncthreads();

@@ -71,7 +71,7 @@ __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(const NormPa
         }
     }
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) sq += __shfl_xor(sq, o);
+    for (int o = 32; o >= 1; o >>= 1) sq += mdx::xor_lanes(sq, o);
     if ((tid & 63) == 0) wave_sums[tid >> 6] = sq;
     __syncthreads();
     float total = 0.f;
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(THREADS) void add_rms_norm_partials_kernel(const No
         for (int e = 0; e < 4; ++e) sq += s[i][e] * s[i][e];
     }
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) sq += __shfl_xor(sq, o);
+    for (int o = 32; o >= 1; o >>= 1) sq += mdx::xor_lanes(sq, o);
     if ((tid & 63) == 0) wave_sums[tid >> 6] = sq;
     __syncthreads();
     float total = 0.f;

@@ -85,7 +85,7 @@ template <int MT> struct Rows {
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
             for (int off = 16; off <= 32; off <<= 1)
-                merge(st[mt], __shfl_xor(st[mt].m, off), __shfl_xor(st[mt].s, off), __shfl_xor(st[mt].idx, off), c[mt]);
+                merge(st[mt], mdx::xor_lanes(st[mt].m, off), mdx::xor_lanes(st[mt].s, off), mdx::xor_lanes(st[mt].idx, off), c[mt]);
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // the x tiles have been read by everybody
         State* states = reinterpret_cast<State*>(lds);                       // [wave][16 MT]
         if (lane < 16) {

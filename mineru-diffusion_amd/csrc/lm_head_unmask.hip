@@ -200,8 +200,8 @@ __global__ __launch_bounds__(kFoldThreads) void lm_head_finalize_kernel(const Lm
     }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
-        const float m2 = __shfl_xor(m, off), s2 = __shfl_xor(s, off);
-        const int i2 = __shfl_xor(idx, off);
+        const float m2 = mdx::xor_lanes(m, off), s2 = mdx::xor_lanes(s, off);
+        const int i2 = mdx::xor_lanes(idx, off);
         fold(m2, s2, i2);
     }
     if (lane == 0) {

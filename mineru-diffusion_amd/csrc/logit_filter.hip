@@ -105,7 +105,7 @@ __device__ uint32_t floor_from_counts(const RowView& row, uint32_t* hist, Scratc
     if (top_p >= 1.0f) return floor_key;
 
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) top = max(top, __shfl_xor(top, off));
+    for (int off = 32; off >= 1; off >>= 1) top = max(top, mdx::xor_lanes(top, off));
     __syncthreads();
     if (lane == 0) sh.islot[tid >> 6] = top;
     __syncthreads();

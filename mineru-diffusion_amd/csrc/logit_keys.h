@@ -78,7 +78,7 @@ __device__ __forceinline__ bool has_masses(float m, float c) { return m > -INFIN
 
 template <typename V> __device__ __forceinline__ V wave_total(V v) {
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off);
+    for (int off = 32; off >= 1; off >>= 1) v += mdx::xor_lanes(v, off);
     return v;
 }
 
@@ -112,7 +112,7 @@ __device__ uint32_t floor_by_bisection(const RowView& row, int tid, int top_k, f
     if (top_p < 1.0f) {
         scan_row<THREADS>(row, tid, [&](uint32_t b, int) { mk = max(mk, key_of(b)); });
 #pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) mk = max(mk, (uint32_t)__shfl_xor((int)mk, off));
+        for (int off = 32; off >= 1; off >>= 1) mk = max(mk, (uint32_t)mdx::xor_lanes((int)mk, off));
         __syncthreads();
         if ((tid & 63) == 0) islot[tid >> 6] = (int)mk;
         __syncthreads();

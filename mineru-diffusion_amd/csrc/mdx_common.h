@@ -82,6 +82,31 @@ __device__ __forceinline__ int wave_max(int x) {                         // same
     return __builtin_amdgcn_readlane(v, 63);
 }
 
+// The value (of 4 or 8 bytes) of the lane whose number differs in the one bit `mask`, a constant once loops are unrolled; all 64 lanes take part.  In the vector unit: a permute
+// through LDS is a trip of over 100 cycles, and a reduction over a wavefront is six of them one behind the other.  Norms, the pick behind a filter, by permutes / so: one request through the
+// engine 61.9 / 61.2 ms, 12 x 32 rows filtered with a top-k of 50 34.1 / 33.8 us, of 400 54.6 / 53.1, 3 x 32 rows 20.1 / 19.6.  Not everywhere: the vocabulary pass, whose reduction ends
+// every workgroup, is slower so (32 rows 10.97 / 11.99 us; why is not known), and the head's epilogue too (100 rows 155.0 / 155.5).
+__device__ __forceinline__ unsigned xor_lanes_word(unsigned x, int mask) {
+    const bool upper = (__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0)) & mask) != 0;
+    switch (mask) {
+    case 1: return __builtin_amdgcn_update_dpp(0, x, 0xb1, 0xf, 0xf, false);                                                             // quad_perm 1 0 3 2
+    case 2: return __builtin_amdgcn_update_dpp(0, x, 0x4e, 0xf, 0xf, false);                                                             // quad_perm 2 3 0 1
+    case 4: return __builtin_amdgcn_update_dpp(0, __builtin_amdgcn_update_dpp(0, x, 0x141, 0xf, 0xf, false), 0x1b, 0xf, 0xf, false);     // row_half_mirror, quad_perm 3 2 1 0
+    case 8: return __builtin_amdgcn_update_dpp(0, x, 0x128, 0xf, 0xf, false);                                                            // row_ror:8
+    case 16: { const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false); return upper ? r[0] : r[1]; }
+    default: { const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false); return upper ? r[0] : r[1]; }
+    }
+}
+template <typename V> __device__ __forceinline__ V xor_lanes(V v, int mask) {
+    static_assert(sizeof(V) == 4 || sizeof(V) == 8, "words");
+    if constexpr (sizeof(V) == 4) {
+        return __builtin_bit_cast(V, xor_lanes_word(__builtin_bit_cast(unsigned, v), mask));
+    } else {
+        const unsigned long long x = __builtin_bit_cast(unsigned long long, v);
+        return __builtin_bit_cast(V, (unsigned long long)xor_lanes_word((unsigned)(x >> 32), mask) << 32 | xor_lanes_word((unsigned)x, mask));
+    }
+}
+
 // n / d of wavefront-uniform numbers for a d that the compiler doesn't know and that is mostly a power of two (heads, groups of heads, tiles): the general
 // sequence goes through a float reciprocal in the vector unit and back, in every workgroup's start.  Attention calls, us, by that sequence / so: paged, one sequence of 1337 keys 14.6 / 14.35, four of 1000-3000
 // 23.0 / 22.7, 32 of 600-2400 55.9 / 55.5; prompts 3 x 40-150 7.75 / 7.6, 500 13.4 / 13.2.  (In fp32 arithmetic 20.2 / 20.4: not there.)

@@ -66,9 +66,9 @@ __device__ __forceinline__ void finish_row(const RowParams& P, int64_t tok, int 
         float ss = 0.f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) { const float x = (float)a[e], y = (float)b[e]; ss += x * x + y * y; }
-        ss += __shfl_xor(ss, 1);
-        ss += __shfl_xor(ss, 2);
-        ss += __shfl_xor(ss, 4);
+        ss += mdx::xor_lanes(ss, 1);
+        ss += mdx::xor_lanes(ss, 2);
+        ss += mdx::xor_lanes(ss, 4);
         const float inv = rsqrtf(ss * (1.0f / kHeadDim) + P.eps);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
