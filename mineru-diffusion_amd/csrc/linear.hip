@@ -36,7 +36,8 @@ struct LinearParams {
     Operands in;
     __bf16* y; float* partials;                    // y: [M, N]; partials: [splits, M, N]
     int64_t y_stride;                              // elements between rows
-    int K, m_tiles, n_tiles, splits;
+    int k_split, splits;                           // elements of K per slice
+    Places places;
     RowParams rows;                                // heads
 };
 
@@ -70,8 +71,8 @@ __global__ __launch_bounds__(T::kThreads, T::kWaves / 4) void linear_kernel(cons
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     constexpr int TM = T::TM, TN = T::TN;
     const T tile;
-    const Place at = place_of((int)blockIdx.x + mdx::fetch_arguments<sizeof(LinearParams)>(gridDim.x), A.m_tiles, A.n_tiles);
-    const int m0 = at.m * T::BM, n0 = at.n * T::kCols, k_split = A.K / A.splits;
+    const Place at = place_of(blockIdx.x + mdx::fetch_arguments<sizeof(LinearParams)>(), A.places);
+    const int m0 = at.m * T::BM, n0 = at.n * T::kCols;
     // heads: a column tile is one head row of every token, eight lanes of this thread's go to a token's; its place in the rotation
     // and the cache is asked for ahead of the product
     constexpr int kTokens = T::kThreads / mdx_qk::kLanesPerRow, kPasses = FORM == kHeads ? T::BM / kTokens : 1;
@@ -84,7 +85,7 @@ __global__ __launch_bounds__(T::kThreads, T::kWaves / 4) void linear_kernel(cons
         weight = mdx_qk::weight_of_row(A.rows, at.n, j8);
     }
     typename T::Sums acc;
-    tile.product(A.in, m0, n0, (int64_t)at.split * k_split, k_split / kStepK, lds, acc);
+    tile.product(A.in, m0, n0, (int64_t)at.split * A.k_split, A.k_split / kStepK, lds, acc);
 
     // where two wavefronts share a tile, each holds the sums over its halves of the steps, and finishes half of the rows
     constexpr int H = TM / T::WK;
@@ -172,10 +173,11 @@ int launch(LinearParams A, hipStream_t stream)
     static std::atomic<bool> raised[64];
     const int rc = reserve_lds(reinterpret_cast<const void*>(linear_kernel<T, FORM>), kLdsBytes, raised, "linear");
     if (rc != MDX_OK) return rc;
-    A.m_tiles = (A.in.M + BM - 1) / BM;
-    A.n_tiles = (A.in.N + T::kCols - 1) / T::kCols;
-    const int64_t grid = (int64_t)A.m_tiles * A.n_tiles * A.splits;
+    const int m_tiles = (A.in.M + BM - 1) / BM, n_tiles = (A.in.N + T::kCols - 1) / T::kCols;
+    const int64_t grid = (int64_t)m_tiles * n_tiles * A.splits;
     MDX_REQUIRE(grid < ((int64_t)1 << 31), MDX_EUNSUPPORTED, "linear: %lld tiles", (long long)grid);
+    A.places = places_of(m_tiles, n_tiles, grid);
+    A.k_split /= A.splits;
     linear_kernel<T, FORM><<<(unsigned)grid, T::kThreads, kLdsBytes, stream>>>(A);
     return mdx::check_launch("linear");
 }
@@ -289,7 +291,7 @@ LinearParams params_of(const void* x, int64_t x_row_stride, const void* w, int64
 {
     LinearParams A{};
     A.in = Operands{(const __bf16*)x, (const __bf16*)w, x_row_stride, w_row_stride, (int)rows, (int)n};
-    A.K = (int)k; A.splits = 1;
+    A.k_split = (int)k; A.splits = 1;
     return A;
 }
 

@@ -21,7 +21,8 @@ struct LmHeadParams {
 __device__ __forceinline__ float row_scale(const LmHeadParams& P, int row) {
     if (!P.temperatures || row >= P.rows) return kLog2e;
     const int64_t id = P.row_ids ? P.row_ids[row] : row;
-    return kLog2e / P.temperatures[id / P.rows_per_temp];
+    const int per = P.rows_per_temp;                // mostly 1 or a block's length: a shift, where a division of 64 bits per row stood in every tile's start
+    return kLog2e / P.temperatures[(per & (per - 1)) == 0 ? id >> __builtin_ctz(per) : id / per];
 }
 
 // The form for few rows: whether it covers the shape, and its launch (records only; n_slices is set to their number per row).

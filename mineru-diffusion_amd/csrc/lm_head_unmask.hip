@@ -41,11 +41,11 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
 }
 
 template <typename T>
-__global__ __launch_bounds__(T::kThreads, T::kWaves / 4) void lm_head_confidence_kernel(const LmHeadParams P)
+__global__ __launch_bounds__(T::kThreads, T::kWaves / 4) void lm_head_confidence_kernel(const LmHeadParams P, const Places places)
 {
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     const T tile;
-    const Place at = place_of((int)blockIdx.x, P.n_row_tiles, P.n_vocab_tiles);
+    const Place at = place_of(blockIdx.x, places);
     const int xr0 = at.m * T::BM, v0 = at.n * T::BN;
     const int row0 = tile.wm * (T::BM / T::WM) + tile.l16;        // this lane's first x row in the tile
     float c[T::TM];
@@ -224,7 +224,8 @@ int launch_tiles(LmHeadParams& P, hipStream_t stream)
     if (rc != MDX_OK) return rc;
     P.n_row_tiles = (P.rows + BM - 1) / BM;
     P.n_vocab_tiles = P.n_slices = (P.vocab + BN - 1) / BN;
-    lm_head_confidence_kernel<T><<<(unsigned)(P.n_row_tiles * P.n_vocab_tiles), T::kThreads, T::kStepsBytes, stream>>>(P);
+    const int64_t grid = (int64_t)P.n_row_tiles * P.n_vocab_tiles;
+    lm_head_confidence_kernel<T><<<(unsigned)grid, T::kThreads, T::kStepsBytes, stream>>>(P, places_of(P.n_row_tiles, P.n_vocab_tiles, grid));
     return mdx::check_launch("lm_head_confidence");
 }
 

@@ -112,6 +112,11 @@ template <typename V> __device__ __forceinline__ V xor_lanes(V v, int mask) {
 // 23.0 / 22.7, 32 of 600-2400 55.9 / 55.5; prompts 3 x 40-150 7.75 / 7.6, 500 13.4 / 13.2.  (In fp32 arithmetic 20.2 / 20.4: not there.)
 __device__ __forceinline__ unsigned quotient(unsigned n, unsigned d) { return (d & (d - 1)) == 0 ? n >> __builtin_ctz(d) : n / d; }
 
+// Division of 0 .. n_max by d with one multiplication (the host's choice of the factor; where it does not suffice, 0, by the general sequence).
+struct Divisor { unsigned d, factor; };
+inline Divisor divisor(uint64_t d, uint64_t n_max) { return Divisor{(unsigned)d, d > 1 && n_max * d < ((uint64_t)1 << 32) ? (unsigned)((((uint64_t)1 << 32) + d - 1) / d) : 0u}; }
+__device__ __forceinline__ unsigned quotient(unsigned n, Divisor by) { return by.factor ? __umulhi(n, by.factor) : by.d == 1 ? n : n / by.d; }
+
 // A kernel's arguments come through the scalar cache, 64 bytes at a time, and the compiler asks for them where they are first used, some of them behind
 // other loads.  This asks for all lines of BYTES bytes of arguments, and for the grid's size if it is given, at once.  Returns 0 in a way that the
 // compiler doesn't see, to be added to something that is used early.  (Not a volatile asm: behind one, the compiler no longer takes page tables and

@@ -30,3 +30,12 @@ def test_small_tiles_keep_slices_of_four_steps():
 def test_second_rounds_of_small_tiles_are_not_taken_for_free():
     """480 tiles of 32 x 64 would be two rounds on 256 CUs: two slices of K in larger tiles, which are one."""
     assert mdx._lib.lib().mdx_linear_splits(160, 6144, 2048) == 2
+
+
+def test_division_by_one_multiplication():
+    """What the tiles' places are computed by: the factor that divisor() of mdx_common.h chooses gives the quotient for every number up to its bound."""
+    for d in [2, 3, 5, 6, 7, 24, 48, 64, 96, 192, 594, 1187, 3561, 65535]:
+        factor = ((1 << 32) + d - 1) // d
+        n_max = ((1 << 32) - 1) // d
+        edges = {0, 1, d - 1, d, d + 1, n_max} | {m * d + e for m in (1, 2, 1000, n_max // d) for e in (-1, 0, 1)}
+        assert all(n * factor >> 32 == n // d for n in edges if 0 <= n <= n_max)
