@@ -63,7 +63,7 @@ __global__ __launch_bounds__(THREADS, 8) void topk_candidates_kernel(
     const int tid = threadIdx.x, split = blockIdx.y;
     const int64_t r = blockIdx.x;
     const RowView row = row_view(logits + r * row_stride, vocab);
-    const int per_split = (row.nchunk + nsplit - 1) / nsplit;               // <= THREADS * kChunksPerThread (the host's split)
+    const int per_split = mdx::quotient(row.nchunk + nsplit - 1, nsplit);               // <= THREADS * kChunksPerThread (the host's split)
     const int cbeg = split * per_split, cend = min(row.nchunk, cbeg + per_split);
     constexpr uint32_t kNothing = Bits16<T>::kNegInf | (Bits16<T>::kNegInf << 16);
 
@@ -279,7 +279,7 @@ __global__ __launch_bounds__(kPickThreads) void filtered_pick_kernel(
     __shared__ uint2 cand[kMaxCandidates];
     const int64_t r = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63;
-    const float T_ = temperatures ? temperatures[r / rows_per_temp] : 1.0f;
+    const float T_ = temperatures ? temperatures[mdx::quotient((unsigned)r, rows_per_temp)] : 1.0f;
     const float c = kLog2e / T_;
     Drawn<NOISE> drawn;
     drawn.np = NOISE == 1 ? N.noise + r * N.noise_row_stride : nullptr;

@@ -156,7 +156,7 @@ __global__ __launch_bounds__(kFilterThreads) void logit_filter_kernel(
     const int64_t r = blockIdx.x;
     const int tid = threadIdx.x;
     const RowView row = row_view(logits + r * row_stride, vocab);
-    const float c = kLog2e / (temperatures ? temperatures[r / rows_per_temp] : 1.0f);
+    const float c = kLog2e / (temperatures ? temperatures[mdx::quotient((unsigned)r, rows_per_temp)] : 1.0f);
     const uint32_t floor_key = floor_from_counts<T>(row, hist, sh, tid, top_k, top_p, c);
     if (!WRITE) {
         // (a cut-off below -inf is a NaN's; one above +inf drops every number, as it should)
