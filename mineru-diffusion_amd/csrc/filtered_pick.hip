@@ -36,15 +36,31 @@ __device__ __forceinline__ s16x2 ordered(uint32_t w) {
     return b ^ ((b >> 15) & s16x2{0x7fff, 0x7fff});
 }
 
-// The largest key (of 16 bits) that at least `want` of the wavefront's n x 64 keys reach; 0 if fewer keys than that are nonzero.
+// The largest key (of 16 bits) that at least `want` of the wavefront's n x 64 keys reach; 0 if fewer keys than that are nonzero.  Bit by bit, below those that all nonzero keys have in
+// common: what a top-k lists lies within a factor of two or four, 8 or 9 bits of bf16.  (Us, all 16 bits / so: 12 sequences, top-k 50 32.5 / 31.6, three 18.7 / 18.0, one 15.7 /
+// 14.7, top-k 400 53.3 / 52.1; fp16 keys spread wider, top-k 400 of six 42.4 / 42.6.  Two bits at a time, three counts beside each other: 32.5 / 33.2.)
 template <int N> __device__ __forceinline__ uint32_t kth_key(const uint32_t (&key)[N], int want) {
-    uint32_t t = 0;
-    for (int bit = 15; bit >= 0; --bit) {
-        const uint32_t trial = t | (1u << bit);
-        int n = 0;
+    uint32_t hi = 0, lo = 0xffff;
+    int n = 0;
 #pragma unroll
-        for (int i = 0; i < N; ++i) n += __popcll(__ballot(key[i] >= trial));
-        if (n >= want) t = trial;
+    for (int i = 0; i < N; ++i) {
+        hi = max(hi, key[i]);
+        lo = min(lo, key[i] ? key[i] : 0xffffu);
+        n += __popcll(__ballot(key[i] != 0));
+    }
+    if (n < want) return 0;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) { hi = max(hi, mdx::xor_lanes(hi, off)); lo = min(lo, mdx::xor_lanes(lo, off)); }
+    hi = __builtin_amdgcn_readfirstlane(hi);
+    lo = __builtin_amdgcn_readfirstlane(lo);
+    const int bits = hi == lo ? 0 : 32 - __builtin_clz(hi ^ lo);             // below them all keys are alike
+    uint32_t t = hi >> bits << bits;
+    for (int bit = bits - 1; bit >= 0; --bit) {
+        const uint32_t trial = t | (1u << bit);
+        int reached = 0;
+#pragma unroll
+        for (int i = 0; i < N; ++i) reached += __popcll(__ballot(key[i] >= trial));
+        if (reached >= want) t = trial;
     }
     return t;
 }
@@ -149,6 +165,35 @@ template <int NOISE> struct Drawn {
     }
 };
 
+// A wavefront's words in falling order over the lanes (a bitonic network in the vector unit).
+__device__ __forceinline__ uint32_t sorted_down(uint32_t word) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int size = 2; size <= 64; size <<= 1)
+#pragma unroll
+        for (int stride = size / 2; stride >= 1; stride >>= 1) {
+            const uint32_t other = mdx::xor_lanes(word, stride);
+            const bool larger = ((lane & stride) == 0) == ((lane & size) == 0);
+            word = larger ? max(word, other) : min(word, other);
+        }
+    return word;
+}
+// The sum over the lanes up to this one.
+__device__ __forceinline__ Mass running_total(Mass v) {
+    auto add = [&](auto control, auto rows) {
+        constexpr int C = decltype(control)::value, R = decltype(rows)::value;
+        const uint32_t lo = __builtin_amdgcn_update_dpp(0, (uint32_t)v, C, R, 0xf, false), hi = __builtin_amdgcn_update_dpp(0, (uint32_t)(v >> 32), C, R, 0xf, false);
+        v += ((Mass)hi << 32) | lo;
+    };
+    add(std::integral_constant<int, 0x111>(), std::integral_constant<int, 0xf>());        // row_shr:1, 2, 4, 8
+    add(std::integral_constant<int, 0x112>(), std::integral_constant<int, 0xf>());
+    add(std::integral_constant<int, 0x114>(), std::integral_constant<int, 0xf>());
+    add(std::integral_constant<int, 0x118>(), std::integral_constant<int, 0xf>());
+    add(std::integral_constant<int, 0x142>(), std::integral_constant<int, 0xa>());        // row_bcast:15 into rows 1 and 3
+    add(std::integral_constant<int, 0x143>(), std::integral_constant<int, 0xc>());        // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
 // One wavefront: token and confidence from the elements that the top-k has kept, N per lane (key 0: none).
 template <typename T, int NOISE, int N>
 __device__ __forceinline__ void pick_from_kept(uint32_t (&key)[N], const int (&column)[N], float top_p, float c, const Drawn<NOISE>& drawn, int64_t& x0, float& x0_p)
@@ -177,18 +222,13 @@ __device__ __forceinline__ void pick_from_kept(uint32_t (&key)[N], const int (&c
         const Mass target = share_of(total, top_p);
         uint32_t floor_key = 0;
         if (N == 1) {
-            // the mass at and above this lane's key, lane by lane: shorter than sixteen sums over the wavefront, one behind the other
-            Mass above = 0;
-#pragma unroll
-            for (int j = 0; j < 64; ++j) {
-                const uint32_t other = (uint32_t)__builtin_amdgcn_readlane((int)key[0], j);
-                const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)mass[0], j);
-                const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(mass[0] >> 32), j);
-                above += other >= key[0] ? ((Mass)hi << 32) | lo : 0ull;
-            }
-            floor_key = above > target ? key[0] : 0;
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) floor_key = max(floor_key, (uint32_t)mdx::xor_lanes((int)floor_key, off));
+            // (with the mass at and above each lane's key summed lane by lane, 64 times three words: 12 sequences, top-k 50 33.4 us, so 32.5, one 16.3 / 15.5)
+            // in falling order of the keys, the key at which the mass so far first exceeds the target (of equal keys any will do: the mass down to
+            // the last of them exceeds it then)
+            const uint32_t word = sorted_down((key[0] << 6) | (uint32_t)(threadIdx.x & 63));
+            const Mass so_far = running_total(__shfl(mass[0], (int)(word & 63)));
+            const unsigned long long enough = __ballot(so_far > target);
+            floor_key = enough ? (uint32_t)__builtin_amdgcn_readlane((int)word, __ffsll((long long)enough) - 1) >> 6 : 0;
         }
         for (int bit = 15; N > 1 && bit >= 0; --bit) {
             const uint32_t trial = floor_key | (1u << bit);

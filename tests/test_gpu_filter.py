@@ -220,6 +220,30 @@ def test_filtered_step_at_the_edges_of_a_lane_and_a_register(dev, V, k, p):
     assert torch.equal(a, b) and torch.equal(got[3], want[3])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("k", [1, 7, 17, 40, 64, 100])
+@pytest.mark.parametrize("p", [0.3, 0.6, 0.9, 0.99])
+def test_filtered_step_with_ties_across_both_cut_offs(dev, dtype, k, p):
+    """Candidates that share all bits but one, none but the sign, or all of them, and runs of equal ones on either side of the k-th and of the top-p
+    cut-off: against the step on the filtered copy, whose cut-offs are found by counting."""
+    import mdx
+    g = torch.Generator(device=dev).manual_seed(100 * k + int(100 * p))
+    V = 5000
+    rows = torch.full((1, 8, V), -60.0, device=dev)
+    values = [[5.0] + [4.5] * 6 + [4.0] * 10 + [3.5] * 30 + [1.0] * 200, [2.0] * 64 + [1.9921875] * 64, [3.0] * 300, [0.25, 0.0, -0.0, -0.25] * 40,
+              [-1.0] * 20 + [-2.0] * 50 + [-4.0] * 60, [8.0] + [-50.0] * 80, [float(v) for v in range(40, -40, -1)], [1.0, 0.5] * 33]
+    for row, v in zip(rows[0], values):
+        row[torch.randperm(V, generator=g, device=dev)[:len(v)]] = torch.tensor(v, device=dev)
+    logits = rows.to(dtype)
+    a = torch.full((1, 8), 9, dtype=torch.int64, device=dev)
+    b = a.clone()
+    got = mdx.unmask_step(logits, a, 9, 0.9, 2, temperatures=None, top_k=k, top_p=p, seed=5, offset=1)
+    want = mdx.unmask_step(mdx.filter_logits(logits, k, p, None), b, 9, 0.9, 2, temperatures=None, seed=5, offset=1)
+    assert torch.equal(got[0], want[0])
+    np.testing.assert_allclose(got[1].cpu().numpy(), want[1].cpu().numpy(), rtol=5e-6)    # as above: fp32 sums in another order
+    assert torch.equal(a, b) and torch.equal(got[3], want[3])
+
+
 @pytest.mark.parametrize("k", [3, 50, 400])
 def test_filtered_step_does_not_depend_on_the_order_of_its_candidates(dev, k):
     """The candidates of a row are listed in whatever order its wavefronts come: rows that hold the same logits at other columns
