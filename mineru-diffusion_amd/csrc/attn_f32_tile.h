@@ -188,7 +188,7 @@ __device__ __forceinline__ void tile_step(const float* lds, const float (&q)[D /
         s[i] = visible(row_of_reg(i, H)) ? s[i] * c : -INFINITY;
         mx = fmaxf(mx, s[i]);
     }
-    mx = fmaxf(mx, mdx::xor_lanes(mx, 32));
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
     const float m_new = fmaxf(st.m, mx);
     const float alpha = __builtin_amdgcn_exp2f(st.m - m_new);
     float sum = 0.f;
@@ -223,7 +223,7 @@ template <int D, int KW, typename Emit>
 __device__ __forceinline__ void fold_states(float* lds, State<D>& st, int wave, int lane, int width, Emit emit) {
     constexpr int kMl = (D / 32) * 16 * 64, kStateFloats = kMl + 2 * 64;       // O as [d tile][register quad][lane][4], then m, l
     const int H = lane >> 5, kw = wave % KW;
-    st.l += mdx::xor_lanes(st.l, 32);                                              // a state is now (m, l, O) per query
+    st.l += __shfl_xor(st.l, 32);                                              // a state is now (m, l, O) per query
     const float* states = lds + (wave - kw) * kStateFloats;
     auto quad = [&](int dt, int g) { return f32x4{st.o[dt][4 * g], st.o[dt][4 * g + 1], st.o[dt][4 * g + 2], st.o[dt][4 * g + 3]}; };
     // MINE: this wavefront's kw.  What it hands out itself stays in its registers.  (All of every state through LDS, four bytes at a time: 3600 cycles of a workgroup's

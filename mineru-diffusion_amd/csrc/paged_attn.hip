@@ -94,6 +94,7 @@ struct PagedParams {
     int chunk, nsplit;                              // keys per split, max splits per sequence
     int nqt;                                        // query tiles of 32 per sequence (grid z)
     int num_q_heads;
+    mdx::Divisor by_bs;
     int head_dim;                                   // <= 128, a multiple of 16: columns beyond it are zeros in LDS and never stored
     float c;                                        // scale * log2(e)
     float* part_o; float* part_ml;                  // [bs, Hq, nqt, nsplit, (d tile, register quad), lane, 4] and [bs, Hq, nqt, nsplit, 32, (m, l)]
@@ -213,16 +214,9 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
     int b, split, span = P.chunk;
     bool paced = false;
     typedef __attribute__((address_space(4))) const int32_t ConstantEntry;
-    constexpr bool kGuesses = sizeof...(AHEAD) == 0 && !MERGE;
-    int b_guessed = -1, pages_guessed = 0;
     int ctx_all = 0;                                // (up to 64 sequences) the clipped length of sequence `lane`
     if (P.bs <= 64) {
         // lengths beyond the page table name keys that do not exist: clipped here and below
-        // the first pages of the sequence that this is if all before it in launch order have as many pieces: on their way with the lengths
-        if (kGuesses) {
-            b_guessed = (int)blockIdx.y - mdx::quotient(blockIdx.y, P.bs) * P.bs;
-            pages_guessed = ((ConstantEntry*)(uintptr_t)P.block_table)[(int64_t)b_guessed * P.bt_stride + min(lane, P.max_pages - 1)];
-        }
         const int ctx_l = lane < P.bs ? min(max(0, P.context_lens[lane]), P.max_pages * P.page_size) : 0;
         ctx_all = ctx_l;
         bool cut = true;                            // false: every sequence is known to be one piece
@@ -305,8 +299,10 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
         } else {
             // the first split of every sequence, then the second of those that have one, ...: the last split of a sequence is its remainder
             // (from the level that the pair would have if all of them had that many: those below it hold a sum)
-            level = mdx::quotient(j, P.bs);
-            j -= level > 0 ? wave_sum(min(n, level)) : 0;
+            if (j >= P.bs) {
+                level = mdx::quotient(j, P.by_bs);
+                j -= wave_sum(min(n, level));
+            }
             for (; level < P.nsplit; ++level) if (among(__ballot(n > level))) break;
         }
         if (b < 0) return;                          // past the last (sequence, split) pair
@@ -334,7 +330,7 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
     const int key_end = __builtin_amdgcn_readfirstlane(min(ctx, key_begin + span));
     const int kvh = mdx::quotient(hg * HPW, P.heads_per_kv);
 
-    // (with the readers' loads in the kernel, or two ways to look pages up, the compiler no longer takes the table for constant by itself)
+    // (by itself the compiler takes the table for constant only in some forms of this kernel)
     auto table_row = [&] {
         const int32_t* row = P.block_table + (int64_t)__builtin_amdgcn_readfirstlane(b) * P.bt_stride;
         return (ConstantEntry*)(uintptr_t)row;
@@ -342,15 +338,16 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
     const auto bt = table_row();
     const int chunk = tid & 15, trow = tid >> 4;    // one pass stages kRowsPerPass rows
     const int n_tiles = (key_end - key_begin + kTileKeys - 1) / kTileKeys;
-    // The loads of a fetch are unconditional (rows past the context or on an invalid page id read a row of the page, or of page 0, instead and are zeroed when they
-    // reach LDS).  Where a tile lies in one page (tile_in_page) its page comes from a register that holds the piece's first 64, and its loads stand one
-    // behind the other; else each pass of kRowsPerPass keys, which never straddles a page (page_size % 32 == 0), looks its page up.  A lookup is 500 to 1700 cycles, waited for before
-    // the pass's loads: with one per pass the first two tiles' loads took 4800 cycles of a workgroup's start, and the first had landed before the last was asked
-    // for.  The layer, us, before / now: one sequence of 1337 keys 14.4 / 14.0, 4000 19.2 / 18.3, 12 000 27.7 / 25.1, four of 1000-3000 22.7 / 22.0, eight 30.3 / 28.8, 12 of 500-2500 34.8 / 32.5.
-    // Not everywhere (`paced`): where the launch fills most of the resident workgroups HBM is the bound, and workgroups that ask for their tiles as soon as they can crowd out
-    // each other; there a lookup per pass spreads the loads behind the first two tiles (16 of 512-4096 44.4 / 41.9, start 42.6, 8 of 3000-6000 42.2 / 41.4).  K's rows of a tile before V's is
-    // the better order there too, and with a pair per CU (32 of 600-2400 56.5 / 56.1), at the start as well, while few workgroups do best with K and V in turn at the start.  And not beside readers:
-    // that launch lasts as long as those do (generating with one request 61.7 ms, 62.1 with tiles looked up at once, eight 57.5 / 58.5).
+    // The loads of a fetch are unconditional (rows past the context or on an invalid page id read row `trow` of page 0 instead and are zeroed when they reach LDS).
+    // Each pass of kRowsPerPass keys, which never straddles a page (page_size % 32 == 0), looks its page up: in the first tiles, whose lookups, through the constant address
+    // space, are all on their way at once.  (Through an ordinary pointer each was waited for before its pass's loads: 4800 cycles of a workgroup's start, and the first tile had
+    // landed before the second was asked for.  From a register that holds the piece's first 64 pages, as behind the first tiles, the start is slower: one sequence of 1337
+    // keys 14.1 us, so 13.3, 17 of 120 13.4 / 12.4.)  Behind them, where a tile lies in one page (paged_tiles), its page comes from that register: a scalar load that is
+    // waited for among the reads from LDS holds them all up.  K's rows of a tile are asked for before V's, which HBM prefers (32 of 600-2400 56.5 / 56.1).  The layer, us, before both / now: one
+    // sequence of 300 keys 11.9 / 11.0, 1337 14.6 / 13.3, 12 000 27.4 / 24.6, four of 1000-3000 23.0 / 21.3, 12 of 500-2500 34.8 / 32.4.  Not where the launch fills most of the resident
+    // workgroups (`paced`): HBM is the bound there, workgroups that ask for their tiles as soon as they can crowd out each other, and a lookup per pass spreads the loads
+    // (16 of 512-4096: 42.9 before, 44.4 without the rule, 41.8 with it); nor beside readers: that launch lasts as long as those do (generating with one request 61.7 ms, 62.1 with it,
+    // eight 57.5 / 58.5); nor with eight wavefronts (32 of 600-2400 56.4 / 56.0).
     struct Staged {
         TileRegs<kTileKeys, kThreads> regs;
         unsigned row_ok;       // bit p: this thread's row of pass p holds a real key
@@ -362,9 +359,7 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
     const bool tile_in_page = sizeof...(AHEAD) == 0 && WAVES == 4 && P.page_shift >= 0 && P.page_size >= kTileKeys && (key_begin & (kTileKeys - 1)) == 0;
     const bool paged_tiles = tile_in_page && !paced;
     auto slot_of = [&](int key) { return P.page_shift >= 0 ? key >> P.page_shift : key / P.page_size; };
-    const bool guessed = kGuesses && b == b_guessed && slot_of(key_end - 1) < 64;
-    const int first_slot = guessed ? 0 : slot_of(key_begin);
-    const int pages = guessed ? pages_guessed : bt[min(first_slot + lane, P.max_pages - 1)];
+    const int first_slot = slot_of(key_begin), pages = bt[min(first_slot + lane, P.max_pages - 1)];
     auto load_k = [&](Staged& sg, int p, int64_t off) { sg.regs.k[p] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(P.k_cache + off)); };
     auto load_v = [&](Staged& sg, int p, int64_t off, bool ok, int key0) {
         sg.regs.v[p] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(P.v_cache + off));
@@ -375,22 +370,17 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
         const int key0 = key_begin + t * kTileKeys;
         sg.row_ok = 0;
         sg.pass_ok = 0;
-        if (first ? tile_in_page : paged_tiles) {
+        if (!first && paged_tiles) {
             const int ahead = slot_of(key0) - first_slot, page = ahead < 64 ? __builtin_amdgcn_readlane(pages, ahead) : bt[first_slot + ahead];
             const bool valid = page >= 0 && page < P.num_pages;
             const int64_t base = valid ? page * P.c_sp + (int64_t)(key0 & (P.page_size - 1)) * P.c_st : 0;
-            auto offset = [&](int p) { return base + (int64_t)(kRowsPerPass * p) * P.c_st + safe_off; };
             auto ok = [&](int p) { return valid && key0 + kRowsPerPass * p < key_end; };
+            auto offset = [&](int p) { return (ok(p) ? base + (int64_t)(kRowsPerPass * p) * P.c_st : 0) + safe_off; };
 #pragma unroll
-            for (int p = 0; p < kPasses; ++p) {
-                load_k(sg, p, offset(p));
-                if (first && !MERGE) load_v(sg, p, offset(p), ok(p), key0);
-            }
-            if (!first || MERGE) {
-                __builtin_amdgcn_sched_barrier(0);
+            for (int p = 0; p < kPasses; ++p) load_k(sg, p, offset(p));
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int p = 0; p < kPasses; ++p) load_v(sg, p, offset(p), ok(p), key0);
-            }
+            for (int p = 0; p < kPasses; ++p) load_v(sg, p, offset(p), ok(p), key0);
         } else {
 #pragma unroll
             for (int p = 0; p < kPasses; ++p) {
@@ -463,11 +453,9 @@ __global__ __launch_bounds__(64 * WAVES, (WAVES / HPW == 2) ? 2 : 1) void paged_
     }
 
     // ---- merge the KW key-slice states of each head through LDS ---------------------------------
-    // Every slice leaves its state in LDS (register quads as 16-byte lanes: 16 stores of 1 KB per wavefront); after one
-    // barrier slice kw folds the d tiles kw, kw + KW, ... of all KW states -- every slice a quarter (half) of the head,
-    // and every slice stores what it folded.  (A tree of pairwise merges with 4-byte LDS accesses and three barriers,
-    // all output from one wavefront, took 2.7 us of every workgroup's end.)  All slices sum in the same order, so they
-    // agree on the head's m and l bit for bit.
+    // Slice kw folds, and stores, the d tiles kw, kw + KW, ... of its head: it leaves the other d tiles of its state in LDS as 16-byte lanes (of four slices: all of them),
+    // and behind one barrier takes its own from the others'.  (A tree of pairwise merges with 4-byte LDS accesses and three barriers, all output from one wavefront, took
+    // 2.7 us of every workgroup's end.)  All slices sum in the same order, so they agree on the head's m and l bit for bit.
     // (single launch: how many splits of this pair have counted themselves in -- asked for here, needed behind the merge)
     __shared__ int counted;
     float* const counter = MERGE ? P.arrive + ((int64_t)b * n_groups + hg) * P.nqt + qt : nullptr;
@@ -871,6 +859,7 @@ int launch_paged_ahead(const void* q, void* o, const void* k_cache, const void* 
     P.chunk = pick_chunk(bs, (int)wg_per_pair, max_pages, page_size, &device_span);
     P.nsplit = nsplit_of(bs, (int64_t)num_q_heads * P.nqt, max_pages, page_size, P.chunk, device_span);
     P.num_q_heads = num_q_heads;
+    P.by_bs = mdx::divisor(bs, (uint64_t)bs * P.nsplit);
     P.head_dim = head_dim;
     P.c = scale * kLog2e;
     P.part_o = nullptr; P.part_ml = nullptr; P.span_out = nullptr; P.arrive = nullptr; P.fit_slots = 0;
